@@ -878,6 +878,17 @@ int ks_lstm_backward_step(KsLstm* lstm, ks_stream_t stream, int64_t M, const flo
                           const float* saved, const uint8_t* fresh, float* d_g, float* dh_in, float* dc_in, void* workspace);
 int ks_lstm_grad_sqnorm(const KsLstm* lstm, ks_stream_t stream, double* acc);
 int ks_lstm_adam_step(KsLstm* lstm, ks_stream_t stream, const KsAdamParams* params /*host*/, const double* sqnorm);
+/* A whole trajectory of one GRU layer in one launch each way, for cells of hidden size 128 in either precision
+ * (ks_gru_sequence_supported returns 1; other cells take the step-by-step entry points).  gi (T, M, 3H) = W_ih x_t + bias for every
+ * step; hs (T, M, H), saved (T, M, 5H) nullable, in the layout of ks_gru_train_forward; with T = 1, hs may alias h0, and
+ * ks_gru_forward / ks_gru_train_forward are this launch with T = 1 for such cells.  Backward: dH (T, M, H) the gradient reaching h_t
+ * from the layer above, d_gi, d_gh (T, M, 3H) out as ks_gru_backward_step returns them per step, dh0 (M, H) nullable.  bf16 cells
+ * round the state and the gate gradients to bf16 on their way into the products and keep both in fp32 otherwise. */
+int ks_gru_sequence_supported(const KsGru* gru);
+int ks_gru_sequence_forward(const KsGru* gru, ks_stream_t stream, int64_t T, int64_t M, const float* gi, const float* h0,
+                            const uint8_t* fresh, float* hs, float* saved);
+int ks_gru_sequence_backward(const KsGru* gru, ks_stream_t stream, int64_t T, int64_t M, const float* dH, const float* saved,
+                             const uint8_t* fresh, float* d_gi, float* d_gh, float* dh0);
 /* A whole trajectory of one LSTM layer in one launch each way: the lax.scan over the T steps of the trajectory inside the loss
  * (ksim/task/ppo.py:572-694 around the model's forward, examples/kbot/train.py:903-915) and what jax.grad derives for it, for
  * fp32 cells of hidden size 128 (ks_lstm_sequence_supported returns 1; other cells take the step-by-step entry points above).

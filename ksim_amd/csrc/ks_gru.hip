@@ -2,6 +2,7 @@
 // layers and run through the MLP entry points (matrix cores for bf16); one streaming kernel then combines the gates.
 #include "ks_common.h"
 
+#include <type_traits>
 #include <vector>
 
 namespace ks {
@@ -394,6 +395,232 @@ void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, co
   }
 }
 
+// ---------------------------------------------------------------- a whole trajectory of one GRU layer in one launch
+// The layout of the LSTM kernels above: eight wavefronts own 4 rows for all T steps, block b = lane / 4 of wavefront w is hidden
+// unit 16 w + b, its B entries are that unit's reset / update / candidate rows of W_hh (the fourth entry is zero), and the four
+// rows' state is the A operand broadcast from one block per instruction.  fp32 cells multiply with v_mfma_f32_4x4x1 (128 per step);
+// bf16 cells with v_mfma_f32_4x4x4 bf16 (32 per step), for which the state, kept in fp32 in a register of the lane that owns it,
+// is rounded to bf16 on its way to LDS, as the per-step products round their input.  Bound by the latency of a step's chain
+// (LDS read, products, gates, LDS write, barrier); the per-step launches this replaces were four per step and layer (512 rows,
+// 24 steps, bf16: 4 x 24 launches of 3-8 us -> one).
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+
+__device__ __forceinline__ short bf16_bits(float x) { return __builtin_bit_cast(short, (__bf16)x); }
+
+template <bool BF>
+__global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gru_seq_forward_kernel(int T, int64_t M, int groups, const float* __restrict__ gi, const void* __restrict__ Wv, int ldw,
+                            const float* __restrict__ bias_n, const float* h0, const uint8_t* __restrict__ fresh, float* hs,
+                            float* __restrict__ saved) {  // with T = 1, hs may be h0
+  constexpr int H = kSeqH;
+  // fp32: the state in seq_slot order, two 16-byte reads per lane and step.  bf16: in natural order, block b reads units 4 b .. 4 b + 3
+  // and 64 + 4 b .. (8 bytes each): the operands of instructions b and 16 + b
+  __shared__ __attribute__((aligned(16))) float sh[2][kSeqRows][kSeqPadH];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 3, blk = lane >> 2, unit = 16 * wave + blk;
+  constexpr int NW = BF ? 1 : H, NB = BF ? H / 4 : 1;
+  float wa[NW];
+  s16x4 wb[NB];
+  if constexpr (BF) {
+    const s16x4* src = reinterpret_cast<const s16x4*>((const short*)Wv + (int64_t)((j < 3 ? j : 0) * H + unit) * ldw);
+#pragma unroll
+    for (int k4 = 0; k4 < NB; ++k4) {
+      const s16x4 v = src[k4];
+      wb[k4] = j < 3 ? v : s16x4{0, 0, 0, 0};
+    }
+  } else {
+    const float4* src = reinterpret_cast<const float4*>((const float*)Wv + (int64_t)((j < 3 ? j : 0) * H + unit) * ldw);
+#pragma unroll
+    for (int k4 = 0; k4 < NW / 4; ++k4) {
+      const float4 v = src[k4];
+      wa[4 * k4] = j < 3 ? v.x : 0.f; wa[4 * k4 + 1] = j < 3 ? v.y : 0.f; wa[4 * k4 + 2] = j < 3 ? v.z : 0.f; wa[4 * k4 + 3] = j < 3 ? v.w : 0.f;
+    }
+  }
+  const float bn = bias_n[unit];
+  for (int grp = 0; grp < groups; ++grp) {  // as in the LSTM kernel: several sets of 4 rows with the same registers of weights
+    const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * kSeqRows;
+    if (r0 >= M) break;  // the same for every thread of the workgroup
+    const int64_t m = r0 + j;
+    const bool row_ok = m < M;
+    const int64_t mc = row_ok ? m : M - 1;  // loads of the rows past the batch are clamped, their stores dropped
+    if (grp > 0) __syncthreads();
+    float hprev = h0[mc * H + unit];
+    if constexpr (BF) reinterpret_cast<short*>(&sh[0][j][0])[unit] = bf16_bits(hprev);
+    else sh[0][j][seq_slot(unit)] = hprev;
+    __syncthreads();
+    int cur = 0;
+    float gnext[3];
+    uint8_t fnext = 0;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) gnext[g] = gi[mc * 3 * H + g * H + unit];
+    if (fresh) fnext = fresh[mc];
+    for (int t = 0; t < T; ++t) {
+      float gin[3];
+#pragma unroll
+      for (int g = 0; g < 3; ++g) gin[g] = gnext[g];
+      const bool f = fnext != 0;
+      if (t + 1 < T) {  // the next step's inputs, fetched under this step's work
+        const int64_t tn = (int64_t)(t + 1) * M + mc;
+#pragma unroll
+        for (int g = 0; g < 3; ++g) gnext[g] = gi[tn * 3 * H + g * H + unit];
+        if (fresh) fnext = fresh[tn];
+      }
+      f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (BF) {
+        const s16x4* row = reinterpret_cast<const s16x4*>(&sh[cur][j][0]);
+        const s16x4 a0 = row[blk], a1 = row[16 + blk];
+#define KS_GRU_MFMA(B)                                                                                    \
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a0, wb[(B)], acc0, 4, (B), 0);                       \
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a1, wb[16 + (B)], acc1, 4, (B), 0);
+#define KS_GRU_MFMA4(B) KS_GRU_MFMA(B) KS_GRU_MFMA((B) + 1) KS_GRU_MFMA((B) + 2) KS_GRU_MFMA((B) + 3)
+        KS_GRU_MFMA4(0) KS_GRU_MFMA4(4) KS_GRU_MFMA4(8) KS_GRU_MFMA4(12)
+#undef KS_GRU_MFMA4
+#undef KS_GRU_MFMA
+      } else {
+        float ha[8];
+        {
+          const float4 a0 = *reinterpret_cast<const float4*>(&sh[cur][j][8 * blk]);
+          const float4 a1 = *reinterpret_cast<const float4*>(&sh[cur][j][8 * blk + 4]);
+          ha[0] = a0.x; ha[1] = a0.y; ha[2] = a0.z; ha[3] = a0.w; ha[4] = a1.x; ha[5] = a1.y; ha[6] = a1.z; ha[7] = a1.w;
+        }
+#define KS_GRU_MFMA(K0)                                                                                            \
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[(K0) >> 4], wa[(K0)], acc0, 4, (K0) & 15, 0);                    \
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[((K0) + 1) >> 4], wa[(K0) + 1], acc1, 4, ((K0) + 1) & 15, 0);
+#define KS_GRU_MFMA8(K0) KS_GRU_MFMA(K0) KS_GRU_MFMA((K0) + 2) KS_GRU_MFMA((K0) + 4) KS_GRU_MFMA((K0) + 6)
+#define KS_GRU_MFMA32(K0) KS_GRU_MFMA8(K0) KS_GRU_MFMA8((K0) + 8) KS_GRU_MFMA8((K0) + 16) KS_GRU_MFMA8((K0) + 24)
+        KS_GRU_MFMA32(0) KS_GRU_MFMA32(32) KS_GRU_MFMA32(64) KS_GRU_MFMA32(96)
+#undef KS_GRU_MFMA32
+#undef KS_GRU_MFMA8
+#undef KS_GRU_MFMA
+      }
+      float pre[4];
+      quad_transpose(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3], j, pre);
+      const float hu = f ? 0.f : hprev;
+      const float hn = bn + (f ? 0.f : pre[2]);
+      const float r = seq_sigmoid(gin[0] + (f ? 0.f : pre[0]));
+      const float z = seq_sigmoid(gin[1] + (f ? 0.f : pre[1]));
+      const float n = seq_tanh(gin[2] + r * hn);
+      hprev = n + z * (hu - n);
+      if constexpr (BF) reinterpret_cast<short*>(&sh[cur ^ 1][j][0])[unit] = bf16_bits(hprev);
+      else sh[cur ^ 1][j][seq_slot(unit)] = hprev;
+      if (row_ok) {
+        const int64_t o = (int64_t)t * M + m;
+        hs[o * H + unit] = hprev;
+        if (saved) {
+          float* sv = saved + o * 5 * H + unit;
+          sv[0] = r; sv[H] = z; sv[2 * H] = n; sv[3 * H] = hn; sv[4 * H] = hu;
+        }
+      }
+      lds_barrier();
+      cur ^= 1;
+    }
+  }
+}
+
+// The reverse sweep (gru_gate_backward_kernel's formulas): dh_{t-1} = dh_t z + d_gh W_hh.  Sixteen blocks = four groups of four units
+// times four quarters of the 3H gate rows, as in the LSTM's sweep.
+template <bool BF>
+__global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gru_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, const float* __restrict__ saved,
+                             const uint8_t* __restrict__ fresh, const void* __restrict__ Wtv, int ldwt, float* __restrict__ d_gi,
+                             float* __restrict__ d_gh, float* __restrict__ dh0) {
+  constexpr int H = kSeqH, KQ = 3 * H / 4;  // gate rows per quarter
+  constexpr int LDG = BF ? 3 * H + 8 : 3 * H + 4;
+  typedef typename std::conditional<BF, short, float>::type G;
+  __shared__ __attribute__((aligned(16))) G sg[kSeqRows][LDG];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 3, ug = (lane >> 2) & 3, kg = lane >> 4;
+  const int unit = 16 * wave + 4 * ug + kg;
+  const int64_t m = (int64_t)blockIdx.x * kSeqRows + j;
+  const bool row_ok = m < M;
+  const int64_t mc = row_ok ? m : M - 1;
+  constexpr int NW = BF ? 1 : KQ, NB = BF ? KQ / 4 : 1;
+  float wa[NW];
+  s16x4 wb[NB];
+  if constexpr (BF) {
+    const s16x4* src = reinterpret_cast<const s16x4*>((const short*)Wtv + (int64_t)(16 * wave + 4 * ug + j) * ldwt + KQ * kg);
+#pragma unroll
+    for (int s4 = 0; s4 < NB; ++s4) wb[s4] = src[s4];
+  } else {
+    const float4* src = reinterpret_cast<const float4*>((const float*)Wtv + (int64_t)(16 * wave + 4 * ug + j) * ldwt + KQ * kg);
+#pragma unroll
+    for (int s4 = 0; s4 < NW / 4; ++s4) {
+      const float4 v = src[s4];
+      wa[4 * s4] = v.x; wa[4 * s4 + 1] = v.y; wa[4 * s4 + 2] = v.z; wa[4 * s4 + 3] = v.w;
+    }
+  }
+  float dhc = 0.f;
+  float nx[6];
+  uint8_t fnext = 0;
+  {
+    const int64_t o = (int64_t)(T - 1) * M + mc;
+    const float* sv = saved + o * 5 * H + unit;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) nx[k] = sv[k * H];
+    nx[5] = dH[o * H + unit];
+    if (fresh) fnext = fresh[o];
+  }
+  for (int t = T - 1; t >= 0; --t) {
+    const bool f = fnext != 0;
+    const float r = nx[0], z = nx[1], n = nx[2], hn = nx[3], h = nx[4];
+    const float d = nx[5] + dhc;
+    if (t > 0) {
+      const int64_t o = (int64_t)(t - 1) * M + mc;
+      const float* sv = saved + o * 5 * H + unit;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) nx[k] = sv[k * H];
+      nx[5] = dH[o * H + unit];
+      if (fresh) fnext = fresh[o];
+    }
+    const float gN = d * (1.f - z) * (1.f - n * n);
+    const float gZ = d * (h - n) * z * (1.f - z);
+    const float gR = gN * hn * r * (1.f - r);
+    const float gNh = gN * r;
+    if constexpr (BF) {
+      sg[j][unit] = bf16_bits(gR); sg[j][H + unit] = bf16_bits(gZ); sg[j][2 * H + unit] = bf16_bits(gNh);
+    } else {
+      sg[j][unit] = gR; sg[j][H + unit] = gZ; sg[j][2 * H + unit] = gNh;
+    }
+    if (row_ok) {
+      const int64_t o = ((int64_t)t * M + m) * 3 * H + unit;
+      d_gi[o] = gR; d_gi[o + H] = gZ; d_gi[o + 2 * H] = gN;
+      d_gh[o] = gR; d_gh[o + H] = gZ; d_gh[o + 2 * H] = gNh;
+    }
+    lds_barrier();
+    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (BF) {
+      const s16x4* grow = reinterpret_cast<const s16x4*>(&sg[j][KQ * kg]);
+#pragma unroll
+      for (int s4 = 0; s4 < NB; s4 += 2) {
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(wb[s4], grow[s4], acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(wb[s4 + 1], grow[s4 + 1], acc1, 0, 0, 0);
+      }
+    } else {
+      const float* grow = &sg[j][KQ * kg];
+#pragma unroll
+      for (int s4 = 0; s4 < NW / 4; ++s4) {
+        const float4 gb = *reinterpret_cast<const float4*>(grow + 4 * s4);
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4], gb.x, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 1], gb.y, acc1, 0, 0, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 2], gb.z, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 3], gb.w, acc1, 0, 0, 0);
+      }
+    }
+    float part[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v = acc0[q] + acc1[q];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      part[q] = v;
+    }
+    const float mine = kg == 0 ? part[0] : (kg == 1 ? part[1] : (kg == 2 ? part[2] : part[3]));
+    dhc = f ? 0.f : d * z + mine;
+    lds_barrier();
+  }
+  if (row_ok && dh0) dh0[m * H + unit] = dhc;
+}
+
 }  // namespace ks
 
 using namespace ks;
@@ -441,6 +668,69 @@ extern "C" int ks_gru_destroy(KsGru* g) {
 
 static int64_t up256(int64_t n) { return (n + 255) / 256 * 256; }
 
+// whether the one-launch sequence kernels cover this cell: hidden size 128, either precision
+static bool gru_seq_weights(const KsGru* g, const void** W, int* ldw, const void** Wt, int* ldwt, bool* bf16) {
+  int np = 0, kp = 0, dt = 0;
+  *W = *Wt = nullptr;
+  if (!g || g->H != kSeqH || mlp_peek_layer(g->proj_h, 0, W, Wt, &np, &kp, &dt) != KS_OK) return false;
+  if (np != 3 * kSeqH || kp < kSeqH || (kp & 7)) return false;
+  *ldw = kp; *ldwt = np; *bf16 = dt == KS_MLP_BF16;
+  return *W != nullptr;
+}
+
+// sets of 4 rows per workgroup of the sequence kernels: one while there is at most one set per CU (long sequences want every CU),
+// more when a short call covers so many rows that re-reading the weights per set would dominate it
+static int seq_groups(int64_t T, int64_t sets) {
+  int groups = 1;
+  if (T * 8 <= 64) while (groups < 8 && sets > (int64_t)256 * groups) groups *= 2;
+  return groups;
+}
+
+extern "C" int ks_gru_sequence_supported(const KsGru* g) {
+  const void *W, *Wt;
+  int a, b;
+  bool bf;
+  return gru_seq_weights(g, &W, &a, &Wt, &b, &bf) ? 1 : 0;
+}
+
+extern "C" int ks_gru_sequence_forward(const KsGru* g, ks_stream_t stream, int64_t T, int64_t M, const float* gi, const float* h0,
+                                       const uint8_t* fresh, float* hs, float* saved) {
+  if (!g || !gi || !h0 || !hs) return fail(KS_EINVAL, "ks_gru_sequence_forward: null argument");
+  if (T < 0 || M < 0) return fail(KS_EINVAL, "ks_gru_sequence_forward: negative size");
+  if (T == 0 || M == 0) return KS_OK;
+  const void *W, *Wt;
+  int ldw, ldwt;
+  bool bf;
+  if (!gru_seq_weights(g, &W, &ldw, &Wt, &ldwt, &bf)) return fail(KS_EINVAL, "ks_gru_sequence_forward: needs a cell of hidden size %d", kSeqH);
+  if (T > 1 && hs == h0) return fail(KS_EINVAL, "ks_gru_sequence_forward: the output may alias the initial state only for T = 1");
+  const int64_t sets = (M + kSeqRows - 1) / kSeqRows;
+  const int groups = seq_groups(T, sets);
+  const int64_t grid = (sets + groups - 1) / groups;
+  if (grid > 0x7fffffff || T > 0x7fffffff) return fail(KS_ELIMIT, "ks_gru_sequence_forward: too many rows or steps");
+  auto kfn = bf ? gru_seq_forward_kernel<true> : gru_seq_forward_kernel<false>;
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, M, groups, gi, W, ldw, g->bias_n,
+                     h0, fresh, hs, saved);
+  return check_launch("ks_gru_sequence_forward");
+}
+
+extern "C" int ks_gru_sequence_backward(const KsGru* g, ks_stream_t stream, int64_t T, int64_t M, const float* dH, const float* saved,
+                                        const uint8_t* fresh, float* d_gi, float* d_gh, float* dh0) {
+  if (!g || !dH || !saved || !d_gi || !d_gh) return fail(KS_EINVAL, "ks_gru_sequence_backward: null argument");
+  if (T < 0 || M < 0) return fail(KS_EINVAL, "ks_gru_sequence_backward: negative size");
+  if (T == 0 || M == 0) return KS_OK;
+  const void *W, *Wt;
+  int ldw, ldwt;
+  bool bf;
+  if (!gru_seq_weights(g, &W, &ldw, &Wt, &ldwt, &bf)) return fail(KS_EINVAL, "ks_gru_sequence_backward: needs a cell of hidden size %d", kSeqH);
+  if (!Wt) return fail(KS_EINVAL, "ks_gru_sequence_backward: ks_gru_train_init has not run");
+  const int64_t grid = (M + kSeqRows - 1) / kSeqRows;
+  if (grid > 0x7fffffff || T > 0x7fffffff) return fail(KS_ELIMIT, "ks_gru_sequence_backward: too many rows or steps");
+  auto kfn = bf ? gru_seq_backward_kernel<true> : gru_seq_backward_kernel<false>;
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, M, dH, saved, fresh, Wt, ldwt, d_gi,
+                     d_gh, dh0);
+  return check_launch("ks_gru_sequence_backward");
+}
+
 extern "C" int64_t ks_gru_workspace_bytes(const KsGru* g, int64_t M) {
   if (!g || M < 0) return -1;
   const int64_t gates = up256(M * 3 * g->H * 4);
@@ -461,6 +751,8 @@ extern "C" int ks_gru_forward(const KsGru* g, ks_stream_t stream, int64_t M, con
   void* wh = w + 2 * gates + up256(ks_mlp_workspace_bytes(g->proj_i, M));
   int rc = ks_mlp_forward(g->proj_i, stream, M, x, gi, wi);
   if (rc != KS_OK) return rc;
+  // one step of the sequence kernel where it applies: a rollout's steps and the replay of its trajectory then give the same bits
+  if (ks_gru_sequence_supported(g)) return ks_gru_sequence_forward(g, stream, 1, M, gi, h_in, fresh, h_out, nullptr);
   rc = ks_mlp_forward(g->proj_h, stream, M, h_in, gh, wh);
   if (rc != KS_OK) return rc;
   const int64_t n = M * g->H, grid = (n + 255) / 256;
@@ -520,6 +812,8 @@ extern "C" int ks_gru_train_forward(const KsGru* g, ks_stream_t stream, int64_t 
   void* wh = w + 2 * gates + up256(ks_mlp_workspace_bytes(g->proj_i, M));
   int rc = ks_mlp_forward(g->proj_i, stream, M, x, gi, wi);
   if (rc != KS_OK) return rc;
+  // one step of the sequence kernel where it applies: a rollout's steps and the replay of its trajectory then give the same bits
+  if (ks_gru_sequence_supported(g)) return ks_gru_sequence_forward(g, stream, 1, M, gi, h_in, fresh, h_out, saved);
   rc = ks_mlp_forward(g->proj_h, stream, M, h_in, gh, wh);
   if (rc != KS_OK) return rc;
   const int64_t n = M * g->H, grid = (n + 255) / 256;
@@ -640,11 +934,8 @@ extern "C" int ks_lstm_sequence_forward(const KsLstm* g, ks_stream_t stream, int
   int ldw, ldwt;
   if (!lstm_seq_weights(g, &W, &ldw, &Wt, &ldwt)) return fail(KS_EINVAL, "ks_lstm_sequence_forward: needs an fp32 cell of hidden size %d", kSeqH);
   if (T > 1 && (hs == h0 || (cs && cs == c0))) return fail(KS_EINVAL, "ks_lstm_sequence_forward: outputs may alias the initial state only for T = 1");
-  // sets of 4 rows per workgroup: one while there is at most one set per CU (long sequences want every CU), more when a short
-  // call covers so many rows that re-reading the weights per set would dominate it
   const int64_t sets = (M + kSeqRows - 1) / kSeqRows;
-  int groups = 1;
-  if (T * 8 <= 64) while (groups < 8 && sets > (int64_t)256 * groups) groups *= 2;
+  const int groups = seq_groups(T, sets);
   const int64_t grid = (sets + groups - 1) / groups;
   if (grid > 0x7fffffff || T > 0x7fffffff) return fail(KS_ELIMIT, "ks_lstm_sequence_forward: too many rows or steps");
   hipLaunchKernelGGL(lstm_seq_forward_kernel, dim3((unsigned)grid), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, M, groups, gi, W,

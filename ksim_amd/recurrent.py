@@ -49,6 +49,7 @@ class GRUCell:
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_gru_create(ctypes.byref(d), ctypes.byref(self._handle)))
         self._ws: torch.Tensor | None = None
+        self._proj: MLP | None = None
 
     def workspace(self, M: int, device) -> torch.Tensor:
         need = int(self._lib.ks_gru_workspace_bytes(self._handle, M))
@@ -99,6 +100,43 @@ class GRUCell:
         _lib.check(self._lib.ks_gru_train_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(h), _lib.ptr(fresh),
                                                   _lib.ptr(out), _lib.ptr(saved), _lib.ptr(self.workspace(M, x.device))))
         return out
+
+    @property
+    def sequence_supported(self) -> bool:
+        """Whether this cell has the one-launch-per-trajectory kernels (`ks_gru_sequence_forward / _backward`)."""
+        return bool(self._lib.ks_gru_sequence_supported(self._handle))
+
+    def _input_projection(self) -> MLP:
+        """W_ih x + b of this cell as a network of one layer; there from the start, trained or not."""
+        if self._proj is None:
+            pi, ph = ctypes.c_void_p(), ctypes.c_void_p()
+            _lib.check(self._lib.ks_gru_projections(self._handle, ctypes.byref(pi), ctypes.byref(ph)))
+            self._proj = MLP._borrow(self._lib, pi, (self.input_size, 3 * self.hidden_size), self.dtype)
+        return self._proj
+
+    def sequence_forward(self, x, h0, fresh, hs, saved) -> None:
+        """The layer over a whole trajectory: x (T, M, input) -> hs (T, M, H) and `saved` (T, M, 5H; None where no backward
+        pass follows), from the carry h0; the input projection is one product over all T M rows, the recurrence one launch."""
+        _lib.require_cuda(x, h0, hs, saved, dtype=torch.float32)
+        _lib.require_cuda(fresh, dtype=torch.uint8)
+        Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
+        if (tuple(x.shape) != (Tn, M, self.input_size) or tuple(h0.shape) != (M, H) or tuple(hs.shape) != (Tn, M, H)
+                or (saved is not None and tuple(saved.shape) != (Tn, M, 5 * H)) or tuple(fresh.shape) != (Tn, M)):
+            raise _lib.KsError("expected x (T, M, input), h0 (M, H), hs (T, M, H), saved (T, M, 5H), fresh (T, M)")
+        gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
+        _lib.check(self._lib.ks_gru_sequence_forward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(gi), _lib.ptr(h0),
+                                                     _lib.ptr(fresh), _lib.ptr(hs), _lib.ptr(saved)))
+
+    def sequence_backward(self, dH, saved, fresh, d_gi, d_gh) -> None:
+        """The reverse sweep over the trajectory: dH (T, M, H), the gradient reaching every h_t from above, -> d_gi, d_gh (T, M, 3H)."""
+        _lib.require_cuda(dH, saved, d_gi, d_gh, dtype=torch.float32)
+        _lib.require_cuda(fresh, dtype=torch.uint8)
+        Tn, M, H = dH.shape[0], dH.shape[1], self.hidden_size
+        if (tuple(dH.shape) != (Tn, M, H) or tuple(saved.shape) != (Tn, M, 5 * H) or tuple(d_gi.shape) != (Tn, M, 3 * H)
+                or tuple(d_gh.shape) != (Tn, M, 3 * H) or tuple(fresh.shape) != (Tn, M)):
+            raise _lib.KsError("expected dH (T, M, H), saved (T, M, 5H), d_gi, d_gh (T, M, 3H), fresh (T, M)")
+        _lib.check(self._lib.ks_gru_sequence_backward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(dH), _lib.ptr(saved),
+                                                      _lib.ptr(fresh), _lib.ptr(d_gi), _lib.ptr(d_gh), None))
 
     def backward_step(self, dh_out, saved, fresh, d_gi, d_gh, dh_in) -> None:
         """One step of the backward pass through time: dh_out (M, H) -> d_gi, d_gh (M, 3H) and dh_in (M, H)."""
@@ -158,6 +196,7 @@ class LSTMCell:
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_lstm_create(ctypes.byref(d), ctypes.byref(self._handle)))
         self._ws: torch.Tensor | None = None
+        self._proj: MLP | None = None
 
     def workspace(self, M: int, device) -> torch.Tensor:
         need = int(self._lib.ks_lstm_workspace_bytes(self._handle, M))
@@ -212,17 +251,26 @@ class LSTMCell:
         """Whether this cell has the one-launch-per-trajectory kernels (`ks_lstm_sequence_forward / _backward`)."""
         return bool(self._lib.ks_lstm_sequence_supported(self._handle))
 
+    def _input_projection(self) -> MLP:
+        """W_ih x + b of this cell as a network of one layer; there from the start, trained or not."""
+        if self._proj is None:
+            pi, ph = ctypes.c_void_p(), ctypes.c_void_p()
+            _lib.check(self._lib.ks_lstm_projections(self._handle, ctypes.byref(pi), ctypes.byref(ph)))
+            self._proj = MLP._borrow(self._lib, pi, (self.input_size, 4 * self.hidden_size), self.dtype)
+        return self._proj
+
     def sequence_forward(self, x, h0, c0, fresh, hs, cs, saved) -> None:
         """The layer over a whole trajectory: x (T, M, input) -> hs, cs (T, M, H) and `saved` (T, M, 7H), from the carry
-        (h0, c0); the input projection is one product over all T M rows, the recurrence one launch."""
+        (h0, c0); the input projection is one product over all T M rows, the recurrence one launch.  `cs` and `saved` may be
+        None where no backward pass follows."""
         _lib.require_cuda(x, h0, c0, hs, cs, saved, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
         if (tuple(x.shape) != (Tn, M, self.input_size) or any(tuple(t.shape) != (M, H) for t in (h0, c0))
-                or any(tuple(t.shape) != (Tn, M, H) for t in (hs, cs)) or tuple(saved.shape) != (Tn, M, 7 * H)
-                or tuple(fresh.shape) != (Tn, M)):
+                or any(t is not None and tuple(t.shape) != (Tn, M, H) for t in (hs, cs))
+                or (saved is not None and tuple(saved.shape) != (Tn, M, 7 * H)) or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected x (T, M, input), h0, c0 (M, H), hs, cs (T, M, H), saved (T, M, 7H), fresh (T, M)")
-        gi = self.proj_i(x.reshape(Tn * M, self.input_size))
+        gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
         _lib.check(self._lib.ks_lstm_sequence_forward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(gi), _lib.ptr(h0),
                                                       _lib.ptr(c0), _lib.ptr(fresh), _lib.ptr(hs), _lib.ptr(cs), _lib.ptr(saved)))
 
@@ -344,6 +392,8 @@ class RecurrentNetwork:
                 for t in range(T_):
                     h0, c0 = (carry0[i, 0], carry0[i, 1]) if t == 0 else (hs[t - 1], cs[t - 1])
                     cell.train_forward(x[t], h0, c0, fresh[t], hs[t], cs[t], sv[t])
+            elif getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
+                cell.sequence_forward(x, carry0[i], fresh, hs, sv)
             else:
                 for t in range(T_):
                     cell.train_forward(x[t], carry0[i] if t == 0 else hs[t - 1], fresh[t], hs[t], sv[t])
@@ -372,11 +422,14 @@ class RecurrentNetwork:
             cell, sv = self.cells[i], tp["saved"][i]
             d_gi = torch.empty(T_, M, G * H, dtype=torch.float32, device=dev)
             d_gh = d_gi if self.lstm else torch.empty(T_, M, G * H, dtype=torch.float32, device=dev)
-            carry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)   # gradient of the hidden state, ping-pong
-            ccarry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)  # and of the cell state (LSTM)
-            fused = self.lstm and cell.sequence_supported
-            if fused:
+            fused = cell.sequence_supported
+            if fused and self.lstm:
                 cell.sequence_backward(dH, sv, tp["fresh"], d_gi)
+            elif fused:
+                cell.sequence_backward(dH, sv, tp["fresh"], d_gi, d_gh)
+            else:
+                carry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)   # gradient of the hidden state, ping-pong
+                ccarry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)  # and of the cell state (LSTM)
             for t in range(T_ - 1, -1, -1) if not fused else ():
                 dH[t] += carry[t & 1]
                 if self.lstm:

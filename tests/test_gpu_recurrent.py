@@ -318,3 +318,39 @@ def test_lstm_sequence_forward_over_many_rows_equals_the_same_rows_in_small_call
     hs1, cs1, sv1 = z(1, M, H), z(1, M, H), z(1, M, 7 * H)
     cell.sequence_forward(x[:1].contiguous(), h0, c0, fresh[:1].contiguous(), hs1, cs1, sv1)
     assert torch.equal(h, hs1[0]) and torch.equal(c, cs1[0])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("Tn,M", [(1, 1), (7, 45), (3, 2102)])
+def test_gru_sequence_kernels_agree_with_the_step_by_step_entry_points(dtype, Tn, M):
+    """One launch over the trajectory against T calls of the per-step entry points: states and saved activations bit for bit
+    (for such a cell a step is that launch with T = 1), gate gradients against the per-step backward, whose product is a kernel of
+    its own: to fp32 rounding, and for bf16 cells to its rounding of every step's product to bf16 (2^-9 of the largest per step).
+    Rows that do not fill the last 4-row set, and enough of them for several sets per workgroup."""
+    from ksim_amd.recurrent import GRUCell
+
+    rng = np.random.default_rng(59)
+    H = 128
+    cell = GRUCell(*_cell_params(rng, H, H), dtype=dtype)
+    assert cell.sequence_supported
+    cell.train_init()
+    x, h0 = t32(rng.normal(size=(Tn, M, H))), t32(rng.normal(size=(M, H)) * 0.5)
+    fresh = torch.tensor(rng.random((Tn, M)) < 0.1, dtype=torch.uint8, device=DEV)
+    z = lambda *s: torch.zeros(*s, device=DEV)  # noqa: E731
+    hs, sv = z(Tn, M, H), z(Tn, M, 5 * H)
+    cell.sequence_forward(x, h0, fresh, hs, sv)
+    hs1, sv1, h = z(Tn, M, H), z(Tn, M, 5 * H), h0.clone()
+    for t in range(Tn):
+        cell.train_forward(x[t], h0 if t == 0 else hs1[t - 1], fresh[t], hs1[t], sv1[t])
+        cell(x[t], h, fresh[t], out=h)  # the rollout's step: the carry advanced in place
+    assert torch.equal(hs, hs1) and torch.equal(sv, sv1) and torch.equal(h, hs[-1])
+    dH = t32(rng.normal(size=(Tn, M, H)))
+    d_gi, d_gh, d_gi1, d_gh1, carry, dH1 = z(Tn, M, 3 * H), z(Tn, M, 3 * H), z(Tn, M, 3 * H), z(Tn, M, 3 * H), z(2, M, H), dH.clone()
+    cell.sequence_backward(dH, sv, fresh, d_gi, d_gh)
+    for t in range(Tn - 1, -1, -1):
+        dH1[t] += carry[t & 1]
+        cell.backward_step(dH1[t], sv[t], fresh[t], d_gi1[t], d_gh1[t], carry[(t + 1) & 1])
+    tol = 1e-5 if dtype == "f32" else Tn * 2.0 ** -9
+    for got, want in ((d_gi, d_gi1), (d_gh, d_gh1)):
+        assert (got - want).abs().max().item() <= tol * want.abs().max().item()
+    assert not GRUCell(*_cell_params(rng, 24, 24), dtype=dtype).sequence_supported
