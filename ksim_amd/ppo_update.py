@@ -442,12 +442,8 @@ def recurrent_on_policy(policy: RecurrentHeadPolicy, actor_obs, critic_obs, acti
     update_model makes once over the whole rollout before any minibatch step (ppo.py:603-607).  With `return_raw` also the
     head's input rows (T, N, width), locations filtered where the policy filters them."""
     Tn, N, nu = action.shape
-    a_carry, c_carry = actor_carry0.clone(), critic_carry0.clone()
-    raw = torch.empty(Tn, N, policy.width(nu), dtype=torch.float32, device=action.device)
-    values = torch.empty(Tn, N, 1, dtype=torch.float32, device=action.device)
-    for t in range(Tn):
-        policy.actor(actor_obs[t], a_carry, fresh=fresh[t], out=raw[t])
-        policy.critic(critic_obs[t], c_carry, fresh=fresh[t], out=values[t])
+    raw = policy.actor.forward_sequence(actor_obs, actor_carry0, fresh)
+    values = policy.critic.forward_sequence(critic_obs, critic_carry0, fresh)
     if policy.lowpass is not None:
         raw = actor_locations(policy, raw, actor_obs.contiguous(), fresh.contiguous(), lpf0)
     lp = torch.empty(Tn, N, nu, dtype=torch.float32, device=action.device)

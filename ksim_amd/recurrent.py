@@ -359,6 +359,30 @@ class RecurrentNetwork:
                 x = cell(x, carry[i], fresh, out=carry[i])
         return self.output_proj(x, out=out)
 
+    def forward_sequence(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor) -> torch.Tensor:
+        """The network over a trajectory without keeping anything for a backward pass: obs (T, M, in), carry0 the carry of the
+        first step (left as it is), fresh (T, M) uint8 -> (T, M, out).  The same numbers as T calls, one control step each."""
+        T_, M, H = obs.shape[0], obs.shape[1], self.hidden_size
+        want = (self.depth, 2, M, H) if self.lstm else (self.depth, M, H)
+        if tuple(obs.shape) != (T_, M, self.in_dim) or tuple(carry0.shape) != want or tuple(fresh.shape) != (T_, M):
+            raise _lib.KsError(f"expected obs (T, M, in), carry0 {want}, fresh (T, M)")
+        if not all(c.sequence_supported for c in self.cells):
+            carry = carry0.clone()
+            out = torch.empty(T_, M, self.out_dim, dtype=torch.float32, device=obs.device)
+            for t in range(T_):
+                self(obs[t], carry, fresh=fresh[t], out=out[t])
+            return out
+        x = self.input_proj(obs.contiguous().view(T_ * M, self.in_dim)).view(T_, M, H)
+        fresh = fresh.contiguous()
+        for i, cell in enumerate(self.cells):
+            hs = torch.empty(T_, M, H, dtype=torch.float32, device=obs.device)
+            if self.lstm:
+                cell.sequence_forward(x, carry0[i, 0], carry0[i, 1], fresh, hs, None, None)
+            else:
+                cell.sequence_forward(x, carry0[i], fresh, hs, None)
+            x = hs
+        return self.output_proj(x.view(T_ * M, H)).view(T_, M, self.out_dim)
+
     # ------------------------------------------------------------------ training: backward pass through time
     def train_init(self) -> None:
         self.input_proj.train_init()
