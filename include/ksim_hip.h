@@ -69,6 +69,12 @@ int ks_gae_tn(ks_stream_t stream, int64_t T, int64_t N, const float* values, con
 #define KS_REDUCE_WORKSPACE_BYTES (2 * 1024 * 8 + 64)
 int ks_normalize_advantages(ks_stream_t stream, int64_t n, const float* gae, float* advantages,
                             void* workspace);
+/* Both in two launches (the recursion leaves the moments of its advantages behind): compute_ppo_inputs with normalize_advantages,
+ * ksim/task/ppo.py:54-121.  time_major: (T, N) arrays, n0 = T, n1 = N; else (B, T), n0 = B, n1 = T.  gae and advantages are required,
+ * returns and targets may be NULL. */
+int ks_gae_normalized(ks_stream_t stream, int time_major, int64_t n0, int64_t n1, const float* values, const float* rewards,
+                      const uint8_t* dones, const uint8_t* successes, float gamma, float lam, int monte_carlo_returns,
+                      float* gae, float* returns, float* targets, float* advantages, void* workspace);
 /* The same result with no workspace argument and no allocation of any kind.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The block partials live in a device array of KS_REDUCE_WORKSPACE_BYTES bytes inside the library, one copy

@@ -9,6 +9,8 @@ import ctypes
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int8, c_int32, c_int64, c_uint8, c_void_p
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libksimhip.so")
 
@@ -52,6 +54,8 @@ def load() -> ctypes.CDLL:
     p = c_void_p
     lib.ks_gae_bt.argtypes = [p, c_int64, c_int64, p, p, p, p, c_float, c_float, c_int32, p, p, p]
     lib.ks_gae_tn.argtypes = lib.ks_gae_bt.argtypes
+    lib.ks_gae_normalized.argtypes = [p, c_int32, c_int64, c_int64, p, p, p, p, c_float, c_float, c_int32] + [p] * 5
+    lib.ks_gae_normalized.restype = c_int32
     lib.ks_normalize_advantages.argtypes = [p, c_int64, p, p, p]
     lib.ks_normalize_advantages_static.argtypes = [p, c_int64, p, p]
     lib.ks_normalize_advantages_static.restype = c_int32
@@ -99,15 +103,18 @@ def ptr(t) -> c_void_p:
     return c_void_p(t.data_ptr())
 
 
-def current_stream() -> c_void_p:
-    import torch
+def addr(t) -> int | None:
+    """Device address of a torch tensor as a plain number (None stays None): what a pointer argument of the library takes as it is,
+    without a ctypes object per operand."""
+    return None if t is None else t.data_ptr()
 
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+
+def current_stream() -> int:
+    """The current stream's handle, straight from torch's C layer: no stream object per call."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def require_cuda(*tensors, dtype=None):
-    import torch
-
     for t in tensors:
         if t is None:
             continue

@@ -10,6 +10,43 @@ static thread_local char g_err[256] = "";
 char* err_buf() { return g_err; }
 
 // ---------------------------------------------------------------------------------------------
+// Deterministic two-stage reductions (no atomics): stage 1 writes one partial per block,
+// stage 2 re-reads the <= 1024 partials in a fixed order.
+// ---------------------------------------------------------------------------------------------
+constexpr int kMaxPartials = 1024;
+
+__device__ inline double wave_sum(double x) {
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) x += __shfl_down(x, s);
+  return x;
+}
+
+// Sum over a 256-thread block; result valid in thread 0.
+__device__ inline double block_sum(double x, double* lds4) {
+  x = wave_sum(x);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return lds4[0] + lds4[1] + lds4[2] + lds4[3];
+}
+
+// Sum and sum of squares over a block of WAVES wavefronts into partial[block] and partial[kMaxPartials + block].
+template <int WAVES>
+__device__ inline void block_moments(double s, double ss, double* __restrict__ partial) {
+  __shared__ double lds[2][WAVES];
+  s = wave_sum(s);
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) { lds[0][threadIdx.x >> 6] = s; lds[1][threadIdx.x >> 6] = ss; }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+    for (int w = 0; w < WAVES; ++w) t += lds[threadIdx.x][w];
+    partial[threadIdx.x * kMaxPartials + blockIdx.x] = t;
+  }
+}
+
+
+// ---------------------------------------------------------------------------------------------
 // GAE, (B, T) layout.  One wavefront per env row.  The recurrences R_t = r'_t + g m_t R_{t+1} and
 // A_t = d_t + g l m_t A_{t+1} (ksim/task/ppo.py:66-75) are compositions of affine maps x -> d + c x, which are
 // associative.  Lanes hold time in DESCENDING order (lane i of a 64-step chunk holds t = chunk_end - i), so the
@@ -32,13 +69,15 @@ __device__ __forceinline__ void scan_step(float& c, float& d) {
   c = c * pc;
 }
 
-__device__ __forceinline__ void affine_scan64(float& c, float& d) {
+// over groups of N lanes: the steps that would cross a group's boundary are left out
+template <int N>
+__device__ __forceinline__ void affine_scan(float& c, float& d) {
   scan_step<0x111, 0xf>(c, d);  // row_shr:1
   scan_step<0x112, 0xf>(c, d);  // row_shr:2
   scan_step<0x114, 0xf>(c, d);  // row_shr:4
   scan_step<0x118, 0xf>(c, d);  // row_shr:8
-  scan_step<0x142, 0xa>(c, d);  // row_bcast:15 -> rows 1 and 3
-  scan_step<0x143, 0xc>(c, d);  // row_bcast:31 -> rows 2 and 3
+  if (N >= 32) scan_step<0x142, 0xa>(c, d);  // row_bcast:15 -> rows 1 and 3
+  if (N >= 64) scan_step<0x143, 0xc>(c, d);  // row_bcast:31 -> rows 2 and 3
 }
 
 __device__ __forceinline__ float lane63(float x) {
@@ -47,61 +86,77 @@ __device__ __forceinline__ float lane63(float x) {
 
 constexpr int kGaeMaxChunks = 4;  // rows of up to 256 steps keep every load in flight at once
 
-__global__ __launch_bounds__(256) void gae_bt_kernel(
+// MOMENTS: the block also leaves the sum and the sum of squares of its advantages in `partial` (the first half of their
+// normalisation, which would otherwise read them again in a launch of its own); then a block of 8 wavefronts walks several rows,
+// so that at most kMaxPartials blocks cover the batch.
+// LPR: lanes per row.  Rows of up to 32 (16) steps share a wavefront two (four) at a time: a trajectory of 24 or 32 steps would leave
+// half of the lanes and of the loads in flight unused (16384 x 32 with moments: 13.0 -> 6.9 us).
+template <bool MOMENTS, int LPR>
+__global__ __launch_bounds__(MOMENTS ? 512 : 256) void gae_bt_kernel(
     int64_t B, int64_t T, const float* __restrict__ values, const float* __restrict__ rewards,
     const uint8_t* __restrict__ dones, const uint8_t* __restrict__ successes, float gamma, float lam,
-    int mc, float* __restrict__ gae, float* __restrict__ returns, float* __restrict__ targets) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (row >= B) return;  // whole wavefront leaves together
-  const int64_t base = row * T;
-  const float v_last = values[base + T - 1];  // bootstrap = last value repeated, ppo.py:79
-  const float gl = gamma * lam;
-  const float omg = 1.0f - gamma;
-  float carry_r = 0.f, carry_a = 0.f, v_after = v_last;  // v_after: value at the first step after the chunk
-  const int64_t nchunk = (T + 63) >> 6;
-  for (int64_t c0 = nchunk - 1; c0 >= 0; c0 -= kGaeMaxChunks) {
-    // issue the loads of up to kGaeMaxChunks chunks before any of them is scanned
-    float v[kGaeMaxChunks], r[kGaeMaxChunks];
-    uint8_t dn[kGaeMaxChunks], sc[kGaeMaxChunks];
+    int mc, float* __restrict__ gae, float* __restrict__ returns, float* __restrict__ targets, double* __restrict__ partial) {
+  constexpr int RPW = 64 / LPR, CH = LPR == 64 ? kGaeMaxChunks : 1;
+  const int lane = threadIdx.x & (LPR - 1);
+  double msum = 0.0, msq = 0.0;
+  const int64_t rows_per_pass = (int64_t)(blockDim.x >> 6) * RPW;
+  for (int64_t r0 = (int64_t)blockIdx.x * rows_per_pass + (threadIdx.x >> 6) * RPW; r0 < B; r0 += (int64_t)gridDim.x * rows_per_pass) {
+    const int64_t row = r0 + (threadIdx.x & 63) / LPR;
+    const bool row_ok = RPW == 1 || row < B;
+    const int64_t base = (row_ok ? row : B - 1) * T;
+    const float v_last = values[base + T - 1];  // bootstrap = last value repeated, ppo.py:79
+    const float gl = gamma * lam;
+    const float omg = 1.0f - gamma;
+    float carry_r = 0.f, carry_a = 0.f, v_after = v_last;  // v_after: value at the first step after the chunk
+    const int64_t nchunk = LPR == 64 ? (T + 63) >> 6 : 1;
+    for (int64_t c0 = nchunk - 1; c0 >= 0; c0 -= CH) {
+      // issue the loads of up to CH chunks before any of them is scanned
+      float v[CH], r[CH];
+      uint8_t dn[CH], sc[CH];
 #pragma unroll
-    for (int k = 0; k < kGaeMaxChunks; ++k) {
-      const int64_t c = c0 - k;
-      const int64_t t = (c << 6) + 63 - lane;  // descending time across lanes
-      const bool valid = c >= 0 && t < T;
-      v[k] = valid ? values[base + t] : 0.f;
-      r[k] = valid ? rewards[base + t] : 0.f;
-      dn[k] = valid ? dones[base + t] : (uint8_t)0;
-      sc[k] = (valid && successes) ? successes[base + t] : (uint8_t)0;
-    }
-#pragma unroll
-    for (int k = 0; k < kGaeMaxChunks; ++k) {
-      const int64_t c = c0 - k;
-      if (c < 0) break;
-      const int64_t t = (c << 6) + 63 - lane;
-      const bool valid = t < T;
-      // V(s_{t+1}) sits one lane down; lane 0 takes the first value after the chunk (wave_shr:1 keeps `old` there)
-      float v_up = dpp_take<0x138, 0xf>(v_after, v[k]);
-      if (t + 1 >= T) v_up = v_last;
-      const float mask = dn[k] ? 0.f : 1.f;
-      const float rb = omg * r[k] + gamma * v[k] * (sc[k] ? 1.f : 0.f);  // ppo.py:82-83
-      const float delta = rb + gamma * v_up * mask - v[k];                // ppo.py:86
-      float c_r = valid ? gamma * mask : 1.f, d_r = valid ? rb : 0.f;
-      float c_a = valid ? gl * mask : 1.f, d_a = valid ? delta : 0.f;
-      affine_scan64(c_r, d_r);
-      affine_scan64(c_a, d_a);
-      const float R = d_r + c_r * carry_r;
-      const float A = d_a + c_a * carry_a;
-      if (valid) {
-        if (gae) gae[base + t] = A;
-        if (returns) returns[base + t] = R;
-        if (targets) targets[base + t] = mc ? R : A + v[k];  // ppo.py:107
+      for (int k = 0; k < CH; ++k) {
+        const int64_t c = c0 - k;
+        const int64_t t = c * LPR + LPR - 1 - lane;  // descending time across lanes
+        const bool valid = c >= 0 && t < T && row_ok;
+        v[k] = valid ? values[base + t] : 0.f;
+        r[k] = valid ? rewards[base + t] : 0.f;
+        dn[k] = valid ? dones[base + t] : (uint8_t)0;
+        sc[k] = (valid && successes) ? successes[base + t] : (uint8_t)0;
       }
-      carry_r = lane63(R);
-      carry_a = lane63(A);
-      v_after = lane63(v[k]);
+#pragma unroll
+      for (int k = 0; k < CH; ++k) {
+        const int64_t c = c0 - k;
+        if (c < 0) break;
+        const int64_t t = c * LPR + LPR - 1 - lane;
+        const bool valid = t < T && row_ok;
+        // V(s_{t+1}) sits one lane down; lane 0 takes the first value after the chunk (wave_shr:1 keeps `old` there), and a row's
+        // last step, which is the first of its lanes in use, takes the bootstrap
+        float v_up = dpp_take<0x138, 0xf>(v_after, v[k]);
+        if (t + 1 >= T) v_up = v_last;
+        const float mask = dn[k] ? 0.f : 1.f;
+        const float rb = omg * r[k] + gamma * v[k] * (sc[k] ? 1.f : 0.f);  // ppo.py:82-83
+        const float delta = rb + gamma * v_up * mask - v[k];                // ppo.py:86
+        float c_r = valid ? gamma * mask : 1.f, d_r = valid ? rb : 0.f;
+        float c_a = valid ? gl * mask : 1.f, d_a = valid ? delta : 0.f;
+        affine_scan<LPR>(c_r, d_r);
+        affine_scan<LPR>(c_a, d_a);
+        const float R = d_r + c_r * carry_r;
+        const float A = d_a + c_a * carry_a;
+        if (valid) {
+          if (gae) gae[base + t] = A;
+          if (returns) returns[base + t] = R;
+          if (targets) targets[base + t] = mc ? R : A + v[k];  // ppo.py:107
+          if (MOMENTS) { msum += (double)A; msq += (double)A * (double)A; }
+        }
+        if (LPR == 64) {
+          carry_r = lane63(R);
+          carry_a = lane63(A);
+          v_after = lane63(v[k]);
+        }
+      }
     }
   }
+  if constexpr (MOMENTS) block_moments<8>(msum, msq, partial);
 }
 
 // GAE, (T, N) layout.  A workgroup owns 32 consecutive envs and walks back in time in chunks of 32 steps: all 256
@@ -110,17 +165,20 @@ __global__ __launch_bounds__(256) void gae_bt_kernel(
 // back.  With one lane per env doing its own loads, 8192 envs would be 128 wavefronts with one dependent stream of
 // loads each; here every CU has eight times as many loads in flight and N / 32 workgroups spread over the chip.
 constexpr int kTnEnvs = 32, kTnSteps = 32;
+template <bool MOMENTS>  // as in gae_bt_kernel
 __global__ __launch_bounds__(256) void gae_tn_kernel(
     int64_t T, int64_t N, const float* __restrict__ values, const float* __restrict__ rewards,
     const uint8_t* __restrict__ dones, const uint8_t* __restrict__ successes, float gamma, float lam,
-    int mc, float* __restrict__ gae, float* __restrict__ returns, float* __restrict__ targets) {
+    int mc, float* __restrict__ gae, float* __restrict__ returns, float* __restrict__ targets, int64_t tiles, double* __restrict__ partial) {
   __shared__ float sv[kTnSteps][kTnEnvs], sr[kTnSteps][kTnEnvs], oa[kTnSteps][kTnEnvs], orr[kTnSteps][kTnEnvs];
   __shared__ uint8_t sd[kTnSteps][kTnEnvs], ss[kTnSteps][kTnEnvs];
   const int tx = threadIdx.x & (kTnEnvs - 1), ty = threadIdx.x / kTnEnvs;
   // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Four neighbouring tiles share every 128-byte
   // line of the byte arrays, so neighbouring tiles go to one XCD: workgroup b takes tile (b % 8) * (grid / 8) + b / 8.
-  int64_t tile = blockIdx.x;
-  if (gridDim.x % 8 == 0) tile = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  double msum = 0.0, msq = 0.0;
+  for (int64_t b = blockIdx.x; b < tiles; b += gridDim.x) {
+  int64_t tile = b;
+  if (tiles % 8 == 0) tile = (b % 8) * (tiles / 8) + b / 8;
   const int64_t e = tile * kTnEnvs + tx;
   const bool in = e < N;
   const float gl = gamma * lam, omg = 1.0f - gamma;
@@ -159,30 +217,12 @@ __global__ __launch_bounds__(256) void gae_tn_kernel(
         if (gae) gae[i] = a;
         if (returns) returns[i] = rr;
         if (targets) targets[i] = mc ? rr : a + sv[k][tx];
+        if (MOMENTS) { msum += (double)a; msq += (double)a * (double)a; }
       }
     __syncthreads();
   }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Deterministic two-stage reductions (no atomics): stage 1 writes one partial per block,
-// stage 2 re-reads the <= 1024 partials in a fixed order.
-// ---------------------------------------------------------------------------------------------
-constexpr int kMaxPartials = 1024;
-
-__device__ inline double wave_sum(double x) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) x += __shfl_down(x, s);
-  return x;
-}
-
-// Sum over a 256-thread block; result valid in thread 0.
-__device__ inline double block_sum(double x, double* lds4) {
-  x = wave_sum(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = x;
-  __syncthreads();
-  return lds4[0] + lds4[1] + lds4[2] + lds4[3];
+  }
+  if constexpr (MOMENTS) block_moments<4>(msum, msq, partial);
 }
 
 __global__ __launch_bounds__(256) void moments_kernel(int64_t n, const float* __restrict__ x,
@@ -225,61 +265,129 @@ __global__ __launch_bounds__(256) void normalize_kernel(int64_t n, int nparts, c
   }
   __syncthreads();
   const float mean = s_mean, inv = s_inv;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = (x[i] - mean) * inv;
+  const int64_t n4 = (((uintptr_t)x | (uintptr_t)out) & 15) == 0 ? n / 4 : 0;  // whole 16-byte groups; the rest one by one
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < n4; i += step) {
+    float4 v = reinterpret_cast<const float4*>(x)[i];
+    v.x = (v.x - mean) * inv; v.y = (v.y - mean) * inv; v.z = (v.z - mean) * inv; v.w = (v.w - mean) * inv;
+    reinterpret_cast<float4*>(out)[i] = v;
+  }
+  for (int64_t i = 4 * n4 + i0; i < n; i += step) out[i] = (x[i] - mean) * inv;
 }
 
 // the adaptive-KL factor: a device scalar when the caller keeps it there, otherwise the host's number
 __device__ __forceinline__ float kl_scale_of(const KsPpoLossParams& p) { return p.kl_scale_device ? *p.kl_scale_device : p.kl_scale; }
 
 // ---------------------------------------------------------------------------------------------
-// PPO loss (ppo.py:207-246).  One lane per (b, t) element; the A log-probs of an element are
-// contiguous, so a wavefront touches one contiguous 64*A*4-byte span per array.
+// PPO loss (ppo.py:207-246), one lane per (b, t) element.
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void ppo_loss_kernel(
-    int64_t n, int A, KsPpoLossParams p, const float* __restrict__ adv, const float* __restrict__ tgt,
-    const float* __restrict__ lp_on, const float* __restrict__ v_on, const float* __restrict__ lp_off,
-    const float* __restrict__ v_off, const float* __restrict__ ent, float* __restrict__ o_policy,
-    float* __restrict__ o_value, float* __restrict__ o_kl, float* __restrict__ o_ent,
-    double* __restrict__ partial) {
+struct PpoLossIO {
+  const float *adv, *tgt, *lp_on, *v_on, *lp_off, *v_off, *ent;
+  float *policy, *value, *kl, *entropy;
+};
+
+// The four terms of element i from its log ratio and entropy sum; returns their sum.
+__device__ __forceinline__ float ppo_loss_terms(const PpoLossIO& io, const KsPpoLossParams& p, float kl_scale, int64_t i, float log_ratio,
+                                                float es) {
+  const float lr = fminf(fmaxf(log_ratio, -p.log_clip_value), p.log_clip_value);
+  const float ratio = expf(lr);
+  const float cr = fminf(fmaxf(ratio, 1.f - p.clip_param), 1.f + p.clip_param);
+  const float ad = io.adv[i];
+  const float policy = -fminf(ratio * ad, cr * ad);
+  const float von = io.v_on[i], voff = io.v_off[i], tg = io.tgt[i];
+  float vobj;
+  if (p.use_clipped_value_loss) {
+    const float vc = von + fminf(fmaxf(voff - von, -p.clip_param), p.clip_param);
+    const float ce = vc - tg, er = voff - tg;
+    vobj = 0.5f * fmaxf(er * er, ce * ce);
+  } else {
+    const float er = tg - voff;
+    vobj = 0.5f * er * er;
+  }
+  const float value = vobj * p.value_loss_coef;
+  const float klv = -log_ratio * p.kl_coef * kl_scale;  // the sum of on - off is the log ratio negated, to the bit
+  const float entv = io.ent ? -es * p.entropy_coef : 0.f;
+  if (io.policy) io.policy[i] = policy;
+  if (io.value) io.value[i] = value;
+  if (io.kl) io.kl[i] = klv;
+  if (io.entropy && io.ent) io.entropy[i] = entv;
+  return policy + value + klv + entv;
+}
+
+// Elements whose A actions a lane can read where they lie: A = 1, and the widths whose rows are too long to stage.
+__global__ __launch_bounds__(256) void ppo_loss_kernel(int64_t n, int A, KsPpoLossParams p, PpoLossIO io, double* __restrict__ partial) {
   __shared__ double lds[4];
   double acc = 0.0;
+  const float kl_scale = kl_scale_of(p);
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    float log_ratio = 0.f, kl = 0.f, es = 0.f;
-    const float* a_on = lp_on + i * A;
-    const float* a_off = lp_off + i * A;
-    for (int a = 0; a < A; ++a) {
-      const float on = a_on[a], off = a_off[a];
-      log_ratio += off - on;
-      kl += on - off;
-    }
-    if (ent) {
-      const float* e = ent + i * A;
+    float log_ratio = 0.f, es = 0.f;
+    const float* a_on = io.lp_on + i * A;
+    const float* a_off = io.lp_off + i * A;
+    for (int a = 0; a < A; ++a) log_ratio += a_off[a] - a_on[a];
+    if (io.ent) {
+      const float* e = io.ent + i * A;
       for (int a = 0; a < A; ++a) es += e[a];
     }
-    const float lr = fminf(fmaxf(log_ratio, -p.log_clip_value), p.log_clip_value);
-    const float ratio = expf(lr);
-    const float cr = fminf(fmaxf(ratio, 1.f - p.clip_param), 1.f + p.clip_param);
-    const float ad = adv[i];
-    const float policy = -fminf(ratio * ad, cr * ad);
-    const float von = v_on[i], voff = v_off[i], tg = tgt[i];
-    float vobj;
-    if (p.use_clipped_value_loss) {
-      const float vc = von + fminf(fmaxf(voff - von, -p.clip_param), p.clip_param);
-      const float ce = vc - tg, er = voff - tg;
-      vobj = 0.5f * fmaxf(er * er, ce * ce);
+    acc += (double)ppo_loss_terms(io, p, kl_scale, i, log_ratio, es);
+  }
+  acc = block_sum(acc, lds);
+  if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+}
+
+// The A log-probabilities of an element are contiguous: lanes that walk an element each touch 64 lines per load and miss the
+// vector L1 on most of them (16384 x 32 elements, A = 20: 137 us, 1.0 TB/s).  Here a wavefront copies the contiguous 64 A floats of
+// its 64 elements with one 16-byte load per lane and array at a time, all of them in flight, leaves off - on and the entropies in
+// LDS with an odd row stride, and sums every element's row in order from there: bound by the bytes (31 us at that size).
+constexpr int kLossMaxA = 31;  // four wavefronts' tiles within 64 KB of LDS
+
+__global__ __launch_bounds__(256) void ppo_loss_rows_kernel(int64_t n, int A, int wave_floats, KsPpoLossParams p, PpoLossIO io,
+                                                            double* __restrict__ partial) {
+  extern __shared__ float loss_lds[];
+  __shared__ double lds[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int LD = A | 1;
+  float* sd = loss_lds + wave * wave_floats;
+  float* se = sd + 64 * LD;
+  const float kl_scale = kl_scale_of(p);
+  const unsigned inv_a = 0xffffffffu / (unsigned)A + 1u;  // x / A = mulhi(x, inv_a) for x < 64 * 32 < 2^16
+  double acc = 0.0;
+  const int64_t tiles = (n + 63) / 64;
+  for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < tiles; tile += (int64_t)gridDim.x * 4) {
+    const int64_t i0 = tile * 64;
+    const int rows = (int)(n - i0 < 64 ? n - i0 : 64);
+    const int cnt = rows * A;  // i0 * A is a multiple of 64: the span starts on a 16-byte boundary of its array
+    const float* on = io.lp_on + i0 * A;
+    const float* off = io.lp_off + i0 * A;
+    const float* en = io.ent ? io.ent + i0 * A : nullptr;
+    auto put = [&](float* dst, int x, float v) {
+      const int r = (int)__umulhi((unsigned)x, inv_a);
+      dst[r * LD + (x - r * A)] = v;
+    };
+    if (rows == 64) {
+#pragma unroll 2
+      for (int x = 4 * lane; x < cnt; x += 256) {
+        const float4 f = *reinterpret_cast<const float4*>(off + x), g = *reinterpret_cast<const float4*>(on + x);
+        float4 h = {0.f, 0.f, 0.f, 0.f};
+        if (en) h = *reinterpret_cast<const float4*>(en + x);
+        put(sd, x, f.x - g.x); put(sd, x + 1, f.y - g.y); put(sd, x + 2, f.z - g.z); put(sd, x + 3, f.w - g.w);
+        if (en) { put(se, x, h.x); put(se, x + 1, h.y); put(se, x + 2, h.z); put(se, x + 3, h.w); }
+      }
     } else {
-      const float er = tg - voff;
-      vobj = 0.5f * er * er;
+      for (int x = lane; x < cnt; x += 64) {
+        put(sd, x, off[x] - on[x]);
+        if (en) put(se, x, en[x]);
+      }
     }
-    const float value = vobj * p.value_loss_coef;
-    const float klv = kl * p.kl_coef * kl_scale_of(p);
-    const float entv = ent ? -es * p.entropy_coef : 0.f;
-    if (o_policy) o_policy[i] = policy;
-    if (o_value) o_value[i] = value;
-    if (o_kl) o_kl[i] = klv;
-    if (o_ent && ent) o_ent[i] = entv;
-    acc += (double)(policy + value + klv + entv);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wavefront's own LDS tile: no other wavefront touches it
+    __builtin_amdgcn_wave_barrier();
+    if (lane < rows) {
+      float log_ratio = 0.f, es = 0.f;
+      for (int a = 0; a < A; ++a) log_ratio += sd[lane * LD + a];
+      if (en) for (int a = 0; a < A; ++a) es += se[lane * LD + a];
+      acc += (double)ppo_loss_terms(io, p, kl_scale, i0 + lane, log_ratio, es);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
   acc = block_sum(acc, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = acc;
@@ -387,11 +495,12 @@ extern "C" int ks_gae_bt(ks_stream_t stream, int64_t B, int64_t T, const float* 
                          int monte_carlo_returns, float* gae, float* returns, float* targets) {
   if (int rc = check_gae_args(B, T, values, rewards, dones)) return rc;
   if (B == 0 || T == 0) return KS_OK;
-  const int rows_per_block = 4;
+  const int rows_per_block = 4 * (T <= 16 ? 4 : (T <= 32 ? 2 : 1));
   const int64_t grid = (B + rows_per_block - 1) / rows_per_block;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_gae_bt: B too large");
-  hipLaunchKernelGGL(gae_bt_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, B, T, values, rewards,
-                     dones, successes, gamma, lam, monte_carlo_returns, gae, returns, targets);
+  auto kfn = T <= 16 ? gae_bt_kernel<false, 16> : (T <= 32 ? gae_bt_kernel<false, 32> : gae_bt_kernel<false, 64>);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, B, T, values, rewards,
+                     dones, successes, gamma, lam, monte_carlo_returns, gae, returns, targets, nullptr);
   return check_launch("ks_gae_bt");
 }
 
@@ -402,9 +511,33 @@ extern "C" int ks_gae_tn(ks_stream_t stream, int64_t T, int64_t N, const float* 
   if (N == 0 || T == 0) return KS_OK;
   const int64_t grid = (N + kTnEnvs - 1) / kTnEnvs;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_gae_tn: N too large");
-  hipLaunchKernelGGL(gae_tn_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, T, N, values, rewards,
-                     dones, successes, gamma, lam, monte_carlo_returns, gae, returns, targets);
+  hipLaunchKernelGGL(gae_tn_kernel<false>, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, T, N, values, rewards,
+                     dones, successes, gamma, lam, monte_carlo_returns, gae, returns, targets, grid, nullptr);
   return check_launch("ks_gae_tn");
+}
+
+extern "C" int ks_gae_normalized(ks_stream_t stream, int time_major, int64_t n0, int64_t n1, const float* values, const float* rewards,
+                                 const uint8_t* dones, const uint8_t* successes, float gamma, float lam, int monte_carlo_returns,
+                                 float* gae, float* returns, float* targets, float* advantages, void* workspace) {
+  if (int rc = check_gae_args(n0, n1, values, rewards, dones)) return rc;
+  if (n0 == 0 || n1 == 0) return KS_OK;
+  if (!gae || !advantages || !workspace) return fail(KS_EINVAL, "ks_gae_normalized: null pointer");
+  const int64_t n = n0 * n1;
+  double* partial = (double*)workspace;
+  int g;
+  if (time_major) {
+    const int64_t tiles = (n1 + kTnEnvs - 1) / kTnEnvs;
+    g = (int)(tiles < kMaxPartials ? tiles : kMaxPartials);
+    hipLaunchKernelGGL(gae_tn_kernel<true>, dim3(g), dim3(256), 0, (hipStream_t)stream, n0, n1, values, rewards, dones, successes, gamma, lam,
+                       monte_carlo_returns, gae, returns, targets, tiles, partial);
+  } else {
+    g = grid_for(n0, 8 * (n1 <= 16 ? 4 : (n1 <= 32 ? 2 : 1)), kMaxPartials);
+    auto kfn = n1 <= 16 ? gae_bt_kernel<true, 16> : (n1 <= 32 ? gae_bt_kernel<true, 32> : gae_bt_kernel<true, 64>);
+    hipLaunchKernelGGL(kfn, dim3(g), dim3(512), 0, (hipStream_t)stream, n0, n1, values, rewards, dones, successes, gamma, lam,
+                       monte_carlo_returns, gae, returns, targets, partial);
+  }
+  hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 1024, 1024)), dim3(256), 0, (hipStream_t)stream, n, g, gae, partial, advantages);
+  return check_launch("ks_gae_normalized");
 }
 
 extern "C" int ks_normalize_advantages(ks_stream_t stream, int64_t n, const float* gae, float* advantages,
@@ -415,7 +548,7 @@ extern "C" int ks_normalize_advantages(ks_stream_t stream, int64_t n, const floa
   const int g = grid_for(n, 256 * 4, kMaxPartials);
   double* partial = (double*)workspace;
   hipLaunchKernelGGL(moments_kernel, dim3(g), dim3(256), 0, (hipStream_t)stream, n, gae, partial);
-  hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 256, 4096)), dim3(256), 0, (hipStream_t)stream, n, g, gae,
+  hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 1024, 1024)), dim3(256), 0, (hipStream_t)stream, n, g, gae,
                      partial, advantages);
   return check_launch("ks_normalize_advantages");
 }
@@ -463,7 +596,7 @@ extern "C" int ks_normalize_advantages_static(ks_stream_t stream, int64_t n, con
   // every partial that stage 2 reads is written by stage 1 of the same call, so nothing has to be cleared
   const int g = grid_for(n, 256 * 4, kMaxPartials);
   hipLaunchKernelGGL(moments_kernel, dim3(g), dim3(256), 0, (hipStream_t)stream, n, gae, partial);
-  hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 256, 4096)), dim3(256), 0, (hipStream_t)stream, n, g, gae,
+  hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 1024, 1024)), dim3(256), 0, (hipStream_t)stream, n, g, gae,
                      partial, advantages);
   return check_launch("ks_normalize_advantages_static");
 }
@@ -480,9 +613,16 @@ extern "C" int ks_ppo_loss(ks_stream_t stream, int64_t n, int32_t A, const KsPpo
     return fail(KS_EINVAL, "ks_ppo_loss: null pointer");
   const int g = grid_for(n, 256, kMaxPartials);
   double* partial = (double*)workspace;
-  hipLaunchKernelGGL(ppo_loss_kernel, dim3(g), dim3(256), 0, (hipStream_t)stream, n, (int)A, *params, advantages,
-                     value_targets, on_log_probs, on_values, off_log_probs, off_values, off_entropy, policy_loss,
-                     value_loss, kl_loss, entropy_loss, partial);
+  const PpoLossIO io = {advantages, value_targets, on_log_probs, on_values, off_log_probs, off_values, off_entropy,
+                        policy_loss, value_loss, kl_loss, entropy_loss};
+  const bool aligned = (((uintptr_t)on_log_probs | (uintptr_t)off_log_probs | (uintptr_t)off_entropy) & 15) == 0;
+  if (A > 1 && A <= kLossMaxA && aligned) {
+    const int wave_floats = 64 * (A | 1) * (off_entropy ? 2 : 1);
+    hipLaunchKernelGGL(ppo_loss_rows_kernel, dim3(g), dim3(256), 4 * wave_floats * (int)sizeof(float), (hipStream_t)stream, n, (int)A, wave_floats,
+                       *params, io, partial);
+  } else {
+    hipLaunchKernelGGL(ppo_loss_kernel, dim3(g), dim3(256), 0, (hipStream_t)stream, n, (int)A, *params, io, partial);
+  }
   if (loss_out)
     hipLaunchKernelGGL(mean_finish_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, g, n, partial, loss_out);
   return check_launch("ks_ppo_loss");
@@ -536,71 +676,94 @@ __global__ __launch_bounds__(256) void gaussian_log_prob_kernel(int64_t n, int n
   if (ent) ent[idx] = 0.5f + kHalfLog2Pi + ls;
 }
 
-// One thread per row m; every workgroup also accumulates the log-std gradient of its rows, reduced in a fixed
-// order (block partials, then ppo_grad_finish_kernel), so the result does not depend on scheduling.
-__global__ __launch_bounds__(256) void ppo_loss_grad_kernel(int64_t M, int nu, KsPpoLossParams p, const float* __restrict__ mean,
-                                                           const float* __restrict__ log_std, const float* __restrict__ action,
-                                                           const float* __restrict__ on_lp, const float* __restrict__ adv,
-                                                           const float* __restrict__ tgt, const float* __restrict__ on_v,
-                                                           const float* __restrict__ v, float* __restrict__ d_mean,
-                                                           float* __restrict__ d_value, float* __restrict__ partial) {
-  __shared__ float red[256];
-  float dls[KS_MAX_ACTIONS];
-#pragma unroll
-  for (int a = 0; a < KS_MAX_ACTIONS; ++a) dls[a] = 0.f;
-  const float inv_m = 1.0f / (float)M;
-  for (int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x; m < M; m += (int64_t)gridDim.x * 256) {
-    // new log-probabilities and the log ratio
-    float logr = 0.f;
-    for (int a = 0; a < nu; ++a) {
-      const float ls = log_std[a];
-      const float z = (action[m * nu + a] - mean[m * nu + a]) * __expf(-ls);
-      logr += (-0.5f * z * z - ls - kHalfLog2Pi) - on_lp[m * nu + a];
-    }
-    const bool log_inside = logr > -p.log_clip_value && logr < p.log_clip_value;
-    const float ratio = __expf(fminf(fmaxf(logr, -p.log_clip_value), p.log_clip_value));
-    const float A = adv[m];
-    const float lo = 1.f - p.clip_param, hi = 1.f + p.clip_param;
-    const float s1 = ratio * A, s2 = fminf(fmaxf(ratio, lo), hi) * A;
-    // d(-min(s1, s2)) / d(log ratio); inside the clip range both surrogates coincide
-    const bool ratio_inside = ratio > lo && ratio < hi;
-    float g_logr = 0.f;
-    if (log_inside) {
-      if (s1 < s2 || ratio_inside) g_logr = -A * ratio;   // the unclipped surrogate is active (or both are the same)
-    }
-    // kl term: (on_lp - lp) * kl_coef * kl_scale per action
-    const float g_lp = (g_logr - p.kl_coef * kl_scale_of(p)) * inv_m;
-    const float g_ent = -p.entropy_coef * inv_m;
-    for (int a = 0; a < nu; ++a) {
-      const float ls = log_std[a];
-      const float is = __expf(-ls);
-      const float z = (action[m * nu + a] - mean[m * nu + a]) * is;
-      d_mean[m * nu + a] = g_lp * z * is;
-      dls[a] += g_lp * (z * z - 1.f) + g_ent;
-    }
-    // value term
-    const float vv = v[m], vo = on_v[m], t = tgt[m];
-    float gv;
-    if (p.use_clipped_value_loss) {
-      const float dvv = vv - vo;
-      const float vc = vo + fminf(fmaxf(dvv, -p.clip_param), p.clip_param);
-      const float e = vv - t, ec = vc - t;
-      if (e * e >= ec * ec) gv = e;
-      else gv = (dvv > -p.clip_param && dvv < p.clip_param) ? ec : 0.f;
-    } else {
-      gv = vv - t;
-    }
-    d_value[m] = p.value_loss_coef * gv * inv_m;
+// What the three gradient kernels below share: the gradient of the mean objective with respect to one action's log-density, from
+// the row's log ratio, and with respect to the value.
+__device__ __forceinline__ float surrogate_grad(const KsPpoLossParams& p, float kl_scale, float logr, float A, float inv_m) {
+  const bool log_inside = logr > -p.log_clip_value && logr < p.log_clip_value;
+  const float ratio = __expf(fminf(fmaxf(logr, -p.log_clip_value), p.log_clip_value));
+  const float lo = 1.f - p.clip_param, hi = 1.f + p.clip_param;
+  const float s1 = ratio * A, s2 = fminf(fmaxf(ratio, lo), hi) * A;
+  // d(-min(s1, s2)) / d(log ratio); inside the clip range both surrogates coincide
+  const bool ratio_inside = ratio > lo && ratio < hi;
+  const float g_logr = log_inside && (s1 < s2 || ratio_inside) ? -A * ratio : 0.f;
+  return (g_logr - p.kl_coef * kl_scale) * inv_m;  // kl term: (on_lp - lp) * kl_coef * kl_scale per action
+}
+
+__device__ __forceinline__ float value_grad(const KsPpoLossParams& p, float vv, float vo, float t, float inv_m) {
+  float gv;
+  if (p.use_clipped_value_loss) {
+    const float dvv = vv - vo;
+    const float vc = vo + fminf(fmaxf(dvv, -p.clip_param), p.clip_param);
+    const float e = vv - t, ec = vc - t;
+    if (e * e >= ec * ec) gv = e;
+    else gv = (dvv > -p.clip_param && dvv < p.clip_param) ? ec : 0.f;
+  } else {
+    gv = vv - t;
   }
-  for (int a = 0; a < nu; ++a) {
-    red[threadIdx.x] = dls[a];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
+  return p.value_loss_coef * gv * inv_m;
+}
+
+// The gradient kernels give every (row, action) pair a thread: a workgroup takes whole rows, the pairs leave their log-density
+// differences in LDS, one thread per row adds them in action order and turns the sum into the row's gradient factor, and the pairs
+// finish with it.  With one thread per row the lanes walked rows 80-2000 bytes apart, twice, and a batch of 12288 rows was 96
+// wavefronts (mixture of 10, 17 actions: 610 us, most of it private-memory traffic of the run-time-indexed component arrays).
+struct PpoGradIO {
+  const float *action, *on_lp, *adv, *tgt, *on_v, *v;
+  float* d_value;
+};
+
+// sel[r] <- gradient factor of row row0 + r from the per-pair differences el[r * nu + a]; also writes the rows' value gradients.
+// Barriers on both sides; every thread of the workgroup calls it.
+__device__ __forceinline__ void row_factors(const PpoGradIO& io, const KsPpoLossParams& p, float kl_scale, float inv_m, int64_t M, int64_t row0,
+                                            int rows, int nu, const float* el, float* sel) {
+  __syncthreads();
+  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
+    const int64_t m = row0 + r;
+    if (m < M) {
+      float logr = 0.f;
+      for (int a = 0; a < nu; ++a) logr += el[r * nu + a];
+      sel[r] = surrogate_grad(p, kl_scale, logr, io.adv[m], inv_m);
+      io.d_value[m] = value_grad(p, io.v[m], io.on_v[m], io.tgt[m], inv_m);
     }
-    if (threadIdx.x == 0) partial[(int64_t)blockIdx.x * nu + a] = red[0];
-    __syncthreads();
+  }
+  __syncthreads();
+}
+
+// Gaussian with one log deviation per action.  The log-std gradient of a thread's action is accumulated in its register over the
+// workgroup's rows (blockDim.x / nu whole rows at a time, so a thread keeps its action), then over the threads in a fixed order:
+// block partials, then ppo_grad_finish_kernel, so the result does not depend on scheduling.  1024 threads: at most 256 workgroups
+// (the partials' buffer) still keep 16 wavefronts per CU in flight (65536 rows x 20 actions: 36 -> 19 us).
+__global__ __launch_bounds__(1024) void ppo_loss_grad_kernel(int64_t M, int nu, KsPpoLossParams p, const float* __restrict__ mean,
+                                                            const float* __restrict__ log_std, PpoGradIO io, float* __restrict__ d_mean,
+                                                            float* __restrict__ partial) {
+  __shared__ float el[1024], sel[1024];
+  const int rows = 1024 / nu, r = threadIdx.x / nu, a = threadIdx.x - r * nu;
+  const bool mine = r < rows;
+  const float inv_m = 1.0f / (float)M, kl_scale = kl_scale_of(p), g_ent = -p.entropy_coef * inv_m;
+  const float ls = mine ? log_std[a] : 0.f, is = __expf(-ls);
+  float dls = 0.f;
+  for (int64_t row0 = (int64_t)blockIdx.x * rows; row0 < M; row0 += (int64_t)gridDim.x * rows) {
+    const bool ok = mine && row0 + r < M;
+    const int64_t i = row0 * nu + threadIdx.x;  // the pairs of whole rows are contiguous
+    float z = 0.f;
+    if (ok) {
+      z = (io.action[i] - mean[i]) * is;
+      el[threadIdx.x] = (-0.5f * z * z - ls - kHalfLog2Pi) - io.on_lp[i];
+    }
+    row_factors(io, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
+    if (ok) {
+      const float g_lp = sel[r];
+      d_mean[i] = g_lp * z * is;
+      dls += g_lp * (z * z - 1.f) + g_ent;
+    }
+    __syncthreads();  // the next rows reuse el and sel
+  }
+  el[threadIdx.x] = dls;
+  __syncthreads();
+  if ((int)threadIdx.x < nu) {
+    float s = 0.f;
+    for (int k = 0; k < rows; ++k) s += el[k * nu + threadIdx.x];
+    partial[(int64_t)blockIdx.x * nu + threadIdx.x] = s;
   }
 }
 
@@ -621,162 +784,127 @@ __global__ __launch_bounds__(256) void gaussian_head_log_prob_kernel(int64_t n, 
   if (ent) ent[idx] = 0.5f + kHalfLog2Pi + ls;
 }
 
-// The same objective for a network that emits its own deviations: raw (M, 2 nu) = means | raw deviations,
-// std = min((softplus(raw_std) + min_std) * var_scale, max_std).  One thread per row; d_raw receives the gradient of both halves.
-__global__ __launch_bounds__(256) void ppo_loss_grad_head_kernel(int64_t M, int nu, KsPpoLossParams p, KsGaussianHead hd,
-                                                                const float* __restrict__ raw, const float* __restrict__ action,
-                                                                const float* __restrict__ on_lp, const float* __restrict__ adv,
-                                                                const float* __restrict__ tgt, const float* __restrict__ on_v,
-                                                                const float* __restrict__ v, float* __restrict__ d_raw,
-                                                                float* __restrict__ d_value) {
-  const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (m >= M) return;
-  const float inv_m = 1.0f / (float)M;
-  const float* rm = raw + m * 2 * nu;
-  float logr = 0.f;
-  for (int a = 0; a < nu; ++a) {
-    const float mean = rm[a] + (hd.mean_bias ? hd.mean_bias[a] : 0.f);
-    const float r = rm[nu + a];
-    const float sp = r > 20.f ? r : log1pf(expf(r));
-    const float sd = fminf((sp + hd.min_std) * hd.var_scale, hd.max_std);
-    const float z = (action[m * nu + a] - mean) / sd;
-    logr += (-0.5f * z * z - logf(sd) - kHalfLog2Pi) - on_lp[m * nu + a];
-  }
-  const bool log_inside = logr > -p.log_clip_value && logr < p.log_clip_value;
-  const float ratio = __expf(fminf(fmaxf(logr, -p.log_clip_value), p.log_clip_value));
-  const float A = adv[m];
-  const float lo = 1.f - p.clip_param, hi = 1.f + p.clip_param;
-  const float s1 = ratio * A, s2 = fminf(fmaxf(ratio, lo), hi) * A;
-  const bool ratio_inside = ratio > lo && ratio < hi;
-  float g_logr = 0.f;
-  if (log_inside && (s1 < s2 || ratio_inside)) g_logr = -A * ratio;
-  const float g_lp = (g_logr - p.kl_coef * kl_scale_of(p)) * inv_m;
-  const float g_ent = -p.entropy_coef * inv_m;
-  for (int a = 0; a < nu; ++a) {
-    const float mean = rm[a] + (hd.mean_bias ? hd.mean_bias[a] : 0.f);
-    const float r = rm[nu + a];
-    const float sp = r > 20.f ? r : log1pf(expf(r));
+// One (row, action) pair of the mean | raw deviation head: raw (M, 2 nu) = means | raw deviations,
+// std = min((softplus(raw_std) + min_std) * var_scale, max_std).
+struct HeadPair {
+  float z, sd, sig;
+  bool capped;
+
+  // the log-density of the pair's action
+  __device__ __forceinline__ float eval(const KsGaussianHead& hd, const float* __restrict__ raw, int64_t m, int a, int nu, float action) {
+    const float mean = raw[m * 2 * nu + a] + (hd.mean_bias ? hd.mean_bias[a] : 0.f);
+    const float x = raw[m * 2 * nu + nu + a];
+    const float sp = x > 20.f ? x : log1pf(expf(x));
     const float pre = (sp + hd.min_std) * hd.var_scale;
-    const bool capped = pre >= hd.max_std;
-    const float sd = capped ? hd.max_std : pre;
-    const float z = (action[m * nu + a] - mean) / sd;
+    capped = pre >= hd.max_std;
+    sd = capped ? hd.max_std : pre;
+    sig = x > 20.f ? 1.f : 1.f / (1.f + expf(-x));
+    z = (action - mean) / sd;
+    return -0.5f * z * z - logf(sd) - kHalfLog2Pi;
+  }
+  __device__ __forceinline__ void grad(const KsGaussianHead& hd, float g_lp, float g_ent, int64_t m, int a, int nu, float* __restrict__ d_raw) const {
     d_raw[m * 2 * nu + a] = g_lp * z / sd;
     // d/d log(std) of the log-density is z^2 - 1 and of the entropy 1; then through the cap, the scale and the softplus
     const float d_ls = g_lp * (z * z - 1.f) + g_ent;
-    const float sig = r > 20.f ? 1.f : 1.f / (1.f + expf(-r));
     d_raw[m * 2 * nu + nu + a] = capped ? 0.f : d_ls / sd * hd.var_scale * sig;
   }
-  const float vv = v[m], vo = on_v[m], t = tgt[m];
-  float gv;
-  if (p.use_clipped_value_loss) {
-    const float dvv = vv - vo;
-    const float vc = vo + fminf(fmaxf(dvv, -p.clip_param), p.clip_param);
-    const float e = vv - t, ec = vc - t;
-    if (e * e >= ec * ec) gv = e;
-    else gv = (dvv > -p.clip_param && dvv < p.clip_param) ? ec : 0.f;
-  } else {
-    gv = vv - t;
-  }
-  d_value[m] = p.value_loss_coef * gv * inv_m;
-}
+};
 
-// The same objective for the mixture-of-Gaussians head: raw (M, 3 nu K) = component means, raw deviations and logits per
-// action.  One thread per row walks its actions twice (log ratio, then gradients).  The entropy term uses the usual
-// upper bound of a mixture's entropy, sum_k pi_k H_k + H(pi).
-__global__ __launch_bounds__(128) void ppo_loss_grad_mixture_kernel(int64_t M, int nu, KsPpoLossParams p, KsMixtureHead hd,
-                                                                   const float* __restrict__ raw, const float* __restrict__ action,
-                                                                   const float* __restrict__ on_lp, const float* __restrict__ adv,
-                                                                   const float* __restrict__ tgt, const float* __restrict__ on_v,
-                                                                   const float* __restrict__ v, float* __restrict__ d_raw,
-                                                                   float* __restrict__ d_value) {
-  const int64_t m = (int64_t)blockIdx.x * 128 + threadIdx.x;
-  if (m >= M) return;
-  const int K = hd.num_mixtures;
-  const float inv_m = 1.0f / (float)M;
-  const float* rm = raw + m * 3 * nu * K;
-  float* dm = d_raw + m * 3 * nu * K;
-  auto component = [&](int a, int k, float& mean, float& sd, bool& mean_clipped, bool& sd_capped, float& sig) {
-    const float r0 = rm[a * K + k] + (hd.mean_bias ? hd.mean_bias[a] : 0.f);
+// One pair of the mixture-of-Gaussians head: raw (M, 3 nu K) = component means, raw deviations and logits per action.  The entropy
+// term uses the usual upper bound of a mixture's entropy, sum_k pi_k H_k + H(pi).  The components stay in registers between the two
+// halves: KMAX is the compile-time bound of the loops over K.
+template <int KMAX>
+struct MixturePair {
+  float lpi[KMAX], z[KMAX], sd[KMAX], sig[KMAX], lsd[KMAX], lp;
+  unsigned mean_clipped, sd_capped;
+
+  __device__ __forceinline__ float eval(const KsMixtureHead& hd, const float* __restrict__ raw, int64_t m, int a, int nu, float action) {
+    const int K = hd.num_mixtures;
+    const float* rm = raw + m * 3 * nu * K;
+    const float bias = hd.mean_bias ? hd.mean_bias[a] : 0.f;
     const float lo = hd.clip_lo ? hd.clip_lo[a] : -INFINITY, hi = hd.clip_hi ? hd.clip_hi[a] : INFINITY;
-    mean = fminf(fmaxf(r0, lo), hi);
-    mean_clipped = r0 < lo || r0 > hi;
-    const float r = rm[(nu + a) * K + k];
-    const float sp = r > 20.f ? r : log1pf(expf(r));
-    const float pre = (sp + hd.min_std) * hd.var_scale;
-    sd_capped = pre >= hd.max_std;
-    sd = sd_capped ? hd.max_std : pre;
-    sig = r > 20.f ? 1.f : 1.f / (1.f + expf(-r));
-  };
-  auto log_mix = [&](int a, float x, float& lse_logits) {  // log density of the mixture at x, and the logits' normaliser
+    mean_clipped = sd_capped = 0;
     float lmax = -INFINITY;
-    for (int k = 0; k < K; ++k) lmax = fmaxf(lmax, rm[(2 * nu + a) * K + k]);
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) { lpi[k] = rm[(2 * nu + a) * K + k]; lmax = fmaxf(lmax, lpi[k]); }
     float zs = 0.f;
-    for (int k = 0; k < K; ++k) zs += expf(rm[(2 * nu + a) * K + k] - lmax);
-    lse_logits = lmax + logf(zs);
-    float tmax = -INFINITY, t[KS_MAX_MIXTURES];
-    for (int k = 0; k < K; ++k) {
-      float mean, sd, sg; bool c1, c2;
-      component(a, k, mean, sd, c1, c2, sg);
-      const float z = (x - mean) / sd;
-      t[k] = (rm[(2 * nu + a) * K + k] - lse_logits) - 0.5f * z * z - logf(sd) - kHalfLog2Pi;
-      tmax = fmaxf(tmax, t[k]);
-    }
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) zs += expf(lpi[k] - lmax);
+    const float lse = lmax + logf(zs);  // the logits' normaliser
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) {
+        lpi[k] -= lse;
+        const float r0 = rm[a * K + k] + bias;
+        const float mean = fminf(fmaxf(r0, lo), hi);
+        if (r0 < lo || r0 > hi) mean_clipped |= 1u << k;
+        const float y = rm[(nu + a) * K + k];
+        const float sp = y > 20.f ? y : log1pf(expf(y));
+        const float pre = (sp + hd.min_std) * hd.var_scale;
+        if (pre >= hd.max_std) sd_capped |= 1u << k;
+        sd[k] = pre >= hd.max_std ? hd.max_std : pre;
+        sig[k] = y > 20.f ? 1.f : 1.f / (1.f + expf(-y));
+        z[k] = (action - mean) / sd[k];
+        lsd[k] = logf(sd[k]);
+        tmax = fmaxf(tmax, lpi[k] - 0.5f * z[k] * z[k] - lsd[k] - kHalfLog2Pi);
+      }
     float acc = 0.f;
-    for (int k = 0; k < K; ++k) acc += expf(t[k] - tmax);
-    return tmax + logf(acc);
-  };
-  float logr = 0.f;
-  for (int a = 0; a < nu; ++a) {
-    float lse;
-    logr += log_mix(a, action[m * nu + a], lse) - on_lp[m * nu + a];
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) acc += expf(lpi[k] - 0.5f * z[k] * z[k] - lsd[k] - kHalfLog2Pi - tmax);
+    lp = tmax + logf(acc);
+    return lp;
   }
-  const bool log_inside = logr > -p.log_clip_value && logr < p.log_clip_value;
-  const float ratio = __expf(fminf(fmaxf(logr, -p.log_clip_value), p.log_clip_value));
-  const float A = adv[m];
-  const float lo_r = 1.f - p.clip_param, hi_r = 1.f + p.clip_param;
-  const float s1 = ratio * A, s2 = fminf(fmaxf(ratio, lo_r), hi_r) * A;
-  const bool ratio_inside = ratio > lo_r && ratio < hi_r;
-  float g_logr = 0.f;
-  if (log_inside && (s1 < s2 || ratio_inside)) g_logr = -A * ratio;
-  const float g_lp = (g_logr - p.kl_coef * kl_scale_of(p)) * inv_m;
-  const float g_ent = -p.entropy_coef * inv_m;
-  for (int a = 0; a < nu; ++a) {
-    const float x = action[m * nu + a];
-    float lse;
-    const float lp = log_mix(a, x, lse);
+  __device__ __forceinline__ void grad(const KsMixtureHead& hd, float g_lp, float g_ent, int64_t m, int a, int nu, float* __restrict__ d_raw) const {
+    const int K = hd.num_mixtures;
     // entropy bound: sum_k pi_k (h_k - log pi_k), h_k = 1/2 + log sqrt(2 pi) + log sd_k
     float gbar = 0.f;
-    for (int k = 0; k < K; ++k) {
-      float mean, sd, sg; bool c1, c2;
-      component(a, k, mean, sd, c1, c2, sg);
-      const float lpi = rm[(2 * nu + a) * K + k] - lse;
-      gbar += expf(lpi) * (0.5f + kHalfLog2Pi + logf(sd) - lpi);
-    }
-    for (int k = 0; k < K; ++k) {
-      float mean, sd, sg; bool mean_clipped, sd_capped;
-      component(a, k, mean, sd, mean_clipped, sd_capped, sg);
-      const float lpi = rm[(2 * nu + a) * K + k] - lse, pi = expf(lpi);
-      const float z = (x - mean) / sd;
-      const float resp = expf(lpi - 0.5f * z * z - logf(sd) - kHalfLog2Pi - lp);  // responsibility of component k
-      dm[a * K + k] = mean_clipped ? 0.f : g_lp * resp * z / sd;
-      const float d_ls = g_lp * resp * (z * z - 1.f) + g_ent * pi;
-      dm[(nu + a) * K + k] = sd_capped ? 0.f : d_ls / sd * hd.var_scale * sg;
-      const float gk = 0.5f + kHalfLog2Pi + logf(sd) - lpi;
-      dm[(2 * nu + a) * K + k] = g_lp * (resp - pi) + g_ent * pi * (gk - gbar);
-    }
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) gbar += expf(lpi[k]) * (0.5f + kHalfLog2Pi + lsd[k] - lpi[k]);
+    float* dm = d_raw + m * 3 * nu * K;
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (k < K) {
+        const float pi = expf(lpi[k]);
+        const float resp = expf(lpi[k] - 0.5f * z[k] * z[k] - lsd[k] - kHalfLog2Pi - lp);  // responsibility of component k
+        dm[a * K + k] = (mean_clipped >> k & 1u) ? 0.f : g_lp * resp * z[k] / sd[k];
+        const float d_ls = g_lp * resp * (z[k] * z[k] - 1.f) + g_ent * pi;
+        dm[(nu + a) * K + k] = (sd_capped >> k & 1u) ? 0.f : d_ls / sd[k] * hd.var_scale * sig[k];
+        dm[(2 * nu + a) * K + k] = g_lp * (resp - pi) + g_ent * pi * (0.5f + kHalfLog2Pi + lsd[k] - lpi[k] - gbar);
+      }
   }
-  const float vv = v[m], vo = on_v[m], t = tgt[m];
-  float gv;
-  if (p.use_clipped_value_loss) {
-    const float dvv = vv - vo;
-    const float vc = vo + fminf(fmaxf(dvv, -p.clip_param), p.clip_param);
-    const float e = vv - t, ec = vc - t;
-    if (e * e >= ec * ec) gv = e;
-    else gv = (dvv > -p.clip_param && dvv < p.clip_param) ? ec : 0.f;
+};
+
+// The gradient with respect to the raw head outputs.  A workgroup takes 256 / nu whole rows; a head of more than 256 actions takes
+// a row per workgroup and evaluates its pairs once for the row's sum and again for the gradient.
+template <typename Pair, typename Head>
+__global__ __launch_bounds__(256) void ppo_loss_grad_pairs_kernel(int64_t M, int nu, KsPpoLossParams p, Head hd, const float* __restrict__ raw,
+                                                                 PpoGradIO io, float* __restrict__ d_raw) {
+  __shared__ float el[256], sel[256];
+  const float inv_m = 1.0f / (float)M, kl_scale = kl_scale_of(p), g_ent = -p.entropy_coef * inv_m;
+  Pair pair;
+  if (nu <= 256) {
+    const int rows = 256 / nu, r = threadIdx.x / nu, a = threadIdx.x - r * nu;
+    const int64_t row0 = (int64_t)blockIdx.x * rows, m = row0 + r;
+    const bool ok = r < rows && m < M;
+    if (ok) el[threadIdx.x] = pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]) - io.on_lp[m * nu + a];
+    row_factors(io, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
+    if (ok) pair.grad(hd, sel[r], g_ent, m, a, nu, d_raw);
   } else {
-    gv = vv - t;
+    const int64_t m = blockIdx.x;
+    float part = 0.f;
+    for (int a = threadIdx.x; a < nu; a += 256) part += pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]) - io.on_lp[m * nu + a];
+    el[threadIdx.x] = part;
+    row_factors(io, p, kl_scale, inv_m, M, m, 1, 256, el, sel);
+    for (int a = threadIdx.x; a < nu; a += 256) {
+      pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]);
+      pair.grad(hd, sel[0], g_ent, m, a, nu, d_raw);
+    }
   }
-  d_value[m] = p.value_loss_coef * gv * inv_m;
 }
 
 // d_log_std[a] = sum over the blocks' partial sums: one workgroup per action, a fixed tree over up to 256 partials (one
@@ -1042,10 +1170,11 @@ extern "C" int ks_ppo_loss_grad(ks_stream_t stream, int64_t M, int32_t nu, const
   if (!mean || !log_std || !action || !on_log_probs || !advantages || !value_targets || !on_values || !values || !d_mean ||
       !d_value || !d_log_std || !workspace)
     return ks::fail(KS_EINVAL, "ks_ppo_loss_grad: null pointer");
-  const int64_t want = (M + 255) / 256;
+  const int64_t want = (M + 1024 / nu - 1) / (1024 / nu);
   const int blocks = (int)(want < KS_PPO_GRAD_BLOCKS ? want : KS_PPO_GRAD_BLOCKS);
-  hipLaunchKernelGGL(ks::ppo_loss_grad_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, M, nu, *params, mean, log_std, action,
-                     on_log_probs, advantages, value_targets, on_values, values, d_mean, d_value, (float*)workspace);
+  const ks::PpoGradIO io = {action, on_log_probs, advantages, value_targets, on_values, values, d_value};
+  hipLaunchKernelGGL(ks::ppo_loss_grad_kernel, dim3(blocks), dim3(1024), 0, (hipStream_t)stream, M, nu, *params, mean, log_std, io, d_mean,
+                     (float*)workspace);
   hipLaunchKernelGGL(ks::ppo_grad_finish_kernel, dim3(nu), dim3(256), 0, (hipStream_t)stream, blocks, nu, (const float*)workspace,
                      d_log_std);
   return ks::check_launch("ks_ppo_loss_grad");
@@ -1061,10 +1190,11 @@ extern "C" int ks_ppo_loss_grad_head(ks_stream_t stream, int64_t M, int32_t nu, 
     return ks::fail(KS_EINVAL, "ks_ppo_loss_grad_head: null pointer");
   if (!(head->max_std > 0.f) || head->min_std < 0.f || !(head->var_scale > 0.f))
     return ks::fail(KS_EINVAL, "ks_ppo_loss_grad_head: bad deviation bounds");
-  const int64_t grid = (M + 255) / 256;
+  const int64_t rows = nu <= 256 ? 256 / nu : 1, grid = (M + rows - 1) / rows;
   if (grid > 0x7fffffff) return ks::fail(KS_ELIMIT, "ks_ppo_loss_grad_head: too many rows");
-  hipLaunchKernelGGL(ks::ppo_loss_grad_head_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M, nu, *params, *head, raw,
-                     action, on_log_probs, advantages, value_targets, on_values, values, d_raw, d_value);
+  const ks::PpoGradIO io = {action, on_log_probs, advantages, value_targets, on_values, values, d_value};
+  hipLaunchKernelGGL((ks::ppo_loss_grad_pairs_kernel<ks::HeadPair, KsGaussianHead>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M,
+                     nu, *params, *head, raw, io, d_raw);
   return ks::check_launch("ks_ppo_loss_grad_head");
 }
 
@@ -1095,9 +1225,13 @@ extern "C" int ks_ppo_loss_grad_mixture(ks_stream_t stream, int64_t M, int32_t n
   if (!(head->max_std > 0.f) || head->min_std < 0.f || !(head->var_scale > 0.f))
     return ks::fail(KS_EINVAL, "ks_ppo_loss_grad_mixture: bad deviation bounds");
   if ((head->clip_lo == nullptr) != (head->clip_hi == nullptr)) return ks::fail(KS_EINVAL, "ks_ppo_loss_grad_mixture: clip_lo and clip_hi come together");
-  const int64_t grid = (M + 127) / 128;
+  const int64_t rows = nu <= 256 ? 256 / nu : 1, grid = (M + rows - 1) / rows;
   if (grid > 0x7fffffff) return ks::fail(KS_ELIMIT, "ks_ppo_loss_grad_mixture: too many rows");
-  hipLaunchKernelGGL(ks::ppo_loss_grad_mixture_kernel, dim3((unsigned)grid), dim3(128), 0, (hipStream_t)stream, M, nu, *params, *head, raw,
-                     action, on_log_probs, advantages, value_targets, on_values, values, d_raw, d_value);
+  const ks::PpoGradIO io = {action, on_log_probs, advantages, value_targets, on_values, values, d_value};
+  const int K = head->num_mixtures;  // the loops over the components are unrolled to the next bound
+  auto kfn = K <= 5 ? ks::ppo_loss_grad_pairs_kernel<ks::MixturePair<5>, KsMixtureHead>
+                    : (K <= 10 ? ks::ppo_loss_grad_pairs_kernel<ks::MixturePair<10>, KsMixtureHead>
+                               : ks::ppo_loss_grad_pairs_kernel<ks::MixturePair<KS_MAX_MIXTURES>, KsMixtureHead>);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M, nu, *params, *head, raw, io, d_raw);
   return ks::check_launch("ks_ppo_loss_grad_mixture");
 }

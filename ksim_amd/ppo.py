@@ -66,22 +66,19 @@ def compute_ppo_inputs(
         raise _lib.KsError("values, rewards and dones must share one 2-D shape")
     if succ is not None and succ.shape != values_bt.shape:
         raise _lib.KsError("successes must have the shape of values")
-    gae = torch.empty_like(values_bt)
-    ret = torch.empty_like(values_bt)
-    tgt = torch.empty_like(values_bt)
-    fn = lib.ks_gae_tn if time_major else lib.ks_gae_bt
-    _lib.check(
-        fn(_lib.current_stream(), values_bt.shape[0], values_bt.shape[1], _lib.ptr(values_bt), _lib.ptr(rewards_bt),
-           _lib.ptr(dones), _lib.ptr(succ), float(decay_gamma), float(gae_lambda), int(monte_carlo_returns),
-           _lib.ptr(gae), _lib.ptr(ret), _lib.ptr(tgt))
-    )
-    adv = gae
+    stream, addr = _lib.current_stream(), _lib.addr
+    # one allocation for all outputs, handed out as its rows
+    gae, ret, tgt, *adv = torch.empty((4 if normalize_advantages else 3, *values_bt.shape), dtype=torch.float32, device=values_bt.device).unbind(0)
     if normalize_advantages:
-        adv = torch.empty_like(gae)
-        ws = _workspace(gae.device)
-        _lib.check(lib.ks_normalize_advantages(_lib.current_stream(), gae.numel(), _lib.ptr(gae), _lib.ptr(adv),
-                                               _lib.ptr(ws)))
-    return PPOInputs(advantages_bt=adv, value_targets_bt=tgt, gae_bt=gae, returns_bt=ret)
+        ws = _workspace(values_bt.device)
+        _lib.check(lib.ks_gae_normalized(stream, time_major, *values_bt.shape, addr(values_bt), addr(rewards_bt), addr(dones), addr(succ),
+                                         decay_gamma, gae_lambda, int(monte_carlo_returns), addr(gae), addr(ret), addr(tgt), addr(adv[0]),
+                                         addr(ws)))
+    else:
+        fn = lib.ks_gae_tn if time_major else lib.ks_gae_bt
+        _lib.check(fn(stream, *values_bt.shape, addr(values_bt), addr(rewards_bt), addr(dones), addr(succ), decay_gamma, gae_lambda,
+                      int(monte_carlo_returns), addr(gae), addr(ret), addr(tgt)))
+    return PPOInputs(advantages_bt=adv[0] if adv else gae, value_targets_bt=tgt, gae_bt=gae, returns_bt=ret)
 
 
 def compute_ppo_loss(
@@ -111,19 +108,16 @@ def compute_ppo_loss(
     _lib.require_cuda(on.log_probs, on.values, off.log_probs, off.values, off.entropy, ppo_inputs.advantages_bt,
                       ppo_inputs.value_targets_bt, dtype=torch.float32)
     dev = on.values.device
-    out = {k: torch.empty((B, T), dtype=torch.float32, device=dev) for k in ("policy", "value", "kl")}
-    if off.entropy is not None:
-        out["entropy"] = torch.empty((B, T), dtype=torch.float32, device=dev)
+    names = ("policy", "value", "kl") if off.entropy is None else ("policy", "value", "kl", "entropy")
+    out = dict(zip(names, torch.empty((len(names), B, T), dtype=torch.float32, device=dev).unbind(0)))
     total = torch.empty((), dtype=torch.float32, device=dev)
     params = _lib.KsPpoLossParams(clip_param, value_loss_coef, entropy_coef, kl_coef, log_clip_value, kl_scale,
                                   int(use_clipped_value_loss))
-    ws = _workspace(dev)
+    ws, addr = _workspace(dev), _lib.addr
     _lib.check(
-        lib.ks_ppo_loss(_lib.current_stream(), B * T, A, params, _lib.ptr(ppo_inputs.advantages_bt),
-                        _lib.ptr(ppo_inputs.value_targets_bt), _lib.ptr(on.log_probs), _lib.ptr(on.values),
-                        _lib.ptr(off.log_probs), _lib.ptr(off.values), _lib.ptr(off.entropy), _lib.ptr(out["policy"]),
-                        _lib.ptr(out["value"]), _lib.ptr(out["kl"]), _lib.ptr(out.get("entropy")), _lib.ptr(total),
-                        _lib.ptr(ws))
+        lib.ks_ppo_loss(_lib.current_stream(), B * T, A, params, addr(ppo_inputs.advantages_bt), addr(ppo_inputs.value_targets_bt),
+                        addr(on.log_probs), addr(on.values), addr(off.log_probs), addr(off.values), addr(off.entropy), addr(out["policy"]),
+                        addr(out["value"]), addr(out["kl"]), addr(out.get("entropy")), addr(total), addr(ws))
     )
     if off.aux_losses is not None:  # ppo.py:242-244 — user terms pass through and join the mean
         aux_sum = None

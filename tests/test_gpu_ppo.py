@@ -144,3 +144,26 @@ def test_reward_total_and_done_success():
     wd, ws = oterms.combine_terminations([tvals[j] for j in range(k)])
     assert np.array_equal(done.cpu().numpy().astype(bool), wd)  # bit-exact masks
     assert np.array_equal(succ.cpu().numpy().astype(bool), ws)
+
+
+@pytest.mark.parametrize("B,T", [(1, 16), (70, 8), (6, 17), (33, 32), (4, 33), (9000, 24)])
+@pytest.mark.parametrize("time_major", [False, True])
+def test_normalized_gae_of_short_rows(B, T, time_major):
+    """The two-launch path with normalisation, at the row lengths where several rows share a wavefront, and past the batch where
+    a workgroup walks several rows."""
+    from ksim_amd import ppo
+
+    v, r, done, succ = _inputs(B + T, B, T, p_done=0.05)
+    want = oppo.compute_ppo_inputs(v, r, done, succ, 0.99, 0.95, normalize_advantages=True)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a.T) if time_major else a).to("cuda:0")  # noqa: E731
+    out = ppo.compute_ppo_inputs(t(v), t(r), t(done), t(succ), 0.99, 0.95, normalize_advantages=True, time_major=time_major)
+    back = (lambda x: x.T) if time_major else (lambda x: x)
+    for got, key in ((out.gae_bt, "gae"), (out.returns_bt, "returns"), (out.value_targets_bt, "value_targets"), (out.advantages_bt, "advantages")):
+        _close(back(got), want[key])
+
+
+@pytest.mark.parametrize("n,A,with_entropy", [(1, 20, True), (65, 2, True), (64, 31, True), (130, 32, False), (1000, 3, False)])
+def test_ppo_loss_rows(n, A, with_entropy):
+    """Row lengths around what a wavefront stages (31 actions; longer rows and A = 1 take the direct kernel), a last tile of one
+    element and of all 64."""
+    test_ppo_loss_parity(n, 1, A, with_entropy)

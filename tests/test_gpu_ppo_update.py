@@ -666,3 +666,39 @@ def test_mirror_losses_match_autograd_and_vanish_for_a_symmetric_policy():
     for a, b in zip(pol2.actor.parameters(gradients=True) + pol2.critic.parameters(gradients=True),
                     pol3.actor.parameters(gradients=True) + pol3.critic.parameters(gradients=True)):
         assert rel(a[0].cpu().numpy(), b[0].cpu().numpy()) < 1e-5 and rel(a[1].cpu().numpy(), b[1].cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("M,A,K", [(3, 300, 0), (1, 1, 0), (257, 256, 0), (41, 7, 1), (9, 13, 16), (2, 260, 3)])
+def test_head_gradients_at_the_edges_of_the_row_split(M, A, K):
+    """Rows per workgroup 256 / A: one pair, rows as long as a workgroup, and heads of more actions than it has threads (a row per
+    workgroup); mixtures at the bounds of the unrolled component loops.  fp32 against float64 autograd.  A pair's log-density is a
+    few units large when the action lies within a few deviations of the mean and is rounded at 2^-24 of that in each of its few
+    terms (about 1e-6); the row's log ratio adds A of them, and the gradient is proportional to its exponential: hence 1e-6 A.
+    (Actions hundreds of deviations out have log-densities of 1e4, whose rounding alone is 6e-4 of the ratio: not drawn.)"""
+    from ksim_amd import _lib, _lib_terms as T
+
+    lib = _lib.load()
+    rng = np.random.default_rng(M + A + K)
+    W = 3 * A * K if K else 2 * A
+    raw = rng.normal(size=(M, W))
+    hd = dict(min_std=0.01, max_std=1.5, var_scale=0.5)
+    bias = torch.tensor(rng.normal(size=A) * 0.1)
+    tr, first = torch.tensor(raw, requires_grad=True), raw.reshape(M, -1, A, max(K, 1))[..., 0]  # means, raw deviations of one component
+    sd = np.minimum((np.log1p(np.exp(first[:, 1])) + 0.01) * 0.5, 1.5)
+    act = torch.tensor(first[:, 0] + bias.numpy() + sd * rng.uniform(-2, 2, size=(M, A)))
+    dist = (lambda r: ou.mixture_head(r, act, K, mean_bias=bias, **hd)) if K else (lambda r: ou.gaussian_head(r, act, mean_bias=bias, **hd))
+    on_lp = dist(torch.tensor(raw + rng.normal(size=raw.shape) * 0.02 / np.sqrt(A)))[0]
+    adv, tgt, on_v, v = (rng.normal(size=M) for _ in range(4))
+    tv = torch.tensor(v, requires_grad=True)
+    lp, ent = dist(tr)
+    ou.ppo_loss_torch(torch.tensor(adv), torch.tensor(tgt), on_lp, torch.tensor(on_v), lp, tv, ent, CFG, 1.0)[0].backward()
+    p = _lib.KsPpoLossParams(0.2, 0.5, 0.008, 1e-3, 5.0, 1.0, 1)
+    bias_d = t32(bias)
+    head = T.KsMixtureHead(K, 0.01, 1.5, 0.5, 0, _lib.addr(bias_d), None, None) if K else T.KsGaussianHead(0.01, 1.5, 0.5, 0, _lib.addr(bias_d))
+    d_raw, d_value = torch.empty(M, W, device=DEV), torch.empty(M, device=DEV)
+    args = [t32(a) for a in (raw, act, on_lp.detach(), adv, tgt, on_v, v)]
+    fn = lib.ks_ppo_loss_grad_mixture if K else lib.ks_ppo_loss_grad_head
+    _lib.check(fn(_lib.current_stream(), M, A, ctypes.byref(p), ctypes.byref(head), *[_lib.ptr(a) for a in args], _lib.ptr(d_raw), _lib.ptr(d_value)))
+    for got, want in ((d_raw, tr.grad), (d_value, tv.grad)):
+        want = want.numpy()
+        assert np.abs(got.cpu().numpy() - want).max() <= (1e-4 + 1e-6 * A) * np.abs(want).max()
