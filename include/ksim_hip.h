@@ -853,6 +853,10 @@ int ks_adam_step(ks_stream_t stream, int64_t n, float* param, const float* grad,
 /* Copies of the parameters and gradients in the caller's (out, in) layout, for checks and checkpoints. */
 int ks_mlp_get_params(const KsMlp* mlp, ks_stream_t stream, int32_t layer, float* weight /*(out,in) dev*/, float* bias /*(out) dev*/,
                       int32_t gradients /*0: parameters, 1: gradients*/);
+/* Every weight and bias of the network at once, packed: layer l's weight (out, in) starts ks_mlp_param_floats(mlp, l) floats into
+ * `out`, its bias behind it at the next multiple of four floats; ks_mlp_param_floats(mlp, n_layers) is the whole length. */
+int64_t ks_mlp_param_floats(const KsMlp* mlp, int32_t layer);
+int ks_mlp_get_all_params(const KsMlp* mlp, ks_stream_t stream, float* out /*dev*/, int32_t gradients);
 
 /* Backward pass through time of a GRU stack (the jax.grad through the lax.scan over the trajectory in
  * PPOTask._single_step, ksim/task/ppo.py:572-694, for the recurrent actors and critics of examples/walking.py:40-208).

@@ -289,6 +289,10 @@ def bind(lib) -> None:
     lib.ks_mlp_grad_sqnorm.argtypes = [c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_adam_step.argtypes = [c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
     lib.ks_adam_step.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
+    lib.ks_mlp_param_floats.argtypes = [c_void_p, c_int32]
+    lib.ks_mlp_param_floats.restype = c_int64
+    lib.ks_mlp_get_all_params.argtypes = [c_void_p, c_void_p, c_void_p, c_int32]
+    lib.ks_mlp_get_all_params.restype = c_int32
     lib.ks_mlp_get_params.argtypes = [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32]
     lib.ks_gaussian_log_prob.argtypes = [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     for name in ("ks_mlp_train_init", "ks_mlp_train_forward", "ks_mlp_train_backward", "ks_grad_sqnorm",

@@ -34,14 +34,24 @@ def loop_slice(clip: torch.Tensor, start: int, window_t: int) -> torch.Tensor:
     return clip[idx]
 
 
+def _gather(motions: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
+    """`motions` rows picked by index vectors drawn on the host, which travel in one copy that nothing waits for (a copy from
+    pageable memory would hold the host until the GPU has caught up)."""
+    if motions.is_cuda:
+        rows = torch.empty(rows.shape, dtype=torch.int64, pin_memory=True).copy_(rows).to(motions.device, non_blocking=True)
+    return motions.index_select(0, rows)
+
+
 def make_real_batch(motions: torch.Tensor, window_t: int, batch_b: int, generator: torch.Generator) -> torch.Tensor:
     """`batch_b` windows from reference clips (N, T_clip, F): a clip drawn uniformly, then a uniform start in it
     (amp.py:570-625; the draws come from `generator`, not from jax's key splitting)."""
-    clip_idx = torch.randint(0, motions.shape[0], (batch_b,), generator=generator)
-    starts = torch.randint(0, motions.shape[1], (batch_b,), generator=generator)
+    n, t_clip = motions.shape[0], motions.shape[1]
+    clip_idx = torch.randint(0, n, (batch_b,), generator=generator)
+    starts = torch.randint(0, t_clip, (batch_b,), generator=generator)
     # every window of the batch in one gather: frame (start + t) mod T_clip of the drawn clip, as loop_slice takes them
-    frames = (starts[:, None] + torch.arange(window_t)[None, :]) % motions.shape[1]
-    return motions[clip_idx[:, None].to(motions.device), frames.to(motions.device)]
+    frames = (starts[:, None] + torch.arange(window_t)[None, :]) % t_clip
+    flat = motions.reshape(n * t_clip, *motions.shape[2:])
+    return _gather(flat, (clip_idx[:, None] * t_clip + frames).view(-1)).view(batch_b, window_t, *motions.shape[2:])
 
 
 def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> torch.Tensor:
@@ -49,7 +59,7 @@ def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Gen
     num_envs = sim_motions.shape[0]
     if num_envs % batch_b != 0:
         raise ValueError(f"amp_reference_batch_size ({batch_b}) must divide batch_size ({num_envs}).")
-    return sim_motions[torch.randperm(num_envs, generator=generator)[:batch_b].to(sim_motions.device)]
+    return _gather(sim_motions, torch.randperm(num_envs, generator=generator)[:batch_b])
 
 
 class DiscriminatorUpdate:
@@ -88,4 +98,4 @@ class DiscriminatorUpdate:
             sim = make_sim_batch(sim_motions, self.cfg.amp_reference_batch_size, generator)
             for k, v in self.step(real, sim).items():
                 sums[k] = v if k not in sums else sums[k] + v
-        return {k: v / self.cfg.disc_num_passes for k, v in sums.items()}
+        return sums if self.cfg.disc_num_passes == 1 else {k: v / self.cfg.disc_num_passes for k, v in sums.items()}

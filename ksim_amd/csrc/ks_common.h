@@ -27,5 +27,6 @@ constexpr int kWave = 64;
 
 // defined beside the MLP handle: weight matrix (npad, kpad) of layer l in working precision and its transpose (after train_init)
 int mlp_peek_layer(const KsMlp* h, int l, const void** W, const void** Wt, int* npad, int* kpad, int* dtype);
+const float* mlp_peek_bias(const KsMlp* h, int l);
 
 }  // namespace ks

@@ -628,8 +628,9 @@ using namespace ks;
 struct KsGru {
   int I, H;
   KsMlp *proj_i, *proj_h;
-  float* bias_n;    // device (H)
-  float* bias_tmp;  // device (3H), training only
+  float* bias_n;        // device (H), as given at creation
+  const float* bias_nt; // training handles: the same entries of the hidden projection's bias, which the optimiser updates in place
+  const float* bn() const { return bias_nt ? bias_nt : bias_n; }
 };
 
 extern "C" int ks_gru_create(const KsGruDesc* d, KsGru** out) {
@@ -661,7 +662,6 @@ extern "C" int ks_gru_destroy(KsGru* g) {
   ks_mlp_destroy(g->proj_i);
   ks_mlp_destroy(g->proj_h);
   if (g->bias_n) (void)hipFree(g->bias_n);
-  if (g->bias_tmp) (void)hipFree(g->bias_tmp);
   delete g;
   return KS_OK;
 }
@@ -708,7 +708,7 @@ extern "C" int ks_gru_sequence_forward(const KsGru* g, ks_stream_t stream, int64
   const int64_t grid = (sets + groups - 1) / groups;
   if (grid > 0x7fffffff || T > 0x7fffffff) return fail(KS_ELIMIT, "ks_gru_sequence_forward: too many rows or steps");
   auto kfn = bf ? gru_seq_forward_kernel<true> : gru_seq_forward_kernel<false>;
-  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, M, groups, gi, W, ldw, g->bias_n,
+  hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, M, groups, gi, W, ldw, g->bn(),
                      h0, fresh, hs, saved);
   return check_launch("ks_gru_sequence_forward");
 }
@@ -758,7 +758,7 @@ extern "C" int ks_gru_forward(const KsGru* g, ks_stream_t stream, int64_t M, con
   const int64_t n = M * g->H, grid = (n + 255) / 256;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_gru_forward: too many elements");
   hipLaunchKernelGGL(gru_gate_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M, g->H, gi, gh, h_in,
-                     g->bias_n, fresh, h_out);
+                     g->bn(), fresh, h_out);
   return check_launch("ks_gru_forward");
 }
 
@@ -768,8 +768,7 @@ extern "C" int ks_gru_train_init(KsGru* g) {
   if (rc == KS_OK) rc = ks_mlp_train_init(g->proj_h);
   // the hidden projection's bias is (0, 0, b_n): only its candidate part is a parameter of the cell
   if (rc == KS_OK) rc = ks_mlp_freeze_bias_prefix(g->proj_h, 0, 2 * g->H);
-  if (rc == KS_OK && !g->bias_tmp && hipMalloc((void**)&g->bias_tmp, 3 * (size_t)g->H * 4) != hipSuccess)
-    rc = fail(KS_ELAUNCH, "ks_gru_train_init: allocation failed");
+  if (rc == KS_OK) g->bias_nt = mlp_peek_bias(g->proj_h, 0) + 2 * g->H;
   return rc;
 }
 
@@ -787,15 +786,9 @@ extern "C" int ks_gru_grad_sqnorm(const KsGru* g, ks_stream_t stream, double* ac
 }
 
 extern "C" int ks_gru_adam_step(KsGru* g, ks_stream_t stream, const KsAdamParams* params, const double* sqnorm) {
-  if (!g || !g->bias_tmp) return fail(KS_EINVAL, "ks_gru_adam_step: call ks_gru_train_init first");
-  int rc = ks_mlp_adam_step(g->proj_i, stream, params, sqnorm);
-  if (rc == KS_OK) rc = ks_mlp_adam_step(g->proj_h, stream, params, sqnorm);
-  // the gate kernel's own copy of b_n (used for envs that start an episode) follows the hidden projection's bias
-  if (rc == KS_OK) rc = ks_mlp_get_params(g->proj_h, stream, 0, nullptr, g->bias_tmp, 0);
-  if (rc == KS_OK && hipMemcpyAsync(g->bias_n, g->bias_tmp + 2 * (size_t)g->H, (size_t)g->H * 4, hipMemcpyDeviceToDevice,
-                                    (hipStream_t)stream) != hipSuccess)
-    rc = fail(KS_ELAUNCH, "ks_gru_adam_step: bias copy failed");
-  return rc;
+  if (!g || !g->bias_nt) return fail(KS_EINVAL, "ks_gru_adam_step: call ks_gru_train_init first");
+  const int rc = ks_mlp_adam_step(g->proj_i, stream, params, sqnorm);
+  return rc != KS_OK ? rc : ks_mlp_adam_step(g->proj_h, stream, params, sqnorm);
 }
 
 extern "C" int ks_gru_train_forward(const KsGru* g, ks_stream_t stream, int64_t M, const float* x, const float* h_in,
@@ -819,7 +812,7 @@ extern "C" int ks_gru_train_forward(const KsGru* g, ks_stream_t stream, int64_t 
   const int64_t n = M * g->H, grid = (n + 255) / 256;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_gru_train_forward: too many elements");
   hipLaunchKernelGGL(gru_gate_train_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M, g->H, gi, gh, h_in,
-                     g->bias_n, fresh, h_out, saved);
+                     g->bn(), fresh, h_out, saved);
   return check_launch("ks_gru_train_forward");
 }
 

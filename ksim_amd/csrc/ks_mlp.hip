@@ -1306,6 +1306,8 @@ int mlp_peek_layer(const KsMlp* h, int l, const void** W, const void** Wt, int* 
   *npad = h->m.npad[l]; *kpad = h->m.kpad[l]; *dtype = h->m.dtype;
   return KS_OK;
 }
+// fp32 master bias of layer l (training handles), padded to the layer's width; updated in place by the optimiser step
+const float* mlp_peek_bias(const KsMlp* h, int l) { return h && h->m.train && l >= 0 && l < h->m.n_layers ? h->m.mb[l] : nullptr; }
 }  // namespace ks
 
 extern "C" int ks_mlp_destroy(KsMlp* h) {
@@ -1781,9 +1783,8 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
   return KS_OK;
 }
 
-template <bool A_KC, bool B_KC>
-static void sgemm(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                  int64_t ldc, const float* bias, int act, bool accumulate, float* part, float* colsum = nullptr, float* colpart = nullptr);
+static void sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                        int64_t ldc, float* part, float* colsum, float* colpart);
 
 template <typename T>
 static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws,
@@ -1834,8 +1835,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
       // weight gradient dZ^T X and the bias gradient, the column sums of dZ, in one pass over the row-major operands as they
       // are, on the 128 x 128 tiles of the long-reduction product; no transposed copies.
       float* colpart = ws.part + (int64_t)kDiscMaxSlices * np * kp;
-      sgemm<false, false>(s, np, m.dims[0], M, (const float*)dz, np, x, m.dims[0], m.gW[0], kp, nullptr, KS_ACT_NONE, false, ws.part,
-                          m.gb[0], colpart);
+      sgemm_tn128(s, np, m.dims[0], M, (const float*)dz, np, x, m.dims[0], m.gW[0], kp, ws.part, m.gb[0], colpart);
       break;
     }
     if (want_w && !have_bias) {
@@ -2027,63 +2027,216 @@ extern "C" int ks_mlp_adam_step(KsMlp* h, ks_stream_t stream, const KsAdamParams
 // master weights, the products on the fp32 matrix-core instruction.
 namespace ks {
 
-// C(i, j) (+)= sum_k A(i, k) B(k, j) in fp32 on the matrix cores: 64 x 64 tile per workgroup, 16-deep slices through LDS,
-// each of the four wavefronts accumulating one 32 x 32 quadrant with v_mfma_f32_32x32x2_f32 (lane c + 32 h feeds
-// A(c, 2 s + h) and B(2 s + h, c) of step s and ends up with C(8 g + 4 h + e, c) in accumulator register 4 g + e).
+// first and second derivative of the activation from its output y = f(z)
+__device__ __forceinline__ void act_derivatives(int act, float y, float& d1, float& d2) {
+  d1 = 1.f; d2 = 0.f;
+  if (act == KS_ACT_ELU) { if (y <= 0.f) { d1 = y + 1.f; d2 = y + 1.f; } }  // exp(z) = elu(z) + 1 for z <= 0
+  else if (act == KS_ACT_RELU) d1 = y > 0.f ? 1.f : 0.f;
+  else if (act == KS_ACT_TANH) { d1 = 1.f - y * y; d2 = -2.f * y * d1; }
+}
+
+// Words that workgroups on different XCDs hand each other inside one launch: written through, and read past, the L2 of the writer's and
+// reader's XCD.  A device-scope fence does the same for everything at once by writing back and invalidating whole L2s: with one per
+// workgroup the weight-gradient products below took 41 us instead of 9.5 (and 18.8 with one uncut slice).
+__device__ __forceinline__ void device_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float device_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// What becomes of an entry of the product, at (i, j) of the output and of the arrays beside it (all with the output's stride):
+enum { kEpiStore,    // C (+)= v
+       kEpiLayer,    // C = act(v + bias_j): a layer of the forward pass
+       kEpiDelta,    // C = v, C2 = f'(Y) v: a_l and d_l of the input gradient's chain
+       kEpiPenalty,  // C = scale v, and the tile's sum of v^2 to sums[tile]: the penalty's gradient and value
+       kEpiTangent,  // C = f'(Y) v, C2 = f''(Y) X v: v_l and r_l of the sweep back through that chain
+       kEpiDz };     // C = f'(Y) v (+ X on the first x_rows rows): the ordinary backward pass
+struct SgemmArgs {
+  int M, N, K;
+  const float *A, *A2;  // A2: rows (or, stored (k, i), reduction steps) from a_split on come from this second array
+  int64_t lda;
+  int a_split;
+  const float *B, *B2;
+  int64_t ldb;
+  int b_split;
+  float* C;
+  int64_t ldc;
+  int kslice;
+  int epi, act, accumulate;
+  const float *bias, *Y, *X;
+  int x_rows;
+  float* C2;
+  float scale;
+  double* sums;
+  float* colsum;        // sum_k A(i, k) per row i of the output, never accumulated
+  // reduction cut into gridDim.z slices: slice z leaves its tile in part[z] (tile-major, column sums behind the 1024 entries) and the last
+  // workgroup to arrive at a tile adds the slices up in slice order.  counters: one zero per tile, zero again afterwards.
+  float* part;
+  unsigned* counters;
+};
+constexpr int kTilePart = 1024 + 32;
+
+// C(i, j) (+)= sum_k A(i, k) B(k, j) in fp32 on the matrix cores, for the discriminator's batches of a thousand rows or so: a
+// 32 x 32 tile per workgroup, whose wavefronts cut the reduction between them, each straight from memory into registers (a chunk
+// of 32 steps' loads in flight under the previous chunk's 16 v_mfma_f32_32x32x2_f32), and add their tiles up in LDS.  A product of
+// 1024 x 256 x 256 is then 256 workgroups and one memory latency plus 0.9 us of matrix work; 64 x 64 tiles with the whole
+// reduction behind one barrier per 16 steps left it on 64 CUs for 22 us.
 // A_KC: A is stored (i, k) with k contiguous, otherwise (k, i); B_KC: B is stored (j, k) with k contiguous, otherwise (k, j).
-// gridDim.z cuts the k range into slices of kslice; with more than one slice, slice z writes its partial product (M, N)
-// densely to C + z * M * N and sum_slices_kernel adds them up in a fixed order.
-template <bool A_KC, bool B_KC>
-__global__ __launch_bounds__(256) void sgemm_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
-                                                    const float* __restrict__ B, int64_t ldb, float* __restrict__ C, int64_t ldc,
-                                                    int kslice, const float* __restrict__ bias, int act, int accumulate) {
-  __shared__ float As[16][68];
-  __shared__ float Bs[16][68];
-  const int t = threadIdx.x, i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-  const int kbeg = blockIdx.z * kslice, kend = min(K, kbeg + kslice);
-  const int wave = t >> 6, lane = t & 63, c = lane & 31, h = lane >> 5;
-  const int wi = (wave >> 1) * 32, wj = (wave & 1) * 32;
+// A lane of half h feeds steps k = 8 (s / 4) + 4 h + s % 4 of a chunk, so that k-contiguous rows are read 16 bytes at a time.
+template <bool KC>
+__device__ __forceinline__ void sgemm_fetch(float (&v)[16], const float* __restrict__ p, const float* __restrict__ p2, int split, int64_t ld,
+                                            int k0, int kend, int h, bool wide) {
+  if (k0 + 32 <= kend && (KC || k0 + 32 <= split || k0 >= split)) {  // a whole chunk of one array: no checks per load
+    if (KC) {
+      const float* q = p + k0 + 4 * h;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (wide) {
+          const float4 t = *reinterpret_cast<const float4*>(q + 8 * s);
+          v[4 * s] = t.x; v[4 * s + 1] = t.y; v[4 * s + 2] = t.z; v[4 * s + 3] = t.w;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[4 * s + e] = q[8 * s + e];
+        }
+      }
+    } else {
+      const float* q = (k0 >= split ? p2 + (int64_t)(k0 - split) * ld : p + (int64_t)k0 * ld) + 4 * h * ld;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) v[s] = q[(8 * (s >> 2) + (s & 3)) * ld];
+    }
+    return;
+  }
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const int k = k0 + 8 * (s >> 2) + 4 * h + (s & 3);
+    float x = 0.f;
+    if (k < kend) x = KC ? p[k] : (k < split ? p[(int64_t)k * ld] : p2[(int64_t)(k - split) * ld]);
+    v[s] = x;
+  }
+}
+
+template <bool A_KC, bool B_KC, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
+  constexpr int RW = WAVES > 8 ? 8 : WAVES;  // tiles held in LDS at a time
+  __shared__ float red[RW][1024];
+  __shared__ float cred[WAVES][64];
+  __shared__ double sred[WAVES];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
+  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
+  const int zbeg = blockIdx.z * g.kslice, zend = min(g.K, zbeg + g.kslice);
+  const int per = ((zend - zbeg + WAVES - 1) / WAVES + 7) / 8 * 8;
+  const int kbeg = zbeg + wave * per, kend = min(zend, kbeg + per);
+  // rows and columns past the matrix repeat the last one; their results are not stored
+  const int ia = min(i0 + c, g.M - 1), jb = min(j0 + c, g.N - 1);
+  const float *pa, *pa2 = nullptr, *pb, *pb2 = nullptr;
+  if (A_KC) pa = ia < g.a_split ? g.A + (int64_t)ia * g.lda : g.A2 + (int64_t)(ia - g.a_split) * g.lda;
+  else { pa = g.A + ia; pa2 = g.A2 + ia; }
+  if (B_KC) pb = g.B + (int64_t)jb * g.ldb;
+  else { pb = g.B + jb; pb2 = g.B2 + jb; }
+  const bool wa = A_KC && g.lda % 4 == 0 && (((uintptr_t)g.A | (uintptr_t)g.A2) & 15) == 0;  // kbeg is a multiple of 8
+  const bool wb = B_KC && g.ldb % 4 == 0 && ((uintptr_t)g.B & 15) == 0;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  for (int k0 = kbeg; k0 < kend; k0 += 16) {
+  float cs = 0.f;
+  float a[16], b[16];
+  if (kbeg < kend) {
+    sgemm_fetch<A_KC>(a, pa, pa2, g.a_split, g.lda, kbeg, kend, h, wa);
+    sgemm_fetch<B_KC>(b, pb, pb2, g.b_split, g.ldb, kbeg, kend, h, wb);
+  }
+  for (int k0 = kbeg; k0 < kend; k0 += 32) {
+    float a1[16], b1[16];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int ka = A_KC ? t % 16 : t / 64 + 4 * r, ia = A_KC ? t / 16 + 16 * r : t % 64;
-      const int gi = i0 + ia, gka = k0 + ka;
-      As[ka][ia] = (gi < M && gka < kend) ? (A_KC ? A[(int64_t)gi * lda + gka] : A[(int64_t)gka * lda + gi]) : 0.f;
-      const int kb = B_KC ? t % 16 : t / 64 + 4 * r, jb = B_KC ? t / 16 + 16 * r : t % 64;
-      const int gj = j0 + jb, gkb = k0 + kb;
-      Bs[kb][jb] = (gj < N && gkb < kend) ? (B_KC ? B[(int64_t)gj * ldb + gkb] : B[(int64_t)gkb * ldb + gj]) : 0.f;
+    for (int s = 0; s < 16; ++s) a1[s] = b1[s] = 0.f;
+    if (k0 + 32 < kend) {
+      sgemm_fetch<A_KC>(a1, pa, pa2, g.a_split, g.lda, k0 + 32, kend, h, wa);
+      sgemm_fetch<B_KC>(b1, pb, pb2, g.b_split, g.ldb, k0 + 32, kend, h, wb);
     }
-    __syncthreads();
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[2 * s + h][wi + c], Bs[2 * s + h][wj + c], acc, 0, 0, 0);
+    for (int s = 0; s < 16; ++s) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+      cs += a[s];
+    }
+#pragma unroll
+    for (int s = 0; s < 16; ++s) { a[s] = a1[s]; b[s] = b1[s]; }
+  }
+  cred[wave][lane] = cs;
+  if (WAVES > RW) {  // the upper half's tiles first, added by the lower half
+    if (wave >= RW)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[wave - RW][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + c] = acc[r];
+    __syncthreads();
+    if (wave < RW)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + c];
     __syncthreads();
   }
-  const bool sliced = gridDim.z > 1;
-  float* out = sliced ? C + (int64_t)blockIdx.z * M * N : C;
-  const int64_t ld = sliced ? N : ldc;
-  const int gj = j0 + wj + c;
-  if (gj >= N) return;
-  const float bj = (!sliced && bias) ? bias[gj] : 0.f;
+  if (wave < RW)
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int gi = i0 + wi + 8 * g + 4 * h + e;
-      if (gi >= M) continue;
-      float v = acc[4 * g + e];
-      if (!sliced) {
-        v += bj;
-        if (act == KS_ACT_ELU) v = v > 0.f ? v : expm1f(v);
-        else if (act == KS_ACT_RELU) v = fmaxf(v, 0.f);
-        else if (act == KS_ACT_TANH) v = tanhf(v);
-        if (accumulate) v += out[(int64_t)gi * ld + gj];
-      }
-      out[(int64_t)gi * ld + gj] = v;
+    for (int r = 0; r < 16; ++r) red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + c] = acc[r];
+  __syncthreads();
+  const bool sliced = gridDim.z > 1, want_cs = g.colsum && blockIdx.x == 0;
+  const int tile = blockIdx.y * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y;
+  float csum = 0.f;
+  if (want_cs && threadIdx.x < 32)
+    for (int w = 0; w < WAVES; ++w) csum += cred[w][threadIdx.x] + cred[w][threadIdx.x + 32];
+  if (sliced) {
+    float* mine = g.part + ((int64_t)blockIdx.z * tiles + tile) * kTilePart;
+    for (int x = threadIdx.x; x < 1024; x += 64 * WAVES) {
+      float v = 0.f;
+      for (int w = 0; w < RW; ++w) v += red[w][x];
+      device_store(mine + x, v);
     }
+    if (want_cs && threadIdx.x < 32) device_store(mine + 1024 + threadIdx.x, csum);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's part has reached memory
+    __syncthreads();
+    __shared__ unsigned last;
+    if (threadIdx.x == 0) last = atomicAdd(&g.counters[tile], 1u) == gridDim.z - 1;
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) g.counters[tile] = 0;
+    for (int x = threadIdx.x; x < kTilePart; x += 64 * WAVES) {
+      float v = 0.f;
+      for (int z = 0; z < (int)gridDim.z; ++z) v += device_load(g.part + ((int64_t)z * tiles + tile) * kTilePart + x);
+      if (x < 1024) red[0][x] = v;
+      else csum = v;  // x = 1024 + thread: the tile is a whole number of passes
+    }
+    __syncthreads();
+  }
+  if (want_cs && threadIdx.x < 32 && i0 + (int)threadIdx.x < g.M) g.colsum[i0 + threadIdx.x] = csum;
+  double sq = 0.0;
+#pragma unroll
+  for (int x = threadIdx.x; x < 1024; x += 64 * WAVES) {
+    const int il = x >> 5, jl = x & 31, i = i0 + il, j = j0 + jl;
+    float v = 0.f;
+    for (int w = 0; w < (sliced ? 1 : RW); ++w) v += red[w][x];
+    if (i >= g.M || j >= g.N) continue;
+    const int64_t o = (int64_t)i * g.ldc + j;
+    float d1 = 1.f, d2 = 0.f;
+    if (g.epi == kEpiDelta || g.epi == kEpiTangent || g.epi == kEpiDz) act_derivatives(g.act, g.Y[o], d1, d2);
+    switch (g.epi) {
+      case kEpiLayer:
+        v += g.bias[j];
+        if (g.act == KS_ACT_ELU) v = v > 0.f ? v : expm1f(v);
+        else if (g.act == KS_ACT_RELU) v = fmaxf(v, 0.f);
+        else if (g.act == KS_ACT_TANH) v = tanhf(v);
+        g.C[o] = v;
+        break;
+      case kEpiDelta: g.C[o] = v; g.C2[o] = d1 * v; break;
+      case kEpiPenalty: g.C[o] = g.scale * v; sq += (double)v * v; break;
+      case kEpiTangent: g.C2[o] = v * g.X[o] * d2; g.C[o] = v * d1; break;
+      case kEpiDz: v *= d1; if (i < g.x_rows) v += g.X[o]; g.C[o] = v; break;
+      default: g.C[o] = g.accumulate ? g.C[o] + v : v;
+    }
+  }
+  if (g.sums) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sq += __shfl_down(sq, d);
+    if (lane == 0) sred[wave] = sq;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int w = 0; w < WAVES; ++w) t += sred[w];
+      g.sums[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+    }
+  }
 }
 
 // The same product for the weight and bias gradients of wide layers, C(i, j) (+)= sum_k A(k, i) B(k, j) with both operands
@@ -2202,28 +2355,17 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(int M, int N, int nz, c
   C[(int64_t)i * ldc + j] = accumulate ? C[(int64_t)i * ldc + j] + s : s;
 }
 
-__global__ __launch_bounds__(256) void fill_kernel(int64_t n, float v, float* __restrict__ p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx < n) p[idx] = v;
-}
-
-// first and second derivative of the activation from its output y = f(z)
-__device__ __forceinline__ void act_derivatives(int act, float y, float& d1, float& d2) {
-  d1 = 1.f; d2 = 0.f;
-  if (act == KS_ACT_ELU) { if (y <= 0.f) { d1 = y + 1.f; d2 = y + 1.f; } }  // exp(z) = elu(z) + 1 for z <= 0
-  else if (act == KS_ACT_RELU) d1 = y > 0.f ? 1.f : 0.f;
-  else if (act == KS_ACT_TANH) { d1 = 1.f - y * y; d2 = -2.f * y * d1; }
-}
-
 // dz = out - target (target +1 on the first n_real rows, -1 on the rest) and the two squared-error sums (one workgroup)
 __global__ __launch_bounds__(1024) void disc_signal_kernel(int64_t n_real, int64_t n, const float* __restrict__ out, float* __restrict__ dz,
+                                                           float* __restrict__ ones, unsigned* __restrict__ counters,
                                                            float* __restrict__ losses) {
   __shared__ double sh[2][1024];
+  if (threadIdx.x < 512) counters[threadIdx.x] = 0;
   double a = 0.0, b = 0.0;
   for (int64_t i = threadIdx.x; i < n; i += 1024) {
     const float e = out[i] - (i < n_real ? 1.f : -1.f);
     dz[i] = e;
-    if (i < n_real) a += 0.5 * (double)e * e; else b += 0.5 * (double)e * e;
+    if (i < n_real) { ones[i] = 1.f; a += 0.5 * (double)e * e; } else b += 0.5 * (double)e * e;
   }
   sh[0][threadIdx.x] = a; sh[1][threadIdx.x] = b;
   __syncthreads();
@@ -2231,60 +2373,21 @@ __global__ __launch_bounds__(1024) void disc_signal_kernel(int64_t n_real, int64
     if ((int)threadIdx.x < w) { sh[0][threadIdx.x] += sh[0][threadIdx.x + w]; sh[1][threadIdx.x] += sh[1][threadIdx.x + w]; }
     __syncthreads();
   }
-  if (threadIdx.x == 0) { losses[0] = (float)sh[0][0]; losses[1] = (float)sh[1][0]; }
+  if (threadIdx.x == 0) { losses[0] = (float)sh[0][0]; losses[1] = (float)sh[1][0]; losses[2] = 0.f; }
 }
 
-// penalty value coef / 2 * sum g^2 / n_motions and, in place, its gradient v = coef / n_motions * g (one workgroup)
-__global__ __launch_bounds__(1024) void disc_penalty_kernel(int64_t n, float coef, float inv_motions, float* __restrict__ g,
-                                                            float* __restrict__ loss) {
-  __shared__ double sh[1024];
+// penalty value: factor * the sum of the tiles' sums of squares, in a fixed order (one workgroup)
+__global__ __launch_bounds__(256) void disc_penalty_kernel(int64_t n, double factor, const double* __restrict__ sums, float* __restrict__ loss) {
+  __shared__ double sh[256];
   double a = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    const float v = g[i];
-    a += (double)v * v;
-    g[i] = coef * inv_motions * v;
-  }
+  for (int64_t i = threadIdx.x; i < n; i += 256) a += sums[i];
   sh[threadIdx.x] = a;
   __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
+  for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *loss = (float)(0.5 * coef * inv_motions * sh[0]);
-}
-
-// d = f'(y) * a
-__global__ __launch_bounds__(256) void disc_delta_kernel(int64_t n, int act, const float* __restrict__ y, const float* __restrict__ a,
-                                                         float* __restrict__ d) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= n) return;
-  float d1, d2;
-  act_derivatives(act, y[idx], d1, d2);
-  d[idx] = d1 * a[idx];
-}
-
-// v = u * f'(y), r = u * a * f''(y)
-__global__ __launch_bounds__(256) void disc_tangent_kernel(int64_t n, int act, const float* __restrict__ y, const float* __restrict__ a,
-                                                           const float* __restrict__ u, float* __restrict__ v, float* __restrict__ r) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= n) return;
-  float d1, d2;
-  act_derivatives(act, y[idx], d1, d2);
-  const float uu = u[idx];
-  v[idx] = uu * d1;
-  r[idx] = uu * a[idx] * d2;
-}
-
-// dz = dy * f'(y) (+ r on the first n_extra elements)
-__global__ __launch_bounds__(256) void disc_dz_kernel(int64_t n, int64_t n_extra, int act, const float* __restrict__ y,
-                                                      const float* __restrict__ r, float* __restrict__ dz) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= n) return;
-  float d1, d2;
-  act_derivatives(act, y[idx], d1, d2);
-  float v = dz[idx] * d1;
-  if (idx < n_extra) v += r[idx];
-  dz[idx] = v;
+  if (threadIdx.x == 0) *loss = (float)(factor * sh[0]);
 }
 
 }  // namespace ks
@@ -2296,8 +2399,12 @@ struct DiscWs {
   float* a[KS_MAX_LAYERS];      // real rows: W_{l+1}^T d_{l+1}
   float* d[KS_MAX_LAYERS];      // real rows: d_l
   float* r[KS_MAX_LAYERS];      // real rows: extra gradient of z_l
-  float *out, *dz0, *dz1, *g, *u, *v, *ones, *part, *colpart;
+  float *out, *dz0, *dz1, *g, *u, *v, *ones, *part;
+  unsigned* counters;
+  double* sums;                 // one sum of squares per tile of the input gradient
 };
+
+static int64_t disc_penalty_tiles(const DevMlp& m, int64_t R) { return ((R + 31) / 32) * ((m.dims[0] + 31) / 32); }
 
 static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, DiscWs* ws) {
   int64_t off = 0;
@@ -2309,9 +2416,7 @@ static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, Dis
   DiscWs w;
   std::memset(&w, 0, sizeof(w));
   int wmax = 1;
-  int64_t maxw = 1;
   for (int l = 0; l <= m.n_layers; ++l) wmax = m.dims[l] > wmax ? m.dims[l] : wmax;
-  for (int l = 0; l < m.n_layers; ++l) maxw = (int64_t)m.dims[l] * m.dims[l + 1] > maxw ? (int64_t)m.dims[l] * m.dims[l + 1] : maxw;
   for (int l = 0; l + 1 < m.n_layers; ++l) {
     w.y[l] = take(M * m.dims[l + 1]);
     w.a[l] = take(R * m.dims[l + 1]);
@@ -2324,65 +2429,57 @@ static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, Dis
   w.g = take(R * m.dims[0]);
   w.u = take(R * wmax);
   w.v = take(R * wmax);
-  w.ones = take(M);
-  w.part = take(kDiscMaxSlices * maxw);
-  w.colpart = take((int64_t)kDiscMaxSlices * wmax);
+  w.ones = take(R);
+  w.sums = (double*)take(2 * disc_penalty_tiles(m, R));
+  w.part = take((int64_t)512 * kTilePart);  // a sliced product has at most 512 (slice, tile) pairs
+  w.counters = (unsigned*)take(512);
   if (ws) *ws = w;
   return off;
 }
 
-// launches one product; cuts the k range when the output alone would leave most of the chip idle
-// colsum / colpart (wide row reductions only): colsum (M) += sum_k A(k, i) from the same pass, colpart its (slices, M) partials
+static void launch_sum_slices(hipStream_t s, int M, int N, int slices, const float* part, float* C, int64_t ldc, bool accumulate) {
+  const int64_t n = (int64_t)M * N;
+  hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, N, slices, part, C, ldc, accumulate ? 1 : 0);
+}
+
+// One product of sgemm_kernel; g.kslice is set here.  Products over activations have reductions of a layer's width: four wavefronts
+// share one.  Weight gradients (both operands stored (k, .)) reduce over the rows, sixteen wavefronts to a workgroup, and are cut into
+// slices while their few tiles leave CUs idle and a slice keeps the 512 rows that give every wavefront one chunk of loads.
 template <bool A_KC, bool B_KC>
-static void sgemm(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                  int64_t ldc, const float* bias, int act, bool accumulate, float* part, float* colsum, float* colpart) {
-  if (M <= 0 || N <= 0 || K <= 0) return;  // every caller with an empty sum adds into its output
-  if (!A_KC && !B_KC && M == 1 && N >= 128 && !bias && act == KS_ACT_NONE) {
-    // one output row: the same numbers as the (N, 1) product with the operands exchanged, which takes the wide path below
-    sgemm<false, false>(s, N, 1, K, B, ldb, A, lda, C, 1, nullptr, KS_ACT_NONE, accumulate, part);
-    return;
-  }
-  if (!A_KC && !B_KC && M >= 128 && !bias && act == KS_ACT_NONE) {  // gradients of wide layers: long reductions over the rows
-    const int vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0;
-    const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    int slices = 1;
-    if (part && K >= 2048) {
-      slices = (int)((512 + tiles - 1) / tiles);
-      if (slices > kDiscMaxSlices) slices = kDiscMaxSlices;
-      if ((int64_t)slices * 256 > K) slices = (int)(K / 256);
-    }
-    int kslice = (int)((K + slices - 1) / slices);
-    kslice = (kslice + 15) / 16 * 16;
-    slices = (int)((K + kslice - 1) / kslice);
-    hipLaunchKernelGGL(sgemm_tn128_kernel, dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128), (unsigned)slices), dim3(256), 0, s,
-                       (int)M, N, (int)K, A, lda, B, ldb, slices > 1 ? part : C, ldc, kslice, accumulate ? 1 : 0, vec_a, vec_b,
-                       colsum ? (slices > 1 ? colpart : colsum) : (float*)nullptr);
-    if (slices > 1) {
-      const int64_t n = M * N;
-      hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (int)M, N, slices, part, C, ldc, accumulate ? 1 : 0);
-      if (colsum)
-        hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, s, (int)M, 1, slices, colpart, colsum, (int64_t)1,
-                           accumulate ? 1 : 0);
-    }
-    return;
-  }
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+static void sgemm_go(hipStream_t s, SgemmArgs g) {
+  if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
+  if (!g.A2) { g.A2 = g.A; g.a_split = 0x7fffffff; }
+  if (!g.B2) { g.B2 = g.B; g.b_split = 0x7fffffff; }
+  constexpr bool TN = !A_KC && !B_KC;
+  const dim3 tiles((unsigned)((g.N + 31) / 32), (unsigned)((g.M + 31) / 32));
   int slices = 1;
-  if (part && tiles < 128 && K >= 2048) {
-    slices = (int)((K + 511) / 512);
-    const int64_t want = (512 + tiles - 1) / tiles;
-    if (slices > want) slices = (int)want;
+  if (TN && g.part)
+    while (slices < kDiscMaxSlices && g.K >= 1024 * slices && tiles.x * tiles.y * slices * 2 <= 512) slices *= 2;
+  g.kslice = (((g.K + slices - 1) / slices) + 15) / 16 * 16;
+  slices = (g.K + g.kslice - 1) / g.kslice;
+  hipLaunchKernelGGL((sgemm_kernel<A_KC, B_KC, TN ? 16 : 4>), dim3(tiles.x, tiles.y, (unsigned)slices), dim3(TN ? 1024 : 256), 0, s, g);
+}
+
+// C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single wide
+// fp32 layer.  The rows are cut so that about 512 workgroups share them.
+static void sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                        int64_t ldc, float* part, float* colsum, float* colpart) {
+  const int vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0;
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  int slices = 1;
+  if (K >= 2048) {
+    slices = (int)((512 + tiles - 1) / tiles);
     if (slices > kDiscMaxSlices) slices = kDiscMaxSlices;
+    if ((int64_t)slices * 256 > K) slices = (int)(K / 256);
   }
   int kslice = (int)((K + slices - 1) / slices);
   kslice = (kslice + 15) / 16 * 16;
   slices = (int)((K + kslice - 1) / kslice);
-  if (slices < 1) slices = 1;
-  hipLaunchKernelGGL((sgemm_kernel<A_KC, B_KC>), dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)slices), dim3(256), 0, s,
-                     (int)M, N, (int)K, A, lda, B, ldb, slices > 1 ? part : C, ldc, kslice, bias, act, accumulate ? 1 : 0);
+  hipLaunchKernelGGL(sgemm_tn128_kernel, dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128), (unsigned)slices), dim3(256), 0, s,
+                     (int)M, N, (int)K, A, lda, B, ldb, slices > 1 ? part : C, ldc, kslice, 0, vec_a, vec_b, slices > 1 ? colpart : colsum);
   if (slices > 1) {
-    const int64_t n = M * N;
-    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (int)M, N, slices, part, C, ldc, accumulate ? 1 : 0);
+    launch_sum_slices(s, (int)M, N, slices, part, C, ldc, false);
+    launch_sum_slices(s, (int)M, 1, slices, colpart, colsum, 1, false);
   }
 }
 
@@ -2408,73 +2505,73 @@ extern "C" int ks_mlp_disc_loss_grad(KsMlp* h, ks_stream_t stream, int64_t n_rea
   hipStream_t s = (hipStream_t)stream;
   DiscWs ws;
   carve_disc(m, R, M, (char*)workspace, &ws);
-  auto blocks = [](int64_t n) { return dim3((unsigned)((n + 255) / 256)); };
-  for (int l = 0; l < L; ++l) {  // everything below adds into the gradient buffers
-    const int64_t nw = (int64_t)m.npad[l] * m.kpad[l];
-    hipLaunchKernelGGL(fill_kernel, blocks(nw), dim3(256), 0, s, nw, 0.f, m.gW[l]);
-    hipLaunchKernelGGL(fill_kernel, blocks(m.npad[l]), dim3(256), 0, s, (int64_t)m.npad[l], 0.f, m.gb[l]);
-  }
-  hipLaunchKernelGGL(fill_kernel, blocks(M), dim3(256), 0, s, M, 1.f, ws.ones);
-  hipLaunchKernelGGL(fill_kernel, dim3(1), dim3(256), 0, s, (int64_t)3, 0.f, losses);
-
+  SgemmArgs z = {};  // fields left out below are zero
   // forward over the real rows, then the simulated ones
   for (int l = 0; l < L; ++l) {
     const bool last = l == L - 1;
-    float* outp = last ? ws.out : ws.y[l];
-    const int n = m.dims[l + 1], k = m.dims[l];
-    const int a_l = last ? KS_ACT_NONE : act;
-    if (l == 0) {
-      sgemm<true, true>(s, R, n, k, real, k, m.mW[0], m.kpad[0], outp, n, m.mb[0], a_l, false, nullptr);
-      sgemm<true, true>(s, n_sim, n, k, sim, k, m.mW[0], m.kpad[0], outp + R * n, n, m.mb[0], a_l, false, nullptr);
-    } else {
-      sgemm<true, true>(s, M, n, k, ws.y[l - 1], k, m.mW[l], m.kpad[l], outp, n, m.mb[l], a_l, false, nullptr);
-    }
+    SgemmArgs g = z;
+    g.M = (int)M; g.N = m.dims[l + 1]; g.K = m.dims[l];
+    if (l > 0) g.A = ws.y[l - 1];
+    else if (R == 0 || n_sim == 0) g.A = R ? real : sim;
+    else { g.A = real; g.A2 = sim; g.a_split = (int)R; }
+    g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l];
+    g.C = last ? ws.out : ws.y[l]; g.ldc = g.N; g.bias = m.mb[l]; g.epi = kEpiLayer; g.act = last ? KS_ACT_NONE : act;
+    sgemm_go<true, true>(s, g);
   }
-  hipLaunchKernelGGL(disc_signal_kernel, dim3(1), dim3(1024), 0, s, R, M, ws.out, ws.dz0, losses);
+  hipLaunchKernelGGL(disc_signal_kernel, dim3(1), dim3(1024), 0, s, R, M, ws.out, ws.dz0, ws.ones, ws.counters, losses);
 
   if (penalty) {
-    // input gradient on the real rows: d_L = 1, down to g = d_1 W_1
+    // input gradient on the real rows: d_L = 1, down to g = d_1 W_1, which leaves its tiles as the penalty's gradient
     const float* dnext = ws.ones;
-    for (int l = L - 1; l >= 1; --l) {  // hidden layer l (its output is y[l - 1])
-      const int n = m.dims[l], k = m.dims[l + 1];
-      sgemm<true, false>(s, R, n, k, dnext, k, m.mW[l], m.kpad[l], ws.a[l - 1], n, nullptr, KS_ACT_NONE, false, nullptr);
-      hipLaunchKernelGGL(disc_delta_kernel, blocks(R * n), dim3(256), 0, s, R * n, act, ws.y[l - 1], ws.a[l - 1], ws.d[l - 1]);
-      dnext = ws.d[l - 1];
+    for (int l = L - 1; l >= 0; --l) {  // hidden layer l (its output is y[l - 1]); l = 0: the input
+      SgemmArgs g = z;
+      g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l + 1];
+      g.A = dnext; g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l]; g.ldc = g.N; g.act = act;
+      if (l > 0) { g.C = ws.a[l - 1]; g.C2 = ws.d[l - 1]; g.Y = ws.y[l - 1]; g.epi = kEpiDelta; dnext = ws.d[l - 1]; }
+      else { g.C = ws.g; g.epi = kEpiPenalty; g.scale = grad_penalty_coef * (1.f / (float)n_motions); g.sums = ws.sums; }
+      sgemm_go<true, false>(s, g);
     }
-    sgemm<true, false>(s, R, m.dims[0], m.dims[1], dnext, m.dims[1], m.mW[0], m.kpad[0], ws.g, m.dims[0], nullptr, KS_ACT_NONE, false, nullptr);
-    hipLaunchKernelGGL(disc_penalty_kernel, dim3(1), dim3(1024), 0, s, R * m.dims[0], grad_penalty_coef, 1.f / (float)n_motions, ws.g,
-                       losses + 2);
-    // the sweep back through that computation, first layer to last
+    hipLaunchKernelGGL(disc_penalty_kernel, dim3(1), dim3(256), 0, s, disc_penalty_tiles(m, R),
+                       0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions), ws.sums, losses + 2);
+    // the sweep back through that computation, first layer to last; its share opens every weight gradient
     const float* prev = ws.g;
-    float *u = ws.u, *v = ws.v;
+    float* v = ws.v;
     for (int l = 1; l <= L; ++l) {
       const int n = m.dims[l], k = m.dims[l - 1];
-      const float* dl = l == L ? ws.ones : ws.d[l - 1];
-      sgemm<false, false>(s, n, k, R, dl, n, prev, k, m.gW[l - 1], m.kpad[l - 1], nullptr, KS_ACT_NONE, true, ws.part);
+      SgemmArgs g = z;
+      g.M = n; g.N = k; g.K = (int)R; g.A = l == L ? ws.ones : ws.d[l - 1]; g.lda = n; g.B = prev; g.ldb = k;
+      g.C = m.gW[l - 1]; g.ldc = m.kpad[l - 1];
+      g.part = ws.part; g.counters = ws.counters;
+      sgemm_go<false, false>(s, g);
       if (l == L) break;
-      sgemm<true, true>(s, R, n, k, prev, k, m.mW[l - 1], m.kpad[l - 1], u, n, nullptr, KS_ACT_NONE, false, nullptr);
-      hipLaunchKernelGGL(disc_tangent_kernel, blocks(R * n), dim3(256), 0, s, R * n, act, ws.y[l - 1], ws.a[l - 1], u, v, ws.r[l - 1]);
-      prev = v;  // the next layer's products read v and write u; only then does its elementwise pass overwrite v
+      g = z;
+      g.M = (int)R; g.N = n; g.K = k; g.A = prev; g.lda = k; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+      g.C = v; g.C2 = ws.r[l - 1]; g.ldc = n; g.Y = ws.y[l - 1]; g.X = ws.a[l - 1]; g.act = act; g.epi = kEpiTangent;
+      sgemm_go<true, true>(s, g);
+      prev = v;
+      v = v == ws.v ? ws.u : ws.v;  // the next product reads this one's result
     }
   }
 
-  // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows
+  // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows; the bias gradients are the
+  // column sums that ride on the weight gradients' pass over dz
   float *dz = ws.dz0, *dnx = ws.dz1;
   for (int l = L; l >= 1; --l) {
     const int n = m.dims[l], k = m.dims[l - 1];
-    // wide layers: the bias gradient (the column sums of dz) rides on the weight gradient's pass over dz
-    const bool with_bias = n >= 128;
-    float* gb = with_bias ? m.gb[l - 1] : nullptr;
-    if (l == 1) {
-      sgemm<false, false>(s, n, k, R, dz, n, real, k, m.gW[0], m.kpad[0], nullptr, KS_ACT_NONE, true, ws.part, gb, ws.colpart);
-      sgemm<false, false>(s, n, k, n_sim, dz + R * n, n, sim, k, m.gW[0], m.kpad[0], nullptr, KS_ACT_NONE, true, ws.part, gb, ws.colpart);
-    } else {
-      sgemm<false, false>(s, n, k, M, dz, n, ws.y[l - 2], k, m.gW[l - 1], m.kpad[l - 1], nullptr, KS_ACT_NONE, true, ws.part, gb, ws.colpart);
-    }
-    if (!with_bias) sgemm<false, false>(s, n, 1, M, dz, n, ws.ones, 1, m.gb[l - 1], 1, nullptr, KS_ACT_NONE, true, ws.part);
+    SgemmArgs g = z;
+    g.M = n; g.N = k; g.K = (int)M; g.A = dz; g.lda = n; g.ldb = k;
+    if (l > 1) g.B = ws.y[l - 2];
+    else if (R == 0 || n_sim == 0) g.B = R ? real : sim;
+    else { g.B = real; g.B2 = sim; g.b_split = (int)R; }
+    g.C = m.gW[l - 1]; g.ldc = m.kpad[l - 1]; g.accumulate = penalty ? 1 : 0;  // the weight gradient may hold the penalty's share
+    g.colsum = m.gb[l - 1];
+    g.part = ws.part; g.counters = ws.counters;
+    sgemm_go<false, false>(s, g);
     if (l == 1) break;
-    sgemm<true, false>(s, M, k, n, dz, n, m.mW[l - 1], m.kpad[l - 1], dnx, k, nullptr, KS_ACT_NONE, false, nullptr);
-    hipLaunchKernelGGL(disc_dz_kernel, blocks(M * k), dim3(256), 0, s, M * k, penalty ? R * k : (int64_t)0, act, ws.y[l - 2], ws.r[l - 2], dnx);
+    g = z;
+    g.M = (int)M; g.N = k; g.K = n; g.A = dz; g.lda = n; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+    g.C = dnx; g.ldc = k; g.Y = ws.y[l - 2]; g.X = ws.r[l - 2]; g.x_rows = penalty ? (int)R : 0; g.act = act; g.epi = kEpiDz;
+    sgemm_go<true, false>(s, g);
     float* tmp = dz; dz = dnx; dnx = tmp;
   }
   return check_launch("ks_mlp_disc_loss_grad");
@@ -2500,4 +2597,52 @@ extern "C" int ks_mlp_get_params(const KsMlp* h, ks_stream_t stream, int32_t l, 
     hipLaunchKernelGGL(unpad_kernel, dim3((unsigned)((out + 255) / 256)), dim3(256), 0, (hipStream_t)stream, 1, out, out,
                        gradients ? m.gb[l] : m.mb[l], bias);
   return check_launch("ks_mlp_get_params");
+}
+
+// Every weight and bias of a network in one launch: the caller's layouts one after the other in `out`, entry 2 l / 2 l + 1 = weight /
+// bias of layer l, each starting at a multiple of four floats.
+struct UnpadArgs {
+  int n;
+  int first_block[2 * KS_MAX_LAYERS + 1];
+  int rows[2 * KS_MAX_LAYERS], cols[2 * KS_MAX_LAYERS], ld[2 * KS_MAX_LAYERS];
+  const float* src[2 * KS_MAX_LAYERS];
+  int64_t dst[2 * KS_MAX_LAYERS];
+};
+__global__ __launch_bounds__(256) void unpad_net_kernel(UnpadArgs a, float* __restrict__ out) {
+  int e = 0;
+  while (e + 1 < a.n && (int)blockIdx.x >= a.first_block[e + 1]) ++e;
+  const int64_t total = (int64_t)a.rows[e] * a.cols[e];
+  const int64_t idx = ((int64_t)blockIdx.x - a.first_block[e]) * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const int r = (int)(idx / a.cols[e]), c = (int)(idx - (int64_t)r * a.cols[e]);
+  out[a.dst[e] + idx] = a.src[e][(int64_t)r * a.ld[e] + c];
+}
+
+extern "C" int64_t ks_mlp_param_floats(const KsMlp* h, int32_t layer) {
+  if (!h || layer < 0 || layer > h->m.n_layers) return -1;
+  int64_t off = 0;
+  for (int l = 0; l < layer; ++l)
+    off += ((int64_t)h->m.dims[l] * h->m.dims[l + 1] + 3) / 4 * 4 + ((int64_t)h->m.dims[l + 1] + 3) / 4 * 4;
+  return off;
+}
+
+extern "C" int ks_mlp_get_all_params(const KsMlp* h, ks_stream_t stream, float* out, int32_t gradients) {
+  if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_get_all_params: call ks_mlp_train_init first");
+  if (!out) return fail(KS_EINVAL, "ks_mlp_get_all_params: null pointer");
+  const DevMlp& m = h->m;
+  UnpadArgs a;
+  a.n = 2 * m.n_layers;
+  int blocks = 0;
+  for (int l = 0; l < m.n_layers; ++l) {
+    const int o = m.dims[l + 1], i = m.dims[l];
+    const int64_t off = ks_mlp_param_floats(h, l);
+    const int w = 2 * l, b = 2 * l + 1;
+    a.rows[w] = o; a.cols[w] = i; a.ld[w] = m.kpad[l]; a.src[w] = gradients ? m.gW[l] : m.mW[l]; a.dst[w] = off;
+    a.rows[b] = 1; a.cols[b] = o; a.ld[b] = o; a.src[b] = gradients ? m.gb[l] : m.mb[l]; a.dst[b] = off + ((int64_t)o * i + 3) / 4 * 4;
+    a.first_block[w] = blocks; blocks += (int)(((int64_t)o * i + 255) / 256);
+    a.first_block[b] = blocks; blocks += (o + 255) / 256;
+  }
+  a.first_block[a.n] = blocks;
+  hipLaunchKernelGGL(unpad_net_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, out);
+  return check_launch("ks_mlp_get_all_params");
 }

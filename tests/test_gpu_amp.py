@@ -135,3 +135,38 @@ def test_discriminator_argument_errors():
     clips, starts = torch.randint(0, 4, (6,), generator=g), torch.randint(0, 7, (6,), generator=g)
     want = torch.stack([amp.loop_slice(motions[int(c)], int(s0), 10) for c, s0 in zip(clips, starts)])
     assert batch.shape == (6, 10, 2) and torch.equal(batch, want)
+
+
+@pytest.mark.parametrize("dims,shapes", [((5, 33, 1), ((1, 1), (2, 3))), ((71, 128, 96, 1), ((3, 11), (1, 33))), ((64, 32, 1), ((4, 8), (0, 1))),
+                                         ((64, 32, 1), ((0, 1), (4, 8))), ((40, 256, 64, 1), ((2, 700), (3, 1000)))])
+def test_discriminator_gradient_at_the_edges_of_its_tiles(dims, shapes):
+    """Rows and widths around the 32 x 32 tiles and the 32-step chunks of the products, frames that are not 16-byte rows, either set
+    of motions empty, and row counts that cut the weight gradients into slices.  fp32 against float64 autograd: sums of up to 4400
+    rows, each rounded at 2^-24 of its size."""
+    from ksim_amd.mlp import random_mlp
+
+    rng = np.random.default_rng(sum(dims))
+    net, ws, bs = random_mlp(dims, 3, dtype="f32")
+    net.train_init()
+    real, sim = (rng.normal(size=(*s, dims[0])) for s in shapes)
+    losses = net.disc_loss_grad(torch.tensor(real, dtype=torch.float32, device=DEV), torch.tensor(sim, dtype=torch.float32, device=DEV), 10.0)
+    tw, tb = [torch.tensor(w, dtype=torch.float64, requires_grad=True) for w in ws], [torch.tensor(b, dtype=torch.float64, requires_grad=True) for b in bs]
+
+    def score(x):
+        for i, (w, b) in enumerate(zip(tw, tb)):
+            x = x @ w.T + b
+            x = torch.nn.functional.elu(x) if i + 1 < len(tw) else x
+        return x[..., 0]
+
+    r, s = torch.tensor(real, requires_grad=True), torch.tensor(sim)
+    out = score(r)
+    terms = [0.5 * ((out - 1) ** 2).sum(), 0.5 * ((score(s) + 1) ** 2).sum(), torch.zeros((), dtype=torch.float64)]
+    if real.size:
+        g, = torch.autograd.grad(out.sum(), r, create_graph=True)
+        terms[2] = 5.0 * (g ** 2).sum() / real.shape[0]
+    sum(terms).backward()
+    for got, want in zip(losses.tolist(), terms):
+        assert abs(got - want.item()) <= 1e-5 * max(1.0, abs(want.item()))
+    for (gw, gb), w, b in zip(net.parameters(gradients=True), tw, tb):
+        for got, want in ((gw, w.grad), (gb, b.grad)):
+            assert np.abs(got.cpu().numpy() - want.numpy()).max() <= 2e-5 * max(np.abs(want.numpy()).max(), 1e-3)
