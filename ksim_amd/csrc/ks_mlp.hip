@@ -1581,7 +1581,8 @@ static void refresh_layers(DevMlp& m, hipStream_t s) {
 }
 
 constexpr int kDwSplit = 32;  // most slices the weight-gradient reduction over the rows is cut into
-constexpr int kDiscMaxSlices = 64;  // most slices a long row reduction of the fp32 products (sgemm below) is cut into
+constexpr int kTnMaxSlices = 256;   // most slices of the row reduction of a single fp32 layer's gradient (sgemm_tn128)
+constexpr int kDiscMaxSlices = 64;  // most slices of a weight-gradient product of the discriminator (sgemm_kernel)
 
 // workspace: hidden activations of every layer, two (M, widest) gradient buffers, two transposes (widest, Mp)
 struct TrainWs {
@@ -1632,7 +1633,7 @@ static int64_t carve_train(const DevMlp& m, int64_t M, char* base, TrainWs* ws) 
   for (int l = 0; l < m.n_layers; ++l) maxw = (int64_t)m.npad[l] * m.kpad[l] > maxw ? (int64_t)m.npad[l] * m.kpad[l] : maxw;
   int64_t nparts = kDwSplit * maxw > (int64_t)4 * kColsumSlices * wz ? kDwSplit * maxw : (int64_t)4 * kColsumSlices * wz;
   if (m.n_layers == 1 && esz == 4)  // the one-pass weight and bias gradient of a single fp32 layer: slices of both
-    nparts = nparts > (int64_t)kDiscMaxSlices * (maxw + wz) ? nparts : (int64_t)kDiscMaxSlices * (maxw + wz);
+    nparts = nparts > (int64_t)kTnMaxSlices * (maxw + wz) ? nparts : (int64_t)kTnMaxSlices * (maxw + wz);
   w.part = (float*)take(nparts * 4);
   w.Mp = Mp;
   w.Mp128 = (M + 127) / 128 * 128;
@@ -1783,8 +1784,8 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
   return KS_OK;
 }
 
-static void sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                        int64_t ldc, float* part, float* colsum, float* colpart);
+static int sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                       int64_t ldc, float* part, float* colsum, float* colpart);
 
 template <typename T>
 static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws,
@@ -1834,8 +1835,9 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
       // A single fp32 layer (the projections of the recurrent cells, over all the (step, env) rows of a trajectory slice): the
       // weight gradient dZ^T X and the bias gradient, the column sums of dZ, in one pass over the row-major operands as they
       // are, on the 128 x 128 tiles of the long-reduction product; no transposed copies.
-      float* colpart = ws.part + (int64_t)kDiscMaxSlices * np * kp;
-      sgemm_tn128(s, np, m.dims[0], M, (const float*)dz, np, x, m.dims[0], m.gW[0], kp, ws.part, m.gb[0], colpart);
+      float* colpart = ws.part + (int64_t)kTnMaxSlices * np * kp;
+      const int rc = sgemm_tn128(s, np, m.dims[0], M, (const float*)dz, np, x, m.dims[0], m.gW[0], kp, ws.part, m.gb[0], colpart);
+      if (rc != KS_OK) return rc;
       break;
     }
     if (want_w && !have_bias) {
@@ -2239,21 +2241,38 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
   }
 }
 
-// The same product for the weight and bias gradients of wide layers, C(i, j) (+)= sum_k A(k, i) B(k, j) with both operands
-// stored (k, .) and a long reduction over the rows: a 128 x 128 tile per workgroup (each wavefront a 64 x 64 block = 2 x 2 MFMA tiles, so a value read
-// from LDS feeds two matrix instructions), 16-byte global loads (vec_a / vec_b: the operand's rows are 16-byte aligned) whose
-// next slice is in flight while the matrix cores work on this one.  A narrow B (71 columns, or the single column of ones that
-// makes the product a column sum) wastes matrix work, not memory traffic, which is what bounds these products.  `colsum`
-// (nullable) also receives sum_k A(k, i), the bias gradient that goes with a weight gradient, from the tiles that pass through
-// LDS anyway.  Slices and partial outputs as in sgemm_kernel.
-__global__ __launch_bounds__(256) void sgemm_tn128_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
-                                                          const float* __restrict__ B, int64_t ldb, float* __restrict__ C, int64_t ldc,
-                                                          int kslice, int accumulate, int vec_a, int vec_b,
-                                                          float* __restrict__ colsum) {
-  __shared__ __attribute__((aligned(16))) float As[16][132];
-  __shared__ __attribute__((aligned(16))) float Bs[16][132];
-  const int t = threadIdx.x, i0 = blockIdx.y * 128, j0 = blockIdx.x * 128;
-  const int kbeg = blockIdx.z * kslice, kend = min(K, kbeg + kslice);
+// The same product for the weight and bias gradient of a single wide layer over a hundred thousand rows, C(i, j) = sum_k A(k, i) B(k, j)
+// with both operands stored (k, .): a 128 x 128 tile per workgroup of two groups of four wavefronts; each group takes half of the
+// slice's rows and each of its wavefronts a 64 x 64 block (2 x 2 MFMA tiles, so a value read from LDS feeds two matrix instructions),
+// and the second group's tile is added to the first's at the end.  Loads (16 bytes wide where VA / VB: the operand's rows are
+// 16-byte aligned, its width whole tiles) are two 16-row stages ahead of the matrix work: one in flight in registers, one in the other
+// half of the LDS buffer, so that a stage costs one barrier; a step's LDS reads are issued before the previous step's products.  Two
+// workgroups share a CU: four wavefronts per SIMD.  One group of four with two barriers per stage and one workgroup per CU took 172 us
+// at 102400 x 512 x 128 (78 TFLOP/s), this 130; with the loads left out it takes 118 us, and the matrix instructions alone are 87.
+// `colsum` also receives sum_k A(k, i), the bias gradient, from the registers the tiles pass through anyway.
+// gridDim.y cuts the k range into slices of kslice; with more than one slice, slice z writes its partial product (M, N) densely to
+// C + z * M * N and its column sums to colsum + z * M, and sum_slices_kernel adds them up in a fixed order.
+constexpr int kTnStage = 16 * 132;  // floats of one operand's 16-row stage in LDS
+constexpr int kTnLds = 2 * 2 * 2 * kTnStage * (int)sizeof(float);  // groups x buffers x operands
+template <bool VA, bool VB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void sgemm_tn128_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
+                                             const float* __restrict__ B, int64_t ldb, float* __restrict__ C, int64_t ldc,
+                                             int kslice, float* __restrict__ colsum) {
+  extern __shared__ __attribute__((aligned(16))) float tn_lds[];
+  // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD one after the other (the number of
+  // slices is a multiple of 8 whenever there are several)
+  int tile = blockIdx.x, z = blockIdx.y;
+  if (gridDim.y > 1) {
+    const int l = blockIdx.y * gridDim.x + blockIdx.x, q = l >> 3;
+    tile = q % gridDim.x;
+    z = (q / gridDim.x) * 8 + (l & 7);
+  }
+  const int tiles_n = (N + 127) / 128;
+  const int grp = threadIdx.x >> 8, t = threadIdx.x & 255, i0 = tile / tiles_n * 128, j0 = tile % tiles_n * 128;
+  float* lds = tn_lds + grp * 4 * kTnStage;  // [buffer][operand][16][132]
+  const int zbeg = min(K, z * kslice), zend = min(K, zbeg + kslice);
+  const int half = ((zend - zbeg + 31) / 32) * 16;  // rows per group, in whole stages; both groups run the same number of stages
+  const int kbeg = zbeg + grp * half, kend = min(zend, kbeg + half), stages = half / 16;
   const int wave = t >> 6, lane = t & 63, c = lane & 31, h = lane >> 5;
   const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
   f32x16 acc[2][2];
@@ -2264,60 +2283,104 @@ __global__ __launch_bounds__(256) void sgemm_tn128_kernel(int M, int N, int K, c
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
   float4 ra[2], rb[2];
-  float cs = 0.f;  // colsum: this thread's column of A, summed over the slice
-  // thread t loads rows k = t / 32 and 8 + t / 32 of the slice, four consecutive columns from 4 (t % 32)
+  float4 cs = {0.f, 0.f, 0.f, 0.f};  // this thread's four columns of A, summed over the rows it loads
+  // thread t loads rows k = t / 32 and 8 + t / 32 of a stage, four consecutive columns from 4 (t % 32); columns past the matrix repeat
+  // the last one, their products are not stored
   const int lk = t >> 5, l4 = (t & 31) * 4;
-#define KS_TN_FETCH(K0)                                                                                           \
-  _Pragma("unroll") for (int r = 0; r < 2; ++r) {                                                                 \
-    const int k = (K0) + lk + 8 * r;                                                                              \
-    const int gi = i0 + l4, gj = j0 + l4;                                                                         \
-    ra[r] = float4{0.f, 0.f, 0.f, 0.f};                                                                           \
-    rb[r] = float4{0.f, 0.f, 0.f, 0.f};                                                                           \
-    if (k < kend) {                                                                                               \
-      if (gi + 3 < M && vec_a) ra[r] = *reinterpret_cast<const float4*>(A + (int64_t)k * lda + gi);               \
-      else if (gi < M) {                                                                                          \
-        const float* q = A + (int64_t)k * lda + gi;                                                               \
-        ra[r].x = q[0]; if (gi + 1 < M) ra[r].y = q[1]; if (gi + 2 < M) ra[r].z = q[2]; if (gi + 3 < M) ra[r].w = q[3]; \
-      }                                                                                                           \
-      if (gj + 3 < N && vec_b) rb[r] = *reinterpret_cast<const float4*>(B + (int64_t)k * ldb + gj);               \
-      else if (gj < N) {                                                                                          \
-        const float* q = B + (int64_t)k * ldb + gj;                                                               \
-        rb[r].x = q[0]; if (gj + 1 < N) rb[r].y = q[1]; if (gj + 2 < N) rb[r].z = q[2]; if (gj + 3 < N) rb[r].w = q[3]; \
-      }                                                                                                           \
-    }                                                                                                             \
-  }
-  KS_TN_FETCH(kbeg)
-  for (int k0 = kbeg; k0 < kend; k0 += 16) {
+  const float* pa = A + (int64_t)(kbeg + lk) * lda + (VA ? i0 + l4 : 0);
+  const float* pb = B + (int64_t)(kbeg + lk) * ldb + (VB ? j0 + l4 : 0);
+  int ic[4], jc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { ic[e] = min(i0 + l4 + e, M - 1); jc[e] = min(j0 + l4 + e, N - 1); }
+  auto load4 = [](const float* q, bool vec, const int (&at)[4]) __attribute__((always_inline)) {
+    return vec ? *reinterpret_cast<const float4*>(q) : float4{q[at[0]], q[at[1]], q[at[2]], q[at[3]]};
+  };
+  const int64_t a8 = 8 * lda, b8 = 8 * ldb;
+  auto fetch = [&](int n) __attribute__((always_inline)) {
+    if (kbeg + 16 * n + 16 <= kend) {
+      ra[0] = load4(pa, VA, ic); ra[1] = load4(pa + a8, VA, ic);
+      rb[0] = load4(pb, VB, jc); rb[1] = load4(pb + b8, VB, jc);
+      pa += 2 * a8; pb += 2 * b8;
+    } else {  // the group's last rows, and zeros beyond them
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const int k = kbeg + 16 * n + lk + 8 * r;
+        ra[r] = rb[r] = float4{0.f, 0.f, 0.f, 0.f};
+        if (k < kend) { ra[r] = load4(pa + r * a8, VA, ic); rb[r] = load4(pb + r * b8, VB, jc); }
+      }
+    }
+  };
+  auto put = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-      *reinterpret_cast<float4*>(&As[lk + 8 * r][l4]) = ra[r];
-      *reinterpret_cast<float4*>(&Bs[lk + 8 * r][l4]) = rb[r];
+      *reinterpret_cast<float4*>(lds + buf * 2 * kTnStage + (lk + 8 * r) * 132 + l4) = ra[r];
+      *reinterpret_cast<float4*>(lds + buf * 2 * kTnStage + kTnStage + (lk + 8 * r) * 132 + l4) = rb[r];
+      cs.x += ra[r].x; cs.y += ra[r].y; cs.z += ra[r].z; cs.w += ra[r].w;
     }
-    __syncthreads();
-    KS_TN_FETCH(k0 + 16)  // beyond the slice: zeros that are never stored
-    if (colsum && blockIdx.x == 0 && t < 128) {  // sum_k A(k, i) on the side: the tile is in LDS anyway
-#pragma unroll
-      for (int k = 0; k < 16; ++k) cs += As[k][t];
+  };
+  fetch(0);
+  put(0);
+  fetch(1);
+  __syncthreads();
+  for (int n = 0; n < stages; ++n) {
+    const float* As = lds + (n & 1) * 2 * kTnStage + h * 132 + wi + c;
+    const float* Bs = lds + (n & 1) * 2 * kTnStage + kTnStage + h * 132 + wj + c;
+    float fa[2][2], fb[2][2];
+    fa[0][0] = As[0]; fa[0][1] = As[32]; fb[0][0] = Bs[0]; fb[0][1] = Bs[32];
+    if (n + 1 < stages) {
+      put((n + 1) & 1);  // the stage fetched one step ago, into the half nobody reads until the barrier
+      fetch(n + 2);
     }
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      const float a0 = As[2 * s + h][wi + c], a1 = As[2 * s + h][wi + 32 + c];
-      const float b0 = Bs[2 * s + h][wj + c], b1 = Bs[2 * s + h][wj + 32 + c];
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
+      const int q = s & 1;
+      if (s < 7) {
+        fa[q ^ 1][0] = As[(2 * s + 2) * 132]; fa[q ^ 1][1] = As[(2 * s + 2) * 132 + 32];
+        fb[q ^ 1][0] = Bs[(2 * s + 2) * 132]; fb[q ^ 1][1] = Bs[(2 * s + 2) * 132 + 32];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0], fb[q][0], acc[0][0], 0, 0, 0);
+      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0], fb[q][1], acc[0][1], 0, 0, 0);
+      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1], fb[q][0], acc[1][0], 0, 0, 0);
+      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1], fb[q][1], acc[1][1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
   }
-#undef KS_TN_FETCH
-  const bool sliced = gridDim.z > 1;
-  float* out = sliced ? C + (int64_t)blockIdx.z * M * N : C;
-  const int64_t ld = sliced ? N : ldc;
-  if (colsum && blockIdx.x == 0 && t < 128 && i0 + t < M) {  // sliced: partial row z of (slices, M); else the sums themselves
-    float* q = colsum + (sliced ? (int64_t)blockIdx.z * M : 0) + i0 + t;
-    *q = (!sliced && accumulate) ? *q + cs : cs;
+  // the second group hands its tile over in two halves through the buffers, which are free now
+  float* mine = tn_lds + (wave * 64 + lane) * 33;  // 33: the lanes' rows start in different banks
+  for (int a = 0; a < 2; ++a) {
+    if (grp == 1) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[16 * b + r] = a == 0 ? acc[0][b][r] : acc[1][b][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          if (a == 0) acc[0][b][r] += mine[16 * b + r];
+          else acc[1][b][r] += mine[16 * b + r];
+        }
+    }
+    __syncthreads();
   }
+  const bool sliced = gridDim.y > 1;
+  if (colsum && j0 == 0) {
+    *reinterpret_cast<float4*>(tn_lds + (grp * 8 + lk) * 128 + l4) = cs;
+    __syncthreads();
+    if (threadIdx.x < 128 && i0 + (int)threadIdx.x < M) {
+      float v = 0.f;
+      for (int r = 0; r < 16; ++r) v += tn_lds[r * 128 + threadIdx.x];
+      colsum[(sliced ? (int64_t)z * M : 0) + i0 + threadIdx.x] = v;
+    }
+  }
+  if (grp == 1) return;
+  float* out = sliced ? C + (int64_t)z * M * N : C;
+  const int64_t ld = sliced ? N : ldc;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -2330,29 +2393,37 @@ __global__ __launch_bounds__(256) void sgemm_tn128_kernel(int M, int N, int K, c
         for (int e = 0; e < 4; ++e) {
           const int gi = i0 + wi + 32 * a + 8 * g + 4 * h + e;
           if (gi >= M) continue;
-          float v = acc[a][b][4 * g + e];
-          if (!sliced && accumulate) v += out[(int64_t)gi * ld + gj];
-          out[(int64_t)gi * ld + gj] = v;
+          out[(int64_t)gi * ld + gj] = acc[a][b][4 * g + e];
         }
     }
 }
 
+// C = the sum of nz slices of (M, N), and colsum = the sum of nz rows of M behind it in the same launch.  A workgroup takes 64 entries,
+// a quarter of the slices to each wavefront with 16 loads in flight, then adds the four in order.
 __global__ __launch_bounds__(256) void sum_slices_kernel(int M, int N, int nz, const float* __restrict__ part, float* __restrict__ C,
-                                                         int64_t ldc, int accumulate) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)M * N) return;
+                                                         int64_t ldc, const float* __restrict__ colpart, float* __restrict__ colsum) {
+  __shared__ float sh[256];
+  const int64_t mn = (int64_t)M * N, wblocks = (mn + 63) / 64;
+  const bool col = blockIdx.x >= wblocks;
+  const int64_t n = col ? M : mn, idx = ((int64_t)blockIdx.x - (col ? wblocks : 0)) * 64 + (threadIdx.x & 63);
+  const float* src = col ? colpart : part;
+  const int w = threadIdx.x >> 6, per = (nz + 3) / 4, zb = w * per, ze = min(nz, zb + per);
   float s = 0.f;
-  const int64_t mn = (int64_t)M * N;
-  for (int z0 = 0; z0 < nz; z0 += 8) {  // eight slices' loads in flight, added in slice order as before
-    float v[8];
+  if (idx < n)
+    for (int z0 = zb; z0 < ze; z0 += 16) {
+      float v[16];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = z0 + k < nz ? part[(int64_t)(z0 + k) * mn + idx] : 0.f;
+      for (int k = 0; k < 16; ++k) v[k] = z0 + k < ze ? src[(int64_t)(z0 + k) * n + idx] : 0.f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (z0 + k < nz) s += v[k];
-  }
+      for (int k = 0; k < 16; ++k) s += v[k];
+    }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (w > 0 || idx >= n) return;
+  s = sh[threadIdx.x] + sh[threadIdx.x + 64] + sh[threadIdx.x + 128] + sh[threadIdx.x + 192];
+  if (col) { colsum[idx] = s; return; }
   const int i = (int)(idx / N), j = (int)(idx - (int64_t)i * N);
-  C[(int64_t)i * ldc + j] = accumulate ? C[(int64_t)i * ldc + j] + s : s;
+  C[(int64_t)i * ldc + j] = s;
 }
 
 // dz = out - target (target +1 on the first n_real rows, -1 on the rest) and the two squared-error sums (one workgroup)
@@ -2391,8 +2462,6 @@ __global__ __launch_bounds__(256) void disc_penalty_kernel(int64_t n, double fac
 }
 
 }  // namespace ks
-
-// kDiscMaxSlices is defined beside kDwSplit: the training backward pass of single fp32 layers shares these products
 
 struct DiscWs {
   float* y[KS_MAX_LAYERS];      // hidden outputs, all rows
@@ -2437,11 +2506,6 @@ static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, Dis
   return off;
 }
 
-static void launch_sum_slices(hipStream_t s, int M, int N, int slices, const float* part, float* C, int64_t ldc, bool accumulate) {
-  const int64_t n = (int64_t)M * N;
-  hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, N, slices, part, C, ldc, accumulate ? 1 : 0);
-}
-
 // One product of sgemm_kernel; g.kslice is set here.  Products over activations have reductions of a layer's width: four wavefronts
 // share one.  Weight gradients (both operands stored (k, .)) reduce over the rows, sixteen wavefronts to a workgroup, and are cut into
 // slices while their few tiles leave CUs idle and a slice keeps the 512 rows that give every wavefront one chunk of loads.
@@ -2461,26 +2525,31 @@ static void sgemm_go(hipStream_t s, SgemmArgs g) {
 }
 
 // C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single wide
-// fp32 layer.  The rows are cut so that about 512 workgroups share them.
-static void sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                        int64_t ldc, float* part, float* colsum, float* colpart) {
-  const int vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0;
+// fp32 layer.  The rows are cut so that about 512 workgroups, two per CU, share them.
+static int sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                       int64_t ldc, float* part, float* colsum, float* colpart) {
+  const bool vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && M % 128 == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0 && N % 128 == 0;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   int slices = 1;
   if (K >= 2048) {
     slices = (int)((512 + tiles - 1) / tiles);
-    if (slices > kDiscMaxSlices) slices = kDiscMaxSlices;
+    if (slices > kTnMaxSlices) slices = kTnMaxSlices;
     if ((int64_t)slices * 256 > K) slices = (int)(K / 256);
   }
   int kslice = (int)((K + slices - 1) / slices);
-  kslice = (kslice + 15) / 16 * 16;
+  kslice = (kslice + 31) / 32 * 32;
   slices = (int)((K + kslice - 1) / kslice);
-  hipLaunchKernelGGL(sgemm_tn128_kernel, dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128), (unsigned)slices), dim3(256), 0, s,
-                     (int)M, N, (int)K, A, lda, B, ldb, slices > 1 ? part : C, ldc, kslice, 0, vec_a, vec_b, slices > 1 ? colpart : colsum);
-  if (slices > 1) {
-    launch_sum_slices(s, (int)M, N, slices, part, C, ldc, false);
-    launch_sum_slices(s, (int)M, 1, slices, colpart, colsum, 1, false);
-  }
+  if (slices > 1) slices = (slices + 7) / 8 * 8;  // for the XCD mapping; slices past the last row add zeros
+  auto kfn = vec_a ? (vec_b ? sgemm_tn128_kernel<true, true> : sgemm_tn128_kernel<true, false>)
+                   : (vec_b ? sgemm_tn128_kernel<false, true> : sgemm_tn128_kernel<false, false>);
+  if (hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, kTnLds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", kTnLds);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)tiles, (unsigned)slices), dim3(512), kTnLds, s, (int)M, N, (int)K, A, lda, B, ldb,
+                     slices > 1 ? part : C, ldc, kslice, slices > 1 ? colpart : colsum);
+  if (slices > 1)
+    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((M * N + 63) / 64 + (M + 63) / 64)), dim3(256), 0, s, (int)M, N, slices, part, C, ldc,
+                       colpart, colsum);
+  return KS_OK;
 }
 
 extern "C" int64_t ks_mlp_disc_workspace_bytes(const KsMlp* h, int64_t n_real, int64_t n_sim) {

@@ -702,3 +702,27 @@ def test_head_gradients_at_the_edges_of_the_row_split(M, A, K):
     for got, want in ((d_raw, tr.grad), (d_value, tv.grad)):
         want = want.numpy()
         assert np.abs(got.cpu().numpy() - want).max() <= (1e-4 + 1e-6 * A) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dims,M", [
+    ((128, 512), 1), ((128, 512), 2051),      # fewer rows than a stage; a last slice that is short
+    ((97, 140), 5003),                        # rows on no 16-byte boundary, widths of no whole tile
+    ((52, 384), 33000), ((128, 128), 40001),  # many slices
+])
+def test_weight_gradient_of_a_single_layer_over_many_rows(dims, M):
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims) + M)
+    w, b = rng.normal(size=(dims[1], dims[0])).astype(np.float32), rng.normal(size=dims[1]).astype(np.float32)
+    x, dy = rng.normal(size=(M, dims[0])).astype(np.float32), rng.normal(size=(M, dims[1])).astype(np.float32)
+    net = MLP([w], [b], activation="none", dtype="f32")
+    net.train_init()
+    xd = t32(x)
+    net.train_forward(xd)
+    net.backward(xd, t32(dy))
+    gw, gb = net.parameters(gradients=True)[0]
+    want = dy.astype(np.float64).T @ x.astype(np.float64)
+    # a sum of M terms of size one in some order: at most M roundings of 2^-24, which add up like a random walk (8 deviations)
+    bound = 8 * 2.0 ** -24 * max(np.sqrt(M) * np.sqrt(M), 1.0)
+    assert np.abs(gw.cpu().numpy() - want).max() < max(bound, 1e-5)
+    assert np.abs(gb.cpu().numpy() - dy.astype(np.float64).sum(0)).max() < max(bound, 1e-5)
