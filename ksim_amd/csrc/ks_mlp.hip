@@ -1,11 +1,6 @@
-// MLP forward on the gfx950 matrix cores: one fused GEMM + bias + activation kernel per layer.
-//
-// Tile: a 256-thread workgroup (4 wavefronts, 2 x 2) owns a 128 x 128 block of the layer output;
-// each wavefront accumulates a 64 x 64 sub-block as 2 x 2 MFMA 32x32 tiles in 64 fp32 registers.
-// The K loop stages 128 x BK slices of the activations and of the weights through LDS.
-//   bf16 path: v_mfma_f32_32x32x16_bf16 (A/B fragments: 8 consecutive k per lane), BK = 32
-//   fp32 path: v_mfma_f32_32x32x2_f32   (A/B fragments: 1 k per lane),             BK = 16
-// Output fragment layout (both): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, column l%32.
+// MLP forward and backward on the gfx950 matrix cores: fused GEMM + bias + activation kernels per layer (mlp_layer_kernel: bf16 on
+// v_mfma_f32_32x32x16_bf16, 8 consecutive k per lane; sgemm_layer_kernel: fp32 on v_mfma_f32_32x32x2_f32, 1 k per lane) and
+// whole-network kernels.  Output fragment layout (both): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "ks_common.h"
 
 #include <cmath>
@@ -61,24 +56,17 @@ __device__ __forceinline__ u32x4 load_first(const float* __restrict__ x, int64_t
 #pragma unroll
     for (int e = 0; e < VEC; ++e) f[e] = (m < M && k + e < Kreal) ? x[m * ldx + k + e] : 0.f;
   }
-  u32x4 out;
-  if constexpr (sizeof(T) == 2) {
-    unsigned w[4];
+  unsigned w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned lo = __builtin_bit_cast(unsigned short, (__bf16)f[2 * e]);
-      const unsigned hi = __builtin_bit_cast(unsigned short, (__bf16)f[2 * e + 1]);
-      w[e] = lo | (hi << 16);
-    }
-    out = u32x4{w[0], w[1], w[2], w[3]};
-  } else {
-    out = u32x4{__builtin_bit_cast(unsigned, f[0]), __builtin_bit_cast(unsigned, f[1]),
-                __builtin_bit_cast(unsigned, f[2]), __builtin_bit_cast(unsigned, f[3])};
+  for (int e = 0; e < 4; ++e) {
+    const unsigned lo = __builtin_bit_cast(unsigned short, (__bf16)f[2 * e]);
+    const unsigned hi = __builtin_bit_cast(unsigned short, (__bf16)f[2 * e + 1]);
+    w[e] = lo | (hi << 16);
   }
-  return out;
+  return u32x4{w[0], w[1], w[2], w[3]};
 }
 
-// T = math/storage type of activations and weights (__bf16 or float).
+// T = math/storage type of activations and weights (__bf16).
 // FIRST: x is the caller's unpadded fp32 input (row stride ldx = in_dim).
 // LAST: y is the caller's unpadded fp32 output (row stride ldy = out_dim).
 // BM: rows per workgroup (128, or 64 for small batches so that the grid still covers every CU twice).
@@ -90,9 +78,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
                                                         const T* __restrict__ W /*(Np, K)*/,
                                                         const float* __restrict__ bias /*(Np)*/,
                                                         void* __restrict__ yout, int64_t ldy) {
-  constexpr bool BF = sizeof(T) == 2;
-  constexpr int BK = (BF ? 64 : 32) * KMUL;  // elements of K per slice (KMUL 2: half the barriers per flop, twice the LDS)
-  constexpr int PAD = BF ? 8 : 4;        // keeps 16-byte row alignment and spreads LDS banks
+  static_assert(sizeof(T) == 2, "fp32 layers have a kernel of their own");
+  constexpr int BK = 64 * KMUL;          // elements of K per slice (KMUL 2: half the barriers per flop, twice the LDS)
+  constexpr int PAD = 8;                 // keeps 16-byte row alignment and spreads LDS banks
   constexpr int VEC = 16 / sizeof(T);    // elements per 16-byte load
   constexpr int NT = 64 * WAVES_M * WAVES_N;    // threads per workgroup
   constexpr int A_VECS = BM * BK / VEC / NT;    // 16-byte loads per thread for the A slice
@@ -105,8 +93,19 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
   T (*Bs)[BK + PAD] = reinterpret_cast<T (*)[BK + PAD]>(mlp_lds + sizeof(T) * BM * (BK + PAD));
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int64_t m0 = (int64_t)blockIdx.x * BM;
-  const int n0 = blockIdx.y * BN;
+  // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
+  // other, so that its rows are fetched once (102400 x 128 -> 512 in fp32 reads 64 MB instead of 210).  Row tiles past the last whole eight
+  // follow in plain order.
+  int64_t m_tile = blockIdx.x;
+  int n_tile = blockIdx.y;
+  if (gridDim.y > 1) {
+    const int64_t l = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, whole = (int64_t)(gridDim.x & ~7u) * gridDim.y;
+    const int64_t q = l < whole ? l >> 3 : l - whole;
+    n_tile = (int)(q % gridDim.y);
+    m_tile = l < whole ? (q / gridDim.y) * 8 + (l & 7) : (int64_t)(gridDim.x & ~7u) + q / gridDim.y;
+  }
+  const int64_t m0 = m_tile * BM;
+  const int n0 = n_tile * BN;
   f32x16 acc[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -158,34 +157,18 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
     // re-reads its own slice) so that the register arrays are plain loop-carried values.
     const int kn = k0 + BK < kend ? k0 + BK : k0;
     KS_FETCH(kn)
-    if constexpr (BF) {
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 16) {
-        bf16x8 af[MI], bfr[NI];
+    for (int kk = 0; kk < BK; kk += 16) {
+      bf16x8 af[MI], bfr[NI];
 #pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = *(const bf16x8*)&As[wm * WM + i * 32 + (lane & 31)][kk + (lane >> 5) * 8];
+      for (int i = 0; i < MI; ++i) af[i] = *(const bf16x8*)&As[wm * WM + i * 32 + (lane & 31)][kk + (lane >> 5) * 8];
 #pragma unroll
-        for (int j = 0; j < NI; ++j) bfr[j] = *(const bf16x8*)&Bs[wn * WN + j * 32 + (lane & 31)][kk + (lane >> 5) * 8];
+      for (int j = 0; j < NI; ++j) bfr[j] = *(const bf16x8*)&Bs[wn * WN + j * 32 + (lane & 31)][kk + (lane >> 5) * 8];
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < NI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < BK; kk += 2) {
-        float af[MI], bfr[NI];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = (float)As[wm * WM + i * 32 + (lane & 31)][kk + (lane >> 5)];
-#pragma unroll
-        for (int j = 0; j < NI; ++j) bfr[j] = (float)Bs[wn * WN + j * 32 + (lane & 31)][kk + (lane >> 5)];
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bfr[j], acc[i][j], 0, 0, 0);
-      }
+        for (int j = 0; j < NI; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
     }
     __syncthreads();
   }
@@ -205,12 +188,150 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
         if (LAST) {
           if (col < Nreal) ((float*)yout)[(int64_t)blockIdx.z * M * ldy + row * ldy + col] = v;
         } else {
-          const float h = activate<ACT, BF>(v);
-          ((T*)yout)[row * ldy + col] = BF ? (T)to_bf16(h) : (T)h;
+          ((T*)yout)[row * ldy + col] = to_bf16(activate<ACT, true>(v));
         }
       }
     }
 }
+
+// fp32 layers: y = act(x W^T + b) on BM x 128 tiles, four wavefronts of BM / 2 x 64 each.  Operands pass through LDS transposed,
+// [k][row] with a stride of BM + 4 (128 + 4) floats, so that a matrix instruction's operand is one conflict-free 4-byte read per lane
+// (row-major, its 32 rows fall into 8 banks); a 16-byte load along k becomes four 4-byte writes into 64 different banks.  The LDS
+// buffer is double: stage n + 1 is written and stage n + 2 requested while stage n is multiplied, one barrier per 16 steps, and a
+// step's operands are read before the previous step's products.  At most 128 registers: four wavefronts per SIMD.
+// Every fp32 forward kernel here starts from the bias and adds the products in one order (k = 8 g + e and 8 g + 4 + e together, e = 0..3,
+// then the next g), so a row's numbers do not depend on the batch it comes in or the kernel that batch takes.
+//   102400 x 128 -> 512: 173 -> 163 us, of 87 in matrix instructions
+// x (M, Kreal) with row stride ldx; K: Kreal padded to 32 (W's stride; its padding is zero).  Columns of y past Nreal are not written when y is
+// the caller's (LAST); otherwise y is as wide as the padded layer.  gridDim.z > 1 (LAST): slice z of the reduction goes to its own copy
+// of the output.
+template <int BM, bool VA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void sgemm_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __restrict__ x, int64_t ldx, const float* __restrict__ W,
+                        const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, int act) {
+  constexpr int LA = BM + 4, LB = 132, MI = BM / 64, AV = BM / 64;
+  __shared__ __attribute__((aligned(16))) float As[2][16 * LA], Bs[2][16 * LB];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 31, h = lane >> 5;
+  // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
+  // other, so that its rows are fetched once.  Row tiles past the last whole eight follow in plain order.
+  int64_t m_tile = blockIdx.x;
+  int n_tile = blockIdx.y;
+  if (gridDim.y > 1) {
+    const int64_t l = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, whole = (int64_t)(gridDim.x & ~7u) * gridDim.y;
+    const int64_t q = l < whole ? l >> 3 : l - whole;
+    n_tile = (int)(q % gridDim.y);
+    m_tile = l < whole ? (q / gridDim.y) * 8 + (l & 7) : (int64_t)(gridDim.x & ~7u) + q / gridDim.y;
+  }
+  const int64_t m0 = m_tile * BM;
+  const int n0 = n_tile * 128;
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 64;
+  f32x16 acc[MI][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float b = blockIdx.z == 0 ? bias[n0 + wn + 32 * j + c] : 0.f;  // padded to whole tiles
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = b;
+  }
+  const int kslice = K / (int)gridDim.z, kbeg = (int)blockIdx.z * kslice, stages = kslice / 16;
+  // thread t loads rows t / 4 + 64 r, four steps from 4 (t % 4); rows past the batch repeat the last one, their results are dropped
+  const int lrow = t >> 2, lk = (t & 3) * 4;
+  const float* pa[AV];
+#pragma unroll
+  for (int r = 0; r < AV; ++r) {
+    const int64_t m = m0 + lrow + 64 * r;
+    pa[r] = x + (m < M ? m : M - 1) * ldx + kbeg + lk;
+  }
+  const float* pb = W + (int64_t)(n0 + lrow) * K + kbeg + lk;
+  const int64_t b64 = (int64_t)64 * K;
+  float4 ra[AV], rb[2];
+  auto fetch = [&](int n) __attribute__((always_inline)) {
+    const int k = 16 * n;
+#pragma unroll
+    for (int r = 0; r < AV; ++r) {
+      const float* q = pa[r] + k;
+      const int left = Kreal - (kbeg + lk + k);  // steps of the row still inside the input (VA: a multiple of four)
+      if (VA) {
+        ra[r] = float4{0.f, 0.f, 0.f, 0.f};
+        if (left > 0) ra[r] = *reinterpret_cast<const float4*>(q);
+      } else {
+        ra[r] = float4{left > 0 ? q[0] : 0.f, left > 1 ? q[1] : 0.f, left > 2 ? q[2] : 0.f, left > 3 ? q[3] : 0.f};
+      }
+    }
+    rb[0] = *reinterpret_cast<const float4*>(pb + k);
+    rb[1] = *reinterpret_cast<const float4*>(pb + b64 + k);
+  };
+  auto put = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < AV; ++r) {
+      float* q = &As[buf][lk * LA + lrow + 64 * r];
+      q[0] = ra[r].x; q[LA] = ra[r].y; q[2 * LA] = ra[r].z; q[3 * LA] = ra[r].w;
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      float* q = &Bs[buf][lk * LB + lrow + 64 * r];
+      q[0] = rb[r].x; q[LB] = rb[r].y; q[2 * LB] = rb[r].z; q[3 * LB] = rb[r].w;
+    }
+  };
+  fetch(0);
+  put(0);
+  if (stages > 1) fetch(1);
+  __syncthreads();
+  for (int n = 0; n < stages; ++n) {
+    const float* A = &As[n & 1][4 * h * LA + wm + c];
+    const float* B = &Bs[n & 1][4 * h * LB + wn + c];
+    float fa[2][MI], fb[2][2];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) fa[0][i] = A[32 * i];
+    fb[0][0] = B[0]; fb[0][1] = B[32];
+    if (n + 1 < stages) {
+      put((n + 1) & 1);
+      if (n + 2 < stages) fetch(n + 2);
+    }
+#define KS_STEP(S) (8 * ((S) >> 2) + ((S) & 3))  // the lower k of step S of a stage
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int q = s & 1;
+      if (s < 7) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[q ^ 1][i] = A[KS_STEP(s + 1) * LA + 32 * i];
+        fb[q ^ 1][0] = B[KS_STEP(s + 1) * LB]; fb[q ^ 1][1] = B[KS_STEP(s + 1) * LB + 32];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][i], fb[q][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#undef KS_STEP
+    __syncthreads();
+  }
+  float* out = y + (int64_t)blockIdx.z * M * ldy;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = n0 + wn + 32 * j + c;
+      if (col >= Nreal) continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (row >= M) continue;
+        float v = acc[i][j][r];
+        switch (act) {
+          case KS_ACT_ELU: v = activate<KS_ACT_ELU, false>(v); break;
+          case KS_ACT_RELU: v = activate<KS_ACT_RELU, false>(v); break;
+          case KS_ACT_TANH: v = activate<KS_ACT_TANH, false>(v); break;
+          case KS_ACT_GELU: v = activate<KS_ACT_GELU, false>(v); break;
+          default: break;
+        }
+        out[row * ldy + col] = v;
+      }
+    }
+}
+
 
 
 // ---------------------------------------------------------------- matrix-core yardstick
@@ -218,6 +339,102 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
 // kernel's own count), no loads, no LDS, no epilogue.  What this loop reaches is the most any kernel built on that
 // instruction can reach on this part at the clock it sustains under matrix load.  Per workgroup: stamps[2 b] = shader
 // clock cycles of the loop, stamps[2 b + 1] = the same interval on the constant 100 MHz counter.
+// A layer of an fp32 network over few rows: the whole-network kernel would give 32 rows to one CU, whose matrix rate then takes 80 us
+// for three layers of 512.  A wavefront owns a 32 x 32 tile of the layer with both operands straight from memory in registers (weights in
+// fragment order, eight groups of 8 k ahead) and the layers are launches of their own: rows x width / 1024 wavefronts over the chip.
+// SHARE wavefronts cut the reduction of a narrow output layer as the whole-network kernel's do (same parts, same order of the sum).
+// blockIdx.z picks one of two networks over the same rows (actor and critic).
+struct SmallLayer {
+  const float* x;
+  int64_t ldx;
+  int Kreal, nk, nt, Nreal, act, vec;
+  const u32x4* Wp;
+  const float* bp;
+  float* y;
+  int64_t ldy;
+};
+
+template <int SHARE>
+__global__ __launch_bounds__(256) void sgemm_small_kernel(int64_t M, SmallLayer p0, SmallLayer p1) {
+  constexpr int TPW = 4 / SHARE;  // tiles per workgroup
+  __shared__ float red[SHARE > 1 ? 4 : 1][SHARE > 1 ? 1024 : 1];
+  const SmallLayer& p = blockIdx.z == 0 ? p0 : p1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
+  const int part = wave % SHARE, tile = (int)blockIdx.x * TPW + wave / SHARE;
+  const bool on = tile < p.nt;
+  const int j = on ? tile : 0;
+  const int64_t m0 = (int64_t)blockIdx.y * 32, m = m0 + c < M ? m0 + c : M - 1;  // rows past the batch repeat the last one
+  const int per = (p.nk + SHARE - 1) / SHARE, g0 = part * per, g1 = on ? (g0 + per < p.nk ? g0 + per : p.nk) : 0;
+  f32x16 acc;
+  const float b = part == 0 ? p.bp[32 * j + c] : 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = b;
+  const float* xr = p.x + m * p.ldx;
+  const u32x4* wr = p.Wp + (int64_t)j * p.nk * 64 + lane;
+  typedef __attribute__((ext_vector_type(4))) float f32x4v;
+  // groups past the end and columns past the row's end load something valid; the columns count as zero, the groups are not used
+  auto load_x = [&](int g) __attribute__((always_inline)) {
+    const int k = 8 * g + 4 * h, last = p.Kreal - 1;
+    f32x4v v;
+    if (p.vec) v = *reinterpret_cast<const f32x4v*>(xr + (k < last - 3 ? k : last - 3));
+    else v = f32x4v{xr[k < last ? k : last], xr[k + 1 < last ? k + 1 : last], xr[k + 2 < last ? k + 2 : last], xr[k + 3 < last ? k + 3 : last]};
+    return v;
+  };
+  auto mma = [&](int g, f32x4v xv, f32x4v wv) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(8 * g + 4 * h + e < p.Kreal ? xv[e] : 0.f, wv[e], acc, 0, 0, 0);
+  };
+  constexpr int PF = 8;
+  f32x4v xf[PF], wf[PF];
+  if (g0 < g1) {
+    const int gl = g1 - 1;
+    auto request = [&](int u, int g) __attribute__((always_inline)) {
+      g = g < gl ? g : gl;
+      xf[u] = load_x(g);
+      wf[u] = __builtin_bit_cast(f32x4v, wr[(int64_t)g * 64]);
+    };
+#pragma unroll
+    for (int u = 0; u < PF; ++u) request(u, g0 + u);
+    int g = g0;
+    for (; g + PF <= g1; g += PF)
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        mma(g + u, xf[u], wf[u]);
+        request(u, g + u + PF);
+      }
+#pragma unroll
+    for (int u = 0; u < PF; ++u)
+      if (g + u < g1) mma(g + u, xf[u], wf[u]);
+  }
+  if constexpr (SHARE > 1) {
+    if (part > 0)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[wave][r * 64 + lane] = acc[r];
+    __syncthreads();
+    if (part > 0) return;
+    for (int q = 1; q < SHARE; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += red[wave + q][r * 64 + lane];
+  }
+  const int col = 32 * j + c;
+  if (!on || col >= p.Nreal) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int64_t row = m0 + 8 * (r >> 2) + 4 * h + (r & 3);
+    if (row >= M) continue;
+    float v = acc[r];
+    switch (p.act) {
+      case KS_ACT_ELU: v = activate<KS_ACT_ELU, false>(v); break;
+      case KS_ACT_RELU: v = activate<KS_ACT_RELU, false>(v); break;
+      case KS_ACT_TANH: v = activate<KS_ACT_TANH, false>(v); break;
+      case KS_ACT_GELU: v = activate<KS_ACT_GELU, false>(v); break;
+      default: break;
+    }
+    p.y[row * p.ldy + col] = v;
+  }
+}
+
 __global__ __launch_bounds__(256) void mfma_yardstick_kernel(int iters, float* __restrict__ out, long long* __restrict__ stamps) {
   f32x16 acc[8];
 #pragma unroll
@@ -272,8 +489,8 @@ struct FusedArgs {
   const float* x;
   float* y;
   long long* prof;  // phase time stamps of wavefront 0, written only by -DKS_PROFILE builds
-  // training forward: hidden layer l's activations also go to save[l], (M, save_ld[l]) bf16 row-major, for the backward pass
-  __bf16* save[KS_MAX_LAYERS];
+  // training forward: hidden layer l's activations also go to save[l], (M, save_ld[l]) row-major in working precision, for the backward pass
+  void* save[KS_MAX_LAYERS];
   int save_ld[KS_MAX_LAYERS];
   // training forward for the whole-network backward kernel: hidden layer l's activations transposed, keep_t[l]: (width, ldt).
   // The weight-gradient product takes them as they are, and the backward kernel's epilogue reads its f'(Y) from them.
@@ -298,14 +515,30 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
+// One fragment step of both operands: 16 k of bf16 in one matrix instruction, or 8 k of fp32 in four (lane half h holds k = 8 step +
+// 4 h + e in element e, so instruction e multiplies k = 8 step + e and 8 step + 4 + e); 16 bytes of each operand per lane either way.
+template <typename T>
+__device__ __forceinline__ f32x16 fused_mma(const u32x4& w, const u32x4& b, f32x16 acc) {
+  if constexpr (sizeof(T) == 2) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+  } else {
+    typedef __attribute__((ext_vector_type(4))) float f32x4v;
+    const f32x4v wf = __builtin_bit_cast(f32x4v, w), bf = __builtin_bit_cast(f32x4v, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[e], bf[e], acc, 0, 0, 0);
+  }
+  return acc;
+}
+
 // One layer's MFMA work of one wavefront: NT output tiles (weights w[t]) times MI row tiles.  `arow` points at
 // this lane's activation fragment of K step 0 (row lane % 32 of the first row tile, k half lane / 32).
 // Weight fragments sit in a register ring kPF steps ahead; activation fragments are read one step ahead.
-template <int NT, int MI, int kPF>
+template <typename T, int NT, int MI, int kPF>
 __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x4* __restrict__ w0,
-                                                const u32x4* __restrict__ w1, int nk, const __bf16* __restrict__ arow,
+                                                const u32x4* __restrict__ w1, int nk, const T* __restrict__ arow,
                                                 int lda) {
   static_assert(kPF % 2 == 0, "the activation double buffer relies on an even ring depth");
+  constexpr int SK = 32 / (int)sizeof(T);  // k per step
   u32x4 rw[kPF][NT];
 #pragma unroll
   for (int u = 0; u < kPF; ++u) {
@@ -313,9 +546,9 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
     rw[u][0] = w0[st * 64];
     if (NT > 1) rw[u][NT - 1] = w1[st * 64];
   }
-  bf16x8 bq[2][MI];
+  u32x4 bq[2][MI];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) bq[0][i] = *(const bf16x8*)(arow + i * 32 * lda);
+  for (int i = 0; i < MI; ++i) bq[0][i] = *(const u32x4*)(arow + i * 32 * lda);
   int s = 0;
   for (; s + kPF <= nk; s += kPF) {
 #pragma unroll
@@ -323,18 +556,17 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
       const int step = s + u;
       const int nstep = step + 1 < nk ? step + 1 : step;
 #pragma unroll
-      for (int i = 0; i < MI; ++i) bq[(u + 1) & 1][i] = *(const bf16x8*)(arow + i * 32 * lda + nstep * 16);
-      bf16x8 wf[NT];
+      for (int i = 0; i < MI; ++i) bq[(u + 1) & 1][i] = *(const u32x4*)(arow + i * 32 * lda + nstep * SK);
+      u32x4 wf[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wf[t] = __builtin_bit_cast(bf16x8, rw[u][t]);
+      for (int t = 0; t < NT; ++t) wf[t] = rw[u][t];
       const int nx = step + kPF < nk ? step + kPF : nk - 1;
       rw[u][0] = w0[nx * 64];
       if (NT > 1) rw[u][NT - 1] = w1[nx * 64];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-          acc[t][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[t], bq[u & 1][i], acc[t][i], 0, 0, 0);
+        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T>(wf[t], bq[u & 1][i], acc[t][i]);
     }
   }
 #pragma unroll
@@ -343,13 +575,11 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
       const int step = s + u;
       const int nstep = step + 1 < nk ? step + 1 : step;
 #pragma unroll
-      for (int i = 0; i < MI; ++i) bq[(u + 1) & 1][i] = *(const bf16x8*)(arow + i * 32 * lda + nstep * 16);
+      for (int i = 0; i < MI; ++i) bq[(u + 1) & 1][i] = *(const u32x4*)(arow + i * 32 * lda + nstep * SK);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-          acc[t][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, rw[u][t]), bq[u & 1][i],
-                                                              acc[t][i], 0, 0, 0);
+        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T>(rw[u][t], bq[u & 1][i], acc[t][i]);
     }
   }
 }
@@ -366,12 +596,17 @@ __device__ __forceinline__ void fused_bias_init(f32x16& acc, const float* __rest
 // Hidden layer: activation, round to bf16, back into the tile (4 consecutive features = one 8-byte LDS store).
 // `keep_t` (nullable) points at the transposed copy's entry (feature 0, this lane's row): across the 32 lanes of a half the
 // same register holds 32 consecutive rows of one feature, so a 2-byte store per lane writes two whole 64-byte runs.
-template <int ACT>
-__device__ __forceinline__ void fused_store_hidden(const f32x16& acc, __bf16* __restrict__ act, int lda, int j,
+template <int ACT, typename T>
+__device__ __forceinline__ void fused_store_hidden(const f32x16& acc, T* __restrict__ act, int lda, int j,
                                                    int row, int lane, __bf16* __restrict__ keep_t = nullptr, int64_t ldt = 0) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int f0 = j * 32 + 8 * g + 4 * (lane >> 5);
+    if constexpr (sizeof(T) == 4) {
+      *reinterpret_cast<float4*>(act + row * lda + f0) =
+          float4{activate<ACT, false>(acc[4 * g]), activate<ACT, false>(acc[4 * g + 1]), activate<ACT, false>(acc[4 * g + 2]), activate<ACT, false>(acc[4 * g + 3])};
+      continue;
+    }
     const uint2 packed = {pack_bf16(activate<ACT, true>(acc[4 * g]), activate<ACT, true>(acc[4 * g + 1])),
                           pack_bf16(activate<ACT, true>(acc[4 * g + 2]), activate<ACT, true>(acc[4 * g + 3]))};
     *reinterpret_cast<uint2*>(act + row * lda + f0) = packed;
@@ -425,27 +660,68 @@ __device__ __forceinline__ void fused_store_output(const f32x16& acc, float* __r
   }
 }
 
+// How many wavefronts cut the reduction of a narrow fp32 layer of nt <= 2 tiles (their partial tiles, 4 KB each per row tile, have to fit the
+// activation tile)
+__host__ __device__ inline int fused_share(int nt, int lda) {
+  int share = nt == 1 ? 4 : 2;
+  while (share > 1 && share * nt * 1024 > 32 * lda) share >>= 1;
+  return share;
+}
+
 // One layer of the whole-network kernel for one wavefront: MFMA work, barrier, epilogue, barrier.
-template <int ACT, int MI, bool LAST, bool KEEP>
-__device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, __bf16* __restrict__ act, int64_t m0, int lane,
+template <int ACT, typename T, int MI, bool LAST, bool KEEP>
+__device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __restrict__ act, int64_t m0, int lane,
                                             int wave, int64_t tile) {
   const int nk = a.fk[l], nt = a.fn[l], lda = a.lda;
-  const __bf16* arow = act + (lane & 31) * lda + (lane >> 5) * 8;
+  const T* arow = act + (lane & 31) * lda + (lane >> 5) * (16 / (int)sizeof(T));
   const int row = lane & 31;
-  if (nt * MI <= kFusedWaves) {  // few tiles: one (feature tile, row tile) pair per wavefront
+  if (sizeof(T) == 4 && MI <= 2 && nt <= 2) {
+    // Few tiles in fp32 (an output layer of 21 or 1 columns): one wavefront's 8 k per 256 cycles would leave the others idle for the
+    // layer's whole reduction (256 wide: 3.4 us of 25), so 2 or 4 wavefronts cut a tile's reduction and add up through the tile's
+    // own LDS, as many as it has room for (4 KB each).
+    // The same number for every row tile: a row's sums must not depend on the batch it comes in.
+    const int share = fused_share(nt, lda);
+    const bool busy = wave < share * nt * MI;
+    const int tl = busy ? wave / share : 0, part = busy ? wave % share : 0, j = tl / MI, i = tl % MI;
+    const int per = (nk + share - 1) / share, k0 = part * per, kn = busy ? (nk - k0 < per ? nk - k0 : per) : 0;
+    f32x16 acc[2][1];
+    fused_bias_init(acc[0][0], a.bp[l], j, lane);
+    if (part > 0)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][0][r] = 0.f;
+    const u32x4* w0 = a.Wp[l] + ((int64_t)j * nk + k0) * 64 + lane;
+    if (kn > 0) fused_layer_mma<T, 1, 1, 2>(acc, w0, w0, kn, arow + i * 32 * lda + k0 * 8, lda);
+    __syncthreads();  // every wavefront has read this layer's input; the tile can be overwritten
+    float* sc = reinterpret_cast<float*>(act);
+    if (share > 1) {
+      if (busy && part > 0)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[wave * 1024 + r * 64 + lane] = acc[0][0][r];
+      __syncthreads();
+      if (busy && part == 0)
+        for (int q = 1; q < share; ++q)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[0][0][r] += sc[(wave + q) * 1024 + r * 64 + lane];
+      __syncthreads();
+    }
+    if (busy && part == 0) {
+      if (LAST) fused_store_output(acc[0][0], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
+      else fused_store_hidden<ACT, T>(acc[0][0], act, lda, j, i * 32 + row, lane);
+    }
+  } else if (nt * MI <= kFusedWaves) {  // few tiles: one (feature tile, row tile) pair per wavefront
     const bool busy = wave < nt * MI;
     const int j = busy ? wave / MI : 0, i = busy ? wave % MI : 0;
     f32x16 acc[2][1];
     fused_bias_init(acc[0][0], a.bp[l], j, lane);
     acc[1][0] = acc[0][0];
     const u32x4* w0 = a.Wp[l] + (int64_t)j * nk * 64 + lane;
-    if (busy) fused_layer_mma<1, 1, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow + i * 32 * lda, lda);
+    if (busy) fused_layer_mma<T, 1, 1, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow + i * 32 * lda, lda);
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();  // every wavefront has read this layer's input; the tile can be overwritten
     KS_MLP_STAMP2(3 + 3 * l)
     if (busy) {
       if (LAST) fused_store_output(acc[0][0], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
-      else fused_store_hidden<ACT>(acc[0][0], act, lda, j, i * 32 + row, lane);
+      else fused_store_hidden<ACT, T>(acc[0][0], act, lda, j, i * 32 + row, lane);
     }
   } else {
     const int mine = wave < nt ? (wave + kFusedWaves < nt ? 2 : 1) : 0;
@@ -460,8 +736,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, __bf16* _
     }
     const u32x4* w0 = a.Wp[l] + (int64_t)j0 * nk * 64 + lane;
     const u32x4* w1 = a.Wp[l] + (int64_t)j1 * nk * 64 + lane;
-    if (mine == 2) fused_layer_mma<2, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w1, nk, arow, lda);
-    else if (mine == 1) fused_layer_mma<1, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow, lda);
+    if (mine == 2) fused_layer_mma<T, 2, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w1, nk, arow, lda);
+    else if (mine == 1) fused_layer_mma<T, 1, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow, lda);
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();
     KS_MLP_STAMP2(3 + 3 * l)
@@ -472,7 +748,7 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, __bf16* _
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
           if (LAST) fused_store_output(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
-          else fused_store_hidden<ACT>(acc[t][i], act, lda, j, i * 32 + row, lane,
+          else fused_store_hidden<ACT, T>(acc[t][i], act, lda, j, i * 32 + row, lane,
                                        (KEEP && MI == 4) ? a.keep_t[l] + m0 + i * 32 + row : nullptr, a.ldt);
         }
       }
@@ -482,40 +758,42 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, __bf16* _
   if (!LAST && a.save[l]) {
     // the finished tile, 16 bytes per thread and pass, rows as contiguous runs; the next layer only reads the tile until every
     // wavefront (this copy included, which sits before its matrix work in program order) has passed the next barrier
-    const int w8 = nt * 4;  // 16-byte pieces per row (32 features = 4 pieces)
-    __bf16* dst = a.save[l];
+    constexpr int PC = 16 / (int)sizeof(T);  // entries of a 16-byte piece
+    const int w8 = nt * (32 / PC);
+    T* dst = reinterpret_cast<T*>(a.save[l]);
     const int ld = a.save_ld[l];
     for (int idx = threadIdx.x; idx < MI * 32 * w8; idx += 64 * kFusedWaves) {
       const int r = idx / w8, c8 = idx - r * w8;
-      if (m0 + r < a.M) *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c8 * 8) = *reinterpret_cast<const uint4*>(act + r * lda + c8 * 8);
+      if (m0 + r < a.M) *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c8 * PC) = *reinterpret_cast<const uint4*>(act + r * lda + c8 * PC);
     }
   }
 }
 
-template <int ACT, int BM, bool KEEP = false>
+template <int ACT, typename T, int BM, bool KEEP = false>
 __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile) {
   constexpr int MI = BM / 32;
   constexpr int NTHR = 64 * kFusedWaves;
   extern __shared__ __attribute__((aligned(16))) unsigned char mlp_lds[];
-  __bf16* act = reinterpret_cast<__bf16*>(mlp_lds);
+  T* act = reinterpret_cast<T*>(mlp_lds);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t m0 = tile * BM;
   const int lda = a.lda;
+  constexpr int SK = 32 / (int)sizeof(T);
   KS_MLP_STAMP(0)
-  {  // network input -> bf16 tile; zero beyond the batch and in the K padding of the first layer
+  {  // network input -> tile; zero beyond the batch and in the K padding of the first layer
     const int in_dim = a.in_dim;
-    const int K0 = (KEEP && a.in_t_width > a.fk[0] * 16) ? a.in_t_width : a.fk[0] * 16;  // the transposed copy is padded further
+    const int K0 = (KEEP && a.in_t_width > a.fk[0] * SK) ? a.in_t_width : a.fk[0] * SK;  // the transposed copy is padded further
     const int64_t rows_left = a.M - m0;
     const int rows = rows_left < BM ? (int)rows_left : BM;
     const float* src = a.x + m0 * in_dim;
     const int padw = K0 - in_dim;
     for (int idx = tid; idx < BM * padw; idx += NTHR) {
       const int r = idx / padw, c = idx - r * padw;
-      act[r * lda + in_dim + c] = (__bf16)0.0f;
+      act[r * lda + in_dim + c] = (T)0.0f;
     }
     for (int idx = rows * in_dim + tid; idx < BM * in_dim; idx += NTHR) {
       const int r = idx / in_dim, c = idx - r * in_dim;
-      act[r * lda + c] = (__bf16)0.0f;
+      act[r * lda + c] = (T)0.0f;
     }
     if ((in_dim & 3) == 0) {  // rows are 16-byte aligned: four wide loads in flight per thread
       const float4* src4 = reinterpret_cast<const float4*>(src);
@@ -532,7 +810,8 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
           const int idx = base + q * NTHR;
           if (idx < total4) {
             const int r = idx * 4 / in_dim, c = idx * 4 - r * in_dim;
-            *reinterpret_cast<uint2*>(act + r * lda + c) = uint2{pack_bf16(v[q].x, v[q].y), pack_bf16(v[q].z, v[q].w)};
+            if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(act + r * lda + c) = v[q];
+            else *reinterpret_cast<uint2*>(act + r * lda + c) = uint2{pack_bf16(v[q].x, v[q].y), pack_bf16(v[q].z, v[q].w)};
           }
         }
       }
@@ -550,7 +829,7 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
           const int idx = base + q * NTHR;
           if (idx < total) {
             const int r = idx / in_dim, c = idx - r * in_dim;
-            act[r * lda + c] = (__bf16)v[q];
+            act[r * lda + c] = (T)v[q];
           }
         }
       }
@@ -558,25 +837,25 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   }
   __syncthreads();
   KS_MLP_STAMP(1)
-  if (KEEP && BM == 128 && a.keep_t_in && tid < a.in_t_width / 2)  // the first layer overwrites the tile only after its barrier
+  if constexpr (KEEP && BM == 128) if (a.keep_t_in && tid < a.in_t_width / 2)  // the first layer overwrites the tile only after its barrier
     (void)tile_transposed_out(act, lda, tid, a.keep_t_in, a.ldt, m0);
   for (int l = 0; l + 1 < a.n_layers; ++l) {
-    fused_layer<ACT, MI, false, KEEP>(a, l, act, m0, lane, wave, tile);
+    fused_layer<ACT, T, MI, false, KEEP>(a, l, act, m0, lane, wave, tile);
   }
-  fused_layer<ACT, MI, true, KEEP>(a, a.n_layers - 1, act, m0, lane, wave, tile);
+  fused_layer<ACT, T, MI, true, KEEP>(a, a.n_layers - 1, act, m0, lane, wave, tile);
 }
 
 // KEEP: the training forward that also stores every hidden layer's activations and the network input transposed
 // (FusedArgs::keep_t, keep_t_in; 128-row tiles only)
-template <int ACT, int BM, bool KEEP = false>
+template <int ACT, typename T, int BM, bool KEEP = false>
 __global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
 void mlp_fused_kernel(const FusedArgs a) {
-  mlp_fused_body<ACT, BM, KEEP>(a, blockIdx.x);
+  mlp_fused_body<ACT, T, BM, KEEP>(a, blockIdx.x);
 }
 
 // Two networks over the same rows in one launch (actor and critic of a control step): blockIdx.y picks the network, so
 // the second network's workgroups fill the CUs next to the first one's instead of waiting for their launch to drain.
-template <int ACT, int BM>
+template <int ACT, typename T, int BM>
 __global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
 void mlp_fused_pair_kernel(const FusedArgs a, const FusedArgs b) {
   // Workgroup L of the launch runs on XCD L % 8.  XCDs 0-3 take the first network and 4-7 the second, so that an XCD's L2
@@ -589,8 +868,8 @@ void mlp_fused_pair_kernel(const FusedArgs a, const FusedArgs b) {
     net = (int)(L % 8) / 4;
     tile = (L / 8) * 4 + (L % 8) % 4;
   }
-  if (net == 0) mlp_fused_body<ACT, BM>(a, tile);
-  else mlp_fused_body<ACT, BM>(b, tile);
+  if (net == 0) mlp_fused_body<ACT, T, BM>(a, tile);
+  else mlp_fused_body<ACT, T, BM>(b, tile);
 }
 
 // ---------------------------------------------------------------- whole-network backward pass of the hidden layers
@@ -653,8 +932,8 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
         for (int r = 0; r < 16; ++r) acc[t][i][r] = 0.f;
     const u32x4* w0 = a.WtP[l] + (int64_t)j0 * nk * 64 + lane;
     const u32x4* w1 = a.WtP[l] + (int64_t)j1 * nk * 64 + lane;
-    if (mine == 2) fused_layer_mma<2, MI, kPF>(acc, w0, w1, nk, arow, lda);
-    else if (mine == 1) fused_layer_mma<1, MI, kPF>(acc, w0, w0, nk, arow, lda);
+    if (mine == 2) fused_layer_mma<__bf16, 2, MI, kPF>(acc, w0, w1, nk, arow, lda);
+    else if (mine == 1) fused_layer_mma<__bf16, 1, MI, kPF>(acc, w0, w0, nk, arow, lda);
     __syncthreads();  // every wavefront has read dZ_l; the tile can take dZ_{l-1}
     // Epilogue in blocks of one (feature tile, row tile) pair = 16 accumulator registers.  A block's 16 activations Y_{l-1} come
     // from the transposed copy (per feature, 32 lanes read 32 consecutive rows); the next block's loads are issued before this
@@ -1069,8 +1348,9 @@ __global__ __launch_bounds__(256) void adam_kernel(int64_t n, float* __restrict_
 // the fragment-ordered copy [tile][k step][lane][8]
 template <typename T>
 __global__ __launch_bounds__(256) void refresh_kernel(int npad, int kpad, const float* __restrict__ mW, T* __restrict__ W,
-                                                      T* __restrict__ Wt, __bf16* __restrict__ Wp, int fk, int fn,
+                                                      T* __restrict__ Wt, T* __restrict__ Wp, int fk, int fn,
                                                       __bf16* __restrict__ WtP) {
+  constexpr int G = 16 / (int)sizeof(T);  // entries of a lane's fragment
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx < (int64_t)npad * kpad) {
     const int o = (int)(idx / kpad), i = (int)(idx - (int64_t)o * kpad);
@@ -1078,12 +1358,12 @@ __global__ __launch_bounds__(256) void refresh_kernel(int npad, int kpad, const 
     W[idx] = from_f32<T>(v);
     if (Wt) Wt[(int64_t)i * npad + o] = from_f32<T>(v);
   }
-  if (Wp && idx < (int64_t)fn * fk * 64 * 8) {
-    const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
-    const int64_t js = idx >> 9;
+  if (Wp && idx < (int64_t)fn * fk * 64 * G) {
+    const int e = (int)(idx % G), lane = (int)((idx / G) & 63);
+    const int64_t js = idx / (64 * G);
     const int st = (int)(js % fk), j = (int)(js / fk);
-    const int o = j * 32 + (lane & 31), i = st * 16 + (lane >> 5) * 8 + e;
-    Wp[idx] = (__bf16)((o < npad && i < kpad) ? mW[(int64_t)o * kpad + i] : 0.f);
+    const int o = j * 32 + (lane & 31), i = st * 2 * G + (lane >> 5) * G + e;
+    Wp[idx] = from_f32<T>((o < npad && i < kpad) ? mW[(int64_t)o * kpad + i] : 0.f);
   }
   if (WtP && idx < (int64_t)fn * fk * 64 * 8) {  // the transposed roles: tiles over the inputs, 2 fn steps over the outputs
     const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
@@ -1105,7 +1385,8 @@ struct AdamNetArgs {
   float *mW[KS_MAX_LAYERS], *m1W[KS_MAX_LAYERS], *m2W[KS_MAX_LAYERS], *mb[KS_MAX_LAYERS], *m1b[KS_MAX_LAYERS], *m2b[KS_MAX_LAYERS];
   const float *gW[KS_MAX_LAYERS], *gb[KS_MAX_LAYERS];
   void *W[KS_MAX_LAYERS], *Wt[KS_MAX_LAYERS];
-  __bf16 *Wp[KS_MAX_LAYERS], *WtP[KS_MAX_LAYERS];
+  void* Wp[KS_MAX_LAYERS];
+  __bf16* WtP[KS_MAX_LAYERS];
   float *b[KS_MAX_LAYERS], *bp[KS_MAX_LAYERS];
 };
 
@@ -1137,12 +1418,13 @@ __global__ __launch_bounds__(256) void adam_net_kernel(AdamNetArgs n, KsAdamPara
     const int o = (int)(idx / kpad), i = (int)(idx - (int64_t)o * kpad);
     reinterpret_cast<T*>(n.W[l])[idx] = from_f32<T>(v);
     if (n.Wt[l]) reinterpret_cast<T*>(n.Wt[l])[(int64_t)i * npad + o] = from_f32<T>(v);
-    // [tile o / 32][k step i / 16][lane (o % 32) + 32 ((i % 16) / 8)][i % 8].  The fragment copy is padded to 32 outputs and 16
-    // inputs, the master to the coarser tiles of the per-layer kernel: master entries beyond the fragment copy are padding
+    // [tile o / 32][k step i / 2G][lane (o % 32) + 32 ((i % 2G) / G)][i % G], G = 8 (bf16) or 4 (fp32).  The fragment copy is padded to
+    // 32 outputs and 2G inputs, the master to the coarser tiles of the per-layer kernel: master entries beyond the fragment copy are padding
     // (zero weights with zero gradients) and have no place in it.
-    if (n.Wp[l] && o < n.fn[l] * 32 && i < n.fk[l] * 16) {
-      const int64_t at = ((((int64_t)(o >> 5) * n.fk[l] + (i >> 4)) * 64 + (o & 31) + 32 * ((i >> 3) & 1)) << 3) + (i & 7);
-      n.Wp[l][at] = (__bf16)v;
+    constexpr int G = 16 / (int)sizeof(T);
+    if (n.Wp[l] && o < n.fn[l] * 32 && i < n.fk[l] * 2 * G) {
+      const int64_t at = (((int64_t)(o >> 5) * n.fk[l] + i / (2 * G)) * 64 + (o & 31) + 32 * ((i / G) & 1)) * G + i % G;
+      reinterpret_cast<T*>(n.Wp[l])[at] = from_f32<T>(v);
       if (n.WtP[l]) {  // the same entry with the roles of input and output exchanged
         const int64_t att = ((((int64_t)(i >> 5) * (2 * n.fn[l]) + (o >> 4)) * 64 + (i & 31) + 32 * ((o >> 3) & 1)) << 3) + (o & 7);
         n.WtP[l][att] = (__bf16)v;
@@ -1174,7 +1456,7 @@ static uint16_t f32_to_bf16_rne(float f) {
 template <typename T, bool FIRST, bool LAST, int BM, int BN, int WAVES_M, int WAVES_N, int KMUL = 1>
 static int launch_layer_tile(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x,
                              int64_t ldx, const void* W, const float* b, void* y, int64_t ldy, int ksplit = 1) {
-  constexpr int BK = (sizeof(T) == 2 ? 64 : 32) * KMUL, PAD = sizeof(T) == 2 ? 8 : 4;
+  constexpr int BK = 64 * KMUL, PAD = 8;
   constexpr int lds = (int)sizeof(T) * (BM + BN) * (BK + PAD);
   const dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)(npad / BN), (unsigned)ksplit);
   const dim3 block(64 * WAVES_M * WAVES_N);
@@ -1198,17 +1480,36 @@ static int launch_layer_tile(int act, hipStream_t s, int64_t M, int npad, int K,
   return KS_OK;
 }
 
-// Tile choice.  Large batches take the whole layer width per workgroup (BN = 512 or 256) so that the activations
+// fp32 layers.  A launch ends with the CU that got most of the tiles: below eight 128-row tiles per CU, 64-row ones leave less of a last
+// round (102400 x 512 -> 128: 151 -> 137 us) and keep small batches on more CUs.
+static int launch_layer_f32(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x, int64_t ldx, const void* W,
+                            const float* b, void* y, int64_t ldy, int ksplit = 1) {
+  const bool small = (M + 127) / 128 * (npad / kBN) * ksplit < 2048;
+  const bool va = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && Kreal % 4 == 0;
+  auto kfn = small ? (va ? sgemm_layer_kernel<64, true> : sgemm_layer_kernel<64, false>)
+                   : (va ? sgemm_layer_kernel<128, true> : sgemm_layer_kernel<128, false>);
+  const int bm = small ? 64 : 128;
+  hipLaunchKernelGGL(kfn, dim3((unsigned)((M + bm - 1) / bm), (unsigned)(npad / kBN), (unsigned)ksplit), dim3(256), 0, s, M, K, Kreal, Nreal,
+                     (const float*)x, ldx, (const float*)W, b, (float*)y, ldy, act);
+  return KS_OK;
+}
+
+// bf16 tile choice.  Large batches take the whole layer width per workgroup (BN = 512 or 256) so that the activations
 // are read from HBM once per layer; small (rollout-sized) batches take 64 x 128 tiles so that the grid still
 // covers the 256 CUs more than once.
 template <typename T, bool FIRST, bool LAST>
 static int launch_layer(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x,
                         int64_t ldx, const void* W, const float* b, void* y, int64_t ldy) {
 #define KS_ARGS act, s, M, npad, K, Kreal, Nreal, x, ldx, W, b, y, ldy
-  if (M >= 32768 && npad % 512 == 0 && sizeof(T) == 2) return launch_layer_tile<T, FIRST, LAST, 128, 512, 2, 4>(KS_ARGS);
-  if (M >= 32768 && npad % 256 == 0) return launch_layer_tile<T, FIRST, LAST, 128, 256, 2, 2>(KS_ARGS);
-  if (M * (npad / kBN) <= 128 * 512) return launch_layer_tile<T, FIRST, LAST, 64, 128, 2, 2>(KS_ARGS);
-  return launch_layer_tile<T, FIRST, LAST, 128, 128, 2, 2>(KS_ARGS);
+  if constexpr (sizeof(T) == 4) {
+    // between layers the rows are as wide as the padded layer, and so is the reduction
+    return launch_layer_f32(LAST ? KS_ACT_NONE : act, s, M, npad, K, FIRST ? Kreal : K, LAST ? Nreal : npad, x, ldx, W, b, y, ldy);
+  } else {
+    if (M >= 32768 && npad % 512 == 0) return launch_layer_tile<T, FIRST, LAST, 128, 512, 2, 4>(KS_ARGS);
+    if (M >= 32768 && npad % 256 == 0) return launch_layer_tile<T, FIRST, LAST, 128, 256, 2, 2>(KS_ARGS);
+    if (M * (npad / kBN) <= 128 * 512) return launch_layer_tile<T, FIRST, LAST, 64, 128, 2, 2>(KS_ARGS);
+    return launch_layer_tile<T, FIRST, LAST, 128, 128, 2, 2>(KS_ARGS);
+  }
 #undef KS_ARGS
 }
 
@@ -1259,38 +1560,43 @@ extern "C" int ks_mlp_create(const KsMlpDesc* d, KsMlp** out) {
       return fail(KS_ELAUNCH, "ks_mlp_create: upload of layer %d failed", l);
     }
   }
-  // fragment-ordered copy for the whole-network kernel
-  bool fusable = d->dtype == KS_MLP_BF16;
+  // fragment-ordered copy for the whole-network kernel and the small-batch kernel.  A single fp32 layer over many rows stays with the
+  // per-layer kernel (fused = 0): there is nothing to keep on chip between layers, and its output rows leave in longer runs.
+  bool fusable = true;
   for (int l = 0; l <= d->n_layers && fusable; ++l)
     if (round_up(d->dims[l], 32) > kFusedMaxWidth) fusable = false;
   if (fusable) {
+    const int G = 16 / (int)esz, sk = 2 * G;  // entries of a lane's fragment, k per step
     int kmax = 0;
     for (int l = 0; l < d->n_layers; ++l) {
       m.fn[l] = round_up(d->dims[l + 1], 32) / 32;
-      m.fk[l] = (l == 0 ? round_up(d->dims[0], 16) : m.fn[l - 1] * 32) / 16;
-      kmax = m.fk[l] * 16 > kmax ? m.fk[l] * 16 : kmax;
+      m.fk[l] = (l == 0 ? round_up(d->dims[0], sk) : m.fn[l - 1] * 32) / sk;
+      kmax = m.fk[l] * sk > kmax ? m.fk[l] * sk : kmax;
       if (l + 1 < d->n_layers && m.fn[l] * 32 > kmax) kmax = m.fn[l] * 32;
-      const size_t n = (size_t)m.fn[l] * m.fk[l] * 64 * 8;
-      std::vector<uint16_t> w(n, 0);
+      const size_t n = (size_t)m.fn[l] * m.fk[l] * 64 * G;
+      std::vector<unsigned char> w(n * esz, 0);
       for (int j = 0; j < m.fn[l]; ++j)
         for (int st = 0; st < m.fk[l]; ++st)
           for (int lane = 0; lane < 64; ++lane)
-            for (int e = 0; e < 8; ++e) {
-              const int o = j * 32 + (lane & 31), i = st * 16 + (lane >> 5) * 8 + e;
-              if (o < d->dims[l + 1] && i < d->dims[l])
-                w[(((size_t)j * m.fk[l] + st) * 64 + lane) * 8 + e] = f32_to_bf16_rne(d->weights[l][(size_t)o * d->dims[l] + i]);
+            for (int e = 0; e < G; ++e) {
+              const int o = j * 32 + (lane & 31), i = st * sk + (lane >> 5) * G + e;
+              if (o >= d->dims[l + 1] || i >= d->dims[l]) continue;
+              const float v = d->weights[l][(size_t)o * d->dims[l] + i];
+              const size_t at = (((size_t)j * m.fk[l] + st) * 64 + lane) * G + e;
+              if (esz == 2) ((uint16_t*)w.data())[at] = f32_to_bf16_rne(v);
+              else ((float*)w.data())[at] = v;
             }
       std::vector<float> b(m.fn[l] * 32, 0.f);
       for (int o = 0; o < d->dims[l + 1]; ++o) b[o] = d->biases[l][o];
-      if (hipMalloc(&m.Wp[l], n * 2) != hipSuccess || hipMalloc((void**)&m.bp[l], b.size() * 4) != hipSuccess ||
-          hipMemcpy(m.Wp[l], w.data(), n * 2, hipMemcpyHostToDevice) != hipSuccess ||
+      if (hipMalloc(&m.Wp[l], n * esz) != hipSuccess || hipMalloc((void**)&m.bp[l], b.size() * 4) != hipSuccess ||
+          hipMemcpy(m.Wp[l], w.data(), n * esz, hipMemcpyHostToDevice) != hipSuccess ||
           hipMemcpy(m.bp[l], b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
         ks_mlp_destroy(h);
         return fail(KS_ELAUNCH, "ks_mlp_create: upload of layer %d failed", l);
       }
     }
-    m.lda = kmax + 8;  // +16 bytes per row: 16-byte aligned rows that start 4 banks apart
-    m.fused = 1;
+    m.lda = kmax + 16 / (int)esz;  // +16 bytes per row: 16-byte aligned rows that start 4 banks apart
+    m.fused = d->dtype == KS_MLP_BF16 || d->n_layers > 1;
   }
   *out = h;
   return KS_OK;
@@ -1344,25 +1650,26 @@ static FusedArgs fused_args(const DevMlp& m, int64_t M, const float* x, float* y
 struct TrainWs;
 static void keep_args(FusedArgs& a, const DevMlp& m, const TrainWs* ws);
 
-template <int BM>
+template <typename T, int BM>
 static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const float* x, float* y, char* const* save,
                              const TrainWs* keep = nullptr) {
   FusedArgs a = fused_args(m, M, x, y);
   if (save)
     for (int l = 0; l + 1 < m.n_layers; ++l) {
-      a.save[l] = (__bf16*)save[l];
+      a.save[l] = save[l];
       a.save_ld[l] = m.npad[l];
     }
   if (keep) keep_args(a, m, keep);
 #ifdef KS_PROFILE
   if (const char* e = getenv("KS_MLP_PROF_PTR")) a.prof = (long long*)strtoull(e, nullptr, 16);
 #endif
-  const int lds = BM * m.lda * 2;
+  const int lds = BM * m.lda * (int)sizeof(T);
   const int64_t blocks = (M + BM - 1) / BM;
   if (blocks > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward: too many rows");
 #define KS_LAUNCH(A)                                                                                           \
   {                                                                                                            \
-    auto kfn = (keep && BM == 128) ? mlp_fused_kernel<A, BM, BM == 128> : mlp_fused_kernel<A, BM, false>;      \
+    constexpr bool kKeep = BM == 128 && sizeof(T) == 2;                                                        \
+    auto kfn = (keep && kKeep) ? mlp_fused_kernel<A, T, BM, kKeep> : mlp_fused_kernel<A, T, BM, false>;        \
     if (lds > 64 * 1024 &&                                                                                     \
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
       return fail(KS_ELAUNCH, "ks_mlp_forward: cannot raise the LDS limit to %d bytes", lds);                  \
@@ -1382,29 +1689,35 @@ static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const fl
 // Row tile: 128 rows amortise each weight fragment over four MFMAs; smaller batches take smaller tiles so that
 // the grid still reaches every CU.
 static int launch_fused(const DevMlp& m, hipStream_t s, int64_t M, const float* x, float* y, char* const* save = nullptr) {
+  if (m.dtype == KS_MLP_F32) {
+    // 64 rows share a weight fragment between two row tiles where that still leaves every CU a workgroup (and the tile fits LDS: up to
+    // 512 wide); the fp32 matrix rate, not the weights' way from L2, bounds both
+    if (M >= 64 * 256) return launch_fused_tile<float, 64>(m, s, M, x, y, save);
+    return launch_fused_tile<float, 32>(m, s, M, x, y, save);
+  }
 #ifdef KS_PROFILE
   if (const char* e = getenv("KS_MLP_BM")) {
     const int bm = atoi(e);
-    if (bm == 128) return launch_fused_tile<128>(m, s, M, x, y, save);
-    if (bm == 64) return launch_fused_tile<64>(m, s, M, x, y, save);
-    if (bm == 32) return launch_fused_tile<32>(m, s, M, x, y, save);
+    if (bm == 128) return launch_fused_tile<__bf16, 128>(m, s, M, x, y, save);
+    if (bm == 64) return launch_fused_tile<__bf16, 64>(m, s, M, x, y, save);
+    if (bm == 32) return launch_fused_tile<__bf16, 32>(m, s, M, x, y, save);
   }
 #endif
-  if (M >= 128 * 256) return launch_fused_tile<128>(m, s, M, x, y, save);
-  if (M >= 64 * 256) return launch_fused_tile<64>(m, s, M, x, y, save);
-  return launch_fused_tile<32>(m, s, M, x, y, save);
+  if (M >= 128 * 256) return launch_fused_tile<__bf16, 128>(m, s, M, x, y, save);
+  if (M >= 64 * 256) return launch_fused_tile<__bf16, 64>(m, s, M, x, y, save);
+  return launch_fused_tile<__bf16, 32>(m, s, M, x, y, save);
 }
 
-template <int BM>
+template <typename T, int BM>
 static int launch_fused_pair_tile(const DevMlp& m0, const DevMlp& m1, hipStream_t s, int64_t M, const float* x0, float* y0,
                                   const float* x1, float* y1) {
   const FusedArgs a = fused_args(m0, M, x0, y0), b = fused_args(m1, M, x1, y1);
-  const int lds = BM * (m0.lda > m1.lda ? m0.lda : m1.lda) * 2;
+  const int lds = BM * (m0.lda > m1.lda ? m0.lda : m1.lda) * (int)sizeof(T);
   const int64_t blocks = (M + BM - 1) / BM;
   if (blocks > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward_pair: too many rows");
 #define KS_LAUNCH(A)                                                                                           \
   {                                                                                                            \
-    auto kfn = mlp_fused_pair_kernel<A, BM>;                                                                   \
+    auto kfn = mlp_fused_pair_kernel<A, T, BM>;                                                                \
     if (lds > 64 * 1024 &&                                                                                     \
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
       return fail(KS_ELAUNCH, "ks_mlp_forward_pair: cannot raise the LDS limit to %d bytes", lds);             \
@@ -1421,6 +1734,60 @@ static int launch_fused_pair_tile(const DevMlp& m0, const DevMlp& m1, hipStream_
   return check_launch("ks_mlp_forward_pair");
 }
 
+// Whether M rows go through the small-batch kernel.  Networks of several layers: up to 2048 rows (one tile per SIMD at 512 wide) where the
+// whole-network kernel gives its wavefronts two tiles of a layer (68-512-512-512-20: 83 -> 52 us at 256 rows, 61 at 2048; 256 wide it takes 30
+// to this one's 40).  Single layers: up to 2048 tiles, two per SIMD; past that the reuse in the per-layer kernel's larger tiles wins
+// (128 -> 512: 12.0 us of 13.3 at 4096 rows, 21.1 of 17.8 at 8192).
+static bool small_ok(const DevMlp& m, int64_t M) {
+  if (m.dtype != KS_MLP_F32 || !m.Wp[0]) return false;
+  if (m.n_layers == 1) return (M + 31) / 32 * m.fn[0] <= 2048;
+  int wide = 0;
+  for (int l = 0; l + 1 < m.n_layers; ++l) wide = m.fn[l] > wide ? m.fn[l] : wide;
+  return wide > kFusedWaves && M <= 2048;
+}
+
+static int64_t small_ws_floats(const DevMlp& m, int64_t M) {  // two buffers of hidden activations
+  int wide = 0;
+  for (int l = 0; l + 1 < m.n_layers; ++l) wide = m.fn[l] * 32 > wide ? m.fn[l] * 32 : wide;
+  return (M * wide + 63) / 64 * 64;
+}
+
+static SmallLayer small_layer(const DevMlp& m, int64_t M, int l, const float* x, float* y, float* ws) {
+  const bool last = l == m.n_layers - 1;
+  const int64_t half = small_ws_floats(m, M);
+  SmallLayer p;
+  p.x = l == 0 ? x : ws + (l & 1 ? 0 : half);
+  p.Kreal = l == 0 ? m.dims[0] : m.fn[l - 1] * 32;
+  p.ldx = p.Kreal;
+  p.nk = m.fk[l]; p.nt = m.fn[l];
+  p.y = last ? y : ws + (l & 1 ? half : 0);
+  p.Nreal = last ? m.dims[l + 1] : m.fn[l] * 32;
+  p.ldy = p.Nreal;
+  p.act = last ? KS_ACT_NONE : m.activation;
+  p.vec = p.ldx % 4 == 0 && ((uintptr_t)p.x & 15) == 0;  // then Kreal is at least 4
+  p.Wp = (const u32x4*)m.Wp[l]; p.bp = m.bp[l];
+  return p;
+}
+
+// one network, or two of the same depth over the same number of rows
+static int launch_small(const DevMlp& a, const DevMlp* b, hipStream_t s, int64_t M, const float* xa, float* ya, void* wa, const float* xb,
+                        float* yb, void* wb) {
+  for (int l = 0; l < a.n_layers; ++l) {
+    const SmallLayer p = small_layer(a, M, l, xa, ya, (float*)wa), q = b ? small_layer(*b, M, l, xb, yb, (float*)wb) : p;
+    const int nets = b ? 2 : 1, nt = p.nt > q.nt ? p.nt : q.nt;
+    // the whole-network kernel cuts narrow layers only where it has layers to itself: a single layer is one wavefront's reduction
+    const int sa = a.n_layers > 1 && p.nt <= 2 ? fused_share(p.nt, a.lda) : 1, sb = b ? (q.nt <= 2 ? fused_share(q.nt, b->lda) : 1) : sa;
+    auto go = [&](int share, const SmallLayer& u, const SmallLayer& v, int n, int tiles) {
+      const dim3 grid((unsigned)((tiles * share + 3) / 4), (unsigned)((M + 31) / 32), (unsigned)n);
+      auto kfn = share == 4 ? sgemm_small_kernel<4> : (share == 2 ? sgemm_small_kernel<2> : sgemm_small_kernel<1>);
+      hipLaunchKernelGGL(kfn, grid, dim3(256), 0, s, M, u, v);
+    };
+    if (sa == sb) go(sa, p, q, nets, nt);
+    else { go(sa, p, p, 1, p.nt); go(sb, q, q, 1, q.nt); }
+  }
+  return check_launch("ks_mlp_forward");
+}
+
 extern "C" int ks_mlp_forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t stream, int64_t M, const float* x0,
                                    float* y0, const float* x1, float* y1, void* workspace0, void* workspace1) {
   if (!h0 || !h1) return fail(KS_EINVAL, "ks_mlp_forward_pair: null handle");
@@ -1429,9 +1796,14 @@ extern "C" int ks_mlp_forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t
   if (!x0 || !y0 || !x1 || !y1) return fail(KS_EINVAL, "ks_mlp_forward_pair: null pointer");
   if (y0 == y1) return fail(KS_EINVAL, "ks_mlp_forward_pair: the two outputs must differ");
   hipStream_t s = (hipStream_t)stream;
+  if (small_ok(h0->m, M) && small_ok(h1->m, M) && h0->m.n_layers == h1->m.n_layers && h0->m.n_layers > 1 && workspace0 && workspace1 &&
+      workspace0 != workspace1)
+    return launch_small(h0->m, &h1->m, s, M, x0, y0, workspace0, x1, y1, workspace1);
   // one launch when both networks run as whole-network kernels with the same activation and row tile; else one each
-  if (h0->m.fused && h1->m.fused && h0->m.activation == h1->m.activation && M < 64 * 256)
-    return launch_fused_pair_tile<32>(h0->m, h1->m, s, M, x0, y0, x1, y1);
+  if (h0->m.fused && h1->m.fused && h0->m.activation == h1->m.activation && h0->m.dtype == h1->m.dtype && M < 64 * 256) {
+    if (h0->m.dtype == KS_MLP_F32) return launch_fused_pair_tile<float, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1);
+    return launch_fused_pair_tile<__bf16, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1);
+  }
   const int rc = ks_mlp_forward(h0, stream, M, x0, y0, workspace0);
   if (rc != KS_OK) return rc;
   return ks_mlp_forward(h1, stream, M, x1, y1, workspace1);
@@ -1447,6 +1819,7 @@ extern "C" int ks_mfma_yardstick(ks_stream_t stream, int32_t workgroups, int32_t
 
 extern "C" int64_t ks_mlp_workspace_bytes(const KsMlp* h, int64_t M) {
   if (!h || M < 0) return 0;
+  if (h->m.n_layers > 1 && small_ok(h->m, M)) return 2 * 4 * small_ws_floats(h->m, M);
   if (h->m.fused) return 0;
   int widest = 0;
   for (int l = 0; l + 1 < h->m.n_layers; ++l) widest = h->m.npad[l] > widest ? h->m.npad[l] : widest;
@@ -1460,6 +1833,7 @@ extern "C" int ks_mlp_forward(const KsMlp* h, ks_stream_t stream, int64_t M, con
   if (M == 0) return KS_OK;
   if (!x || !y) return fail(KS_EINVAL, "ks_mlp_forward: null pointer");
   const DevMlp& m = h->m;
+  if (small_ok(m, M) && (m.n_layers == 1 || workspace)) return launch_small(m, nullptr, (hipStream_t)stream, M, x, y, workspace, nullptr, nullptr, nullptr);
   if (m.fused) return launch_fused(m, (hipStream_t)stream, M, x, y);
   if (m.n_layers > 1 && !workspace) return fail(KS_EINVAL, "ks_mlp_forward: workspace required");
   if ((M + kBM - 1) / kBM > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward: too many rows");
@@ -1549,7 +1923,7 @@ extern "C" int ks_mlp_train_init(KsMlp* h) {
     const size_t nt = l == 0 ? (size_t)round_up(m.kpad[0], kBN) * m.npad[0] : n;
     if (hipMalloc(&m.Wt[l], nt * esz) != hipSuccess || hipMemset(m.Wt[l], 0, nt * esz) != hipSuccess)
       return give_up("allocation");
-    if (m.fused && l >= 1) {  // as many fragments as the forward copy: (fk / 2) tiles of inputs x (2 fn) steps over outputs
+    if (m.fused && esz == 2 && l >= 1) {  // bf16: as many fragments as the forward copy, (fk / 2) tiles of inputs x (2 fn) steps over outputs
       const size_t np = (size_t)m.fn[l] * m.fk[l] * 512 * 2;
       if (hipMalloc(&m.WtP[l], np) != hipSuccess || hipMemset(m.WtP[l], 0, np) != hipSuccess) return give_up("allocation");
     }
@@ -1571,12 +1945,12 @@ template <typename T>
 static void refresh_layers(DevMlp& m, hipStream_t s) {
   for (int l = 0; l < m.n_layers; ++l) {
     const int64_t n = (int64_t)m.npad[l] * m.kpad[l];
-    const int64_t np = m.fused ? (int64_t)m.fn[l] * m.fk[l] * 512 : 0;
+    const int64_t np = m.Wp[l] ? (int64_t)m.fn[l] * m.fk[l] * 512 : 0;
     const int64_t tot = n > np ? n : np;
     hipLaunchKernelGGL(refresh_kernel<T>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, m.npad[l], m.kpad[l], m.mW[l],
-                       (T*)m.W[l], (T*)m.Wt[l], m.fused ? (__bf16*)m.Wp[l] : (__bf16*)nullptr, m.fk[l], m.fn[l], (__bf16*)m.WtP[l]);
+                       (T*)m.W[l], (T*)m.Wt[l], (T*)m.Wp[l], m.fk[l], m.fn[l], (__bf16*)m.WtP[l]);
     (void)hipMemcpyAsync(m.b[l], m.mb[l], (size_t)m.npad[l] * 4, hipMemcpyDeviceToDevice, s);
-    if (m.fused) (void)hipMemcpyAsync(m.bp[l], m.mb[l], (size_t)m.fn[l] * 32 * 4, hipMemcpyDeviceToDevice, s);
+    if (m.bp[l]) (void)hipMemcpyAsync(m.bp[l], m.mb[l], (size_t)m.fn[l] * 32 * 4, hipMemcpyDeviceToDevice, s);
   }
 }
 
@@ -1668,14 +2042,14 @@ extern "C" int64_t ks_mlp_train_workspace_bytes(const KsMlp* h, int64_t M) {
 
 template <typename T>
 static int train_forward(DevMlp& m, hipStream_t s, int64_t M, const float* x, float* y, const TrainWs& ws) {
-  // bf16 networks that fit the whole-network kernel run it, with every hidden layer's activations written out for the backward
+  // networks that fit the whole-network kernel run it, with every hidden layer's activations written out for the backward
   // pass as well; the stored rows must have the width the backward pass expects (its padding is in units of 64, the kernel's 32)
-  bool whole = m.fused && m.dtype == KS_MLP_BF16 && m.activation != KS_ACT_GELU;
+  bool whole = m.fused && m.activation != KS_ACT_GELU;
   for (int l = 0; whole && l + 1 < m.n_layers; ++l) whole = m.npad[l] == m.fn[l] * 32;
   m.chain_saved = 0;
   if (whole && chain_ok(m, M)) {  // activations in the formats of the whole-network backward pass, not row-major
     m.chain_saved = 1;
-    return launch_fused_tile<128>(m, s, M, x, y, nullptr, &ws);
+    return launch_fused_tile<__bf16, 128>(m, s, M, x, y, nullptr, &ws);
   }
   if (whole) return launch_fused(m, s, M, x, y, ws.act);
   const void* in = x;
@@ -1792,7 +2166,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
                           float* dx = nullptr, bool want_w = true, bool accumulate_dx = false, const uint8_t* zero_rows = nullptr) {
   const int L = m.n_layers;
   const int64_t Mp = ws.Mp;
-  if (m.chain_saved && sizeof(T) == 2) {
+  if constexpr (sizeof(T) == 2) if (m.chain_saved) {
     if (want_w && !dx) return train_backward_chain<T>(m, s, M, x, dy, ws);
     // the layer-by-layer pass below reads row-major activations: rebuild them from the transposed copies
     for (int l = 0; l + 1 < L; ++l)
@@ -1901,7 +2275,10 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
     const bool wide = Mp >= 32768 && np % 128 == 0;
     int ksplit = wide ? kDwSplit : kDwSplit / 2;
     while (ksplit > 1 && (Mp / 64) % ksplit != 0) ksplit >>= 1;
-    if (wide)
+    if constexpr (sizeof(T) == 4)
+      rc = launch_layer_f32(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, ws.t1, m.zero_bias,
+                            ksplit > 1 ? (void*)ws.part : (void*)m.gW[l], kp, ksplit);
+    else if (wide)
       rc = launch_layer_tile<T, false, true, 128, 128, 2, 2>(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, ws.t1,
                                                               m.zero_bias, ksplit > 1 ? (void*)ws.part : (void*)m.gW[l], kp, ksplit);
     else
@@ -2008,8 +2385,8 @@ extern "C" int ks_mlp_adam_step(KsMlp* h, ks_stream_t stream, const KsAdamParams
     blocks += (int)(((int64_t)m.npad[l] * m.kpad[l] + 255) / 256);  // npad * kpad >= npad: the bias rides on the first threads
     n.mW[l] = m.mW[l]; n.m1W[l] = m.m1W[l]; n.m2W[l] = m.m2W[l]; n.gW[l] = m.gW[l];
     n.mb[l] = m.mb[l]; n.m1b[l] = m.m1b[l]; n.m2b[l] = m.m2b[l]; n.gb[l] = m.gb[l];
-    n.W[l] = m.W[l]; n.Wt[l] = m.Wt[l]; n.Wp[l] = m.fused ? (__bf16*)m.Wp[l] : nullptr; n.WtP[l] = (__bf16*)m.WtP[l];
-    n.b[l] = m.b[l]; n.bp[l] = m.fused ? m.bp[l] : nullptr;
+    n.W[l] = m.W[l]; n.Wt[l] = m.Wt[l]; n.Wp[l] = m.Wp[l]; n.WtP[l] = (__bf16*)m.WtP[l];
+    n.b[l] = m.b[l]; n.bp[l] = m.bp[l];
   }
   n.first_block[m.n_layers] = blocks;
   if (m.dtype == KS_MLP_BF16) hipLaunchKernelGGL(adam_net_kernel<__bf16>, dim3((unsigned)blocks), dim3(256), 0, s, n, *p, sqnorm);

@@ -87,3 +87,34 @@ def test_paired_forward_equals_two_single_forwards(M):
         assert torch.equal(y0, actor(x0)) and torch.equal(y1, other(x1))
     with pytest.raises(_lib.KsError):
         actor.forward_pair(x0, torch.empty(M, 20, device=DEV), critic, x1[:-1], torch.empty(M - 1, 1, device=DEV))
+
+
+@pytest.mark.parametrize("dims", [
+    (68, 512, 512, 512, 20),      # output tile cut over four wavefronts
+    (71, 256, 256, 256, 33),      # two output tiles, two wavefronts each; rows of the input on no 16-byte boundary
+    (5, 40, 3), (33, 130, 130, 2),
+    (128, 512), (97, 140),        # single layers: 2048 tiles are the last batch of the kernel for few rows
+])
+def test_fp32_batches_of_every_size_give_a_row_the_same_bits(dims):
+    """Few rows (32 x 32 tiles, a launch per layer), 32-row and 64-row whole-network tiles, per-layer tiles: the last row count of one
+    kernel and the first of the next, ragged ends included."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims))
+    ws = [rng.normal(scale=1 / np.sqrt(i), size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])]
+    bs = [rng.normal(scale=0.1, size=o).astype(np.float32) for o in dims[1:]]
+    net = MLP(ws, bs, activation="elu", dtype="f32")
+    edge = 2048 // ((dims[1] + 31) // 32) * 32 if len(dims) == 2 else 2048
+    sizes = sorted({1, 31, 33, 65, edge, edge + 1, 4000, 16383, 16384 + 37})
+    x = rng.normal(size=(max(sizes), dims[0])).astype(np.float32)
+    X = torch.from_numpy(x).to(DEV)
+    want = reference(x, ws, bs, "elu", False)
+    full = net(X)
+    # a rounding of 2^-24 per product and sum, of sums of at most 512 terms whose squares add up to about 1, over at most 4 layers
+    assert np.abs(full.cpu().numpy() - want).max() <= 2e-5 * np.abs(want).max()
+    for M in sizes:
+        assert torch.equal(net(X[:M].contiguous()), full[:M]), M
+        y0, y1 = torch.full((M, dims[-1]), 7.0, device=DEV), torch.full((M, dims[-1]), 7.0, device=DEV)
+        other = MLP(ws, bs, activation="elu", dtype="f32")
+        net.forward_pair(X[:M].contiguous(), y0, other, X[-M:].contiguous(), y1)
+        assert torch.equal(y0, full[:M]) and torch.equal(y1, full[-M:]), M
