@@ -1018,7 +1018,7 @@ struct DevMlp {
   float *gW[KS_MAX_LAYERS], *gb[KS_MAX_LAYERS];
   float *m1W[KS_MAX_LAYERS], *m2W[KS_MAX_LAYERS], *m1b[KS_MAX_LAYERS], *m2b[KS_MAX_LAYERS];
   void* Wt[KS_MAX_LAYERS];      // (kpad, npad) working-precision transpose
-  void* WtP[KS_MAX_LAYERS];     // l >= 1, whole-network kernel only: W_l^T in fragment order, for the whole-network backward pass
+  void* WtP[KS_MAX_LAYERS];     // whole-network kernel only, l >= 1 or a single layer: W_l^T in fragment order, for the input gradients
   int chain_saved;              // the last training forward kept the activations in the whole-network backward pass's formats
   int bias_frozen[KS_MAX_LAYERS];  // leading bias entries of the layer that the optimiser leaves alone
   float* zero_bias;             // zeros, as wide as the widest GEMM output
@@ -1365,7 +1365,7 @@ __global__ __launch_bounds__(256) void refresh_kernel(int npad, int kpad, const 
     const int o = j * 32 + (lane & 31), i = st * 2 * G + (lane >> 5) * G + e;
     Wp[idx] = from_f32<T>((o < npad && i < kpad) ? mW[(int64_t)o * kpad + i] : 0.f);
   }
-  if (WtP && idx < (int64_t)fn * fk * 64 * 8) {  // the transposed roles: tiles over the inputs, 2 fn steps over the outputs
+  if (WtP && idx < (int64_t)((fk + 1) / 2) * (2 * fn) * 64 * 8) {  // the transposed roles: tiles over the inputs, 2 fn steps over the outputs
     const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
     const int64_t js = idx >> 9;
     const int st = (int)(js % (2 * fn)), j = (int)(js / (2 * fn));
@@ -1647,6 +1647,9 @@ static FusedArgs fused_args(const DevMlp& m, int64_t M, const float* x, float* y
   return a;
 }
 
+// A single bf16 layer given by its arguments (no hidden layers, nothing kept), on the row tiles of launch_fused
+static int launch_fused_args(const FusedArgs& a, hipStream_t s);
+
 struct TrainWs;
 static void keep_args(FusedArgs& a, const DevMlp& m, const TrainWs* ws);
 
@@ -1706,6 +1709,16 @@ static int launch_fused(const DevMlp& m, hipStream_t s, int64_t M, const float* 
   if (M >= 128 * 256) return launch_fused_tile<__bf16, 128>(m, s, M, x, y, save);
   if (M >= 64 * 256) return launch_fused_tile<__bf16, 64>(m, s, M, x, y, save);
   return launch_fused_tile<__bf16, 32>(m, s, M, x, y, save);
+}
+
+static int launch_fused_args(const FusedArgs& a, hipStream_t s) {
+  const int bm = a.M >= 128 * 256 ? 128 : a.M >= 64 * 256 ? 64 : 32, lds = bm * a.lda * 2;
+  auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128> : bm == 64 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 64>
+                                                                                : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)((a.M + bm - 1) / bm)), dim3(64 * kFusedWaves), lds, s, a);
+  return KS_OK;
 }
 
 template <typename T, int BM>
@@ -1923,8 +1936,8 @@ extern "C" int ks_mlp_train_init(KsMlp* h) {
     const size_t nt = l == 0 ? (size_t)round_up(m.kpad[0], kBN) * m.npad[0] : n;
     if (hipMalloc(&m.Wt[l], nt * esz) != hipSuccess || hipMemset(m.Wt[l], 0, nt * esz) != hipSuccess)
       return give_up("allocation");
-    if (m.fused && esz == 2 && l >= 1) {  // bf16: as many fragments as the forward copy, (fk / 2) tiles of inputs x (2 fn) steps over outputs
-      const size_t np = (size_t)m.fn[l] * m.fk[l] * 512 * 2;
+    if (m.fused && esz == 2 && (l >= 1 || m.n_layers == 1)) {  // bf16: (fk / 2, rounded up) tiles of inputs x (2 fn) steps over outputs
+      const size_t np = (size_t)((m.fk[l] + 1) / 2) * (2 * m.fn[l]) * 512 * 2;
       if (hipMalloc(&m.WtP[l], np) != hipSuccess || hipMemset(m.WtP[l], 0, np) != hipSuccess) return give_up("allocation");
     }
   }
@@ -1955,7 +1968,16 @@ static void refresh_layers(DevMlp& m, hipStream_t s) {
 }
 
 constexpr int kDwSplit = 32;  // most slices the weight-gradient reduction over the rows is cut into
-constexpr int kTnMaxSlices = 256;   // most slices of the row reduction of a single fp32 layer's gradient (sgemm_tn128)
+// Slices of the row reduction of a single layer's weight gradient (wgrad_kernel, 128 x 128 tiles): a workgroup per CU (its registers
+// admit no second one), a slice of at least three stages per group, below which the start and the slice sum cost as much as the
+// products; a multiple of eight, for the XCD mapping, once there are that many.
+static int wgrad_slices(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  int64_t slices = (256 + tiles - 1) / tiles;
+  if (slices > K / 192) slices = K / 192;
+  if (slices >= 8) slices = slices / 8 * 8;
+  return slices > 1 ? (int)slices : 1;
+}
 constexpr int kDiscMaxSlices = 64;  // most slices of a weight-gradient product of the discriminator (sgemm_kernel)
 
 // workspace: hidden activations of every layer, two (M, widest) gradient buffers, two transposes (widest, Mp)
@@ -2006,8 +2028,8 @@ static int64_t carve_train(const DevMlp& m, int64_t M, char* base, TrainWs* ws) 
   int64_t maxw = 0;
   for (int l = 0; l < m.n_layers; ++l) maxw = (int64_t)m.npad[l] * m.kpad[l] > maxw ? (int64_t)m.npad[l] * m.kpad[l] : maxw;
   int64_t nparts = kDwSplit * maxw > (int64_t)4 * kColsumSlices * wz ? kDwSplit * maxw : (int64_t)4 * kColsumSlices * wz;
-  if (m.n_layers == 1 && esz == 4)  // the one-pass weight and bias gradient of a single fp32 layer: slices of both
-    nparts = nparts > (int64_t)kTnMaxSlices * (maxw + wz) ? nparts : (int64_t)kTnMaxSlices * (maxw + wz);
+  if (m.n_layers == 1)  // the one-pass weight and bias gradient of a single layer: slices of both
+    nparts = (int64_t)wgrad_slices(m.dims[1], m.dims[0], M) * m.dims[1] * (m.dims[0] + 1);
   w.part = (float*)take(nparts * 4);
   w.Mp = Mp;
   w.Mp128 = (M + 127) / 128 * 128;
@@ -2158,14 +2180,55 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
   return KS_OK;
 }
 
-static int sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                       int64_t ldc, float* part, float* colsum, float* colpart);
+template <int PARTS>
+static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                 int64_t ldc, float* part, float* colsum);
+
+// Backward pass of a single layer (the projections of the recurrent cells and their networks, over all the (step, env) rows of a
+// trajectory slice): no activation to pass through, so the caller's gradient and input are the operands of both products as they are.
+template <typename T>
+static int train_backward_single(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws, float* dx,
+                                 bool want_w, bool accumulate_dx, const uint8_t* zero_rows) {
+  const int np = m.npad[0], in = m.dims[0], out = m.dims[1], kp128 = round_up(m.kpad[0], kBN);
+  const bool plain = !accumulate_dx && !zero_rows;
+  if (dx && sizeof(T) == 2 && plain && m.WtP[0]) {
+    // dX = dZ W: the whole-network kernel over the transposed fragments
+    FusedArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.M = M; a.n_layers = 1; a.in_dim = out; a.out_dim = in; a.lda = 32 * m.fn[0] + 8;
+    a.fk[0] = 2 * m.fn[0]; a.fn[0] = (m.fk[0] + 1) / 2;
+    a.Wp[0] = (const u32x4*)m.WtP[0]; a.bp[0] = m.zero_bias;
+    a.x = dy; a.y = dx;
+    const int rc = launch_fused_args(a, s);
+    if (rc != KS_OK) return rc;
+  } else if (dx) {
+    int rc;
+    T* tmp = (T*)ws.d1;
+    if constexpr (sizeof(T) == 4) {
+      rc = launch_layer_f32(KS_ACT_NONE, s, M, kp128, np, out, plain ? in : kp128, dy, out, m.Wt[0], m.zero_bias, plain ? dx : tmp,
+                            plain ? in : kp128);
+    } else {
+      const int64_t n = M * np;
+      hipLaunchKernelGGL(cast_pad_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, out, np, dy, (T*)ws.d0);
+      rc = launch_layer<T, false, false>(KS_ACT_NONE, s, M, kp128, np, np, kp128, ws.d0, np, m.Wt[0], m.zero_bias, tmp, kp128);
+    }
+    if (rc != KS_OK) return rc;
+    if (sizeof(T) == 2 || !plain) {
+      const int64_t n = M * in;
+      hipLaunchKernelGGL(unpad_cast_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, in, kp128, (const T*)tmp, dx,
+                         accumulate_dx ? 1 : 0, zero_rows);
+    }
+  }
+  if (!want_w) return KS_OK;
+  return wgrad<sizeof(T) == 2 ? 1 : 3>(s, out, in, M, dy, out, x, in, m.gW[0], m.kpad[0], ws.part, m.gb[0]);
+}
 
 template <typename T>
 static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws,
                           float* dx = nullptr, bool want_w = true, bool accumulate_dx = false, const uint8_t* zero_rows = nullptr) {
   const int L = m.n_layers;
   const int64_t Mp = ws.Mp;
+  if (L == 1) return train_backward_single<T>(m, s, M, x, dy, ws, dx, want_w, accumulate_dx, zero_rows);
   if constexpr (sizeof(T) == 2) if (m.chain_saved) {
     if (want_w && !dx) return train_backward_chain<T>(m, s, M, x, dy, ws);
     // the layer-by-layer pass below reads row-major activations: rebuild them from the transposed copies
@@ -2176,11 +2239,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
   }
   T* dz = (T*)ws.d0;
   T* dnext = (T*)ws.d1;
-  if (L == 1 && sizeof(T) == 4 && m.dims[1] == m.npad[0]) {
-    // a single fp32 layer whose width needs no padding (the projections of the recurrent cells): the caller's gradient is
-    // already the operand, and with one layer nothing below writes into this buffer
-    dz = (T*)const_cast<float*>(dy);
-  } else {  // the output gradient in working precision, padded to the last layer's width
+  {  // the output gradient in working precision, padded to the last layer's width
     const int64_t n = M * m.npad[L - 1];
     hipLaunchKernelGGL(cast_pad_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, m.dims[L], m.npad[L - 1], dy, dz);
   }
@@ -2205,15 +2264,6 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
       }
     }
     if (!want_w && l == 0) break;
-    if (L == 1 && sizeof(T) == 4 && np >= 128) {
-      // A single fp32 layer (the projections of the recurrent cells, over all the (step, env) rows of a trajectory slice): the
-      // weight gradient dZ^T X and the bias gradient, the column sums of dZ, in one pass over the row-major operands as they
-      // are, on the 128 x 128 tiles of the long-reduction product; no transposed copies.
-      float* colpart = ws.part + (int64_t)kTnMaxSlices * np * kp;
-      const int rc = sgemm_tn128(s, np, m.dims[0], M, (const float*)dz, np, x, m.dims[0], m.gW[0], kp, ws.part, m.gb[0], colpart);
-      if (rc != KS_OK) return rc;
-      break;
-    }
     if (want_w && !have_bias) {
       const int nz = M >= 32768 ? 4 * kColsumSlices : kColsumSlices;  // narrow layers: more row slices fill the chip
       hipLaunchKernelGGL(colsum_kernel<T>, dim3((unsigned)((np + 63) / 64), nz), dim3(256), 0, s, M, np, dz, ws.part);
@@ -2618,120 +2668,179 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
   }
 }
 
-// The same product for the weight and bias gradient of a single wide layer over a hundred thousand rows, C(i, j) = sum_k A(k, i) B(k, j)
-// with both operands stored (k, .): a 128 x 128 tile per workgroup of two groups of four wavefronts; each group takes half of the
-// slice's rows and each of its wavefronts a 64 x 64 block (2 x 2 MFMA tiles, so a value read from LDS feeds two matrix instructions),
-// and the second group's tile is added to the first's at the end.  Loads (16 bytes wide where VA / VB: the operand's rows are
-// 16-byte aligned, its width whole tiles) are two 16-row stages ahead of the matrix work: one in flight in registers, one in the other
-// half of the LDS buffer, so that a stage costs one barrier; a step's LDS reads are issued before the previous step's products.  Two
-// workgroups share a CU: four wavefronts per SIMD.  One group of four with two barriers per stage and one workgroup per CU took 172 us
-// at 102400 x 512 x 128 (78 TFLOP/s), this 130; with the loads left out it takes 118 us, and the matrix instructions alone are 87.
-// `colsum` also receives sum_k A(k, i), the bias gradient, from the registers the tiles pass through anyway.
+// The weight and bias gradient of a single layer over many rows, C(i, j) = sum_k A(k, i) B(k, j) with both operands fp32 and stored
+// (k, .), on the bf16 matrix instruction.  PARTS = 1: operands rounded to bf16, what a bf16 network's products take.  PARTS = 3: every
+// fp32 value is cut into three bf16 values whose sum is the value itself (8 + 8 + 8 bits), and of the nine products of two cut values
+// the six that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding per 16 rows where the
+// fp32 instruction has eight, the other five, 2^-8 of it, in a second one.
+// A 128 x 128 tile per workgroup of two groups of four wavefronts; each group takes half of the slice's rows in stages of 32 and each of
+// its wavefronts a 64 x 64 block.  The groups take turns: while one multiplies out of its LDS buffer the other cuts the stage it has in
+// registers, writes it to its own and requests the next, so a SIMD has one wavefront of matrix work and one of vector work at any time.
+// A thread holds 8 rows x 4 columns of a stage, and a fragment is 8 rows of one column: 16-byte loads and 16-byte LDS writes.  Column
+// 4 l + e of the tile goes to slot 32 e + l, so that neighbouring lanes write neighbouring fragments; a matrix tile is then every fourth
+// column.
+// `colsum` also receives sum_k A(k, i), the bias gradient, from the fp32 values in the loaders' registers.
 // gridDim.y cuts the k range into slices of kslice; with more than one slice, slice z writes its partial product (M, N) densely to
 // C + z * M * N and its column sums to colsum + z * M, and sum_slices_kernel adds them up in a fixed order.
-constexpr int kTnStage = 16 * 132;  // floats of one operand's 16-row stage in LDS
-constexpr int kTnLds = 2 * 2 * 2 * kTnStage * (int)sizeof(float);  // groups x buffers x operands
-template <bool VA, bool VB>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void sgemm_tn128_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
-                                             const float* __restrict__ B, int64_t ldb, float* __restrict__ C, int64_t ldc,
-                                             int kslice, float* __restrict__ colsum) {
-  extern __shared__ __attribute__((aligned(16))) float tn_lds[];
-  // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD one after the other (the number of
-  // slices is a multiple of 8 whenever there are several)
+// Bound by the matrix instructions (six per product of 16 rows, 48 us at the first size below) and the cuts beside them; the operands
+// take 44 us at the card's copy rate.  The predecessor multiplied on the fp32 instruction, whose time alone is 87 us there.
+//   102400 x 512 x 128, fp32: 122 -> 79 us (110 -> 170 TFLOP/s); relative error against 64 bits 7.3e-7 -> 1.9e-7
+//   12288 x 384 x 128, bf16: 44 us in five launches (cast, two transposes, product, column sums) -> 11.4
+// VA / VB: the operand's rows are 16-byte aligned and its width is a multiple of four.
+constexpr int kTnKB = 32;  // rows of a stage
+__host__ __device__ constexpr int tn_buf(int parts) { return parts * (kTnKB / 8) * 256; }  // one group's LDS buffer, in 16-byte fragments
+
+// Eight values of a column to PARTS fragments.  The clamp keeps a value that would round up to infinity finite, and an infinite one in
+// the last part, where its products with the other operand's first part still come out infinite.
+template <int PARTS>
+__device__ __forceinline__ void cut_bf16(const float (&v)[8], u32x4 (&out)[PARTS]) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = v[e];
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float a = x[2 * q], b = x[2 * q + 1];
+      if (p + 1 < PARTS) {
+        constexpr float kBf16Max = 3.3895313892515355e38f;
+        a = __builtin_amdgcn_fmed3f(a, -kBf16Max, kBf16Max);
+        b = __builtin_amdgcn_fmed3f(b, -kBf16Max, kBf16Max);
+      }
+      const unsigned w = pack_bf16(a, b);
+      out[p][q] = w;
+      if (p + 1 < PARTS) {
+        x[2 * q] -= __builtin_bit_cast(float, w << 16);
+        x[2 * q + 1] -= __builtin_bit_cast(float, w & 0xffff0000u);
+      }
+    }
+  }
+}
+
+template <int PARTS, bool VA, bool VB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
+                  float* __restrict__ C, int64_t ldc, int kslice, float* __restrict__ colsum) {
+  extern __shared__ __attribute__((aligned(16))) u32x4 tn_lds[];  // [group][part][8 rows][slot: 128 of A, 128 of B]
+  // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD one after the other
   int tile = blockIdx.x, z = blockIdx.y;
-  if (gridDim.y > 1) {
+  if (gridDim.y % 8 == 0) {
     const int l = blockIdx.y * gridDim.x + blockIdx.x, q = l >> 3;
     tile = q % gridDim.x;
     z = (q / gridDim.x) * 8 + (l & 7);
   }
   const int tiles_n = (N + 127) / 128;
   const int grp = threadIdx.x >> 8, t = threadIdx.x & 255, i0 = tile / tiles_n * 128, j0 = tile % tiles_n * 128;
-  float* lds = tn_lds + grp * 4 * kTnStage;  // [buffer][operand][16][132]
   const int zbeg = min(K, z * kslice), zend = min(K, zbeg + kslice);
-  const int half = ((zend - zbeg + 31) / 32) * 16;  // rows per group, in whole stages; both groups run the same number of stages
-  const int kbeg = zbeg + grp * half, kend = min(zend, kbeg + half), stages = half / 16;
+  const int half = ((zend - zbeg + 2 * kTnKB - 1) / (2 * kTnKB)) * kTnKB;  // rows per group, in whole stages; the same number for both
+  const int kbeg = min(zend, zbeg + grp * half), kend = min(zend, kbeg + half), stages = half / kTnKB;
   const int wave = t >> 6, lane = t & 63, c = lane & 31, h = lane >> 5;
-  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
-  f32x16 acc[2][2];
+  const int ea = (wave >> 1) * 2, eb = (wave & 1) * 2;  // first of the wavefront's two matrix tiles of either operand
+  f32x16 acc[2][2], low[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-  float4 ra[2], rb[2];
-  float4 cs = {0.f, 0.f, 0.f, 0.f};  // this thread's four columns of A, summed over the rows it loads
-  // thread t loads rows k = t / 32 and 8 + t / 32 of a stage, four consecutive columns from 4 (t % 32); columns past the matrix repeat
-  // the last one, their products are not stored
-  const int lk = t >> 5, l4 = (t & 31) * 4;
-  const float* pa = A + (int64_t)(kbeg + lk) * lda + (VA ? i0 + l4 : 0);
-  const float* pb = B + (int64_t)(kbeg + lk) * ldb + (VB ? j0 + l4 : 0);
-  int ic[4], jc[4];
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = low[a][b][r] = 0.f;
+  // threads 0-127 of a group load A, the others B: rows 8 kg + r, columns 4 l + e; columns past the matrix repeat its last ones, whose
+  // products are not stored
+  const bool isb = t >= 128;
+  const int kg = (t & 127) >> 5, l = t & 31;
+  const int width = isb ? N : M, c0 = (isb ? j0 : i0) + 4 * l;
+  const bool vec = isb ? VB : VA;
+  const int64_t ld = isb ? ldb : lda;
+  const float* src = (isb ? B : A) + (int64_t)(kbeg + 8 * kg) * ld;
+  int at[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) { ic[e] = min(i0 + l4 + e, M - 1); jc[e] = min(j0 + l4 + e, N - 1); }
-  auto load4 = [](const float* q, bool vec, const int (&at)[4]) __attribute__((always_inline)) {
-    return vec ? *reinterpret_cast<const float4*>(q) : float4{q[at[0]], q[at[1]], q[at[2]], q[at[3]]};
+  for (int e = 0; e < 4; ++e) at[e] = vec ? min(c0, width - 4) + e : min(c0 + e, width - 1);
+  float4 v[8];
+  float4 cs = {0.f, 0.f, 0.f, 0.f};
+  auto load4 = [&](const float* q) __attribute__((always_inline)) {
+    if (vec) return *reinterpret_cast<const float4*>(q + at[0]);
+    return float4{q[at[0]], q[at[1]], q[at[2]], q[at[3]]};
   };
-  const int64_t a8 = 8 * lda, b8 = 8 * ldb;
   auto fetch = [&](int n) __attribute__((always_inline)) {
-    if (kbeg + 16 * n + 16 <= kend) {
-      ra[0] = load4(pa, VA, ic); ra[1] = load4(pa + a8, VA, ic);
-      rb[0] = load4(pb, VB, jc); rb[1] = load4(pb + b8, VB, jc);
-      pa += 2 * a8; pb += 2 * b8;
+    const int k0 = kbeg + kTnKB * n + 8 * kg;
+    const float* q = src + (int64_t)n * kTnKB * ld;
+    if (kbeg + kTnKB * (n + 1) <= kend) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] = load4(q + r * ld);
     } else {  // the group's last rows, and zeros beyond them
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int k = kbeg + 16 * n + lk + 8 * r;
-        ra[r] = rb[r] = float4{0.f, 0.f, 0.f, 0.f};
-        if (k < kend) { ra[r] = load4(pa + r * a8, VA, ic); rb[r] = load4(pb + r * b8, VB, jc); }
+      for (int r = 0; r < 8; ++r) {
+        v[r] = float4{0.f, 0.f, 0.f, 0.f};
+        if (k0 + r < kend) v[r] = load4(q + r * ld);
       }
     }
   };
-  auto put = [&](int buf) __attribute__((always_inline)) {
+  u32x4* buf = tn_lds + grp * tn_buf(PARTS);
+  auto put = [&]() __attribute__((always_inline)) {
+    if (!isb)
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      *reinterpret_cast<float4*>(lds + buf * 2 * kTnStage + (lk + 8 * r) * 132 + l4) = ra[r];
-      *reinterpret_cast<float4*>(lds + buf * 2 * kTnStage + kTnStage + (lk + 8 * r) * 132 + l4) = rb[r];
-      cs.x += ra[r].x; cs.y += ra[r].y; cs.z += ra[r].z; cs.w += ra[r].w;
+      for (int r = 0; r < 8; ++r) { cs.x += v[r].x; cs.y += v[r].y; cs.z += v[r].z; cs.w += v[r].w; }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float f[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f[r] = e == 0 ? v[r].x : e == 1 ? v[r].y : e == 2 ? v[r].z : v[r].w;
+      u32x4 part[PARTS];
+      cut_bf16<PARTS>(f, part);
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) buf[(p * (kTnKB / 8) + kg) * 256 + (isb ? 128 : 0) + 32 * e + l] = part[p];
     }
   };
-  fetch(0);
-  put(0);
-  fetch(1);
-  __syncthreads();
-  for (int n = 0; n < stages; ++n) {
-    const float* As = lds + (n & 1) * 2 * kTnStage + h * 132 + wi + c;
-    const float* Bs = lds + (n & 1) * 2 * kTnStage + kTnStage + h * 132 + wj + c;
-    float fa[2][2], fb[2][2];
-    fa[0][0] = As[0]; fa[0][1] = As[32]; fb[0][0] = Bs[0]; fb[0][1] = Bs[32];
-    if (n + 1 < stages) {
-      put((n + 1) & 1);  // the stage fetched one step ago, into the half nobody reads until the barrier
-      fetch(n + 2);
-    }
+  auto multiply = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int q = s & 1;
-      if (s < 7) {
-        fa[q ^ 1][0] = As[(2 * s + 2) * 132]; fa[q ^ 1][1] = As[(2 * s + 2) * 132 + 32];
-        fb[q ^ 1][0] = Bs[(2 * s + 2) * 132]; fb[q ^ 1][1] = Bs[(2 * s + 2) * 132 + 32];
+    for (int s = 0; s < kTnKB / 16; ++s) {
+      bf16x8 fa[PARTS][2], fb[PARTS][2];
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const u32x4* at_k = buf + (p * (kTnKB / 8) + 2 * s + h) * 256 + c;
+          fa[p][q] = __builtin_bit_cast(bf16x8, at_k[32 * (ea + q)]);
+          fb[p][q] = __builtin_bit_cast(bf16x8, at_k[128 + 32 * (eb + q)]);
+        }
+#define KS_MMA(ACC, P, Q)                                                                                            \
+  _Pragma("unroll") for (int a = 0; a < 2; ++a) _Pragma("unroll") for (int b = 0; b < 2; ++b) ACC[a][b] =            \
+      __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[P][a], fb[Q][b], ACC[a][b], 0, 0, 0);
+      if constexpr (PARTS == 3) {
+        KS_MMA(low, 2, 0) KS_MMA(low, 0, 2) KS_MMA(low, 1, 1) KS_MMA(low, 1, 0) KS_MMA(low, 0, 1)
       }
-      __builtin_amdgcn_sched_barrier(0);
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0], fb[q][0], acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0], fb[q][1], acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1], fb[q][0], acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1], fb[q][1], acc[1][1], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+      KS_MMA(acc, 0, 0)
+#undef KS_MMA
     }
-    __syncthreads();
+  };
+  if (stages > 0) fetch(0);
+  for (int p = 0; p <= 2 * stages; ++p) {
+    const int n = (p - grp) >> 1;
+    if (((p ^ grp) & 1) == 0) {
+      if (n < stages) {
+        put();
+        if (n + 1 < stages) fetch(n + 1);
+      }
+    } else if (p > grp) {
+      multiply();
+    }
+    // LDS only: the requested rows stay in flight over it
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
+  if constexpr (PARTS == 3)
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][b][r] += low[a][b][r];
   // the second group hands its tile over in two halves through the buffers, which are free now
-  float* mine = tn_lds + (wave * 64 + lane) * 33;  // 33: the lanes' rows start in different banks
+  float* mine = reinterpret_cast<float*>(tn_lds) + t;
   for (int a = 0; a < 2; ++a) {
     if (grp == 1) {
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mine[16 * b + r] = a == 0 ? acc[0][b][r] : acc[1][b][r];
+        for (int r = 0; r < 16; ++r) mine[(16 * b + r) * 256] = a == 0 ? acc[0][b][r] : acc[1][b][r];
     }
     __syncthreads();
     if (grp == 0) {
@@ -2739,39 +2848,41 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          if (a == 0) acc[0][b][r] += mine[16 * b + r];
-          else acc[1][b][r] += mine[16 * b + r];
+          if (a == 0) acc[0][b][r] += mine[(16 * b + r) * 256];
+          else acc[1][b][r] += mine[(16 * b + r) * 256];
         }
     }
     __syncthreads();
   }
   const bool sliced = gridDim.y > 1;
   if (colsum && j0 == 0) {
-    *reinterpret_cast<float4*>(tn_lds + (grp * 8 + lk) * 128 + l4) = cs;
+    float* sums = reinterpret_cast<float*>(tn_lds);  // [group][8 rows][128]
+    if (!isb) *reinterpret_cast<float4*>(sums + (grp * 4 + kg) * 128 + 4 * l) = cs;
     __syncthreads();
     if (threadIdx.x < 128 && i0 + (int)threadIdx.x < M) {
-      float v = 0.f;
-      for (int r = 0; r < 16; ++r) v += tn_lds[r * 128 + threadIdx.x];
-      colsum[(sliced ? (int64_t)z * M : 0) + i0 + threadIdx.x] = v;
+      float s = 0.f;
+      for (int r = 0; r < 8; ++r) s += sums[r * 128 + threadIdx.x];
+      colsum[(sliced ? (int64_t)z * M : 0) + i0 + threadIdx.x] = s;
     }
   }
   if (grp == 1) return;
   float* out = sliced ? C + (int64_t)z * M * N : C;
-  const int64_t ld = sliced ? N : ldc;
+  const int64_t ldo = sliced ? N : ldc;
+  const int gj = j0 + 4 * c + eb;
+  const bool pair = ldo % 2 == 0 && ((uintptr_t)out & 7) == 0;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int gj = j0 + wj + 32 * b + c;
-      if (gj >= N) continue;
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int gi = i0 + wi + 32 * a + 8 * g + 4 * h + e;
-          if (gi >= M) continue;
-          out[(int64_t)gi * ld + gj] = acc[a][b][4 * g + e];
-        }
+    for (int r = 0; r < 16; ++r) {
+      const int gi = i0 + 4 * (8 * (r >> 2) + 4 * h + (r & 3)) + ea + a;
+      if (gi >= M || gj >= N) continue;
+      float* o = out + (int64_t)gi * ldo + gj;
+      if (pair && gj + 1 < N) {
+        *reinterpret_cast<float2*>(o) = float2{acc[a][0][r], acc[a][1][r]};
+      } else {
+        o[0] = acc[a][0][r];
+        if (gj + 1 < N) o[1] = acc[a][1][r];
+      }
     }
 }
 
@@ -2901,27 +3012,21 @@ static void sgemm_go(hipStream_t s, SgemmArgs g) {
   hipLaunchKernelGGL((sgemm_kernel<A_KC, B_KC, TN ? 16 : 4>), dim3(tiles.x, tiles.y, (unsigned)slices), dim3(TN ? 1024 : 256), 0, s, g);
 }
 
-// C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single wide
-// fp32 layer.  The rows are cut so that about 512 workgroups, two per CU, share them.
-static int sgemm_tn128(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
-                       int64_t ldc, float* part, float* colsum, float* colpart) {
-  const bool vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && M % 128 == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0 && N % 128 == 0;
+// C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single layer.
+template <int PARTS>
+static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
+                 int64_t ldc, float* part, float* colsum) {
+  const bool vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && M % 4 == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0 && N % 4 == 0;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  int slices = 1;
-  if (K >= 2048) {
-    slices = (int)((512 + tiles - 1) / tiles);
-    if (slices > kTnMaxSlices) slices = kTnMaxSlices;
-    if ((int64_t)slices * 256 > K) slices = (int)(K / 256);
-  }
-  int kslice = (int)((K + slices - 1) / slices);
-  kslice = (kslice + 31) / 32 * 32;
-  slices = (int)((K + kslice - 1) / kslice);
-  if (slices > 1) slices = (slices + 7) / 8 * 8;  // for the XCD mapping; slices past the last row add zeros
-  auto kfn = vec_a ? (vec_b ? sgemm_tn128_kernel<true, true> : sgemm_tn128_kernel<true, false>)
-                   : (vec_b ? sgemm_tn128_kernel<false, true> : sgemm_tn128_kernel<false, false>);
-  if (hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, kTnLds) != hipSuccess)
-    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", kTnLds);
-  hipLaunchKernelGGL(kfn, dim3((unsigned)tiles, (unsigned)slices), dim3(512), kTnLds, s, (int)M, N, (int)K, A, lda, B, ldb,
+  const int slices = wgrad_slices(M, N, K);
+  const int kslice = (int)(((K + slices - 1) / slices + 2 * kTnKB - 1) / (2 * kTnKB)) * 2 * kTnKB;  // slices past the last row add zeros
+  constexpr int lds = 2 * tn_buf(PARTS) * 16;
+  float* colpart = part + (int64_t)slices * M * N;
+  auto kfn = vec_a ? (vec_b ? wgrad_kernel<PARTS, true, true> : wgrad_kernel<PARTS, true, false>)
+                   : (vec_b ? wgrad_kernel<PARTS, false, true> : wgrad_kernel<PARTS, false, false>);
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)tiles, (unsigned)slices), dim3(512), lds, s, (int)M, N, (int)K, A, lda, B, ldb,
                      slices > 1 ? part : C, ldc, kslice, slices > 1 ? colpart : colsum);
   if (slices > 1)
     hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((M * N + 63) / 64 + (M + 63) / 64)), dim3(256), 0, s, (int)M, N, slices, part, C, ldc,

@@ -726,3 +726,56 @@ def test_weight_gradient_of_a_single_layer_over_many_rows(dims, M):
     bound = 8 * 2.0 ** -24 * max(np.sqrt(M) * np.sqrt(M), 1.0)
     assert np.abs(gw.cpu().numpy() - want).max() < max(bound, 1e-5)
     assert np.abs(gb.cpu().numpy() - dy.astype(np.float64).sum(0)).max() < max(bound, 1e-5)
+
+
+def _bf16(a):
+    return torch.tensor(a).to(torch.bfloat16).double().numpy()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("dims,M", [
+    ((128, 384), 1), ((128, 384), 63), ((128, 510), 65),       # less than a stage per group; widths of no whole tile
+    ((43, 128), 1000), ((340, 128), 2051), ((17, 40), 385),    # rows on no 16-byte boundary, an odd number of 16-wide input steps
+    ((128, 1), 12288), ((128, 20), 16385), ((512, 512), 5000),
+])
+def test_both_gradients_of_a_single_layer(dims, M, dtype):
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims) + M)
+    w, b = rng.normal(size=(dims[1], dims[0])).astype(np.float32), rng.normal(size=dims[1]).astype(np.float32)
+    x, dy = rng.normal(size=(M, dims[0])).astype(np.float32), rng.normal(size=(M, dims[1])).astype(np.float32)
+    net = MLP([w], [b], activation="none", dtype=dtype)
+    net.train_init()
+    xd, dyd = t32(x), t32(dy)
+    net.train_forward(xd)
+    dx = torch.full_like(xd, float("nan"))
+    net.backward_dx(xd, dyd, dx)
+    gw, gb = net.parameters(gradients=True)[0]
+    x64, dy64, w64 = (_bf16(a) if dtype == "bf16" else a.astype(np.float64) for a in (x, dy, w))
+    # sums of n products of size one: n roundings of 2^-24 of a partial sum of size sqrt(n), as a random walk, 8 deviations
+    bound = lambda n: 8 * 2.0 ** -24 * max(n, 16)  # noqa: E731
+    assert np.abs(gw.cpu().numpy() - dy64.T @ x64).max() < bound(M)
+    assert np.abs(gb.cpu().numpy() - dy.astype(np.float64).sum(0)).max() < bound(M)
+    assert np.abs(dx.cpu().numpy() - dy64 @ w64).max() < bound(dims[1])
+
+
+def test_cut_operands_of_the_weight_gradient_keep_the_range_of_fp32():
+    """Values near the largest float, tiny ones, infinities and NaN through the product that cuts fp32 into bf16 parts."""
+    from ksim_amd.mlp import MLP
+
+    M, I, O = 64, 8, 8
+    x, dy = np.zeros((M, I), np.float32), np.zeros((M, O), np.float32)
+    big, tiny = np.float32(3.4e38), np.float32(2.0 ** -100)
+    dy[np.arange(O), np.arange(O)] = 1.0  # row r of x is row r of the gradient
+    x[0] = big; x[1] = -big; x[2] = tiny; x[3] = np.float32(1 + 2.0 ** -23); x[4] = np.inf; x[5] = -np.inf; x[6] = np.nan; x[7] = 0.1
+    dy[8:] = 0.0
+    # infinities and NaN meet the zeros of other columns, which is NaN in any order of the sum: one row at a time
+    net = MLP([np.zeros((O, I), np.float32)], [np.zeros(O, np.float32)], activation="none", dtype="f32")
+    net.train_init()
+    for r in range(8):
+        xr, dr = np.zeros_like(x), np.zeros_like(dy)
+        xr[r], dr[r] = x[r], 1.0
+        net.train_forward(t32(xr))
+        net.backward(t32(xr), t32(dr))
+        gw = net.parameters(gradients=True)[0][0].cpu().numpy()
+        assert np.array_equal(gw, np.broadcast_to(x[r], (O, I)), equal_nan=True), r
