@@ -1,5 +1,5 @@
 // MLP forward and backward on the gfx950 matrix cores: fused GEMM + bias + activation kernels per layer (mlp_layer_kernel: bf16 on
-// v_mfma_f32_32x32x16_bf16, 8 consecutive k per lane; sgemm_layer_kernel: fp32 on v_mfma_f32_32x32x2_f32, 1 k per lane) and
+// v_mfma_f32_32x32x16_bf16, 8 consecutive k per lane; cut_layer_kernel: fp32 on the same instruction, every value in three bf16 parts) and
 // whole-network kernels.  Output fragment layout (both): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "ks_common.h"
 
@@ -12,6 +12,8 @@ namespace ks {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;  // a 16-byte register vector (plain vector type, so arrays of it stay in registers)
 
 constexpr int kBM = 128, kBN = 128;  // kBM: the largest row tile
@@ -194,145 +196,198 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
     }
 }
 
-// fp32 layers: y = act(x W^T + b) on BM x 128 tiles, four wavefronts of BM / 2 x 64 each.  Operands pass through LDS transposed,
-// [k][row] with a stride of BM + 4 (128 + 4) floats, so that a matrix instruction's operand is one conflict-free 4-byte read per lane
-// (row-major, its 32 rows fall into 8 banks); a 16-byte load along k becomes four 4-byte writes into 64 different banks.  The LDS
-// buffer is double: stage n + 1 is written and stage n + 2 requested while stage n is multiplied, one barrier per 16 steps, and a
-// step's operands are read before the previous step's products.  At most 128 registers: four wavefronts per SIMD.
-// Every fp32 forward kernel here starts from the bias and adds the products in one order (k = 8 g + e and 8 g + 4 + e together, e = 0..3,
-// then the next g), so a row's numbers do not depend on the batch it comes in or the kernel that batch takes.
-//   102400 x 128 -> 512: 173 -> 163 us, of 87 in matrix instructions
+// ---------------------------------------------------------------- fp32 products on the bf16 matrix instruction
+// An fp32 value is cut into three bf16 values whose sum is the value itself: its upper 16 bits (8 bits of mantissa, so infinities and NaN
+// stay in the first part), the rest rounded to bf16, and what that leaves, which is at most 8 bits.  Of the nine products of two cut values
+// the six that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding per 16 k where the
+// fp32 instruction has eight, the other five, 2^-7 of it, in a second one.  Six instructions replace eight of twice their time.
+__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+
+// eight values to PARTS fragments; PARTS = 1 rounds them to bf16
+template <int PARTS>
+__device__ __forceinline__ void cut_bf16(const float (&v)[8], u32x4 (&out)[PARTS]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float a = v[2 * q], b = v[2 * q + 1];
+    if constexpr (PARTS == 1) {
+      out[0][q] = pack_bf16(a, b);
+    } else {
+      const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+      out[0][q] = __builtin_amdgcn_perm(ub, ua, 0x07060302);  // the upper halves
+      a -= __builtin_bit_cast(float, ua & 0xffff0000u);
+      b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+      const unsigned w = pack_bf16(a, b);
+      out[1][q] = w;
+      out[2][q] = pack_bf16(a - __builtin_bit_cast(float, w << 16), b - __builtin_bit_cast(float, w & 0xffff0000u));
+    }
+  }
+}
+
+template <int MI, int NJ>
+__device__ __forceinline__ void mma_bf16(const bf16x8 (&a)[MI], const bf16x8 (&b)[NJ], f32x16 (&acc)[MI][NJ]) {
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+}
+
+// The order of the six is part of a result's bits: every kernel that multiplies cut values goes through here, 16 k after 16 k.
+template <int MI, int NJ>
+__device__ __forceinline__ void mma_cut(const bf16x8 (&a)[3][MI], const bf16x8 (&b)[3][NJ], f32x16 (&acc)[MI][NJ], f32x16 (&low)[MI][NJ]) {
+  mma_bf16(a[2], b[0], low);
+  mma_bf16(a[0], b[2], low);
+  mma_bf16(a[1], b[1], low);
+  mma_bf16(a[1], b[0], low);
+  mma_bf16(a[0], b[1], low);
+  mma_bf16(a[0], b[0], acc);
+}
+
+// Where the products overflow, or an operand was infinite or NaN, the first parts alone decide: the others of an infinity are NaN.
+__device__ __forceinline__ float join_cut(float acc, float low) { return fabsf(acc) < __builtin_inff() ? acc + low : acc; }
+
+template <int ACT, int MI>
+__device__ __forceinline__ void activate_tiles(f32x16 (&acc)[MI][2]) {
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = activate<ACT, false>(acc[i][j][r]);
+}
+
+// fp32 layers: y = act(x W^T + b) on BM x 128 tiles, four wavefronts of BM / 2 x 64 each, operands cut on their way to LDS.  A stage is
+// 32 k: thread t cuts the fragment q = t % 4 of rows t / 4 + 64 r, k = 16 (q / 2) + 4 (q % 2) + {0..3, 8..11}, so that four neighbouring
+// lanes read 128 bytes of a row in two loads.  A part's fragments lie [q][row] with two spare ones per q: neighbouring lanes write into
+// different banks and a matrix instruction's operand is one 16-byte read per lane.  The next stage's rows are requested before the
+// products and stay in flight over the barriers.  BM = 128: two workgroups per CU, one cutting while the other multiplies.
+//   102400 x 128 -> 512: 163 -> 109 us, 102400 x 512 -> 128: 139 -> 98 (137 TFLOP/s; on the fp32 instruction, whose time alone is 87 us), of
+//   40 in matrix instructions and 45 of memory traffic; relative error against 64 bits 2.0e-7 -> 0.7e-7 and 4.0e-7 -> 1.3e-7
+// Every fp32 kernel of a single layer starts from the bias and adds the products in one order (mma_cut), so a row's numbers do not depend
+// on the batch it comes in or the kernel that batch takes.
 // x (M, Kreal) with row stride ldx; K: Kreal padded to 32 (W's stride; its padding is zero).  Columns of y past Nreal are not written when y is
 // the caller's (LAST); otherwise y is as wide as the padded layer.  gridDim.z > 1 (LAST): slice z of the reduction goes to its own copy
 // of the output.
 template <int BM, bool VA>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void sgemm_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __restrict__ x, int64_t ldx, const float* __restrict__ W,
-                        const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, int act) {
-  constexpr int LA = BM + 4, LB = 132, MI = BM / 64, AV = BM / 64;
-  __shared__ __attribute__((aligned(16))) float As[2][16 * LA], Bs[2][16 * LB];
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 2 : 3, BM == 128 ? 2 : 3)))
+void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __restrict__ x, int64_t ldx, const float* __restrict__ W,
+                      const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, int act) {
+  constexpr int LA = BM + 2, LB = 128 + 2, MI = BM / 64, AV = BM / 64;
+  __shared__ u32x4 As[3 * 4 * LA], Bs[3 * 4 * LB];  // [part][q][row]
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 31, h = lane >> 5;
   // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
   // other, so that its rows are fetched once.  Row tiles past the last whole eight follow in plain order.
-  int64_t m_tile = blockIdx.x;
-  int n_tile = blockIdx.y;
-  if (gridDim.y > 1) {
-    const int64_t l = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, whole = (int64_t)(gridDim.x & ~7u) * gridDim.y;
-    const int64_t q = l < whole ? l >> 3 : l - whole;
-    n_tile = (int)(q % gridDim.y);
-    m_tile = l < whole ? (q / gridDim.y) * 8 + (l & 7) : (int64_t)(gridDim.x & ~7u) + q / gridDim.y;
+  unsigned m_tile = blockIdx.x, n_tile = blockIdx.y;
+  if (gridDim.y > 1) {  // tiles of an output that fits the card's memory: 32 bits
+    const unsigned l = blockIdx.y * gridDim.x + blockIdx.x, rows8 = gridDim.x & ~7u, whole = rows8 * gridDim.y;
+    const unsigned q = l < whole ? l >> 3 : l - whole, d = q / gridDim.y;
+    n_tile = q - d * gridDim.y;
+    m_tile = l < whole ? d * 8 + (l & 7) : rows8 + d;
   }
-  const int64_t m0 = m_tile * BM;
-  const int n0 = n_tile * 128;
+  const int64_t m0 = (int64_t)m_tile * BM;
+  const int n0 = (int)n_tile * 128;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 64;
-  f32x16 acc[MI][2];
+  f32x16 acc[MI][2], low[MI][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const float b = blockIdx.z == 0 ? bias[n0 + wn + 32 * j + c] : 0.f;  // padded to whole tiles
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = b;
+      for (int r = 0; r < 16; ++r) { acc[i][j][r] = b; low[i][j][r] = 0.f; }
   }
-  const int kslice = K / (int)gridDim.z, kbeg = (int)blockIdx.z * kslice, stages = kslice / 16;
-  // thread t loads rows t / 4 + 64 r, four steps from 4 (t % 4); rows past the batch repeat the last one, their results are dropped
-  const int lrow = t >> 2, lk = (t & 3) * 4;
+  const int kslice = K / (int)gridDim.z, kbeg = (int)blockIdx.z * kslice, stages = kslice / 32;
+  // rows past the batch repeat the last one, their results are dropped
+  const int lrow = t >> 2, q = t & 3, lk = kbeg + 16 * (q >> 1) + 4 * (q & 1);
   const float* pa[AV];
 #pragma unroll
   for (int r = 0; r < AV; ++r) {
     const int64_t m = m0 + lrow + 64 * r;
-    pa[r] = x + (m < M ? m : M - 1) * ldx + kbeg + lk;
+    pa[r] = x + (m < M ? m : M - 1) * ldx;
   }
-  const float* pb = W + (int64_t)(n0 + lrow) * K + kbeg + lk;
+  const float* pb = W + (int64_t)(n0 + lrow) * K + lk;
   const int64_t b64 = (int64_t)64 * K;
-  float4 ra[AV], rb[2];
+  float4 ra[AV][2], rb[2][2];
   auto fetch = [&](int n) __attribute__((always_inline)) {
-    const int k = 16 * n;
 #pragma unroll
-    for (int r = 0; r < AV; ++r) {
-      const float* q = pa[r] + k;
-      const int left = Kreal - (kbeg + lk + k);  // steps of the row still inside the input (VA: a multiple of four)
-      if (VA) {
-        ra[r] = float4{0.f, 0.f, 0.f, 0.f};
-        if (left > 0) ra[r] = *reinterpret_cast<const float4*>(q);
-      } else {
-        ra[r] = float4{left > 0 ? q[0] : 0.f, left > 1 ? q[1] : 0.f, left > 2 ? q[2] : 0.f, left > 3 ? q[3] : 0.f};
+    for (int u = 0; u < 2; ++u) {
+      const int k = lk + 32 * n + 8 * u, left = Kreal - k;  // steps of the row still inside the input (VA: a multiple of four)
+#pragma unroll
+      for (int r = 0; r < AV; ++r) {
+        const float* at = pa[r] + k;
+        ra[r][u] = float4{0.f, 0.f, 0.f, 0.f};
+        if (VA) {
+          if (left > 0) ra[r][u] = *reinterpret_cast<const float4*>(at);
+        } else {
+          if (left > 0) ra[r][u].x = at[0];
+          if (left > 1) ra[r][u].y = at[1];
+          if (left > 2) ra[r][u].z = at[2];
+          if (left > 3) ra[r][u].w = at[3];
+        }
       }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) rb[r][u] = *reinterpret_cast<const float4*>(pb + r * b64 + 32 * n + 8 * u);
     }
-    rb[0] = *reinterpret_cast<const float4*>(pb + k);
-    rb[1] = *reinterpret_cast<const float4*>(pb + b64 + k);
   };
-  auto put = [&](int buf) __attribute__((always_inline)) {
+  auto cut = [&](const float4 (&f)[2], u32x4* to, int stride) __attribute__((always_inline)) {
+    const float v[8] = {f[0].x, f[0].y, f[0].z, f[0].w, f[1].x, f[1].y, f[1].z, f[1].w};
+    u32x4 part[3];
+    cut_bf16<3>(v, part);
 #pragma unroll
-    for (int r = 0; r < AV; ++r) {
-      float* q = &As[buf][lk * LA + lrow + 64 * r];
-      q[0] = ra[r].x; q[LA] = ra[r].y; q[2 * LA] = ra[r].z; q[3 * LA] = ra[r].w;
-    }
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      float* q = &Bs[buf][lk * LB + lrow + 64 * r];
-      q[0] = rb[r].x; q[LB] = rb[r].y; q[2 * LB] = rb[r].z; q[3 * LB] = rb[r].w;
-    }
+    for (int p = 0; p < 3; ++p) to[p * 4 * stride] = part[p];
   };
   fetch(0);
-  put(0);
-  if (stages > 1) fetch(1);
-  __syncthreads();
   for (int n = 0; n < stages; ++n) {
-    const float* A = &As[n & 1][4 * h * LA + wm + c];
-    const float* B = &Bs[n & 1][4 * h * LB + wn + c];
-    float fa[2][MI], fb[2][2];
+    if (n > 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS only: the requested rows stay in flight
 #pragma unroll
-    for (int i = 0; i < MI; ++i) fa[0][i] = A[32 * i];
-    fb[0][0] = B[0]; fb[0][1] = B[32];
-    if (n + 1 < stages) {
-      put((n + 1) & 1);
-      if (n + 2 < stages) fetch(n + 2);
-    }
-#define KS_STEP(S) (8 * ((S) >> 2) + ((S) & 3))  // the lower k of step S of a stage
+    for (int r = 0; r < AV; ++r) cut(ra[r], As + q * LA + lrow + 64 * r, LA);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int q = s & 1;
-      if (s < 7) {
+    for (int r = 0; r < 2; ++r) cut(rb[r], Bs + q * LB + lrow + 64 * r, LB);
+    if (n + 1 < stages) fetch(n + 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < MI; ++i) fa[q ^ 1][i] = A[KS_STEP(s + 1) * LA + 32 * i];
-        fb[q ^ 1][0] = B[KS_STEP(s + 1) * LB]; fb[q ^ 1][1] = B[KS_STEP(s + 1) * LB + 32];
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 fa[3][MI], fb[3][2];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[p][i] = __builtin_bit_cast(bf16x8, As[(p * 4 + 2 * s + h) * LA + wm + 32 * i + c]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[p][j] = __builtin_bit_cast(bf16x8, Bs[(p * 4 + 2 * s + h) * LB + wn + 32 * j + c]);
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][i], fb[q][j], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+      mma_cut(fa, fb, acc, low);
     }
-#undef KS_STEP
-    __syncthreads();
   }
-  float* out = y + (int64_t)blockIdx.z * M * ldy;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn + 32 * j + c;
-      if (col >= Nreal) continue;
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (row >= M) continue;
-        float v = acc[i][j][r];
-        switch (act) {
-          case KS_ACT_ELU: v = activate<KS_ACT_ELU, false>(v); break;
-          case KS_ACT_RELU: v = activate<KS_ACT_RELU, false>(v); break;
-          case KS_ACT_TANH: v = activate<KS_ACT_TANH, false>(v); break;
-          case KS_ACT_GELU: v = activate<KS_ACT_GELU, false>(v); break;
-          default: break;
-        }
-        out[row * ldy + col] = v;
-      }
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = join_cut(acc[i][j][r], low[i][j][r]);
+  switch (act) {
+    case KS_ACT_ELU: activate_tiles<KS_ACT_ELU>(acc); break;
+    case KS_ACT_RELU: activate_tiles<KS_ACT_RELU>(acc); break;
+    case KS_ACT_TANH: activate_tiles<KS_ACT_TANH>(acc); break;
+    case KS_ACT_GELU: activate_tiles<KS_ACT_GELU>(acc); break;
+    default: break;
+  }
+  // one row of the tile after the other: uniform steps from one address per lane
+  const int64_t row0 = m0 + wm + 4 * h;
+  const int col = n0 + wn + c;
+  float* out = y + ((int64_t)blockIdx.z * M + row0) * ldy + col;
+  const bool on0 = col < Nreal, on1 = col + 32 < Nreal, whole = m0 + BM <= M;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int down = 32 * i + 8 * (r >> 2) + (r & 3);
+      const bool on = whole || row0 + down < M;
+      float* o = out + down * ldy;
+      if (on && on0) o[0] = acc[i][0][r];
+      if (on && on1) o[32] = acc[i][1][r];
     }
 }
-
-
 
 // ---------------------------------------------------------------- matrix-core yardstick
 // Nothing but 32x32x16 bf16 MFMAs on register operands: eight independent accumulator tiles per wavefront (the fused
@@ -353,6 +408,70 @@ struct SmallLayer {
   float* y;
   int64_t ldy;
 };
+
+// A single fp32 layer over few rows: the same tiles, products of cut values (mma_cut) in cut_layer_kernel's order.  Bound by latency: 4096 x
+// 128 -> 40: 11.1 -> 6.3 us.
+__global__ __launch_bounds__(256) void cut_small_kernel(int64_t M, SmallLayer p) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
+  const int j = (int)blockIdx.x * 4 + wave;
+  if (j >= p.nt) return;
+  const int64_t m0 = (int64_t)blockIdx.y * 32, m = m0 + c < M ? m0 + c : M - 1;  // rows past the batch repeat the last one
+  f32x16 acc[1][1], low[1][1];
+  const float b = p.bp[32 * j + c];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) { acc[0][0][r] = b; low[0][0][r] = 0.f; }
+  const float* xr = p.x + m * p.ldx;
+  const u32x4* wr = p.Wp + (int64_t)j * p.nk * 64 + lane;
+  typedef __attribute__((ext_vector_type(4))) float f32x4v;
+  const int steps = (p.nk + 1) / 2, last = p.Kreal - 1;  // a step is two groups of 8 k
+  constexpr int PF = 4;
+  f32x4v xf[PF][2], wf[PF][2];
+  // groups past the end and columns past the row's end load something valid and count as zero
+  auto request = [&](int u, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int g = 2 * s + e < p.nk ? 2 * s + e : p.nk - 1, k = 8 * g + 4 * h;
+      if (p.vec) xf[u][e] = *reinterpret_cast<const f32x4v*>(xr + (k < last - 3 ? k : last - 3));
+      else xf[u][e] = f32x4v{xr[k < last ? k : last], xr[k + 1 < last ? k + 1 : last], xr[k + 2 < last ? k + 2 : last], xr[k + 3 < last ? k + 3 : last]};
+      wf[u][e] = __builtin_bit_cast(f32x4v, wr[(int64_t)g * 64]);
+    }
+  };
+  auto step = [&](int u, int s) __attribute__((always_inline)) {
+    float xv[8], wv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int k = 16 * s + 8 * (e >> 2) + 4 * h + (e & 3);
+      xv[e] = k < p.Kreal ? xf[u][e >> 2][e & 3] : 0.f;
+      wv[e] = k < p.Kreal ? wf[u][e >> 2][e & 3] : 0.f;
+    }
+    u32x4 xp[3], wp[3];
+    cut_bf16<3>(xv, xp);
+    cut_bf16<3>(wv, wp);
+    bf16x8 a[3][1], w[3][1];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) { a[q][0] = __builtin_bit_cast(bf16x8, xp[q]); w[q][0] = __builtin_bit_cast(bf16x8, wp[q]); }
+    mma_cut(a, w, acc, low);
+  };
+#pragma unroll
+  for (int u = 0; u < PF; ++u) request(u, u);
+  int s = 0;
+  for (; s + PF <= steps; s += PF)
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      step(u, s + u);
+      request(u, s + u + PF);
+    }
+#pragma unroll
+  for (int u = 0; u < PF; ++u)
+    if (s + u < steps) step(u, s + u);
+  const int col = 32 * j + c;
+  if (col >= p.Nreal) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int64_t row = m0 + 8 * (r >> 2) + 4 * h + (r & 3);
+    if (row < M) p.y[row * p.ldy + col] = join_cut(acc[0][0][r], low[0][0][r]);
+  }
+}
 
 template <int SHARE>
 __global__ __launch_bounds__(256) void sgemm_small_kernel(int64_t M, SmallLayer p0, SmallLayer p1) {
@@ -507,13 +626,6 @@ struct FusedArgs {
 #define KS_MLP_STAMP(k)
 #define KS_MLP_STAMP2(k)
 #endif
-
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-
-__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
-}
 
 // One fragment step of both operands: 16 k of bf16 in one matrix instruction, or 8 k of fp32 in four (lane half h holds k = 8 step +
 // 4 h + e in element e, so instruction e multiplies k = 8 step + e and 8 step + 4 + e); 16 bytes of each operand per lane either way.
@@ -1480,14 +1592,14 @@ static int launch_layer_tile(int act, hipStream_t s, int64_t M, int npad, int K,
   return KS_OK;
 }
 
-// fp32 layers.  A launch ends with the CU that got most of the tiles: below eight 128-row tiles per CU, 64-row ones leave less of a last
-// round (102400 x 512 -> 128: 151 -> 137 us) and keep small batches on more CUs.
+// fp32 layers.  128-row tiles from one and a half per CU on: fewer leave CUs idle (25600 x 512 -> 128, 200 tiles: 34.6 us of 64-row tiles'
+// 30.8; 51200, 400 tiles: 49.0 of 58.8; 16384 x 128 -> 512, 512 tiles: 19.3 of 21.3).
 static int launch_layer_f32(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x, int64_t ldx, const void* W,
                             const float* b, void* y, int64_t ldy, int ksplit = 1) {
-  const bool small = (M + 127) / 128 * (npad / kBN) * ksplit < 2048;
+  const bool small = (M + 127) / 128 * (npad / kBN) * ksplit < 400;
   const bool va = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && Kreal % 4 == 0;
-  auto kfn = small ? (va ? sgemm_layer_kernel<64, true> : sgemm_layer_kernel<64, false>)
-                   : (va ? sgemm_layer_kernel<128, true> : sgemm_layer_kernel<128, false>);
+  auto kfn = small ? (va ? cut_layer_kernel<64, true> : cut_layer_kernel<64, false>)
+                   : (va ? cut_layer_kernel<128, true> : cut_layer_kernel<128, false>);
   const int bm = small ? 64 : 128;
   hipLaunchKernelGGL(kfn, dim3((unsigned)((M + bm - 1) / bm), (unsigned)(npad / kBN), (unsigned)ksplit), dim3(256), 0, s, M, K, Kreal, Nreal,
                      (const float*)x, ldx, (const float*)W, b, (float*)y, ldy, act);
@@ -1749,11 +1861,11 @@ static int launch_fused_pair_tile(const DevMlp& m0, const DevMlp& m1, hipStream_
 
 // Whether M rows go through the small-batch kernel.  Networks of several layers: up to 2048 rows (one tile per SIMD at 512 wide) where the
 // whole-network kernel gives its wavefronts two tiles of a layer (68-512-512-512-20: 83 -> 52 us at 256 rows, 61 at 2048; 256 wide it takes 30
-// to this one's 40).  Single layers: up to 2048 tiles, two per SIMD; past that the reuse in the per-layer kernel's larger tiles wins
-// (128 -> 512: 12.0 us of 13.3 at 4096 rows, 21.1 of 17.8 at 8192).
+// to this one's 40).  Single layers: up to 1024 tiles, one per SIMD; past that the reuse in the per-layer kernel's larger tiles wins
+// (128 -> 512: 7.3 us at 2048 rows, 10.9 of 9.0 at 4096; 475 -> 128: 29.2 at 8192 rows, 49.2 of 25 at 16384).
 static bool small_ok(const DevMlp& m, int64_t M) {
   if (m.dtype != KS_MLP_F32 || !m.Wp[0]) return false;
-  if (m.n_layers == 1) return (M + 31) / 32 * m.fn[0] <= 2048;
+  if (m.n_layers == 1) return (M + 31) / 32 * m.fn[0] <= 1024;
   int wide = 0;
   for (int l = 0; l + 1 < m.n_layers; ++l) wide = m.fn[l] > wide ? m.fn[l] : wide;
   return wide > kFusedWaves && M <= 2048;
@@ -1792,6 +1904,10 @@ static int launch_small(const DevMlp& a, const DevMlp* b, hipStream_t s, int64_t
     const int sa = a.n_layers > 1 && p.nt <= 2 ? fused_share(p.nt, a.lda) : 1, sb = b ? (q.nt <= 2 ? fused_share(q.nt, b->lda) : 1) : sa;
     auto go = [&](int share, const SmallLayer& u, const SmallLayer& v, int n, int tiles) {
       const dim3 grid((unsigned)((tiles * share + 3) / 4), (unsigned)((M + 31) / 32), (unsigned)n);
+      if (a.n_layers == 1) {
+        hipLaunchKernelGGL(cut_small_kernel, grid, dim3(256), 0, s, M, u);
+        return;
+      }
       auto kfn = share == 4 ? sgemm_small_kernel<4> : (share == 2 ? sgemm_small_kernel<2> : sgemm_small_kernel<1>);
       hipLaunchKernelGGL(kfn, grid, dim3(256), 0, s, M, u, v);
     };
@@ -2669,10 +2785,8 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
 }
 
 // The weight and bias gradient of a single layer over many rows, C(i, j) = sum_k A(k, i) B(k, j) with both operands fp32 and stored
-// (k, .), on the bf16 matrix instruction.  PARTS = 1: operands rounded to bf16, what a bf16 network's products take.  PARTS = 3: every
-// fp32 value is cut into three bf16 values whose sum is the value itself (8 + 8 + 8 bits), and of the nine products of two cut values
-// the six that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding per 16 rows where the
-// fp32 instruction has eight, the other five, 2^-8 of it, in a second one.
+// (k, .), on the bf16 matrix instruction.  PARTS = 1: operands rounded to bf16, what a bf16 network's products take.  PARTS = 3: fp32, every
+// value cut in three (cut_bf16, mma_cut).
 // A 128 x 128 tile per workgroup of two groups of four wavefronts; each group takes half of the slice's rows in stages of 32 and each of
 // its wavefronts a 64 x 64 block.  The groups take turns: while one multiplies out of its LDS buffer the other cuts the stage it has in
 // registers, writes it to its own and requests the next, so a SIMD has one wavefront of matrix work and one of vector work at any time.
@@ -2689,33 +2803,6 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
 // VA / VB: the operand's rows are 16-byte aligned and its width is a multiple of four.
 constexpr int kTnKB = 32;  // rows of a stage
 __host__ __device__ constexpr int tn_buf(int parts) { return parts * (kTnKB / 8) * 256; }  // one group's LDS buffer, in 16-byte fragments
-
-// Eight values of a column to PARTS fragments.  The clamp keeps a value that would round up to infinity finite, and an infinite one in
-// the last part, where its products with the other operand's first part still come out infinite.
-template <int PARTS>
-__device__ __forceinline__ void cut_bf16(const float (&v)[8], u32x4 (&out)[PARTS]) {
-  float x[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = v[e];
-#pragma unroll
-  for (int p = 0; p < PARTS; ++p) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float a = x[2 * q], b = x[2 * q + 1];
-      if (p + 1 < PARTS) {
-        constexpr float kBf16Max = 3.3895313892515355e38f;
-        a = __builtin_amdgcn_fmed3f(a, -kBf16Max, kBf16Max);
-        b = __builtin_amdgcn_fmed3f(b, -kBf16Max, kBf16Max);
-      }
-      const unsigned w = pack_bf16(a, b);
-      out[p][q] = w;
-      if (p + 1 < PARTS) {
-        x[2 * q] -= __builtin_bit_cast(float, w << 16);
-        x[2 * q + 1] -= __builtin_bit_cast(float, w & 0xffff0000u);
-      }
-    }
-  }
-}
 
 template <int PARTS, bool VA, bool VB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -2802,14 +2889,8 @@ void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
           fa[p][q] = __builtin_bit_cast(bf16x8, at_k[32 * (ea + q)]);
           fb[p][q] = __builtin_bit_cast(bf16x8, at_k[128 + 32 * (eb + q)]);
         }
-#define KS_MMA(ACC, P, Q)                                                                                            \
-  _Pragma("unroll") for (int a = 0; a < 2; ++a) _Pragma("unroll") for (int b = 0; b < 2; ++b) ACC[a][b] =            \
-      __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[P][a], fb[Q][b], ACC[a][b], 0, 0, 0);
-      if constexpr (PARTS == 3) {
-        KS_MMA(low, 2, 0) KS_MMA(low, 0, 2) KS_MMA(low, 1, 1) KS_MMA(low, 1, 0) KS_MMA(low, 0, 1)
-      }
-      KS_MMA(acc, 0, 0)
-#undef KS_MMA
+      if constexpr (PARTS == 3) mma_cut(fa, fb, acc, low);
+      else mma_bf16(fa[0], fb[0], acc);
     }
   };
   if (stages > 0) fetch(0);
@@ -2832,7 +2913,7 @@ void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[a][b][r] += low[a][b][r];
+        for (int r = 0; r < 16; ++r) acc[a][b][r] = join_cut(acc[a][b][r], low[a][b][r]);
   // the second group hands its tile over in two halves through the buffers, which are free now
   float* mine = reinterpret_cast<float*>(tn_lds) + t;
   for (int a = 0; a < 2; ++a) {

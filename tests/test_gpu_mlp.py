@@ -93,19 +93,24 @@ def test_paired_forward_equals_two_single_forwards(M):
     (68, 512, 512, 512, 20),      # output tile cut over four wavefronts
     (71, 256, 256, 256, 33),      # two output tiles, two wavefronts each; rows of the input on no 16-byte boundary
     (5, 40, 3), (33, 130, 130, 2),
-    (128, 512), (97, 140),        # single layers: 2048 tiles are the last batch of the kernel for few rows
+    (128, 512), (97, 140), (475, 128), (40, 1),  # single layers: 1024 tiles are the last batch of the kernel for few rows
 ])
 def test_fp32_batches_of_every_size_give_a_row_the_same_bits(dims):
-    """Few rows (32 x 32 tiles, a launch per layer), 32-row and 64-row whole-network tiles, per-layer tiles: the last row count of one
-    kernel and the first of the next, ragged ends included."""
+    """Few rows (32 x 32 tiles, a launch per layer), 32-row and 64-row whole-network tiles, per-layer tiles of 64 and 128 rows: the last row
+    count of one kernel and the first of the next, ragged ends included."""
     from ksim_amd.mlp import MLP
 
     rng = np.random.default_rng(sum(dims))
     ws = [rng.normal(scale=1 / np.sqrt(i), size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])]
     bs = [rng.normal(scale=0.1, size=o).astype(np.float32) for o in dims[1:]]
     net = MLP(ws, bs, activation="elu", dtype="f32")
-    edge = 2048 // ((dims[1] + 31) // 32) * 32 if len(dims) == 2 else 2048
-    sizes = sorted({1, 31, 33, 65, edge, edge + 1, 4000, 16383, 16384 + 37})
+    sizes = {1, 31, 33, 65, 4000, 16383, 16384 + 37}
+    if len(dims) == 2:
+        few, wide = 1024 // ((dims[1] + 31) // 32) * 32, 400 // ((dims[1] + 127) // 128) * 128
+        sizes |= {few, few + 1, wide - 128, wide + 37}
+    else:
+        sizes |= {2048, 2049}
+    sizes = sorted(sizes)
     x = rng.normal(size=(max(sizes), dims[0])).astype(np.float32)
     X = torch.from_numpy(x).to(DEV)
     want = reference(x, ws, bs, "elu", False)
@@ -118,3 +123,25 @@ def test_fp32_batches_of_every_size_give_a_row_the_same_bits(dims):
         other = MLP(ws, bs, activation="elu", dtype="f32")
         net.forward_pair(X[:M].contiguous(), y0, other, X[-M:].contiguous(), y1)
         assert torch.equal(y0, full[:M]) and torch.equal(y1, full[-M:]), M
+
+
+@pytest.mark.parametrize("M", [1, 33, 4000, 20000])
+def test_single_fp32_layers_keep_the_range_of_fp32(M):
+    """Single layers multiply operands cut into bf16 parts: values near the largest float, tiny ones, infinities, NaN and products that
+    overflow come out as the fp32 product has them."""
+    from ksim_amd.mlp import MLP
+
+    values = np.array([3.4028235e38, -3.4028235e38, 3.3961776e38, 2.0 ** -100, 1 + 2.0 ** -23, np.inf, -np.inf, np.nan, 0.1], np.float32)
+    weights = np.array([1.0, -1.0, 301.3, -0.0013, 1.0 + 2.0 ** -20], np.float32)
+    w = np.zeros((200, 20), np.float32)
+    w[:, 3] = np.resize(weights, 200)
+    x = np.zeros((M, 20), np.float32)
+    x[:, 3] = np.resize(values, M)
+    y = MLP([w], [np.zeros(200, np.float32)], activation="none", dtype="f32")(torch.from_numpy(x).to(DEV)).cpu().numpy()
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = x[:, 3:4] * w[:, 3][None, :]
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
+    finite = np.isfinite(want)
+    assert np.array_equal(y[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    # six products of 16 significant bits each are exact, the three left out are below 2^-23 together, and five sums round
+    assert np.all(np.abs(y[finite] - want[finite]) <= 2.0 ** -21 * np.abs(want[finite]))
