@@ -629,8 +629,10 @@ struct FusedArgs {
 
 // One fragment step of both operands: 16 k of bf16 in one matrix instruction, or 8 k of fp32 in four (lane half h holds k = 8 step +
 // 4 h + e in element e, so instruction e multiplies k = 8 step + e and 8 step + 4 + e); 16 bytes of each operand per lane either way.
-template <typename T>
+// SWAP: the operands change places, so that a lane holds 16 rows of one feature instead of 16 features of one row; the same sums.
+template <typename T, bool SWAP = false>
 __device__ __forceinline__ f32x16 fused_mma(const u32x4& w, const u32x4& b, f32x16 acc) {
+  if constexpr (SWAP) return fused_mma<T, false>(b, w, acc);
   if constexpr (sizeof(T) == 2) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
   } else {
@@ -645,7 +647,7 @@ __device__ __forceinline__ f32x16 fused_mma(const u32x4& w, const u32x4& b, f32x
 // One layer's MFMA work of one wavefront: NT output tiles (weights w[t]) times MI row tiles.  `arow` points at
 // this lane's activation fragment of K step 0 (row lane % 32 of the first row tile, k half lane / 32).
 // Weight fragments sit in a register ring kPF steps ahead; activation fragments are read one step ahead.
-template <typename T, int NT, int MI, int kPF>
+template <typename T, int NT, int MI, int kPF, bool SWAP = false>
 __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x4* __restrict__ w0,
                                                 const u32x4* __restrict__ w1, int nk, const T* __restrict__ arow,
                                                 int lda) {
@@ -678,7 +680,7 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T>(wf[t], bq[u & 1][i], acc[t][i]);
+        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T, SWAP>(wf[t], bq[u & 1][i], acc[t][i]);
     }
   }
 #pragma unroll
@@ -691,7 +693,7 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T>(rw[u][t], bq[u & 1][i], acc[t][i]);
+        for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T, SWAP>(rw[u][t], bq[u & 1][i], acc[t][i]);
     }
   }
 }
@@ -772,6 +774,22 @@ __device__ __forceinline__ void fused_store_output(const f32x16& acc, float* __r
   }
 }
 
+// The output of a single layer, which the stores bound: with a lane per feature (SWAP) a store is two runs of 128 bytes, with a lane per row
+// 64 pieces of 16 (12288 x 128 -> 384: 13.5 -> 8.3 us, 65536 rows: 44.9 -> 28.3, of 27 at the card's copy rate).  Networks keep a lane per row:
+// their outputs are narrow, and the second form of the last layer cost them 1 %.
+__device__ __forceinline__ void fused_store_output_swapped(const f32x16& acc, float* __restrict__ y, int64_t M, int out_dim, int j, int64_t m0,
+                                                           int lane) {
+  const int col = 32 * j + (lane & 31);
+  if (col >= out_dim) return;
+  const int64_t row0 = m0 + 4 * (lane >> 5);
+  float* dst = y + row0 * out_dim + col;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int down = 8 * (r >> 2) + (r & 3);
+    if (row0 + down < M) dst[(int64_t)down * out_dim] = acc[r];
+  }
+}
+
 // How many wavefronts cut the reduction of a narrow fp32 layer of nt <= 2 tiles (their partial tiles, 4 KB each per row tile, have to fit the
 // activation tile)
 __host__ __device__ inline int fused_share(int nt, int lda) {
@@ -781,7 +799,7 @@ __host__ __device__ inline int fused_share(int nt, int lda) {
 }
 
 // One layer of the whole-network kernel for one wavefront: MFMA work, barrier, epilogue, barrier.
-template <int ACT, typename T, int MI, bool LAST, bool KEEP>
+template <int ACT, typename T, int MI, bool LAST, bool KEEP, bool SWAP = false>
 __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __restrict__ act, int64_t m0, int lane,
                                             int wave, int64_t tile) {
   const int nk = a.fk[l], nt = a.fn[l], lda = a.lda;
@@ -824,23 +842,34 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
     const bool busy = wave < nt * MI;
     const int j = busy ? wave / MI : 0, i = busy ? wave % MI : 0;
     f32x16 acc[2][1];
-    fused_bias_init(acc[0][0], a.bp[l], j, lane);
+    if (SWAP) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][0][r] = a.bp[l][j * 32 + row];
+    } else {
+      fused_bias_init(acc[0][0], a.bp[l], j, lane);
+    }
     acc[1][0] = acc[0][0];
     const u32x4* w0 = a.Wp[l] + (int64_t)j * nk * 64 + lane;
-    if (busy) fused_layer_mma<T, 1, 1, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow + i * 32 * lda, lda);
+    if (busy) fused_layer_mma<T, 1, 1, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow + i * 32 * lda, lda);
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();  // every wavefront has read this layer's input; the tile can be overwritten
     KS_MLP_STAMP2(3 + 3 * l)
     if (busy) {
-      if (LAST) fused_store_output(acc[0][0], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
+      if (SWAP) fused_store_output_swapped(acc[0][0], a.y, a.M, a.out_dim, j, m0 + i * 32, lane);
+      else if (LAST) fused_store_output(acc[0][0], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
       else fused_store_hidden<ACT, T>(acc[0][0], act, lda, j, i * 32 + row, lane);
     }
   } else {
     const int mine = wave < nt ? (wave + kFusedWaves < nt ? 2 : 1) : 0;
     const int j0 = wave < nt ? wave : 0, j1 = wave + kFusedWaves < nt ? wave + kFusedWaves : j0;
     f32x16 acc[2][MI];
-    fused_bias_init(acc[0][0], a.bp[l], j0, lane);
-    fused_bias_init(acc[1][0], a.bp[l], j1, lane);
+    if (SWAP) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) { acc[0][0][r] = a.bp[l][j0 * 32 + row]; acc[1][0][r] = a.bp[l][j1 * 32 + row]; }
+    } else {
+      fused_bias_init(acc[0][0], a.bp[l], j0, lane);
+      fused_bias_init(acc[1][0], a.bp[l], j1, lane);
+    }
 #pragma unroll
     for (int i = 1; i < MI; ++i) {
       acc[0][i] = acc[0][0];
@@ -848,8 +877,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
     }
     const u32x4* w0 = a.Wp[l] + (int64_t)j0 * nk * 64 + lane;
     const u32x4* w1 = a.Wp[l] + (int64_t)j1 * nk * 64 + lane;
-    if (mine == 2) fused_layer_mma<T, 2, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w1, nk, arow, lda);
-    else if (mine == 1) fused_layer_mma<T, 1, MI, (MI == 2 ? 2 : kPF)>(acc, w0, w0, nk, arow, lda);
+    if (mine == 2) fused_layer_mma<T, 2, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w1, nk, arow, lda);
+    else if (mine == 1) fused_layer_mma<T, 1, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow, lda);
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();
     KS_MLP_STAMP2(3 + 3 * l)
@@ -859,7 +888,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
         const int j = t == 0 ? j0 : j1;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-          if (LAST) fused_store_output(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
+          if (SWAP) fused_store_output_swapped(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32, lane);
+          else if (LAST) fused_store_output(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
           else fused_store_hidden<ACT, T>(acc[t][i], act, lda, j, i * 32 + row, lane,
                                        (KEEP && MI == 4) ? a.keep_t[l] + m0 + i * 32 + row : nullptr, a.ldt);
         }
@@ -881,7 +911,7 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
   }
 }
 
-template <int ACT, typename T, int BM, bool KEEP = false>
+template <int ACT, typename T, int BM, bool KEEP = false, bool SINGLE = false>
 __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile) {
   constexpr int MI = BM / 32;
   constexpr int NTHR = 64 * kFusedWaves;
@@ -951,18 +981,17 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   KS_MLP_STAMP(1)
   if constexpr (KEEP && BM == 128) if (a.keep_t_in && tid < a.in_t_width / 2)  // the first layer overwrites the tile only after its barrier
     (void)tile_transposed_out(act, lda, tid, a.keep_t_in, a.ldt, m0);
-  for (int l = 0; l + 1 < a.n_layers; ++l) {
-    fused_layer<ACT, T, MI, false, KEEP>(a, l, act, m0, lane, wave, tile);
-  }
-  fused_layer<ACT, T, MI, true, KEEP>(a, a.n_layers - 1, act, m0, lane, wave, tile);
+  if constexpr (!SINGLE)
+    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false, KEEP>(a, l, act, m0, lane, wave, tile);
+  fused_layer<ACT, T, MI, true, KEEP, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
 }
 
 // KEEP: the training forward that also stores every hidden layer's activations and the network input transposed
-// (FusedArgs::keep_t, keep_t_in; 128-row tiles only)
-template <int ACT, typename T, int BM, bool KEEP = false>
+// (FusedArgs::keep_t, keep_t_in; 128-row tiles only).  SINGLE: one bf16 layer
+template <int ACT, typename T, int BM, bool KEEP = false, bool SINGLE = false>
 __global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
 void mlp_fused_kernel(const FusedArgs a) {
-  mlp_fused_body<ACT, T, BM, KEEP>(a, blockIdx.x);
+  mlp_fused_body<ACT, T, BM, KEEP, SINGLE>(a, blockIdx.x);
 }
 
 // Two networks over the same rows in one launch (actor and critic of a control step): blockIdx.y picks the network, so
@@ -1785,6 +1814,8 @@ static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const fl
   {                                                                                                            \
     constexpr bool kKeep = BM == 128 && sizeof(T) == 2;                                                        \
     auto kfn = (keep && kKeep) ? mlp_fused_kernel<A, T, BM, kKeep> : mlp_fused_kernel<A, T, BM, false>;        \
+    if constexpr (sizeof(T) == 2 && BM != 64)                                                                  \
+      if (m.n_layers == 1) kfn = mlp_fused_kernel<KS_ACT_NONE, T, BM, false, true>;                            \
     if (lds > 64 * 1024 &&                                                                                     \
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
       return fail(KS_ELAUNCH, "ks_mlp_forward: cannot raise the LDS limit to %d bytes", lds);                  \
@@ -1819,14 +1850,15 @@ static int launch_fused(const DevMlp& m, hipStream_t s, int64_t M, const float* 
   }
 #endif
   if (M >= 128 * 256) return launch_fused_tile<__bf16, 128>(m, s, M, x, y, save);
-  if (M >= 64 * 256) return launch_fused_tile<__bf16, 64>(m, s, M, x, y, save);
+  // a single layer with a lane per feature: 64 rows of it need more than 128 registers (20000 x 128 -> 384: 16.4 us of 12.1), and narrow ones
+  // are better off with a lane per row (20000 x 128 -> 20: 4.7 us of 5.5)
+  if (M >= 64 * 256 && (m.n_layers > 1 || m.fn[0] <= 2)) return launch_fused_tile<__bf16, 64>(m, s, M, x, y, save);
   return launch_fused_tile<__bf16, 32>(m, s, M, x, y, save);
 }
 
 static int launch_fused_args(const FusedArgs& a, hipStream_t s) {
-  const int bm = a.M >= 128 * 256 ? 128 : a.M >= 64 * 256 ? 64 : 32, lds = bm * a.lda * 2;
-  auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128> : bm == 64 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 64>
-                                                                                : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32>;
+  const int bm = a.M >= 128 * 256 ? 128 : 32, lds = bm * a.lda * 2;
+  auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128, false, true> : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32, false, true>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
   hipLaunchKernelGGL(kfn, dim3((unsigned)((a.M + bm - 1) / bm)), dim3(64 * kFusedWaves), lds, s, a);

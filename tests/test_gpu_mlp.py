@@ -145,3 +145,26 @@ def test_single_fp32_layers_keep_the_range_of_fp32(M):
     assert np.array_equal(y[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
     # six products of 16 significant bits each are exact, the three left out are below 2^-23 together, and five sums round
     assert np.all(np.abs(y[finite] - want[finite]) <= 2.0 ** -21 * np.abs(want[finite]))
+
+
+@pytest.mark.parametrize("dims", [(128, 384), (340, 128), (97, 70), (128, 510), (33, 5)])
+def test_single_bf16_layers_of_every_batch_size(dims):
+    """32-, 64- and 128-row tiles of a single bf16 layer, with a lane per feature or (narrow layers) per row: the first and last row count
+    of each, ragged ends, the same bits for a row in all of them, nothing written past the output."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims))
+    w = (rng.normal(size=(dims[1], dims[0])) / np.sqrt(dims[0])).astype(np.float32)
+    b = rng.normal(scale=0.1, size=dims[1]).astype(np.float32)
+    net = MLP([w], [b], activation="none", dtype="bf16")
+    sizes = [1, 31, 33, 16383, 16384 + 37, 32767, 32768 + 45]
+    x = rng.normal(size=(max(sizes), dims[0])).astype(np.float32)
+    X = torch.from_numpy(x).to(DEV)
+    full = net(X)
+    want = reference(x, [w], [b], "none", True)
+    # products of bf16 values are exact in fp32: a rounding of 2^-24 per sum of up to 340 terms whose squares add up to about 1
+    assert np.abs(full.cpu().numpy() - want).max() <= 2e-5 * np.abs(want).max()
+    for M in sizes:
+        y = torch.full((M * dims[1] + 64,), 7.0, device=DEV)
+        got = net(X[:M].contiguous(), out=y[:M * dims[1]].view(M, dims[1]))
+        assert torch.equal(got, full[:M]) and torch.equal(y[M * dims[1]:], torch.full((64,), 7.0, device=DEV)), M
