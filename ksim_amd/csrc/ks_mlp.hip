@@ -1768,7 +1768,6 @@ extern "C" int ks_mlp_destroy(KsMlp* h) {
     for (float* q : t)
       if (q) (void)hipFree(q);
     if (h->m.Wt[l]) (void)hipFree(h->m.Wt[l]);
-    if (h->m.WtP[l]) (void)hipFree(h->m.WtP[l]);
   }
   if (h->m.zero_bias) (void)hipFree(h->m.zero_bias);
   if (h->m.sq_part) (void)hipFree(h->m.sq_part);
@@ -2053,7 +2052,6 @@ extern "C" int ks_mlp_train_init(KsMlp* h) {
       }
       if (m.Wt[l]) (void)hipFree(m.Wt[l]);
       m.Wt[l] = nullptr;
-      if (m.WtP[l]) (void)hipFree(m.WtP[l]);
       m.WtP[l] = nullptr;
     }
     if (m.zero_bias) (void)hipFree(m.zero_bias);
@@ -2082,12 +2080,12 @@ extern "C" int ks_mlp_train_init(KsMlp* h) {
       return give_up("upload");
     // the first layer's transpose is padded to whole output tiles of the input-gradient product; the padding stays zero
     const size_t nt = l == 0 ? (size_t)round_up(m.kpad[0], kBN) * m.npad[0] : n;
-    if (hipMalloc(&m.Wt[l], nt * esz) != hipSuccess || hipMemset(m.Wt[l], 0, nt * esz) != hipSuccess)
-      return give_up("allocation");
-    if (m.fused && esz == 2 && (l >= 1 || m.n_layers == 1)) {  // bf16: (fk / 2, rounded up) tiles of inputs x (2 fn) steps over outputs
-      const size_t np = (size_t)((m.fk[l] + 1) / 2) * (2 * m.fn[l]) * 512 * 2;
-      if (hipMalloc(&m.WtP[l], np) != hipSuccess || hipMemset(m.WtP[l], 0, np) != hipSuccess) return give_up("allocation");
-    }
+    size_t np = 0;
+    if (m.fused && esz == 2 && (l >= 1 || m.n_layers == 1))  // bf16: (fk / 2, rounded up) tiles of inputs x (2 fn) steps over outputs
+      np = (size_t)((m.fk[l] + 1) / 2) * (2 * m.fn[l]) * 512 * 2;
+    const size_t ntb = (nt * esz + 255) / 256 * 256;
+    if (hipMalloc(&m.Wt[l], ntb + np) != hipSuccess || hipMemset(m.Wt[l], 0, ntb + np) != hipSuccess) return give_up("allocation");
+    if (np) m.WtP[l] = (char*)m.Wt[l] + ntb;  // freed with Wt
   }
   const int wz = widest_pad(m);
   if (hipMalloc((void**)&m.zero_bias, (size_t)wz * 4) != hipSuccess || hipMemset(m.zero_bias, 0, (size_t)wz * 4) != hipSuccess)

@@ -221,6 +221,11 @@ def test_optimiser_step_refreshes_every_working_copy(dims, dtype):
     assert torch.equal(dx_a, dx_b)
 
 
+@pytest.mark.parametrize("dims,dtype", [((128, 384), "bf16"), ((41, 70), "bf16"), ((128, 512), "f32")])
+def test_optimiser_step_refreshes_the_copies_of_a_single_layer(dims, dtype):
+    test_optimiser_step_refreshes_every_working_copy(dims, dtype)
+
+
 def _setup(seed, Tn, N, od, A, hidden):
     from ksim_amd.mlp import MLP
     from ksim_amd.ppo_update import GaussianMlpPolicy
