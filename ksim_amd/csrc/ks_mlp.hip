@@ -98,9 +98,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
   // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
   // other, so that its rows are fetched once (102400 x 128 -> 512 in fp32 reads 64 MB instead of 210).  Row tiles past the last whole eight
   // follow in plain order.
+  // Slices of the reduction (weight gradients): all tiles of a slice, which read the same rows of both operands, go to one XCD.
   int64_t m_tile = blockIdx.x;
-  int n_tile = blockIdx.y;
-  if (gridDim.y > 1) {
+  int n_tile = blockIdx.y, z = blockIdx.z;
+  if (gridDim.z % 8 == 0) {
+    const unsigned l = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y, q = l >> 3, zq = q / tiles;
+    z = (int)(zq * 8 + (l & 7));
+    n_tile = (int)((q - zq * tiles) / gridDim.x);
+    m_tile = (q - zq * tiles) % gridDim.x;
+  } else if (gridDim.y > 1) {
     const int64_t l = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, whole = (int64_t)(gridDim.x & ~7u) * gridDim.y;
     const int64_t q = l < whole ? l >> 3 : l - whole;
     n_tile = (int)(q % gridDim.y);
@@ -141,7 +147,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
   // gridDim.z > 1: this workgroup reduces only its slice of K and writes partial sums to its own copy of the
   // output (LAST outputs only; the caller adds the copies up in a fixed order)
   const int kslice = K / (int)gridDim.z;
-  const int kbeg = (int)blockIdx.z * kslice, kend = kbeg + kslice;
+  const int kbeg = z * kslice, kend = kbeg + kslice;
   KS_FETCH(kbeg)
   for (int k0 = kbeg; k0 < kend; k0 += BK) {
 #pragma unroll
@@ -181,14 +187,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int col = n0 + wn * WN + j * 32 + (lane & 31);
-      const float b = blockIdx.z == 0 ? bias[col] : 0.f;
+      const float b = z == 0 ? bias[col] : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int64_t row = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         if (row >= M) continue;
         const float v = acc[i][j][r] + b;
         if (LAST) {
-          if (col < Nreal) ((float*)yout)[(int64_t)blockIdx.z * M * ldy + row * ldy + col] = v;
+          if (col < Nreal) ((float*)yout)[(int64_t)z * M * ldy + row * ldy + col] = v;
         } else {
           ((T*)yout)[row * ldy + col] = to_bf16(activate<ACT, true>(v));
         }
@@ -278,8 +284,15 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 31, h = lane >> 5;
   // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
   // other, so that its rows are fetched once.  Row tiles past the last whole eight follow in plain order.
+  // Slices of the reduction: all tiles of a slice go to one XCD.
   unsigned m_tile = blockIdx.x, n_tile = blockIdx.y;
-  if (gridDim.y > 1) {  // tiles of an output that fits the card's memory: 32 bits
+  int z = blockIdx.z;
+  if (gridDim.z % 8 == 0) {
+    const unsigned l = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y, q = l >> 3, zq = q / tiles;
+    z = (int)(zq * 8 + (l & 7));
+    n_tile = (q - zq * tiles) / gridDim.x;
+    m_tile = (q - zq * tiles) % gridDim.x;
+  } else if (gridDim.y > 1) {  // tiles of an output that fits the card's memory: 32 bits
     const unsigned l = blockIdx.y * gridDim.x + blockIdx.x, rows8 = gridDim.x & ~7u, whole = rows8 * gridDim.y;
     const unsigned q = l < whole ? l >> 3 : l - whole, d = q / gridDim.y;
     n_tile = q - d * gridDim.y;
@@ -291,13 +304,13 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
   f32x16 acc[MI][2], low[MI][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const float b = blockIdx.z == 0 ? bias[n0 + wn + 32 * j + c] : 0.f;  // padded to whole tiles
+    const float b = z == 0 ? bias[n0 + wn + 32 * j + c] : 0.f;  // padded to whole tiles
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) { acc[i][j][r] = b; low[i][j][r] = 0.f; }
   }
-  const int kslice = K / (int)gridDim.z, kbeg = (int)blockIdx.z * kslice, stages = kslice / 32;
+  const int kslice = K / (int)gridDim.z, kbeg = z * kslice, stages = kslice / 32;
   // rows past the batch repeat the last one, their results are dropped
   const int lrow = t >> 2, q = t & 3, lk = kbeg + 16 * (q >> 1) + 4 * (q & 1);
   const float* pa[AV];
@@ -375,7 +388,7 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
   // one row of the tile after the other: uniform steps from one address per lane
   const int64_t row0 = m0 + wm + 4 * h;
   const int col = n0 + wn + c;
-  float* out = y + ((int64_t)blockIdx.z * M + row0) * ldy + col;
+  float* out = y + ((int64_t)z * M + row0) * ldy + col;
   const bool on0 = col < Nreal, on1 = col + 32 < Nreal, whole = m0 + BM <= M;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
