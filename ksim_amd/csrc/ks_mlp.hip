@@ -146,9 +146,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
 
   // gridDim.z > 1: this workgroup reduces only its slice of K and writes partial sums to its own copy of the
   // output (LAST outputs only; the caller adds the copies up in a fixed order)
-  const int kslice = K / (int)gridDim.z;
-  const int kbeg = z * kslice, kend = kbeg + kslice;
-  KS_FETCH(kbeg)
+  const int kslice = (K / BK + (int)gridDim.z - 1) / (int)gridDim.z * BK;  // whole stages; the last slices may be shorter or empty
+  const int kbeg = min(K, z * kslice), kend = min(K, kbeg + kslice);
+  KS_FETCH(min(kbeg, K - BK))
   for (int k0 = kbeg; k0 < kend; k0 += BK) {
 #pragma unroll
     for (int c = 0; c < A_VECS; ++c) {
@@ -310,7 +310,8 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
 #pragma unroll
       for (int r = 0; r < 16; ++r) { acc[i][j][r] = b; low[i][j][r] = 0.f; }
   }
-  const int kslice = K / (int)gridDim.z, kbeg = z * kslice, stages = kslice / 32;
+  const int kslice = (K / 32 + (int)gridDim.z - 1) / (int)gridDim.z * 32;  // whole stages; the last slices may be shorter or empty
+  const int kbeg = min(K, z * kslice), stages = min(kslice, K - kbeg) / 32;
   // rows past the batch repeat the last one, their results are dropped
   const int lrow = t >> 2, q = t & 3, lk = kbeg + 16 * (q >> 1) + 4 * (q & 1);
   const float* pa[AV];
@@ -350,7 +351,7 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
 #pragma unroll
     for (int p = 0; p < 3; ++p) to[p * 4 * stride] = part[p];
   };
-  fetch(0);
+  if (stages > 0) fetch(0);
   for (int n = 0; n < stages; ++n) {
     if (n > 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS only: the requested rows stay in flight
 #pragma unroll
@@ -2126,7 +2127,14 @@ static void refresh_layers(DevMlp& m, hipStream_t s) {
   }
 }
 
-constexpr int kDwSplit = 32;  // most slices the weight-gradient reduction over the rows is cut into
+constexpr int kDwSplit = 32;  // slices the weight-gradient reduction over the rows is cut into
+// Behind the whole-network backward pass: more slices where 32 of them leave CUs without a tile, down to 512 rows each
+// (65536 x 512 x 128, 4 tiles: 42 us with 32 slices, 31.5 with 64; 128 add 9 us to the slices' sum for nothing).
+static int chain_dw_slices(int np, int kp128, int64_t Mp) {
+  int ks = kDwSplit;
+  while (ks < 64 && ks * (np / 128) * (kp128 / 128) < 512 && Mp >= 1024 * (int64_t)ks) ks *= 2;
+  return ks;
+}
 // Slices of the row reduction of a single layer's weight gradient (wgrad_kernel, 128 x 128 tiles): a workgroup per CU (its registers
 // admit no second one), a slice of at least three stages per group, below which the start and the slice sum cost as much as the
 // products; a multiple of eight, for the XCD mapping, once there are that many.
@@ -2200,7 +2208,7 @@ static int64_t carve_train(const DevMlp& m, int64_t M, char* base, TrainWs* ws) 
     }
     for (int l = 0; l < m.n_layers; ++l) w.dzT[l] = take((int64_t)m.npad[l] * w.Mp128 * esz);
     w.bpart[m.n_layers - 1] = (float*)take(tiles * m.npad[m.n_layers - 1] * 4);
-    for (int l = 0; l < m.n_layers; ++l) w.wpart[l] = (float*)take((int64_t)kDwSplit * m.npad[l] * m.kpad[l] * 4);
+    for (int l = 0; l < m.n_layers; ++l) w.wpart[l] = (float*)take((int64_t)chain_dw_slices(m.npad[l], round_up(m.kpad[l], kBN), w.Mp128) * m.npad[l] * m.kpad[l] * 4);
     w.yT[m.n_layers - 1] = take((int64_t)round_up(m.kpad[0], kBN) * w.Mp128 * esz);  // the network input, transposed
   }
   if (ws) *ws = w;
@@ -2315,16 +2323,9 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
     const int np = m.npad[l], kp = m.kpad[l], kp128 = round_up(kp, kBN);
     const T* dzT = (const T*)ws.dzT[l];
     const T* yT = l > 0 ? (const T*)ws.yT[l - 1] : xT;
-    const bool wide = np % 128 == 0;
-    int ksplit = wide ? kDwSplit : kDwSplit / 2;
-    while (ksplit > 1 && (Mp / 128) % ksplit != 0) ksplit >>= 1;  // K slices of 128 rows per pass
-    int rc;
-    if (wide)
-      rc = launch_layer_tile<T, false, true, 128, 128, 2, 2, 2>(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, yT, m.zero_bias,
-                                                                 (void*)ws.wpart[l], kp, ksplit);
-    else
-      rc = launch_layer_tile<T, false, true, 64, 128, 2, 2>(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, yT, m.zero_bias,
-                                                             (void*)ws.wpart[l], kp, ksplit);
+    const int ksplit = chain_dw_slices(np, kp128, Mp);
+    const int rc = launch_layer_tile<T, false, true, 128, 128, 2, 2, 2>(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, yT, m.zero_bias,
+                                                                        (void*)ws.wpart[l], kp, ksplit);
     if (rc != KS_OK) return rc;
     g.nz[l] = ksplit; g.nW[l] = (int64_t)np * kp; g.nb[l] = np;
     g.wpart[l] = ws.wpart[l]; g.bpart[l] = ws.bpart[l]; g.gW[l] = m.gW[l]; g.gb[l] = m.gb[l];
@@ -2483,7 +2484,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
     // wide layers over many rows: 128 x 128 output tiles halve the operand traffic per flop, twice the slices keep the grid
     const bool wide = Mp >= 32768 && np % 128 == 0;
     int ksplit = wide ? kDwSplit : kDwSplit / 2;
-    while (ksplit > 1 && (Mp / 64) % ksplit != 0) ksplit >>= 1;
+    while (ksplit > 1 && Mp / 64 < ksplit) ksplit >>= 1;
     if constexpr (sizeof(T) == 4)
       rc = launch_layer_f32(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, ws.t1, m.zero_bias,
                             ksplit > 1 ? (void*)ws.part : (void*)m.gW[l], kp, ksplit);

@@ -784,3 +784,27 @@ def test_cut_operands_of_the_weight_gradient_keep_the_range_of_fp32():
         net.backward(t32(xr), t32(dr))
         gw = net.parameters(gradients=True)[0][0].cpu().numpy()
         assert np.array_equal(gw, np.broadcast_to(x[r], (O, I)), equal_nan=True), r
+
+
+@pytest.mark.parametrize("dims,dtype,M0,extra", [
+    ((68, 256, 256, 20), "bf16", 32768, 133), ((68, 512, 512, 1), "bf16", 65536, 70), ((40, 128, 128, 21), "bf16", 32768, 1),  # whole-network pass
+    ((68, 256, 20), "bf16", 1024, 61), ((68, 256, 20), "f32", 1024, 61), ((68, 256, 20), "f32", 64, 1), ((68, 256, 20), "bf16", 40, 3),
+])
+def test_weight_gradients_over_row_counts_that_slices_do_not_divide(dims, dtype, M0, extra):
+    """Rows whose output gradient is zero add nothing: M0 rows, which the slices divide, and M0 + extra, which they do not."""
+    from ksim_amd.mlp import random_mlp
+
+    rng = np.random.default_rng(M0 + extra)
+    net, _, _ = random_mlp(dims, 5, dtype=dtype)
+    net.train_init()
+    x, dy = t32(rng.normal(size=(M0 + extra, dims[0]))), t32(rng.normal(size=(M0 + extra, dims[-1])))
+    dy[M0:] = 0
+    grads = []
+    for M in (M0, M0 + extra):
+        net.train_forward(x[:M].contiguous())
+        net.backward(x[:M].contiguous(), dy[:M].contiguous())
+        grads.append([g.clone() for pair in net.parameters(gradients=True) for g in pair])
+    for a, b in zip(*grads):
+        assert torch.isfinite(b).all()
+        # the same products in another order of sums of up to M0 terms: 2^-24 of a partial sum per addition, as a random walk
+        assert (a - b).abs().max() <= 8 * 2.0 ** -24 * np.sqrt(M0) * max(float(a.abs().max()), 1e-3), (a - b).abs().max()
