@@ -694,7 +694,8 @@ int ks_sample_action_mixture(ks_stream_t stream, int64_t N, int32_t nu, const fl
  * reference's linear layers.  KS_MLP_BF16 rounds weights and activations to bf16 and
  * accumulates in fp32 on the matrix cores; KS_MLP_F32 keeps fp32 throughout.
  * ks_mlp_create uploads (allocates); ks_mlp_forward allocates nothing: the caller
- * provides ks_mlp_workspace_bytes(mlp, M) bytes of device scratch.
+ * provides ks_mlp_workspace_bytes(mlp, M) bytes of device scratch, which also do for any smaller batch (as do those of
+ * the other *_workspace_bytes functions).
  */
 #define KS_MAX_LAYERS 8
 enum { KS_ACT_NONE = 0, KS_ACT_ELU = 1, KS_ACT_RELU = 2, KS_ACT_TANH = 3,

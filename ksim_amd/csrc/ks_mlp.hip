@@ -1909,12 +1909,13 @@ static int launch_fused_pair_tile(const DevMlp& m0, const DevMlp& m1, hipStream_
 // whole-network kernel gives its wavefronts two tiles of a layer (68-512-512-512-20: 83 -> 52 us at 256 rows, 61 at 2048; 256 wide it takes 30
 // to this one's 40).  Single layers: up to 1024 tiles, one per SIMD; past that the reuse in the per-layer kernel's larger tiles wins
 // (128 -> 512: 7.3 us at 2048 rows, 10.9 of 9.0 at 4096; 475 -> 128: 29.2 at 8192 rows, 49.2 of 25 at 16384).
+constexpr int64_t kSmallRows = 2048;
 static bool small_ok(const DevMlp& m, int64_t M) {
   if (m.dtype != KS_MLP_F32 || !m.Wp[0]) return false;
   if (m.n_layers == 1) return (M + 31) / 32 * m.fn[0] <= 1024;
   int wide = 0;
   for (int l = 0; l + 1 < m.n_layers; ++l) wide = m.fn[l] > wide ? m.fn[l] : wide;
-  return wide > kFusedWaves && M <= 2048;
+  return wide > kFusedWaves && M <= kSmallRows;
 }
 
 static int64_t small_ws_floats(const DevMlp& m, int64_t M) {  // two buffers of hidden activations
@@ -1992,9 +1993,12 @@ extern "C" int ks_mfma_yardstick(ks_stream_t stream, int32_t workgroups, int32_t
   return check_launch("ks_mfma_yardstick");
 }
 
+// Enough for M rows and for any smaller batch: a caller sizes one buffer for its largest batch.  Batches too large for the small-batch
+// kernel need nothing themselves, but the smaller ones do.
 extern "C" int64_t ks_mlp_workspace_bytes(const KsMlp* h, int64_t M) {
   if (!h || M < 0) return 0;
-  if (h->m.n_layers > 1 && small_ok(h->m, M)) return 2 * 4 * small_ws_floats(h->m, M);
+  const int64_t few = M < kSmallRows ? M : kSmallRows;
+  if (h->m.n_layers > 1 && small_ok(h->m, few)) return 2 * 4 * small_ws_floats(h->m, few);
   if (h->m.fused) return 0;
   int widest = 0;
   for (int l = 0; l + 1 < h->m.n_layers; ++l) widest = h->m.npad[l] > widest ? h->m.npad[l] : widest;

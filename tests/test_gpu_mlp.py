@@ -168,3 +168,26 @@ def test_single_bf16_layers_of_every_batch_size(dims):
         y = torch.full((M * dims[1] + 64,), 7.0, device=DEV)
         got = net(X[:M].contiguous(), out=y[:M * dims[1]].view(M, dims[1]))
         assert torch.equal(got, full[:M]) and torch.equal(y[M * dims[1]:], torch.full((64,), 7.0, device=DEV)), M
+
+
+@pytest.mark.parametrize("dims,dtype", [((68, 512, 512, 20), "f32"), ((30, 320, 5), "f32"), ((30, 256, 5), "f32"), ((68, 640, 20), "f32"),
+                                        ((128, 512), "f32"), ((68, 512, 512, 20), "bf16"), ((128, 384), "bf16"), ((68, 640, 20), "bf16")])
+def test_scratch_for_the_largest_batch_does_for_smaller_ones(dims, dtype):
+    """A caller sizes one buffer for its largest batch: none of the size queries may shrink as the row count grows, and a small batch given
+    that buffer writes nothing behind it."""
+    from ksim_amd import _lib
+    from ksim_amd.mlp import random_mlp
+
+    net, _, _ = random_mlp(dims, seed=sum(dims), dtype=dtype)
+    rows = sorted({0, 1, 31, 32, 33, 191, 192, 193, 256, 400, 2047, 2048, 2049, 4000, 8192, 16384, 32767, 32768, 32769, 65536, 100000, 131072})
+    lib, handle = _lib.load(), net._handle
+    for size in (lambda M: lib.ks_mlp_workspace_bytes(handle, M), lambda M: lib.ks_mlp_train_workspace_bytes(handle, M),
+                 lambda M: lib.ks_mlp_disc_workspace_bytes(handle, M, 2 * M)):
+        need = [int(size(M)) for M in rows]
+        assert need == sorted(need), list(zip(rows, need))
+    need, M = int(lib.ks_mlp_workspace_bytes(handle, 5000)), 256
+    buf = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=DEV)
+    x, y = torch.randn(M, dims[0], device=DEV), torch.empty(M, dims[-1], device=DEV)
+    _lib.check(lib.ks_mlp_forward(handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(y), _lib.ptr(buf)))
+    assert torch.equal(buf[need:], torch.full((4096,), 0x5A, dtype=torch.uint8, device=DEV))
+    assert torch.equal(y, net(x))
