@@ -2713,7 +2713,7 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
   __shared__ float cred[WAVES][64];
   __shared__ double sred[WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
-  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32;
+  const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;  // rows on x: y admits 65536 tiles only
   const int zbeg = blockIdx.z * g.kslice, zend = min(g.K, zbeg + g.kslice);
   const int per = ((zend - zbeg + WAVES - 1) / WAVES + 7) / 8 * 8;
   const int kbeg = zbeg + wave * per, kend = min(zend, kbeg + per);
@@ -2766,7 +2766,7 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + c] = acc[r];
   __syncthreads();
-  const bool sliced = gridDim.z > 1, want_cs = g.colsum && blockIdx.x == 0;
+  const bool sliced = gridDim.z > 1, want_cs = g.colsum && blockIdx.y == 0;
   const int tile = blockIdx.y * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y;
   float csum = 0.f;
   if (want_cs && threadIdx.x < 32)
@@ -3133,7 +3133,7 @@ static void sgemm_go(hipStream_t s, SgemmArgs g) {
   if (!g.A2) { g.A2 = g.A; g.a_split = 0x7fffffff; }
   if (!g.B2) { g.B2 = g.B; g.b_split = 0x7fffffff; }
   constexpr bool TN = !A_KC && !B_KC;
-  const dim3 tiles((unsigned)((g.N + 31) / 32), (unsigned)((g.M + 31) / 32));
+  const dim3 tiles((unsigned)((g.M + 31) / 32), (unsigned)((g.N + 31) / 32));
   int slices = 1;
   if (TN && g.part)
     while (slices < kDiscMaxSlices && g.K >= 1024 * slices && tiles.x * tiles.y * slices * 2 <= 512) slices *= 2;

@@ -170,3 +170,29 @@ def test_discriminator_gradient_at_the_edges_of_its_tiles(dims, shapes):
     for (gw, gb), w, b in zip(net.parameters(gradients=True), tw, tb):
         for got, want in ((gw, w.grad), (gb, b.grad)):
             assert np.abs(got.cpu().numpy() - want.numpy()).max() <= 2e-5 * max(np.abs(want.numpy()).max(), 1e-3)
+
+
+def test_discriminator_over_more_rows_than_a_grid_dimension_counts_tiles():
+    """Two million frames and more (65536 row tiles of 32) against the same gradient added up over parts of them.  Frames repeat every 4096 rows,
+    so the result is a known multiple of one period's: sums of R terms in fp32 slices, each rounding 2^-24 of a partial sum."""
+    from ksim_amd.mlp import random_mlp
+
+    period, repeats = 4096, 520  # 2 129 920 rows
+    real = torch.randn(1, period, 6, device=DEV)
+    grads = []
+    for n in (1, repeats):
+        net, _, _ = random_mlp((6, 8, 1), 3, dtype="f32")
+        net.train_init()
+        # penalty: the mean over motions, so that `n` motions of one period each carry the same share
+        losses = net.disc_loss_grad(real.expand(n, period, 6).contiguous(), torch.empty(0, 1, 6, device=DEV), 10.0)
+        grads.append((losses.double(), [g.double() for pair in net.parameters(gradients=True) for g in pair]))
+    (l1, g1), (ln, gn) = grads
+    assert torch.allclose(ln, torch.stack([l1[0] * repeats, l1[1], l1[2]]), rtol=1e-5)
+    # the squared-error gradient grows with the repeats, the penalty's does not: take the latter from a run of its own size
+    net, _, _ = random_mlp((6, 8, 1), 3, dtype="f32")
+    net.train_init()
+    net.disc_loss_grad(real, torch.empty(0, 1, 6, device=DEV), 0.0)
+    g0 = [g.double() for pair in net.parameters(gradients=True) for g in pair]
+    for a, b, c in zip(g0, g1, gn):
+        want = a * repeats + (b - a)
+        assert (c - want).abs().max() <= 1e-4 * want.abs().max()
