@@ -497,9 +497,10 @@ void gru_seq_forward_kernel(int T, int64_t M, int groups, const float* __restric
       quad_transpose(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3], j, pre);
       const float hu = f ? 0.f : hprev;
       const float hn = bn + (f ? 0.f : pre[2]);
-      const float r = seq_sigmoid(gin[0] + (f ? 0.f : pre[0]));
-      const float z = seq_sigmoid(gin[1] + (f ? 0.f : pre[1]));
-      const float n = seq_tanh(gin[2] + r * hn);
+      // the library's functions and IEEE division, as in gru_gate_kernel: seq_tanh cancels near zero (1.5e-7 absolute, three digits of 1e-4)
+      const float r = sigmoid_ks(gin[0] + (f ? 0.f : pre[0]));
+      const float z = sigmoid_ks(gin[1] + (f ? 0.f : pre[1]));
+      const float n = tanhf(gin[2] + r * hn);
       hprev = n + z * (hu - n);
       if constexpr (BF) reinterpret_cast<short*>(&sh[cur ^ 1][j][0])[unit] = bf16_bits(hprev);
       else sh[cur ^ 1][j][seq_slot(unit)] = hprev;

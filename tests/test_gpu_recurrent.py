@@ -354,3 +354,35 @@ def test_gru_sequence_kernels_agree_with_the_step_by_step_entry_points(dtype, Tn
     for got, want in ((d_gi, d_gi1), (d_gh, d_gh1)):
         assert (got - want).abs().max().item() <= tol * want.abs().max().item()
     assert not GRUCell(*_cell_params(rng, 24, 24), dtype=dtype).sequence_supported
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("H", [128, 24])
+def test_gru_gates_are_accurate_to_the_last_bits(dtype, H):
+    """The gates against float64, one input each: a candidate of size 1e-6 has the relative error of one of size 1, and so have the sigmoids far
+    out.  Library functions and IEEE division stay within 4 ulp (2^-22); 1 - 2 / (e^2x + 1) would lose three digits at 1e-4."""
+    from ksim_amd.recurrent import GRUCell
+
+    v = np.concatenate([np.logspace(-6, 1.3, 200), np.linspace(0.01, 85.0, 184)])
+    v = np.concatenate([v, -v])
+    if dtype == "bf16":
+        v = _bf16(v)
+    x = np.resize(v, (v.size, H)).astype(np.float32)
+    for shift in range(x.shape[0]):  # every unit of the cell meets every value
+        x[shift] = np.resize(np.roll(v, shift), H)
+    eye = np.eye(H)
+    zero = np.zeros((H, H))
+    M = x.shape[0]
+    fresh = torch.ones(M, dtype=torch.uint8, device=DEV)
+    xt, h0 = t32(x), torch.zeros(M, H, device=DEV)
+    for gate in range(3):
+        wi = np.concatenate([eye if g == gate else zero for g in range(3)])
+        cell = GRUCell(wi, np.zeros((3 * H, H)), dtype=dtype)
+        cell.train_init()
+        out, saved = torch.empty(M, H, device=DEV), torch.empty(M, 5 * H, device=DEV)
+        cell.train_forward(xt, h0, fresh, out, saved)
+        got = saved[:, gate * H:(gate + 1) * H].double().cpu().numpy()
+        x64 = x.astype(np.float64)
+        want = np.tanh(x64) if gate == 2 else 1 / (1 + np.exp(-x64))
+        err = np.abs(got - want) / np.abs(want)
+        assert err.max() <= 2.0 ** -22, (gate, err.max(), x.ravel()[err.argmax()])
