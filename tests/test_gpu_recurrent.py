@@ -137,6 +137,17 @@ def test_lstm_cell_and_network(N, I, H):
 
 @pytest.mark.parametrize("dtype,tol,act", [("f32", 2e-4, "elu"), ("bf16", 6e-2, "elu"), ("f32", 2e-4, "gelu")])
 def test_backward_through_time_matches_the_oracle(dtype, tol, act):
+    _check_backward_through_time(dtype, tol, act, 64, 96)
+
+
+@pytest.mark.parametrize("dtype,tol", [("f32", 2e-4), ("bf16", 6e-2)])
+@pytest.mark.parametrize("N", [77, 16])
+def test_backward_through_time_of_the_sequence_kernels_matches_the_oracle(dtype, tol, N):
+    """Hidden size 128: one launch per trajectory and direction (`ks_gru_sequence_*`), rows that do not fill the last set of four."""
+    _check_backward_through_time(dtype, tol, "elu", 128, N)
+
+
+def _check_backward_through_time(dtype, tol, act, H, N):
     """Gradients of a GRU actor over a trajectory (input projection, two GRU layers, ELU or GELU output network) with episode
     starts inside it, against torch float64 reverse-mode differentiation of the oracle network; then one optimiser step.
     Tolerances are relative to the largest entry of each gradient array: fp32 accumulation only for f32; for bf16 the
@@ -146,7 +157,7 @@ def test_backward_through_time_matches_the_oracle(dtype, tol, act):
     from ksim_amd.recurrent import GRUCell, RecurrentNetwork
 
     rng = np.random.default_rng(41)
-    Tn, N, I, H, O = 12, 96, 37, 64, 10
+    Tn, I, O = 12, 37, 10
     proj = (rng.normal(size=(H, I)) / np.sqrt(I), rng.normal(size=H) * 0.1)
     cells = [(rng.normal(size=(3 * H, H)) / np.sqrt(H), rng.normal(size=(3 * H, H)) / np.sqrt(H), rng.normal(size=3 * H) * 0.1,
               rng.normal(size=H) * 0.1) for _ in range(2)]
@@ -163,6 +174,7 @@ def test_backward_through_time_matches_the_oracle(dtype, tol, act):
 
     net = RecurrentNetwork(proj, [GRUCell(*c, dtype=dtype) for c in cells], MLP(ow, ob, activation=act, dtype=dtype), dtype=dtype)
     net.train_init()
+    assert all(c.sequence_supported == (H == 128) for c in net.cells)
     out = net.train_forward(t32(obs), t32(carry0), torch.tensor(fresh, dtype=torch.uint8, device=DEV))
     scale = np.abs(want_out).max()
     assert np.abs(out.cpu().numpy() - want_out).max() <= (1e-4 if dtype == "f32" else 3e-2) * scale
