@@ -692,7 +692,9 @@ int ks_sample_action_mixture(ks_stream_t stream, int64_t N, int32_t nu, const fl
  * heads) and the AMP discriminator forward (ksim/task/amp.py:327-358).
  * y = W_L act(... act(W_1 x + b_1) ...) + b_L, weights (out, in) row-major like the
  * reference's linear layers.  KS_MLP_BF16 rounds weights and activations to bf16 and
- * accumulates in fp32 on the matrix cores; KS_MLP_F32 keeps fp32 throughout.
+ * accumulates in fp32 on the matrix cores; KS_MLP_F32 keeps fp32 throughout.  Products of single fp32 layers, of fp32 layers
+ * wider than 512 and of the fp32 backward pass are formed from operands cut into three bf16 parts: exact to 2^-31 of each
+ * product, infinities and NaN as in the fp32 product; an operand below 2^-110 counts with an error of up to 2^-133.
  * ks_mlp_create uploads (allocates); ks_mlp_forward allocates nothing: the caller
  * provides ks_mlp_workspace_bytes(mlp, M) bytes of device scratch, which also do for any smaller batch (as do those of
  * the other *_workspace_bytes functions).

@@ -205,9 +205,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
 
 // ---------------------------------------------------------------- fp32 products on the bf16 matrix instruction
 // An fp32 value is cut into three bf16 values whose sum is the value itself: its upper 16 bits (8 bits of mantissa, so infinities and NaN
-// stay in the first part), the rest rounded to bf16, and what that leaves, which is at most 8 bits.  Of the nine products of two cut values
-// the six that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding per 16 k where the
-// fp32 instruction has eight, the other five, 2^-7 of it, in a second one.  Six instructions replace eight of twice their time.
+// stay in the first part), the rest, below 2^-7 of it, rounded to bf16, and what that leaves, below 2^-16 and at most 8 bits.  Of the nine
+// products of two cut values the eight that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding
+// per 16 k where the fp32 instruction has eight, the other seven, below 2^-6 of it, in a second one; the ninth is below 2^-32.  A reduction of
+// one term, or one term among zeros, then rounds once, as the fp32 product does (without the products of second and third parts, 2^-23 each at
+// most, it was 3.9 roundings off), and longer ones round less than on the fp32 instruction: relative error against 64 bits, in 2^-24,
+// 0.43 -> 0.43 for 1 term, 0.73 -> 0.46 for 5, 3.4 -> 1.1 for 128, 6.5 -> 2.0 for 475.  Eight instructions replace eight of twice their time.
+// Range: bf16 ends at 2^-133, so a value below 2^-110 loses what lies under 2^-134 of it: at most 2^-133 times the other operand.
 __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
@@ -240,9 +244,11 @@ __device__ __forceinline__ void mma_bf16(const bf16x8 (&a)[MI], const bf16x8 (&b
     for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
 }
 
-// The order of the six is part of a result's bits: every kernel that multiplies cut values goes through here, 16 k after 16 k.
+// The order of the eight is part of a result's bits: every kernel that multiplies cut values goes through here, 16 k after 16 k.
 template <int MI, int NJ>
 __device__ __forceinline__ void mma_cut(const bf16x8 (&a)[3][MI], const bf16x8 (&b)[3][NJ], f32x16 (&acc)[MI][NJ], f32x16 (&low)[MI][NJ]) {
+  mma_bf16(a[2], b[1], low);
+  mma_bf16(a[1], b[2], low);
   mma_bf16(a[2], b[0], low);
   mma_bf16(a[0], b[2], low);
   mma_bf16(a[1], b[1], low);
@@ -269,8 +275,9 @@ __device__ __forceinline__ void activate_tiles(f32x16 (&acc)[MI][2]) {
 // lanes read 128 bytes of a row in two loads.  A part's fragments lie [q][row] with two spare ones per q: neighbouring lanes write into
 // different banks and a matrix instruction's operand is one 16-byte read per lane.  The next stage's rows are requested before the
 // products and stay in flight over the barriers.  BM = 128: two workgroups per CU, one cutting while the other multiplies.
-//   102400 x 128 -> 512: 163 -> 109 us, 102400 x 512 -> 128: 139 -> 98 (137 TFLOP/s; on the fp32 instruction, whose time alone is 87 us), of
-//   40 in matrix instructions and 45 of memory traffic; relative error against 64 bits 2.0e-7 -> 0.7e-7 and 4.0e-7 -> 1.3e-7
+//   102400 x 128 -> 512: 163 us on the fp32 instruction, 127 here; 102400 x 512 -> 128: 139, 110 here (122 TFLOP/s; the fp32 instruction's
+//   time alone is 87 us), of 53 in matrix instructions and 45 of memory traffic; relative error against 64 bits 2.0e-7 -> 0.64e-7 and
+//   4.0e-7 -> 1.2e-7
 // Every fp32 kernel of a single layer starts from the bias and adds the products in one order (mma_cut), so a row's numbers do not depend
 // on the batch it comes in or the kernel that batch takes.
 // x (M, Kreal) with row stride ldx; K: Kreal padded to 32 (W's stride; its padding is zero).  Columns of y past Nreal are not written when y is
@@ -425,7 +432,7 @@ struct SmallLayer {
 };
 
 // A single fp32 layer over few rows: the same tiles, products of cut values (mma_cut) in cut_layer_kernel's order.  Bound by latency: 4096 x
-// 128 -> 40: 11.1 -> 6.3 us.
+// 128 -> 40: 11.1 -> 6.9 us.
 __global__ __launch_bounds__(256) void cut_small_kernel(int64_t M, SmallLayer p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
   const int j = (int)blockIdx.x * 4 + wave;
@@ -1636,8 +1643,8 @@ static int launch_layer_tile(int act, hipStream_t s, int64_t M, int npad, int K,
   return KS_OK;
 }
 
-// fp32 layers.  128-row tiles from one and a half per CU on: fewer leave CUs idle (25600 x 512 -> 128, 200 tiles: 34.6 us of 64-row tiles'
-// 30.8; 51200, 400 tiles: 49.0 of 58.8; 16384 x 128 -> 512, 512 tiles: 19.3 of 21.3).
+// fp32 layers.  128-row tiles from one and a half per CU on: fewer leave CUs idle (25600 x 512 -> 128, 200 tiles: 39.7 us of 64-row tiles'
+// 34.3; 51200, 400 tiles: 62.2 of 74.2; 16384 x 128 -> 512, 512 tiles: 22.5 of 24.4).
 static int launch_layer_f32(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x, int64_t ldx, const void* W,
                             const float* b, void* y, int64_t ldy, int ksplit = 1) {
   const bool small = (M + 127) / 128 * (npad / kBN) * ksplit < 400;
@@ -1908,7 +1915,8 @@ static int launch_fused_pair_tile(const DevMlp& m0, const DevMlp& m1, hipStream_
 // Whether M rows go through the small-batch kernel.  Networks of several layers: up to 2048 rows (one tile per SIMD at 512 wide) where the
 // whole-network kernel gives its wavefronts two tiles of a layer (68-512-512-512-20: 83 -> 52 us at 256 rows, 61 at 2048; 256 wide it takes 30
 // to this one's 40).  Single layers: up to 1024 tiles, one per SIMD; past that the reuse in the per-layer kernel's larger tiles wins
-// (128 -> 512: 7.3 us at 2048 rows, 10.9 of 9.0 at 4096; 475 -> 128: 29.2 at 8192 rows, 49.2 of 25 at 16384).
+// (128 -> 512: 8.1 us of 9.0 at 2048 rows, 12.4 of 10.1 at 4096; 475 -> 128: 31 of 27 at 8192 rows, 53 of 30 at 16384; 128 -> 40: 7.0 of 8.2
+// at 4096).
 constexpr int64_t kSmallRows = 2048;
 static bool small_ok(const DevMlp& m, int64_t M) {
   if (m.dtype != KS_MLP_F32 || !m.Wp[0]) return false;
@@ -2845,9 +2853,9 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
 // `colsum` also receives sum_k A(k, i), the bias gradient, from the fp32 values in the loaders' registers.
 // gridDim.y cuts the k range into slices of kslice; with more than one slice, slice z writes its partial product (M, N) densely to
 // C + z * M * N and its column sums to colsum + z * M, and sum_slices_kernel adds them up in a fixed order.
-// Bound by the matrix instructions (six per product of 16 rows, 48 us at the first size below) and the cuts beside them; the operands
+// Bound by the matrix instructions (eight per product of 16 rows, 64 us at the first size below) and the cuts beside them; the operands
 // take 44 us at the card's copy rate.  The predecessor multiplied on the fp32 instruction, whose time alone is 87 us there.
-//   102400 x 512 x 128, fp32: 122 -> 79 us (110 -> 170 TFLOP/s); relative error against 64 bits 7.3e-7 -> 1.9e-7
+//   102400 x 512 x 128, fp32: 122 -> 93 us (110 -> 145 TFLOP/s); relative error against 64 bits 7.3e-7 -> 1.9e-7
 //   12288 x 384 x 128, bf16: 44 us in five launches (cast, two transposes, product, column sums) -> 11.4
 // VA / VB: the operand's rows are 16-byte aligned and its width is a multiple of four.
 constexpr int kTnKB = 32;  // rows of a stage

@@ -143,8 +143,26 @@ def test_single_fp32_layers_keep_the_range_of_fp32(M):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
     finite = np.isfinite(want)
     assert np.array_equal(y[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
-    # six products of 16 significant bits each are exact, the three left out are below 2^-23 together, and five sums round
-    assert np.all(np.abs(y[finite] - want[finite]) <= 2.0 ** -21 * np.abs(want[finite]))
+    # eight products of 16 significant bits each are exact, the one left out is below 2^-32; the sum of the seven small ones, below 2^-6 of the
+    # result, rounds six times and the last sum once, as does the product it is compared with
+    assert np.all(np.abs(y[finite] - want[finite]) <= 2.0 ** -22.9 * np.abs(want[finite]))
+
+
+@pytest.mark.parametrize("M", [1, 33, 4000, 20000])
+def test_tiny_values_in_single_fp32_layers(M):
+    """Values whose second and third bf16 parts are denormal or below the smallest: each part rounds by at most 2^-134 (bf16 ends at 2^-133), so a
+    product is off by 2^-133 of the other operand, beside its own roundings."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    tiny = np.ldexp(rng.uniform(1, 2, 4096), rng.integers(-126, -98, 4096)).astype(np.float32) * rng.choice([-1.0, 1.0], 4096).astype(np.float32)
+    plain = rng.uniform(1, 2, 4096).astype(np.float32)
+    for xv, wv in ((tiny, plain), (plain, tiny)):
+        x, w = np.zeros((M, 20), np.float32), np.zeros((200, 20), np.float32)
+        x[:, 3], w[:, 3] = np.resize(xv, M), wv[:200]
+        y = MLP([w], [np.zeros(200, np.float32)], activation="none", dtype="f32")(torch.from_numpy(x).to(DEV)).cpu().numpy().astype(np.float64)
+        want = x[:, 3:4].astype(np.float64) * w[:, 3].astype(np.float64)[None, :]
+        assert np.all(np.abs(y - want) <= 2.0 * 2.0 ** -133 + 2.0 ** -23.9 * np.abs(want) + 2.0 ** -149)
 
 
 @pytest.mark.parametrize("dims", [(128, 384), (340, 128), (97, 70), (128, 510), (33, 5)])
@@ -191,3 +209,48 @@ def test_scratch_for_the_largest_batch_does_for_smaller_ones(dims, dtype):
     _lib.check(lib.ks_mlp_forward(handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(y), _lib.ptr(buf)))
     assert torch.equal(buf[need:], torch.full((4096,), 0x5A, dtype=torch.uint8, device=DEV))
     assert torch.equal(y, net(x))
+
+
+def _error_in_roundings(got, want):
+    """Largest and root mean square relative error in units of 2^-24, one rounding of fp32."""
+    e = np.abs(got.astype(np.float64) - want) / np.abs(want) * 2.0 ** 24
+    return e.max(), np.sqrt((e ** 2).mean())
+
+
+@pytest.mark.parametrize("M", [1, 33, 4000, 20000])
+def test_single_products_of_fp32_layers_round_once(M):
+    """Reductions of one term: forward (one input), input gradient (one output) and weight gradient (one row), and one term among zeros.  The
+    operands' parts are exact, eight of their nine products are added and the ninth is 2^-32, so what rounds is the final sum: 1 unit at most and
+    0.42 root mean square for uniformly spread results, plus seven roundings of the small products' sum, 2^-6 of it each."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    u = lambda *s: (rng.uniform(1, 2, s) * rng.choice([-1.0, 1.0], s)).astype(np.float32)  # noqa: E731
+    n = 130
+    x, w, b0 = u(M, 1), u(n, 1), np.zeros(n, np.float32)
+    cases = {}
+    cases["forward"] = (MLP([w], [b0], activation="none", dtype="f32")(torch.from_numpy(x).to(DEV)), x.astype(np.float64) * w[:, 0].astype(np.float64))
+    rows = np.zeros((M, 40), np.float32)
+    at = rng.integers(0, 40, M)
+    rows[np.arange(M), at] = x[:, 0]
+    wide = u(n, 40)
+    cases["one input of many"] = (MLP([wide], [b0], activation="none", dtype="f32")(torch.from_numpy(rows).to(DEV)),
+                                  x.astype(np.float64) * wide.T.astype(np.float64)[at])
+    critic = u(1, n)
+    net = MLP([critic], [np.zeros(1, np.float32)], activation="none", dtype="f32")
+    net.train_init()
+    inputs, dx = torch.from_numpy(u(M, n)).to(DEV), torch.empty(M, n, device=DEV)
+    net.train_forward(inputs)
+    net.backward_dx(inputs, torch.from_numpy(x).to(DEV), dx)
+    cases["input gradient"] = (dx, x.astype(np.float64) * critic.astype(np.float64))
+    net = MLP([u(70, n)], [np.zeros(70, np.float32)], activation="none", dtype="f32")
+    net.train_init()
+    row, dy = np.zeros((M, n), np.float32), np.zeros((M, 70), np.float32)
+    row[M // 2], dy[M // 2] = u(n), u(70)
+    rd, dyd = torch.from_numpy(row).to(DEV), torch.from_numpy(dy).to(DEV)
+    net.train_forward(rd)
+    net.backward(rd, dyd)
+    cases["weight gradient"] = (net.parameters(gradients=True)[0][0], np.outer(dy[M // 2].astype(np.float64), row[M // 2].astype(np.float64)))
+    for name, (got, want) in cases.items():
+        worst, rms = _error_in_roundings(got.cpu().numpy(), want)
+        assert worst <= 1.15 and (rms <= 0.45 or want.size < 1000), (name, worst, rms)
