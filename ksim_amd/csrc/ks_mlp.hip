@@ -923,12 +923,14 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
     // the finished tile, 16 bytes per thread and pass, rows as contiguous runs; the next layer only reads the tile until every
     // wavefront (this copy included, which sits before its matrix work in program order) has passed the next barrier
     constexpr int PC = 16 / (int)sizeof(T);  // entries of a 16-byte piece
-    const int w8 = nt * (32 / PC);
     T* dst = reinterpret_cast<T*>(a.save[l]);
-    const int ld = a.save_ld[l];
+    // rows are as wide as the backward pass's layers, which is more than the tile's (zeros) where the width is no multiple of 128
+    const int ld = a.save_ld[l], w8 = ld / PC, held = nt * (32 / PC);
     for (int idx = threadIdx.x; idx < MI * 32 * w8; idx += 64 * kFusedWaves) {
       const int r = idx / w8, c8 = idx - r * w8;
-      if (m0 + r < a.M) *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c8 * PC) = *reinterpret_cast<const uint4*>(act + r * lda + c8 * PC);
+      if (m0 + r < a.M)
+        *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c8 * PC) =
+            c8 < held ? *reinterpret_cast<const uint4*>(act + r * lda + c8 * PC) : uint4{0u, 0u, 0u, 0u};
     }
   }
 }
@@ -1724,8 +1726,11 @@ extern "C" int ks_mlp_create(const KsMlpDesc* d, KsMlp** out) {
     }
   }
   // fragment-ordered copy for the whole-network kernel and the small-batch kernel.  A single fp32 layer over many rows stays with the
-  // per-layer kernel (fused = 0): there is nothing to keep on chip between layers, and its output rows leave in longer runs.
-  bool fusable = true;
+  // per-layer kernel (fused = 0): there is nothing to keep on chip between layers, and its output rows leave in longer runs.  fp32 networks
+  // with GELU stay with it, too: the backward pass needs their pre-activations, which the whole-network kernel does not keep, and inference has to
+  // give the training forward's bits: the ratio of a policy update's first step is exactly one (68-256-256-20, 4096 rows: 39 us, 22 on the
+  // whole-network kernel).
+  bool fusable = d->dtype == KS_MLP_BF16 || d->n_layers == 1 || d->activation != KS_ACT_GELU;
   for (int l = 0; l <= d->n_layers && fusable; ++l)
     if (round_up(d->dims[l], 32) > kFusedMaxWidth) fusable = false;
   if (fusable) {
@@ -2245,9 +2250,10 @@ extern "C" int64_t ks_mlp_train_workspace_bytes(const KsMlp* h, int64_t M) {
 template <typename T>
 static int train_forward(DevMlp& m, hipStream_t s, int64_t M, const float* x, float* y, const TrainWs& ws) {
   // networks that fit the whole-network kernel run it, with every hidden layer's activations written out for the backward
-  // pass as well; the stored rows must have the width the backward pass expects (its padding is in units of 64, the kernel's 32)
+  // pass as well, in rows of the width that pass expects (its padding is in units of 128, the kernel's of 32)
   bool whole = m.fused && m.activation != KS_ACT_GELU;
-  for (int l = 0; whole && l + 1 < m.n_layers; ++l) whole = m.npad[l] == m.fn[l] * 32;
+  if (sizeof(T) == 2)  // bf16 networks of other widths take the per-layer kernel
+    for (int l = 0; whole && l + 1 < m.n_layers; ++l) whole = m.npad[l] == m.fn[l] * 32;
   m.chain_saved = 0;
   if (whole && chain_ok(m, M)) {  // activations in the formats of the whole-network backward pass, not row-major
     m.chain_saved = 1;

@@ -254,3 +254,39 @@ def test_single_products_of_fp32_layers_round_once(M):
     for name, (got, want) in cases.items():
         worst, rms = _error_in_roundings(got.cpu().numpy(), want)
         assert worst <= 1.15 and (rms <= 0.45 or want.size < 1000), (name, worst, rms)
+
+
+@pytest.mark.parametrize("dims,act", [((68, 200, 100, 20), "elu"), ((40, 64, 64, 1), "tanh"), ((30, 300, 5), "relu"), ((68, 512, 320, 20), "elu"),
+                                      ((68, 256, 256, 20), "gelu"), ((33, 500, 7), "gelu"), ((71, 256, 256, 21), "elu"), ((30, 640, 5), "elu"),
+                                      ((128, 384), "none"), ((20, 1), "none")])
+def test_fp32_training_and_inference_forward_are_bit_equal(dims, act):
+    """The first ratio of a policy update is exactly one: `train_forward` and the call give a row the same bits, whatever the hidden widths
+    (multiples of 32, of 128, neither), the activation and the batch; the padding the backward pass reads is zero, so its gradients are finite and
+    match float64."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims))
+    ws = [rng.normal(scale=1 / np.sqrt(i), size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])]
+    bs = [rng.normal(scale=0.1, size=o).astype(np.float32) for o in dims[1:]]
+    net = MLP(ws, bs, activation=act, dtype="f32")
+    net.train_init()
+    for M in (1, 45, 2048, 2049, 16384 + 37):
+        x = torch.from_numpy(rng.normal(size=(M, dims[0])).astype(np.float32)).to(DEV)
+        net._tws = torch.full((int(net._lib.ks_mlp_train_workspace_bytes(net._handle, M)),), 0xFF, dtype=torch.uint8, device=DEV)  # NaN
+        got = net.train_forward(x)
+        assert torch.equal(got, net(x)), M
+        other, y0, y1 = MLP(ws, bs, activation=act, dtype="f32"), torch.empty_like(got), torch.empty_like(got)
+        net.forward_pair(x, y0, other, x, y1)
+        assert torch.equal(y0, got) and torch.equal(y1, got), M
+        dy = torch.from_numpy(rng.normal(size=(M, dims[-1])).astype(np.float32)).to(DEV)
+        net.backward(x, dy)
+        tw = [torch.tensor(w, dtype=torch.float64, requires_grad=True) for w in ws]
+        h = x.double().cpu()
+        fn = {"elu": F.elu, "tanh": torch.tanh, "relu": F.relu, "none": lambda t: t, "gelu": lambda t: F.gelu(t, approximate="tanh")}[act]
+        for i, (w, b) in enumerate(zip(tw, bs)):
+            h = F.linear(h, w, torch.from_numpy(b).double())
+            h = fn(h) if i + 1 < len(tw) else h
+        h.backward(dy.double().cpu())
+        for (gw, _), w in zip(net.parameters(gradients=True), tw):
+            # fp32 sums of up to M rows of terms whose own error is a few 2^-24; ReLU's kink is met by no row here that a rounding moves
+            assert (gw.double().cpu() - w.grad).abs().max() <= 1e-4 * w.grad.abs().max()
