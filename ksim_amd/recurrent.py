@@ -18,6 +18,11 @@ from . import _lib_terms as T
 from .mlp import MLP
 
 
+# (step, env) rows that `RecurrentNetwork.forward_sequence` takes through the layers at a time: a layer keeps its input, its projected input and
+# its states of that many, 0.5 GB for an LSTM of hidden size 128, whatever the length of the rollout
+SEQUENCE_ROWS = 131072
+
+
 def _f32(a) -> np.ndarray:
     return np.ascontiguousarray(a.detach().cpu().numpy() if isinstance(a, torch.Tensor) else a, dtype=np.float32)
 
@@ -361,7 +366,8 @@ class RecurrentNetwork:
 
     def forward_sequence(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor) -> torch.Tensor:
         """The network over a trajectory without keeping anything for a backward pass: obs (T, M, in), carry0 the carry of the
-        first step (left as it is), fresh (T, M) uint8 -> (T, M, out).  The same numbers as T calls, one control step each."""
+        first step (left as it is), fresh (T, M) uint8 -> (T, M, out).  The same numbers as T calls, one control step each.  Long
+        trajectories go through in stretches of `SEQUENCE_ROWS` rows, whole steps, each from the carry the last one left."""
         T_, M, H = obs.shape[0], obs.shape[1], self.hidden_size
         want = (self.depth, 2, M, H) if self.lstm else (self.depth, M, H)
         if tuple(obs.shape) != (T_, M, self.in_dim) or tuple(carry0.shape) != want or tuple(fresh.shape) != (T_, M):
@@ -372,16 +378,23 @@ class RecurrentNetwork:
             for t in range(T_):
                 self(obs[t], carry, fresh=fresh[t], out=out[t])
             return out
-        x = self.input_proj(obs.contiguous().view(T_ * M, self.in_dim)).view(T_, M, H)
+        out = torch.empty(T_, M, self.out_dim, dtype=torch.float32, device=obs.device)
         fresh = fresh.contiguous()
-        for i, cell in enumerate(self.cells):
-            hs = torch.empty(T_, M, H, dtype=torch.float32, device=obs.device)
-            if self.lstm:
-                cell.sequence_forward(x, carry0[i, 0], carry0[i, 1], fresh, hs, None, None)
-            else:
-                cell.sequence_forward(x, carry0[i], fresh, hs, None)
-            x = hs
-        return self.output_proj(x.view(T_ * M, H)).view(T_, M, self.out_dim)
+        steps = max(1, SEQUENCE_ROWS // max(M, 1))
+        carry = [carry0[i].unbind(0) if self.lstm else (carry0[i],) for i in range(self.depth)]  # per layer (h, c) or (h,)
+        for t0 in range(0, T_, steps):
+            n = min(steps, T_ - t0)
+            x = self.input_proj(obs[t0:t0 + n].contiguous().view(n * M, self.in_dim)).view(n, M, H)
+            for i, cell in enumerate(self.cells):
+                states = [torch.empty(n, M, H, dtype=torch.float32, device=obs.device)]
+                if self.lstm:  # the cell state only where another stretch starts from it
+                    states.append(torch.empty_like(states[0]) if t0 + n < T_ else None)
+                cell.sequence_forward(x, *carry[i], fresh[t0:t0 + n], *states, None)
+                x = states[0]
+                if t0 + n < T_:
+                    carry[i] = tuple(s[-1].clone() for s in states)
+            self.output_proj(x.view(n * M, H), out=out[t0:t0 + n].view(n * M, self.out_dim))
+        return out
 
     # ------------------------------------------------------------------ training: backward pass through time
     def train_init(self) -> None:

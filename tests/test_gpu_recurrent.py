@@ -398,3 +398,42 @@ def test_gru_gates_are_accurate_to_the_last_bits(dtype, H):
         want = np.tanh(x64) if gate == 2 else 1 / (1 + np.exp(-x64))
         err = np.abs(got - want) / np.abs(want)
         assert err.max() <= 2.0 ** -22, (gate, err.max(), x.ravel()[err.argmax()])
+
+
+@pytest.mark.parametrize("kind", ["gru", "lstm"])
+def test_sequence_without_a_backward_pass_is_bounded_in_memory(kind, monkeypatch):
+    """A trajectory longer than what is kept at a time goes through in stretches of steps, from carry to carry: the same bits as in one piece and as
+    step by step, and scratch that does not grow with the number of steps."""
+    from ksim_amd import recurrent
+    from ksim_amd.mlp import random_mlp
+
+    rng = np.random.default_rng(61)
+    Tn, M, H, I = 37, 45, 128, 19
+    G, cls = (3, recurrent.GRUCell) if kind == "gru" else (4, recurrent.LSTMCell)
+    cells = [cls(rng.normal(size=(G * H, H)) / np.sqrt(H), rng.normal(size=(G * H, H)) / np.sqrt(H), rng.normal(size=G * H) * 0.1, dtype="f32")
+             for _ in range(2)]
+    out, _, _ = random_mlp((H, 7), 3, activation="none", dtype="f32")
+    net = recurrent.RecurrentNetwork((rng.normal(size=(H, I)) / np.sqrt(I), np.zeros(H)), cells, out, dtype="f32")
+    obs = t32(rng.normal(size=(Tn, M, I)))
+    carry = t32(rng.normal(size=net.initial_carry(M).shape) * 0.5)
+    kept = carry.clone()
+    fresh = torch.tensor(rng.random((Tn, M)) < 0.1, dtype=torch.uint8, device=DEV)
+    want, c = torch.empty(Tn, M, 7, device=DEV), carry.clone()
+    for t in range(Tn):
+        net(obs[t], c, fresh=fresh[t], out=want[t])
+    strided = torch.stack([obs, obs], 2)[:, :, 0]  # not contiguous
+    for rows in (10 ** 9, 5 * M, 5 * M - 1, M, 1):  # the last: less than a step, which is then a stretch of its own
+        monkeypatch.setattr(recurrent, "SEQUENCE_ROWS", rows)
+        for o in (obs, strided):
+            assert torch.equal(net.forward_sequence(o, carry, fresh), want)
+        assert torch.equal(carry, kept)
+    monkeypatch.undo()
+    Tn, M = 64, 16384
+    obs = torch.randn(Tn, M, I, device=DEV)
+    carry, fresh = net.initial_carry(M), torch.zeros(Tn, M, dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    net.forward_sequence(obs, carry, fresh)
+    # the output, and for each row of a stretch the input, projected input, hidden and cell state of a layer and the next layer's
+    assert torch.cuda.max_memory_allocated() - before <= Tn * M * 7 * 4 + recurrent.SEQUENCE_ROWS * (4 + G) * H * 4 + (1 << 24)
