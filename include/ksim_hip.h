@@ -860,6 +860,8 @@ int ks_mlp_get_params(const KsMlp* mlp, ks_stream_t stream, int32_t layer, float
  * `out`, its bias behind it at the next multiple of four floats; ks_mlp_param_floats(mlp, n_layers) is the whole length. */
 int64_t ks_mlp_param_floats(const KsMlp* mlp, int32_t layer);
 int ks_mlp_get_all_params(const KsMlp* mlp, ks_stream_t stream, float* out /*dev*/, int32_t gradients);
+/* The same in one launch into arrays of the caller's: weights[l] (out, in) and biases[l] (out), device pointers in host tables of n_layers. */
+int ks_mlp_copy_params(const KsMlp* mlp, ks_stream_t stream, float* const* weights, float* const* biases, int32_t gradients);
 
 /* Backward pass through time of a GRU stack (the jax.grad through the lax.scan over the trajectory in
  * PPOTask._single_step, ksim/task/ppo.py:572-694, for the recurrent actors and critics of examples/walking.py:40-208).

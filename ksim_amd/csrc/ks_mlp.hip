@@ -3294,23 +3294,22 @@ extern "C" int ks_mlp_get_params(const KsMlp* h, ks_stream_t stream, int32_t l, 
   return check_launch("ks_mlp_get_params");
 }
 
-// Every weight and bias of a network in one launch: the caller's layouts one after the other in `out`, entry 2 l / 2 l + 1 = weight /
-// bias of layer l, each starting at a multiple of four floats.
+// Every weight and bias of a network in one launch, entry 2 l / 2 l + 1 = weight / bias of layer l.
 struct UnpadArgs {
   int n;
   int first_block[2 * KS_MAX_LAYERS + 1];
   int rows[2 * KS_MAX_LAYERS], cols[2 * KS_MAX_LAYERS], ld[2 * KS_MAX_LAYERS];
   const float* src[2 * KS_MAX_LAYERS];
-  int64_t dst[2 * KS_MAX_LAYERS];
+  float* dst[2 * KS_MAX_LAYERS];
 };
-__global__ __launch_bounds__(256) void unpad_net_kernel(UnpadArgs a, float* __restrict__ out) {
+__global__ __launch_bounds__(256) void unpad_net_kernel(UnpadArgs a) {
   int e = 0;
   while (e + 1 < a.n && (int)blockIdx.x >= a.first_block[e + 1]) ++e;
   const int64_t total = (int64_t)a.rows[e] * a.cols[e];
   const int64_t idx = ((int64_t)blockIdx.x - a.first_block[e]) * 256 + threadIdx.x;
   if (idx >= total) return;
   const int r = (int)(idx / a.cols[e]), c = (int)(idx - (int64_t)r * a.cols[e]);
-  out[a.dst[e] + idx] = a.src[e][(int64_t)r * a.ld[e] + c];
+  a.dst[e][idx] = a.src[e][(int64_t)r * a.ld[e] + c];
 }
 
 extern "C" int64_t ks_mlp_param_floats(const KsMlp* h, int32_t layer) {
@@ -3321,23 +3320,36 @@ extern "C" int64_t ks_mlp_param_floats(const KsMlp* h, int32_t layer) {
   return off;
 }
 
-extern "C" int ks_mlp_get_all_params(const KsMlp* h, ks_stream_t stream, float* out, int32_t gradients) {
-  if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_get_all_params: call ks_mlp_train_init first");
-  if (!out) return fail(KS_EINVAL, "ks_mlp_get_all_params: null pointer");
+extern "C" int ks_mlp_copy_params(const KsMlp* h, ks_stream_t stream, float* const* weights, float* const* biases, int32_t gradients) {
+  if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_copy_params: call ks_mlp_train_init first");
+  if (!weights || !biases) return fail(KS_EINVAL, "ks_mlp_copy_params: null pointer");
   const DevMlp& m = h->m;
+  for (int l = 0; l < m.n_layers; ++l)
+    if (!weights[l] || !biases[l]) return fail(KS_EINVAL, "ks_mlp_copy_params: layer %d has no destination", l);
   UnpadArgs a;
   a.n = 2 * m.n_layers;
   int blocks = 0;
   for (int l = 0; l < m.n_layers; ++l) {
     const int o = m.dims[l + 1], i = m.dims[l];
-    const int64_t off = ks_mlp_param_floats(h, l);
     const int w = 2 * l, b = 2 * l + 1;
-    a.rows[w] = o; a.cols[w] = i; a.ld[w] = m.kpad[l]; a.src[w] = gradients ? m.gW[l] : m.mW[l]; a.dst[w] = off;
-    a.rows[b] = 1; a.cols[b] = o; a.ld[b] = o; a.src[b] = gradients ? m.gb[l] : m.mb[l]; a.dst[b] = off + ((int64_t)o * i + 3) / 4 * 4;
+    a.rows[w] = o; a.cols[w] = i; a.ld[w] = m.kpad[l]; a.src[w] = gradients ? m.gW[l] : m.mW[l]; a.dst[w] = weights[l];
+    a.rows[b] = 1; a.cols[b] = o; a.ld[b] = o; a.src[b] = gradients ? m.gb[l] : m.mb[l]; a.dst[b] = biases[l];
     a.first_block[w] = blocks; blocks += (int)(((int64_t)o * i + 255) / 256);
     a.first_block[b] = blocks; blocks += (o + 255) / 256;
   }
   a.first_block[a.n] = blocks;
-  hipLaunchKernelGGL(unpad_net_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a, out);
-  return check_launch("ks_mlp_get_all_params");
+  hipLaunchKernelGGL(unpad_net_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  return check_launch("ks_mlp_copy_params");
+}
+
+// packed one after the other, each starting at a multiple of four floats
+extern "C" int ks_mlp_get_all_params(const KsMlp* h, ks_stream_t stream, float* out, int32_t gradients) {
+  if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_get_all_params: call ks_mlp_train_init first");
+  if (!out) return fail(KS_EINVAL, "ks_mlp_get_all_params: null pointer");
+  float *weights[KS_MAX_LAYERS], *biases[KS_MAX_LAYERS];
+  for (int l = 0; l < h->m.n_layers; ++l) {
+    weights[l] = out + ks_mlp_param_floats(h, l);
+    biases[l] = weights[l] + ((int64_t)h->m.dims[l] * h->m.dims[l + 1] + 3) / 4 * 4;
+  }
+  return ks_mlp_copy_params(h, stream, weights, biases, gradients);
 }

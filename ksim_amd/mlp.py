@@ -48,7 +48,6 @@ class MLP:
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_mlp_create(ctypes.byref(d), ctypes.byref(self._handle)))
         self._ws: dict | None = None
-        self._param_sizes: list[int] | None = None
 
     @property
     def in_dim(self) -> int:
@@ -178,7 +177,7 @@ class MLP:
         """A view of a network that another object owns (the projections inside a GRU cell): never destroyed here."""
         self = cls.__new__(cls)
         self._lib, self._handle, self.dims, self.dtype, self.activation = lib, handle, list(dims), dtype, "none"
-        self._ws = self._param_sizes = None
+        self._ws = None
         self._borrowed = True
         return self
 
@@ -190,13 +189,13 @@ class MLP:
         _lib.check(self._lib.ks_mlp_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
 
     def parameters(self, gradients: bool = False) -> list[tuple[torch.Tensor, torch.Tensor]]:
-        """[(weight (out, in), bias (out))] copies of the fp32 master parameters, or of their gradients (views of one buffer)."""
-        if self._param_sizes is None:  # lengths in the packed buffer: weight, bias, weight ... each padded to four floats
-            self._param_sizes = [-(-n // 4) * 4 for i, o in zip(self.dims[:-1], self.dims[1:]) for n in (o * i, o)]
-        flat = torch.empty(sum(self._param_sizes), dtype=torch.float32, device="cuda")
-        _lib.check(self._lib.ks_mlp_get_all_params(self._handle, _lib.current_stream(), flat.data_ptr(), int(gradients)))
-        parts = flat.split(self._param_sizes)
-        return [(w[:o * i].view(o, i), b[:o]) for w, b, i, o in zip(parts[::2], parts[1::2], self.dims[:-1], self.dims[1:])]
+        """[(weight (out, in), bias (out))] copies of the fp32 master parameters, or of their gradients."""
+        out = [(torch.empty((o, i), dtype=torch.float32, device="cuda"), torch.empty((o,), dtype=torch.float32, device="cuda"))
+               for i, o in zip(self.dims[:-1], self.dims[1:])]
+        table = ctypes.c_void_p * len(out)
+        _lib.check(self._lib.ks_mlp_copy_params(self._handle, _lib.current_stream(), table(*(w.data_ptr() for w, _ in out)),
+                                                table(*(b.data_ptr() for _, b in out)), int(gradients)))
+        return out
 
     def close(self) -> None:
         if getattr(self, "_borrowed", False):

@@ -67,18 +67,18 @@ def compute_ppo_inputs(
     if succ is not None and succ.shape != values_bt.shape:
         raise _lib.KsError("successes must have the shape of values")
     stream, addr = _lib.current_stream(), _lib.addr
-    # one allocation for all outputs, handed out as its rows
-    gae, ret, tgt, *adv = torch.empty((4 if normalize_advantages else 3, *values_bt.shape), dtype=torch.float32, device=values_bt.device).unbind(0)
+    gae, ret, tgt = torch.empty_like(values_bt), torch.empty_like(values_bt), torch.empty_like(values_bt)
+    adv = gae
     if normalize_advantages:
-        ws = _workspace(values_bt.device)
+        adv, ws = torch.empty_like(values_bt), _workspace(values_bt.device)
         _lib.check(lib.ks_gae_normalized(stream, time_major, *values_bt.shape, addr(values_bt), addr(rewards_bt), addr(dones), addr(succ),
-                                         decay_gamma, gae_lambda, int(monte_carlo_returns), addr(gae), addr(ret), addr(tgt), addr(adv[0]),
+                                         decay_gamma, gae_lambda, int(monte_carlo_returns), addr(gae), addr(ret), addr(tgt), addr(adv),
                                          addr(ws)))
     else:
         fn = lib.ks_gae_tn if time_major else lib.ks_gae_bt
         _lib.check(fn(stream, *values_bt.shape, addr(values_bt), addr(rewards_bt), addr(dones), addr(succ), decay_gamma, gae_lambda,
                       int(monte_carlo_returns), addr(gae), addr(ret), addr(tgt)))
-    return PPOInputs(advantages_bt=adv[0] if adv else gae, value_targets_bt=tgt, gae_bt=gae, returns_bt=ret)
+    return PPOInputs(advantages_bt=adv, value_targets_bt=tgt, gae_bt=gae, returns_bt=ret)
 
 
 def compute_ppo_loss(
@@ -109,7 +109,7 @@ def compute_ppo_loss(
                       ppo_inputs.value_targets_bt, dtype=torch.float32)
     dev = on.values.device
     names = ("policy", "value", "kl") if off.entropy is None else ("policy", "value", "kl", "entropy")
-    out = dict(zip(names, torch.empty((len(names), B, T), dtype=torch.float32, device=dev).unbind(0)))
+    out = {k: torch.empty_like(on.values) for k in names}
     total = torch.empty((), dtype=torch.float32, device=dev)
     params = _lib.KsPpoLossParams(clip_param, value_loss_coef, entropy_coef, kl_coef, log_clip_value, kl_scale,
                                   int(use_clipped_value_loss))

@@ -167,7 +167,7 @@ class GRUCell:
         """Copies of weight_ih, weight_hh, bias (3H) and bias_n (H), or of their gradients."""
         (wi, bi), = self.proj_i.parameters(gradients)
         (wh, bh), = self.proj_h.parameters(gradients)
-        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:])
+        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:].clone())
 
     def __del__(self):
         h = getattr(self, "_handle", None)

@@ -167,3 +167,29 @@ def test_ppo_loss_rows(n, A, with_entropy):
     """Row lengths around what a wavefront stages (31 actions; longer rows and A = 1 take the direct kernel), a last tile of one
     element and of all 64."""
     test_ppo_loss_parity(n, 1, A, with_entropy)
+
+
+def test_outputs_are_tensors_of_their_own():
+    """Advantages, loss terms and parameter copies can be changed in place by numbers under differentiation, kept one at a time, and start on
+    16-byte boundaries for sizes that are no multiple of four."""
+    from ksim_amd import ppo
+    from ksim_amd.mlp import random_mlp
+    from ksim_amd.recurrent import GRUCell
+
+    values, rewards, dones, succ = (torch.as_tensor(a, device="cuda") for a in _inputs(3, 7, 9))
+    inputs = ppo.compute_ppo_inputs(values, rewards, dones, succ, 0.99, 0.95, normalize_advantages=True)
+    lp = torch.randn(7, 9, 3, device="cuda")
+    off = ppo.PPOVariables(lp, values, torch.rand(7, 9, 3, device="cuda"))
+    loss = ppo.compute_ppo_loss(inputs, ppo.PPOVariables(lp.clone(), values.clone()), off)
+    net, _, _ = random_mlp((5, 7, 3), 1, dtype="f32")
+    net.train_init()
+    rng = np.random.default_rng(0)
+    cell = GRUCell(rng.normal(size=(9, 4)), rng.normal(size=(9, 3)), dtype="f32")
+    cell.train_init()
+    outputs = [inputs.advantages_bt, inputs.value_targets_bt, inputs.gae_bt, inputs.returns_bt, *loss.values(),
+               *(t for pair in net.parameters() for t in pair), *cell.parameters().values()]
+    scale = torch.ones((), device="cuda", requires_grad=True)
+    for t in outputs:
+        assert t._base is None and t.is_contiguous() and t.data_ptr() % 16 == 0
+        assert t.untyped_storage().nbytes() == t.numel() * 4
+        t.mul_(scale)  # raises on one of several views
