@@ -34,12 +34,12 @@ def loop_slice(clip: torch.Tensor, start: int, window_t: int) -> torch.Tensor:
     return clip[idx]
 
 
-def _gather(motions: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
-    """`motions` rows picked by index vectors drawn on the host, which travel in one copy that nothing waits for (a copy from
-    pageable memory would hold the host until the GPU has caught up)."""
-    if motions.is_cuda:
-        rows = torch.empty(rows.shape, dtype=torch.int64, pin_memory=True).copy_(rows).to(motions.device, non_blocking=True)
-    return motions.index_select(0, rows)
+def _on_device(rows: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """Indices drawn on the host, where the motions are: in one copy that nothing waits for (a copy from pageable memory would hold the host until
+    the GPU has caught up)."""
+    if device.type == "cuda":
+        rows = torch.empty(rows.shape, dtype=torch.int64, pin_memory=True).copy_(rows).to(device, non_blocking=True)
+    return rows
 
 
 def make_real_batch(motions: torch.Tensor, window_t: int, batch_b: int, generator: torch.Generator) -> torch.Tensor:
@@ -50,8 +50,12 @@ def make_real_batch(motions: torch.Tensor, window_t: int, batch_b: int, generato
     starts = torch.randint(0, t_clip, (batch_b,), generator=generator)
     # every window of the batch in one gather: frame (start + t) mod T_clip of the drawn clip, as loop_slice takes them
     frames = (starts[:, None] + torch.arange(window_t)[None, :]) % t_clip
-    flat = motions.reshape(n * t_clip, *motions.shape[2:])
-    return _gather(flat, (clip_idx[:, None] * t_clip + frames).view(-1)).view(batch_b, window_t, *motions.shape[2:])
+    if motions.is_contiguous():
+        rows = _on_device((clip_idx[:, None] * t_clip + frames).view(-1), motions.device)
+        return motions.view(n * t_clip, *motions.shape[2:]).index_select(0, rows).view(batch_b, window_t, *motions.shape[2:])
+    # strided or expanded clips: indexed where they are (a flat view of them would be a copy of every clip)
+    both = _on_device(torch.stack([clip_idx[:, None].expand_as(frames), frames]), motions.device)
+    return motions[both[0], both[1]]
 
 
 def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> torch.Tensor:
@@ -59,7 +63,7 @@ def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Gen
     num_envs = sim_motions.shape[0]
     if num_envs % batch_b != 0:
         raise ValueError(f"amp_reference_batch_size ({batch_b}) must divide batch_size ({num_envs}).")
-    return _gather(sim_motions, torch.randperm(num_envs, generator=generator)[:batch_b])
+    return sim_motions.index_select(0, _on_device(torch.randperm(num_envs, generator=generator)[:batch_b], sim_motions.device))
 
 
 class DiscriminatorUpdate:

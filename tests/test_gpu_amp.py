@@ -196,3 +196,22 @@ def test_discriminator_over_more_rows_than_a_grid_dimension_counts_tiles():
     for a, b, c in zip(g0, g1, gn):
         want = a * repeats + (b - a)
         assert (c - want).abs().max() <= 1e-4 * want.abs().max()
+
+
+def test_reference_windows_of_strided_clips_are_gathered_in_place():
+    """Clips given as a slice of a larger array or expanded along an axis: the same windows, and no copy of the clips."""
+    from ksim_amd import amp
+
+    whole = torch.randn(6, 40, 3, 8, device=DEV)
+    views = [whole[:, ::2, 1], whole[1::2, 5:, 2, :5], whole[:1, :, 0].expand(64, 40, 8), whole[:, :1, 0].expand(6, 4000, 8), whole[:, :, 0, 2:3]]
+    for motions in views:
+        want = amp.make_real_batch(motions.contiguous(), 10, 6, torch.Generator().manual_seed(5))
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        got = amp.make_real_batch(motions, 10, 6, torch.Generator().manual_seed(5))
+        assert torch.equal(got, want)
+        if motions.numel() > 16384:
+            assert torch.cuda.max_memory_allocated() - before < motions.numel() * 4
+    big = torch.zeros(1, 1, 1, device=DEV).expand(100000, 100000, 64)  # 2.5 TB if it were copied
+    assert amp.make_real_batch(big, 4, 2, torch.Generator().manual_seed(1)).shape == (2, 4, 64)
