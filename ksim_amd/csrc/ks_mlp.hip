@@ -1167,9 +1167,9 @@ struct DevMlp {
   int dims[KS_MAX_LAYERS + 1];
   int kpad[KS_MAX_LAYERS];  // padded input width of layer l
   int npad[KS_MAX_LAYERS];  // padded output width of layer l
-  void* W[KS_MAX_LAYERS];
+  void* W[KS_MAX_LAYERS];   // one allocation per layer: W, b and, where there are any, Wp and bp
   float* b[KS_MAX_LAYERS];
-  // whole-network kernel (bf16, every padded width <= kFusedMaxWidth): weights re-ordered into MFMA fragments
+  // whole-network and small-batch kernels (every padded width <= kFusedMaxWidth): weights re-ordered into MFMA fragments
   int fused;                    // 1 when the tables below are valid
   int fk[KS_MAX_LAYERS];        // K steps of 16 per layer
   int fn[KS_MAX_LAYERS];        // 32-wide output tiles per layer
@@ -1701,68 +1701,56 @@ extern "C" int ks_mlp_create(const KsMlpDesc* d, KsMlp** out) {
   const int bk = d->dtype == KS_MLP_BF16 ? 64 : 32;
   const size_t esz = d->dtype == KS_MLP_BF16 ? 2 : 4;
   for (int l = 0; l <= d->n_layers; ++l) m.dims[l] = d->dims[l];
-  for (int l = 0; l < d->n_layers; ++l) {
-    if (!d->weights[l] || !d->biases[l]) { ks_mlp_destroy(h); return fail(KS_EINVAL, "ks_mlp_create: layer %d has no weights", l); }
-    h->host_w[l].assign(d->weights[l], d->weights[l] + (size_t)d->dims[l + 1] * d->dims[l]);
-    h->host_b[l].assign(d->biases[l], d->biases[l] + d->dims[l + 1]);
-    m.npad[l] = round_up(d->dims[l + 1], kBN);
-    // hidden activations are stored with the producer's padded width, so the consumer's K equals it
-    m.kpad[l] = l == 0 ? round_up(d->dims[0], bk) : m.npad[l - 1];
-    const size_t n = (size_t)m.npad[l] * m.kpad[l];
-    std::vector<unsigned char> w(n * esz, 0);
-    for (int o = 0; o < d->dims[l + 1]; ++o)
-      for (int i = 0; i < d->dims[l]; ++i) {
-        const float v = d->weights[l][(size_t)o * d->dims[l] + i];
-        if (esz == 2) ((uint16_t*)w.data())[(size_t)o * m.kpad[l] + i] = f32_to_bf16_rne(v);
-        else ((float*)w.data())[(size_t)o * m.kpad[l] + i] = v;
-      }
-    std::vector<float> b(m.npad[l], 0.f);
-    for (int o = 0; o < d->dims[l + 1]; ++o) b[o] = d->biases[l][o];
-    if (hipMalloc(&m.W[l], n * esz) != hipSuccess || hipMalloc((void**)&m.b[l], b.size() * 4) != hipSuccess ||
-        hipMemcpy(m.W[l], w.data(), n * esz, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(m.b[l], b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
-      ks_mlp_destroy(h);
-      return fail(KS_ELAUNCH, "ks_mlp_create: upload of layer %d failed", l);
-    }
-  }
-  // fragment-ordered copy for the whole-network kernel and the small-batch kernel.  A single fp32 layer over many rows stays with the
-  // per-layer kernel (fused = 0): there is nothing to keep on chip between layers, and its output rows leave in longer runs.  fp32 networks
-  // with GELU stay with it, too: the backward pass needs their pre-activations, which the whole-network kernel does not keep, and inference has to
-  // give the training forward's bits: the ratio of a policy update's first step is exactly one (68-256-256-20, 4096 rows: 39 us, 22 on the
-  // whole-network kernel).
+  // Beside the row-major copy of the weights a fragment-ordered one, for the whole-network kernel and the small-batch kernel.  A single fp32 layer
+  // over many rows stays with the per-layer kernel (fused = 0): there is nothing to keep on chip between layers, and its output rows leave in
+  // longer runs.  fp32 networks with GELU stay with it, too: the backward pass needs their pre-activations, which the whole-network kernel does not
+  // keep, and inference has to give the training forward's bits: the ratio of a policy update's first step is exactly one (68-256-256-20, 4096
+  // rows: 39 us, 22 on the whole-network kernel).
   bool fusable = d->dtype == KS_MLP_BF16 || d->n_layers == 1 || d->activation != KS_ACT_GELU;
   for (int l = 0; l <= d->n_layers && fusable; ++l)
     if (round_up(d->dims[l], 32) > kFusedMaxWidth) fusable = false;
-  if (fusable) {
-    const int G = 16 / (int)esz, sk = 2 * G;  // entries of a lane's fragment, k per step
-    int kmax = 0;
-    for (int l = 0; l < d->n_layers; ++l) {
-      m.fn[l] = round_up(d->dims[l + 1], 32) / 32;
-      m.fk[l] = (l == 0 ? round_up(d->dims[0], sk) : m.fn[l - 1] * 32) / sk;
+  const int G = 16 / (int)esz, sk = 2 * G;  // entries of a lane's fragment, k per step
+  int kmax = 0;
+  for (int l = 0; l < d->n_layers; ++l) {
+    if (!d->weights[l] || !d->biases[l]) { ks_mlp_destroy(h); return fail(KS_EINVAL, "ks_mlp_create: layer %d has no weights", l); }
+    const int out = d->dims[l + 1], in = d->dims[l];
+    h->host_w[l].assign(d->weights[l], d->weights[l] + (size_t)out * in);
+    h->host_b[l].assign(d->biases[l], d->biases[l] + out);
+    m.npad[l] = round_up(out, kBN);
+    // hidden activations are stored with the producer's padded width, so the consumer's K equals it
+    m.kpad[l] = l == 0 ? round_up(in, bk) : m.npad[l - 1];
+    if (fusable) {
+      m.fn[l] = round_up(out, 32) / 32;
+      m.fk[l] = (l == 0 ? round_up(in, sk) : m.fn[l - 1] * 32) / sk;
       kmax = m.fk[l] * sk > kmax ? m.fk[l] * sk : kmax;
       if (l + 1 < d->n_layers && m.fn[l] * 32 > kmax) kmax = m.fn[l] * 32;
-      const size_t n = (size_t)m.fn[l] * m.fk[l] * 64 * G;
-      std::vector<unsigned char> w(n * esz, 0);
-      for (int j = 0; j < m.fn[l]; ++j)
-        for (int st = 0; st < m.fk[l]; ++st)
-          for (int lane = 0; lane < 64; ++lane)
-            for (int e = 0; e < G; ++e) {
-              const int o = j * 32 + (lane & 31), i = st * sk + (lane >> 5) * G + e;
-              if (o >= d->dims[l + 1] || i >= d->dims[l]) continue;
-              const float v = d->weights[l][(size_t)o * d->dims[l] + i];
-              const size_t at = (((size_t)j * m.fk[l] + st) * 64 + lane) * G + e;
-              if (esz == 2) ((uint16_t*)w.data())[at] = f32_to_bf16_rne(v);
-              else ((float*)w.data())[at] = v;
-            }
-      std::vector<float> b(m.fn[l] * 32, 0.f);
-      for (int o = 0; o < d->dims[l + 1]; ++o) b[o] = d->biases[l][o];
-      if (hipMalloc(&m.Wp[l], n * esz) != hipSuccess || hipMalloc((void**)&m.bp[l], b.size() * 4) != hipSuccess ||
-          hipMemcpy(m.Wp[l], w.data(), n * esz, hipMemcpyHostToDevice) != hipSuccess ||
-          hipMemcpy(m.bp[l], b.data(), b.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
-        ks_mlp_destroy(h);
-        return fail(KS_ELAUNCH, "ks_mlp_create: upload of layer %d failed", l);
-      }
     }
+    // one allocation and one upload per layer: weights, biases and, where there are any, their fragment-ordered copies
+    const size_t nw = (size_t)m.npad[l] * m.kpad[l], np = (size_t)m.fn[l] * m.fk[l] * 64 * G;
+    auto up = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t at_b = up(nw * esz), at_wp = at_b + up((size_t)m.npad[l] * 4), at_bp = at_wp + up(np * esz);
+    std::vector<unsigned char> host(at_bp + (size_t)m.fn[l] * 32 * 4, 0);
+    for (int o = 0; o < out; ++o) {
+      unsigned char* row = host.data() + (size_t)o * m.kpad[l] * esz;
+      const float* src = d->weights[l] + (size_t)o * in;
+      if (esz == 4) std::memcpy(row, src, (size_t)in * 4);
+      else for (int i = 0; i < in; ++i) ((uint16_t*)row)[i] = f32_to_bf16_rne(src[i]);
+      if (!fusable) continue;
+      // inputs i .. i + G - 1 of output o: [tile o / 32][k step i / sk][lane (o % 32) + 32 ((i % sk) / G)]
+      unsigned char* to = host.data() + at_wp + ((size_t)(o >> 5) * m.fk[l] * 64 + (o & 31)) * 16;
+      for (int c = 0; c * G < in; ++c)
+        std::memcpy(to + ((size_t)(c >> 1) * 64 + 32 * (c & 1)) * 16, row + (size_t)c * 16, (size_t)(in - c * G < G ? in - c * G : G) * esz);
+    }
+    std::memcpy(host.data() + at_b, d->biases[l], (size_t)out * 4);
+    if (fusable) std::memcpy(host.data() + at_bp, d->biases[l], (size_t)out * 4);
+    if (hipMalloc(&m.W[l], host.size()) != hipSuccess || hipMemcpy(m.W[l], host.data(), host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      ks_mlp_destroy(h);
+      return fail(KS_ELAUNCH, "ks_mlp_create: upload of layer %d failed", l);
+    }
+    m.b[l] = (float*)((char*)m.W[l] + at_b);
+    if (fusable) { m.Wp[l] = (char*)m.W[l] + at_wp; m.bp[l] = (float*)((char*)m.W[l] + at_bp); }
+  }
+  if (fusable) {
     m.lda = kmax + 16 / (int)esz;  // +16 bytes per row: 16-byte aligned rows that start 4 banks apart
     m.fused = d->dtype == KS_MLP_BF16 || d->n_layers > 1;
   }
@@ -1787,10 +1775,7 @@ const float* mlp_peek_bias(const KsMlp* h, int l) { return h && h->m.train && l 
 extern "C" int ks_mlp_destroy(KsMlp* h) {
   if (!h) return KS_OK;
   for (int l = 0; l < KS_MAX_LAYERS; ++l) {
-    if (h->m.W[l]) (void)hipFree(h->m.W[l]);
-    if (h->m.b[l]) (void)hipFree(h->m.b[l]);
-    if (h->m.Wp[l]) (void)hipFree(h->m.Wp[l]);
-    if (h->m.bp[l]) (void)hipFree(h->m.bp[l]);
+    if (h->m.W[l]) (void)hipFree(h->m.W[l]);  // the biases and the fragment-ordered copies live behind it
     float* t[] = {h->m.mW[l], h->m.mb[l], h->m.gW[l], h->m.gb[l], h->m.m1W[l], h->m.m2W[l], h->m.m1b[l], h->m.m2b[l]};
     for (float* q : t)
       if (q) (void)hipFree(q);
