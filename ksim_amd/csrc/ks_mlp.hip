@@ -96,8 +96,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
-  // other, so that its rows are fetched once (102400 x 128 -> 512 in fp32 reads 64 MB instead of 210).  Row tiles past the last whole eight
-  // follow in plain order.
+  // other, so that its rows are fetched once.  Row tiles past the last whole eight follow in plain order.
   // Slices of the reduction (weight gradients) of 512 rows or more: all tiles of a slice, which read the same rows of both operands, go to one
   // XCD (65536 x 512 x 512: 70 -> 62 us).  Shorter ones are over before the rows come round again.
   int64_t m_tile = blockIdx.x;
@@ -291,7 +290,8 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
   __shared__ u32x4 As[3 * 4 * LA], Bs[3 * 4 * LB];  // [part][q][row]
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = lane & 31, h = lane >> 5;
   // Workgroup l of a launch runs on XCD l % 8, each with its own L2: the column tiles of one row tile go to one XCD, one after the
-  // other, so that its rows are fetched once.  Row tiles past the last whole eight follow in plain order.
+  // other, so that its rows are fetched once (102400 x 128 -> 512 reads 64 MB instead of 210).  Row tiles past the last whole eight follow in
+  // plain order.
   // Slices of the reduction, 512 rows or more: all tiles of a slice go to one XCD.
   unsigned m_tile = blockIdx.x, n_tile = blockIdx.y;
   int z = blockIdx.z;
@@ -411,12 +411,8 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
     }
 }
 
-// ---------------------------------------------------------------- matrix-core yardstick
-// Nothing but 32x32x16 bf16 MFMAs on register operands: eight independent accumulator tiles per wavefront (the fused
-// kernel's own count), no loads, no LDS, no epilogue.  What this loop reaches is the most any kernel built on that
-// instruction can reach on this part at the clock it sustains under matrix load.  Per workgroup: stamps[2 b] = shader
-// clock cycles of the loop, stamps[2 b + 1] = the same interval on the constant 100 MHz counter.
-// A layer of an fp32 network over few rows: the whole-network kernel would give 32 rows to one CU, whose matrix rate then takes 80 us
+// ---------------------------------------------------------------- fp32 layers over few rows
+// A layer of an fp32 network over few rows (sgemm_small_kernel): the whole-network kernel would give 32 rows to one CU, whose matrix rate then takes 80 us
 // for three layers of 512.  A wavefront owns a 32 x 32 tile of the layer with both operands straight from memory in registers (weights in
 // fragment order, eight groups of 8 k ahead) and the layers are launches of their own: rows x width / 1024 wavefronts over the chip.
 // SHARE wavefronts cut the reduction of a narrow output layer as the whole-network kernel's do (same parts, same order of the sum).
@@ -576,6 +572,11 @@ __global__ __launch_bounds__(256) void sgemm_small_kernel(int64_t M, SmallLayer 
   }
 }
 
+// ---------------------------------------------------------------- matrix-core yardstick
+// Nothing but 32x32x16 bf16 MFMAs on register operands: eight independent accumulator tiles per wavefront (the fused
+// kernel's own count), no loads, no LDS, no epilogue.  What this loop reaches is the most any kernel built on that
+// instruction can reach on this part at the clock it sustains under matrix load.  Per workgroup: stamps[2 b] = shader
+// clock cycles of the loop, stamps[2 b + 1] = the same interval on the constant 100 MHz counter.
 __global__ __launch_bounds__(256) void mfma_yardstick_kernel(int iters, float* __restrict__ out, long long* __restrict__ stamps) {
   f32x16 acc[8];
 #pragma unroll
@@ -608,8 +609,8 @@ __global__ __launch_bounds__(256) void mfma_yardstick_kernel(int iters, float* _
   }
 }
 
-// ---------------------------------------------------------------- whole network in one kernel (bf16)
-// A 512-thread workgroup keeps a BM-row tile of activations in LDS as bf16 for the whole network and walks the
+// ---------------------------------------------------------------- whole network in one kernel
+// A 512-thread workgroup keeps a BM-row tile of activations in LDS for the whole network (bf16, or fp32 in fp32 networks) and walks the
 // layers in place; only the network input and output touch HBM.  The product is computed transposed,
 // C^T = W * A^T: the weights are the MFMA "A" operand (32 output features x 16 k), the activations the "B"
 // operand (16 k x 32 batch rows), so that a lane's accumulators hold 4 consecutive features of one batch row
@@ -1170,10 +1171,10 @@ struct DevMlp {
   void* W[KS_MAX_LAYERS];   // one allocation per layer: W, b and, where there are any, Wp and bp
   float* b[KS_MAX_LAYERS];
   // whole-network and small-batch kernels (every padded width <= kFusedMaxWidth): weights re-ordered into MFMA fragments
-  int fused;                    // 1 when the tables below are valid
-  int fk[KS_MAX_LAYERS];        // K steps of 16 per layer
+  int fused;                    // 1: the whole-network kernel runs this network (the tables below also serve single fp32 layers over few rows)
+  int fk[KS_MAX_LAYERS];        // K steps per layer, of 16 (bf16) or 8 (fp32)
   int fn[KS_MAX_LAYERS];        // 32-wide output tiles per layer
-  int lda;                      // LDS row stride of the activation tile, in bf16 elements
+  int lda;                      // LDS row stride of the activation tile, in elements
   void* Wp[KS_MAX_LAYERS];      // [tile][k step][lane] x 16 bytes
   float* bp[KS_MAX_LAYERS];     // bias padded to 32 * fn
   // training state (ks_mlp_train_init): fp32 master weights in the padded (npad, kpad) layout, their gradients
@@ -1192,7 +1193,7 @@ struct DevMlp {
 
 
 // ---------------------------------------------------------------- training: the small kernels around the GEMMs
-// The three matrix products of a layer's backward pass reuse mlp_layer_kernel (Y = X W^T):
+// The three matrix products of a layer's backward pass reuse the layer kernels (mlp_layer_kernel, cut_layer_kernel: Y = X W^T):
 //   input gradient   dY_prev = dZ W        : X = dZ (M, npad),      "W" = W^T (kpad, npad)
 //   weight gradient  dW = dZ^T Y_prev      : X = dZ^T (npad, Mp),   "W" = Y_prev^T (kpad, Mp), fp32 output
 // so what is left are transposes, the activation derivative, column sums and the optimiser.
