@@ -203,7 +203,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64
 }
 
 // ---------------------------------------------------------------- fp32 products on the bf16 matrix instruction
-// An fp32 value is cut into three bf16 values whose sum is the value itself: its upper 16 bits (8 bits of mantissa, so infinities and NaN
+// An fp32 value is cut into three bf16 values (Henry, Tang and Heinecke, ARITH 2019) whose sum is the value itself: its upper 16 bits (8 bits of mantissa, so infinities and NaN
 // stay in the first part), the rest, below 2^-7 of it, rounded to bf16, and what that leaves, below 2^-16 and at most 8 bits.  Of the nine
 // products of two cut values the eight that reach 2^-24 of the result are added up: the largest in an accumulator of its own, with one rounding
 // per 16 k where the fp32 instruction has eight, the other seven, below 2^-6 of it, in a second one; the ninth is below 2^-32.  A reduction of
