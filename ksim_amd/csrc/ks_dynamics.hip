@@ -21,13 +21,17 @@
 #include "ks_step_args.h"
 
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 
 namespace ks {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-#define KS_SYNC() __syncthreads()
+// Hand-over through LDS between lanes of the workgroup's one wavefront.  The LDS pipeline serves a wavefront's accesses in the order
+// they were issued, so a read behind a write needs no wait: this only keeps the compiler from moving accesses across the line.
+// (__syncthreads() would drain the wavefront's LDS and memory traffic at two dozen places of a substep.)
+#define KS_SYNC() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
 #ifndef KS_STEP_WAVES
 #define KS_STEP_WAVES 4  // wavefronts per SIMD the register allocation aims at
 #endif
@@ -220,9 +224,11 @@ __device__ __forceinline__ float row_dot(const float* row, const float (&vv)[NP]
   return s0 + s1;
 }
 
-// Per-lane constants of one substep, as stored in DevModel::lane_rec (64 dwords, filled by ks_model_create):
+// Per-lane constants of one substep, as stored in DevModel::lane_rec (72 dwords, filled by ks_model_create):
 // lane L's body (L < nb), dof (L < nv), contact sphere (L < ns) and its share of the (i, ancestor j) dof pairs.
 // Lanes beyond a range carry the entries of index 0 (or -1 / zero where the kernel tests for that).
+constexpr int kPairSets = (kMaxPairs + 63) / 64;
+
 struct LaneRec {
   int b_parent, b_jtype, b_qadr, b_dofadr;
   int b_depth;
@@ -235,13 +241,20 @@ struct LaneRec {
   float s_rad, s_invw;
   float s_pos[3];
   unsigned s_mask;
-  int pk[kMaxPairs / 64 + 1];
+  int pk[kPairSets];
   // rows that live on the dof's own lane: hinge limit (range, inverse weight, address of the joint angle) and dry
   // friction (level and the constant stiffness 1 / R of its row)
   int d_limited, d_qadr;
   float d_rlo, d_rhi, d_invw, d_floss, d_frD;
+  // the body's ancestors from the tree root down to itself, 16 bits each: body | first dof << 5 | hinge << 10 | free joint << 11
+  unsigned b_chain[kMaxDepth / 2];
+  int pad2[3];
 };
-static_assert(sizeof(LaneRec) == 256, "LaneRec must fill the 64-dword record");
+static_assert(sizeof(LaneRec) == sizeof(DevModel::lane_rec) / 64, "LaneRec must fill the record");
+static_assert(kMaxB <= 32 && kMaxV <= 32 && kMaxDepth % 2 == 0, "a link of b_chain holds 5 + 5 bits");
+constexpr int kRecPieces = sizeof(LaneRec) / 16;
+// one field of a lane's record
+#define KS_REC(m, lane, field) (__builtin_bit_cast(decltype(LaneRec::field), (m).lane_rec[offsetof(LaneRec, field) / 16][lane][offsetof(LaneRec, field) / 4 % 4]))
 
 struct LsPoint {
   float alpha, cost, d0, d1;
@@ -315,16 +328,23 @@ __device__ __forceinline__ bool in_bracket(const LsPoint& x, const LsPoint& y) {
   return ((x.d0 < y.d0) && (y.d0 < 0.f)) || ((x.d0 > y.d0) && (y.d0 > 0.f));
 }
 
-// sum of one component over a contiguous subtree range of an array with `w` floats per body
+// sum of one component over a contiguous subtree range of an array with `w` floats per body; four reads in flight at a time
+// (the root's range is every body: read by read it is twenty LDS latencies in a row)
 __device__ __forceinline__ float range_sum(const float* base, int w, int b, int e) {
-  float s0 = 0.f, s1 = 0.f;
-  int c = b;
-  for (; c + 1 < e; c += 2) {
-    s0 += base[w * c];
-    s1 += base[w * (c + 1)];
+  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+  const float* p = base + w * b;
+  int left = e - b;
+  for (; left >= 4; left -= 4, p += 4 * w) {
+    const float x0 = p[0], x1 = p[w], x2 = p[2 * w], x3 = p[3 * w];
+    s0 += x0; s1 += x1; s2 += x2; s3 += x3;
   }
-  if (c < e) s0 += base[w * c];
-  return s0 + s1;
+  if (left > 0) {
+    const float x0 = p[0], x1 = p[left > 1 ? w : 0], x2 = p[left > 2 ? 2 * w : 0];
+    s0 += x0;
+    s1 += left > 1 ? x1 : 0.f;
+    s2 += left > 2 ? x2 : 0.f;
+  }
+  return (s0 + s1) + (s2 + s3);
 }
 
 // ------------------------------------------------------------------------------------------- the fused kernel
@@ -389,10 +409,9 @@ void step_kernel(StepArgs a) {
     const bool is_sph = lane < ns;
     LaneRec rec;
     {
-      const uint4* src = reinterpret_cast<const uint4*>(m.lane_rec[lane]);
       uint4* dst = reinterpret_cast<uint4*>(&rec);
 #pragma unroll
-      for (int k = 0; k < 16; ++k) dst[k] = src[k];
+      for (int k = 0; k < kRecPieces; ++k) dst[k] = *reinterpret_cast<const uint4*>(m.lane_rec[k][lane]);
     }
     const int b_parent = rec.b_parent, b_jtype = rec.b_jtype, b_qadr = rec.b_qadr, b_dofadr = rec.b_dofadr,
               b_depth = rec.b_depth;
@@ -409,8 +428,8 @@ void step_kernel(StepArgs a) {
     const float b_mass = is_body ? rec.b_mass * (a.mass_scale ? a.mass_scale[env * nb + bl] : 1.f) : 0.f;
     const int d_body = rec.d_body, d_act = rec.d_act, d_jtype = rec.d_jtype, d_k = rec.d_k;
     const float d_damping = rec.d_damping * ((a.damping_scale && is_dof) ? a.damping_scale[env * nv + lane] : 1.f);
-    const float d_armature = rec.d_armature, d_gear = rec.d_gear, d_lo = rec.d_lo, d_hi = rec.d_hi;
-    (void)d_armature;
+    const float d_armature = rec.d_armature * ((a.armature_scale && is_dof) ? a.armature_scale[env * nv + lane] : 1.f);
+    const float d_gear = rec.d_gear, d_lo = rec.d_lo, d_hi = rec.d_hi;
     const int s_body = rec.s_body;
     V3 s_pos = {rec.s_pos[0], rec.s_pos[1], rec.s_pos[2]};
     float s_rad = rec.s_rad;
@@ -420,9 +439,12 @@ void step_kernel(StepArgs a) {
       s_rad = a.sph_radius[env * ns + lane];
     }
     const unsigned s_mask = rec.s_mask;
-    int pk[kMaxPairs / 64 + 1];
+    unsigned chain[kMaxDepth / 2];
 #pragma unroll
-    for (int k = 0; k < kMaxPairs / 64 + 1; ++k) pk[k] = rec.pk[k];
+    for (int k = 0; k < kMaxDepth / 2; ++k) chain[k] = rec.b_chain[k];
+    int pk[kPairSets];
+#pragma unroll
+    for (int k = 0; k < kPairSets; ++k) pk[k] = rec.pk[k];
 
     // ---- actuators (ksim/engine.py:287-320, ksim/actuators.py:198-217)
     if (!fwd && (sub % a.actuator_period) == 0 && lane < nu) {
@@ -541,14 +563,25 @@ void step_kernel(StepArgs a) {
     {
       V3 pos = {0.f, 0.f, 0.f};
       Quat quat = {1.f, 0.f, 0.f, 0.f};
-      for (int k = 0; k < m.max_depth; ++k) {
+      // two links per step: both poses are on their way from LDS before the first is needed
+      unsigned ch[kMaxDepth / 2];
+#pragma unroll
+      for (int k = 0; k < kMaxDepth / 2; ++k) ch[k] = chain[k];
+      for (int k = 0; k < m.max_depth; k += 2) {
+        const float* p0 = lpose + 7 * (int)(ch[0] & 31u);
+        const float* p1 = lpose + 7 * (int)((ch[0] >> 16) & 31u);
+        const V3 t0 = ld3(p0), t1 = ld3(p1);
+        const Quat q0 = {p0[3], p0[4], p0[5], p0[6]}, q1 = {p1[3], p1[4], p1[5], p1[6]};
         if (k < b_depth) {
-          const int cb = m.body_chain[bl][k];
-          const V3 tl = ld3(lpose + 7 * cb);
-          const Quat ql = {lpose[7 * cb + 3], lpose[7 * cb + 4], lpose[7 * cb + 5], lpose[7 * cb + 6]};
-          pos = pos + mul(q2mat(quat), tl);
-          quat = qmul(quat, ql);
+          pos = pos + mul(q2mat(quat), t0);
+          quat = qmul(quat, q0);
         }
+        if (k + 1 < b_depth) {
+          pos = pos + mul(q2mat(quat), t1);
+          quat = qmul(quat, q1);
+        }
+#pragma unroll
+        for (int i = 0; i + 1 < kMaxDepth / 2; ++i) ch[i] = ch[i + 1];
       }
       if (is_body) {
         quat = qnormalize(quat);
@@ -629,19 +662,30 @@ void step_kernel(StepArgs a) {
       const int b = idx / 10, k = idx - 10 * b;
       l.crb[idx] = b > 0 ? range_sum(l.cinert + k, 10, b, l.sub_end[b]) : 0.f;
     }
-    for (int idx = lane; idx < nv * nvs; idx += 64) l.M[idx] = 0.f;
+    for (int idx = lane; idx < nv * nvs / 4; idx += 64) reinterpret_cast<float4*>(l.M)[idx] = {0.f, 0.f, 0.f, 0.f};  // nvs is a multiple of 4
     KS_SYNC();
-    if (is_dof) st6(l.buf + 6 * lane, inert_mul(l.crb + 10 * d_body, my_cdof));
+    if (is_dof) {
+      const Sp f = inert_mul(l.crb + 10 * d_body, my_cdof);
+      st6(l.buf + 6 * lane, f);
+      l.M[lane * nvs + lane] = dot(my_cdof, f) + d_armature;
+    }
     KS_SYNC();
 #pragma unroll
-    for (int k = 0; k < kMaxPairs / 64 + 1; ++k) {
-      if (pk[k] >= 0) {
-        const int i = pk[k] >> 8, j = pk[k] & 0xff;
-        float v = dot(ld6(l.cdof + 6 * j), ld6(l.buf + 6 * i));
-        if (i == j) v += m.dof_armature[i] * (a.armature_scale ? a.armature_scale[env * nv + i] : 1.f);
-        l.M[i * nvs + j] = v;
-        l.M[j * nvs + i] = v;
+    for (int k0 = 0; k0 < kPairSets; k0 += 4) {  // four sets of 64 pairs: all their reads before the first write
+      if (64 * k0 >= m.npairs) break;
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int p = max(pk[k0 + k], 0);
+        v[k] = dot(ld6(l.cdof + 6 * (p & 0xff)), ld6(l.buf + 6 * (p >> 8)));
       }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (pk[k0 + k] >= 0) {
+          const int i = pk[k0 + k] >> 8, j = pk[k0 + k] & 0xff;
+          l.M[i * nvs + j] = v[k];
+          l.M[j * nvs + i] = v[k];
+        }
     }
 
     KS_PHASE(3)
@@ -650,27 +694,36 @@ void step_kernel(StepArgs a) {
     {
       Sp v = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
       Sp acc = {{0.f, 0.f, 0.f}, {-m.gravity[0], -m.gravity[1], -m.gravity[2]}};
-      for (int k = 0; k < m.max_depth; ++k) {
-        if (k < b_depth) {
-          const int cb = m.body_chain[bl][k];
-          const int jt = m.body_jtype[cb], da = m.body_dofadr[cb];
-          if (jt == kJntFree) {
-            for (int c = 0; c < 3; ++c) v = v + ld6(l.cdof + 6 * (da + c)) * l.qvel[da + c];
-            Sp dv = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-            for (int c = 3; c < 6; ++c) {
-              const Sp cd = ld6(l.cdof + 6 * (da + c));
-              const float qd = l.qvel[da + c];
-              acc = acc + cross_motion(v, cd) * qd;
-              dv = dv + cd * qd;
-            }
-            v = v + dv;
-          } else if (jt == kJntHinge) {
-            const Sp cd = ld6(l.cdof + 6 * da);
-            const float qd = l.qvel[da];
+      auto hinge = [&](const Sp& cd, float qd) {
+        acc = acc + cross_motion(v, cd) * qd;
+        v = v + cd * qd;
+      };
+      auto link = [&](unsigned e, const Sp& cd0, float qd0) {  // cd0, qd0: axis and velocity of the link's first dof
+        if (e & (1u << 10)) {
+          hinge(cd0, qd0);
+        } else if (e & (1u << 11)) {
+          const int da = (int)((e >> 5) & 31u);
+          v = v + cd0 * qd0;
+          for (int c = 1; c < 3; ++c) v = v + ld6(l.cdof + 6 * (da + c)) * l.qvel[da + c];
+          Sp dv = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+          for (int c = 3; c < 6; ++c) {
+            const Sp cd = ld6(l.cdof + 6 * (da + c));
+            const float qd = l.qvel[da + c];
             acc = acc + cross_motion(v, cd) * qd;
-            v = v + cd * qd;
+            dv = dv + cd * qd;
           }
+          v = v + dv;
         }
+      };
+      for (int k = 0; k < m.max_depth; k += 2) {
+        const unsigned e0 = chain[0] & 0xffffu, e1 = chain[0] >> 16;
+        const int d0 = (int)((e0 >> 5) & 31u), d1 = (int)((e1 >> 5) & 31u);
+        const Sp c0 = ld6(l.cdof + 6 * d0), c1 = ld6(l.cdof + 6 * d1);
+        const float v0 = l.qvel[d0], v1 = l.qvel[d1];
+        if (k < b_depth) link(e0, c0, v0);
+        if (k + 1 < b_depth) link(e1, c1, v1);
+#pragma unroll
+        for (int i = 0; i + 1 < kMaxDepth / 2; ++i) chain[i] = chain[i + 1];
       }
       Sp cf = inert_mul(ci, acc) + cross_force(v, inert_mul(ci, v));
       // ---- force pushes (ksim/events.py:240-365): a wrench held on one body enters the Newton-Euler pass as an
@@ -820,21 +873,20 @@ void step_kernel(StepArgs a) {
     if (DR) {
       int lane_r = threadIdx.x;
       asm volatile("" : "+v"(lane_r));
-      const LaneRec* rr = reinterpret_cast<const LaneRec*>(m.lane_rec[lane_r]);
       if (is_dof) {
-        if (rr->d_limited) {
-          const float q = l.qpos[rr->d_qadr];
-          const float dlo = q - rr->d_rlo, dhi = rr->d_rhi - q;
+        if (KS_REC(m, lane_r, d_limited)) {
+          const float q = l.qpos[KS_REC(m, lane_r, d_qadr)];
+          const float dlo = q - KS_REC(m, lane_r, d_rlo), dhi = KS_REC(m, lane_r, d_rhi) - q;
           const float pos = fminf(dlo, dhi);
           if (pos < 0.f) {  // the nearer side, once violated
             dr.lim_s = dlo < dhi ? 1.f : -1.f;
             const float imp = impedance_dof(m, pos);
-            dr.lim_D = 1.f / fmaxf(rr->d_invw * (1.f - imp) / imp, 1e-15f);
+            dr.lim_D = 1.f / fmaxf(KS_REC(m, lane_r, d_invw) * (1.f - imp) / imp, 1e-15f);
             dr.lim_aref = -m.dr_b * dr.lim_s * my_qvel - m.dr_k * imp * pos;
           }
         }
-        dr.fr_fl = a.frictionloss ? ((rr->d_jtype == kJntHinge) ? a.frictionloss[env * nv + lane] : 0.f) : rr->d_floss;
-        dr.fr_D = rr->d_frD;
+        dr.fr_fl = a.frictionloss ? ((KS_REC(m, lane_r, d_jtype) == kJntHinge) ? a.frictionloss[env * nv + lane] : 0.f) : KS_REC(m, lane_r, d_floss);
+        dr.fr_D = KS_REC(m, lane_r, d_frD);
         dr.fr_rf = dr.fr_fl / dr.fr_D;
         dr.fr_aref = -m.dr_b * my_qvel;
       }
@@ -1166,9 +1218,8 @@ void step_kernel(StepArgs a) {
       // are not merged with those at the top of the substep): nothing of it stays live across the solver.
       int lane_e = threadIdx.x;
       asm volatile("" : "+v"(lane_e));
-      const LaneRec* rec_e = reinterpret_cast<const LaneRec*>(m.lane_rec[lane_e]);
-      const int b_jtype = rec_e->b_jtype, b_qadr = rec_e->b_qadr, b_dofadr = rec_e->b_dofadr;
-      const float d_damping = rec_e->d_damping * ((a.damping_scale && lane_e < nv) ? a.damping_scale[env * nv + lane_e] : 1.f);
+      const int b_jtype = KS_REC(m, lane_e, b_jtype), b_qadr = KS_REC(m, lane_e, b_qadr), b_dofadr = KS_REC(m, lane_e, b_dofadr);
+      const float d_damping = KS_REC(m, lane_e, d_damping) * ((a.damping_scale && lane_e < nv) ? a.damping_scale[env * nv + lane_e] : 1.f);
       const float my_qvel = lane_e < nv ? l.qvel[lane_e] : 0.f;
       float qacc_int = qacc;
       if (m.eulerdamp) {
@@ -1321,13 +1372,11 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     for (int k = 0; k < 4; ++k) { m.body_quat[b][k] = (float)d->body_quat[b][k]; m.body_iquat[b][k] = (float)d->body_iquat[b][k]; }
     m.body_mass[b] = (float)d->body_mass[b];
     m.body_invweight0[b] = (float)d->body_invweight0[b];
-    // chain from the root down to b
-    int chain[kMaxB], n = 0;
-    for (int c = b; c > 0; c = d->body_parent[c]) chain[n++] = c;
+    int n = 0;  // links from the root down to b
+    for (int c = b; c > 0; c = d->body_parent[c]) ++n;
     if (n > kMaxDepth) { delete km; return fail(KS_ELIMIT, "ks_model_create: tree deeper than %d", kMaxDepth); }
     m.body_depth[b] = n;
     if (n > m.max_depth) m.max_depth = n;
-    for (int k = 0; k < n; ++k) m.body_chain[b][k] = chain[n - 1 - k];
   }
   for (int q = 0; q < d->nq; ++q) m.qpos0[q] = (float)d->qpos0[q];
   for (int j = 0; j < d->nv; ++j) {
@@ -1367,7 +1416,7 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
   // dof masks and (i, ancestor j) pairs
   int np = 0;
   for (int i = 0; i < d->nv; ++i)
-    for (int j = i; j >= 0; j = d->dof_parent[j]) {
+    for (int j = d->dof_parent[i]; j >= 0; j = d->dof_parent[j]) {
       m.pair_i[np] = (short)i; m.pair_j[np] = (short)j; ++np;
     }
   m.npairs = np;
@@ -1386,6 +1435,11 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     const int bl = is_body ? L : 0;
     r.b_parent = m.body_parent[bl]; r.b_jtype = m.body_jtype[bl]; r.b_qadr = m.body_qadr[bl]; r.b_dofadr = m.body_dofadr[bl];
     r.b_depth = is_body ? m.body_depth[bl] : -1;
+    for (int c = bl, k = r.b_depth - 1; c > 0; c = d->body_parent[c], --k) {
+      const unsigned link = (unsigned)c | (unsigned)m.body_dofadr[c] << 5 | (m.body_jtype[c] == kJntHinge ? 1u << 10 : 0u) |
+                            (m.body_jtype[c] == kJntFree ? 1u << 11 : 0u);
+      r.b_chain[k / 2] |= link << (16 * (k & 1));
+    }
     r.b_q0 = (is_body && r.b_jtype == kJntHinge) ? m.qpos0[r.b_qadr] : 0.f;
     r.b_mass = m.body_mass[bl];
     for (int k = 0; k < 3; ++k) {
@@ -1418,11 +1472,11 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     r.s_body = m.sph_body[sl]; r.s_rad = m.sph_radius[sl]; r.s_invw = m.body_invweight0[r.s_body];
     for (int k = 0; k < 3; ++k) r.s_pos[k] = m.sph_pos[sl][k];
     r.s_mask = m.body_dofmask[r.s_body];
-    for (int k = 0; k < kMaxPairs / 64 + 1; ++k) {
+    for (int k = 0; k < kPairSets; ++k) {
       const int p = L + 64 * k;
       r.pk[k] = p < m.npairs ? ((int)m.pair_i[p] << 8) | (int)m.pair_j[p] : -1;
     }
-    std::memcpy(m.lane_rec[L], &r, sizeof(r));
+    for (int k = 0; k < kRecPieces; ++k) std::memcpy(m.lane_rec[k][L], (const char*)&r + 16 * k, 16);
   }
   if (hipGetDevice(&km->device) != hipSuccess) { delete km; return fail(KS_ELAUNCH, "ks_model_create: no HIP device"); }
   if (hipMalloc((void**)&km->dev, sizeof(DevModel)) != hipSuccess) { delete km; return fail(KS_ELAUNCH, "ks_model_create: hipMalloc failed"); }
