@@ -328,6 +328,95 @@ __device__ __forceinline__ bool in_bracket(const LsPoint& x, const LsPoint& y) {
   return ((x.d0 < y.d0) && (y.d0 < 0.f)) || ((x.d0 > y.d0) && (y.d0 > 0.f));
 }
 
+// ---------------------------------------------------------------- line search over contact rows (at most 32 of them)
+// Three step lengths are evaluated at once: the 16-lane groups 0, 1, 2 hold copies of the rows (rows 16..31 as a second set in
+// the same lanes) and take one step length each, so the sums of the constant, linear and quadratic coefficients are three
+// independent DPP reductions within the groups, and cost, slope and the Newton estimate of the next step length are formed
+// for all three points by the same instructions.  What comes out is read into scalar registers as bit patterns, and the
+// bracket is kept there: comparisons of slopes are integer comparisons of sign and magnitude on the scalar unit, which
+// neither occupies the vector issue port nor puts its latency behind vector compares.  The search is the longest part of the
+// wavefronts that a launch ends with (up to eight iterations of it per Newton step): evaluating the points one after the other
+// and bracketing on the vector unit, it was 34 % of their time.
+struct LsBits {  // a point of the search: step length, cost, slope, Newton estimate of the next step length
+  int alpha, cost, d0, next;
+};
+
+// the slope y lies strictly between the slope x and zero (x, y are no NaN)
+__device__ __forceinline__ bool closer(int x, int y) {
+  const unsigned mx = (unsigned)x & 0x7fffffffu, my = (unsigned)y & 0x7fffffffu;
+  return ((x ^ y) >= 0) & (mx > my) & (my != 0u);
+}
+
+__device__ __forceinline__ void take_if(LsBits& a, bool c, const LsBits& b) {  // field by field: the points stay in scalar registers
+  a.alpha = c ? b.alpha : a.alpha; a.cost = c ? b.cost : a.cost;
+  a.d0 = c ? b.d0 : a.d0; a.next = c ? b.next : a.next;
+}
+
+__device__ __forceinline__ float bits_f(int b) { return __builtin_bit_cast(float, b); }
+__device__ __forceinline__ int lane_bits(float x, int lane) { return __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane); }
+
+__device__ __forceinline__ float line_search_rows(int iterations, int nefc, int lane, float Jaref, float jv, float D, float g0, float g1,
+                                                  float g2, float gtol) {
+  const int grp = lane >> 4, r = lane & 15;
+  const bool two = nefc > 16;  // wave-uniform
+  const float j1 = __shfl(Jaref, r), v1 = __shfl(jv, r), D1 = __shfl(D, r);
+  const float a0 = 0.5f * j1 * j1 * D1, a1 = v1 * j1 * D1, a2 = 0.5f * v1 * v1 * D1;
+  float j2 = 0.f, v2 = 0.f, b0 = 0.f, b1 = 0.f, b2 = 0.f;
+  if (two) {
+    j2 = __shfl(Jaref, 16 + r); v2 = __shfl(jv, 16 + r);
+    const float D2 = __shfl(D, 16 + r);
+    b0 = 0.5f * j2 * j2 * D2; b1 = v2 * j2 * D2; b2 = 0.5f * v2 * v2 * D2;
+  }
+  auto eval = [&](float s0, float s1, float s2, LsBits& pa, LsBits& pb, LsBits& pc) {
+    const float al = grp == 0 ? s0 : (grp == 1 ? s1 : s2);
+    const bool on1 = j1 + al * v1 < 0.f;  // rows beyond nefc carry zeros
+    float x0 = on1 ? a0 : 0.f, x1 = on1 ? a1 : 0.f, x2 = on1 ? a2 : 0.f;
+    if (two) {
+      const bool on2 = j2 + al * v2 < 0.f;
+      x0 += on2 ? b0 : 0.f; x1 += on2 ? b1 : 0.f; x2 += on2 ? b2 : 0.f;
+    }
+    x0 += dpp_shift<0x111, 0xf>(x0); x1 += dpp_shift<0x111, 0xf>(x1); x2 += dpp_shift<0x111, 0xf>(x2);
+    x0 += dpp_shift<0x112, 0xf>(x0); x1 += dpp_shift<0x112, 0xf>(x1); x2 += dpp_shift<0x112, 0xf>(x2);
+    x0 += dpp_shift<0x114, 0xf>(x0); x1 += dpp_shift<0x114, 0xf>(x1); x2 += dpp_shift<0x114, 0xf>(x2);
+    x0 += dpp_shift<0x118, 0xf>(x0); x1 += dpp_shift<0x118, 0xf>(x1); x2 += dpp_shift<0x118, 0xf>(x2);
+    // lane 15 of each group holds the group's totals; the other lanes carry numbers nobody reads
+    const float q0 = g0 + x0, q1 = g1 + x1, q2 = g2 + x2;
+    const float cost = al * al * q2 + al * q1 + q0;
+    const float d0 = 2.f * al * q2 + q1, d1 = 2.f * q2 + (q2 == 0.f ? 1e-15f : 0.f);
+    // Newton estimate of the step length: d0 / d1 by reciprocal and product (1 ulp), a tenth of a division's instructions
+    const float next = al - d0 * __builtin_amdgcn_rcpf(d1);
+    const float slope = d0 == d0 ? d0 : 0.f;  // a NaN takes part in no bracket
+    pa = {lane_bits(al, 15), lane_bits(cost, 15), lane_bits(slope, 15), lane_bits(next, 15)};
+    pb = {lane_bits(al, 31), lane_bits(cost, 31), lane_bits(slope, 31), lane_bits(next, 31)};
+    pc = {lane_bits(al, 47), lane_bits(cost, 47), lane_bits(slope, 47), lane_bits(next, 47)};
+  };
+  LsBits p0, lo, hi, pa, pb, pm;
+  eval(0.f, 0.f, 0.f, p0, pb, pm);
+  eval(bits_f(p0.next), bits_f(p0.next), bits_f(p0.next), lo, pb, pm);
+  const bool below = bits_f(lo.d0) < bits_f(p0.d0);
+  hi = lo;
+  take_if(hi, below, p0);
+  take_if(lo, !below, p0);
+  const unsigned tol = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fmaxf(gtol, 0.f)));  // bits of a number >= 0 order like the number
+  bool swap = true;
+  for (int it = 0; it < iterations && swap; ++it) {
+    const unsigned ml = (unsigned)lo.d0 & 0x7fffffffu, mh = (unsigned)hi.d0;
+    if ((lo.d0 < 0) & (ml != 0u) & (ml < tol)) break;  // the slope at lo is negative and within the tolerance
+    if ((hi.d0 > 0) & (mh < tol)) break;               // that at hi positive and within it
+    eval(bits_f(lo.next), bits_f(hi.next), 0.5f * (bits_f(lo.alpha) + bits_f(hi.alpha)), pa, pb, pm);
+    const bool s1 = closer(lo.d0, pa.d0); take_if(lo, s1, pa);
+    const bool s2 = closer(lo.d0, pm.d0); take_if(lo, s2, pm);
+    const bool s3 = closer(lo.d0, pb.d0); take_if(lo, s3, pb);
+    const bool t1 = closer(hi.d0, pb.d0); take_if(hi, t1, pb);
+    const bool t2 = closer(hi.d0, pm.d0); take_if(hi, t2, pm);
+    const bool t3 = closer(hi.d0, pa.d0); take_if(hi, t3, pa);
+    swap = s1 | s2 | s3 | t1 | t2 | t3;
+  }
+  const float cl = bits_f(lo.cost), ch = bits_f(hi.cost), c0 = bits_f(p0.cost);
+  const bool improved = (cl < c0) || (ch < c0);
+  return improved ? (cl < ch ? bits_f(lo.alpha) : bits_f(hi.alpha)) : 0.f;
+}
+
 // sum of one component over a contiguous subtree range of an array with `w` floats per body; four reads in flight at a time
 // (the root's range is every body: read by read it is twenty LDS latencies in a row)
 __device__ __forceinline__ float range_sum(const float* base, int w, int b, int e) {
@@ -980,13 +1069,15 @@ void step_kernel(StepArgs a) {
           KS_SYNC();
           const int jc = (lane & 31) < nv ? (lane & 31) : 0, hh = lane >> 5;
           const int nblk = (nefc + 3) >> 2;
-          for (int b0 = 0; b0 < nblk; b0 += 2) {
-            const bool ok = b0 + hh < nblk;
-            const int bb = ok ? b0 + hh : 0;
-            const float4 f = *reinterpret_cast<const float4*>(l.vbuf + 4 * bb);
-            const float* Jb = l.J + (4 * bb) * js + jc;
-            const float sblk = (Jb[0] * f.x + Jb[js] * f.y) + (Jb[2 * js] * f.z + Jb[3 * js] * f.w);
-            qfc += ok ? sblk : 0.f;
+          for (int b0 = 0; b0 < nblk; b0 += 4) {  // two blocks per half, read together
+            const bool ok0 = b0 + hh < nblk, ok1 = b0 + 2 + hh < nblk;
+            const int k0 = ok0 ? b0 + hh : 0, k1 = ok1 ? b0 + 2 + hh : 0;
+            const float4 f0 = *reinterpret_cast<const float4*>(l.vbuf + 4 * k0), f1 = *reinterpret_cast<const float4*>(l.vbuf + 4 * k1);
+            const float *J0 = l.J + (4 * k0) * js + jc, *J1 = l.J + (4 * k1) * js + jc;
+            const float s0 = (J0[0] * f0.x + J0[js] * f0.y) + (J0[2 * js] * f0.z + J0[3 * js] * f0.w);
+            const float s1 = (J1[0] * f1.x + J1[js] * f1.y) + (J1[2 * js] * f1.z + J1[3 * js] * f1.w);
+            qfc += ok0 ? s0 : 0.f;
+            qfc += ok1 ? s1 : 0.f;
           }
           qfc += __shfl_xor(qfc, 32);
         } else {
@@ -1033,10 +1124,21 @@ void step_kernel(StepArgs a) {
           load_mtile(hc, l.M, nvs, nv, NP, lane);
           const int col = lane & 31, half = lane >> 5;
           const bool col_ok = NP == 32 || col < NP;
-          for (int r0 = 0; r0 < nefc; r0 += 2) {
-            const int r = r0 + half;
-            const float jv = (col_ok && r < nefc) ? l.J[r * js + col] : 0.f;
-            hc = __builtin_amdgcn_mfma_f32_32x32x2f32(l.drow[r] * jv, jv, hc, 0, 0, 0);
+          // the operands of four products at a time are fetched before the first of them (a row past the last counts as zero)
+          for (int r0 = 0; r0 < nefc; r0 += 8) {
+            float jr[4], dj[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int r = r0 + 2 * i + half;
+              const bool row_ok = r < nefc;
+              const int rc = row_ok ? r : 0;
+              const float x = l.J[rc * js + (col_ok ? col : 0)], d = l.drow[rc];
+              jr[i] = (col_ok && row_ok) ? x : 0.f;
+              dj[i] = d * jr[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (r0 + 2 * i < nefc) hc = __builtin_amdgcn_mfma_f32_32x32x2f32(dj[i], jr[i], hc, 0, 0, 0);
           }
           if (DR) {  // unit-vector rows add their stiffness to the diagonal
             const float hd = __shfl(dr_h, col);
@@ -1067,103 +1169,108 @@ void step_kernel(StepArgs a) {
         }
         const float smag = sqrtf(wave_sum(search * search)) * m.meaninertia * (float)(nv > 1 ? nv : 1);
         const float gtol = m.tolerance * m.ls_tolerance * smag;
-        const float q0r = 0.5f * Jaref * Jaref * D, q1r = jv * Jaref * D, q2r = 0.5f * jv * jv * D;
         const float g0 = gauss;
         const float g1 = wave_sum(is_dof ? search * (Ma - qfs) : 0.f);
         const float g2 = 0.5f * wave_sum(is_dof ? search * mv : 0.f);
-        // With at most 16 constraint rows the three sums of a cost evaluation share one reduction: the 16-lane
-        // groups 0, 1, 2 hold copies of the rows with the constant, linear and quadratic coefficient, and one
-        // DPP reduction within the groups yields all three totals.
-        // Rows 16..31 ride along as a second copy in the same lanes, so up to 32 rows need no more reduction steps.
-        const bool packed = nefc <= 32, two = nefc > 16;
-        float pk_j = 0.f, pk_jv = 0.f, pk_q = 0.f, pk_j2 = 0.f, pk_jv2 = 0.f, pk_q2 = 0.f;
-        const int grp = lane >> 4;
-        if (packed) {
-          const int r = lane & 15;
-          pk_j = __shfl(Jaref, r);
-          pk_jv = __shfl(jv, r);
-          const float c0 = __shfl(q0r, r), c1 = __shfl(q1r, r), c2 = __shfl(q2r, r);
-          pk_q = grp == 0 ? c0 : (grp == 1 ? c1 : (grp == 2 ? c2 : 0.f));
-          if (two) {
-            pk_j2 = __shfl(Jaref, 16 + r);
-            pk_jv2 = __shfl(jv, 16 + r);
-            const float e0 = __shfl(q0r, 16 + r), e1 = __shfl(q1r, 16 + r), e2 = __shfl(q2r, 16 + r);
-            pk_q2 = grp == 0 ? e0 : (grp == 1 ? e1 : (grp == 2 ? e2 : 0.f));
-          }
-        }
-        auto point = [&](float alpha) {
-          float q0, q1, q2;
+        float alpha;
+        if (nefc <= 32 && !(DR && ndr > 0)) {
+          alpha = line_search_rows(m.ls_iterations, nefc, lane, Jaref, jv, D, g0, g1, g2, gtol);
+        } else {
+          const float q0r = 0.5f * Jaref * Jaref * D, q1r = jv * Jaref * D, q2r = 0.5f * jv * jv * D;
+          // With at most 16 constraint rows the three sums of a cost evaluation share one reduction: the 16-lane
+          // groups 0, 1, 2 hold copies of the rows with the constant, linear and quadratic coefficient, and one
+          // DPP reduction within the groups yields all three totals.
+          // Rows 16..31 ride along as a second copy in the same lanes, so up to 32 rows need no more reduction steps.
+          const bool packed = DR && nefc <= 32, two = nefc > 16;
+          float pk_j = 0.f, pk_jv = 0.f, pk_q = 0.f, pk_j2 = 0.f, pk_jv2 = 0.f, pk_q2 = 0.f;
+          const int grp = lane >> 4;
           if (packed) {
-            float x = (pk_j + alpha * pk_jv < 0.f) ? pk_q : 0.f;  // rows beyond nefc carry zeros
-            if (two) x += (pk_j2 + alpha * pk_jv2 < 0.f) ? pk_q2 : 0.f;
-            if (DR && ndr > 0) {
-              // The rows on the dof lanes join the same reduction.  Lane j < 32 holds the three coefficients of its own rows:
-              // the constant one belongs in group 0, the linear one in group 1, so each lane keeps the one of its own group
-              // and swaps the other with the lane 16 away; the quadratic ones go to the upper lane half (groups 2 and 3).
+            const int r = lane & 15;
+            pk_j = __shfl(Jaref, r);
+            pk_jv = __shfl(jv, r);
+            const float c0 = __shfl(q0r, r), c1 = __shfl(q1r, r), c2 = __shfl(q2r, r);
+            pk_q = grp == 0 ? c0 : (grp == 1 ? c1 : (grp == 2 ? c2 : 0.f));
+            if (two) {
+              pk_j2 = __shfl(Jaref, 16 + r);
+              pk_jv2 = __shfl(jv, 16 + r);
+              const float e0 = __shfl(q0r, 16 + r), e1 = __shfl(q1r, 16 + r), e2 = __shfl(q2r, 16 + r);
+              pk_q2 = grp == 0 ? e0 : (grp == 1 ? e1 : (grp == 2 ? e2 : 0.f));
+            }
+          }
+          auto point = [&](float alpha) {
+            float q0, q1, q2;
+            if (packed) {
+              float x = (pk_j + alpha * pk_jv < 0.f) ? pk_q : 0.f;  // rows beyond nefc carry zeros
+              if (two) x += (pk_j2 + alpha * pk_jv2 < 0.f) ? pk_q2 : 0.f;
+              if (DR && ndr > 0) {
+                // The rows on the dof lanes join the same reduction.  Lane j < 32 holds the three coefficients of its own rows:
+                // the constant one belongs in group 0, the linear one in group 1, so each lane keeps the one of its own group
+                // and swaps the other with the lane 16 away; the quadratic ones go to the upper lane half (groups 2 and 3).
+                float t0, t1, t2;
+                dofrow_quad(dr, qacc, search, alpha, t0, t1, t2);
+                const float got = __shfl_xor(grp == 0 ? t1 : t0, 16);
+                const float up = __shfl(t2, lane & 31);
+                x += grp == 0 ? t0 + got : (grp == 1 ? t1 + got : up);
+              }
+              x += dpp_shift<0x111, 0xf>(x);
+              x += dpp_shift<0x112, 0xf>(x);
+              x += dpp_shift<0x114, 0xf>(x);
+              x += dpp_shift<0x118, 0xf>(x);  // lane 15 of each 16-lane group holds the group's total
+              q0 = g0 + lane_bcast(x, 15);
+              q1 = g1 + lane_bcast(x, 31);
+              q2 = g2 + lane_bcast(x, 47) + (DR ? lane_bcast(x, 63) : 0.f);
+            } else {
+              const bool on = is_row && (Jaref + alpha * jv < 0.f);
+              q0 = g0 + wave_sum(on ? q0r : 0.f);
+              q1 = g1 + wave_sum(on ? q1r : 0.f);
+              q2 = g2 + wave_sum(on ? q2r : 0.f);
+            }
+            if (DR && ndr > 0 && !packed) {
               float t0, t1, t2;
               dofrow_quad(dr, qacc, search, alpha, t0, t1, t2);
-              const float got = __shfl_xor(grp == 0 ? t1 : t0, 16);
-              const float up = __shfl(t2, lane & 31);
-              x += grp == 0 ? t0 + got : (grp == 1 ? t1 + got : up);
+              q0 += wave_sum(t0);
+              q1 += wave_sum(t1);
+              q2 += wave_sum(t2);
             }
-            x += dpp_shift<0x111, 0xf>(x);
-            x += dpp_shift<0x112, 0xf>(x);
-            x += dpp_shift<0x114, 0xf>(x);
-            x += dpp_shift<0x118, 0xf>(x);  // lane 15 of each 16-lane group holds the group's total
-            q0 = g0 + lane_bcast(x, 15);
-            q1 = g1 + lane_bcast(x, 31);
-            q2 = g2 + lane_bcast(x, 47) + (DR ? lane_bcast(x, 63) : 0.f);
-          } else {
-            const bool on = is_row && (Jaref + alpha * jv < 0.f);
-            q0 = g0 + wave_sum(on ? q0r : 0.f);
-            q1 = g1 + wave_sum(on ? q1r : 0.f);
-            q2 = g2 + wave_sum(on ? q2r : 0.f);
+            LsPoint p;
+            p.alpha = alpha;
+            p.cost = alpha * alpha * q2 + alpha * q1 + q0;
+            p.d0 = 2.f * alpha * q2 + q1;
+            p.d1 = 2.f * q2 + (q2 == 0.f ? 1e-15f : 0.f);
+            return p;
+          };
+          const LsPoint p0 = point(0.f);
+          // Newton estimates of the step length: d0 / d1 by reciprocal and product (1 ulp), a tenth of an IEEE division's instructions
+          auto newton_alpha = [](const LsPoint& x) { return x.alpha - x.d0 * __builtin_amdgcn_rcpf(x.d1); };
+          LsPoint lo = point(newton_alpha(p0));
+          LsPoint hi;
+          if (lo.d0 < p0.d0) { hi = p0; } else { hi = lo; lo = p0; }
+          bool swap = true;
+          int it = 0;
+          while (true) {
+            bool ls_done = it >= m.ls_iterations;
+            ls_done |= !swap;
+            ls_done |= (lo.d0 < 0.f) && (lo.d0 > -gtol);
+            ls_done |= (hi.d0 > 0.f) && (hi.d0 < gtol);
+            if (ls_done) break;
+            const LsPoint lo_next = point(newton_alpha(lo));
+            const LsPoint hi_next = point(newton_alpha(hi));
+            const LsPoint mid = point(0.5f * (lo.alpha + hi.alpha));
+            LsPoint nlo = lo, nhi = hi;
+            const bool s1 = in_bracket(nlo, lo_next); if (s1) nlo = lo_next;
+            const bool s2 = in_bracket(nlo, mid);     if (s2) nlo = mid;
+            const bool s3 = in_bracket(nlo, hi_next); if (s3) nlo = hi_next;
+            const bool t1 = in_bracket(nhi, hi_next); if (t1) nhi = hi_next;
+            const bool t2 = in_bracket(nhi, mid);     if (t2) nhi = mid;
+            const bool t3 = in_bracket(nhi, lo_next); if (t3) nhi = lo_next;
+            lo = nlo; hi = nhi;
+            swap = s1 | s2 | s3 | t1 | t2 | t3;
+            ++it;
           }
-          if (DR && ndr > 0 && !packed) {
-            float t0, t1, t2;
-            dofrow_quad(dr, qacc, search, alpha, t0, t1, t2);
-            q0 += wave_sum(t0);
-            q1 += wave_sum(t1);
-            q2 += wave_sum(t2);
-          }
-          LsPoint p;
-          p.alpha = alpha;
-          p.cost = alpha * alpha * q2 + alpha * q1 + q0;
-          p.d0 = 2.f * alpha * q2 + q1;
-          p.d1 = 2.f * q2 + (q2 == 0.f ? 1e-15f : 0.f);
-          return p;
-        };
-        const LsPoint p0 = point(0.f);
-        // Newton estimates of the step length: d0 / d1 by reciprocal and product (1 ulp), a tenth of an IEEE division's instructions
-        auto newton_alpha = [](const LsPoint& x) { return x.alpha - x.d0 * __builtin_amdgcn_rcpf(x.d1); };
-        LsPoint lo = point(newton_alpha(p0));
-        LsPoint hi;
-        if (lo.d0 < p0.d0) { hi = p0; } else { hi = lo; lo = p0; }
-        bool swap = true;
-        int it = 0;
-        while (true) {
-          bool ls_done = it >= m.ls_iterations;
-          ls_done |= !swap;
-          ls_done |= (lo.d0 < 0.f) && (lo.d0 > -gtol);
-          ls_done |= (hi.d0 > 0.f) && (hi.d0 < gtol);
-          if (ls_done) break;
-          const LsPoint lo_next = point(newton_alpha(lo));
-          const LsPoint hi_next = point(newton_alpha(hi));
-          const LsPoint mid = point(0.5f * (lo.alpha + hi.alpha));
-          LsPoint nlo = lo, nhi = hi;
-          const bool s1 = in_bracket(nlo, lo_next); if (s1) nlo = lo_next;
-          const bool s2 = in_bracket(nlo, mid);     if (s2) nlo = mid;
-          const bool s3 = in_bracket(nlo, hi_next); if (s3) nlo = hi_next;
-          const bool t1 = in_bracket(nhi, hi_next); if (t1) nhi = hi_next;
-          const bool t2 = in_bracket(nhi, mid);     if (t2) nhi = mid;
-          const bool t3 = in_bracket(nhi, lo_next); if (t3) nhi = lo_next;
-          lo = nlo; hi = nhi;
-          swap = s1 | s2 | s3 | t1 | t2 | t3;
-          ++it;
+          const bool improved = (lo.cost < p0.cost) || (hi.cost < p0.cost);
+          alpha = lo.cost < hi.cost ? lo.alpha : hi.alpha;
+          if (!improved) alpha = 0.f;
         }
-        const bool improved = (lo.cost < p0.cost) || (hi.cost < p0.cost);
-        float alpha = lo.cost < hi.cost ? lo.alpha : hi.alpha;
-        if (!improved) alpha = 0.f;
         qacc += alpha * search;
         Ma += alpha * mv;
         Jaref += alpha * jv;
