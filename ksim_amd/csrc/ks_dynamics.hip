@@ -41,26 +41,28 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 #else
 #define KS_TICK(k)
 #endif
-// A phase boundary of the step kernel.  The LDS layout is rebuilt from an offset the compiler cannot see through: the
-// two dozen array addresses are then a few scalar additions at the start of each phase instead of values that stay live
-// from the top of the kernel, where they do not fit the scalar registers and every use reads its address back out of a
-// vector register lane.
-#define KS_PHASE(k) { KS_TICK(k) int off_ = 0; asm volatile("" : "+s"(off_)); l = carve(lds_raw + off_, nb, nq, nv, nu, ns, nvs, js); }
+// A phase boundary of the step kernel.  The part of the LDS layout that depends on the model's sizes is rebuilt from an offset
+// the compiler cannot see through: its array addresses are then a few scalar additions at the start of each phase instead of
+// values that stay live from the top of the kernel, where they do not fit the scalar registers and every use reads its address
+// back out of a vector register lane.
+#define KS_PHASE(k) { KS_TICK(k) int off_ = 0; asm volatile("" : "+s"(off_)); l = carve<NP>(lds_raw, lds_raw + off_, nb, nq, nv, nu, ns); }
 // Register rows (mass matrix, Hessian, Jacobian) are padded from nv to a compile-time width NP, one kernel
 // instantiation per width: the padding rows are unit rows and the padding columns zero, so the factorisation,
 // the triangular solves and the row products run without any bound checks.
 __host__ __device__ inline int padded_nv(int nv) { return nv <= 8 ? 8 : nv <= 16 ? 16 : nv <= 24 ? 24 : nv <= 28 ? 28 : 32; }
-// Row stride of M and J in LDS: rows are 16-byte aligned (read with ds_read_b128, one row per lane) and the
-// stride in 16-byte units is odd, which spreads 16 consecutive rows over all 64 banks.
-__host__ __device__ inline int row_stride(int nv) { return (padded_nv(nv) / 4) % 2 ? padded_nv(nv) : padded_nv(nv) + 4; }
-__host__ __device__ inline int m_stride(int nv) { return row_stride(nv); }
-__host__ __device__ inline int j_stride(int nv) { return row_stride(nv); }
+// Row stride of M and J in LDS, a constant of the instantiation: rows are 16-byte aligned (read with ds_read_b128, one row per
+// lane) and the stride in 16-byte units is odd, which spreads 16 consecutive rows over all 64 banks.
+__host__ __device__ constexpr int stride_of(int np) { return (np / 4) % 2 ? np : np + 4; }
 
 struct Lds {
-  float *qpos, *qvel, *warm, *tau;
-  float *xpos, *xquat, *xanchor, *xaxis;
+  // at the same place for every model of an instantiation
+  float *vbuf, *qvel, *warm, *drow, *M;
+  // behind them, sized by the model
+  float *qpos, *tau;
+  float *xpos, *xquat;
   float *cinert, *crb, *cdof, *buf, *cvel, *cfrc, *fsub;
-  float *M, *J, *vbuf, *drow;
+  float *xanchor, *xaxis;  // joint anchors and axes: dead once the motion axes are built, so they share buf and fsub
+  float* J;
   float *con_off, *con_D, *con_kip;
   int *con_body, *sub_end;
   unsigned* con_mask;
@@ -69,39 +71,43 @@ struct Lds {
 __host__ __device__ inline int up4(int n) { return (n + 3) & ~3; }
 
 __host__ __device__ inline int lds_floats(int nb, int nq, int nv, int nu, int ns) {
-  const int nvs = m_stride(nv), js = j_stride(nv);
+  const int np = padded_nv(nv), js = stride_of(np);
   int n = 0;
-  n += up4(nq) + 32 + up4(nv) + up4(nu);                             // qpos qvel(32) warm tau
-  n += up4(nb * 3) + up4(nb * 4) + 2 * up4(nb * 3);                    // xpos xquat xanchor xaxis
+  n += 32 + 32 + 32 + 64 + np * js;                                  // vbuf qvel warm drow M
+  n += up4(nq) + up4(nu);                                            // qpos tau
+  n += up4(nb * 3) + up4(nb * 4);                                    // xpos xquat
   n += up4(nv * 6) + up4(nb * 6);                                    // cdof cvel
   const int scratch = 2 * up4(nb * 10) + up4(nv * 6) + 2 * up4(nb * 6);  // cinert crb buf fsub cfrc
   const int jsz = up4(4 * ns * js + 32);                             // J overlays that scratch once it is dead
   n += scratch > jsz ? scratch : jsz;
-  n += up4(nv * nvs) + 32 + 64;                                      // M vbuf drow
   n += up4(ns * 3) + 4 * up4(ns) + up4(nb);                          // con_off con_D con_kip con_body con_mask sub_end
   return n + 8;
 }
 
-__device__ __forceinline__ Lds carve(float* p, int nb, int nq, int nv, int nu, int ns, int nvs, int js) {
+template <int NP>
+__device__ __forceinline__ Lds carve(float* base, float* p, int nb, int nq, int nv, int nu, int ns) {
+  constexpr int js = stride_of(NP);
   Lds l;
+  l.vbuf = base; l.qvel = base + 32; l.warm = base + 64; l.drow = base + 96; l.M = base + 160;
+  p += 160 + NP * js;
   auto take = [&](int n) {
     float* r = p;
     p += up4(n);
     return r;
   };
-  l.qpos = take(nq); l.qvel = take(32); l.warm = take(nv); l.tau = take(nu);
-  l.xpos = take(nb * 3); l.xquat = take(nb * 4); l.xanchor = take(nb * 3); l.xaxis = take(nb * 3);
+  l.qpos = take(nq); l.tau = take(nu);
+  l.xpos = take(nb * 3); l.xquat = take(nb * 4);
   l.cdof = take(nv * 6); l.cvel = take(nb * 6);
   {
-    float* base = p;
+    float* first = p;
     l.cinert = take(nb * 10); l.crb = take(nb * 10); l.buf = take(nv * 6);
     l.fsub = take(nb * 6); l.cfrc = take(nb * 6);
+    l.xanchor = l.buf; l.xaxis = l.fsub;
     float* end = p;
-    l.J = base;  // written only after the bias forces are out of fsub
-    float* jend = base + up4(4 * ns * js + 32);
+    l.J = first;  // written only after the bias forces are out of fsub
+    float* jend = first + up4(4 * ns * js + 32);
     p = end > jend ? end : jend;
   }
-  l.M = take(nv * nvs); l.vbuf = take(32); l.drow = take(64);
   l.con_off = take(ns * 3); l.con_D = take(ns); l.con_kip = take(ns);
   l.con_body = reinterpret_cast<int*>(take(ns));
   l.con_mask = reinterpret_cast<unsigned*>(take(ns));
@@ -167,23 +173,16 @@ __device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myin
     }
 }
 
-// Mass matrix (LDS, rows of `stride` floats, zero beyond nv) into the accumulator layout, unit diagonal on the padding.
-__device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ M, int stride, int nv, int np, int lane) {
-  // The lane id is made opaque here: otherwise the sixteen unit-diagonal constants below are computed once, shared by
-  // all the call sites of a substep and kept (spilled) across the whole solver instead of being rebuilt in a few cycles.
-  asm volatile("" : "+v"(lane));
-  const int c = lane & 31, half = lane >> 5;
-  const bool real = c < nv;
-  const float* row = M + (real ? c : 0) * stride;
+// Mass matrix (LDS, NP rows: beyond nv unit rows and zero columns) into the accumulator layout.  What the tile holds outside
+// NP x NP is a copy of entries inside it: the factorisation writes there, but never reads.
+template <int NP>
+__device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ M, int lane) {
+  const int c = min(lane & 31, NP - 1), half = lane >> 5;
+  const float* row = M + c * stride_of(NP);
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const int r0 = 8 * g + 4 * half;
-    const bool inside = r0 + 4 <= np;
-    const float4 v = *reinterpret_cast<const float4*>(row + (inside ? r0 : 0));
-    T[4 * g] = (real && inside) ? v.x : (r0 == c ? 1.f : 0.f);
-    T[4 * g + 1] = (real && inside) ? v.y : (r0 + 1 == c ? 1.f : 0.f);
-    T[4 * g + 2] = (real && inside) ? v.z : (r0 + 2 == c ? 1.f : 0.f);
-    T[4 * g + 3] = (real && inside) ? v.w : (r0 + 3 == c ? 1.f : 0.f);
+    const float4 v = *reinterpret_cast<const float4*>(row + min(8 * g + 4 * half, NP - 4));
+    T[4 * g] = v.x; T[4 * g + 1] = v.y; T[4 * g + 2] = v.z; T[4 * g + 3] = v.w;
   }
 }
 
@@ -277,10 +276,10 @@ __device__ __forceinline__ float impedance_of(float pos, float dmin, float dmax,
   return imp;
 }
 // of the contact rows, and of the rows of joint limits and dry friction
-__device__ __forceinline__ float impedance(const DevModel& m, float pos) {
+__device__ __forceinline__ float impedance(const ModelHead& m, float pos) {
   return impedance_of(pos, m.dmin, m.dmax, m.width, m.mid, m.power, m.imp_a, m.imp_b);
 }
-__device__ __forceinline__ float impedance_dof(const DevModel& m, float pos) {
+__device__ __forceinline__ float impedance_dof(const ModelHead& m, float pos) {
   return impedance_of(pos, m.dr_dmin, m.dr_dmax, m.dr_width, m.dr_mid, m.dr_power, m.dr_imp_a, m.dr_imp_b);
 }
 
@@ -444,6 +443,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KS_STEP_WAVE
 void step_kernel(StepArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds_raw[];
   const DevModel& m = *a.model;
+  const ModelHead& mh = a.head;
   const int lane = threadIdx.x;
   // heaviest envs first when an order is given (ks_work_order, which also keeps neighbouring envs on one XCD); without
   // one, workgroup b takes env (b % 8) (N / 8) + b / 8 for the same reason
@@ -452,24 +452,30 @@ void step_kernel(StepArgs a) {
   else if (a.N % 8 == 0) env = (int64_t)(blockIdx.x % 8) * (a.N / 8) + blockIdx.x / 8;
   if (a.env_mask && !a.env_mask[env]) return;  // wave-uniform
   int work = 0;  // wave-uniform cost estimate of this control step
-  const int nb = m.nb, nq = m.nq, nv = m.nv, nu = m.nu, ns = m.ns, nvs = m.nvs, js = m.js;
-  Lds l = carve(lds_raw, nb, nq, nv, nu, ns, nvs, js);
-  const int rq = (nb > 1 && m.body_jtype[1] == kJntFree) ? 7 : 0;
+  const int nb = mh.nb, nq = mh.nq, nv = mh.nv, nu = mh.nu, ns = mh.ns;
+  constexpr int nvs = stride_of(NP), js = nvs;
+  Lds l = carve<NP>(lds_raw, lds_raw, nb, nq, nv, nu, ns);
+  const int rq = mh.root_free ? 7 : 0;
   const int rv = rq ? 6 : 0;
 
   for (int i = lane; i < nq; i += 64) l.qpos[i] = a.qpos[env * nq + i];
   if (lane < 32) l.qvel[lane] = lane < nv ? a.qvel[env * nv + lane] : 0.f;
   if (lane < nv) l.warm[lane] = a.qacc_warmstart ? a.qacc_warmstart[env * nv + lane] : 0.f;
+  // The mass matrix: a substep writes the entries that couple dofs of one chain, the same ones every time; everything else is
+  // written here, once per launch (zero, and one on the diagonal of the padding rows).
+  for (int i = lane; i < NP * nvs / 4; i += 64) reinterpret_cast<float4*>(l.M)[i] = {0.f, 0.f, 0.f, 0.f};
+  KS_SYNC();
+  if (lane >= nv && lane < NP) l.M[lane * nvs + lane] = 1.f;
   for (int i = lane; i < nu; i += 64) l.tau[i] = a.ctrl_in ? a.ctrl_in[env * nu + i] : 0.f;
   for (int i = lane; i < nb; i += 64) l.sub_end[i] = m.body_subtree_end[i];
   if (lane == 0) {  // world body
-    for (int k = 0; k < 3; ++k) { l.xpos[k] = 0.f; l.xanchor[k] = 0.f; l.xaxis[k] = 0.f; }
+    for (int k = 0; k < 3; ++k) l.xpos[k] = 0.f;
     l.xquat[0] = 1.f; l.xquat[1] = l.xquat[2] = l.xquat[3] = 0.f;
     for (int k = 0; k < 6; ++k) l.cvel[k] = 0.f;
   }
-  const float mu = a.friction ? a.friction[env] : m.friction;
+  const float mu = a.friction ? a.friction[env] : mh.friction;
   const float latency = a.latency ? a.latency[env] : 0.f;
-  const float scale = 1.0f / (m.meaninertia * (float)(nv > 1 ? nv : 1));
+  const float scale = 1.0f / (mh.meaninertia * (float)(nv > 1 ? nv : 1));
   KS_SYNC();
 #ifdef KS_PROFILE
   float prof[16];
@@ -586,7 +592,7 @@ void step_kernel(StepArgs a) {
           const KsEventDesc ev = a.events[e];
           // the timer stays in memory between substeps (lane 0 owns it) so that it costs no register over the solver
           float* tleft = a.event_state + (int64_t)e * a.N + env;
-          float left = lane_bcast(lane == 0 ? *tleft : 0.f, 0) - m.dt;
+          float left = lane_bcast(lane == 0 ? *tleft : 0.f, 0) - mh.dt;
           if (left <= 0.f) {  // wave-uniform
             float u0, u1, u2;
             if (a.event_uniform) {
@@ -606,7 +612,7 @@ void step_kernel(StepArgs a) {
                 l.qvel[5] += (u0 < 0.5f ? -mag : mag) * ev.level_scale;
               } else if (ev.kind == KS_EVENT_JUMP) {
                 const float h = (ev.lo + u0 * (ev.hi - ev.lo)) * ev.level_scale;
-                for (int k = 0; k < 3; ++k) l.qvel[k] += sqrtf(2.f * -m.gravity[k] * h);
+                for (int k = 0; k < 3; ++k) l.qvel[k] += sqrtf(2.f * -mh.gravity[k] * h);
               }
             }
             left = ev.interval_lo + u2 * (ev.interval_hi - ev.interval_lo);
@@ -656,7 +662,7 @@ void step_kernel(StepArgs a) {
       unsigned ch[kMaxDepth / 2];
 #pragma unroll
       for (int k = 0; k < kMaxDepth / 2; ++k) ch[k] = chain[k];
-      for (int k = 0; k < m.max_depth; k += 2) {
+      for (int k = 0; k < mh.max_depth; k += 2) {
         const float* p0 = lpose + 7 * (int)(ch[0] & 31u);
         const float* p1 = lpose + 7 * (int)((ch[0] >> 16) & 31u);
         const V3 t0 = ld3(p0), t1 = ld3(p1);
@@ -751,7 +757,6 @@ void step_kernel(StepArgs a) {
       const int b = idx / 10, k = idx - 10 * b;
       l.crb[idx] = b > 0 ? range_sum(l.cinert + k, 10, b, l.sub_end[b]) : 0.f;
     }
-    for (int idx = lane; idx < nv * nvs / 4; idx += 64) reinterpret_cast<float4*>(l.M)[idx] = {0.f, 0.f, 0.f, 0.f};  // nvs is a multiple of 4
     KS_SYNC();
     if (is_dof) {
       const Sp f = inert_mul(l.crb + 10 * d_body, my_cdof);
@@ -761,7 +766,7 @@ void step_kernel(StepArgs a) {
     KS_SYNC();
 #pragma unroll
     for (int k0 = 0; k0 < kPairSets; k0 += 4) {  // four sets of 64 pairs: all their reads before the first write
-      if (64 * k0 >= m.npairs) break;
+      if (64 * k0 >= mh.npairs) break;
       float v[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -782,7 +787,7 @@ void step_kernel(StepArgs a) {
     // body accumulates them over the dofs of its own ancestor chain, root first (no pass per tree level)
     {
       Sp v = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-      Sp acc = {{0.f, 0.f, 0.f}, {-m.gravity[0], -m.gravity[1], -m.gravity[2]}};
+      Sp acc = {{0.f, 0.f, 0.f}, {-mh.gravity[0], -mh.gravity[1], -mh.gravity[2]}};
       auto hinge = [&](const Sp& cd, float qd) {
         acc = acc + cross_motion(v, cd) * qd;
         v = v + cd * qd;
@@ -804,7 +809,7 @@ void step_kernel(StepArgs a) {
           v = v + dv;
         }
       };
-      for (int k = 0; k < m.max_depth; k += 2) {
+      for (int k = 0; k < mh.max_depth; k += 2) {
         const unsigned e0 = chain[0] & 0xffffu, e1 = chain[0] >> 16;
         const int d0 = (int)((e0 >> 5) & 31u), d1 = (int)((e1 >> 5) & 31u);
         const Sp c0 = ld6(l.cdof + 6 * d0), c1 = ld6(l.cdof + 6 * d1);
@@ -830,7 +835,7 @@ void step_kernel(StepArgs a) {
           float s7[7];
 #pragma unroll
           for (int k = 0; k < 7; ++k) s7[k] = lane_bcast(lane == 0 ? st[k] : 0.f, 0);
-          float dur = s7[0] - m.dt, left = lane_bcast(lane == 0 ? *tleft : 0.f, 0) - m.dt;
+          float dur = s7[0] - mh.dt, left = lane_bcast(lane == 0 ? *tleft : 0.f, 0) - mh.dt;
 #pragma unroll
           for (int k = 0; k < 6; ++k) s7[1 + k] *= ev.level_scale;   // events.py:296: the carried wrench itself is rescaled
           const bool on = dur > 0.f && lane == ev.body;                // events.py:297-299, 302-307
@@ -917,7 +922,7 @@ void step_kernel(StepArgs a) {
     const bool touching = is_sph && (dist < 0.f);
     const unsigned long long cmask = __ballot(touching);
     const int ncon = __popcll(cmask);
-    const bool frictionless = m.frictionless != 0;
+    const bool frictionless = mh.frictionless != 0;
     const int nefc = frictionless ? ncon : 4 * ncon;
     // A launch ends with its slowest wavefront, and an env with many contacts runs several times longer than an airborne
     // one: waves with more constraint rows get a higher issue priority on their SIMD, which shortens exactly those.
@@ -930,11 +935,11 @@ void step_kernel(StepArgs a) {
       l.con_body[c] = s_body;
       l.con_mask[c] = s_mask;
       st3(l.con_off + 3 * c, cpos - com);
-      const float invweight = frictionless ? s_invw : (s_invw + mu * mu * s_invw) * 2.f * mu * mu / m.impratio;
-      const float imp = impedance(m, dist);
+      const float invweight = frictionless ? s_invw : (s_invw + mu * mu * s_invw) * 2.f * mu * mu / mh.impratio;
+      const float imp = impedance(mh, dist);
       const float Rr = fmaxf(invweight * (1.f - imp) / imp, 1e-15f);
       l.con_D[c] = 1.0f / Rr;
-      l.con_kip[c] = m.con_k * imp * dist;
+      l.con_kip[c] = mh.con_k * imp * dist;
     }
     KS_SYNC();
 
@@ -944,7 +949,7 @@ void step_kernel(StepArgs a) {
     float myinv;
     {
       f32x16 T;
-      load_mtile(T, l.M, nvs, nv, NP, lane);
+      load_mtile<NP>(T, l.M, lane);
       chol_tile<NP>(T, R, myinv, lane, nv);
     }
     const float qas_all = solve_regs<NP>(R, myinv, lane, qfs, nv);
@@ -969,15 +974,15 @@ void step_kernel(StepArgs a) {
           const float pos = fminf(dlo, dhi);
           if (pos < 0.f) {  // the nearer side, once violated
             dr.lim_s = dlo < dhi ? 1.f : -1.f;
-            const float imp = impedance_dof(m, pos);
+            const float imp = impedance_dof(mh, pos);
             dr.lim_D = 1.f / fmaxf(KS_REC(m, lane_r, d_invw) * (1.f - imp) / imp, 1e-15f);
-            dr.lim_aref = -m.dr_b * dr.lim_s * my_qvel - m.dr_k * imp * pos;
+            dr.lim_aref = -mh.dr_b * dr.lim_s * my_qvel - mh.dr_k * imp * pos;
           }
         }
         dr.fr_fl = a.frictionloss ? ((KS_REC(m, lane_r, d_jtype) == kJntHinge) ? a.frictionloss[env * nv + lane] : 0.f) : KS_REC(m, lane_r, d_floss);
         dr.fr_D = KS_REC(m, lane_r, d_frD);
         dr.fr_rf = dr.fr_fl / dr.fr_D;
-        dr.fr_aref = -m.dr_b * my_qvel;
+        dr.fr_aref = -mh.dr_b * my_qvel;
       }
       ndr = __popcll(__ballot(dr.lim_s != 0.f)) + __popcll(__ballot(dr.fr_fl > 0.f));
     }
@@ -1012,7 +1017,7 @@ void step_kernel(StepArgs a) {
           float vv[NP];
           load_row<NP>(l.qvel, vv);
           const float vel = row_dot<NP>(l.J + lane * js, vv);
-          aref = -m.con_b * vel - l.con_kip[c];
+          aref = -mh.con_b * vel - l.con_kip[c];
           D = l.con_D[c];
         }
       }
@@ -1105,10 +1110,10 @@ void step_kernel(StepArgs a) {
         const float grad = is_dof ? Ma - qfs - qfc : 0.f;
         const float improvement = scale * (prev_cost - cost);
         const float gradient = scale * sqrtf(wave_sum(grad * grad));
-        bool done = niter >= m.iterations;
-        done |= improvement < m.tolerance;
-        done |= gradient < m.tolerance;
-        if (done && !(m.iterations == 1 && niter == 0)) break;
+        bool done = niter >= mh.iterations;
+        done |= improvement < mh.tolerance;
+        done |= gradient < mh.tolerance;
+        if (done && !(mh.iterations == 1 && niter == 0)) break;
         KS_PHASE(10)
         // ---- Newton direction: H = M + J^T diag(D active) J.  The rank-nefc term runs on the matrix cores: one
         // 32x32x2 fp32 MFMA per pair of constraint rows, operands straight from the LDS copy of J (lane = column,
@@ -1121,7 +1126,7 @@ void step_kernel(StepArgs a) {
           l.drow[lane] = active ? D : 0.f;
           KS_SYNC();
           f32x16 hc;
-          load_mtile(hc, l.M, nvs, nv, NP, lane);
+          load_mtile<NP>(hc, l.M, lane);
           const int col = lane & 31, half = lane >> 5;
           const bool col_ok = NP == 32 || col < NP;
           // the operands of four products at a time are fetched before the first of them (a row past the last counts as zero)
@@ -1167,14 +1172,14 @@ void step_kernel(StepArgs a) {
           if (is_dof) mv = row_dot<NP>(Mrow, vv);
           if (is_row) jv = row_dot<NP>(l.J + (is_row ? lane : 0) * js, vv);
         }
-        const float smag = sqrtf(wave_sum(search * search)) * m.meaninertia * (float)(nv > 1 ? nv : 1);
-        const float gtol = m.tolerance * m.ls_tolerance * smag;
+        const float smag = sqrtf(wave_sum(search * search)) * mh.meaninertia * (float)(nv > 1 ? nv : 1);
+        const float gtol = mh.tolerance * mh.ls_tolerance * smag;
         const float g0 = gauss;
         const float g1 = wave_sum(is_dof ? search * (Ma - qfs) : 0.f);
         const float g2 = 0.5f * wave_sum(is_dof ? search * mv : 0.f);
         float alpha;
         if (nefc <= 32 && !(DR && ndr > 0)) {
-          alpha = line_search_rows(m.ls_iterations, nefc, lane, Jaref, jv, D, g0, g1, g2, gtol);
+          alpha = line_search_rows(mh.ls_iterations, nefc, lane, Jaref, jv, D, g0, g1, g2, gtol);
         } else {
           const float q0r = 0.5f * Jaref * Jaref * D, q1r = jv * Jaref * D, q2r = 0.5f * jv * jv * D;
           // With at most 16 constraint rows the three sums of a cost evaluation share one reduction: the 16-lane
@@ -1248,7 +1253,7 @@ void step_kernel(StepArgs a) {
           bool swap = true;
           int it = 0;
           while (true) {
-            bool ls_done = it >= m.ls_iterations;
+            bool ls_done = it >= mh.ls_iterations;
             ls_done |= !swap;
             ls_done |= (lo.d0 < 0.f) && (lo.d0 > -gtol);
             ls_done |= (hi.d0 > 0.f) && (hi.d0 < gtol);
@@ -1329,13 +1334,13 @@ void step_kernel(StepArgs a) {
       const float d_damping = KS_REC(m, lane_e, d_damping) * ((a.damping_scale && lane_e < nv) ? a.damping_scale[env * nv + lane_e] : 1.f);
       const float my_qvel = lane_e < nv ? l.qvel[lane_e] : 0.f;
       float qacc_int = qacc;
-      if (m.eulerdamp) {
+      if (mh.eulerdamp) {
         // implicit in the joint damping: (M + dt diag(damping)) a = M qacc.  For torque motors, whose force does
         // not depend on velocity, this is MuJoCo's implicitfast step; qacc itself (warm start, output) is unchanged.
         f32x16 T;
-        load_mtile(T, l.M, nvs, nv, NP, lane);
+        load_mtile<NP>(T, l.M, lane);
         const int c = lane & 31, half = lane >> 5;
-        const float hd = m.dt * __shfl(is_dof ? d_damping : 0.f, c);
+        const float hd = mh.dt * __shfl(is_dof ? d_damping : 0.f, c);
 #pragma unroll
         for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -1346,23 +1351,23 @@ void step_kernel(StepArgs a) {
         const float sol = solve_regs<NP>(R2, inv2, lane, is_dof ? Mqacc : 0.f, nv);
         qacc_int = is_dof ? sol : 0.f;
       }
-      if (is_dof) l.qvel[lane] = my_qvel + m.dt * qacc_int;
+      if (is_dof) l.qvel[lane] = my_qvel + mh.dt * qacc_int;
       KS_SYNC();
       if (is_body) {
         const int qa = b_qadr, da = b_dofadr;
         if (b_jtype == kJntFree) {
-          for (int k = 0; k < 3; ++k) l.qpos[qa + k] += m.dt * l.qvel[da + k];
+          for (int k = 0; k < 3; ++k) l.qpos[qa + k] += mh.dt * l.qvel[da + k];
           const V3 w = ld3(l.qvel + da + 3);
           const float n = sqrtf(dot(w, w));
           Quat q = {l.qpos[qa + 3], l.qpos[qa + 4], l.qpos[qa + 5], l.qpos[qa + 6]};
           if (n > 1e-15f) {
-            const float h = 0.5f * n * m.dt, s = sinf(h) / n;
+            const float h = 0.5f * n * mh.dt, s = sinf(h) / n;
             q = qmul(q, {cosf(h), w.x * s, w.y * s, w.z * s});
           }
           q = qnormalize(q);
           l.qpos[qa + 3] = q.w; l.qpos[qa + 4] = q.x; l.qpos[qa + 5] = q.y; l.qpos[qa + 6] = q.z;
         } else if (b_jtype == kJntHinge) {
-          l.qpos[qa] += m.dt * l.qvel[da];
+          l.qpos[qa] += mh.dt * l.qvel[da];
         }
       }
     }
@@ -1380,7 +1385,7 @@ void step_kernel(StepArgs a) {
     if (a.work && lane == 0) a.work[env] = work;
     if (a.time && lane == 0) {  // dt added once per substep in fp32, like the reference's accumulation
       float time = a.time[env];
-      for (int k = 0; k < nsub; ++k) time += m.dt;
+      for (int k = 0; k < nsub; ++k) time += mh.dt;
       a.time[env] = time;
     }
     if (a.last_ctrl) {
@@ -1426,8 +1431,6 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
   m.nb = d->nb; m.nq = d->nq; m.nv = d->nv; m.nu = d->nu; m.ns = d->ns;
   m.iterations = d->iterations; m.ls_iterations = d->ls_iterations; m.eulerdamp = d->eulerdamp;
   m.frictionless = d->condim == 1 ? 1 : 0;
-  m.nvs = m_stride(d->nv);
-  m.js = j_stride(d->nv);
   m.dt = (float)d->dt;
   for (int k = 0; k < 3; ++k) m.gravity[k] = (float)d->gravity[k];
   m.tolerance = (float)d->tolerance; m.ls_tolerance = (float)d->ls_tolerance;
@@ -1485,6 +1488,7 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     m.body_depth[b] = n;
     if (n > m.max_depth) m.max_depth = n;
   }
+  m.root_free = d->nb > 1 && m.body_jtype[1] == kJntFree;
   for (int q = 0; q < d->nq; ++q) m.qpos0[q] = (float)d->qpos0[q];
   for (int j = 0; j < d->nv; ++j) {
     m.dof_body[j] = d->dof_body[j]; m.dof_parent[j] = d->dof_parent[j]; m.dof_act[j] = -1;
@@ -1616,6 +1620,7 @@ static int launch_step(const KsModel* km, ks_stream_t stream, const KsStepIO* io
   StepArgs a;
   std::memset(&a, 0, sizeof(a));
   a.model = km->dev;
+  a.head = m;
   a.N = io->N;
   a.qpos = io->qpos; a.qvel = io->qvel; a.qacc_warmstart = io->qacc_warmstart; a.time = io->time;
   a.friction = io->friction; a.mass_scale = io->mass_scale; a.env_mask = io->env_mask; a.fresh = io->fresh;

@@ -16,11 +16,11 @@ constexpr int kMaxPairs = kMaxV * (kMaxV - 1) / 2;
 
 enum { kJntNone = 0, kJntFree = 1, kJntHinge = 2 };
 
-// Immutable after ks_model_create(); lives in device global memory and is read through the
-// vector L1 / scalar cache (it is ~10 KB and shared by every wavefront).
-struct DevModel {
-  int nb, nq, nv, nu, ns, iterations, ls_iterations, eulerdamp, npairs, nvs /* row stride of the mass matrix in LDS, a multiple of 4 */, max_depth,
-      js /* row stride of the constraint Jacobian in LDS, a multiple of 4 */,
+// The sizes and scalar constants of a model.  They ride in the kernel arguments: the compiler knows those as constant and reads
+// them through the scalar unit, where the same values behind the model pointer are vector loads that a substep waits for.
+struct ModelHead {
+  int nb, nq, nv, nu, ns, iterations, ls_iterations, eulerdamp, npairs, max_depth,
+      root_free /* 1: body 1 hangs on a free joint */,
       dofrows /* 1 when a joint is limited or has dry friction */, nfriction /* dofs with dry friction */,
       invw_ok /* 1 when every hinge dof has a positive inverse weight (what rows on the dof lanes are regularised with) */,
       frictionless /* 1: condim 1, one normal row per contact instead of the four pyramid edges */;
@@ -30,6 +30,11 @@ struct DevModel {
   float imp_a, imp_b;  // 1 / mid^(power-1) and 1 / (1-mid)^(power-1), the constant factors of the impedance curve
   // the same constants for the rows of joint limits and dry friction
   float dr_k, dr_b, dr_dmin, dr_dmax, dr_width, dr_mid, dr_power, dr_imp_a, dr_imp_b;
+};
+
+// Immutable after ks_model_create(); lives in device global memory and is read through the
+// vector L1 / scalar cache (it is ~30 KB and shared by every wavefront).
+struct DevModel : ModelHead {
   int body_parent[kMaxB], body_jtype[kMaxB], body_qadr[kMaxB], body_dofadr[kMaxB], body_subtree_end[kMaxB],
       body_depth[kMaxB];
   unsigned body_dofmask[kMaxB];      // bit j set when dof j moves the body

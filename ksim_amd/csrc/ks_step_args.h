@@ -3,13 +3,13 @@
 #include <stdint.h>
 
 #include "../../include/ksim_hip.h"
+#include "ks_model.h"
 
 namespace ks {
 
-struct DevModel;
-
 struct StepArgs {
   const DevModel* model;
+  ModelHead head;
   int64_t N;
   int substeps, actuator_period, actuator_type;
   float action_scale;
