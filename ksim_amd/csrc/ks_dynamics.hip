@@ -223,31 +223,30 @@ __device__ __forceinline__ float row_dot(const float* row, const float (&vv)[NP]
   return s0 + s1;
 }
 
-// Per-lane constants of one substep, as stored in DevModel::lane_rec (72 dwords, filled by ks_model_create):
+// Per-lane constants of one substep, as stored in DevModel::lane_rec (64 dwords, filled by ks_model_create):
 // lane L's body (L < nb), dof (L < nv), contact sphere (L < ns) and its share of the (i, ancestor j) dof pairs.
 // Lanes beyond a range carry the entries of index 0 (or -1 / zero where the kernel tests for that).
 constexpr int kPairSets = (kMaxPairs + 63) / 64;
 
 struct LaneRec {
-  int b_parent, b_jtype, b_qadr, b_dofadr;
-  int b_depth;
+  int b_jtype, b_qadr, b_dofadr, b_depth;
   float b_q0, b_mass, d_stiffness;  // d_stiffness: spring of the hinge whose dof this lane holds
-  float b_pos[3], b_ipos[3], b_inertia[3], b_jaxis[3], b_jpos[3], pad1;
+  float d_damping;
+  float b_pos[3], d_armature, b_jaxis[3], d_gear, b_jpos[3], d_lo;
   float b_quat[4], b_iquat[4];
   int d_body, d_act, d_jtype, d_k;
-  float d_damping, d_armature, d_gear, d_lo, d_hi;
+  float d_hi;
   int s_body;
-  float s_rad, s_invw;
-  float s_pos[3];
+  float s_invw;
   unsigned s_mask;
   int pk[kPairSets];
+  // the body's ancestors from the tree root down to itself, 16 bits each: body | first dof << 5 | hinge << 10 | free joint << 11
+  unsigned b_chain[kMaxDepth / 2];
   // rows that live on the dof's own lane: hinge limit (range, inverse weight, address of the joint angle) and dry
   // friction (level and the constant stiffness 1 / R of its row)
   int d_limited, d_qadr;
   float d_rlo, d_rhi, d_invw, d_floss, d_frD;
-  // the body's ancestors from the tree root down to itself, 16 bits each: body | first dof << 5 | hinge << 10 | free joint << 11
-  unsigned b_chain[kMaxDepth / 2];
-  int pad2[3];
+  int pad[7];
 };
 static_assert(sizeof(LaneRec) == sizeof(DevModel::lane_rec) / 64, "LaneRec must fill the record");
 static_assert(kMaxB <= 32 && kMaxV <= 32 && kMaxDepth % 2 == 0, "a link of b_chain holds 5 + 5 bits");
@@ -260,9 +259,9 @@ struct LsPoint {
 };
 
 // constraint impedance d(|pos|) of a solimp whose parameters are already clamped
-__device__ __forceinline__ float impedance_of(float pos, float dmin, float dmax, float width, float mid, float power, float imp_a,
+__device__ __forceinline__ float impedance_of(float pos, float dmin, float dmax, float width_inv, float mid, float power, float imp_a,
                                               float imp_b) {
-  const float ix = fabsf(pos) / width;
+  const float ix = fabsf(pos) * width_inv;
   // x^power: the default power of 2 (and 1) without the general power function
   const float ox = 1.f - ix;
   const float px = power == 2.f ? ix * ix : (power == 1.f ? ix : powf(ix, power));
@@ -277,10 +276,10 @@ __device__ __forceinline__ float impedance_of(float pos, float dmin, float dmax,
 }
 // of the contact rows, and of the rows of joint limits and dry friction
 __device__ __forceinline__ float impedance(const ModelHead& m, float pos) {
-  return impedance_of(pos, m.dmin, m.dmax, m.width, m.mid, m.power, m.imp_a, m.imp_b);
+  return impedance_of(pos, m.dmin, m.dmax, m.width_inv, m.mid, m.power, m.imp_a, m.imp_b);
 }
 __device__ __forceinline__ float impedance_dof(const ModelHead& m, float pos) {
-  return impedance_of(pos, m.dr_dmin, m.dr_dmax, m.dr_width, m.dr_mid, m.dr_power, m.dr_imp_a, m.dr_imp_b);
+  return impedance_of(pos, m.dr_dmin, m.dr_dmax, m.dr_width_inv, m.dr_mid, m.dr_power, m.dr_imp_a, m.dr_imp_b);
 }
 
 // The rows a dof lane carries itself: the violated limit of its hinge (J = lim_s e_j, lim_s = +-1, 0 when none) and its
@@ -484,6 +483,7 @@ void step_kernel(StepArgs a) {
 #endif
 
   const int nsub = FWD ? 1 : a.substeps;
+  int act_wait = 0;  // substeps until the next actuator update
   // An env that the termination pass has just reset still owes the forward pass of its reset (engine.py:213: derived
   // quantities and the warm start of the new episode, from the reset state with zero controls).  With `fresh` given the
   // step does it itself, as a pass `sub = -1` that neither actuates nor integrates, instead of a masked launch of the
@@ -508,31 +508,27 @@ void step_kernel(StepArgs a) {
 #pragma unroll
       for (int k = 0; k < kRecPieces; ++k) dst[k] = *reinterpret_cast<const uint4*>(m.lane_rec[k][lane]);
     }
-    const int b_parent = rec.b_parent, b_jtype = rec.b_jtype, b_qadr = rec.b_qadr, b_dofadr = rec.b_dofadr,
-              b_depth = rec.b_depth;
-    (void)b_parent;
+    // the row of an optional operand: this env's, or row 0 of what stands in for it
+    auto row_of = [&](unsigned bit) -> int64_t { return (a.given & bit) ? env : 0; };
+    const int b_jtype = rec.b_jtype, b_qadr = rec.b_qadr, b_dofadr = rec.b_dofadr, b_depth = rec.b_depth;
     const V3 b_pos = {rec.b_pos[0], rec.b_pos[1], rec.b_pos[2]};
-    V3 b_ipos = {rec.b_ipos[0], rec.b_ipos[1], rec.b_ipos[2]}, b_inertia = {rec.b_inertia[0], rec.b_inertia[1], rec.b_inertia[2]};
-    if (a.body_ipos && is_body) b_ipos = ld3(a.body_ipos + (env * nb + bl) * 3);        // per-env centres of mass
-    if (a.body_inertia && is_body) b_inertia = ld3(a.body_inertia + (env * nb + bl) * 3);  // and principal inertias
-    const V3
-             b_jaxis = {rec.b_jaxis[0], rec.b_jaxis[1], rec.b_jaxis[2]}, b_jpos = {rec.b_jpos[0], rec.b_jpos[1], rec.b_jpos[2]};
+    const V3 b_ipos = ld3(a.body_ipos + (row_of(kOptIpos) * nb + bl) * 3);          // per-env centres of mass
+    const V3 b_inertia = ld3(a.body_inertia + (row_of(kOptInertia) * nb + bl) * 3);  // and principal inertias
+    const V3 b_jaxis = {rec.b_jaxis[0], rec.b_jaxis[1], rec.b_jaxis[2]}, b_jpos = {rec.b_jpos[0], rec.b_jpos[1], rec.b_jpos[2]};
     const Quat b_quat = {rec.b_quat[0], rec.b_quat[1], rec.b_quat[2], rec.b_quat[3]};
     const Quat b_iquat = {rec.b_iquat[0], rec.b_iquat[1], rec.b_iquat[2], rec.b_iquat[3]};
     const float b_q0 = rec.b_q0;
-    const float b_mass = is_body ? rec.b_mass * (a.mass_scale ? a.mass_scale[env * nb + bl] : 1.f) : 0.f;
+    const float b_scale = a.mass_scale[row_of(kOptMass) * nb + bl];
+    const float b_mass = is_body ? rec.b_mass * b_scale : 0.f;
     const int d_body = rec.d_body, d_act = rec.d_act, d_jtype = rec.d_jtype, d_k = rec.d_k;
-    const float d_damping = rec.d_damping * ((a.damping_scale && is_dof) ? a.damping_scale[env * nv + lane] : 1.f);
-    const float d_armature = rec.d_armature * ((a.armature_scale && is_dof) ? a.armature_scale[env * nv + lane] : 1.f);
+    const int dl = is_dof ? lane : 0;
+    const float d_damping = rec.d_damping * a.damping_scale[row_of(kOptDamping) * nv + dl];
+    const float d_armature = rec.d_armature * a.armature_scale[row_of(kOptArmature) * nv + dl];
     const float d_gear = rec.d_gear, d_lo = rec.d_lo, d_hi = rec.d_hi;
-    const int s_body = rec.s_body;
-    V3 s_pos = {rec.s_pos[0], rec.s_pos[1], rec.s_pos[2]};
-    float s_rad = rec.s_rad;
+    const int s_body = rec.s_body, sl = is_sph ? lane : 0;
+    const V3 s_pos = ld3(a.sph_pos + (row_of(kOptSphere) * ns + sl) * 3);  // per-env contact spheres
+    const float s_rad = a.sph_radius[row_of(kOptSphere) * ns + sl];
     const float s_invw = rec.s_invw;
-    if (a.sph_pos && lane < ns) {  // per-env contact spheres
-      s_pos = ld3(a.sph_pos + (env * ns + lane) * 3);
-      s_rad = a.sph_radius[env * ns + lane];
-    }
     const unsigned s_mask = rec.s_mask;
     unsigned chain[kMaxDepth / 2];
 #pragma unroll
@@ -542,42 +538,42 @@ void step_kernel(StepArgs a) {
     for (int k = 0; k < kPairSets; ++k) pk[k] = rec.pk[k];
 
     // ---- actuators (ksim/engine.py:287-320, ksim/actuators.py:198-217)
-    if (!fwd && (sub % a.actuator_period) == 0 && lane < nu) {
+    const bool actuate = !fwd && act_wait == 0;
+    if (!fwd) act_wait = (act_wait == 0 ? a.actuator_period : act_wait) - 1;
+    if (actuate && lane < nu) {
       const int u = lane;
       // the actuator inputs of this control step are read again at every actuator update (they stay in the caches):
       // held in registers they would be live across the solver of every substep
       const bool posvel = a.actuator_type == KS_ACT_POSITION_VELOCITY;
       const int na = posvel ? 2 * nu : nu;  // width of the action vector
-      const int64_t ea = env * na + lane, eu = env * nu + lane;
+      const int64_t ea = env * na + lane, srow = (int64_t)sub * a.N + env;
+      const int64_t noise_a = ((a.given & kOptActionNoise) ? srow : 0) * na + u, noise_t = ((a.given & kOptTorqueNoise) ? srow : 0) * nu + u;
       const float u_last = a.last_ctrl[ea], u_act = a.action[ea];
-      const bool u_drop = a.drop && a.drop[ea];
-      const float u_zero = a.zero_offset ? a.zero_offset[eu] : 0.f;
-      float u_kp = 0.f, u_kd = 0.f, u_lim = 0.f, u_abias = 0.f, u_tbias = 0.f;
-      if (a.actuator_type != KS_ACT_TORQUE) {
-        u_kp = a.kp[lane] * (a.kp_scale ? a.kp_scale[env] : 1.f);
-        u_kd = a.kd[lane] * (a.kd_scale ? a.kd_scale[env] : 1.f);
-        u_lim = a.ctrl_clip[lane] * (a.torque_limit_scale ? a.torque_limit_scale[env] : 1.f);
-        u_abias = a.action_bias ? a.action_bias[eu] : 0.f;
-        u_tbias = a.torque_bias ? a.torque_bias[eu] : 0.f;
-      }
+      const int64_t drop_at = row_of(kOptDrop) * na + u;
+      const bool u_drop = a.drop[drop_at] != 0;
+      const float u_kp = a.kp[lane] * a.kp_scale[row_of(kOptKp)];
+      const float u_kd = a.kd[lane] * a.kd_scale[row_of(kOptKd)];
+      const float u_lim = a.ctrl_clip[lane] * a.torque_limit_scale[row_of(kOptLimit)];
+      const float u_zero = a.zero_offset[row_of(kOptZero) * nu + u];
+      const float u_abias = a.action_bias[row_of(kOptActionBias) * nu + u], u_tbias = a.torque_bias[row_of(kOptTorqueBias) * nu + u];
+      const float u_anoise = a.action_noise[noise_a], u_tnoise = a.torque_noise[noise_t];
       float prct = (float)sub - latency;
       prct = fminf(fmaxf(prct, 0.f), 1.f);
       const float c = u_drop ? u_last : u_last * (1.0f - prct) + u_act * prct;
-      const int64_t su = ((int64_t)sub * a.N + env) * nu + u, sa = ((int64_t)sub * a.N + env) * na + u;
       float t;
       if (a.actuator_type == KS_ACT_TORQUE) {
-        t = c + (a.torque_noise ? a.torque_noise[su] : 0.f);
+        t = c + u_tnoise;
       } else {
         float target_vel = 0.f;
         if (posvel) {  // the velocity targets ride in the second half of the action vector
           const float v_last = a.last_ctrl[ea + nu], v_act = a.action[ea + nu];
-          const bool v_drop = a.drop && a.drop[ea + nu];
-          target_vel = (v_drop ? v_last : v_last * (1.0f - prct) + v_act * prct) + (a.action_noise ? a.action_noise[sa + nu] : 0.f);
+          const bool v_drop = a.drop[drop_at + nu] != 0;
+          target_vel = (v_drop ? v_last : v_last * (1.0f - prct) + v_act * prct) + a.action_noise[noise_a + nu];
         }
-        const float target = c * a.action_scale + (a.action_noise ? a.action_noise[sa] : 0.f) + u_abias;
+        const float target = c * a.action_scale + u_anoise + u_abias;
         const float q = l.qpos[rq + u] - u_zero;
         t = u_kp * (target - q) + u_kd * (target_vel - l.qvel[rv + u]);
-        t = t + (a.torque_noise ? a.torque_noise[su] : 0.f) + u_tbias;
+        t = t + u_tnoise + u_tbias;
         t = fminf(fmaxf(t, -u_lim), u_lim);
       }
       l.tau[u] = t;
@@ -935,10 +931,10 @@ void step_kernel(StepArgs a) {
       l.con_body[c] = s_body;
       l.con_mask[c] = s_mask;
       st3(l.con_off + 3 * c, cpos - com);
-      const float invweight = frictionless ? s_invw : (s_invw + mu * mu * s_invw) * 2.f * mu * mu / mh.impratio;
+      const float invweight = frictionless ? s_invw : (s_invw + mu * mu * s_invw) * 2.f * mu * mu * mh.impratio_inv;
       const float imp = impedance(mh, dist);
-      const float Rr = fmaxf(invweight * (1.f - imp) / imp, 1e-15f);
-      l.con_D[c] = 1.0f / Rr;
+      const float Rr = fmaxf(invweight * (1.f - imp) * __builtin_amdgcn_rcpf(imp), 1e-15f);  // imp lies in [1e-4, 1)
+      l.con_D[c] = __builtin_amdgcn_rcpf(Rr);
       l.con_kip[c] = mh.con_k * imp * dist;
     }
     KS_SYNC();
@@ -1109,7 +1105,7 @@ void step_kernel(StepArgs a) {
         // ---- gradient; stop before paying for another Hessian when the solver is done
         const float grad = is_dof ? Ma - qfs - qfc : 0.f;
         const float improvement = scale * (prev_cost - cost);
-        const float gradient = scale * sqrtf(wave_sum(grad * grad));
+        const float gradient = scale * __builtin_amdgcn_sqrtf(wave_sum(grad * grad));
         bool done = niter >= mh.iterations;
         done |= improvement < mh.tolerance;
         done |= gradient < mh.tolerance;
@@ -1172,7 +1168,7 @@ void step_kernel(StepArgs a) {
           if (is_dof) mv = row_dot<NP>(Mrow, vv);
           if (is_row) jv = row_dot<NP>(l.J + (is_row ? lane : 0) * js, vv);
         }
-        const float smag = sqrtf(wave_sum(search * search)) * mh.meaninertia * (float)(nv > 1 ? nv : 1);
+        const float smag = __builtin_amdgcn_sqrtf(wave_sum(search * search)) * mh.meaninertia * (float)(nv > 1 ? nv : 1);
         const float gtol = mh.tolerance * mh.ls_tolerance * smag;
         const float g0 = gauss;
         const float g1 = wave_sum(is_dof ? search * (Ma - qfs) : 0.f);
@@ -1331,7 +1327,7 @@ void step_kernel(StepArgs a) {
       int lane_e = threadIdx.x;
       asm volatile("" : "+v"(lane_e));
       const int b_jtype = KS_REC(m, lane_e, b_jtype), b_qadr = KS_REC(m, lane_e, b_qadr), b_dofadr = KS_REC(m, lane_e, b_dofadr);
-      const float d_damping = KS_REC(m, lane_e, d_damping) * ((a.damping_scale && lane_e < nv) ? a.damping_scale[env * nv + lane_e] : 1.f);
+      const float d_damping = KS_REC(m, lane_e, d_damping) * a.damping_scale[((a.given & kOptDamping) ? env : 0) * nv + (lane_e < nv ? lane_e : 0)];
       const float my_qvel = lane_e < nv ? l.qvel[lane_e] : 0.f;
       float qacc_int = qacc;
       if (mh.eulerdamp) {
@@ -1434,9 +1430,9 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
   m.dt = (float)d->dt;
   for (int k = 0; k < 3; ++k) m.gravity[k] = (float)d->gravity[k];
   m.tolerance = (float)d->tolerance; m.ls_tolerance = (float)d->ls_tolerance;
-  m.meaninertia = (float)d->meaninertia; m.friction = (float)d->friction; m.impratio = (float)d->impratio;
+  m.meaninertia = (float)d->meaninertia; m.friction = (float)d->friction; m.impratio_inv = (float)(1.0 / d->impratio);
   {  // solref / solimp -> (k, b) and clamped impedance parameters, for the contact rows and for the dof-lane rows
-    auto convert = [&](const double* solref, const double* solimp, float* out /*k b dmin dmax width mid power imp_a imp_b*/) {
+    auto convert = [&](const double* solref, const double* solimp, float* out /*k b dmin dmax 1/width mid power imp_a imp_b*/) {
       double timeconst = solref[0], dampratio = solref[1];
       double dmin = solimp[0], dmax = solimp[1], width = solimp[2], mid = solimp[3], power = solimp[4];
       if (timeconst < 2 * d->dt) timeconst = 2 * d->dt;
@@ -1446,18 +1442,18 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
       double k = 1.0 / (dmax * dmax * timeconst * timeconst * dampratio * dampratio), b = 2.0 / (dmax * timeconst);
       if (solref[0] <= 0) k = -solref[0] / (dmax * dmax);
       if (solref[1] <= 0) b = -solref[1] / dmax;
-      out[0] = (float)k; out[1] = (float)b; out[2] = (float)dmin; out[3] = (float)dmax; out[4] = (float)width;
+      out[0] = (float)k; out[1] = (float)b; out[2] = (float)dmin; out[3] = (float)dmax; out[4] = (float)(1.0 / width);
       out[5] = (float)mid; out[6] = (float)power;
       out[7] = (float)(1.0 / std::pow(mid, power - 1.0)); out[8] = (float)(1.0 / std::pow(1.0 - mid, power - 1.0));
     };
     float c[9];
     convert(d->solref, d->solimp, c);
-    m.con_k = c[0]; m.con_b = c[1]; m.dmin = c[2]; m.dmax = c[3]; m.width = c[4]; m.mid = c[5]; m.power = c[6]; m.imp_a = c[7]; m.imp_b = c[8];
+    m.con_k = c[0]; m.con_b = c[1]; m.dmin = c[2]; m.dmax = c[3]; m.width_inv = c[4]; m.mid = c[5]; m.power = c[6]; m.imp_a = c[7]; m.imp_b = c[8];
     bool own = false;
     for (int k = 0; k < 2; ++k) own |= d->dof_solref[k] != 0.0;
     for (int k = 0; k < 5; ++k) own |= d->dof_solimp[k] != 0.0;
     if (own) convert(d->dof_solref, d->dof_solimp, c);
-    m.dr_k = c[0]; m.dr_b = c[1]; m.dr_dmin = c[2]; m.dr_dmax = c[3]; m.dr_width = c[4]; m.dr_mid = c[5]; m.dr_power = c[6];
+    m.dr_k = c[0]; m.dr_b = c[1]; m.dr_dmin = c[2]; m.dr_dmax = c[3]; m.dr_width_inv = c[4]; m.dr_mid = c[5]; m.dr_power = c[6];
     m.dr_imp_a = c[7]; m.dr_imp_b = c[8];
   }
   for (int b = 0; b < d->nb; ++b) {
@@ -1540,11 +1536,12 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     m.body_dofmask[b] = mask;
   }
   for (int L = 0; L < 64; ++L) {
+    m.ones[L] = 1.f;
     LaneRec r;
     std::memset(&r, 0, sizeof(r));
     const bool is_body = L > 0 && L < d->nb;
     const int bl = is_body ? L : 0;
-    r.b_parent = m.body_parent[bl]; r.b_jtype = m.body_jtype[bl]; r.b_qadr = m.body_qadr[bl]; r.b_dofadr = m.body_dofadr[bl];
+    r.b_jtype = m.body_jtype[bl]; r.b_qadr = m.body_qadr[bl]; r.b_dofadr = m.body_dofadr[bl];
     r.b_depth = is_body ? m.body_depth[bl] : -1;
     for (int c = bl, k = r.b_depth - 1; c > 0; c = d->body_parent[c], --k) {
       const unsigned link = (unsigned)c | (unsigned)m.body_dofadr[c] << 5 | (m.body_jtype[c] == kJntHinge ? 1u << 10 : 0u) |
@@ -1554,7 +1551,7 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
     r.b_q0 = (is_body && r.b_jtype == kJntHinge) ? m.qpos0[r.b_qadr] : 0.f;
     r.b_mass = m.body_mass[bl];
     for (int k = 0; k < 3; ++k) {
-      r.b_pos[k] = m.body_pos[bl][k]; r.b_ipos[k] = m.body_ipos[bl][k]; r.b_inertia[k] = m.body_inertia[bl][k];
+      r.b_pos[k] = m.body_pos[bl][k];
       r.b_jaxis[k] = m.jnt_axis[bl][k]; r.b_jpos[k] = m.jnt_pos[bl][k];
     }
     for (int k = 0; k < 4; ++k) { r.b_quat[k] = m.body_quat[bl][k]; r.b_iquat[k] = m.body_iquat[bl][k]; }
@@ -1580,8 +1577,7 @@ extern "C" int ks_model_create(const KsModelDesc* d, KsModel** out) {
       r.d_frD = (float)(1.0 / std::max(d->dof_invweight0[dl] * (1.0 - imp0) / imp0, 1e-15));
     }
     const int sl = L < d->ns ? L : 0;
-    r.s_body = m.sph_body[sl]; r.s_rad = m.sph_radius[sl]; r.s_invw = m.body_invweight0[r.s_body];
-    for (int k = 0; k < 3; ++k) r.s_pos[k] = m.sph_pos[sl][k];
+    r.s_body = m.sph_body[sl]; r.s_invw = m.body_invweight0[r.s_body];
     r.s_mask = m.body_dofmask[r.s_body];
     for (int k = 0; k < kPairSets; ++k) {
       const int p = L + 64 * k;
@@ -1674,6 +1670,18 @@ static int launch_step(const KsModel* km, ks_stream_t stream, const KsStepIO* io
       a.event_state = io->event_state; a.event_uniform = io->event_uniform; a.event_rng = io->event_rng;
     }
   }
+  // stand-ins for the operands that were not given
+  const DevModel* dm = km->dev;
+  auto stand_in = [&](const float*& p, unsigned bit, const float* other) { if (p) a.given |= bit; else p = other; };
+  stand_in(a.mass_scale, kOptMass, dm->ones); stand_in(a.damping_scale, kOptDamping, dm->ones); stand_in(a.armature_scale, kOptArmature, dm->ones);
+  stand_in(a.body_ipos, kOptIpos, &dm->body_ipos[0][0]); stand_in(a.body_inertia, kOptInertia, &dm->body_inertia[0][0]);
+  stand_in(a.sph_pos, kOptSphere, &dm->sph_pos[0][0]); stand_in(a.sph_radius, kOptSphere, dm->sph_radius);
+  stand_in(a.kp_scale, kOptKp, dm->ones); stand_in(a.kd_scale, kOptKd, dm->ones); stand_in(a.torque_limit_scale, kOptLimit, dm->ones);
+  stand_in(a.zero_offset, kOptZero, dm->zeros); stand_in(a.action_bias, kOptActionBias, dm->zeros);
+  stand_in(a.torque_bias, kOptTorqueBias, dm->zeros); stand_in(a.action_noise, kOptActionNoise, dm->zeros);
+  stand_in(a.torque_noise, kOptTorqueNoise, dm->zeros);
+  stand_in(a.kp, 0u, dm->zeros); stand_in(a.kd, 0u, dm->zeros); stand_in(a.ctrl_clip, 0u, dm->zeros);  // torque actuators
+  if (a.drop) a.given |= kOptDrop; else a.drop = reinterpret_cast<const uint8_t*>(dm->zeros);
   const int bytes = lds_floats(m.nb, m.nq, m.nv, m.nu, m.ns) * 4;
   if (bytes > 160 * 1024) return fail(KS_ELIMIT, "ks_step: model needs %d bytes of LDS", bytes);
   void (*fn)(StepArgs) = nullptr;

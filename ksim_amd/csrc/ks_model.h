@@ -24,12 +24,12 @@ struct ModelHead {
       dofrows /* 1 when a joint is limited or has dry friction */, nfriction /* dofs with dry friction */,
       invw_ok /* 1 when every hinge dof has a positive inverse weight (what rows on the dof lanes are regularised with) */,
       frictionless /* 1: condim 1, one normal row per contact instead of the four pyramid edges */;
-  float dt, gravity[3], tolerance, ls_tolerance, meaninertia, friction, impratio;
+  float dt, gravity[3], tolerance, ls_tolerance, meaninertia, friction, impratio_inv;
   // contact impedance constants, already clamped the way the constraint builder wants them
-  float con_k, con_b, dmin, dmax, width, mid, power;
+  float con_k, con_b, dmin, dmax, width_inv, mid, power;
   float imp_a, imp_b;  // 1 / mid^(power-1) and 1 / (1-mid)^(power-1), the constant factors of the impedance curve
   // the same constants for the rows of joint limits and dry friction
-  float dr_k, dr_b, dr_dmin, dr_dmax, dr_width, dr_mid, dr_power, dr_imp_a, dr_imp_b;
+  float dr_k, dr_b, dr_dmin, dr_dmax, dr_width_inv, dr_mid, dr_power, dr_imp_a, dr_imp_b;
 };
 
 // Immutable after ks_model_create(); lives in device global memory and is read through the
@@ -48,11 +48,13 @@ struct DevModel : ModelHead {
   int sph_body[kMaxS];
   float sph_pos[kMaxS][3], sph_radius[kMaxS];
   short pair_i[kMaxPairs], pair_j[kMaxPairs];  // (i, j): j is an ancestor dof of i
-  // What lane L reads at the top of every substep: its 72-dword record (layout: LaneRec in ks_dynamics.hip) in eighteen
+  // What an optional operand that was not given reads instead: a scale of one, an offset of zero.
+  float ones[64], zeros[64];
+  // What lane L reads at the top of every substep: its 64-dword record (layout: LaneRec in ks_dynamics.hip) in sixteen
   // pieces of 16 bytes, the same piece of all lanes side by side, so that a load of the wavefront covers eight cache lines.
   // (Record after record, every load touched 64 lines, and the sixteen wavefronts of a CU queued for its vector L1: with the
   // actuator law that phase took 83 K of 463 K cycles per control step at 4096 envs, 41 K now.)
-  alignas(16) unsigned lane_rec[18][64][4];
+  alignas(16) unsigned lane_rec[16][64][4];
 };
 
 // ---------------------------------------------------------------- wavefront reductions (DPP, no LDS)

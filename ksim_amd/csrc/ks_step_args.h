@@ -7,9 +7,19 @@
 
 namespace ks {
 
+// Operands that a call may leave out.  Their pointers are never null in the kernel: what is not given points at ones, zeros or the
+// model's own values, and its bit in StepArgs::given is clear, which takes the env out of the index.  The loads of a substep are then
+// straight-line code with one latency between them, where a branch around each was a round trip of its own.
+enum StepOptional : unsigned {
+  kOptMass = 1u << 0, kOptDamping = 1u << 1, kOptArmature = 1u << 2, kOptIpos = 1u << 3, kOptInertia = 1u << 4, kOptSphere = 1u << 5,
+  kOptKp = 1u << 6, kOptKd = 1u << 7, kOptLimit = 1u << 8, kOptZero = 1u << 9, kOptDrop = 1u << 10, kOptActionBias = 1u << 11,
+  kOptTorqueBias = 1u << 12, kOptActionNoise = 1u << 13, kOptTorqueNoise = 1u << 14,
+};
+
 struct StepArgs {
   const DevModel* model;
   ModelHead head;
+  unsigned given;
   int64_t N;
   int substeps, actuator_period, actuator_type;
   float action_scale;
