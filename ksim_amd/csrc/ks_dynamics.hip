@@ -339,17 +339,6 @@ struct LsBits {  // a point of the search: step length, cost, slope, Newton esti
   int alpha, cost, d0, next;
 };
 
-// the slope y lies strictly between the slope x and zero (x, y are no NaN)
-__device__ __forceinline__ bool closer(int x, int y) {
-  const unsigned mx = (unsigned)x & 0x7fffffffu, my = (unsigned)y & 0x7fffffffu;
-  return ((x ^ y) >= 0) & (mx > my) & (my != 0u);
-}
-
-__device__ __forceinline__ void take_if(LsBits& a, bool c, const LsBits& b) {  // field by field: the points stay in scalar registers
-  a.alpha = c ? b.alpha : a.alpha; a.cost = c ? b.cost : a.cost;
-  a.d0 = c ? b.d0 : a.d0; a.next = c ? b.next : a.next;
-}
-
 __device__ __forceinline__ float bits_f(int b) { return __builtin_bit_cast(float, b); }
 __device__ __forceinline__ int lane_bits(float x, int lane) { return __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane); }
 
@@ -365,8 +354,9 @@ __device__ __forceinline__ float line_search_rows(int iterations, int nefc, int 
     const float D2 = __shfl(D, 16 + r);
     b0 = 0.5f * j2 * j2 * D2; b1 = v2 * j2 * D2; b2 = 0.5f * v2 * v2 * D2;
   }
-  auto eval = [&](float s0, float s1, float s2, LsBits& pa, LsBits& pb, LsBits& pc) {
-    const float al = grp == 0 ? s0 : (grp == 1 ? s1 : s2);
+  float al, cost, slope, next;  // of the lane's group, in its lane 15
+  auto eval = [&](float step) {
+    al = step;
     const bool on1 = j1 + al * v1 < 0.f;  // rows beyond nefc carry zeros
     float x0 = on1 ? a0 : 0.f, x1 = on1 ? a1 : 0.f, x2 = on1 ? a2 : 0.f;
     if (two) {
@@ -379,36 +369,36 @@ __device__ __forceinline__ float line_search_rows(int iterations, int nefc, int 
     x0 += dpp_shift<0x118, 0xf>(x0); x1 += dpp_shift<0x118, 0xf>(x1); x2 += dpp_shift<0x118, 0xf>(x2);
     // lane 15 of each group holds the group's totals; the other lanes carry numbers nobody reads
     const float q0 = g0 + x0, q1 = g1 + x1, q2 = g2 + x2;
-    const float cost = al * al * q2 + al * q1 + q0;
+    cost = al * al * q2 + al * q1 + q0;
     const float d0 = 2.f * al * q2 + q1, d1 = 2.f * q2 + (q2 == 0.f ? 1e-15f : 0.f);
     // Newton estimate of the step length: d0 / d1 by reciprocal and product (1 ulp), a tenth of a division's instructions
-    const float next = al - d0 * __builtin_amdgcn_rcpf(d1);
-    const float slope = d0 == d0 ? d0 : 0.f;  // a NaN takes part in no bracket
-    pa = {lane_bits(al, 15), lane_bits(cost, 15), lane_bits(slope, 15), lane_bits(next, 15)};
-    pb = {lane_bits(al, 31), lane_bits(cost, 31), lane_bits(slope, 31), lane_bits(next, 31)};
-    pc = {lane_bits(al, 47), lane_bits(cost, 47), lane_bits(slope, 47), lane_bits(next, 47)};
+    next = al - d0 * __builtin_amdgcn_rcpf(d1);
+    slope = d0 == d0 ? d0 : 0.f;  // a NaN takes part in no bracket
   };
-  LsBits p0, lo, hi, pa, pb, pm;
-  eval(0.f, 0.f, 0.f, p0, pb, pm);
-  eval(bits_f(p0.next), bits_f(p0.next), bits_f(p0.next), lo, pb, pm);
-  const bool below = bits_f(lo.d0) < bits_f(p0.d0);
-  hi = lo;
-  take_if(hi, below, p0);
-  take_if(lo, !below, p0);
+  auto fetch = [&](LsBits& p, int at) { p = {lane_bits(al, at), lane_bits(cost, at), lane_bits(slope, at), lane_bits(next, at)}; };
+  LsBits p0, lo, hi;
+  eval(0.f);
+  fetch(p0, 15);
+  eval(bits_f(p0.next));
+  if (bits_f(lane_bits(slope, 15)) < bits_f(p0.d0)) { fetch(lo, 15); hi = p0; } else { fetch(hi, 15); lo = p0; }
   const unsigned tol = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fmaxf(gtol, 0.f)));  // bits of a number >= 0 order like the number
-  bool swap = true;
-  for (int it = 0; it < iterations && swap; ++it) {
-    const unsigned ml = (unsigned)lo.d0 & 0x7fffffffu, mh = (unsigned)hi.d0;
+  for (int it = 0; it < iterations; ++it) {
+    const unsigned ml = (unsigned)lo.d0 & 0x7fffffffu, mh = (unsigned)hi.d0 & 0x7fffffffu;
     if ((lo.d0 < 0) & (ml != 0u) & (ml < tol)) break;  // the slope at lo is negative and within the tolerance
     if ((hi.d0 > 0) & (mh < tol)) break;               // that at hi positive and within it
-    eval(bits_f(lo.next), bits_f(hi.next), 0.5f * (bits_f(lo.alpha) + bits_f(hi.alpha)), pa, pb, pm);
-    const bool s1 = closer(lo.d0, pa.d0); take_if(lo, s1, pa);
-    const bool s2 = closer(lo.d0, pm.d0); take_if(lo, s2, pm);
-    const bool s3 = closer(lo.d0, pb.d0); take_if(lo, s3, pb);
-    const bool t1 = closer(hi.d0, pb.d0); take_if(hi, t1, pb);
-    const bool t2 = closer(hi.d0, pm.d0); take_if(hi, t2, pm);
-    const bool t3 = closer(hi.d0, pa.d0); take_if(hi, t3, pa);
-    swap = s1 | s2 | s3 | t1 | t2 | t3;
+    eval(grp == 0 ? bits_f(lo.next) : (grp == 1 ? bits_f(hi.next) : 0.5f * (bits_f(lo.alpha) + bits_f(hi.alpha))));
+    const int s0 = lane_bits(slope, 15), s1 = lane_bits(slope, 31), s2 = lane_bits(slope, 47);
+    // Each end of the bracket moves to the candidate whose slope has its sign and is the nearest to zero, if one is nearer than its
+    // own (and not zero).  Magnitude - 1 as an unsigned number puts a zero slope last; a tie goes to the candidate asked first.
+    const unsigned m0 = ((unsigned)s0 & 0x7fffffffu) - 1u, m1 = ((unsigned)s1 & 0x7fffffffu) - 1u, m2 = ((unsigned)s2 & 0x7fffffffu) - 1u;
+    const unsigned own_l = ml ? ml - 1u : 0u, own_h = mh ? mh - 1u : 0u;
+    const unsigned l0 = (s0 ^ lo.d0) < 0 ? ~0u : m0, l1 = (s1 ^ lo.d0) < 0 ? ~0u : m1, l2 = (s2 ^ lo.d0) < 0 ? ~0u : m2;
+    const unsigned h0 = (s0 ^ hi.d0) < 0 ? ~0u : m0, h1 = (s1 ^ hi.d0) < 0 ? ~0u : m1, h2 = (s2 ^ hi.d0) < 0 ? ~0u : m2;
+    const unsigned bl = min(l0, min(l1, l2)), bh = min(h0, min(h1, h2));
+    const bool move_l = bl < own_l, move_h = bh < own_h;
+    if (!(move_l | move_h)) break;
+    if (move_l) fetch(lo, bl == l0 ? 15 : (bl == l2 ? 47 : 31));  // asked in the order lo's estimate, middle, hi's estimate
+    if (move_h) fetch(hi, bh == h1 ? 31 : (bh == h2 ? 47 : 15));  // hi's estimate, middle, lo's
   }
   const float cl = bits_f(lo.cost), ch = bits_f(hi.cost), c0 = bits_f(p0.cost);
   const bool improved = (cl < c0) || (ch < c0);
