@@ -174,16 +174,31 @@ __device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myin
 }
 
 // Mass matrix (LDS, NP rows: beyond nv unit rows and zero columns) into the accumulator layout.  What the tile holds outside
-// NP x NP is a copy of entries inside it: the factorisation writes there, but never reads.
+// NP x NP is a copy of entries inside it, which the factorisation writes but never reads, except that column 31 is the right-hand
+// side `rhs` (32 floats in LDS) where the matrix leaves room for it (chol_solve).
 template <int NP>
-__device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ M, int lane) {
-  const int c = min(lane & 31, NP - 1), half = lane >> 5;
-  const float* row = M + c * stride_of(NP);
+__device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ M, const float* __restrict__ rhs, int lane) {
+  const int c = lane & 31, half = lane >> 5;
+  const float* row = M + min(c, NP - 1) * stride_of(NP);
+  if (NP < 32) row = c == 31 ? rhs : row;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const float4 v = *reinterpret_cast<const float4*>(row + min(8 * g + 4 * half, NP - 4));
     T[4 * g] = v.x; T[4 * g + 1] = v.y; T[4 * g + 2] = v.z; T[4 * g + 3] = v.w;
   }
+}
+
+// L^T x = y, lane i holding r_i = y_i * L[i][i] and returning x_i
+template <int NP>
+__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, int lane, float r, int nv) {
+  const float myinv2 = myinv * myinv;
+#pragma unroll
+  for (int k = NP - 1; k >= 0; --k) {  // in the scaled form  sum_{k>i} R[k] x_k + L[i][i]^2 x_i = r_i
+    if (k >= padded_from(NP) && k >= nv) continue;  // padded unknowns are zero and couple to nothing
+    const float xk = lane_bcast(r * myinv2, k);
+    r = lane < k ? r - R[k] * xk : r;
+  }
+  return r * myinv2;
 }
 
 // x = (L L^T)^-1 b, lane i holding b_i and returning x_i
@@ -197,14 +212,31 @@ __device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, i
     const float yj = lane_bcast(r * myinv, j);
     r = lane > j ? r - R[j] * yj : r;
   }
-  const float myinv2 = myinv * myinv;
+  return back_substitute<NP>(R, myinv, lane, r, nv);
+}
+
+// Factors the tile and returns x = (L L^T)^-1 b, lane i holding b_i (zero beyond nv).  A matrix of fewer than 32 columns carries b
+// along as column 31 of its tile (load_mtile): the rank-1 updates of the factorisation then are the forward substitution too, and what
+// is left of it is to hand y = L^-1 b, which the two lanes of that column hold, to the lanes of its rows, through LDS (`vbuf`, 32
+// floats).  A substitution step is four instructions of a chain, 26 of them for 26 dofs.
+template <int NP>
+__device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& myinv, int lane, float b, int nv, float* vbuf) {
+  chol_tile<NP>(T, R, myinv, lane, nv);
+  if constexpr (NP == 32) {
+    return solve_regs<NP>(R, myinv, lane, b, nv);
+  } else {
+    asm volatile("" : "+v"(lane));
+    KS_SYNC();
+    if ((lane & 31) == 31) {
+      float4* dst = reinterpret_cast<float4*>(vbuf) + (lane >> 5);
 #pragma unroll
-  for (int k = NP - 1; k >= 0; --k) {  // L^T x = y in the scaled form  sum_{k>i} R[k] x_k + L[i][i]^2 x_i = r_i
-    if (k >= padded_from(NP) && k >= nv) continue;
-    const float xk = lane_bcast(r * myinv2, k);
-    r = lane < k ? r - R[k] * xk : r;
+      for (int g = 0; g < 4; ++g) dst[2 * g] = {T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]};
+    }
+    KS_SYNC();
+    const float y = vbuf[lane & 31];
+    KS_SYNC();
+    return back_substitute<NP>(R, myinv, lane, y * __builtin_amdgcn_rcpf(myinv), nv);
   }
-  return r * myinv2;
 }
 
 // dot product of an LDS row (per-lane address, 16-byte aligned) with a broadcast register vector
@@ -932,13 +964,14 @@ void step_kernel(StepArgs a) {
     KS_PHASE(6)
     // ---- Cholesky of M and the unconstrained acceleration (registers only)
     float R[NP];
-    float myinv;
+    float myinv, qas_all;
     {
       f32x16 T;
-      load_mtile<NP>(T, l.M, lane);
-      chol_tile<NP>(T, R, myinv, lane, nv);
+      if (lane < 32) l.vbuf[lane] = qfs;
+      KS_SYNC();
+      load_mtile<NP>(T, l.M, l.vbuf, lane);
+      qas_all = chol_solve<NP>(T, R, myinv, lane, qfs, nv, l.vbuf);
     }
-    const float qas_all = solve_regs<NP>(R, myinv, lane, qfs, nv);
     const float qas = is_dof ? qas_all : 0.f;  // lanes that hold no row carry meaningless numbers
     if (a.dbg_qacc_smooth && is_dof) a.dbg_qacc_smooth[env * nv + lane] = qas;
 
@@ -1108,11 +1141,13 @@ void step_kernel(StepArgs a) {
         // lane i < 32 ends up with row i of H in registers, as the factorisation wants it.
         // H depends on the iterate only through the active set: while that stays the same (the usual case once the
         // solver closes in) the factor of the previous iteration is still the factor of H and is kept.
+        float step_all;
         if (!have_factor || am != am_factored || (DR && amd != amd_factored)) {
           l.drow[lane] = active ? D : 0.f;
+          if (lane < 32) l.vbuf[lane] = grad;
           KS_SYNC();
           f32x16 hc;
-          load_mtile<NP>(hc, l.M, lane);
+          load_mtile<NP>(hc, l.M, l.vbuf, lane);
           const int col = lane & 31, half = lane >> 5;
           const bool col_ok = NP == 32 || col < NP;
           // the operands of four products at a time are fetched before the first of them (a row past the last counts as zero)
@@ -1139,13 +1174,14 @@ void step_kernel(StepArgs a) {
               for (int e = 0; e < 4; ++e) hc[4 * g + e] += (8 * g + 4 * half + e == col) ? hd : 0.f;
           }
           KS_PHASE(11)
-          chol_tile<NP>(hc, R, myinv, lane, nv);
+          step_all = chol_solve<NP>(hc, R, myinv, lane, grad, nv, l.vbuf);
           am_factored = am;
           amd_factored = amd;
           have_factor = true;
+        } else {
+          step_all = solve_regs<NP>(R, myinv, lane, grad, nv);
         }
-        const float search_all = -solve_regs<NP>(R, myinv, lane, grad, nv);
-        const float search = is_dof ? search_all : 0.f;
+        const float search = is_dof ? -step_all : 0.f;
         KS_PHASE(12)
         // ---- exact line search along `search`
         float mv = 0.f, jv = 0.f;
@@ -1324,17 +1360,19 @@ void step_kernel(StepArgs a) {
         // implicit in the joint damping: (M + dt diag(damping)) a = M qacc.  For torque motors, whose force does
         // not depend on velocity, this is MuJoCo's implicitfast step; qacc itself (warm start, output) is unchanged.
         f32x16 T;
-        load_mtile<NP>(T, l.M, lane);
+        const float b = is_dof ? Mqacc : 0.f;
+        if (lane < 32) l.vbuf[lane] = b;
+        KS_SYNC();
+        load_mtile<NP>(T, l.M, l.vbuf, lane);
         const int c = lane & 31, half = lane >> 5;
         const float hd = mh.dt * __shfl(is_dof ? d_damping : 0.f, c);
 #pragma unroll
         for (int g = 0; g < 4; ++g)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) T[4 * g + e] += (8 * g + 4 * half + e == c) ? hd : 0.f;
+          for (int e = 0; e < 4; ++e) T[4 * g + e] += (8 * g + 4 * half + e == c) ? hd : 0.f;  // lanes of column 31: dof 31 or none
         float R2[NP];
         float inv2;
-        chol_tile<NP>(T, R2, inv2, lane, nv);
-        const float sol = solve_regs<NP>(R2, inv2, lane, is_dof ? Mqacc : 0.f, nv);
+        const float sol = chol_solve<NP>(T, R2, inv2, lane, b, nv, l.vbuf);
         qacc_int = is_dof ? sol : 0.f;
       }
       if (is_dof) l.qvel[lane] = my_qvel + mh.dt * qacc_int;
