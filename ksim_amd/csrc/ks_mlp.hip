@@ -1038,6 +1038,168 @@ void mlp_fused_pair_kernel(const FusedArgs a, const FusedArgs b) {
   else mlp_fused_body<ACT, T, BM>(b, tile);
 }
 
+// ---------------------------------------------------------------- few rows through a wide bf16 network
+// Over a few row tiles the whole-network kernel is bound by how fast a CU takes in weights (66 GB/s whatever is in flight: 1.1 MB of a
+// 3 x 512 network are 16 us), so here the 32-wide output tiles of a layer go to as many CUs.  A layer needs the whole of the one before
+// it, which is a launch boundary, 3 to 4 us; the first launch makes up for its own by taking the first layer, whose weights are few,
+// in every workgroup, and the last hidden layer's launch also runs the output layer in the workgroup that arrives last at a row tile.
+// Per output the sums are the whole-network kernel's in the same order, so the results do not depend on the path.
+//   68-512-512-512-20: one row 17.6 -> 12.4 us, 256 rows 17.8 -> 13.8; as one of a pair, 64 rows 17.9 -> 12.6
+constexpr int kSplitTile = 2 * (kFusedMaxWidth / 32) * 64;  // 16-byte fragments of a 32-row tile of activations: [k step][lane]
+
+// What a launch needs of a network, resolved on the host: the arguments are a scalar load away, and one that depends on another is two.
+struct SplitFirst {
+  const float* x;
+  const u32x4 *w0, *w1;
+  const float *b0, *b1;
+  u32x4* h;           // activations of every row tile for the next launch, in the order of the matrix operand
+  unsigned* arrived;  // per row tile: zeroed here, counted by the last hidden layer's launch
+  int M, in_dim, lda, nk0, nt0, nk1, nt1;
+};
+struct SplitLayer {
+  const u32x4 *h, *w;
+  const float* b;
+  u32x4* h_out;  // null: this is the output layer
+  const u32x4* wo;  // the output layer, where it follows in this launch, else null
+  const float* bo;
+  float* y;
+  unsigned* arrived;
+  int M, out_dim, nk, nt, nko, nto;
+};
+
+__device__ __forceinline__ void device_store8(void* p, uint2 v) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u32x4 device_load16(const u32x4* p) {
+  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(p);
+  const uint2 lo = __builtin_bit_cast(uint2, __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  const uint2 hi = __builtin_bit_cast(uint2, __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  return u32x4{lo.x, lo.y, hi.x, hi.y};
+}
+
+// A finished tile j of 32 features, activated and rounded, as fragments of the next layer's operand.  ACROSS: written past this XCD's L2, for
+// a reader inside this launch.
+template <int ACT, bool ACROSS>
+__device__ __forceinline__ void split_store(const f32x16& acc, u32x4* __restrict__ h, int j, int lane) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const uint2 v = {pack_bf16(activate<ACT, true>(acc[4 * g]), activate<ACT, true>(acc[4 * g + 1])),
+                     pack_bf16(activate<ACT, true>(acc[4 * g + 2]), activate<ACT, true>(acc[4 * g + 3]))};
+    uint2* to = reinterpret_cast<uint2*>(h + (2 * j + (g >> 1)) * 64 + (lane & 31) + 32 * (g & 1)) + (lane >> 5);
+    if (ACROSS) device_store8(to, v);
+    else *to = v;
+  }
+}
+
+constexpr int kSplitSteps = kFusedMaxWidth / 16;  // K steps of the widest layer
+
+__device__ __forceinline__ void split_fetch(u32x4 (&f)[kSplitSteps], const u32x4* __restrict__ src, int nk, int lane) {
+#pragma unroll
+  for (int u = 0; u < kSplitSteps; ++u) f[u] = src[min(u, nk - 1) * 64 + lane];
+}
+
+// 32 rows of the network input, rounded, to the tile: sixteen threads a row, eight values (zero beyond the batch and the row) each and pass
+__device__ __forceinline__ void split_stage_input(const SplitFirst& s, __bf16* __restrict__ act, int64_t m0, int tid) {
+  const int row = tid >> 4;
+  const bool in = m0 + row < s.M;
+  const float* src = s.x + (m0 + (in ? row : 0)) * s.in_dim;
+  for (int c = (tid & 15) * 8; c < s.nk0 * 16; c += 128) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = src[min(c + e, s.in_dim - 1)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = in && c + e < s.in_dim ? v[e] : 0.f;
+    *reinterpret_cast<u32x4*>(act + row * s.lda + c) = u32x4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+  }
+}
+
+template <int ACT>
+__device__ __forceinline__ void split_first_body(const SplitFirst& s) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char mlp_lds[];
+  __bf16* act = reinterpret_cast<__bf16*>(mlp_lds);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = blockIdx.x;
+  const int64_t tile = blockIdx.y, m0 = tile * 32;
+  if (j >= s.nt1) return;  // the other network of the launch is wider
+  const int j0 = min(wave, s.nt0 - 1), j1 = min(wave + kFusedWaves, s.nt0 - 1);
+  const u32x4 *w0 = s.w0 + (int64_t)j0 * s.nk0 * 64 + lane, *w1 = s.w0 + (int64_t)j1 * s.nk0 * 64 + lane;
+  f32x16 acc0[2][1];
+  fused_bias_init(acc0[0][0], s.b0, j0, lane);
+  fused_bias_init(acc0[1][0], s.b0, j1, lane);
+  split_stage_input(s, act, m0, tid);
+  u32x4 w[kSplitSteps];  // this workgroup's tile of the second layer, on its way during the first
+  if (wave == 0) split_fetch(w, s.w1 + (int64_t)j * s.nk1 * 64, s.nk1, lane);
+  __syncthreads();
+  const __bf16* arow = act + (lane & 31) * s.lda + (lane >> 5) * 8;
+  fused_layer_mma<__bf16, 2, 1, kPF>(acc0, w0, w1, s.nk0, arow, s.lda);
+  __syncthreads();  // every wavefront has read the input; the tile takes the first layer's output
+  if (wave < s.nt0) fused_store_hidden<ACT, __bf16>(acc0[0][0], act, s.lda, j0, lane & 31, lane);
+  if (wave + kFusedWaves < s.nt0) fused_store_hidden<ACT, __bf16>(acc0[1][0], act, s.lda, j1, lane & 31, lane);
+  __syncthreads();
+  if (wave != 0) return;
+  if (j == 0 && lane == 0) s.arrived[tile] = 0;
+  f32x16 acc;
+  fused_bias_init(acc, s.b1, j, lane);
+#pragma unroll
+  for (int u = 0; u < kSplitSteps; ++u)
+    if (u < s.nk1) acc = fused_mma<__bf16>(w[u], *reinterpret_cast<const u32x4*>(arow + u * 16), acc);
+  split_store<ACT, false>(acc, s.h + tile * kSplitTile, j, lane);
+}
+
+// The first two layers: workgroup (j, tile, network) computes output tile j of the second one.
+template <int ACT>
+__global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void mlp_split_first_kernel(const SplitFirst p, const SplitFirst q) {
+  if (blockIdx.z == 0) split_first_body<ACT>(p);
+  else split_first_body<ACT>(q);
+}
+
+template <int ACT>
+__device__ __forceinline__ void split_layer_body(const SplitLayer& s) {
+  const int lane = threadIdx.x, j = blockIdx.x;
+  const int64_t tile = blockIdx.y, m = tile * 32 + (lane & 31);
+  if (j >= s.nt) return;
+  u32x4 w[kSplitSteps], x[kSplitSteps];
+  split_fetch(w, s.w + (int64_t)j * s.nk * 64, s.nk, lane);
+  split_fetch(x, s.h + tile * kSplitTile, s.nk, lane);
+  f32x16 acc;
+  fused_bias_init(acc, s.b, j, lane);
+#pragma unroll
+  for (int u = 0; u < kSplitSteps; ++u)
+    if (u < s.nk) acc = fused_mma<__bf16>(w[u], x[u], acc);
+  if (!s.h_out) {
+    fused_store_output(acc, s.y, s.M, s.out_dim, j, m, lane);
+    return;
+  }
+  u32x4* h = s.h_out + tile * kSplitTile;
+  if (!s.wo) {
+    split_store<ACT, false>(acc, h, j, lane);
+    return;
+  }
+  split_store<ACT, true>(acc, h, j, lane);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this tile has reached memory
+  unsigned before = 0;
+  if (lane == 0) before = atomicAdd(s.arrived + tile, 1u);
+  if (__builtin_amdgcn_readfirstlane(before) != (unsigned)s.nt - 1u) return;
+#pragma unroll
+  for (int u = 0; u < kSplitSteps; ++u) x[u] = device_load16(h + min(u, s.nko - 1) * 64 + lane);
+  for (int t = 0; t < s.nto; ++t) {
+    split_fetch(w, s.wo + (int64_t)t * s.nko * 64, s.nko, lane);
+    fused_bias_init(acc, s.bo, t, lane);
+#pragma unroll
+    for (int u = 0; u < kSplitSteps; ++u)
+      if (u < s.nko) acc = fused_mma<__bf16>(w[u], x[u], acc);
+    fused_store_output(acc, s.y, s.M, s.out_dim, t, m, lane);
+  }
+}
+
+// A later layer, a wavefront per output tile; the last hidden layer's launch ends with the output layer.
+template <int ACT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void mlp_split_layer_kernel(const SplitLayer p, const SplitLayer q) {
+  if (blockIdx.z == 0) split_layer_body<ACT>(p);
+  else split_layer_body<ACT>(q);
+}
+
 // ---------------------------------------------------------------- whole-network backward pass of the hidden layers
 // dZ_{l-1} = (dZ_l W_l) * f'(Y_{l-1}) for l = L-1 .. 1 in one launch, a 128-row tile per workgroup that never leaves LDS: the
 // product is the forward kernel's K loop over the fragment-ordered transposed weights, its epilogue reads f'(Y) from the
@@ -1963,6 +2125,68 @@ static int launch_small(const DevMlp& a, const DevMlp* b, hipStream_t s, int64_t
   return check_launch("ks_mlp_forward");
 }
 
+// Whether M rows of a bf16 network go through the layer-wise kernels for few rows.  The hidden layers have to be wide enough for their
+// weights to be worth the second launch (one row of 68-3 x 384-20: 13.9 -> 11.7 us, 68-2 x 384-20: 9.9 -> 9.0, 3 x 352: 13.1
+// -> 12.4, 3 x 288: 11.1 -> 11.4, a layer of 320 columns being 10 tiles), and every row tile repeats the first layer in every workgroup,
+// which past 256 rows costs a pair of networks more than it gains (512 rows: 17.9 -> 23).
+constexpr int64_t kSplitRows = 256;
+constexpr int kSplitTiles = 12;
+static bool split_ok(const DevMlp& m, int64_t M) {
+  if (m.dtype != KS_MLP_BF16 || !m.fused || m.n_layers < 3 || m.fn[m.n_layers - 1] > 2) return false;
+  for (int l = 0; l + 1 < m.n_layers; ++l)
+    if (m.fn[l] < kSplitTiles) return false;
+  return M <= kSplitRows;
+}
+
+static int64_t split_ws_bytes(int64_t M) {
+  const int64_t tiles = (M + 31) / 32;
+  return tiles * (2 * kSplitTile * 16 + 4) + 256;
+}
+
+// where the launches of a call keep their activations: two buffers, then the counters
+static u32x4* split_buffer(void* ws, int64_t M, int k) {
+  return reinterpret_cast<u32x4*>(((uintptr_t)ws + 15) & ~(uintptr_t)15) + k * ((M + 31) / 32) * kSplitTile;
+}
+
+static SplitFirst split_first(const DevMlp& m, int64_t M, const float* x, void* ws) {
+  return {x, (const u32x4*)m.Wp[0], (const u32x4*)m.Wp[1], m.bp[0], m.bp[1], split_buffer(ws, M, 0), reinterpret_cast<unsigned*>(split_buffer(ws, M, 2)),
+          (int)M, m.dims[0], m.lda, m.fk[0], m.fn[0], m.fk[1], m.fn[1]};
+}
+
+static SplitLayer split_layer(const DevMlp& m, int64_t M, int l, float* y, void* ws) {
+  const int out = m.n_layers - 1;
+  const bool ends = l + 1 == out;
+  return {split_buffer(ws, M, l & 1), (const u32x4*)m.Wp[l], m.bp[l], l == out ? nullptr : split_buffer(ws, M, (l & 1) ^ 1),
+          ends ? (const u32x4*)m.Wp[out] : nullptr, m.bp[out], y, reinterpret_cast<unsigned*>(split_buffer(ws, M, 2)),
+          (int)M, m.dims[m.n_layers], m.fk[l], m.fn[l], m.fk[out], m.fn[out]};
+}
+
+// one network, or two of the same depth and activation over the same number of rows
+static int launch_split(const DevMlp& a, const DevMlp* b, hipStream_t s, int64_t M, const float* xa, float* ya, void* wa, const float* xb,
+                        float* yb, void* wb) {
+  const SplitFirst p = split_first(a, M, xa, wa), q = b ? split_first(*b, M, xb, wb) : p;
+  const unsigned tiles = (unsigned)((M + 31) / 32), nets = b ? 2 : 1;
+  auto wide = [&](int l) { return (unsigned)(b && b->fn[l] > a.fn[l] ? b->fn[l] : a.fn[l]); };
+  const int lds = 32 * (b && b->lda > a.lda ? b->lda : a.lda) * 2;
+#define KS_LAUNCH(A)                                                                                                                     \
+  {                                                                                                                                      \
+    hipLaunchKernelGGL(mlp_split_first_kernel<A>, dim3(wide(1), tiles, nets), dim3(64 * kFusedWaves), lds, s, p, q);                     \
+    for (int l = 2; l == 2 || l + 1 < a.n_layers; ++l) {                                                                                 \
+      const SplitLayer u = split_layer(a, M, l, ya, wa), v = b ? split_layer(*b, M, l, yb, wb) : u;                                      \
+      hipLaunchKernelGGL(mlp_split_layer_kernel<A>, dim3(wide(l), tiles, nets), dim3(64), 0, s, u, v);                                   \
+    }                                                                                                                                    \
+  }
+  switch (a.activation) {
+    case KS_ACT_ELU: KS_LAUNCH(KS_ACT_ELU) break;
+    case KS_ACT_RELU: KS_LAUNCH(KS_ACT_RELU) break;
+    case KS_ACT_TANH: KS_LAUNCH(KS_ACT_TANH) break;
+    case KS_ACT_GELU: KS_LAUNCH(KS_ACT_GELU) break;
+    default: KS_LAUNCH(KS_ACT_NONE) break;
+  }
+#undef KS_LAUNCH
+  return check_launch("ks_mlp_forward");
+}
+
 extern "C" int ks_mlp_forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t stream, int64_t M, const float* x0,
                                    float* y0, const float* x1, float* y1, void* workspace0, void* workspace1) {
   if (!h0 || !h1) return fail(KS_EINVAL, "ks_mlp_forward_pair: null handle");
@@ -1974,6 +2198,9 @@ extern "C" int ks_mlp_forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t
   if (small_ok(h0->m, M) && small_ok(h1->m, M) && h0->m.n_layers == h1->m.n_layers && h0->m.n_layers > 1 && workspace0 && workspace1 &&
       workspace0 != workspace1)
     return launch_small(h0->m, &h1->m, s, M, x0, y0, workspace0, x1, y1, workspace1);
+  if (split_ok(h0->m, M) && split_ok(h1->m, M) && h0->m.n_layers == h1->m.n_layers && h0->m.activation == h1->m.activation && workspace0 &&
+      workspace1 && workspace0 != workspace1)
+    return launch_split(h0->m, &h1->m, s, M, x0, y0, workspace0, x1, y1, workspace1);
   // one launch when both networks run as whole-network kernels with the same activation and row tile; else one each
   if (h0->m.fused && h1->m.fused && h0->m.activation == h1->m.activation && h0->m.dtype == h1->m.dtype && M < 64 * 256) {
     if (h0->m.dtype == KS_MLP_F32) return launch_fused_pair_tile<float, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1);
@@ -1998,6 +2225,7 @@ extern "C" int64_t ks_mlp_workspace_bytes(const KsMlp* h, int64_t M) {
   if (!h || M < 0) return 0;
   const int64_t few = M < kSmallRows ? M : kSmallRows;
   if (h->m.n_layers > 1 && small_ok(h->m, few)) return 2 * 4 * small_ws_floats(h->m, few);
+  if (split_ok(h->m, 1)) return split_ws_bytes(M < kSplitRows ? M : kSplitRows);
   if (h->m.fused) return 0;
   int widest = 0;
   for (int l = 0; l + 1 < h->m.n_layers; ++l) widest = h->m.npad[l] > widest ? h->m.npad[l] : widest;
@@ -2012,6 +2240,7 @@ extern "C" int ks_mlp_forward(const KsMlp* h, ks_stream_t stream, int64_t M, con
   if (!x || !y) return fail(KS_EINVAL, "ks_mlp_forward: null pointer");
   const DevMlp& m = h->m;
   if (small_ok(m, M) && (m.n_layers == 1 || workspace)) return launch_small(m, nullptr, (hipStream_t)stream, M, x, y, workspace, nullptr, nullptr, nullptr);
+  if (split_ok(m, M) && workspace) return launch_split(m, nullptr, (hipStream_t)stream, M, x, y, workspace, nullptr, nullptr, nullptr);
   if (m.fused) return launch_fused(m, (hipStream_t)stream, M, x, y);
   if (m.n_layers > 1 && !workspace) return fail(KS_EINVAL, "ks_mlp_forward: workspace required");
   if ((M + kBM - 1) / kBM > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward: too many rows");

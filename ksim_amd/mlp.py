@@ -6,6 +6,7 @@ use plain MLP stacks.  Weights are given as (out, in) fp32 arrays, like the refe
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import Sequence
 
 import numpy as np
@@ -61,9 +62,10 @@ class MLP:
         return 2 * sum(a * b for a, b in zip(self.dims[:-1], self.dims[1:]))
 
     def workspace(self, M: int, device) -> torch.Tensor:
-        """Scratch of the per-layer path, one buffer per stream: calls on different streams may overlap on the GPU."""
+        """Scratch of the paths that take several launches, one buffer per stream and thread: calls on different streams may overlap
+        on the GPU, and the launches of two threads may alternate on one stream."""
         need = int(self._lib.ks_mlp_workspace_bytes(self._handle, M))
-        key = torch.cuda.current_stream().cuda_stream if need else 0
+        key = (torch.cuda.current_stream().cuda_stream, threading.get_ident()) if need else 0
         if self._ws is None:
             self._ws = {}
         ws = self._ws.get(key)

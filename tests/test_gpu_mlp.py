@@ -290,3 +290,38 @@ def test_fp32_training_and_inference_forward_are_bit_equal(dims, act):
         for (gw, _), w in zip(net.parameters(gradients=True), tw):
             # fp32 sums of up to M rows of terms whose own error is a few 2^-24; ReLU's kink is met by no row here that a rounding moves
             assert (gw.double().cpu() - w.grad).abs().max() <= 1e-4 * w.grad.abs().max()
+
+
+@pytest.mark.parametrize("dims,act", [((68, 512, 512, 512, 20), "elu"), ((475, 500, 512, 33), "tanh"), ((1, 361, 384, 353, 512, 1), "relu"),
+                                      ((96, 384, 400, 64), "elu"), ((97, 512, 353, 5), "gelu")])
+def test_few_rows_of_wide_bf16_networks(dims, act):
+    """Up to 256 rows of a wide bf16 network spread every layer over CUs, a launch per layer: the same sums in the same order as the
+    whole-network kernel's, which a call without scratch takes.  Scratch is garbage at first, and misaligned once."""
+    import ctypes
+
+    from ksim_amd import _lib
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(sum(dims))
+    nets = [MLP([rng.normal(scale=1 / np.sqrt(i), size=(o, i)).astype(np.float32) for i, o in zip(d[:-1], d[1:])],
+                [rng.normal(scale=0.1, size=o).astype(np.float32) for o in d[1:]], activation=act, dtype="bf16")
+            for d in (dims, dims[:-2] + (512, 1))]
+    lib, p = nets[0]._lib, lambda t: ctypes.c_void_p(t.data_ptr())
+    for M in (1, 31, 32, 33, 255, 256, 257):
+        need = [lib.ks_mlp_workspace_bytes(n._handle, M) for n in nets]
+        assert min(need) > 0
+        ws = [torch.full((k + 8,), 255, dtype=torch.uint8, device=DEV) for k in need]
+        x = [torch.randn(M, dims[0], device=DEV) for _ in nets]
+        plain = [torch.empty(M, n.out_dim, device=DEV) for n in nets]
+        for n, a, o in zip(nets, x, plain):
+            assert lib.ks_mlp_forward(n._handle, _lib.current_stream(), M, p(a), p(o), None) == 0
+        for at in (0, 4):
+            out = [torch.full((M + 1, n.out_dim), 7.0, device=DEV) for n in nets]
+            for n, a, o, w in zip(nets, x, out, ws):
+                assert lib.ks_mlp_forward(n._handle, _lib.current_stream(), M, p(a), p(o), ctypes.c_void_p(w.data_ptr() + at)) == 0
+            pair = [torch.full((M + 1, n.out_dim), 7.0, device=DEV) for n in nets]
+            assert lib.ks_mlp_forward_pair(nets[0]._handle, nets[1]._handle, _lib.current_stream(), M, p(x[0]), p(pair[0]), p(x[1]), p(pair[1]),
+                                           p(ws[0]), p(ws[1])) == 0
+            for o, q, want in zip(out, pair, plain):
+                assert torch.equal(o[:M], want) and torch.equal(q[:M], want)
+                assert bool((o[M] == 7.0).all()) and bool((q[M] == 7.0).all())  # nothing behind the last row
