@@ -851,6 +851,9 @@ int ks_ppo_adapt_kl(ks_stream_t stream, int64_t rows, int32_t A, const float* on
                     float kl_coef, float desired_kl, float* kl_scale, float* workspace);
 int ks_mlp_grad_sqnorm(const KsMlp* mlp, ks_stream_t stream, double* acc);
 int ks_mlp_adam_step(KsMlp* mlp, ks_stream_t stream, const KsAdamParams* params /*host*/, const double* sqnorm);
+/* The same over `count` networks that are optimised together (host table of handles), in a launch for all of them. */
+int ks_mlps_grad_sqnorm(const KsMlp* const* mlps, int32_t count, ks_stream_t stream, double* acc);
+int ks_mlps_adam_step(KsMlp* const* mlps, int32_t count, ks_stream_t stream, const KsAdamParams* params /*host*/, const double* sqnorm);
 int ks_adam_step(ks_stream_t stream, int64_t n, float* param, const float* grad, float* m1, float* m2,
                  const KsAdamParams* params /*host*/, const double* sqnorm);
 /* Copies of the parameters and gradients in the caller's (out, in) layout, for checks and checkpoints. */

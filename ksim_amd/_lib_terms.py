@@ -288,6 +288,8 @@ def bind(lib) -> None:
     lib.ks_mlp_disc_loss_grad.restype = c_int32
     lib.ks_mlp_grad_sqnorm.argtypes = [c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_adam_step.argtypes = [c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
+    lib.ks_mlps_grad_sqnorm.argtypes = [c_void_p, c_int32, c_void_p, c_void_p]
+    lib.ks_mlps_adam_step.argtypes = [c_void_p, c_int32, c_void_p, POINTER(KsAdamParams), c_void_p]
     lib.ks_adam_step.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
     lib.ks_mlp_param_floats.argtypes = [c_void_p, c_int32]
     lib.ks_mlp_param_floats.restype = c_int64
@@ -298,7 +300,7 @@ def bind(lib) -> None:
     lib.ks_mlp_get_params.argtypes = [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32]
     lib.ks_gaussian_log_prob.argtypes = [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     for name in ("ks_mlp_train_init", "ks_mlp_train_forward", "ks_mlp_train_backward", "ks_grad_sqnorm",
-                 "ks_mlp_grad_sqnorm", "ks_mlp_adam_step", "ks_adam_step", "ks_mlp_get_params", "ks_gaussian_log_prob"):
+                 "ks_mlp_grad_sqnorm", "ks_mlp_adam_step", "ks_mlps_grad_sqnorm", "ks_mlps_adam_step", "ks_adam_step", "ks_mlp_get_params", "ks_gaussian_log_prob"):
         getattr(lib, name).restype = c_int32
     for name in ("ks_terms_create", "ks_terms_destroy", "ks_observe", "ks_terminate_reset", "ks_sample_action",
                  "ks_mlp_create", "ks_mlp_destroy", "ks_mlp_forward", "ks_mlp_forward_pair"):

@@ -782,14 +782,14 @@ extern "C" int ks_gru_projections(KsGru* g, KsMlp** input_projection, KsMlp** hi
 
 extern "C" int ks_gru_grad_sqnorm(const KsGru* g, ks_stream_t stream, double* acc) {
   if (!g || !acc) return fail(KS_EINVAL, "ks_gru_grad_sqnorm: null argument");
-  const int rc = ks_mlp_grad_sqnorm(g->proj_i, stream, acc);
-  return rc != KS_OK ? rc : ks_mlp_grad_sqnorm(g->proj_h, stream, acc);
+  const KsMlp* nets[] = {g->proj_i, g->proj_h};
+  return ks_mlps_grad_sqnorm(nets, 2, stream, acc);
 }
 
 extern "C" int ks_gru_adam_step(KsGru* g, ks_stream_t stream, const KsAdamParams* params, const double* sqnorm) {
   if (!g || !g->bias_nt) return fail(KS_EINVAL, "ks_gru_adam_step: call ks_gru_train_init first");
-  const int rc = ks_mlp_adam_step(g->proj_i, stream, params, sqnorm);
-  return rc != KS_OK ? rc : ks_mlp_adam_step(g->proj_h, stream, params, sqnorm);
+  KsMlp* nets[] = {g->proj_i, g->proj_h};
+  return ks_mlps_adam_step(nets, 2, stream, params, sqnorm);
 }
 
 extern "C" int ks_gru_train_forward(const KsGru* g, ks_stream_t stream, int64_t M, const float* x, const float* h_in,
@@ -1017,12 +1017,12 @@ extern "C" int ks_lstm_backward_step(KsLstm* g, ks_stream_t stream, int64_t M, c
 
 extern "C" int ks_lstm_grad_sqnorm(const KsLstm* g, ks_stream_t stream, double* acc) {
   if (!g || !acc) return fail(KS_EINVAL, "ks_lstm_grad_sqnorm: null argument");
-  const int rc = ks_mlp_grad_sqnorm(g->proj_i, stream, acc);
-  return rc != KS_OK ? rc : ks_mlp_grad_sqnorm(g->proj_h, stream, acc);
+  const KsMlp* nets[] = {g->proj_i, g->proj_h};
+  return ks_mlps_grad_sqnorm(nets, 2, stream, acc);
 }
 
 extern "C" int ks_lstm_adam_step(KsLstm* g, ks_stream_t stream, const KsAdamParams* params, const double* sqnorm) {
   if (!g) return fail(KS_EINVAL, "ks_lstm_adam_step: null handle");
-  const int rc = ks_mlp_adam_step(g->proj_i, stream, params, sqnorm);
-  return rc != KS_OK ? rc : ks_mlp_adam_step(g->proj_h, stream, params, sqnorm);
+  KsMlp* nets[] = {g->proj_i, g->proj_h};
+  return ks_mlps_adam_step(nets, 2, stream, params, sqnorm);
 }

@@ -1602,9 +1602,11 @@ __global__ __launch_bounds__(256) void grad_finish_kernel(GradFinishArgs a) {
 // Every addition happens in a fixed order (a strided pass per lane, a tree over the lanes, then the partial sums one after
 // the other), so the clip factor, and with it a whole update, is the same bits on every run.
 constexpr int kSqBlocks = 64;
+constexpr int kSqTensors = 64;  // gradient tensors per launch
 struct SqTensors {
-  const float* g[2 * KS_MAX_LAYERS];
-  int64_t n[2 * KS_MAX_LAYERS];
+  const float* g[kSqTensors];
+  int64_t n[kSqTensors];
+  double* part[kSqTensors];  // kSqBlocks of them
 };
 
 __device__ __forceinline__ double block_sqsum(const float* __restrict__ g, int64_t n, int first, int stride, double* red) {
@@ -1623,24 +1625,36 @@ __device__ __forceinline__ double block_sqsum(const float* __restrict__ g, int64
 }
 
 // grid (kSqBlocks, tensors): part[tensor][block] = this block's share of the tensor
-__global__ __launch_bounds__(256) void sqnorm_parts_kernel(SqTensors t, double* __restrict__ part) {
+__global__ __launch_bounds__(256) void sqnorm_parts_kernel(SqTensors t) {
   __shared__ double red[256];
   const double v = block_sqsum(t.g[blockIdx.y], t.n[blockIdx.y], (int)(blockIdx.x * 256 + threadIdx.x), kSqBlocks * 256, red);
-  if (threadIdx.x == 0) part[blockIdx.y * kSqBlocks + blockIdx.x] = v;
+  if (threadIdx.x == 0) t.part[blockIdx.y][blockIdx.x] = v;
 }
 
-// one workgroup: *acc += the partial sums, in index order
-__global__ __launch_bounds__(256) void sqnorm_finish_kernel(int n, const double* __restrict__ part, double* __restrict__ acc) {
-  __shared__ double red[256];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+// one workgroup: *acc += every network's partial sums, a wavefront per network, the networks in order
+constexpr int kSqNets = 32;
+struct SqNets {
+  double* acc;
+  int nets;
+  int n[kSqNets];
+  const double* part[kSqNets];
+};
+__global__ __launch_bounds__(1024) void sqnorm_finish_kernel(SqNets t) {
+  __shared__ double sum[kSqNets];
+  const int lane = threadIdx.x & 63;
+  for (int k = threadIdx.x >> 6; k < t.nets; k += 16) {
+    double s = 0.0;
+    for (int i = lane; i < t.n[k]; i += 64) s += t.part[k][i];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d);
+    if (lane == 0) sum[k] = s;
   }
-  if (threadIdx.x == 0) *acc += red[0];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double v = *t.acc;
+    for (int k = 0; k < t.nets; ++k) v += sum[k];
+    *t.acc = v;
+  }
 }
 
 // one workgroup over a whole buffer (small tensors that belong to no network: log standard deviations, head parameters)
@@ -1702,72 +1716,98 @@ __global__ __launch_bounds__(256) void refresh_kernel(int npad, int kpad, const 
   }
 }
 
-// One optimiser step of a whole network in one launch: every weight and bias element goes through the chain of adam_kernel,
-// and the thread that updates a master weight also writes its working copies (W, W^T, the fragment-ordered copy of the
-// whole-network kernel), as refresh_kernel does; the thread of a layer's element o < npad updates bias o as well.  The same
-// arithmetic per element as the per-tensor launches, which it replaces (two dozen launches and copies per network).
-struct AdamNetArgs {
-  int n_layers;
-  int npad[KS_MAX_LAYERS], kpad[KS_MAX_LAYERS], fk[KS_MAX_LAYERS], fn[KS_MAX_LAYERS], frozen[KS_MAX_LAYERS];
-  int first_block[KS_MAX_LAYERS + 1];  // workgroups [first_block[l], first_block[l + 1]) belong to layer l
-  float *mW[KS_MAX_LAYERS], *m1W[KS_MAX_LAYERS], *m2W[KS_MAX_LAYERS], *mb[KS_MAX_LAYERS], *m1b[KS_MAX_LAYERS], *m2b[KS_MAX_LAYERS];
-  const float *gW[KS_MAX_LAYERS], *gb[KS_MAX_LAYERS];
-  void *W[KS_MAX_LAYERS], *Wt[KS_MAX_LAYERS];
-  void* Wp[KS_MAX_LAYERS];
-  __bf16* WtP[KS_MAX_LAYERS];
-  float *b[KS_MAX_LAYERS], *bp[KS_MAX_LAYERS];
+// One optimiser step of several networks in one launch: every weight and bias element goes through the chain of adam_kernel, and the
+// workgroup that updates a 32 x 32 tile of a master weight also writes the tile's working copies (W, W^T, the fragment-ordered copies), as
+// refresh_kernel does; the transposed ones go through LDS, so that all leave in runs of 64 bytes and more.  The biases of a tile's rows ride
+// on the first tile of those rows.  Bound by memory for the large networks (28 bytes of state and up to 10 of copies per weight), by its launch for the
+// small ones, of which a recurrent policy has a dozen: actor and critic of 3 x 512 in bf16 2 x 13.5 -> 12.9 us, the twelve networks of a GRU
+// policy 12 x 6 -> 10 us.
+constexpr int kOptLayers = 24;  // layers per launch
+struct AdamLayer {
+  int npad, kpad, fk, fn, frozen, first_block;
+  float *mW, *m1W, *m2W, *mb, *m1b, *m2b;
+  const float *gW, *gb;
+  void *W, *Wt, *Wp;
+  __bf16* WtP;
+  float *b, *bp;
+};
+struct AdamTable {
+  int n;
+  AdamLayer layer[kOptLayers];
+};
+struct AdamStep {
+  float lr, b1, b2, eps, weight_decay, max_grad_norm, c1, c2;  // c1, c2: 1 - b^step
 };
 
-__device__ __forceinline__ float adam_element(float p, float g, float& m1, float& m2, const KsAdamParams& a, const double* sqnorm) {
+__device__ __forceinline__ float adam_element(float p, float g, float& m1, float& m2, const AdamStep& a, float norm) {
   float gv = g;
   if (!(gv == gv)) gv = 0.f;                                       // zero_nans
-  if (a.max_grad_norm > 0.f && sqnorm) {                           // clip_by_global_norm
-    const float norm = (float)sqrt(*sqnorm);
-    if (norm > a.max_grad_norm) gv = gv / norm * a.max_grad_norm;
-  }
+  if (a.max_grad_norm > 0.f && norm > a.max_grad_norm) gv = gv / norm * a.max_grad_norm;  // clip_by_global_norm
   gv += a.weight_decay * p;                                        // add_decayed_weights
   m1 = a.b1 * m1 + (1.f - a.b1) * gv;                              // scale_by_adam
   m2 = a.b2 * m2 + (1.f - a.b2) * gv * gv;
-  const float mhat = m1 / (1.f - powf(a.b1, (float)a.step));
-  const float vhat = m2 / (1.f - powf(a.b2, (float)a.step));
+  const float mhat = m1 / a.c1;
+  const float vhat = m2 / a.c2;
   return p - a.lr * mhat / (sqrtf(vhat) + a.eps);
 }
 
+// four neighbouring entries in working precision
 template <typename T>
-__global__ __launch_bounds__(256) void adam_net_kernel(AdamNetArgs n, KsAdamParams a, const double* __restrict__ sqnorm) {
+__device__ __forceinline__ void store4(T* to, const float (&v)[4]) {
+  if constexpr (sizeof(T) == 2) *reinterpret_cast<uint2*>(to) = uint2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+  else *reinterpret_cast<float4*>(to) = float4{v[0], v[1], v[2], v[3]};
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void adam_layers_kernel(AdamTable t, AdamStep a, const double* __restrict__ sqnorm) {
+  __shared__ float tr[32][33];
   int l = 0;
-  while (l + 1 < n.n_layers && (int)blockIdx.x >= n.first_block[l + 1]) ++l;
-  const int npad = n.npad[l], kpad = n.kpad[l];
-  const int64_t idx = (int64_t)(blockIdx.x - n.first_block[l]) * 256 + threadIdx.x;
-  if (idx < (int64_t)npad * kpad) {
-    float m1 = n.m1W[l][idx], m2 = n.m2W[l][idx];
-    const float v = adam_element(n.mW[l][idx], n.gW[l][idx], m1, m2, a, sqnorm);
-    n.m1W[l][idx] = m1; n.m2W[l][idx] = m2; n.mW[l][idx] = v;
-    const int o = (int)(idx / kpad), i = (int)(idx - (int64_t)o * kpad);
-    reinterpret_cast<T*>(n.W[l])[idx] = from_f32<T>(v);
-    if (n.Wt[l]) reinterpret_cast<T*>(n.Wt[l])[(int64_t)i * npad + o] = from_f32<T>(v);
+  while (l + 1 < t.n && (int)blockIdx.x >= t.layer[l + 1].first_block) ++l;
+  const AdamLayer& n = t.layer[l];
+  const int tile = (int)blockIdx.x - n.first_block, ti = n.kpad / 32, o0 = tile / ti * 32, i0 = (tile - tile / ti * ti) * 32;
+  const float norm = a.max_grad_norm > 0.f && sqnorm ? (float)sqrt(*sqnorm) : 0.f;
+  constexpr int G = 16 / (int)sizeof(T);  // entries of a lane's fragment
+  const int x = threadIdx.x >> 3, y = (threadIdx.x & 7) * 4;
+  {
+    const int o = o0 + x, i = i0 + y;
+    const int64_t idx = (int64_t)o * n.kpad + i;
+    const float4 p4 = *reinterpret_cast<const float4*>(n.mW + idx), g4 = *reinterpret_cast<const float4*>(n.gW + idx);
+    float4 m14 = *reinterpret_cast<const float4*>(n.m1W + idx), m24 = *reinterpret_cast<const float4*>(n.m2W + idx);
+    float v[4];
+    v[0] = adam_element(p4.x, g4.x, m14.x, m24.x, a, norm);
+    v[1] = adam_element(p4.y, g4.y, m14.y, m24.y, a, norm);
+    v[2] = adam_element(p4.z, g4.z, m14.z, m24.z, a, norm);
+    v[3] = adam_element(p4.w, g4.w, m14.w, m24.w, a, norm);
+    *reinterpret_cast<float4*>(n.m1W + idx) = m14;
+    *reinterpret_cast<float4*>(n.m2W + idx) = m24;
+    *reinterpret_cast<float4*>(n.mW + idx) = float4{v[0], v[1], v[2], v[3]};
+    store4<T>(reinterpret_cast<T*>(n.W) + idx, v);
     // [tile o / 32][k step i / 2G][lane (o % 32) + 32 ((i % 2G) / G)][i % G], G = 8 (bf16) or 4 (fp32).  The fragment copy is padded to
     // 32 outputs and 2G inputs, the master to the coarser tiles of the per-layer kernel: master entries beyond the fragment copy are padding
     // (zero weights with zero gradients) and have no place in it.
-    constexpr int G = 16 / (int)sizeof(T);
-    if (n.Wp[l] && o < n.fn[l] * 32 && i < n.fk[l] * 2 * G) {
-      const int64_t at = (((int64_t)(o >> 5) * n.fk[l] + i / (2 * G)) * 64 + (o & 31) + 32 * ((i / G) & 1)) * G + i % G;
-      reinterpret_cast<T*>(n.Wp[l])[at] = from_f32<T>(v);
-      if (n.WtP[l]) {  // the same entry with the roles of input and output exchanged
-        const int64_t att = ((((int64_t)(i >> 5) * (2 * n.fn[l]) + (o >> 4)) * 64 + (i & 31) + 32 * ((o >> 3) & 1)) << 3) + (o & 7);
-        n.WtP[l][att] = (__bf16)v;
-      }
-    }
+    if (n.Wp && o < n.fn * 32 && i < n.fk * 2 * G)
+      store4<T>(reinterpret_cast<T*>(n.Wp) + (((int64_t)(o >> 5) * n.fk + i / (2 * G)) * 64 + (o & 31) + 32 * ((i / G) & 1)) * G + i % G, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tr[y + e][x] = v[e];
   }
-  if (idx < npad) {
-    float v = n.mb[l][idx];
-    if (idx >= n.frozen[l]) {
-      float m1 = n.m1b[l][idx], m2 = n.m2b[l][idx];
-      v = adam_element(v, n.gb[l][idx], m1, m2, a, sqnorm);
-      n.m1b[l][idx] = m1; n.m2b[l][idx] = m2; n.mb[l][idx] = v;
+  if (n.Wt || n.WtP) {  // the same for the whole workgroup
+    __syncthreads();
+    const int i = i0 + x, o = o0 + y;
+    const float v[4] = {tr[x][y], tr[x][y + 1], tr[x][y + 2], tr[x][y + 3]};
+    if (n.Wt) store4<T>(reinterpret_cast<T*>(n.Wt) + (int64_t)i * n.npad + o, v);
+    if (n.WtP && o < n.fn * 32 && i < n.fk * 2 * G)  // the fragment copy with the roles of input and output exchanged
+      store4<__bf16>(n.WtP + ((((int64_t)(i >> 5) * (2 * n.fn) + (o >> 4)) * 64 + (i & 31) + 32 * ((o >> 3) & 1)) << 3) + (o & 7), v);
+  }
+  if (i0 == 0 && threadIdx.x < 32) {
+    const int o = o0 + (int)threadIdx.x;
+    float v = n.mb[o];
+    if (o >= n.frozen) {
+      float m1 = n.m1b[o], m2 = n.m2b[o];
+      v = adam_element(v, n.gb[o], m1, m2, a, norm);
+      n.m1b[o] = m1; n.m2b[o] = m2; n.mb[o] = v;
     }
-    n.b[l][idx] = v;
-    if (n.bp[l] && idx < n.fn[l] * 32) n.bp[l][idx] = v;
+    n.b[o] = v;
+    if (n.bp && o < n.fn * 32) n.bp[o] = v;
   }
 }
 
@@ -2779,22 +2819,36 @@ extern "C" int ks_grad_sqnorm(ks_stream_t stream, int64_t n, const float* g, dou
   return check_launch("ks_grad_sqnorm");
 }
 
+extern "C" int ks_mlps_grad_sqnorm(const KsMlp* const* nets, int32_t count, ks_stream_t stream, double* acc) {
+  if (count < 0 || (count > 0 && !nets) || !acc) return fail(KS_EINVAL, "ks_mlps_grad_sqnorm: bad argument");
+  for (int k = 0; k < count; ++k)
+    if (!nets[k] || !nets[k]->m.train) return fail(KS_EINVAL, "ks_mlps_grad_sqnorm: network %d: call ks_mlp_train_init first", k);
+  for (int k = 0; k < count;) {  // as many networks at a time as the tables hold
+    SqTensors t;
+    SqNets f;
+    f.nets = 0; f.acc = acc;
+    int nt = 0;
+    for (; k < count && f.nets < kSqNets && nt + 2 * nets[k]->m.n_layers <= kSqTensors; ++k) {
+      const DevMlp& m = nets[k]->m;
+      const int first = nt;
+      auto add = [&](const float* g, int64_t n) { t.g[nt] = g; t.n[nt] = n; t.part[nt] = m.sq_part + (nt - first) * kSqBlocks; ++nt; };
+      for (int l = 0; l < m.n_layers; ++l) {
+        add(m.gW[l], (int64_t)m.npad[l] * m.kpad[l]);
+        const int fz = m.bias_frozen[l];
+        if (m.npad[l] > fz) add(m.gb[l] + fz, (int64_t)m.npad[l] - fz);
+      }
+      f.n[f.nets] = (nt - first) * kSqBlocks;
+      f.part[f.nets++] = m.sq_part;
+    }
+    hipLaunchKernelGGL(sqnorm_parts_kernel, dim3(kSqBlocks, (unsigned)nt), dim3(256), 0, (hipStream_t)stream, t);
+    hipLaunchKernelGGL(sqnorm_finish_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, f);
+  }
+  return check_launch("ks_mlps_grad_sqnorm");
+}
+
 extern "C" int ks_mlp_grad_sqnorm(const KsMlp* h, ks_stream_t stream, double* acc) {
   if (!h || !h->m.train || !acc) return fail(KS_EINVAL, "ks_mlp_grad_sqnorm: bad argument");
-  SqTensors t;
-  int nt = 0;
-  for (int l = 0; l < h->m.n_layers; ++l) {
-    t.g[nt] = h->m.gW[l];
-    t.n[nt++] = (int64_t)h->m.npad[l] * h->m.kpad[l];
-    const int fz = h->m.bias_frozen[l];
-    if (h->m.npad[l] > fz) {
-      t.g[nt] = h->m.gb[l] + fz;
-      t.n[nt++] = (int64_t)h->m.npad[l] - fz;
-    }
-  }
-  hipLaunchKernelGGL(sqnorm_parts_kernel, dim3(kSqBlocks, (unsigned)nt), dim3(256), 0, (hipStream_t)stream, t, h->m.sq_part);
-  hipLaunchKernelGGL(sqnorm_finish_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, nt * kSqBlocks, h->m.sq_part, acc);
-  return check_launch("ks_mlp_grad_sqnorm");
+  return ks_mlps_grad_sqnorm(&h, 1, stream, acc);
 }
 
 static int check_adam(const KsAdamParams* p, const char* who) {
@@ -2814,28 +2868,39 @@ extern "C" int ks_adam_step(ks_stream_t stream, int64_t n, float* param, const f
   return check_launch("ks_adam_step");
 }
 
+extern "C" int ks_mlps_adam_step(KsMlp* const* nets, int32_t count, ks_stream_t stream, const KsAdamParams* p, const double* sqnorm) {
+  if (count < 0 || (count > 0 && !nets)) return fail(KS_EINVAL, "ks_mlps_adam_step: bad argument");
+  for (int k = 0; k < count; ++k)
+    if (!nets[k] || !nets[k]->m.train) return fail(KS_EINVAL, "ks_mlps_adam_step: network %d: call ks_mlp_train_init first", k);
+  const int rc = check_adam(p, "ks_mlps_adam_step");
+  if (rc != KS_OK) return rc;
+  const AdamStep a = {p->lr, p->b1, p->b2, p->eps, p->weight_decay, p->max_grad_norm, (float)(1.0 - std::pow((double)p->b1, (double)p->step)),
+                      (float)(1.0 - std::pow((double)p->b2, (double)p->step))};
+  for (int k = 0; k < count;) {  // networks of one precision, each once, as many as the table holds
+    AdamTable t;
+    t.n = 0;
+    int blocks = 0;
+    const int from = k, dtype = nets[k]->m.dtype;
+    for (; k < count; ++k) {
+      const DevMlp& m = nets[k]->m;
+      bool again = false;
+      for (int q = from; q < k; ++q) again |= nets[q] == nets[k];
+      if (again || m.dtype != dtype || t.n + m.n_layers > kOptLayers) break;
+      for (int l = 0; l < m.n_layers; ++l) {
+        t.layer[t.n++] = {m.npad[l], m.kpad[l], m.fk[l], m.fn[l], m.bias_frozen[l], blocks, m.mW[l], m.m1W[l], m.m2W[l], m.mb[l], m.m1b[l], m.m2b[l],
+                          m.gW[l], m.gb[l], m.W[l], m.Wt[l], m.Wp[l], (__bf16*)m.WtP[l], m.b[l], m.bp[l]};
+        blocks += m.npad[l] / 32 * (m.kpad[l] / 32);  // npad: whole tiles of 128; kpad: of 64 (bf16) or 32
+      }
+    }
+    if (dtype == KS_MLP_BF16) hipLaunchKernelGGL(adam_layers_kernel<__bf16>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, t, a, sqnorm);
+    else hipLaunchKernelGGL(adam_layers_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, t, a, sqnorm);
+  }
+  return check_launch("ks_mlps_adam_step");
+}
+
 extern "C" int ks_mlp_adam_step(KsMlp* h, ks_stream_t stream, const KsAdamParams* p, const double* sqnorm) {
   if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_adam_step: call ks_mlp_train_init first");
-  const int rc = check_adam(p, "ks_mlp_adam_step");
-  if (rc != KS_OK) return rc;
-  DevMlp& m = h->m;
-  hipStream_t s = (hipStream_t)stream;
-  AdamNetArgs n{};
-  n.n_layers = m.n_layers;
-  int blocks = 0;
-  for (int l = 0; l < m.n_layers; ++l) {
-    n.npad[l] = m.npad[l]; n.kpad[l] = m.kpad[l]; n.fk[l] = m.fk[l]; n.fn[l] = m.fn[l]; n.frozen[l] = m.bias_frozen[l];
-    n.first_block[l] = blocks;
-    blocks += (int)(((int64_t)m.npad[l] * m.kpad[l] + 255) / 256);  // npad * kpad >= npad: the bias rides on the first threads
-    n.mW[l] = m.mW[l]; n.m1W[l] = m.m1W[l]; n.m2W[l] = m.m2W[l]; n.gW[l] = m.gW[l];
-    n.mb[l] = m.mb[l]; n.m1b[l] = m.m1b[l]; n.m2b[l] = m.m2b[l]; n.gb[l] = m.gb[l];
-    n.W[l] = m.W[l]; n.Wt[l] = m.Wt[l]; n.Wp[l] = m.Wp[l]; n.WtP[l] = (__bf16*)m.WtP[l];
-    n.b[l] = m.b[l]; n.bp[l] = m.bp[l];
-  }
-  n.first_block[m.n_layers] = blocks;
-  if (m.dtype == KS_MLP_BF16) hipLaunchKernelGGL(adam_net_kernel<__bf16>, dim3((unsigned)blocks), dim3(256), 0, s, n, *p, sqnorm);
-  else hipLaunchKernelGGL(adam_net_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, s, n, *p, sqnorm);
-  return check_launch("ks_mlp_adam_step");
+  return ks_mlps_adam_step(&h, 1, stream, p, sqnorm);
 }
 
 // ---------------------------------------------------------------- discriminator update (ksim/task/amp.py:360-438)

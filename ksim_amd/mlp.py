@@ -183,6 +183,10 @@ class MLP:
         self._borrowed = True
         return self
 
+    def networks(self) -> list["MLP"]:
+        """The networks whose parameters an optimiser step over this one updates."""
+        return [self]
+
     def grad_sqnorm(self, acc: torch.Tensor) -> None:
         _lib.require_cuda(acc, dtype=torch.float64)
         _lib.check(self._lib.ks_mlp_grad_sqnorm(self._handle, _lib.current_stream(), _lib.ptr(acc)))
@@ -211,6 +215,21 @@ class MLP:
             self.close()
         except Exception:
             pass
+
+
+def _handles(nets: Sequence[MLP]):
+    return (ctypes.c_void_p * len(nets))(*(net._handle for net in nets))
+
+
+def grad_sqnorm(nets: Sequence[MLP], acc: torch.Tensor) -> None:
+    """Adds the squared gradient norm over all of `nets` to `acc`."""
+    _lib.require_cuda(acc, dtype=torch.float64)
+    _lib.check(_lib.load().ks_mlps_grad_sqnorm(_handles(nets), len(nets), _lib.current_stream(), _lib.ptr(acc)))
+
+
+def adam_step(nets: Sequence[MLP], params: "T.KsAdamParams", sqnorm: torch.Tensor | None) -> None:
+    """One optimiser step of all of `nets`; `sqnorm` is the squared gradient norm over everything optimised together."""
+    _lib.check(_lib.load().ks_mlps_adam_step(_handles(nets), len(nets), _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
 
 
 def random_mlp(dims: Sequence[int], seed: int, activation: str = "elu", dtype: str = "bf16"):

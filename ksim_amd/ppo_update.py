@@ -20,6 +20,7 @@ from . import _lib
 from . import _lib_terms as T
 from . import ppo as ppo_mod
 from .actions import LowPass
+from . import mlp as mlp_mod
 from .mlp import MLP
 
 
@@ -191,13 +192,12 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     policy.critic.backward(c_in, d_value_all)
     # optimiser chain over every parameter together: global norm first
     sq = torch.zeros(1, dtype=torch.float64, device=mean.device)
-    policy.actor.grad_sqnorm(sq)
-    policy.critic.grad_sqnorm(sq)
+    nets = policy.actor.networks() + policy.critic.networks()
+    mlp_mod.grad_sqnorm(nets, sq)
     _lib.check(lib.ks_grad_sqnorm(_lib.current_stream(), nu, _lib.ptr(d_log_std), _lib.ptr(sq)))
     policy.opt_step += 1
     ap = _adam(cfg, policy.opt_step)
-    policy.actor.adam_step(ap, sq)
-    policy.critic.adam_step(ap, sq)
+    mlp_mod.adam_step(nets, ap, sq)
     _lib.check(lib.ks_adam_step(_lib.current_stream(), nu, _lib.ptr(policy.log_std), _lib.ptr(d_log_std),
                                 _lib.ptr(policy._m1), _lib.ptr(policy._m2), ctypes.byref(ap), _lib.ptr(sq)))
     metrics = {"grad_norm": sq.sqrt(), "d_mean": d_mean, "d_value": d_value, "d_log_std": d_log_std,
@@ -413,12 +413,11 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
     policy.actor.backward(d_raw_all)
     policy.critic.backward(d_value_all)
     sq = torch.zeros(1, dtype=torch.float64, device=dev)
-    policy.actor.grad_sqnorm(sq)
-    policy.critic.grad_sqnorm(sq)
+    nets = policy.actor.networks() + policy.critic.networks()
+    mlp_mod.grad_sqnorm(nets, sq)
     policy.opt_step += 1
     ap = _adam(cfg, policy.opt_step)
-    policy.actor.adam_step(ap, sq)
-    policy.critic.adam_step(ap, sq)
+    mlp_mod.adam_step(nets, ap, sq)
     metrics = {"grad_norm": sq.sqrt(), "d_raw": d_raw, "d_value": d_value, "raw": raw, "values": value,
                "advantages": inputs.advantages_bt, **aux}
     if cfg.adaptive_kl:  # ppo.py:546-563 on the log-probabilities of this step's forward pass

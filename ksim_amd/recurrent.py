@@ -15,6 +15,7 @@ import torch
 
 from . import _lib
 from . import _lib_terms as T
+from . import mlp as mlp_mod
 from .mlp import MLP
 
 
@@ -480,10 +481,14 @@ class RecurrentNetwork:
             dH = dX
         self.input_proj.backward(tp["obs"].view(T_ * M, self.in_dim), dH.view(T_ * M, H))
 
+    def networks(self) -> list[MLP]:
+        """Every network whose parameters an optimiser step updates: the projections and both products of every cell."""
+        if any(getattr(c, "proj_i", None) is None for c in self.cells):
+            raise _lib.KsError("call train_init first")
+        return [self.input_proj, *(p for c in self.cells for p in (c.proj_i, c.proj_h)), self.output_proj]
+
     def grad_sqnorm(self, acc: torch.Tensor) -> None:
-        for net in (self.input_proj, *self.cells, self.output_proj):
-            net.grad_sqnorm(acc)
+        mlp_mod.grad_sqnorm(self.networks(), acc)
 
     def adam_step(self, params, sqnorm) -> None:
-        for net in (self.input_proj, *self.cells, self.output_proj):
-            net.adam_step(params, sqnorm)
+        mlp_mod.adam_step(self.networks(), params, sqnorm)

@@ -325,3 +325,57 @@ def test_few_rows_of_wide_bf16_networks(dims, act):
             for o, q, want in zip(out, pair, plain):
                 assert torch.equal(o[:M], want) and torch.equal(q[:M], want)
                 assert bool((o[M] == 7.0).all()) and bool((q[M] == 7.0).all())  # nothing behind the last row
+
+
+def test_networks_optimised_together_match_one_by_one():
+    """One squared norm and one optimiser step over many networks: mixed precisions, more layers than a launch's table holds, ragged widths, a
+    frozen bias and a network named twice (two steps); against the same calls network by network."""
+    import ctypes
+
+    from ksim_amd import _lib, _lib_terms as T, mlp
+    from ksim_amd.mlp import MLP
+
+    shapes = [((68, 512, 512, 512, 20), "bf16"), ((33, 130, 7), "bf16"), ((128, 384), "bf16"), ((475, 128), "f32"), ((5, 3), "f32"),
+              ((20, 40, 30, 20, 30, 40, 20, 10, 5), "f32"), ((9, 8, 7, 6, 5, 4, 3, 2, 1), "f32"), ((17, 70, 90, 5), "f32"), ((40, 33), "f32")]
+
+    def make():
+        rng = np.random.default_rng(5)
+        nets = []
+        for dims, dtype in shapes:
+            net = MLP([rng.normal(scale=1 / np.sqrt(i), size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])],
+                      [rng.normal(scale=0.1, size=o).astype(np.float32) for o in dims[1:]], activation="elu", dtype=dtype)
+            net.train_init()
+            x = torch.from_numpy(rng.normal(size=(96, dims[0])).astype(np.float32)).to(DEV)
+            net.train_forward(x)
+            net.backward(x, torch.from_numpy(rng.normal(size=(96, dims[-1])).astype(np.float32)).to(DEV))
+            nets.append((net, x))
+        _lib.check(nets[2][0]._lib.ks_mlp_freeze_bias_prefix(nets[2][0]._handle, 0, 100))
+        return nets
+
+    one, all_ = make(), make()
+    params = T.KsAdamParams(1e-2, 0.9, 0.999, 1e-8, 0.01, 0.5, 3)
+    a, b = (torch.full((1,), 0.25, dtype=torch.float64, device=DEV) for _ in range(2))
+    for net, _ in one:
+        net.grad_sqnorm(a)
+    mlp.grad_sqnorm([n for n, _ in all_], b)
+    want = 0.25
+    for k, (net, _) in enumerate(all_):
+        for w, g in net.parameters(gradients=True):
+            want += float(w.double().square().sum()) + float(g.double()[100 if k == 2 else 0:].square().sum())
+    assert torch.equal(a, b) and abs(float(b) - want) < 1e-9 * want
+    order = list(range(len(one))) + [1]
+    for k in order:
+        one[k][0].adam_step(params, a)
+    mlp.adam_step([all_[k][0] for k in order], params, b)
+    for (n1, x), (n2, _) in zip(one, all_):
+        for (w1, b1), (w2, b2) in zip(n1.parameters(), n2.parameters()):
+            assert torch.equal(w1, w2) and torch.equal(b1, b2)
+        y = n2(x)  # the copies that the forward and backward passes read follow the master weights
+        assert torch.equal(n1(x), y)
+        ws, bs = zip(*n2.parameters())
+        ref = reference(x.cpu().numpy(), [w.cpu().numpy() for w in ws], [c.cpu().numpy() for c in bs], "elu", n2.dtype == "bf16")
+        assert np.abs(y.cpu().numpy() - ref).max() <= (6e-3 if n2.dtype == "bf16" else 2e-5) * np.abs(ref).max()
+        dx1, dx2 = torch.empty_like(x), torch.empty_like(x)
+        dy = torch.ones(x.shape[0], n2.out_dim, device=DEV)
+        n1.train_forward(x); n2.train_forward(x)
+        assert torch.equal(n1.backward_dx(x, dy, dx1), n2.backward_dx(x, dy, dx2))
