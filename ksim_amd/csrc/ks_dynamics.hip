@@ -157,9 +157,9 @@ __device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myin
     const float inv = fminf(__builtin_amdgcn_rsqf(lane_bcast(T[rho], j + 32 * hj)), 1e15f);
     myinv = lane == j ? inv : myinv;
     const bool sel = half == hj && c > j;
-    const float t = T[rho] * inv;
-    const float a = sel ? t : 0.f, na = sel ? -t : 0.f;
-    T[rho] = sel ? t : T[rho];
+    const float u = sel ? T[rho] : 0.f;  // beside the reciprocal root, not behind it
+    const float a = u * inv, na = -u * inv;
+    T[rho] = sel ? a : T[rho];
     // the last real column has nothing right of or below it
     if (j + 1 < NP && !(j + 1 >= padded_from(NP) && j + 1 >= nv)) T = __builtin_amdgcn_mfma_f32_32x32x2f32(na, a, T, 0, 0, 0);
   }
@@ -188,31 +188,33 @@ __device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ 
   }
 }
 
-// L^T x = y, lane i holding r_i = y_i * L[i][i] and returning x_i
+// L^T x = y, lane i holding y_i and returning x_i.  With w_i = y_i / L[i][i] a step is w_i -= (R[k] / L[i][i]^2) x_k, x_k = w_k: the scaled
+// and masked coefficient does not wait for the step before, so the chain is one broadcast and one fused multiply-add per column.
 template <int NP>
-__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, int lane, float r, int nv) {
+__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, int lane, float y, int nv) {
   const float myinv2 = myinv * myinv;
+  float w = y * myinv;
 #pragma unroll
-  for (int k = NP - 1; k >= 0; --k) {  // in the scaled form  sum_{k>i} R[k] x_k + L[i][i]^2 x_i = r_i
+  for (int k = NP - 1; k >= 0; --k) {
     if (k >= padded_from(NP) && k >= nv) continue;  // padded unknowns are zero and couple to nothing
-    const float xk = lane_bcast(r * myinv2, k);
-    r = lane < k ? r - R[k] * xk : r;
+    const float coef = lane < k ? R[k] * myinv2 : 0.f;
+    w -= coef * lane_bcast(w, k);
   }
-  return r * myinv2;
+  return w;
 }
 
 // x = (L L^T)^-1 b, lane i holding b_i and returning x_i
 template <int NP>
 __device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, int lane, float b, int nv) {
   asm volatile("" : "+v"(lane));  // as in chol_tile: the masks lane > j, lane < k are rebuilt here, not kept
-  float r = b;
+  float y = b * myinv;
 #pragma unroll
-  for (int j = 0; j < NP; ++j) {  // L y = b; lane j keeps r_j = y_j * L[j][j]
-    if (j >= padded_from(NP) && j >= nv) continue;  // padded unknowns are zero and couple to nothing
-    const float yj = lane_bcast(r * myinv, j);
-    r = lane > j ? r - R[j] * yj : r;
+  for (int j = 0; j < NP; ++j) {  // L y = b in the same form
+    if (j >= padded_from(NP) && j >= nv) continue;
+    const float coef = lane > j ? R[j] * myinv : 0.f;
+    y -= coef * lane_bcast(y, j);
   }
-  return back_substitute<NP>(R, myinv, lane, r, nv);
+  return back_substitute<NP>(R, myinv, lane, y, nv);
 }
 
 // Factors the tile and returns x = (L L^T)^-1 b, lane i holding b_i (zero beyond nv).  A matrix of fewer than 32 columns carries b
@@ -235,7 +237,7 @@ __device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& my
     KS_SYNC();
     const float y = vbuf[lane & 31];
     KS_SYNC();
-    return back_substitute<NP>(R, myinv, lane, y * __builtin_amdgcn_rcpf(myinv), nv);
+    return back_substitute<NP>(R, myinv, lane, y, nv);
   }
 }
 
