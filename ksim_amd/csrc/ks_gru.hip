@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void lstm_gate_backward_kernel(int64_t M, int 
 // cell state in a register; a step is 128 MFMAs (the fp32 matrix rate: 4 rows x 512 x 128 multiply-adds per CU), the gate
 // arithmetic of one (unit, row) per lane, and one barrier.  fp32 cells of hidden size 128.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-constexpr int kSeqRows = 4, kSeqH = 128, kSeqWaves = 8, kSeqPadH = kSeqH + 4, kSeqPadG = 4 * kSeqH + 4;
+constexpr int kSeqRows = 4, kSeqH = 128, kSeqWaves = 8, kSeqPadH = kSeqH + 4;
 
 __device__ __forceinline__ float sigmoid_ks(float x) { return 1.f / (1.f + expf(-x)); }
 
@@ -186,21 +186,36 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 __device__ __forceinline__ int seq_slot(int u) { return 8 * (u & 15) + (u >> 4); }
 
 // Transpose of a 4 x 4 block held by four neighbouring lanes (lane j of the group holds a0..a3): out[g] = a_j of lane g.
-// Three lane exchanges within the group (DPP quad permutes): for d = 1, 2, 3 lane s sends its entry s ^ d to lane s ^ d.
-__device__ __forceinline__ float pick4(float a0, float a1, float a2, float a3, int i) {
-  return i == 0 ? a0 : (i == 1 ? a1 : (i == 2 ? a2 : a3));
+// Two stages of exchanges within the group (DPP quad permutes) and selects: lanes that differ in the low bit swap what lies off their
+// diagonal in the pairs (a0, a1), (a2, a3), then lanes that differ in the high bit in the pairs (0, 2), (1, 3).  (A select by lane index per
+// entry became branches: 221 -> 198 us for 100 steps of an LSTM layer.)
+template <int CTRL>
+__device__ __forceinline__ float quad_perm(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ void quad_swap(float& lo, float& hi, bool upper) {  // the upper lane sends `lo`, the lower one `hi`
+  const float got = quad_perm<CTRL>(upper ? lo : hi);
+  lo = upper ? got : lo;
+  hi = upper ? hi : got;
 }
 __device__ __forceinline__ void quad_transpose(float a0, float a1, float a2, float a3, int j, float (&out)[4]) {
-  const float own = pick4(a0, a1, a2, a3, j);
-  const float s1 = pick4(a0, a1, a2, a3, j ^ 1), s2 = pick4(a0, a1, a2, a3, j ^ 2), s3 = pick4(a0, a1, a2, a3, j ^ 3);
-  const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s1), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
-  const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s2), 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
-  const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s3), 0x1B, 0xf, 0xf, true));  // quad_perm [3,2,1,0]
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int d = g ^ j;
-    out[g] = d == 0 ? own : (d == 1 ? r1 : (d == 2 ? r2 : r3));
-  }
+  const bool odd = (j & 1) != 0, high = (j & 2) != 0;
+  quad_swap<0xB1>(a0, a1, odd);   // quad_perm [1,0,3,2]
+  quad_swap<0xB1>(a2, a3, odd);
+  quad_swap<0x4E>(a0, a2, high);  // quad_perm [2,3,0,1]
+  quad_swap<0x4E>(a1, a3, high);
+  out[0] = a0; out[1] = a1; out[2] = a2; out[3] = a3;
+}
+
+// Sums over the four 16-lane rows of a wavefront, scattered: row q of lanes ends up with the total of v[q], added up as
+// (row 0 + row 1) + (row 2 + row 3).  A swap exchanges half of one register with half of the other, which is the whole exchange of a
+// stage; through LDS the same sums were eight permutes of a hundred cycles.
+__device__ __forceinline__ float rows_reduce_scatter(float v0, float v1, float v2, float v3) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3));
+  float lo = v0 + v1, hi = v2 + v3;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
+  return lo + hi;
 }
 
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -307,26 +322,34 @@ void lstm_seq_forward_kernel(int T, int64_t M, int groups, const float* __restri
 // The reverse sweep of the same layer: dH (T, M, H) is the gradient reaching h_t from the layer above; the gradient through
 // W_hh and that of the cell state are carried in registers.  Per step: the gate derivatives from the saved activations
 // (lstm_gate_backward_kernel's formulas) into d_g (T, M, 4H) and LDS, then dh_{t-1} = d_g W_hh over the transposed weights.
-// Here the sixteen blocks of an MFMA are four groups of four units (entries i) times four quarters of the 4H gate rows
-// (K split four ways): lane (b, j) accumulates, for row j, the partial sums over gate rows [128 (b / 4), 128 (b / 4) + 128) of the
-// units 16 w + 4 (b % 4) + {0..3}; two lane exchanges add the quarters, and the lane keeps the unit 16 w + 4 (b % 4) + b / 4.
+// Here the sixteen blocks of an MFMA are four quarters of the 4H gate rows (K split four ways: quarter kg = lane / 16 is gate kg) times
+// four groups of four units.  The gate gradients are the A operand (entries = the four rows), the same for the four blocks of a quarter and
+// broadcast to them from one block per instruction (CBSZ = 2, ABID = k mod 4): a lane fetches 32 of its quarter's 128 gate rows, eight 16-byte
+// reads per step.  (Fetched by every block, they were 32 reads per lane, as many cycles of the LDS pipe as the products are of the matrix
+// cores.)  A lane accumulates, for its unit, the four rows' partial sums over its quarter; the quarters are added up and scattered over
+// the lane rows, which leaves lane l with unit 16 w + l % 16 of row l / 16.
+// 1024 rows, 100 steps: 248 -> 169 us, of which the 128 products of two wavefronts per SIMD are 85.
+// where the gradient of gate row g H + u of a row sits in LDS: lane (quarter g, block a = u mod 4, row) reads its 32 as consecutive floats;
+// the paddings put the sixteen lanes of a quarter on different banks
+constexpr int kSeqGateA = 36, kSeqGateRow = 4 * 4 * kSeqGateA + 16;
+
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, const float* __restrict__ saved,
                               const uint8_t* __restrict__ fresh, const float* __restrict__ Wt, int ldwt,
                               float* __restrict__ d_g, float* __restrict__ dh0, float* __restrict__ dc0) {
   constexpr int H = kSeqH;
-  __shared__ __attribute__((aligned(16))) float sg[kSeqRows][kSeqPadG];
+  __shared__ __attribute__((aligned(16))) float sg[2][kSeqRows * kSeqGateRow];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int j = lane & 3, ug = (lane >> 2) & 3, kg = lane >> 4;
-  const int unit = 16 * wave + 4 * ug + kg;  // the (unit, row j) whose gate arithmetic and carried gradients this lane owns
+  const int kg = lane >> 4, blk = (lane >> 2) & 3, i = lane & 3;
+  const int unit = 16 * wave + (lane & 15);  // the (unit, row kg) whose gate arithmetic and carried gradients this lane owns
   const int64_t r0 = (int64_t)blockIdx.x * kSeqRows;
-  const int64_t m = r0 + j;
+  const int64_t m = r0 + kg;
   const bool row_ok = m < M;
   const int64_t mc = row_ok ? m : M - 1;
-  // A operand of block b, entry i = lane % 4: Wt[unit 16 w + 4 ug + i][gate row 128 kg + s]
+  // B operand, entry lane % 4 of block (kg, lane / 4 % 4): Wt[unit][gate row 128 kg + s]
   float wa[128];
   {
-    const float4* src = reinterpret_cast<const float4*>(Wt + (int64_t)(16 * wave + 4 * ug + j) * ldwt + 128 * kg);
+    const float4* src = reinterpret_cast<const float4*>(Wt + (int64_t)unit * ldwt + 128 * kg);
 #pragma unroll
     for (int s4 = 0; s4 < 32; ++s4) {
       const float4 v = src[s4];
@@ -334,6 +357,8 @@ void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, co
     }
   }
   float dhc = 0.f, dc = 0.f;
+  const int put = kg * kSeqGateRow + (unit & 3) * kSeqGateA + (unit >> 2);  // of gate 0; the next gate 4 kSeqGateA on
+  const int get = i * kSeqGateRow + (4 * kg + blk) * kSeqGateA;
   // the step's inputs from memory are fetched one step ahead, under the matrix work of the step before
   float nx[7];
   uint8_t fnext = 0;
@@ -345,6 +370,7 @@ void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, co
     nx[6] = dH[o * H + unit];
     if (fresh) fnext = fresh[o];
   }
+  int cur = 0;
   for (int t = T - 1; t >= 0; --t) {
     const bool f = fnext != 0;
     const float si = nx[0], sf = nx[1], tg = nx[2], so = nx[3], tc = nx[4], cp = nx[5];
@@ -361,33 +387,33 @@ void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, co
     const float gI = dct * tg * si * (1.f - si), gF = dct * cp * sf * (1.f - sf), gG = dct * si * (1.f - tg * tg),
                 gO = dh * tc * so * (1.f - so);
     dc = f ? 0.f : dct * sf;
-    sg[j][unit] = gI; sg[j][H + unit] = gF; sg[j][2 * H + unit] = gG; sg[j][3 * H + unit] = gO;
+    float* to = &sg[cur][put];
+    to[0] = gI; to[4 * kSeqGateA] = gF; to[8 * kSeqGateA] = gG; to[12 * kSeqGateA] = gO;
     if (row_ok) {
       float* dg = d_g + ((int64_t)t * M + m) * 4 * H + unit;
       dg[0] = gI; dg[H] = gF; dg[2 * H] = gG; dg[3 * H] = gO;
     }
-    lds_barrier();
+    lds_barrier();  // the gate gradients are complete; the buffer of the step before is free for the step after
+    float ga[32];
+    {
+      const float4* src = reinterpret_cast<const float4*>(&sg[cur][get]);
+#pragma unroll
+      for (int q4 = 0; q4 < 8; ++q4) {
+        const float4 v = src[q4];
+        ga[4 * q4] = v.x; ga[4 * q4 + 1] = v.y; ga[4 * q4 + 2] = v.z; ga[4 * q4 + 3] = v.w;
+      }
+    }
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    const float* grow = &sg[j][128 * kg];
 #pragma unroll
-    for (int s4 = 0; s4 < 32; ++s4) {
-      const float4 gb = *reinterpret_cast<const float4*>(grow + 4 * s4);
-      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4], gb.x, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 1], gb.y, acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 2], gb.z, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 3], gb.w, acc1, 0, 0, 0);
+    for (int q = 0; q < 32; ++q) {  // k = 4 q .. 4 q + 3 of the quarter, even k into one accumulator and odd k into the other
+      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q], acc0, 2, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 1], acc1, 2, 1, 0);
+      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 2], acc0, 2, 2, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 3], acc1, 2, 3, 0);
     }
-    float part[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v = acc0[r] + acc1[r];
-      v += __shfl_xor(v, 16);
-      v += __shfl_xor(v, 32);
-      part[r] = v;
-    }
-    const float mine = kg == 0 ? part[0] : (kg == 1 ? part[1] : (kg == 2 ? part[2] : part[3]));
+    const float mine = rows_reduce_scatter(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3]);
     dhc = f ? 0.f : mine;
-    lds_barrier();  // every wavefront has read this step's gate gradients
+    cur ^= 1;
   }
   if (row_ok) {
     if (dh0) dh0[m * H + unit] = dhc;
@@ -402,7 +428,7 @@ void lstm_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, co
 // bf16 cells with v_mfma_f32_4x4x4 bf16 (32 per step), for which the state, kept in fp32 in a register of the lane that owns it,
 // is rounded to bf16 on its way to LDS, as the per-step products round their input.  Bound by the latency of a step's chain
 // (LDS read, products, gates, LDS write, barrier); the per-step launches this replaces were four per step and layer (512 rows,
-// 24 steps, bf16: 4 x 24 launches of 3-8 us -> one of 30 us; 40 backward).
+// 24 steps, bf16: 4 x 24 launches of 3-8 us -> one of 27 us; 30 backward).
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 
 __device__ __forceinline__ short bf16_bits(float x) { return __builtin_bit_cast(short, (__bf16)x); }
@@ -518,38 +544,47 @@ void gru_seq_forward_kernel(int T, int64_t M, int groups, const float* __restric
   }
 }
 
-// The reverse sweep (gru_gate_backward_kernel's formulas): dh_{t-1} = dh_t z + d_gh W_hh.  Sixteen blocks = four groups of four units
-// times four quarters of the 3H gate rows, as in the LSTM's sweep.
+// The reverse sweep (gru_gate_backward_kernel's formulas): dh_{t-1} = dh_t z + d_gh W_hh.  Sixteen blocks = four quarters of the 3H gate
+// rows (96 each) times four groups of four units, operands and sums as in the LSTM's sweep; in bf16 a step of four k is one block's entry.
 template <bool BF>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gru_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, const float* __restrict__ saved,
                              const uint8_t* __restrict__ fresh, const void* __restrict__ Wtv, int ldwt, float* __restrict__ d_gi,
                              float* __restrict__ d_gh, float* __restrict__ dh0) {
   constexpr int H = kSeqH, KQ = 3 * H / 4;  // gate rows per quarter
-  constexpr int LDG = BF ? 3 * H + 8 : 3 * H + 4;
   typedef typename std::conditional<BF, short, float>::type G;
-  __shared__ __attribute__((aligned(16))) G sg[kSeqRows][LDG];
+  // what a lane reads (KQ / 4 consecutive entries), padded so that the sixteen lanes of a quarter hit different banks
+  constexpr int LA = BF ? 24 : 28, LR = 16 * LA + (BF ? 64 : 16);
+  __shared__ __attribute__((aligned(16))) G sg[2][kSeqRows * LR];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int j = lane & 3, ug = (lane >> 2) & 3, kg = lane >> 4;
-  const int unit = 16 * wave + 4 * ug + kg;
-  const int64_t m = (int64_t)blockIdx.x * kSeqRows + j;
+  const int kg = lane >> 4, blk = (lane >> 2) & 3, i = lane & 3;
+  const int unit = 16 * wave + (lane & 15);
+  const int64_t m = (int64_t)blockIdx.x * kSeqRows + kg;
   const bool row_ok = m < M;
   const int64_t mc = row_ok ? m : M - 1;
   constexpr int NW = BF ? 1 : KQ, NB = BF ? KQ / 4 : 1;
   float wa[NW];
   s16x4 wb[NB];
   if constexpr (BF) {
-    const s16x4* src = reinterpret_cast<const s16x4*>((const short*)Wtv + (int64_t)(16 * wave + 4 * ug + j) * ldwt + KQ * kg);
+    const s16x4* src = reinterpret_cast<const s16x4*>((const short*)Wtv + (int64_t)unit * ldwt + KQ * kg);
 #pragma unroll
     for (int s4 = 0; s4 < NB; ++s4) wb[s4] = src[s4];
   } else {
-    const float4* src = reinterpret_cast<const float4*>((const float*)Wtv + (int64_t)(16 * wave + 4 * ug + j) * ldwt + KQ * kg);
+    const float4* src = reinterpret_cast<const float4*>((const float*)Wtv + (int64_t)unit * ldwt + KQ * kg);
 #pragma unroll
     for (int s4 = 0; s4 < NW / 4; ++s4) {
       const float4 v = src[s4];
       wa[4 * s4] = v.x; wa[4 * s4 + 1] = v.y; wa[4 * s4 + 2] = v.z; wa[4 * s4 + 3] = v.w;
     }
   }
+  // where gate row g H + unit of this lane's row goes: quarter, block (fp32: k mod 4; bf16: k / 4 mod 4) and place among the block's entries
+  int put[3];
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    const int row = g * H + unit, q = row / KQ, k = row - q * KQ;
+    put[g] = kg * LR + (BF ? (4 * q + ((k >> 2) & 3)) * LA + (k >> 4) * 4 + (k & 3) : (4 * q + (k & 3)) * LA + (k >> 2));
+  }
+  const int get = i * LR + (4 * kg + blk) * LA;
   float dhc = 0.f;
   float nx[6];
   uint8_t fnext = 0;
@@ -561,6 +596,7 @@ void gru_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, con
     nx[5] = dH[o * H + unit];
     if (fresh) fnext = fresh[o];
   }
+  int cur = 0;
   for (int t = T - 1; t >= 0; --t) {
     const bool f = fnext != 0;
     const float r = nx[0], z = nx[1], n = nx[2], hn = nx[3], h = nx[4];
@@ -578,9 +614,9 @@ void gru_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, con
     const float gR = gN * hn * r * (1.f - r);
     const float gNh = gN * r;
     if constexpr (BF) {
-      sg[j][unit] = bf16_bits(gR); sg[j][H + unit] = bf16_bits(gZ); sg[j][2 * H + unit] = bf16_bits(gNh);
+      sg[cur][put[0]] = bf16_bits(gR); sg[cur][put[1]] = bf16_bits(gZ); sg[cur][put[2]] = bf16_bits(gNh);
     } else {
-      sg[j][unit] = gR; sg[j][H + unit] = gZ; sg[j][2 * H + unit] = gNh;
+      sg[cur][put[0]] = gR; sg[cur][put[1]] = gZ; sg[cur][put[2]] = gNh;
     }
     if (row_ok) {
       const int64_t o = ((int64_t)t * M + m) * 3 * H + unit;
@@ -590,34 +626,36 @@ void gru_seq_backward_kernel(int T, int64_t M, const float* __restrict__ dH, con
     lds_barrier();
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
     if constexpr (BF) {
-      const s16x4* grow = reinterpret_cast<const s16x4*>(&sg[j][KQ * kg]);
+      s16x4 ga[6];
+      const s16x4* src = reinterpret_cast<const s16x4*>(&sg[cur][get]);
 #pragma unroll
-      for (int s4 = 0; s4 < NB; s4 += 2) {
-        acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(wb[s4], grow[s4], acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(wb[s4 + 1], grow[s4 + 1], acc1, 0, 0, 0);
+      for (int q = 0; q < 6; ++q) ga[q] = src[q];
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ga[q], wb[4 * q], acc0, 2, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ga[q], wb[4 * q + 1], acc1, 2, 1, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ga[q], wb[4 * q + 2], acc0, 2, 2, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ga[q], wb[4 * q + 3], acc1, 2, 3, 0);
       }
     } else {
-      const float* grow = &sg[j][KQ * kg];
+      float ga[24];
+      const float4* src = reinterpret_cast<const float4*>(&sg[cur][get]);
 #pragma unroll
-      for (int s4 = 0; s4 < NW / 4; ++s4) {
-        const float4 gb = *reinterpret_cast<const float4*>(grow + 4 * s4);
-        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4], gb.x, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 1], gb.y, acc1, 0, 0, 0);
-        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 2], gb.z, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(wa[4 * s4 + 3], gb.w, acc1, 0, 0, 0);
+      for (int q4 = 0; q4 < 6; ++q4) {
+        const float4 v = src[q4];
+        ga[4 * q4] = v.x; ga[4 * q4 + 1] = v.y; ga[4 * q4 + 2] = v.z; ga[4 * q4 + 3] = v.w;
+      }
+#pragma unroll
+      for (int q = 0; q < 24; ++q) {
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q], acc0, 2, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 1], acc1, 2, 1, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 2], acc0, 2, 2, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 3], acc1, 2, 3, 0);
       }
     }
-    float part[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float v = acc0[q] + acc1[q];
-      v += __shfl_xor(v, 16);
-      v += __shfl_xor(v, 32);
-      part[q] = v;
-    }
-    const float mine = kg == 0 ? part[0] : (kg == 1 ? part[1] : (kg == 2 ? part[2] : part[3]));
+    const float mine = rows_reduce_scatter(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3]);
     dhc = f ? 0.f : d * z + mine;
-    lds_barrier();
+    cur ^= 1;
   }
   if (row_ok && dh0) dh0[m * H + unit] = dhc;
 }
