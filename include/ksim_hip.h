@@ -809,6 +809,16 @@ int64_t ks_mlp_disc_workspace_bytes(const KsMlp* mlp, int64_t n_real, int64_t n_
 int ks_mlp_disc_loss_grad(KsMlp* mlp, ks_stream_t stream, int64_t n_real, const float* real, int64_t n_sim, const float* sim,
                           float grad_penalty_coef, int64_t n_motions, float* losses, void* workspace);
 int ks_grad_sqnorm(ks_stream_t stream, int64_t n, const float* g, double* acc);
+/* The env columns of a minibatch (ppo.py:572-694 indexes every array of the rollout with them), `n` arrays in one launch:
+ * dst (outer, picked, inner) from src (outer, columns, inner), inner in bytes, dst[o][j] = src[o][index[j]]; index (picked) device.
+ * An index outside [0, columns) reads the nearest column. */
+#define KS_GATHER_ARRAYS 24
+typedef struct KsGatherArray {
+  const void* src;
+  void* dst;
+  int64_t outer, inner;
+} KsGatherArray;
+int ks_gather_columns(ks_stream_t stream, int32_t n, const KsGatherArray* arrays /*host*/, int64_t columns, int64_t picked, const int64_t* index);
 /* Mirror (left / right symmetry) losses of a task, examples/kbot/train.py:1458-1477, for networks applied to flat rows.
  * A mirror map is a signed permutation: mirrored[j] = sign[j] * x[perm[j]] (mirror_joints / mirror_obs / mirror_cmd,
  * train.py:1565-1760, each negate and reorder entries of their vector).

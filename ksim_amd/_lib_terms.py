@@ -184,6 +184,13 @@ class KsLstmDesc(ctypes.Structure):
                 ("weight_hh", c_void_p), ("bias", c_void_p)]
 
 
+KS_GATHER_ARRAYS = 24
+
+
+class KsGatherArray(ctypes.Structure):
+    _fields_ = [("src", c_void_p), ("dst", c_void_p), ("outer", c_int64), ("inner", c_int64)]
+
+
 class KsAdamParams(ctypes.Structure):
     _fields_ = [("lr", c_float), ("b1", c_float), ("b2", c_float), ("eps", c_float), ("weight_decay", c_float),
                 ("max_grad_norm", c_float), ("step", c_int64)]
@@ -288,6 +295,8 @@ def bind(lib) -> None:
     lib.ks_mlp_disc_loss_grad.restype = c_int32
     lib.ks_mlp_grad_sqnorm.argtypes = [c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_adam_step.argtypes = [c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
+    lib.ks_gather_columns.argtypes = [c_void_p, c_int32, POINTER(KsGatherArray), c_int64, c_int64, c_void_p]
+    lib.ks_gather_columns.restype = c_int32
     lib.ks_mlps_grad_sqnorm.argtypes = [c_void_p, c_int32, c_void_p, c_void_p]
     lib.ks_mlps_adam_step.argtypes = [c_void_p, c_int32, c_void_p, POINTER(KsAdamParams), c_void_p]
     lib.ks_adam_step.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]

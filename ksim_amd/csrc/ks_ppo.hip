@@ -448,6 +448,54 @@ static inline int grid_for(int64_t n, int block, int cap) {
   return (int)g;
 }
 
+// ---------------------------------------------------------------- a minibatch's columns of every array of a trajectory
+// dst[o][j] = src[o][index[j]] for pieces of `inner` bytes, several arrays per launch: the env columns of a minibatch.  An array goes in words
+// as wide as its pieces and pointers allow, four words in flight per thread.  Bound by memory for
+// the observations and by the launch for the small arrays: the thirteen arrays of a K-Bot minibatch (512 of 1024 envs x 100 steps, 230 MB both
+// ways) 130 us in thirteen launches -> 75, the eight of 2048 envs x 32 steps with 68 observations 55 -> 28.
+struct GatherArray {
+  const char* src;
+  char* dst;
+  uint32_t words, inner;  // words in all, words per piece
+  uint32_t log_bytes;     // of a word: 0 .. 4
+  uint32_t first_block;
+};
+struct GatherTable {
+  GatherArray a[KS_GATHER_ARRAYS];
+  int n;
+};
+constexpr int kGatherWords = 1024;  // per workgroup
+
+template <typename T>
+__device__ __forceinline__ void gather_words(const GatherArray& a, int64_t columns, uint32_t picked, const int64_t* __restrict__ index) {
+  const T* src = reinterpret_cast<const T*>(a.src);
+  T* dst = reinterpret_cast<T*>(a.dst);
+  const uint32_t base = (blockIdx.x - a.first_block) * kGatherWords + threadIdx.x;
+  T v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t w = min(base + 256 * k, a.words - 1), piece = w / a.inner, c = w - piece * a.inner, o = piece / picked;
+    const int64_t at = index[piece - o * picked];
+    v[k] = src[((int64_t)o * columns + min(max(at, (int64_t)0), columns - 1)) * a.inner + c];  // an index outside the array stays inside it
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (base + 256 * k < a.words) dst[base + 256 * k] = v[k];
+}
+
+__global__ __launch_bounds__(256) void gather_columns_kernel(GatherTable t, int64_t columns, uint32_t picked, const int64_t* __restrict__ index) {
+  int e = 0;
+  while (e + 1 < t.n && blockIdx.x >= t.a[e + 1].first_block) ++e;
+  const GatherArray& a = t.a[e];
+  switch (a.log_bytes) {
+    case 4: gather_words<uint4>(a, columns, picked, index); break;
+    case 3: gather_words<uint2>(a, columns, picked, index); break;
+    case 2: gather_words<uint32_t>(a, columns, picked, index); break;
+    case 1: gather_words<uint16_t>(a, columns, picked, index); break;
+    default: gather_words<uint8_t>(a, columns, picked, index);
+  }
+}
+
 }  // namespace ks
 
 using namespace ks;
@@ -1234,4 +1282,31 @@ extern "C" int ks_ppo_loss_grad_mixture(ks_stream_t stream, int64_t M, int32_t n
                                : ks::ppo_loss_grad_pairs_kernel<ks::MixturePair<KS_MAX_MIXTURES>, KsMixtureHead>);
   hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, M, nu, *params, *head, raw, io, d_raw);
   return ks::check_launch("ks_ppo_loss_grad_mixture");
+}
+
+extern "C" int ks_gather_columns(ks_stream_t stream, int32_t n, const KsGatherArray* arrays, int64_t columns, int64_t picked, const int64_t* index) {
+  if (n < 0 || (n > 0 && !arrays) || columns < 0 || picked < 0) return ks::fail(KS_EINVAL, "ks_gather_columns: bad argument");
+  if (n > KS_GATHER_ARRAYS) return ks::fail(KS_ELIMIT, "ks_gather_columns: %d arrays (0..%d)", n, KS_GATHER_ARRAYS);
+  if (picked > 0 && (columns == 0 || !index)) return ks::fail(KS_EINVAL, "ks_gather_columns: nothing to pick from");
+  if (picked > 0x7fffffff) return ks::fail(KS_ELIMIT, "ks_gather_columns: too many columns");
+  ks::GatherTable t;
+  t.n = 0;
+  int64_t blocks = 0;
+  for (int k = 0; k < n; ++k) {
+    const KsGatherArray& a = arrays[k];
+    if (a.outer < 0 || a.inner < 0) return ks::fail(KS_EINVAL, "ks_gather_columns: array %d: negative size", k);
+    if (a.outer == 0 || a.inner == 0 || picked == 0) continue;
+    if (!a.src || !a.dst) return ks::fail(KS_EINVAL, "ks_gather_columns: array %d: null pointer", k);
+    const uint64_t bits = (uint64_t)(uintptr_t)a.src | (uint64_t)(uintptr_t)a.dst | (uint64_t)a.inner;
+    uint32_t lb = 0;
+    while (lb < 4 && !(bits >> lb & 1)) ++lb;
+    const int64_t inner = a.inner >> lb;
+    if (a.outer > 0xffffffffll / inner / picked) return ks::fail(KS_ELIMIT, "ks_gather_columns: array %d is too large", k);
+    const int64_t words = a.outer * inner * picked;
+    t.a[t.n++] = {(const char*)a.src, (char*)a.dst, (uint32_t)words, (uint32_t)inner, lb, (uint32_t)blocks};
+    blocks += (words + ks::kGatherWords - 1) / ks::kGatherWords;
+  }
+  if (t.n == 0) return KS_OK;
+  hipLaunchKernelGGL(ks::gather_columns_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, t, columns, (uint32_t)picked, index);
+  return ks::check_launch("ks_gather_columns");
 }

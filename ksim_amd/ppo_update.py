@@ -11,6 +11,7 @@ Trajectories are time-major (T, N, ...), the rollout buffers' own layout; a mini
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass, field
 from typing import Sequence
 
@@ -208,6 +209,29 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     return metrics
 
 
+def _columns(idx: torch.Tensor, own: bool, arrays: Sequence[tuple[torch.Tensor | None, int]]) -> list:
+    """The env columns `idx` of every (array, env axis), contiguous, in one launch.  Only for indices that were drawn here (`own`): a caller's are
+    checked where torch checks them, as are arrays that are not plain contiguous device memory."""
+    N = next(t.shape[d] for t, d in arrays if t is not None)
+    picked, out = idx.numel(), [None] * len(arrays)
+    table, keep = [], idx.contiguous()
+    for k, (t, d) in enumerate(arrays):
+        if t is None:
+            continue
+        if not own or t.shape[d] != N or not t.is_contiguous() or not t.is_cuda or t.requires_grad or len(table) == T.KS_GATHER_ARRAYS:
+            out[k] = t.index_select(d, idx).contiguous()
+            continue
+        shape = list(t.shape)
+        shape[d] = picked
+        out[k] = torch.empty(shape, dtype=t.dtype, device=t.device)
+        inner = t.stride(d) * t.element_size()
+        table.append(T.KsGatherArray(t.data_ptr(), out[k].data_ptr(), math.prod(shape[:d]), inner))
+    if table:
+        rc = _lib.load().ks_gather_columns(_lib.current_stream(), len(table), (T.KsGatherArray * len(table))(*table), N, picked, keep.data_ptr())
+        _lib.check(rc)
+    return out
+
+
 def update_model(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, critic_obs, action, rewards, done, success,
                  permutations: list[torch.Tensor] | None = None, seed: int = 0, after_step=None) -> list[dict]:
     """num_passes x (N / batch_size) minibatch steps over a (T, N) rollout (ppo.py:572-694).
@@ -233,9 +257,8 @@ def update_model(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, cri
     for k in range(cfg.num_passes):
         perm = permutations[k] if permutations is not None else torch.randperm(N, generator=gen, device=done.device)
         for idx in perm.view(-1, bs):
-            sel = lambda t: t.index_select(1, idx).contiguous()  # noqa: E731
-            out.append(single_step(policy, cfg, sel(actor_obs), sel(critic_obs), sel(action), sel(rewards), sel(done),
-                                   sel(success), sel(on_lp), sel(on_v)))
+            arrays = (actor_obs, critic_obs, action, rewards, done, success, on_lp, on_v)
+            out.append(single_step(policy, cfg, *_columns(idx, permutations is None, [(t, 1) for t in arrays])))
             if after_step is not None:
                 out[-1]["after_step"] = after_step(idx)
     return out
@@ -477,12 +500,8 @@ def update_model_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, ac
     for k in range(cfg.num_passes):
         perm = permutations[k] if permutations is not None else torch.randperm(N, generator=gen, device=done.device)
         for idx in perm.view(-1, bs):
-            sel = lambda t: t.index_select(1, idx).contiguous()  # noqa: E731
-            ca = actor_carry0.index_select(env_axis[actor_carry0.dim() == 4], idx).contiguous()
-            cc = critic_carry0.index_select(env_axis[critic_carry0.dim() == 4], idx).contiguous()
-            env_sel = lambda c: None if c is None else c.index_select(env_axis[c.dim() == 4], idx).contiguous()  # noqa: E731
-            rows_sel = lambda c: None if c is None else c.index_select(0, idx).contiguous()  # noqa: E731
-            out.append(single_step_recurrent(policy, cfg, sel(actor_obs), sel(critic_obs), sel(action), sel(rewards), sel(done),
-                                             sel(success), sel(on_lp), sel(on_v), ca, cc, sel(fresh), rows_sel(lpf0),
-                                             MirrorCarries(env_sel(mc.actor), env_sel(mc.critic), rows_sel(mc.lpf))))
+            arrays = [(t, 1) for t in (actor_obs, critic_obs, action, rewards, done, success, on_lp, on_v)]
+            arrays += [(c, None if c is None else env_axis[c.dim() == 4]) for c in (actor_carry0, critic_carry0, mc.actor, mc.critic)]
+            *steps, ca, cc, ma, mcc, fr, l0, ml = _columns(idx, permutations is None, arrays + [(fresh, 1), (lpf0, 0), (mc.lpf, 0)])
+            out.append(single_step_recurrent(policy, cfg, *steps, ca, cc, fr, l0, MirrorCarries(ma, mcc, ml)))
     return out

@@ -808,3 +808,29 @@ def test_weight_gradients_over_row_counts_that_slices_do_not_divide(dims, dtype,
         assert torch.isfinite(b).all()
         # the same products in another order of sums of up to M0 terms: 2^-24 of a partial sum per addition, as a random walk
         assert (a - b).abs().max() <= 8 * 2.0 ** -24 * np.sqrt(M0) * max(float(a.abs().max()), 1e-3), (a - b).abs().max()
+
+
+@pytest.mark.parametrize("T_,N,picked", [(1, 1, 1), (5, 7, 3), (3, 300, 300), (33, 130, 65), (2, 64, 1), (4, 9, 0), (0, 4, 2)])
+def test_minibatch_columns_equal_index_select(T_, N, picked):
+    """Every word width (1 to 16 bytes), pointers aligned to less than the pieces, an env axis that is not the second, None, and arrays that
+    fall back (strided, on other env counts); the index drawn here or the caller's."""
+    from ksim_amd.ppo_update import _columns
+
+    gen = torch.Generator(device="cuda").manual_seed(T_ * 1000 + N)
+    raw = lambda *s: torch.randint(0, 255, s, device="cuda", generator=gen, dtype=torch.uint8)  # noqa: E731
+    arrays = [(raw(T_, N), 1), (raw(T_, N) > 128, 1), (raw(T_, N, 3), 1), (raw(T_, N, 2).view(torch.float16), 1), (torch.randn(T_, N, 1, device="cuda"), 1)]
+    for inner in (2, 4, 5, 6, 128, 475):
+        arrays.append((torch.randn(T_, N, inner, device="cuda"), 1))
+        flat = torch.randn(T_ * N * inner + 3, device="cuda")
+        arrays.append((flat[3:].view(T_, N, inner), 1))  # 4-byte aligned only
+    arrays += [(torch.randn(2, 2, N, 128, device="cuda"), 2), (torch.randn(N, 20, device="cuda"), 0), (None, None), (torch.randn(2, N, 64, device="cuda"), 1),
+               (torch.randn(T_, N, 8, device="cuda").transpose(0, 1).contiguous().transpose(0, 1), 1), (torch.randn(T_, N + 5, 3, device="cuda"), 1)]
+    idx = torch.randperm(N, device="cuda", generator=gen)[:picked]
+    for own in (True, False):
+        for (t, d), got in zip(arrays, _columns(idx, own, arrays)):
+            if t is None:
+                assert got is None
+                continue
+            want = t.index_select(d, idx)
+            assert got.shape == want.shape and got.dtype == want.dtype and got.is_contiguous()
+            assert torch.equal(got.view(torch.uint8) if got.dtype != torch.bool else got, want.contiguous().view(torch.uint8) if got.dtype != torch.bool else want)
