@@ -906,6 +906,18 @@ int ks_lstm_backward_step(KsLstm* lstm, ks_stream_t stream, int64_t M, const flo
                           const float* saved, const uint8_t* fresh, float* d_g, float* dh_in, float* dc_in, void* workspace);
 int ks_lstm_grad_sqnorm(const KsLstm* lstm, ks_stream_t stream, double* acc);
 int ks_lstm_adam_step(KsLstm* lstm, ks_stream_t stream, const KsAdamParams* params /*host*/, const double* sqnorm);
+/* One recurrent layer over a trajectory, as the entry points below that end in _sequences_ take it: `n` (1 or 2) layers of one kind, precision and
+ * step count in one launch, e.g. the actor's and the critic's of one depth; their operands are those of the entry points for one layer. */
+typedef struct KsSequence {
+  const void* cell; /* KsGru or KsLstm */
+  int64_t M;
+  const float* in;      /* forward: gi; backward: dH */
+  const float *h0, *c0; /* forward (c0: LSTM) */
+  const uint8_t* fresh;
+  float* saved;       /* forward: written where given; backward: read */
+  float *out0, *out1; /* forward: hs, cs (LSTM, nullable); backward: d_g (LSTM) or d_gi, d_gh (GRU) */
+  float *dh0, *dc0;   /* backward, nullable */
+} KsSequence;
 /* A whole trajectory of one GRU layer in one launch each way, for cells of hidden size 128 in either precision
  * (ks_gru_sequence_supported returns 1; other cells take the step-by-step entry points).  gi (T, M, 3H) = W_ih x_t + bias for every
  * step; hs (T, M, H), saved (T, M, 5H) nullable, in the layout of ks_gru_train_forward; with T = 1, hs may alias h0, and
@@ -917,6 +929,8 @@ int ks_gru_sequence_forward(const KsGru* gru, ks_stream_t stream, int64_t T, int
                             const uint8_t* fresh, float* hs, float* saved);
 int ks_gru_sequence_backward(const KsGru* gru, ks_stream_t stream, int64_t T, int64_t M, const float* dH, const float* saved,
                              const uint8_t* fresh, float* d_gi, float* d_gh, float* dh0);
+int ks_gru_sequences_forward(ks_stream_t stream, int32_t n, int64_t T, const KsSequence* layers /*host*/);
+int ks_gru_sequences_backward(ks_stream_t stream, int32_t n, int64_t T, const KsSequence* layers /*host*/);
 /* A whole trajectory of one LSTM layer in one launch each way: the lax.scan over the T steps of the trajectory inside the loss
  * (ksim/task/ppo.py:572-694 around the model's forward, examples/kbot/train.py:903-915) and what jax.grad derives for it, for
  * fp32 cells of hidden size 128 (ks_lstm_sequence_supported returns 1; other cells take the step-by-step entry points above).
@@ -936,6 +950,8 @@ int ks_lstm_sequence_forward(const KsLstm* lstm, ks_stream_t stream, int64_t T, 
                              const float* c0, const uint8_t* fresh, float* hs, float* cs, float* saved);
 int ks_lstm_sequence_backward(const KsLstm* lstm, ks_stream_t stream, int64_t T, int64_t M, const float* dH, const float* saved,
                               const uint8_t* fresh, float* d_g, float* dh0, float* dc0);
+int ks_lstm_sequences_forward(ks_stream_t stream, int32_t n, int64_t T, const KsSequence* layers /*host*/);
+int ks_lstm_sequences_backward(ks_stream_t stream, int32_t n, int64_t T, const KsSequence* layers /*host*/);
 
 /* Gaussian policy head and the gradient of the PPO objective (ppo.py:149-246, total 473-486):
  *   ks_gaussian_log_prob: per action dimension log N(action; mean, exp(log_std)) and entropy

@@ -184,6 +184,10 @@ class KsLstmDesc(ctypes.Structure):
                 ("weight_hh", c_void_p), ("bias", c_void_p)]
 
 
+class KsSequence(ctypes.Structure):
+    _fields_ = [("cell", c_void_p), ("M", c_int64)] + [(n, c_void_p) for n in ("in_", "h0", "c0", "fresh", "saved", "out0", "out1", "dh0", "dc0")]
+
+
 KS_GATHER_ARRAYS = 24
 
 
@@ -295,6 +299,9 @@ def bind(lib) -> None:
     lib.ks_mlp_disc_loss_grad.restype = c_int32
     lib.ks_mlp_grad_sqnorm.argtypes = [c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_adam_step.argtypes = [c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]
+    for name in ("ks_gru_sequences_forward", "ks_gru_sequences_backward", "ks_lstm_sequences_forward", "ks_lstm_sequences_backward"):
+        getattr(lib, name).argtypes = [c_void_p, c_int32, c_int64, POINTER(KsSequence)]
+        getattr(lib, name).restype = c_int32
     lib.ks_gather_columns.argtypes = [c_void_p, c_int32, POINTER(KsGatherArray), c_int64, c_int64, c_void_p]
     lib.ks_gather_columns.restype = c_int32
     lib.ks_mlps_grad_sqnorm.argtypes = [c_void_p, c_int32, c_void_p, c_void_p]

@@ -23,6 +23,7 @@ from . import ppo as ppo_mod
 from .actions import LowPass
 from . import mlp as mlp_mod
 from .mlp import MLP
+from .recurrent import lockstep
 
 
 @dataclass
@@ -376,8 +377,9 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
     a_in = both(actor_obs, "actor_obs") if mirror_a else actor_obs.contiguous()
     c_in = both(critic_obs, "critic_obs") if mirror_c else critic_obs.contiguous()
     a_fresh, c_fresh = (fresh2 if mirror_a else fresh), (fresh2 if mirror_c else fresh)
-    raw_all = policy.actor.train_forward(a_in, _cat_env(actor_carry0, mc.actor) if mirror_a else actor_carry0, a_fresh)
-    value_all = policy.critic.train_forward(c_in, _cat_env(critic_carry0, mc.critic) if mirror_c else critic_carry0, c_fresh)
+    raw_all, value_all = lockstep(
+        policy.actor.train_forward_pass(a_in, _cat_env(actor_carry0, mc.actor) if mirror_a else actor_carry0, a_fresh),
+        policy.critic.train_forward_pass(c_in, _cat_env(critic_carry0, mc.critic) if mirror_c else critic_carry0, c_fresh))
     y0 = None
     if policy.lowpass is not None:
         y0 = lpf0 if lpf0 is not None else torch.zeros(b, nu, dtype=torch.float32, device=dev)
@@ -433,8 +435,7 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
         lp_ = policy.lowpass
         _lib.check(lib.ks_lowpass_scan_backward(st, Tn, d_raw_all.shape[1], nu, 2 * nu, float(lp_.ctrl_dt), float(lp_.cutoff_frequency),
                                                 _lib.ptr(a_fresh), _lib.ptr(d_raw_all), None))
-    policy.actor.backward(d_raw_all)
-    policy.critic.backward(d_value_all)
+    lockstep(policy.actor.backward_pass(d_raw_all), policy.critic.backward_pass(d_value_all))
     sq = torch.zeros(1, dtype=torch.float64, device=dev)
     nets = policy.actor.networks() + policy.critic.networks()
     mlp_mod.grad_sqnorm(nets, sq)
@@ -464,8 +465,8 @@ def recurrent_on_policy(policy: RecurrentHeadPolicy, actor_obs, critic_obs, acti
     update_model makes once over the whole rollout before any minibatch step (ppo.py:603-607).  With `return_raw` also the
     head's input rows (T, N, width), locations filtered where the policy filters them."""
     Tn, N, nu = action.shape
-    raw = policy.actor.forward_sequence(actor_obs, actor_carry0, fresh)
-    values = policy.critic.forward_sequence(critic_obs, critic_carry0, fresh)
+    raw, values = lockstep(policy.actor.forward_sequence_pass(actor_obs, actor_carry0, fresh),
+                           policy.critic.forward_sequence_pass(critic_obs, critic_carry0, fresh))
     if policy.lowpass is not None:
         raw = actor_locations(policy, raw, actor_obs.contiguous(), fresh.contiguous(), lpf0)
     lp = torch.empty(Tn, N, nu, dtype=torch.float32, device=action.device)

@@ -28,6 +28,43 @@ def _f32(a) -> np.ndarray:
     return np.ascontiguousarray(a.detach().cpu().numpy() if isinstance(a, torch.Tensor) else a, dtype=np.float32)
 
 
+class SequenceCall:
+    """The recurrence of one layer over a trajectory, ready to launch; holds what the launch reads and writes."""
+
+    def __init__(self, entry: str, dtype: str, steps: int, rows: int, handle, x, h0, c0, fresh, saved, out0, out1):
+        self.key, self.steps, self.rows, self.handle = (entry, dtype, steps), steps, rows, handle
+        self.tensors = (x, h0, c0, fresh, saved, out0, out1)
+
+    def record(self) -> "T.KsSequence":
+        return T.KsSequence(self.handle.value, self.rows, *map(_lib.addr, self.tensors), None, None)
+
+
+def run_sequences(calls: Sequence[SequenceCall]) -> None:
+    """Launches the calls: two of one kind, precision and length (a layer of the actor and one of the critic) together, which keeps a chip busy
+    that either of them fills halfway; others one after the other."""
+    lib, stream = _lib.load(), _lib.current_stream()
+    calls = list(calls)
+    while calls:
+        n = 2 if len(calls) > 1 and calls[0].key == calls[1].key else 1
+        _lib.check(getattr(lib, calls[0].key[0])(stream, n, calls[0].steps, (T.KsSequence * n)(*(c.record() for c in calls[:n]))))
+        del calls[:n]
+
+
+def lockstep(*passes):
+    """Runs generators that yield the `SequenceCall`s of their layers side by side, launching what they yield together; returns their results."""
+    results, live = [None] * len(passes), list(range(len(passes)))
+    while live:
+        calls = []
+        for k in tuple(live):
+            try:
+                calls.append(next(passes[k]))
+            except StopIteration as stop:
+                results[k] = stop.value
+                live.remove(k)
+        run_sequences(calls)
+    return results
+
+
 class GRUCell:
     """h' = GRU(x, h) for N envs at once (`ks_gru_forward`)."""
 
@@ -120,9 +157,8 @@ class GRUCell:
             self._proj = MLP._borrow(self._lib, pi, (self.input_size, 3 * self.hidden_size), self.dtype)
         return self._proj
 
-    def sequence_forward(self, x, h0, fresh, hs, saved) -> None:
-        """The layer over a whole trajectory: x (T, M, input) -> hs (T, M, H) and `saved` (T, M, 5H; None where no backward
-        pass follows), from the carry h0; the input projection is one product over all T M rows, the recurrence one launch."""
+    def sequence_call(self, x, h0, fresh, hs, saved) -> "SequenceCall":
+        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`)."""
         _lib.require_cuda(x, h0, hs, saved, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
@@ -130,19 +166,26 @@ class GRUCell:
                 or (saved is not None and tuple(saved.shape) != (Tn, M, 5 * H)) or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected x (T, M, input), h0 (M, H), hs (T, M, H), saved (T, M, 5H), fresh (T, M)")
         gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
-        _lib.check(self._lib.ks_gru_sequence_forward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(gi), _lib.ptr(h0),
-                                                     _lib.ptr(fresh), _lib.ptr(hs), _lib.ptr(saved)))
+        return SequenceCall("ks_gru_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, None, fresh, saved, hs, None)
 
-    def sequence_backward(self, dH, saved, fresh, d_gi, d_gh) -> None:
-        """The reverse sweep over the trajectory: dH (T, M, H), the gradient reaching every h_t from above, -> d_gi, d_gh (T, M, 3H)."""
+    def sequence_forward(self, x, h0, fresh, hs, saved) -> None:
+        """The layer over a whole trajectory: x (T, M, input) -> hs (T, M, H) and `saved` (T, M, 5H; None where no backward
+        pass follows), from the carry h0; the input projection is one product over all T M rows, the recurrence one launch."""
+        run_sequences([self.sequence_call(x, h0, fresh, hs, saved)])
+
+    def sequence_backward_call(self, dH, saved, fresh, d_gi, d_gh) -> "SequenceCall":
+        """`sequence_backward`, checked; the caller makes the launch (`run_sequences`)."""
         _lib.require_cuda(dH, saved, d_gi, d_gh, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = dH.shape[0], dH.shape[1], self.hidden_size
         if (tuple(dH.shape) != (Tn, M, H) or tuple(saved.shape) != (Tn, M, 5 * H) or tuple(d_gi.shape) != (Tn, M, 3 * H)
                 or tuple(d_gh.shape) != (Tn, M, 3 * H) or tuple(fresh.shape) != (Tn, M)):
-            raise _lib.KsError("expected dH (T, M, H), saved (T, M, 5H), d_gi, d_gh (T, M, 3H), fresh (T, M)")
-        _lib.check(self._lib.ks_gru_sequence_backward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(dH), _lib.ptr(saved),
-                                                      _lib.ptr(fresh), _lib.ptr(d_gi), _lib.ptr(d_gh), None))
+            raise _lib.KsError("expected dH (T, M, H), saved (T, M, 5H), d_gi and d_gh (T, M, 3H), fresh (T, M)")
+        return SequenceCall("ks_gru_sequences_backward", self.dtype, Tn, M, self._handle, dH, None, None, fresh, saved, d_gi, d_gh)
+
+    def sequence_backward(self, dH, saved, fresh, d_gi, d_gh) -> None:
+        """The reverse sweep over the trajectory: dH (T, M, H), the gradient reaching every h_t from above, -> d_gi, d_gh (T, M, 3H)."""
+        run_sequences([self.sequence_backward_call(dH, saved, fresh, d_gi, d_gh)])
 
     def backward_step(self, dh_out, saved, fresh, d_gi, d_gh, dh_in) -> None:
         """One step of the backward pass through time: dh_out (M, H) -> d_gi, d_gh (M, 3H) and dh_in (M, H)."""
@@ -265,10 +308,8 @@ class LSTMCell:
             self._proj = MLP._borrow(self._lib, pi, (self.input_size, 4 * self.hidden_size), self.dtype)
         return self._proj
 
-    def sequence_forward(self, x, h0, c0, fresh, hs, cs, saved) -> None:
-        """The layer over a whole trajectory: x (T, M, input) -> hs, cs (T, M, H) and `saved` (T, M, 7H), from the carry
-        (h0, c0); the input projection is one product over all T M rows, the recurrence one launch.  `cs` and `saved` may be
-        None where no backward pass follows."""
+    def sequence_call(self, x, h0, c0, fresh, hs, cs, saved) -> "SequenceCall":
+        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`)."""
         _lib.require_cuda(x, h0, c0, hs, cs, saved, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
@@ -277,19 +318,27 @@ class LSTMCell:
                 or (saved is not None and tuple(saved.shape) != (Tn, M, 7 * H)) or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected x (T, M, input), h0, c0 (M, H), hs, cs (T, M, H), saved (T, M, 7H), fresh (T, M)")
         gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
-        _lib.check(self._lib.ks_lstm_sequence_forward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(gi), _lib.ptr(h0),
-                                                      _lib.ptr(c0), _lib.ptr(fresh), _lib.ptr(hs), _lib.ptr(cs), _lib.ptr(saved)))
+        return SequenceCall("ks_lstm_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, c0, fresh, saved, hs, cs)
 
-    def sequence_backward(self, dH, saved, fresh, d_g) -> None:
-        """The reverse sweep over the trajectory: dH (T, M, H), the gradient reaching every h_t from above, -> d_g (T, M, 4H)."""
+    def sequence_forward(self, x, h0, c0, fresh, hs, cs, saved) -> None:
+        """The layer over a whole trajectory: x (T, M, input) -> hs, cs (T, M, H) and `saved` (T, M, 7H), from the carry
+        (h0, c0); the input projection is one product over all T M rows, the recurrence one launch.  `cs` and `saved` may be
+        None where no backward pass follows."""
+        run_sequences([self.sequence_call(x, h0, c0, fresh, hs, cs, saved)])
+
+    def sequence_backward_call(self, dH, saved, fresh, d_g) -> "SequenceCall":
+        """`sequence_backward`, checked; the caller makes the launch (`run_sequences`)."""
         _lib.require_cuda(dH, saved, d_g, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = dH.shape[0], dH.shape[1], self.hidden_size
         if (tuple(dH.shape) != (Tn, M, H) or tuple(saved.shape) != (Tn, M, 7 * H) or tuple(d_g.shape) != (Tn, M, 4 * H)
                 or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected dH (T, M, H), saved (T, M, 7H), d_g (T, M, 4H), fresh (T, M)")
-        _lib.check(self._lib.ks_lstm_sequence_backward(self._handle, _lib.current_stream(), Tn, M, _lib.ptr(dH), _lib.ptr(saved),
-                                                       _lib.ptr(fresh), _lib.ptr(d_g), None, None))
+        return SequenceCall("ks_lstm_sequences_backward", self.dtype, Tn, M, self._handle, dH, None, None, fresh, saved, d_g, None)
+
+    def sequence_backward(self, dH, saved, fresh, d_g) -> None:
+        """The reverse sweep over the trajectory: dH (T, M, H), the gradient reaching every h_t from above, -> d_g (T, M, 4H)."""
+        run_sequences([self.sequence_backward_call(dH, saved, fresh, d_g)])
 
     def backward_step(self, dh_out, dc_out, saved, fresh, d_g, dh_in, dc_in) -> None:
         """One step of the backward pass through time: (dh_out, dc_out) -> d_g (M, 4H), dh_in, dc_in (M, H)."""
@@ -366,6 +415,10 @@ class RecurrentNetwork:
         return self.output_proj(x, out=out)
 
     def forward_sequence(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor) -> torch.Tensor:
+        """`forward_sequence_pass` by itself."""
+        return lockstep(self.forward_sequence_pass(obs, carry0, fresh))[0]
+
+    def forward_sequence_pass(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor):
         """The network over a trajectory without keeping anything for a backward pass: obs (T, M, in), carry0 the carry of the
         first step (left as it is), fresh (T, M) uint8 -> (T, M, out).  The same numbers as T calls, one control step each.  Long
         trajectories go through in stretches of `SEQUENCE_ROWS` rows, whole steps, each from the carry the last one left."""
@@ -390,7 +443,7 @@ class RecurrentNetwork:
                 states = [torch.empty(n, M, H, dtype=torch.float32, device=obs.device)]
                 if self.lstm:  # the cell state only where another stretch starts from it
                     states.append(torch.empty_like(states[0]) if t0 + n < T_ else None)
-                cell.sequence_forward(x, *carry[i], fresh[t0:t0 + n], *states, None)
+                yield cell.sequence_call(x, *carry[i], fresh[t0:t0 + n], *states, None)
                 x = states[0]
                 if t0 + n < T_:
                     carry[i] = tuple(s[-1].clone() for s in states)
@@ -405,6 +458,10 @@ class RecurrentNetwork:
         self.output_proj.train_init()
 
     def train_forward(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor) -> torch.Tensor:
+        """`train_forward_pass` by itself."""
+        return lockstep(self.train_forward_pass(obs, carry0, fresh))[0]
+
+    def train_forward_pass(self, obs: torch.Tensor, carry0: torch.Tensor, fresh: torch.Tensor):
         """The network over a trajectory, obs (T, M, in), starting from carry0 (the rollout's carry layout); envs flagged
         in fresh (T, M) uint8 start an episode at that step (their carry is zero there).  Returns (T, M, out) and keeps
         what `backward` needs.  This is the scan over time inside the loss of PPOTask._single_step
@@ -424,14 +481,14 @@ class RecurrentNetwork:
             sv = torch.empty(T_, M, (7 if self.lstm else 5) * H, dtype=torch.float32, device=dev)
             if self.lstm and getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
                 cs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
-                cell.sequence_forward(x, carry0[i, 0], carry0[i, 1], fresh, hs, cs, sv)
+                yield cell.sequence_call(x, carry0[i, 0], carry0[i, 1], fresh, hs, cs, sv)
             elif self.lstm:
                 cs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
                 for t in range(T_):
                     h0, c0 = (carry0[i, 0], carry0[i, 1]) if t == 0 else (hs[t - 1], cs[t - 1])
                     cell.train_forward(x[t], h0, c0, fresh[t], hs[t], cs[t], sv[t])
             elif getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
-                cell.sequence_forward(x, carry0[i], fresh, hs, sv)
+                yield cell.sequence_call(x, carry0[i], fresh, hs, sv)
             else:
                 for t in range(T_):
                     cell.train_forward(x[t], carry0[i] if t == 0 else hs[t - 1], fresh[t], hs[t], sv[t])
@@ -443,6 +500,10 @@ class RecurrentNetwork:
         return out
 
     def backward(self, d_out: torch.Tensor) -> None:
+        """`backward_pass` by itself."""
+        lockstep(self.backward_pass(d_out))
+
+    def backward_pass(self, d_out: torch.Tensor):
         """Gradients of sum(d_out * output) with respect to every parameter, into the handles (the jax.grad through the
         scan).  Per layer, top to bottom: a sweep over the steps, last to first, that carries the gradient of the
         recurrent state, then one pass over all (step, env) rows for the weight gradients and the gradient of the layer's
@@ -462,9 +523,9 @@ class RecurrentNetwork:
             d_gh = d_gi if self.lstm else torch.empty(T_, M, G * H, dtype=torch.float32, device=dev)
             fused = cell.sequence_supported
             if fused and self.lstm:
-                cell.sequence_backward(dH, sv, tp["fresh"], d_gi)
+                yield cell.sequence_backward_call(dH, sv, tp["fresh"], d_gi)
             elif fused:
-                cell.sequence_backward(dH, sv, tp["fresh"], d_gi, d_gh)
+                yield cell.sequence_backward_call(dH, sv, tp["fresh"], d_gi, d_gh)
             else:
                 carry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)   # gradient of the hidden state, ping-pong
                 ccarry = torch.zeros(2, M, H, dtype=torch.float32, device=dev)  # and of the cell state (LSTM)

@@ -437,3 +437,37 @@ def test_sequence_without_a_backward_pass_is_bounded_in_memory(kind, monkeypatch
     net.forward_sequence(obs, carry, fresh)
     # the output, and for each row of a stretch the input, projected input, hidden and cell state of a layer and the next layer's
     assert torch.cuda.max_memory_allocated() - before <= Tn * M * 7 * 4 + recurrent.SEQUENCE_ROWS * (4 + G) * H * 4 + (1 << 24)
+
+
+@pytest.mark.parametrize("kind,dtype", [("lstm", "f32"), ("gru", "f32"), ("gru", "bf16")])
+@pytest.mark.parametrize("rows,steps", [((1, 6), 3), ((1030, 37), 5), ((4, 1), 2), ((2500, 8), 1)])
+def test_two_layers_in_one_launch_match_one_by_one(kind, dtype, rows, steps):
+    """The actor's and the critic's layer of a depth share a launch: other weights, other row counts (ragged sets of 4), several sets
+    per workgroup for the short call, against the same layers launched by themselves, forward and backward, bit for bit."""
+    from ksim_amd.recurrent import GRUCell, LSTMCell, run_sequences
+
+    H, G, S = 128, 4 if kind == "lstm" else 3, 7 if kind == "lstm" else 5
+    rng = np.random.default_rng(sum(rows) + steps)
+    cells, forward, backward, want = [], [], [], []
+    for M in rows:
+        w = [rng.normal(scale=H ** -0.5, size=s) for s in ((G * H, H), (G * H, H), (G * H,))]
+        cell = LSTMCell(*w, dtype=dtype) if kind == "lstm" else GRUCell(*w, 0.1 * rng.normal(size=H), dtype=dtype)
+        cell.train_init()
+        t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+        x, h0, c0, dH = t(steps, M, H), t(M, H), t(M, H), t(steps, M, H)
+        fresh = torch.from_numpy((rng.random((steps, M)) < 0.2).astype(np.uint8)).cuda()
+        z = lambda n: torch.full((steps, M, n), 3.0, device="cuda")  # noqa: E731
+        state = lambda: (z(H), z(H), z(S * H)) if kind == "lstm" else (z(H), z(S * H))  # noqa: E731
+        grads = lambda: (z(G * H),) if kind == "lstm" else (z(G * H), z(G * H))  # noqa: E731
+        carry = (h0, c0) if kind == "lstm" else (h0,)
+        (*a, sa), (*b, sb), ga, gb = state(), state(), grads(), grads()
+        cell.sequence_forward(x, *carry, fresh, *a, sa)
+        cell.sequence_backward(dH, sa, fresh, *ga)
+        forward.append(cell.sequence_call(x, *carry, fresh, *b, sb))
+        backward.append(cell.sequence_backward_call(dH, sb, fresh, *gb))
+        want += zip((*a, sa, *ga), (*b, sb, *gb))
+        cells.append(cell)
+    run_sequences(forward)
+    run_sequences(backward)
+    for k, (a, b) in enumerate(want):
+        assert torch.equal(a, b), k
