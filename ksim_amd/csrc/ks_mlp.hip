@@ -2935,25 +2935,32 @@ enum { kEpiStore,    // C (+)= v
        kEpiDelta,    // C = v, C2 = f'(Y) v: a_l and d_l of the input gradient's chain
        kEpiPenalty,  // C = scale v, and the tile's sum of v^2 to sums[tile]: the penalty's gradient and value
        kEpiTangent,  // C = f'(Y) v, C2 = f''(Y) X v: v_l and r_l of the sweep back through that chain
-       kEpiDz };     // C = f'(Y) v (+ X on the first x_rows rows): the ordinary backward pass
+       kEpiDz,       // C = f'(Y) v (+ X on the first x_rows rows): the ordinary backward pass
+       kEpiTop,      // C = act(v + bias_j) =: y and, on the first x_rows rows, C2 = X_j, C3 = f'(y) X_j: the last hidden layer, whose input
+                     // gradient starts from the output layer's one row of weights X
+       kEpiOut };    // the output layer, N = 1: C = v + bias - target, the gradient of the squared error (target 1 on the first x_rows rows, where
+                     // C2 = 1 too, and -1 on the others)
 struct SgemmArgs {
   int M, N, K;
   const float *A, *A2;  // A2: rows (or, stored (k, i), reduction steps) from a_split on come from this second array
   int64_t lda;
   int a_split;
-  const float *B, *B2;
+  const float *B, *B2, *B3;  // stored (k, j): reduction steps from b_split on come from the second array, from b_split2 on from the third
   int64_t ldb;
-  int b_split;
+  int b_split, b_split2;
   float* C;
   int64_t ldc;
   int kslice;
   int epi, act, accumulate;
   const float *bias, *Y, *X;
   int x_rows;
-  float* C2;
+  float *C2, *C3;
   float scale;
   double* sums;
-  float* colsum;        // sum_k A(i, k) per row i of the output, never accumulated
+  float* colsum;        // sum_k A(i, k) over the steps k >= cs_from, per row i of the output, never accumulated
+  int cs_from;
+  unsigned* zero;       // the first workgroup clears `zeros` counters for the launches that follow
+  int zeros;
   // reduction cut into gridDim.z slices: slice z leaves its tile in part[z] (tile-major, column sums behind the 1024 entries) and the last
   // workgroup to arrive at a tile adds the slices up in slice order.  counters: one zero per tile, zero again afterwards.
   float* part;
@@ -2968,12 +2975,23 @@ constexpr int kTilePart = 1024 + 32;
 // reduction behind one barrier per 16 steps left it on 64 CUs for 22 us.
 // A_KC: A is stored (i, k) with k contiguous, otherwise (k, i); B_KC: B is stored (j, k) with k contiguous, otherwise (k, j).
 // A lane of half h feeds steps k = 8 (s / 4) + 4 h + s % 4 of a chunk, so that k-contiguous rows are read 16 bytes at a time.
+// The reduction steps of a (k, .) operand may come from up to three arrays one after the other, from steps 0, at1 and at2 on.
+struct SgemmRows {
+  const float *p0, *p1, *p2;
+  int at1, at2;
+  __device__ __forceinline__ const float* row(int k, int64_t ld) const {
+    return k < at1 ? p0 + (int64_t)k * ld : (k < at2 ? p1 + (int64_t)(k - at1) * ld : p2 + (int64_t)(k - at2) * ld);
+  }
+  __device__ __forceinline__ bool together(int k0) const {  // steps k0 .. k0 + 31 lie in one array
+    return k0 + 32 <= at1 || (k0 >= at1 && k0 + 32 <= at2) || k0 >= at2;
+  }
+};
+
 template <bool KC>
-__device__ __forceinline__ void sgemm_fetch(float (&v)[16], const float* __restrict__ p, const float* __restrict__ p2, int split, int64_t ld,
-                                            int k0, int kend, int h, bool wide) {
-  if (k0 + 32 <= kend && (KC || k0 + 32 <= split || k0 >= split)) {  // a whole chunk of one array: no checks per load
+__device__ __forceinline__ void sgemm_fetch(float (&v)[16], const SgemmRows& r, int64_t ld, int k0, int kend, int h, bool wide) {
+  if (k0 + 32 <= kend && (KC || r.together(k0))) {  // a whole chunk of one array: no checks per load
     if (KC) {
-      const float* q = p + k0 + 4 * h;
+      const float* q = r.p0 + k0 + 4 * h;
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         if (wide) {
@@ -2985,7 +3003,7 @@ __device__ __forceinline__ void sgemm_fetch(float (&v)[16], const float* __restr
         }
       }
     } else {
-      const float* q = (k0 >= split ? p2 + (int64_t)(k0 - split) * ld : p + (int64_t)k0 * ld) + 4 * h * ld;
+      const float* q = r.row(k0, ld) + 4 * h * ld;
 #pragma unroll
       for (int s = 0; s < 16; ++s) v[s] = q[(8 * (s >> 2) + (s & 3)) * ld];
     }
@@ -2995,29 +3013,32 @@ __device__ __forceinline__ void sgemm_fetch(float (&v)[16], const float* __restr
   for (int s = 0; s < 16; ++s) {
     const int k = k0 + 8 * (s >> 2) + 4 * h + (s & 3);
     float x = 0.f;
-    if (k < kend) x = KC ? p[k] : (k < split ? p[(int64_t)k * ld] : p2[(int64_t)(k - split) * ld]);
+    if (k < kend) x = KC ? r.p0[k] : *r.row(k, ld);
     v[s] = x;
   }
 }
 
+// workgroup (bx, by, bz) of a grid (gx, gy, gz): row tile, column tile and slice of the reduction
 template <bool A_KC, bool B_KC, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
+__device__ __forceinline__ void sgemm_tile(const SgemmArgs& g, int bx, int by, int bz, int gx, int gy, int gz) {
   constexpr int RW = WAVES > 8 ? 8 : WAVES;  // tiles held in LDS at a time
   __shared__ float red[RW][1024];
   __shared__ float cred[WAVES][64];
   __shared__ double sred[WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
-  const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;  // rows on x: y admits 65536 tiles only
-  const int zbeg = blockIdx.z * g.kslice, zend = min(g.K, zbeg + g.kslice);
+  const int i0 = bx * 32, j0 = by * 32;
+  const int zbeg = bz * g.kslice, zend = min(g.K, zbeg + g.kslice);
   const int per = ((zend - zbeg + WAVES - 1) / WAVES + 7) / 8 * 8;
   const int kbeg = zbeg + wave * per, kend = min(zend, kbeg + per);
   // rows and columns past the matrix repeat the last one; their results are not stored
   const int ia = min(i0 + c, g.M - 1), jb = min(j0 + c, g.N - 1);
-  const float *pa, *pa2 = nullptr, *pb, *pb2 = nullptr;
-  if (A_KC) pa = ia < g.a_split ? g.A + (int64_t)ia * g.lda : g.A2 + (int64_t)(ia - g.a_split) * g.lda;
-  else { pa = g.A + ia; pa2 = g.A2 + ia; }
-  if (B_KC) pb = g.B + (int64_t)jb * g.ldb;
-  else { pb = g.B + jb; pb2 = g.B2 + jb; }
+  SgemmRows ra = {}, rb = {};
+  if (A_KC) ra.p0 = ia < g.a_split ? g.A + (int64_t)ia * g.lda : g.A2 + (int64_t)(ia - g.a_split) * g.lda;
+  else ra = {g.A + ia, g.A2 + ia, g.A2 + ia, g.a_split, 0x7fffffff};
+  if (B_KC) rb.p0 = g.B + (int64_t)jb * g.ldb;
+  else rb = {g.B + jb, g.B2 + jb, g.B3 + jb, g.b_split, g.b_split2};
+  if (g.zero && bx == 0 && by == 0 && bz == 0)
+    for (int x = threadIdx.x; x < g.zeros; x += 64 * WAVES) g.zero[x] = 0;
   const bool wa = A_KC && g.lda % 4 == 0 && (((uintptr_t)g.A | (uintptr_t)g.A2) & 15) == 0;  // kbeg is a multiple of 8
   const bool wb = B_KC && g.ldb % 4 == 0 && ((uintptr_t)g.B & 15) == 0;
   f32x16 acc;
@@ -3026,21 +3047,21 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
   float cs = 0.f;
   float a[16], b[16];
   if (kbeg < kend) {
-    sgemm_fetch<A_KC>(a, pa, pa2, g.a_split, g.lda, kbeg, kend, h, wa);
-    sgemm_fetch<B_KC>(b, pb, pb2, g.b_split, g.ldb, kbeg, kend, h, wb);
+    sgemm_fetch<A_KC>(a, ra, g.lda, kbeg, kend, h, wa);
+    sgemm_fetch<B_KC>(b, rb, g.ldb, kbeg, kend, h, wb);
   }
   for (int k0 = kbeg; k0 < kend; k0 += 32) {
     float a1[16], b1[16];
 #pragma unroll
     for (int s = 0; s < 16; ++s) a1[s] = b1[s] = 0.f;
     if (k0 + 32 < kend) {
-      sgemm_fetch<A_KC>(a1, pa, pa2, g.a_split, g.lda, k0 + 32, kend, h, wa);
-      sgemm_fetch<B_KC>(b1, pb, pb2, g.b_split, g.ldb, k0 + 32, kend, h, wb);
+      sgemm_fetch<A_KC>(a1, ra, g.lda, k0 + 32, kend, h, wa);
+      sgemm_fetch<B_KC>(b1, rb, g.ldb, k0 + 32, kend, h, wb);
     }
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
-      cs += a[s];
+      cs += k0 + 8 * (s >> 2) + 4 * h + (s & 3) >= g.cs_from ? a[s] : 0.f;
     }
 #pragma unroll
     for (int s = 0; s < 16; ++s) { a[s] = a1[s]; b[s] = b1[s]; }
@@ -3060,13 +3081,13 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + c] = acc[r];
   __syncthreads();
-  const bool sliced = gridDim.z > 1, want_cs = g.colsum && blockIdx.y == 0;
-  const int tile = blockIdx.y * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y;
+  const bool sliced = gz > 1, want_cs = g.colsum && by == 0;
+  const int tile = by * gx + bx, tiles = gx * gy;
   float csum = 0.f;
   if (want_cs && threadIdx.x < 32)
     for (int w = 0; w < WAVES; ++w) csum += cred[w][threadIdx.x] + cred[w][threadIdx.x + 32];
   if (sliced) {
-    float* mine = g.part + ((int64_t)blockIdx.z * tiles + tile) * kTilePart;
+    float* mine = g.part + ((int64_t)bz * tiles + tile) * kTilePart;
     for (int x = threadIdx.x; x < 1024; x += 64 * WAVES) {
       float v = 0.f;
       for (int w = 0; w < RW; ++w) v += red[w][x];
@@ -3076,13 +3097,13 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's part has reached memory
     __syncthreads();
     __shared__ unsigned last;
-    if (threadIdx.x == 0) last = atomicAdd(&g.counters[tile], 1u) == gridDim.z - 1;
+    if (threadIdx.x == 0) last = atomicAdd(&g.counters[tile], 1u) == (unsigned)gz - 1u;
     __syncthreads();
     if (!last) return;
     if (threadIdx.x == 0) g.counters[tile] = 0;
     for (int x = threadIdx.x; x < kTilePart; x += 64 * WAVES) {
       float v = 0.f;
-      for (int z = 0; z < (int)gridDim.z; ++z) v += device_load(g.part + ((int64_t)z * tiles + tile) * kTilePart + x);
+      for (int z = 0; z < gz; ++z) v += device_load(g.part + ((int64_t)z * tiles + tile) * kTilePart + x);
       if (x < 1024) red[0][x] = v;
       else csum = v;  // x = 1024 + thread: the tile is a whole number of passes
     }
@@ -3107,6 +3128,22 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
         else if (g.act == KS_ACT_TANH) v = tanhf(v);
         g.C[o] = v;
         break;
+      case kEpiTop:
+        v += g.bias[j];
+        if (g.act == KS_ACT_ELU) v = v > 0.f ? v : expm1f(v);
+        else if (g.act == KS_ACT_RELU) v = fmaxf(v, 0.f);
+        else if (g.act == KS_ACT_TANH) v = tanhf(v);
+        g.C[o] = v;
+        if (i < g.x_rows) {
+          act_derivatives(g.act, v, d1, d2);
+          g.C2[o] = g.X[j];
+          g.C3[o] = d1 * g.X[j];
+        }
+        break;
+      case kEpiOut:
+        g.C[o] = v + g.bias[j] - (i < g.x_rows ? 1.f : -1.f);
+        if (i < g.x_rows) g.C2[o] = 1.f;
+        break;
       case kEpiDelta: g.C[o] = v; g.C2[o] = d1 * v; break;
       case kEpiPenalty: g.C[o] = g.scale * v; sq += (double)v * v; break;
       case kEpiTangent: g.C2[o] = v * g.X[o] * d2; g.C[o] = v * d1; break;
@@ -3122,9 +3159,62 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {
     if (threadIdx.x == 0) {
       double t = 0.0;
       for (int w = 0; w < WAVES; ++w) t += sred[w];
-      g.sums[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = t;
+      g.sums[(int64_t)by * gx + bx] = t;
     }
   }
+}
+
+template <bool A_KC, bool B_KC, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void sgemm_kernel(SgemmArgs g) {  // rows on x: y admits 65536 tiles only
+  sgemm_tile<A_KC, B_KC, WAVES>(g, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, gridDim.z);
+}
+
+// The discriminator's loss terms: half the squared errors of the real and of the simulated rows (the output gradient is the error itself), and
+// the penalty, factor times the sum of its tiles' sums of squares, all in a fixed order.  One workgroup of 1024 threads.
+struct DiscLosses {
+  int64_t n_real, n, tiles;
+  const float* err;
+  const double* sums;
+  double factor;
+  float* losses;
+};
+__device__ __forceinline__ void disc_losses(const DiscLosses& d) {
+  __shared__ double sh[3][1024];
+  double a = 0.0, b = 0.0, c = 0.0;
+  for (int64_t i = threadIdx.x; i < d.n; i += 1024) {
+    const float e = d.err[i];
+    if (i < d.n_real) a += 0.5 * (double)e * e; else b += 0.5 * (double)e * e;
+  }
+  for (int64_t i = threadIdx.x; i < d.tiles; i += 1024) c += d.sums[i];
+  sh[0][threadIdx.x] = a; sh[1][threadIdx.x] = b; sh[2][threadIdx.x] = c;
+  __syncthreads();
+  for (int w = 512; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w)
+      for (int k = 0; k < 3; ++k) sh[k][threadIdx.x] += sh[k][threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) { d.losses[0] = (float)sh[0][0]; d.losses[1] = (float)sh[1][0]; d.losses[2] = (float)(d.factor * sh[2][0]); }
+}
+
+// Every weight and bias gradient of the discriminator in one launch, the penalty's share and the ordinary one as one reduction over both
+// passes' rows; the first workgroup adds up the losses.  They were six launches of 9.5 us, each too small to fill the chip.
+struct SgemmGroup {
+  int n;
+  int first[KS_MAX_LAYERS + 1];  // workgroups [first[l], first[l + 1]) behind the first one belong to product l
+  int slices[KS_MAX_LAYERS];
+  SgemmArgs g[KS_MAX_LAYERS];
+};
+__global__ __launch_bounds__(1024) void disc_wgrad_kernel(SgemmGroup t, DiscLosses d) {
+  if (blockIdx.x == 0) {
+    disc_losses(d);
+    return;
+  }
+  const int b = blockIdx.x - 1;
+  int l = 0;
+  while (l + 1 < t.n && b >= t.first[l + 1]) ++l;
+  const SgemmArgs& g = t.g[l];
+  const int gx = (g.M + 31) / 32, gy = (g.N + 31) / 32, at = b - t.first[l], tile = at % (gx * gy);
+  sgemm_tile<false, false, 16>(g, tile % gx, tile / gx, at / (gx * gy), gx, gy, t.slices[l]);
 }
 
 // The weight and bias gradient of a single layer over many rows, C(i, j) = sum_k A(k, i) B(k, j) with both operands fp32 and stored
@@ -3338,41 +3428,6 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(int M, int N, int nz, c
   C[(int64_t)i * ldc + j] = s;
 }
 
-// dz = out - target (target +1 on the first n_real rows, -1 on the rest) and the two squared-error sums (one workgroup)
-__global__ __launch_bounds__(1024) void disc_signal_kernel(int64_t n_real, int64_t n, const float* __restrict__ out, float* __restrict__ dz,
-                                                           float* __restrict__ ones, unsigned* __restrict__ counters,
-                                                           float* __restrict__ losses) {
-  __shared__ double sh[2][1024];
-  if (threadIdx.x < 512) counters[threadIdx.x] = 0;
-  double a = 0.0, b = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    const float e = out[i] - (i < n_real ? 1.f : -1.f);
-    dz[i] = e;
-    if (i < n_real) { ones[i] = 1.f; a += 0.5 * (double)e * e; } else b += 0.5 * (double)e * e;
-  }
-  sh[0][threadIdx.x] = a; sh[1][threadIdx.x] = b;
-  __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) { sh[0][threadIdx.x] += sh[0][threadIdx.x + w]; sh[1][threadIdx.x] += sh[1][threadIdx.x + w]; }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { losses[0] = (float)sh[0][0]; losses[1] = (float)sh[1][0]; losses[2] = 0.f; }
-}
-
-// penalty value: factor * the sum of the tiles' sums of squares, in a fixed order (one workgroup)
-__global__ __launch_bounds__(256) void disc_penalty_kernel(int64_t n, double factor, const double* __restrict__ sums, float* __restrict__ loss) {
-  __shared__ double sh[256];
-  double a = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 256) a += sums[i];
-  sh[threadIdx.x] = a;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *loss = (float)(factor * sh[0]);
-}
-
 }  // namespace ks
 
 struct DiscWs {
@@ -3380,7 +3435,9 @@ struct DiscWs {
   float* a[KS_MAX_LAYERS];      // real rows: W_{l+1}^T d_{l+1}
   float* d[KS_MAX_LAYERS];      // real rows: d_l
   float* r[KS_MAX_LAYERS];      // real rows: extra gradient of z_l
-  float *out, *dz0, *dz1, *g, *u, *v, *ones, *part;
+  float* v[KS_MAX_LAYERS];      // real rows: v_l of the sweep back, l = 1 .. L - 1
+  float* dz[KS_MAX_LAYERS];     // all rows: gradient of z_l, l = 1 .. L at [l - 1]
+  float *g, *ones, *part;
   unsigned* counters;
   double* sums;                 // one sum of squares per tile of the input gradient
 };
@@ -3396,44 +3453,70 @@ static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, Dis
   };
   DiscWs w;
   std::memset(&w, 0, sizeof(w));
-  int wmax = 1;
-  for (int l = 0; l <= m.n_layers; ++l) wmax = m.dims[l] > wmax ? m.dims[l] : wmax;
+  for (int l = 0; l < m.n_layers; ++l) w.dz[l] = take(M * m.dims[l + 1]);
   for (int l = 0; l + 1 < m.n_layers; ++l) {
+    w.v[l] = take(R * m.dims[l + 1]);
     w.y[l] = take(M * m.dims[l + 1]);
     w.a[l] = take(R * m.dims[l + 1]);
     w.d[l] = take(R * m.dims[l + 1]);
     w.r[l] = take(R * m.dims[l + 1]);
   }
-  w.out = take(M);
-  w.dz0 = take(M * wmax);
-  w.dz1 = take(M * wmax);
   w.g = take(R * m.dims[0]);
-  w.u = take(R * wmax);
-  w.v = take(R * wmax);
   w.ones = take(R);
   w.sums = (double*)take(2 * disc_penalty_tiles(m, R));
-  w.part = take((int64_t)512 * kTilePart);  // a sliced product has at most 512 (slice, tile) pairs
-  w.counters = (unsigned*)take(512);
+  w.part = take((int64_t)m.n_layers * 512 * kTilePart);  // a sliced product has at most 512 (slice, tile) pairs
+  w.counters = (unsigned*)take((int64_t)m.n_layers * 512);
   if (ws) *ws = w;
   return off;
 }
 
-// One product of sgemm_kernel; g.kslice is set here.  Products over activations have reductions of a layer's width: four wavefronts
-// share one.  Weight gradients (both operands stored (k, .)) reduce over the rows, sixteen wavefronts to a workgroup, and are cut into
-// slices while their few tiles leave CUs idle and a slice keeps the 512 rows that give every wavefront one chunk of loads.
-template <bool A_KC, bool B_KC>
-static void sgemm_go(hipStream_t s, SgemmArgs g) {
-  if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
+static void sgemm_finish_args(SgemmArgs& g) {
   if (!g.A2) { g.A2 = g.A; g.a_split = 0x7fffffff; }
   if (!g.B2) { g.B2 = g.B; g.b_split = 0x7fffffff; }
-  constexpr bool TN = !A_KC && !B_KC;
-  const dim3 tiles((unsigned)((g.M + 31) / 32), (unsigned)((g.N + 31) / 32));
-  int slices = 1;
-  if (TN && g.part)
-    while (slices < kDiscMaxSlices && g.K >= 1024 * slices && tiles.x * tiles.y * slices * 2 <= 512) slices *= 2;
-  g.kslice = (((g.K + slices - 1) / slices) + 15) / 16 * 16;
-  slices = (g.K + g.kslice - 1) / g.kslice;
-  hipLaunchKernelGGL((sgemm_kernel<A_KC, B_KC, TN ? 16 : 4>), dim3(tiles.x, tiles.y, (unsigned)slices), dim3(TN ? 1024 : 256), 0, s, g);
+  if (!g.B3) { g.B3 = g.B2; g.b_split2 = 0x7fffffff; }
+}
+
+// One product over activations, whose reduction is a layer's width: four wavefronts share it.
+template <bool B_KC>
+static void sgemm_go(hipStream_t s, SgemmArgs g) {
+  if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
+  sgemm_finish_args(g);
+  g.kslice = (g.K + 15) / 16 * 16;
+  hipLaunchKernelGGL((sgemm_kernel<true, B_KC, 4>), dim3((unsigned)((g.M + 31) / 32), (unsigned)((g.N + 31) / 32)), dim3(256), 0, s, g);
+}
+
+// Slices for the products of a group, whose reductions over the same K rows all get as many: the fewest rounds of workgroups over the CUs (one of
+// 1024 threads at a time each), weighed against the rows left to a wavefront.  A workgroup takes about 8 us beside its products, 32 rows of its
+// sixteen wavefronts 1.7; a slice keeps the 512 rows that give every wavefront a chunk of loads.  (1024 + 1024 frames, 71-256-256-1: 96 tiles
+// in two slices 19 us; sliced one by one, 384 workgroups, they took 29.)
+static int group_slices(int tiles, int widest, int64_t K) {
+  int best = 1;
+  double least = 0.0;
+  for (int s = 1; s <= kDiscMaxSlices && (s == 1 || (K >= 512ll * s && widest * s <= 512)); ++s) {
+    const double t = ((tiles * s + 256) / 256) * (8.0 + 1.7 * (double)((K + 512ll * s - 1) / (512ll * s)));  // one more for the losses
+    if (s == 1 || t < least) { least = t; best = s; }
+  }
+  return best;
+}
+
+static int group_blocks(SgemmGroup& t) {
+  int tiles = 0, widest = 0;
+  for (int k = 0; k < t.n; ++k) {
+    const int n = ((t.g[k].M + 31) / 32) * ((t.g[k].N + 31) / 32);
+    tiles += n;
+    widest = n > widest ? n : widest;
+  }
+  int blocks = 0;
+  for (int k = 0; k < t.n; ++k) {
+    SgemmArgs& g = t.g[k];
+    sgemm_finish_args(g);
+    const int want = group_slices(tiles, widest, g.K);
+    g.kslice = (((g.K + want - 1) / want) + 15) / 16 * 16;
+    t.slices[k] = (g.K + g.kslice - 1) / g.kslice;
+    t.first[k] = blocks;
+    blocks += ((g.M + 31) / 32) * ((g.N + 31) / 32) * t.slices[k];
+  }
+  return blocks;
 }
 
 // C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single layer.
@@ -3481,74 +3564,76 @@ extern "C" int ks_mlp_disc_loss_grad(KsMlp* h, ks_stream_t stream, int64_t n_rea
   DiscWs ws;
   carve_disc(m, R, M, (char*)workspace, &ws);
   SgemmArgs z = {};  // fields left out below are zero
-  // forward over the real rows, then the simulated ones
+  // forward over the real rows, then the simulated ones; the last hidden layer also opens the input gradient's chain (a, d of its output), the
+  // output layer leaves the gradient of the squared errors
   for (int l = 0; l < L; ++l) {
-    const bool last = l == L - 1;
     SgemmArgs g = z;
     g.M = (int)M; g.N = m.dims[l + 1]; g.K = m.dims[l];
     if (l > 0) g.A = ws.y[l - 1];
     else if (R == 0 || n_sim == 0) g.A = R ? real : sim;
     else { g.A = real; g.A2 = sim; g.a_split = (int)R; }
     g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l];
-    g.C = last ? ws.out : ws.y[l]; g.ldc = g.N; g.bias = m.mb[l]; g.epi = kEpiLayer; g.act = last ? KS_ACT_NONE : act;
-    sgemm_go<true, true>(s, g);
+    g.ldc = g.N; g.bias = m.mb[l]; g.act = act; g.x_rows = (int)R;
+    if (l == 0) { g.zero = ws.counters; g.zeros = 512 * L; }
+    if (l == L - 1) { g.epi = kEpiOut; g.C = ws.dz[l]; g.C2 = ws.ones; }
+    else if (l == L - 2 && penalty) { g.epi = kEpiTop; g.C = ws.y[l]; g.X = m.mW[L - 1]; g.C2 = ws.a[l]; g.C3 = ws.d[l]; }
+    else { g.epi = kEpiLayer; g.C = ws.y[l]; }
+    sgemm_go<true>(s, g);
   }
-  hipLaunchKernelGGL(disc_signal_kernel, dim3(1), dim3(1024), 0, s, R, M, ws.out, ws.dz0, ws.ones, ws.counters, losses);
 
+  DiscLosses losses_of = {R, M, 0, ws.dz[L - 1], ws.sums, 0.0, losses};
   if (penalty) {
-    // input gradient on the real rows: d_L = 1, down to g = d_1 W_1, which leaves its tiles as the penalty's gradient
-    const float* dnext = ws.ones;
-    for (int l = L - 1; l >= 0; --l) {  // hidden layer l (its output is y[l - 1]); l = 0: the input
+    // input gradient on the real rows: d_L = 1, d_{L-1} from the forward pass, down to g = d_1 W_1, which leaves its tiles as the penalty's
+    // gradient
+    for (int l = L > 1 ? L - 2 : 0; l >= 0; --l) {  // hidden layer l (its output is y[l - 1]); l = 0: the input
       SgemmArgs g = z;
       g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l + 1];
-      g.A = dnext; g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l]; g.ldc = g.N; g.act = act;
-      if (l > 0) { g.C = ws.a[l - 1]; g.C2 = ws.d[l - 1]; g.Y = ws.y[l - 1]; g.epi = kEpiDelta; dnext = ws.d[l - 1]; }
+      g.A = l + 1 == L ? ws.ones : ws.d[l]; g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l]; g.ldc = g.N; g.act = act;
+      if (l > 0) { g.C = ws.a[l - 1]; g.C2 = ws.d[l - 1]; g.Y = ws.y[l - 1]; g.epi = kEpiDelta; }
       else { g.C = ws.g; g.epi = kEpiPenalty; g.scale = grad_penalty_coef * (1.f / (float)n_motions); g.sums = ws.sums; }
-      sgemm_go<true, false>(s, g);
+      sgemm_go<false>(s, g);
     }
-    hipLaunchKernelGGL(disc_penalty_kernel, dim3(1), dim3(256), 0, s, disc_penalty_tiles(m, R),
-                       0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions), ws.sums, losses + 2);
-    // the sweep back through that computation, first layer to last; its share opens every weight gradient
-    const float* prev = ws.g;
-    float* v = ws.v;
-    for (int l = 1; l <= L; ++l) {
-      const int n = m.dims[l], k = m.dims[l - 1];
+    losses_of.tiles = disc_penalty_tiles(m, R);
+    losses_of.factor = 0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions);
+    for (int l = 1; l < L; ++l) {  // the sweep back through that computation, first layer to last
       SgemmArgs g = z;
-      g.M = n; g.N = k; g.K = (int)R; g.A = l == L ? ws.ones : ws.d[l - 1]; g.lda = n; g.B = prev; g.ldb = k;
-      g.C = m.gW[l - 1]; g.ldc = m.kpad[l - 1];
-      g.part = ws.part; g.counters = ws.counters;
-      sgemm_go<false, false>(s, g);
-      if (l == L) break;
-      g = z;
-      g.M = (int)R; g.N = n; g.K = k; g.A = prev; g.lda = k; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
-      g.C = v; g.C2 = ws.r[l - 1]; g.ldc = n; g.Y = ws.y[l - 1]; g.X = ws.a[l - 1]; g.act = act; g.epi = kEpiTangent;
-      sgemm_go<true, true>(s, g);
-      prev = v;
-      v = v == ws.v ? ws.u : ws.v;  // the next product reads this one's result
+      g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l - 1];
+      g.A = l == 1 ? ws.g : ws.v[l - 2]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+      g.C = ws.v[l - 1]; g.C2 = ws.r[l - 1]; g.ldc = g.N; g.Y = ws.y[l - 1]; g.X = ws.a[l - 1]; g.act = act; g.epi = kEpiTangent;
+      sgemm_go<true>(s, g);
     }
   }
 
-  // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows; the bias gradients are the
-  // column sums that ride on the weight gradients' pass over dz
-  float *dz = ws.dz0, *dnx = ws.dz1;
-  for (int l = L; l >= 1; --l) {
-    const int n = m.dims[l], k = m.dims[l - 1];
+  // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows
+  for (int l = L; l > 1; --l) {
     SgemmArgs g = z;
-    g.M = n; g.N = k; g.K = (int)M; g.A = dz; g.lda = n; g.ldb = k;
-    if (l > 1) g.B = ws.y[l - 2];
-    else if (R == 0 || n_sim == 0) g.B = R ? real : sim;
-    else { g.B = real; g.B2 = sim; g.b_split = (int)R; }
-    g.C = m.gW[l - 1]; g.ldc = m.kpad[l - 1]; g.accumulate = penalty ? 1 : 0;  // the weight gradient may hold the penalty's share
-    g.colsum = m.gb[l - 1];
-    g.part = ws.part; g.counters = ws.counters;
-    sgemm_go<false, false>(s, g);
-    if (l == 1) break;
-    g = z;
-    g.M = (int)M; g.N = k; g.K = n; g.A = dz; g.lda = n; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
-    g.C = dnx; g.ldc = k; g.Y = ws.y[l - 2]; g.X = ws.r[l - 2]; g.x_rows = penalty ? (int)R : 0; g.act = act; g.epi = kEpiDz;
-    sgemm_go<true, false>(s, g);
-    float* tmp = dz; dz = dnx; dnx = tmp;
+    g.M = (int)M; g.N = m.dims[l - 1]; g.K = m.dims[l]; g.A = ws.dz[l - 1]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+    g.C = ws.dz[l - 2]; g.ldc = g.N; g.Y = ws.y[l - 2]; g.X = ws.r[l - 2]; g.x_rows = penalty ? (int)R : 0; g.act = act; g.epi = kEpiDz;
+    sgemm_go<false>(s, g);
   }
+
+  // weight gradients: d_l^T v_{l-1} over the real rows, where there is a penalty, then dz_l^T y_{l-1} over all rows; the bias gradients are the
+  // column sums of dz that ride along
+  SgemmGroup t;
+  t.n = 0;
+  const int P = penalty ? (int)R : 0;
+  for (int l = 1; l <= L; ++l) {
+    SgemmArgs g = z;
+    g.M = m.dims[l]; g.N = m.dims[l - 1]; g.K = P + (int)M; g.lda = g.M; g.ldb = g.N;
+    const float *y0 = l > 1 ? ws.y[l - 2] : (R ? real : sim), *y1 = l == 1 && R && n_sim ? sim : nullptr;  // the rows' inputs, in one or two arrays
+    if (penalty) {
+      g.A = l == L ? ws.ones : ws.d[l - 1]; g.A2 = ws.dz[l - 1]; g.a_split = P;
+      g.B = l == 1 ? ws.g : ws.v[l - 2]; g.B2 = y0; g.b_split = P;
+      g.B3 = y1; g.b_split2 = P + (int)R;
+    } else {
+      g.A = ws.dz[l - 1]; g.B = y0; g.B2 = y1; g.b_split = (int)R;
+    }
+    g.C = m.gW[l - 1]; g.ldc = m.kpad[l - 1]; g.colsum = m.gb[l - 1]; g.cs_from = P;
+    g.part = ws.part + (int64_t)(l - 1) * 512 * kTilePart; g.counters = ws.counters + (l - 1) * 512;
+    t.g[t.n++] = g;
+  }
+  const int blocks = group_blocks(t);
+  hipLaunchKernelGGL(disc_wgrad_kernel, dim3((unsigned)blocks + 1), dim3(1024), 0, s, t, losses_of);
   return check_launch("ks_mlp_disc_loss_grad");
 }
 

@@ -215,3 +215,20 @@ def test_reference_windows_of_strided_clips_are_gathered_in_place():
             assert torch.cuda.max_memory_allocated() - before < motions.numel() * 4
     big = torch.zeros(1, 1, 1, device=DEV).expand(100000, 100000, 64)  # 2.5 TB if it were copied
     assert amp.make_real_batch(big, 4, 2, torch.Generator().manual_seed(1)).shape == (2, 4, 64)
+
+
+@pytest.mark.parametrize("rows", [((3, 13), (2, 45)), ((7, 101), (3, 467))])
+@pytest.mark.parametrize("coef", [0.0, 10.0])
+def test_discriminator_of_five_layers(rows, coef):
+    """One reduction over the penalty's rows and then all rows per weight gradient, every layer in one launch: row counts at which the two meet
+    inside a 32-step chunk and a slice, with one slice and with several."""
+    from ksim_amd.mlp import MLP
+
+    dims = [17, 40, 33, 64, 20, 1]
+    ws, bs = _params(dims, seed=9)
+    disc = MLP(ws, bs, activation="tanh", dtype="f32")
+    disc.train_init()
+    rng = np.random.default_rng(rows[0][1])
+    real, sim = (rng.normal(size=(*s, dims[0])).astype(np.float32) for s in rows)
+    for _ in range(2):  # counters and partial sums of the first call do not reach the second
+        _check(disc, ws, bs, real, sim, coef, "tanh")
