@@ -118,9 +118,10 @@ def require_cuda(*tensors, dtype=None):
     for t in tensors:
         if t is None:
             continue
+        if isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous() and (dtype is None or t.dtype == dtype):
+            continue
         if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise KsError("ksim_amd kernels take torch tensors resident on the GPU (there is no CPU path)")
         if not t.is_contiguous():
             raise KsError("ksim_amd kernels take contiguous tensors")
-        if dtype is not None and t.dtype != dtype:
-            raise KsError(f"expected dtype {dtype}, got {t.dtype}")
+        raise KsError(f"expected dtype {dtype}, got {t.dtype}")

@@ -24,7 +24,7 @@ def _rng(seed: int, step: int, step_base: torch.Tensor | None = None) -> T.KsRng
     """Philox key; `step_base` (one int64 on the device) is added to `step` when the kernel runs."""
     if step_base is not None:
         _lib.require_cuda(step_base, dtype=torch.int64)
-    return T.KsRng(int(seed) & (2**64 - 1), int(step) & (2**64 - 1), _lib.ptr(step_base).value)
+    return T.KsRng(int(seed) & (2**64 - 1), int(step) & (2**64 - 1), _lib.addr(step_base))
 
 
 # Sources an observation element reads besides its own `src`, per kind: the same list `ks_observe` checks for null
@@ -303,8 +303,8 @@ def sample_action(mean: torch.Tensor, log_std: torch.Tensor | None, *, noise: to
         raise _lib.KsError("noise must match the mean's shape")
     if out is None:
         out = torch.empty_like(mean)
-    _lib.check(lib.ks_sample_action(_lib.current_stream(), N, nu, _lib.ptr(mean), _lib.ptr(log_std), _lib.ptr(noise),
-                                    _rng(seed, step, step_base), float(clip_max), _lib.ptr(out)))
+    _lib.check(lib.ks_sample_action(_lib.current_stream(), N, nu, _lib.addr(mean), _lib.addr(log_std), _lib.addr(noise),
+                                    _rng(seed, step, step_base), float(clip_max), _lib.addr(out)))
     return out
 
 
@@ -329,9 +329,9 @@ def sample_action_head(raw: torch.Tensor, *, min_std: float, max_std: float, var
     elif tuple(out.shape) != (N, nu):
         raise _lib.KsError("out must be (N, nu)")
     stats = tuple(torch.empty((N, nu), dtype=torch.float32, device=raw.device) for _ in range(3)) if want_stats else (None,) * 3
-    head = T.KsGaussianHead(float(min_std), float(max_std), float(var_scale), int(bool(deterministic)), _lib.ptr(mean_bias).value)
-    _lib.check(lib.ks_sample_action_head(_lib.current_stream(), N, nu, _lib.ptr(raw), ctypes.byref(head), _lib.ptr(noise),
-                                         _rng(seed, step, step_base), float(clip_max), _lib.ptr(out), *(_lib.ptr(t) for t in stats)))
+    head = T.KsGaussianHead(float(min_std), float(max_std), float(var_scale), int(bool(deterministic)), _lib.addr(mean_bias))
+    _lib.check(lib.ks_sample_action_head(_lib.current_stream(), N, nu, _lib.addr(raw), ctypes.byref(head), _lib.addr(noise),
+                                         _rng(seed, step, step_base), float(clip_max), _lib.addr(out), *(_lib.addr(t) for t in stats)))
     return (out, *stats) if want_stats else out
 
 
@@ -361,8 +361,8 @@ def sample_action_mixture(raw: torch.Tensor, num_mixtures: int, *, min_std: floa
     logp = torch.empty((N, nu), dtype=torch.float32, device=raw.device) if want_stats else None
     comp = torch.empty((N, nu), dtype=torch.int32, device=raw.device) if want_stats else None
     head = T.KsMixtureHead(K, float(min_std), float(max_std), float(var_scale), int(bool(deterministic)),
-                           _lib.ptr(mean_bias).value, _lib.ptr(clip_lo).value, _lib.ptr(clip_hi).value)
-    _lib.check(lib.ks_sample_action_mixture(_lib.current_stream(), N, nu, _lib.ptr(raw), ctypes.byref(head), _lib.ptr(uniform),
-                                            _lib.ptr(noise), _rng(seed, step, step_base), float(clip_max), _lib.ptr(out),
-                                            _lib.ptr(logp), _lib.ptr(comp)))
+                           _lib.addr(mean_bias), _lib.addr(clip_lo), _lib.addr(clip_hi))
+    _lib.check(lib.ks_sample_action_mixture(_lib.current_stream(), N, nu, _lib.addr(raw), ctypes.byref(head), _lib.addr(uniform),
+                                            _lib.addr(noise), _rng(seed, step, step_base), float(clip_max), _lib.addr(out),
+                                            _lib.addr(logp), _lib.addr(comp)))
     return (out, logp, comp) if want_stats else out

@@ -65,7 +65,7 @@ class MLP:
         """Scratch of the paths that take several launches, one buffer per stream and thread: calls on different streams may overlap
         on the GPU, and the launches of two threads may alternate on one stream."""
         need = int(self._lib.ks_mlp_workspace_bytes(self._handle, M))
-        key = (torch.cuda.current_stream().cuda_stream, threading.get_ident()) if need else 0
+        key = (_lib.current_stream(), threading.get_ident()) if need else 0
         if self._ws is None:
             self._ws = {}
         ws = self._ws.get(key)
@@ -86,8 +86,8 @@ class MLP:
             if tuple(out.shape) != (M, self.out_dim):
                 raise _lib.KsError("output has the wrong shape")
         ws = self.workspace(M, x.device)
-        _lib.check(self._lib.ks_mlp_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(out),
-                                            _lib.ptr(ws)))
+        _lib.check(self._lib.ks_mlp_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(out),
+                                            _lib.addr(ws)))
         return out
 
     def forward_pair(self, x: torch.Tensor, out: torch.Tensor, other: "MLP", x_other: torch.Tensor,
@@ -99,10 +99,10 @@ class MLP:
             _lib.require_cuda(o, dtype=torch.float32)
             if tuple(a.shape) != (M, net.in_dim) or tuple(o.shape) != (M, net.out_dim):
                 raise _lib.KsError(f"expected input (M, {net.in_dim}) and output (M, {net.out_dim})")
-        _lib.check(self._lib.ks_mlp_forward_pair(self._handle, other._handle, _lib.current_stream(), M, _lib.ptr(x),
-                                                 _lib.ptr(out), _lib.ptr(x_other), _lib.ptr(out_other),
-                                                 _lib.ptr(self.workspace(M, x.device)),
-                                                 _lib.ptr(other.workspace(M, x.device))))
+        _lib.check(self._lib.ks_mlp_forward_pair(self._handle, other._handle, _lib.current_stream(), M, _lib.addr(x),
+                                                 _lib.addr(out), _lib.addr(x_other), _lib.addr(out_other),
+                                                 _lib.addr(self.workspace(M, x.device)),
+                                                 _lib.addr(other.workspace(M, x.device))))
 
     # ------------------------------------------------------------------ training (ksim/task/ppo.py:495-565)
     def train_init(self) -> None:
@@ -126,8 +126,8 @@ class MLP:
         M = x.shape[0]
         if out is None:
             out = torch.empty((M, self.out_dim), dtype=torch.float32, device=x.device)
-        _lib.check(self._lib.ks_mlp_train_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(out),
-                                                  _lib.ptr(self._train_ws(M, x.device))))
+        _lib.check(self._lib.ks_mlp_train_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(out),
+                                                  _lib.addr(self._train_ws(M, x.device))))
         return out
 
     def backward(self, x: torch.Tensor, dy: torch.Tensor) -> None:
@@ -135,8 +135,8 @@ class MLP:
         _lib.require_cuda(x, dy, dtype=torch.float32)
         if tuple(dy.shape) != (x.shape[0], self.out_dim):
             raise _lib.KsError("dy must have the shape of the network output")
-        _lib.check(self._lib.ks_mlp_train_backward(self._handle, _lib.current_stream(), x.shape[0], _lib.ptr(x),
-                                                   _lib.ptr(dy), _lib.ptr(self._train_ws(x.shape[0], x.device))))
+        _lib.check(self._lib.ks_mlp_train_backward(self._handle, _lib.current_stream(), x.shape[0], _lib.addr(x),
+                                                   _lib.addr(dy), _lib.addr(self._train_ws(x.shape[0], x.device))))
 
     def backward_dx(self, x: torch.Tensor | None, dy: torch.Tensor, dx: torch.Tensor, *, weight_gradients: bool = True,
                     accumulate: bool = False, zero_rows: torch.Tensor | None = None) -> torch.Tensor:
@@ -152,9 +152,9 @@ class MLP:
             _lib.require_cuda(zero_rows, dtype=torch.uint8)
             if tuple(zero_rows.shape) != (M,):
                 raise _lib.KsError("zero_rows must be (M,) uint8")
-        _lib.check(self._lib.ks_mlp_train_backward_dx(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(dy),
-                                                      _lib.ptr(dx), int(weight_gradients), int(accumulate),
-                                                      _lib.ptr(zero_rows), _lib.ptr(self._train_ws(M, dy.device))))
+        _lib.check(self._lib.ks_mlp_train_backward_dx(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(dy),
+                                                      _lib.addr(dx), int(weight_gradients), int(accumulate),
+                                                      _lib.addr(zero_rows), _lib.addr(self._train_ws(M, dy.device))))
         return dx
 
     def disc_loss_grad(self, real: torch.Tensor, sim: torch.Tensor, grad_penalty_coef: float) -> torch.Tensor:
@@ -170,8 +170,8 @@ class MLP:
             ws = torch.empty(need, dtype=torch.uint8, device=real.device)
             self._dws = ws
         losses = torch.empty(3, dtype=torch.float32, device=real.device)
-        _lib.check(self._lib.ks_mlp_disc_loss_grad(self._handle, _lib.current_stream(), n_real, _lib.ptr(real), n_sim, _lib.ptr(sim),
-                                                   float(grad_penalty_coef), max(real.shape[0], 1), _lib.ptr(losses), _lib.ptr(ws)))
+        _lib.check(self._lib.ks_mlp_disc_loss_grad(self._handle, _lib.current_stream(), n_real, _lib.addr(real), n_sim, _lib.addr(sim),
+                                                   float(grad_penalty_coef), max(real.shape[0], 1), _lib.addr(losses), _lib.addr(ws)))
         return losses
 
     @classmethod
@@ -189,19 +189,14 @@ class MLP:
 
     def grad_sqnorm(self, acc: torch.Tensor) -> None:
         _lib.require_cuda(acc, dtype=torch.float64)
-        _lib.check(self._lib.ks_mlp_grad_sqnorm(self._handle, _lib.current_stream(), _lib.ptr(acc)))
+        _lib.check(self._lib.ks_mlp_grad_sqnorm(self._handle, _lib.current_stream(), _lib.addr(acc)))
 
     def adam_step(self, params: "T.KsAdamParams", sqnorm: torch.Tensor | None) -> None:
-        _lib.check(self._lib.ks_mlp_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
+        _lib.check(self._lib.ks_mlp_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.addr(sqnorm)))
 
     def parameters(self, gradients: bool = False) -> list[tuple[torch.Tensor, torch.Tensor]]:
         """[(weight (out, in), bias (out))] copies of the fp32 master parameters, or of their gradients."""
-        out = [(torch.empty((o, i), dtype=torch.float32, device="cuda"), torch.empty((o,), dtype=torch.float32, device="cuda"))
-               for i, o in zip(self.dims[:-1], self.dims[1:])]
-        table = ctypes.c_void_p * len(out)
-        _lib.check(self._lib.ks_mlp_copy_params(self._handle, _lib.current_stream(), table(*(w.data_ptr() for w, _ in out)),
-                                                table(*(b.data_ptr() for _, b in out)), int(gradients)))
-        return out
+        return copy_parameters([self], gradients)[0]
 
     def close(self) -> None:
         if getattr(self, "_borrowed", False):
@@ -218,18 +213,28 @@ class MLP:
 
 
 def _handles(nets: Sequence[MLP]):
-    return (ctypes.c_void_p * len(nets))(*(net._handle for net in nets))
+    return (ctypes.c_void_p * len(nets))(*[net._handle for net in nets])
+
+
+def copy_parameters(nets: Sequence[MLP], gradients: bool = False) -> list[list[tuple[torch.Tensor, torch.Tensor]]]:
+    """`MLP.parameters` of several networks, in one launch."""
+    empty, f32, dev = torch.empty, torch.float32, torch.device("cuda", torch._C._cuda_getDevice())
+    out = [[(empty((o, i), dtype=f32, device=dev), empty((o,), dtype=f32, device=dev)) for i, o in zip(net.dims[:-1], net.dims[1:])] for net in nets]
+    table = ctypes.c_void_p * sum(map(len, out))
+    _lib.check(_lib.load().ks_mlps_copy_params(_handles(nets), len(nets), _lib.current_stream(), table(*[w.data_ptr() for net in out for w, _ in net]),
+                                               table(*[b.data_ptr() for net in out for _, b in net]), int(gradients)))
+    return out
 
 
 def grad_sqnorm(nets: Sequence[MLP], acc: torch.Tensor) -> None:
     """Adds the squared gradient norm over all of `nets` to `acc`."""
     _lib.require_cuda(acc, dtype=torch.float64)
-    _lib.check(_lib.load().ks_mlps_grad_sqnorm(_handles(nets), len(nets), _lib.current_stream(), _lib.ptr(acc)))
+    _lib.check(_lib.load().ks_mlps_grad_sqnorm(_handles(nets), len(nets), _lib.current_stream(), _lib.addr(acc)))
 
 
 def adam_step(nets: Sequence[MLP], params: "T.KsAdamParams", sqnorm: torch.Tensor | None) -> None:
     """One optimiser step of all of `nets`; `sqnorm` is the squared gradient norm over everything optimised together."""
-    _lib.check(_lib.load().ks_mlps_adam_step(_handles(nets), len(nets), _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
+    _lib.check(_lib.load().ks_mlps_adam_step(_handles(nets), len(nets), _lib.current_stream(), ctypes.byref(params), _lib.addr(sqnorm)))
 
 
 def random_mlp(dims: Sequence[int], seed: int, activation: str = "elu", dtype: str = "bf16"):

@@ -116,8 +116,8 @@ def get_ppo_variables(policy: GaussianMlpPolicy, actor_obs: torch.Tensor, critic
     mean = policy.actor.train_forward(actor_obs) if train else policy.actor(actor_obs)
     value = (policy.critic.train_forward(critic_obs) if train else policy.critic(critic_obs)).reshape(-1)
     lp, ent = torch.empty_like(mean), torch.empty_like(mean)
-    _lib.check(lib.ks_gaussian_log_prob(_lib.current_stream(), mean.shape[0], mean.shape[1], _lib.ptr(mean),
-                                        _lib.ptr(policy.log_std), _lib.ptr(action), _lib.ptr(lp), _lib.ptr(ent)))
+    _lib.check(lib.ks_gaussian_log_prob(_lib.current_stream(), mean.shape[0], mean.shape[1], _lib.addr(mean),
+                                        _lib.addr(policy.log_std), _lib.addr(action), _lib.addr(lp), _lib.addr(ent)))
     return lp, value, ent, mean
 
 
@@ -148,7 +148,7 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
             raise _lib.KsError(f"the {name} mirror map has {perm.numel()} entries, the rows have {x.shape[1]}")
         both = torch.empty(2 * rows, x.shape[1], dtype=torch.float32, device=x.device)
         both[:rows].copy_(x)
-        _lib.check(lib.ks_signed_permute(st, rows, x.shape[1], _lib.ptr(both[:rows]), _lib.ptr(perm), _lib.ptr(sign), _lib.ptr(both[rows:])))
+        _lib.check(lib.ks_signed_permute(st, rows, x.shape[1], _lib.addr(both[:rows]), _lib.addr(perm), _lib.addr(sign), _lib.addr(both[rows:])))
         return both
 
     a_in = with_mirrored(a_obs, "actor_obs") if mirror_a else a_obs
@@ -157,7 +157,7 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     value_all = policy.critic.train_forward(c_in)
     mean, value = mean_all[:rows], value_all[:rows].reshape(-1)
     lp, ent = torch.empty_like(mean), torch.empty_like(mean)
-    _lib.check(lib.ks_gaussian_log_prob(st, rows, nu, _lib.ptr(mean), _lib.ptr(policy.log_std), _lib.ptr(act), _lib.ptr(lp), _lib.ptr(ent)))
+    _lib.check(lib.ks_gaussian_log_prob(st, rows, nu, _lib.addr(mean), _lib.addr(policy.log_std), _lib.addr(act), _lib.addr(lp), _lib.addr(ent)))
     inputs = ppo_mod.compute_ppo_inputs(value.view(Tn, b), rewards, done, success, cfg.gamma, cfg.lam,
                                         normalize_advantages=cfg.normalize_advantages,
                                         monte_carlo_returns=cfg.monte_carlo_returns, time_major=True)
@@ -166,47 +166,47 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     if cfg.adaptive_kl and policy.kl_scale is None:
         policy.kl_scale = torch.ones(1, dtype=torch.float32, device=actor_obs.device)
     p = _lib.KsPpoLossParams(cfg.clip_param, cfg.value_loss_coef, cfg.entropy_coef, cfg.kl_coef, cfg.log_clip_value,
-                             1.0, int(cfg.use_clipped_value_loss), _lib.ptr(policy.kl_scale) if cfg.adaptive_kl else None)
+                             1.0, int(cfg.use_clipped_value_loss), _lib.addr(policy.kl_scale) if cfg.adaptive_kl else None)
     d_mean_all = torch.empty_like(mean_all)
     d_value_all = torch.empty(value_all.shape[0], 1, dtype=torch.float32, device=mean.device)
     d_mean, d_value = d_mean_all[:rows], d_value_all[:rows]
     d_log_std = torch.empty_like(policy.log_std)
     ws = torch.empty(256 * nu, dtype=torch.float32, device=mean.device)
     on_lp, on_v = on_log_probs.reshape(rows, nu), on_values.reshape(rows)
-    _lib.check(lib.ks_ppo_loss_grad(_lib.current_stream(), rows, nu, ctypes.byref(p), _lib.ptr(mean),
-                                    _lib.ptr(policy.log_std), _lib.ptr(act), _lib.ptr(on_lp),
-                                    _lib.ptr(inputs.advantages_bt), _lib.ptr(inputs.value_targets_bt), _lib.ptr(on_v),
-                                    _lib.ptr(value), _lib.ptr(d_mean), _lib.ptr(d_value), _lib.ptr(d_log_std), _lib.ptr(ws)))
+    _lib.check(lib.ks_ppo_loss_grad(_lib.current_stream(), rows, nu, ctypes.byref(p), _lib.addr(mean),
+                                    _lib.addr(policy.log_std), _lib.addr(act), _lib.addr(on_lp),
+                                    _lib.addr(inputs.advantages_bt), _lib.addr(inputs.value_targets_bt), _lib.addr(on_v),
+                                    _lib.addr(value), _lib.addr(d_mean), _lib.addr(d_value), _lib.addr(d_log_std), _lib.addr(ws)))
     aux = {}
     if mirror_a:
         perm, sign = policy.mirror.device("action", mean.device)
         aux["action_mirror_loss"] = torch.empty(rows, dtype=torch.float32, device=mean.device)
-        _lib.check(lib.ks_mirror_loss_grad(st, rows, nu, cfg.actor_mirror_loss_scale, _lib.ptr(mean), _lib.ptr(mean_all[rows:]),
-                                           _lib.ptr(perm), _lib.ptr(sign), _lib.ptr(d_mean), _lib.ptr(d_mean_all[rows:]),
-                                           _lib.ptr(aux["action_mirror_loss"])))
+        _lib.check(lib.ks_mirror_loss_grad(st, rows, nu, cfg.actor_mirror_loss_scale, _lib.addr(mean), _lib.addr(mean_all[rows:]),
+                                           _lib.addr(perm), _lib.addr(sign), _lib.addr(d_mean), _lib.addr(d_mean_all[rows:]),
+                                           _lib.addr(aux["action_mirror_loss"])))
     if mirror_c:
         perm, sign = policy.mirror.device("value", mean.device)
         aux["value_mirror_loss"] = torch.empty(rows, dtype=torch.float32, device=mean.device)
-        _lib.check(lib.ks_mirror_loss_grad(st, rows, 1, cfg.critic_mirror_loss_scale, _lib.ptr(value_all), _lib.ptr(value_all[rows:]),
-                                           _lib.ptr(perm), _lib.ptr(sign), _lib.ptr(d_value), _lib.ptr(d_value_all[rows:]),
-                                           _lib.ptr(aux["value_mirror_loss"])))
+        _lib.check(lib.ks_mirror_loss_grad(st, rows, 1, cfg.critic_mirror_loss_scale, _lib.addr(value_all), _lib.addr(value_all[rows:]),
+                                           _lib.addr(perm), _lib.addr(sign), _lib.addr(d_value), _lib.addr(d_value_all[rows:]),
+                                           _lib.addr(aux["value_mirror_loss"])))
     policy.actor.backward(a_in, d_mean_all)
     policy.critic.backward(c_in, d_value_all)
     # optimiser chain over every parameter together: global norm first
     sq = torch.zeros(1, dtype=torch.float64, device=mean.device)
     nets = policy.actor.networks() + policy.critic.networks()
     mlp_mod.grad_sqnorm(nets, sq)
-    _lib.check(lib.ks_grad_sqnorm(_lib.current_stream(), nu, _lib.ptr(d_log_std), _lib.ptr(sq)))
+    _lib.check(lib.ks_grad_sqnorm(_lib.current_stream(), nu, _lib.addr(d_log_std), _lib.addr(sq)))
     policy.opt_step += 1
     ap = _adam(cfg, policy.opt_step)
     mlp_mod.adam_step(nets, ap, sq)
-    _lib.check(lib.ks_adam_step(_lib.current_stream(), nu, _lib.ptr(policy.log_std), _lib.ptr(d_log_std),
-                                _lib.ptr(policy._m1), _lib.ptr(policy._m2), ctypes.byref(ap), _lib.ptr(sq)))
+    _lib.check(lib.ks_adam_step(_lib.current_stream(), nu, _lib.addr(policy.log_std), _lib.addr(d_log_std),
+                                _lib.addr(policy._m1), _lib.addr(policy._m2), ctypes.byref(ap), _lib.addr(sq)))
     metrics = {"grad_norm": sq.sqrt(), "d_mean": d_mean, "d_value": d_value, "d_log_std": d_log_std,
                "log_probs": lp, "values": value, "advantages": inputs.advantages_bt, **aux}
     if cfg.adaptive_kl:
-        _lib.check(lib.ks_ppo_adapt_kl(_lib.current_stream(), rows, nu, _lib.ptr(on_lp), _lib.ptr(lp), cfg.kl_coef,
-                                       cfg.desired_kl, _lib.ptr(policy.kl_scale), _lib.ptr(ws)))
+        _lib.check(lib.ks_ppo_adapt_kl(_lib.current_stream(), rows, nu, _lib.addr(on_lp), _lib.addr(lp), cfg.kl_coef,
+                                       cfg.desired_kl, _lib.addr(policy.kl_scale), _lib.addr(ws)))
     return metrics
 
 
@@ -299,8 +299,8 @@ def actor_locations(policy: "RecurrentHeadPolicy", raw: torch.Tensor, obs: torch
         add, add_ld = ctypes.c_void_p(obs.data_ptr() + 4 * col0), obs.shape[-1]
     out = torch.empty_like(raw)
     _lib.check(_lib.load().ks_lowpass_scan(_lib.current_stream(), Tn, M, nu, W, float(lp.ctrl_dt), float(lp.cutoff_frequency),
-                                           _lib.ptr(raw), _lib.ptr(policy.mean_bias), add, add_ld, a0, cnt, _lib.ptr(lpf0),
-                                           _lib.ptr(fresh), _lib.ptr(out), _lib.ptr(y_last)))
+                                           _lib.addr(raw), _lib.addr(policy.mean_bias), add, add_ld, a0, cnt, _lib.addr(lpf0),
+                                           _lib.addr(fresh), _lib.addr(out), _lib.addr(y_last)))
     return out
 
 
@@ -336,7 +336,7 @@ class RecurrentHeadPolicy:
 
     def _mixture(self) -> "T.KsMixtureHead":
         return T.KsMixtureHead(int(self.num_mixtures), float(self.min_std), float(self.max_std), float(self.var_scale), 0,
-                               _lib.ptr(self.mean_bias).value, _lib.ptr(self.clip_lo).value, _lib.ptr(self.clip_hi).value)
+                               _lib.addr(self.mean_bias), _lib.addr(self.clip_lo), _lib.addr(self.clip_hi))
 
 
 def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, actor_obs, critic_obs, action, rewards, done, success,
@@ -370,7 +370,7 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
             raise _lib.KsError(f"the {name} mirror map has {perm.numel()} entries, the rows have {x.shape[-1]}")
         x = x.contiguous()
         xm = torch.empty_like(x)
-        _lib.check(lib.ks_signed_permute(st, rows, x.shape[-1], _lib.ptr(x), _lib.ptr(perm), _lib.ptr(sign), _lib.ptr(xm)))
+        _lib.check(lib.ks_signed_permute(st, rows, x.shape[-1], _lib.addr(x), _lib.addr(perm), _lib.addr(sign), _lib.addr(xm)))
         return torch.cat([x, xm], dim=1).contiguous()
 
     fresh2 = torch.cat([fresh, fresh], dim=1).contiguous() if (mirror_a or mirror_c) else None
@@ -394,17 +394,17 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
     if cfg.adaptive_kl and policy.kl_scale is None:  # as in single_step: the factor stays on the device
         policy.kl_scale = torch.ones(1, dtype=torch.float32, device=dev)
     p = _lib.KsPpoLossParams(cfg.clip_param, cfg.value_loss_coef, cfg.entropy_coef, cfg.kl_coef, cfg.log_clip_value, 1.0,
-                             int(cfg.use_clipped_value_loss), _lib.ptr(policy.kl_scale) if cfg.adaptive_kl else None)
+                             int(cfg.use_clipped_value_loss), _lib.addr(policy.kl_scale) if cfg.adaptive_kl else None)
     # behind the filter the bias is already inside the location
-    bias_ptr = None if policy.lowpass is not None else _lib.ptr(policy.mean_bias).value
+    bias_ptr = None if policy.lowpass is not None else _lib.addr(policy.mean_bias)
     head = policy._mixture() if mixture else T.KsGaussianHead(float(policy.min_std), float(policy.max_std), float(policy.var_scale), 0, bias_ptr)
     d_raw = torch.empty(Tn, b, policy.width(nu), dtype=torch.float32, device=dev)
     d_value = torch.empty(Tn, b, 1, dtype=torch.float32, device=dev)
     grad_fn = lib.ks_ppo_loss_grad_mixture if mixture else lib.ks_ppo_loss_grad_head
-    _lib.check(grad_fn(st, rows, nu, ctypes.byref(p), ctypes.byref(head), _lib.ptr(raw),
-                       _lib.ptr(action.contiguous()), _lib.ptr(on_log_probs.contiguous()),
-                       _lib.ptr(inputs.advantages_bt), _lib.ptr(inputs.value_targets_bt),
-                       _lib.ptr(on_values.contiguous()), _lib.ptr(value), _lib.ptr(d_raw), _lib.ptr(d_value)))
+    _lib.check(grad_fn(st, rows, nu, ctypes.byref(p), ctypes.byref(head), _lib.addr(raw),
+                       _lib.addr(action.contiguous()), _lib.addr(on_log_probs.contiguous()),
+                       _lib.addr(inputs.advantages_bt), _lib.addr(inputs.value_targets_bt),
+                       _lib.addr(on_values.contiguous()), _lib.addr(value), _lib.addr(d_raw), _lib.addr(d_value)))
     aux = {}
     d_raw_all, d_value_all = d_raw, d_value
     if mirror_a:
@@ -415,8 +415,8 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
         d_mode, d_mode_m = d_raw[..., :nu].contiguous(), torch.empty(Tn, b, nu, dtype=torch.float32, device=dev)
         perm, sign = policy.mirror.device("action", dev)
         aux["action_mirror_loss"] = torch.empty(Tn, b, dtype=torch.float32, device=dev)
-        _lib.check(lib.ks_mirror_loss_grad(st, rows, nu, cfg.actor_mirror_loss_scale, _lib.ptr(mode), _lib.ptr(mode_m), _lib.ptr(perm),
-                                           _lib.ptr(sign), _lib.ptr(d_mode), _lib.ptr(d_mode_m), _lib.ptr(aux["action_mirror_loss"])))
+        _lib.check(lib.ks_mirror_loss_grad(st, rows, nu, cfg.actor_mirror_loss_scale, _lib.addr(mode), _lib.addr(mode_m), _lib.addr(perm),
+                                           _lib.addr(sign), _lib.addr(d_mode), _lib.addr(d_mode_m), _lib.addr(aux["action_mirror_loss"])))
         d_raw_all = torch.zeros(Tn, 2 * b, 2 * nu, dtype=torch.float32, device=dev)  # the mirrored deviations enter nothing
         d_raw_all[:, :b] = d_raw
         d_raw_all[:, :b, :nu] = d_mode
@@ -426,15 +426,15 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
         d_v, d_vm = d_value.view(rows, 1), torch.empty(rows, 1, dtype=torch.float32, device=dev)
         perm, sign = policy.mirror.device("value", dev)
         aux["value_mirror_loss"] = torch.empty(Tn, b, dtype=torch.float32, device=dev)
-        _lib.check(lib.ks_mirror_loss_grad(st, rows, 1, cfg.critic_mirror_loss_scale, _lib.ptr(v_main), _lib.ptr(v_m), _lib.ptr(perm),
-                                           _lib.ptr(sign), _lib.ptr(d_v), _lib.ptr(d_vm), _lib.ptr(aux["value_mirror_loss"])))
+        _lib.check(lib.ks_mirror_loss_grad(st, rows, 1, cfg.critic_mirror_loss_scale, _lib.addr(v_main), _lib.addr(v_m), _lib.addr(perm),
+                                           _lib.addr(sign), _lib.addr(d_v), _lib.addr(d_vm), _lib.addr(aux["value_mirror_loss"])))
         d_value_all = torch.cat([d_value, d_vm.view(Tn, b, 1)], dim=1).contiguous()
     if policy.lowpass is not None:  # dL/d location -> dL/d raw mean, back through the filter's own recursion
         if d_raw_all is d_raw:
             d_raw_all = d_raw.clone()  # d_raw stays what the loss kernel wrote, for the caller's metrics
         lp_ = policy.lowpass
         _lib.check(lib.ks_lowpass_scan_backward(st, Tn, d_raw_all.shape[1], nu, 2 * nu, float(lp_.ctrl_dt), float(lp_.cutoff_frequency),
-                                                _lib.ptr(a_fresh), _lib.ptr(d_raw_all), None))
+                                                _lib.addr(a_fresh), _lib.addr(d_raw_all), None))
     lockstep(policy.actor.backward_pass(d_raw_all), policy.critic.backward_pass(d_value_all))
     sq = torch.zeros(1, dtype=torch.float64, device=dev)
     nets = policy.actor.networks() + policy.critic.networks()
@@ -447,14 +447,14 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
     if cfg.adaptive_kl:  # ppo.py:546-563 on the log-probabilities of this step's forward pass
         lp = torch.empty(rows, nu, dtype=torch.float32, device=dev)
         if mixture:
-            _lib.check(lib.ks_mixture_head_log_prob(st, rows, nu, ctypes.byref(head), _lib.ptr(raw),
-                                                    _lib.ptr(action.contiguous()), _lib.ptr(lp)))
+            _lib.check(lib.ks_mixture_head_log_prob(st, rows, nu, ctypes.byref(head), _lib.addr(raw),
+                                                    _lib.addr(action.contiguous()), _lib.addr(lp)))
         else:
-            _lib.check(lib.ks_gaussian_head_log_prob(st, rows, nu, ctypes.byref(head), _lib.ptr(raw),
-                                                     _lib.ptr(action.contiguous()), _lib.ptr(lp), None))
+            _lib.check(lib.ks_gaussian_head_log_prob(st, rows, nu, ctypes.byref(head), _lib.addr(raw),
+                                                     _lib.addr(action.contiguous()), _lib.addr(lp), None))
         ws = torch.empty(256 * nu, dtype=torch.float32, device=dev)
-        _lib.check(lib.ks_ppo_adapt_kl(st, rows, nu, _lib.ptr(on_log_probs.contiguous()), _lib.ptr(lp), cfg.kl_coef,
-                                       cfg.desired_kl, _lib.ptr(policy.kl_scale), _lib.ptr(ws)))
+        _lib.check(lib.ks_ppo_adapt_kl(st, rows, nu, _lib.addr(on_log_probs.contiguous()), _lib.addr(lp), cfg.kl_coef,
+                                       cfg.desired_kl, _lib.addr(policy.kl_scale), _lib.addr(ws)))
         metrics["log_probs"] = lp
     return metrics
 
@@ -472,13 +472,13 @@ def recurrent_on_policy(policy: RecurrentHeadPolicy, actor_obs, critic_obs, acti
     lp = torch.empty(Tn, N, nu, dtype=torch.float32, device=action.device)
     if policy.num_mixtures:
         head = policy._mixture()
-        _lib.check(_lib.load().ks_mixture_head_log_prob(_lib.current_stream(), Tn * N, nu, ctypes.byref(head), _lib.ptr(raw),
-                                                        _lib.ptr(action.contiguous()), _lib.ptr(lp)))
+        _lib.check(_lib.load().ks_mixture_head_log_prob(_lib.current_stream(), Tn * N, nu, ctypes.byref(head), _lib.addr(raw),
+                                                        _lib.addr(action.contiguous()), _lib.addr(lp)))
     else:
         head = T.KsGaussianHead(float(policy.min_std), float(policy.max_std), float(policy.var_scale), 0,
-                                None if policy.lowpass is not None else _lib.ptr(policy.mean_bias).value)
-        _lib.check(_lib.load().ks_gaussian_head_log_prob(_lib.current_stream(), Tn * N, nu, ctypes.byref(head), _lib.ptr(raw),
-                                                         _lib.ptr(action.contiguous()), _lib.ptr(lp), None))
+                                None if policy.lowpass is not None else _lib.addr(policy.mean_bias))
+        _lib.check(_lib.load().ks_gaussian_head_log_prob(_lib.current_stream(), Tn * N, nu, ctypes.byref(head), _lib.addr(raw),
+                                                         _lib.addr(action.contiguous()), _lib.addr(lp), None))
     return (lp, values[..., 0], raw) if return_raw else (lp, values[..., 0])
 
 

@@ -118,8 +118,8 @@ class GRUCell:
             if tuple(out.shape) != tuple(h.shape):
                 raise _lib.KsError("output has the wrong shape")
         ws = self.workspace(M, x.device)
-        _lib.check(self._lib.ks_gru_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(h),
-                                            _lib.ptr(fresh), _lib.ptr(out), _lib.ptr(ws)))
+        _lib.check(self._lib.ks_gru_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h),
+                                            _lib.addr(fresh), _lib.addr(out), _lib.addr(ws)))
         return out
 
     # ------------------------------------------------------------------ training (ksim/task/ppo.py:572-694)
@@ -140,8 +140,8 @@ class GRUCell:
         M, H = x.shape[0], self.hidden_size
         if tuple(x.shape) != (M, self.input_size) or tuple(h.shape) != (M, H) or tuple(out.shape) != (M, H) or tuple(saved.shape) != (M, 5 * H):
             raise _lib.KsError("expected x (M, input), h and out (M, H), saved (M, 5H)")
-        _lib.check(self._lib.ks_gru_train_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(h), _lib.ptr(fresh),
-                                                  _lib.ptr(out), _lib.ptr(saved), _lib.ptr(self.workspace(M, x.device))))
+        _lib.check(self._lib.ks_gru_train_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h), _lib.addr(fresh),
+                                                  _lib.addr(out), _lib.addr(saved), _lib.addr(self.workspace(M, x.device))))
         return out
 
     @property
@@ -198,19 +198,18 @@ class GRUCell:
         need = int(self._lib.ks_gru_backward_workspace_bytes(self._handle, M))
         if self._bws is None or self._bws.numel() < need or self._bws.device != dh_out.device:
             self._bws = torch.empty(need, dtype=torch.uint8, device=dh_out.device)
-        _lib.check(self._lib.ks_gru_backward_step(self._handle, _lib.current_stream(), M, _lib.ptr(dh_out), _lib.ptr(saved),
-                                                  _lib.ptr(fresh), _lib.ptr(d_gi), _lib.ptr(d_gh), _lib.ptr(dh_in), _lib.ptr(self._bws)))
+        _lib.check(self._lib.ks_gru_backward_step(self._handle, _lib.current_stream(), M, _lib.addr(dh_out), _lib.addr(saved),
+                                                  _lib.addr(fresh), _lib.addr(d_gi), _lib.addr(d_gh), _lib.addr(dh_in), _lib.addr(self._bws)))
 
     def grad_sqnorm(self, acc: torch.Tensor) -> None:
-        _lib.check(self._lib.ks_gru_grad_sqnorm(self._handle, _lib.current_stream(), _lib.ptr(acc)))
+        _lib.check(self._lib.ks_gru_grad_sqnorm(self._handle, _lib.current_stream(), _lib.addr(acc)))
 
     def adam_step(self, params, sqnorm) -> None:
-        _lib.check(self._lib.ks_gru_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
+        _lib.check(self._lib.ks_gru_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.addr(sqnorm)))
 
     def parameters(self, gradients: bool = False) -> dict:
         """Copies of weight_ih, weight_hh, bias (3H) and bias_n (H), or of their gradients."""
-        (wi, bi), = self.proj_i.parameters(gradients)
-        (wh, bh), = self.proj_h.parameters(gradients)
+        ((wi, bi),), ((wh, bh),) = mlp_mod.copy_parameters((self.proj_i, self.proj_h), gradients)
         return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:].clone())
 
     def __del__(self):
@@ -270,8 +269,8 @@ class LSTMCell:
             if tuple(t.shape) != tuple(h.shape):
                 raise _lib.KsError("output has the wrong shape")
         ws = self.workspace(M, x.device)
-        _lib.check(self._lib.ks_lstm_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(h), _lib.ptr(c),
-                                             _lib.ptr(fresh), _lib.ptr(ho), _lib.ptr(co), _lib.ptr(ws)))
+        _lib.check(self._lib.ks_lstm_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h), _lib.addr(c),
+                                             _lib.addr(fresh), _lib.addr(ho), _lib.addr(co), _lib.addr(ws)))
         return ho, co
 
     # ------------------------------------------------------------------ training (ksim/task/ppo.py:572-694)
@@ -291,9 +290,9 @@ class LSTMCell:
         M, H = x.shape[0], self.hidden_size
         if tuple(x.shape) != (M, self.input_size) or any(tuple(t.shape) != (M, H) for t in (h, c, h_out, c_out)) or tuple(saved.shape) != (M, 7 * H):
             raise _lib.KsError("expected x (M, input), h, c and outputs (M, H), saved (M, 7H)")
-        _lib.check(self._lib.ks_lstm_train_forward(self._handle, _lib.current_stream(), M, _lib.ptr(x), _lib.ptr(h), _lib.ptr(c),
-                                                   _lib.ptr(fresh), _lib.ptr(h_out), _lib.ptr(c_out), _lib.ptr(saved),
-                                                   _lib.ptr(self.workspace(M, x.device))))
+        _lib.check(self._lib.ks_lstm_train_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h), _lib.addr(c),
+                                                   _lib.addr(fresh), _lib.addr(h_out), _lib.addr(c_out), _lib.addr(saved),
+                                                   _lib.addr(self.workspace(M, x.device))))
 
     @property
     def sequence_supported(self) -> bool:
@@ -351,20 +350,19 @@ class LSTMCell:
         need = int(self._lib.ks_lstm_backward_workspace_bytes(self._handle, M))
         if self._bws is None or self._bws.numel() < need or self._bws.device != dh_out.device:
             self._bws = torch.empty(need, dtype=torch.uint8, device=dh_out.device)
-        _lib.check(self._lib.ks_lstm_backward_step(self._handle, _lib.current_stream(), M, _lib.ptr(dh_out), _lib.ptr(dc_out),
-                                                   _lib.ptr(saved), _lib.ptr(fresh), _lib.ptr(d_g), _lib.ptr(dh_in),
-                                                   _lib.ptr(dc_in), _lib.ptr(self._bws)))
+        _lib.check(self._lib.ks_lstm_backward_step(self._handle, _lib.current_stream(), M, _lib.addr(dh_out), _lib.addr(dc_out),
+                                                   _lib.addr(saved), _lib.addr(fresh), _lib.addr(d_g), _lib.addr(dh_in),
+                                                   _lib.addr(dc_in), _lib.addr(self._bws)))
 
     def grad_sqnorm(self, acc: torch.Tensor) -> None:
-        _lib.check(self._lib.ks_lstm_grad_sqnorm(self._handle, _lib.current_stream(), _lib.ptr(acc)))
+        _lib.check(self._lib.ks_lstm_grad_sqnorm(self._handle, _lib.current_stream(), _lib.addr(acc)))
 
     def adam_step(self, params, sqnorm) -> None:
-        _lib.check(self._lib.ks_lstm_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.ptr(sqnorm)))
+        _lib.check(self._lib.ks_lstm_adam_step(self._handle, _lib.current_stream(), ctypes.byref(params), _lib.addr(sqnorm)))
 
     def parameters(self, gradients: bool = False) -> dict:
         """Copies of weight_ih, weight_hh and bias (4H), or of their gradients."""
-        (wi, bi), = self.proj_i.parameters(gradients)
-        (wh, _), = self.proj_h.parameters(gradients)
+        ((wi, bi),), ((wh, _),) = mlp_mod.copy_parameters((self.proj_i, self.proj_h), gradients)
         return dict(weight_ih=wi, weight_hh=wh, bias=bi)
 
     def __del__(self):

@@ -230,9 +230,9 @@ class Rollout:
                     col0, a0, cnt = (int(v) for v in lp.obs_bias)
                     add, add_ld = _lib.c_void_p(self.noisy_obs[t].data_ptr() + 4 * col0), self.noisy_obs.shape[-1]
                 _lib.check(_lib.load().ks_lowpass_scan(_lib.current_stream(), 1, self.N, nu_, 2 * nu_, float(lp.ctrl_dt),
-                                                       float(lp.cutoff_frequency), _lib.ptr(self.mean), _lib.ptr(head_bias), add, add_ld,
-                                                       a0, cnt, _lib.ptr(env.lpf_state), _lib.ptr(self.reset_mask), _lib.ptr(self.mean),
-                                                       _lib.ptr(env.lpf_state)))
+                                                       float(lp.cutoff_frequency), _lib.addr(self.mean), _lib.addr(head_bias), add, add_ld,
+                                                       a0, cnt, _lib.addr(env.lpf_state), _lib.addr(self.reset_mask), _lib.addr(self.mean),
+                                                       _lib.addr(env.lpf_state)))
                 head_bias = None  # now inside the filtered location
             sample_action_head(self.mean, min_std=c.head.min_std, max_std=c.head.max_std, var_scale=c.head.var_scale,
                                mean_bias=head_bias, noise=noise.get("action_normal"), seed=env.seed, step=step,
@@ -467,14 +467,14 @@ class SplitRollout:
             if ro.values is None:
                 raise _lib.KsError("a critic is required for GAE")
             with torch.cuda.stream(st):
-                _lib.check(lib.ks_gae_tn(_lib.current_stream(), ro.T, ro.N, _lib.ptr(ro.values), _lib.ptr(rew.total),
-                                         _lib.ptr(ro.done), _lib.ptr(ro.success), float(gamma), float(lam), 0,
-                                         _lib.ptr(self._gae[g]), _lib.ptr(self._ret[g]), _lib.ptr(self._tgt[g])))
+                _lib.check(lib.ks_gae_tn(_lib.current_stream(), ro.T, ro.N, _lib.addr(ro.values), _lib.addr(rew.total),
+                                         _lib.addr(ro.done), _lib.addr(ro.success), float(gamma), float(lam), 0,
+                                         _lib.addr(self._gae[g]), _lib.addr(self._ret[g]), _lib.addr(self._tgt[g])))
         self.join()
         adv = self._gae
         if normalize_advantages:
-            _lib.check(lib.ks_normalize_advantages(_lib.current_stream(), self._gae.numel(), _lib.ptr(self._gae),
-                                                   _lib.ptr(self._adv), _lib.ptr(self._ws)))
+            _lib.check(lib.ks_normalize_advantages(_lib.current_stream(), self._gae.numel(), _lib.addr(self._gae),
+                                                   _lib.addr(self._adv), _lib.addr(self._ws)))
             adv = self._adv
         return [ppo_mod.PPOInputs(advantages_bt=adv[g], value_targets_bt=self._tgt[g], gae_bt=self._gae[g],
                                   returns_bt=self._ret[g]) for g in range(self.splits)]

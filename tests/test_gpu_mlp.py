@@ -379,3 +379,28 @@ def test_networks_optimised_together_match_one_by_one():
         dy = torch.ones(x.shape[0], n2.out_dim, device=DEV)
         n1.train_forward(x); n2.train_forward(x)
         assert torch.equal(n1.backward_dx(x, dy, dx1), n2.backward_dx(x, dy, dx2))
+
+
+def test_parameters_of_several_networks_in_one_launch():
+    """More layers than one launch's table holds, ragged widths, weights and gradients; against the copies network by network."""
+    from ksim_amd import _lib, mlp
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(6)
+    nets = []
+    for dims in ((33, 130, 7), (5, 3), (20, 40, 30, 20, 30, 40, 20, 10, 5), (9, 8, 7, 6, 5, 4, 3, 2, 1), (17, 257, 1)):
+        net = MLP([rng.normal(size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])],
+                  [rng.normal(size=o).astype(np.float32) for o in dims[1:]], activation="elu", dtype="f32")
+        net.train_init()
+        x = torch.from_numpy(rng.normal(size=(32, dims[0])).astype(np.float32)).to(DEV)
+        net.train_forward(x)
+        net.backward(x, torch.ones((32, dims[-1]), device=DEV))
+        nets.append(net)
+    for gradients in (False, True):
+        for net, got in zip(nets, mlp.copy_parameters(nets, gradients)):
+            want = net.parameters(gradients)
+            assert len(got) == len(want) == len(net.dims) - 1
+            assert all(torch.equal(a, c) and torch.equal(b, d) for (a, b), (c, d) in zip(got, want))
+    assert mlp.copy_parameters([]) == []
+    with pytest.raises(_lib.KsError):  # a network without a training state, behind one that has it
+        mlp.copy_parameters([nets[0], MLP([np.ones((2, 3), np.float32)], [np.ones(2, np.float32)], activation="elu", dtype="f32")])
