@@ -269,6 +269,15 @@ __device__ __forceinline__ void activate_tiles(f32x16 (&acc)[MI][2]) {
       for (int r = 0; r < 16; ++r) acc[i][j][r] = activate<ACT, false>(acc[i][j][r]);
 }
 
+// Four neighbouring floats at any address of a float: rows of an odd width start at one, and a 16-byte load needs no more than that.  Against
+// four loads of a float each: 102400 x 475 -> 128 186 -> 155 us, its weight gradient 155 -> 140 (rows of a multiple of four: 106 and 93; what
+// remains is that a row's 128 bytes lie in two cache lines).
+struct __attribute__((packed, aligned(4))) Float4Any { float x, y, z, w; };
+__device__ __forceinline__ float4 load4_any(const float* p) {
+  const Float4Any v = *reinterpret_cast<const Float4Any*>(p);
+  return float4{v.x, v.y, v.z, v.w};
+}
+
 // fp32 layers: y = act(x W^T + b) on BM x 128 tiles, four wavefronts of BM / 2 x 64 each, operands cut on their way to LDS.  A stage is
 // 32 k: thread t cuts the fragment q = t % 4 of rows t / 4 + 64 r, k = 16 (q / 2) + 4 (q % 2) + {0..3, 8..11}, so that four neighbouring
 // lanes read 128 bytes of a row in two loads.  A part's fragments lie [q][row] with two spare ones per q: neighbouring lanes write into
@@ -332,6 +341,7 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
   const int64_t b64 = (int64_t)64 * K;
   float4 ra[AV][2], rb[2][2];
   auto fetch = [&](int n) __attribute__((always_inline)) {
+    const bool inside = kbeg + 32 * (n + 1) <= Kreal;  // the whole stage
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int k = lk + 32 * n + 8 * u, left = Kreal - k;  // steps of the row still inside the input (VA: a multiple of four)
@@ -341,6 +351,8 @@ void cut_layer_kernel(int64_t M, int K, int Kreal, int Nreal, const float* __res
         ra[r][u] = float4{0.f, 0.f, 0.f, 0.f};
         if (VA) {
           if (left > 0) ra[r][u] = *reinterpret_cast<const float4*>(at);
+        } else if (inside) {
+          ra[r][u] = load4_any(at);
         } else {
           if (left > 0) ra[r][u].x = at[0];
           if (left > 1) ra[r][u].y = at[1];
@@ -3233,11 +3245,11 @@ __global__ __launch_bounds__(1024) void disc_wgrad_kernel(SgemmGroup t, DiscLoss
 // take 44 us at the card's copy rate.  The predecessor multiplied on the fp32 instruction, whose time alone is 87 us there.
 //   102400 x 512 x 128, fp32: 122 -> 93 us (110 -> 145 TFLOP/s); relative error against 64 bits 7.3e-7 -> 1.9e-7
 //   12288 x 384 x 128, bf16: 44 us in five launches (cast, two transposes, product, column sums) -> 11.4
-// VA / VB: the operand's rows are 16-byte aligned and its width is a multiple of four.
+// EDGE: a width is no multiple of four.
 constexpr int kTnKB = 32;  // rows of a stage
 __host__ __device__ constexpr int tn_buf(int parts) { return parts * (kTnKB / 8) * 256; }  // one group's LDS buffer, in 16-byte fragments
 
-template <int PARTS, bool VA, bool VB>
+template <int PARTS, bool EDGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
                   float* __restrict__ C, int64_t ldc, int kslice, float* __restrict__ colsum) {
@@ -3268,29 +3280,33 @@ void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
   const bool isb = t >= 128;
   const int kg = (t & 127) >> 5, l = t & 31;
   const int width = isb ? N : M, c0 = (isb ? j0 : i0) + 4 * l;
-  const bool vec = isb ? VB : VA;
   const int64_t ld = isb ? ldb : lda;
   const float* src = (isb ? B : A) + (int64_t)(kbeg + 8 * kg) * ld;
-  int at[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) at[e] = vec ? min(c0, width - 4) + e : min(c0 + e, width - 1);
+  // four columns that reach over the matrix's edge (EDGE; at most one lane of a tile's row) are loaded one by one
+  const bool edge = EDGE && c0 < width + (width < 4 ? 128 : 0) && c0 + 4 > width;
+  const int first = max(0, min(c0, width - 4));
   float4 v[8];
   float4 cs = {0.f, 0.f, 0.f, 0.f};
-  auto load4 = [&](const float* q) __attribute__((always_inline)) {
-    if (vec) return *reinterpret_cast<const float4*>(q + at[0]);
-    return float4{q[at[0]], q[at[1]], q[at[2]], q[at[3]]};
-  };
   auto fetch = [&](int n) __attribute__((always_inline)) {
     const int k0 = kbeg + kTnKB * n + 8 * kg;
     const float* q = src + (int64_t)n * kTnKB * ld;
-    if (kbeg + kTnKB * (n + 1) <= kend) {
+    const bool full = kbeg + kTnKB * (n + 1) <= kend;  // otherwise the group's last rows, and zeros beyond them
+    if (edge) {
+      const int a0 = min(c0, width - 1), a1 = min(c0 + 1, width - 1), a2 = min(c0 + 2, width - 1), a3 = min(c0 + 3, width - 1);
 #pragma unroll
-      for (int r = 0; r < 8; ++r) v[r] = load4(q + r * ld);
-    } else {  // the group's last rows, and zeros beyond them
+      for (int r = 0; r < 8; ++r) {
+        const float* p = q + r * ld;
+        v[r] = float4{0.f, 0.f, 0.f, 0.f};
+        if (full || k0 + r < kend) v[r] = float4{p[a0], p[a1], p[a2], p[a3]};
+      }
+    } else if (full) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] = load4_any(q + r * ld + first);
+    } else {
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         v[r] = float4{0.f, 0.f, 0.f, 0.f};
-        if (k0 + r < kend) v[r] = load4(q + r * ld);
+        if (k0 + r < kend) v[r] = load4_any(q + r * ld + first);
       }
     }
   };
@@ -3523,14 +3539,12 @@ static int group_blocks(SgemmGroup& t) {
 template <int PARTS>
 static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                  int64_t ldc, float* part, float* colsum) {
-  const bool vec_a = lda % 4 == 0 && ((uintptr_t)A & 15) == 0 && M % 4 == 0, vec_b = ldb % 4 == 0 && ((uintptr_t)B & 15) == 0 && N % 4 == 0;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   const int slices = wgrad_slices(M, N, K);
   const int kslice = (int)(((K + slices - 1) / slices + 2 * kTnKB - 1) / (2 * kTnKB)) * 2 * kTnKB;  // slices past the last row add zeros
   constexpr int lds = 2 * tn_buf(PARTS) * 16;
   float* colpart = part + (int64_t)slices * M * N;
-  auto kfn = vec_a ? (vec_b ? wgrad_kernel<PARTS, true, true> : wgrad_kernel<PARTS, true, false>)
-                   : (vec_b ? wgrad_kernel<PARTS, false, true> : wgrad_kernel<PARTS, false, false>);
+  auto kfn = M % 4 || N % 4 ? wgrad_kernel<PARTS, true> : wgrad_kernel<PARTS, false>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
   hipLaunchKernelGGL(kfn, dim3((unsigned)tiles, (unsigned)slices), dim3(512), lds, s, (int)M, N, (int)K, A, lda, B, ldb,

@@ -834,3 +834,29 @@ def test_minibatch_columns_equal_index_select(T_, N, picked):
             want = t.index_select(d, idx)
             assert got.shape == want.shape and got.dtype == want.dtype and got.is_contiguous()
             assert torch.equal(got.view(torch.uint8) if got.dtype != torch.bool else got, want.contiguous().view(torch.uint8) if got.dtype != torch.bool else want)
+
+
+@pytest.mark.parametrize("dims,M", [((475, 128), 2051), ((33, 130), 4097), ((3, 5), 60001), ((65, 36), 8193), ((64, 128), 3000)])
+def test_single_fp32_layers_over_rows_at_any_float(dims, M):
+    """Rows that start 0 to 3 floats past a 16-byte boundary, the last one at the end of its allocation: the bits of the aligned rows, and the
+    products within what 64 bits allow."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    w, b = rng.normal(size=(dims[1], dims[0])).astype(np.float32), rng.normal(size=dims[1]).astype(np.float32)
+    x, dy = rng.normal(size=(M, dims[0])).astype(np.float32), rng.normal(size=(M, dims[1])).astype(np.float32)
+    net = MLP([w], [b], activation="none", dtype="f32")
+    net.train_init()
+    got = []
+    for off in range(4):
+        xo, do = (torch.empty(a.size + off, device=DEV)[off:].view(a.shape) for a in (x, dy))
+        xo.copy_(t32(x)), do.copy_(t32(dy))
+        y = net(xo)
+        net.backward(xo, do)
+        got.append((y, *net.parameters(gradients=True)[0]))
+    # sums of n products of size one: n roundings of 2^-24 of a partial sum of size sqrt(n), as a random walk, 8 deviations
+    bound = lambda n: 8 * 2.0 ** -24 * max(n, 16)  # noqa: E731
+    assert np.abs(got[0][0].cpu().numpy() - (x.astype(np.float64) @ w.astype(np.float64).T + b)).max() < bound(dims[0])
+    assert np.abs(got[0][1].cpu().numpy() - dy.astype(np.float64).T @ x.astype(np.float64)).max() < bound(M)
+    for other in got[1:]:
+        assert all(torch.equal(a, c) for a, c in zip(got[0], other))
