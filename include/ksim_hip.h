@@ -794,6 +794,8 @@ int ks_mlp_train_backward(KsMlp* mlp, ks_stream_t stream, int64_t M, const float
 int ks_mlp_train_backward_dx(KsMlp* mlp, ks_stream_t stream, int64_t M, const float* x, const float* dy, float* dx,
                              int32_t weight_gradients, int32_t accumulate_dx, const uint8_t* zero_rows /*(M) nullable*/,
                              void* workspace);
+/* The weight and bias gradient of a network of one layer from input rows that lie ldx floats apart (ldx >= in). */
+int ks_mlp_layer_weight_grad(KsMlp* mlp, ks_stream_t stream, int64_t M, const float* x, int64_t ldx, const float* dy, void* workspace);
 /* The first `count` bias entries of a layer are constants: the optimiser and the gradient norm skip them. */
 int ks_mlp_freeze_bias_prefix(KsMlp* mlp, int32_t layer, int32_t count);
 

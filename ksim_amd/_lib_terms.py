@@ -247,6 +247,8 @@ def bind(lib) -> None:
     lib.ks_mlp_train_workspace_bytes.restype = c_int64
     lib.ks_mlp_train_forward.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_train_backward.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]
+    lib.ks_mlp_layer_weight_grad.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p]
+    lib.ks_mlp_layer_weight_grad.restype = c_int32
     lib.ks_grad_sqnorm.argtypes = [c_void_p, c_int64, c_void_p, c_void_p]
     lib.ks_mlp_train_backward_dx.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
                                              c_void_p, c_void_p]

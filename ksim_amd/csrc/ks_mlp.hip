@@ -2633,7 +2633,7 @@ static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int
 // Backward pass of a single layer (the projections of the recurrent cells and their networks, over all the (step, env) rows of a
 // trajectory slice): no activation to pass through, so the caller's gradient and input are the operands of both products as they are.
 template <typename T>
-static int train_backward_single(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws, float* dx,
+static int train_backward_single(DevMlp& m, hipStream_t s, int64_t M, const float* x, int64_t ldx, const float* dy, const TrainWs& ws, float* dx,
                                  bool want_w, bool accumulate_dx, const uint8_t* zero_rows) {
   const int np = m.npad[0], in = m.dims[0], out = m.dims[1], kp128 = round_up(m.kpad[0], kBN);
   const bool plain = !accumulate_dx && !zero_rows;
@@ -2666,7 +2666,7 @@ static int train_backward_single(DevMlp& m, hipStream_t s, int64_t M, const floa
     }
   }
   if (!want_w) return KS_OK;
-  return wgrad<sizeof(T) == 2 ? 1 : 3>(s, out, in, M, dy, out, x, in, m.gW[0], m.kpad[0], ws.part, m.gb[0]);
+  return wgrad<sizeof(T) == 2 ? 1 : 3>(s, out, in, M, dy, out, x, ldx, m.gW[0], m.kpad[0], ws.part, m.gb[0]);
 }
 
 template <typename T>
@@ -2674,7 +2674,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
                           float* dx = nullptr, bool want_w = true, bool accumulate_dx = false, const uint8_t* zero_rows = nullptr) {
   const int L = m.n_layers;
   const int64_t Mp = ws.Mp;
-  if (L == 1) return train_backward_single<T>(m, s, M, x, dy, ws, dx, want_w, accumulate_dx, zero_rows);
+  if (L == 1) return train_backward_single<T>(m, s, M, x, m.dims[0], dy, ws, dx, want_w, accumulate_dx, zero_rows);
   if constexpr (sizeof(T) == 2) if (m.chain_saved) {
     if (want_w && !dx) return train_backward_chain<T>(m, s, M, x, dy, ws);
     // the layer-by-layer pass below reads row-major activations: rebuild them from the transposed copies
@@ -2801,6 +2801,20 @@ extern "C" int ks_mlp_train_backward(KsMlp* h, ks_stream_t stream, int64_t M, co
   const int rc = h->m.dtype == KS_MLP_BF16 ? train_backward<__bf16>(h->m, (hipStream_t)stream, M, x, dy, ws)
                                            : train_backward<float>(h->m, (hipStream_t)stream, M, x, dy, ws);
   return rc != KS_OK ? rc : check_launch("ks_mlp_train_backward");
+}
+
+// The hidden projections' gradient: their input is a block of columns of what the recurrence kept per step, and copying it out first was a pass
+// of its own (102400 x 128: 21 us beside a product of 92; the product takes as long on the strided rows).
+extern "C" int ks_mlp_layer_weight_grad(KsMlp* h, ks_stream_t stream, int64_t M, const float* x, int64_t ldx, const float* dy, void* workspace) {
+  if (!h || !h->m.train) return fail(KS_EINVAL, "ks_mlp_layer_weight_grad: call ks_mlp_train_init first");
+  if (h->m.n_layers != 1) return fail(KS_EINVAL, "ks_mlp_layer_weight_grad: the network has %d layers, not one", h->m.n_layers);
+  if (M <= 0 || !x || !dy || !workspace || ldx < h->m.dims[0]) return fail(KS_EINVAL, "ks_mlp_layer_weight_grad: bad argument");
+  if (M > (1 << 30)) return fail(KS_ELIMIT, "ks_mlp_layer_weight_grad: too many rows");
+  TrainWs ws;
+  carve_train(h->m, M, (char*)workspace, &ws);
+  const int rc = h->m.dtype == KS_MLP_BF16 ? train_backward_single<__bf16>(h->m, (hipStream_t)stream, M, x, ldx, dy, ws, nullptr, true, false, nullptr)
+                                           : train_backward_single<float>(h->m, (hipStream_t)stream, M, x, ldx, dy, ws, nullptr, true, false, nullptr);
+  return rc != KS_OK ? rc : check_launch("ks_mlp_layer_weight_grad");
 }
 
 extern "C" int ks_mlp_train_backward_dx(KsMlp* h, ks_stream_t stream, int64_t M, const float* x, const float* dy, float* dx,

@@ -157,6 +157,16 @@ class MLP:
                                                       _lib.addr(zero_rows), _lib.addr(self._train_ws(M, dy.device))))
         return dx
 
+    def layer_weight_grad(self, x: torch.Tensor, dy: torch.Tensor) -> None:
+        """`backward` of a network of one layer whose input rows are a block of columns of wider rows: x (M, in), its columns side by side."""
+        _lib.require_cuda(dy, dtype=torch.float32)
+        if not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] != self.in_dim or x.stride(1) != 1 or x.stride(0) < self.in_dim:
+            raise _lib.KsError(f"expected fp32 rows of {self.in_dim} on the GPU, columns side by side")
+        if tuple(dy.shape) != (x.shape[0], self.out_dim):
+            raise _lib.KsError("dy must have the shape of the network output")
+        _lib.check(self._lib.ks_mlp_layer_weight_grad(self._handle, _lib.current_stream(), x.shape[0], x.data_ptr(), x.stride(0), dy.data_ptr(),
+                                                      _lib.addr(self._train_ws(x.shape[0], x.device))))
+
     def disc_loss_grad(self, real: torch.Tensor, sim: torch.Tensor, grad_penalty_coef: float) -> torch.Tensor:
         """Gradient of the AMP discriminator loss (ksim/task/amp.py:360-438) into the handle: real (B, T, in) reference
         motions, sim (B2, T2, in) simulated ones; returns the (real, simulated, penalty) terms of the loss, on the device."""

@@ -478,8 +478,7 @@ class RecurrentNetwork:
             hs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
             sv = torch.empty(T_, M, (7 if self.lstm else 5) * H, dtype=torch.float32, device=dev)
             if self.lstm and getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
-                cs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
-                yield cell.sequence_call(x, carry0[i, 0], carry0[i, 1], fresh, hs, cs, sv)
+                yield cell.sequence_call(x, carry0[i, 0], carry0[i, 1], fresh, hs, None, sv)
             elif self.lstm:
                 cs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
                 for t in range(T_):
@@ -533,8 +532,8 @@ class RecurrentNetwork:
                     cell.backward_step(dH[t], ccarry[t & 1], sv[t], tp["fresh"][t], d_gi[t], carry[(t + 1) & 1], ccarry[(t + 1) & 1])
                 else:
                     cell.backward_step(dH[t], sv[t], tp["fresh"][t], d_gi[t], d_gh[t], carry[(t + 1) & 1])
-            h_used = sv[:, :, (6 if self.lstm else 4) * H:].contiguous().view(T_ * M, H)
-            cell.proj_h.backward(h_used, d_gh.view(T_ * M, G * H))
+            h_used = sv.view(T_ * M, sv.shape[2])[:, (6 if self.lstm else 4) * H:]
+            cell.proj_h.layer_weight_grad(h_used, d_gh.view(T_ * M, G * H))
             dX = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
             cell.proj_i.backward_dx(tp["xs"][i].reshape(T_ * M, H), d_gi.view(T_ * M, G * H), dX.view(T_ * M, H))
             dH = dX

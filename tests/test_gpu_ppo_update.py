@@ -860,3 +860,26 @@ def test_single_fp32_layers_over_rows_at_any_float(dims, M):
     assert np.abs(got[0][1].cpu().numpy() - dy.astype(np.float64).T @ x.astype(np.float64)).max() < bound(M)
     for other in got[1:]:
         assert all(torch.equal(a, c) for a, c in zip(got[0], other))
+
+
+@pytest.mark.parametrize("dims,dtype,M,wide,first", [((128, 512), "f32", 2051, 896, 768), ((128, 384), "bf16", 385, 640, 512), ((37, 20), "f32", 1000, 111, 74),
+                                                     ((5, 3), "bf16", 1, 5, 0)])
+def test_weight_gradient_from_a_block_of_columns(dims, dtype, M, wide, first):
+    """Input rows inside wider rows: the bits of the same rows copied out; other arrangements are refused."""
+    from ksim_amd._lib import KsError
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    net = MLP([rng.normal(size=dims[::-1]).astype(np.float32)], [np.zeros(dims[1], np.float32)], activation="none", dtype=dtype)
+    net.train_init()
+    rows, dy = t32(rng.normal(size=(M, wide))), t32(rng.normal(size=(M, dims[1])))
+    x = rows[:, first:first + dims[0]]
+    net.backward(x.contiguous(), dy)
+    want = net.parameters(gradients=True)[0]
+    net.layer_weight_grad(x, dy)
+    assert all(torch.equal(a, b) for a, b in zip(want, net.parameters(gradients=True)[0]))
+    for bad in (rows.t()[:dims[0]].t(), x[:, :-1], x.double(), x.cpu()):
+        if tuple(bad.shape) == tuple(x.shape) and bad.stride() == x.stride() and bad.dtype == x.dtype and bad.device == x.device:
+            continue
+        with pytest.raises(KsError):
+            net.layer_weight_grad(bad, dy)
