@@ -825,6 +825,7 @@ int ks_gather_columns(ks_stream_t stream, int32_t n, const KsGatherArray* arrays
  * A mirror map is a signed permutation: mirrored[j] = sign[j] * x[perm[j]] (mirror_joints / mirror_obs / mirror_cmd,
  * train.py:1565-1760, each negate and reorder entries of their vector).
  *   ks_signed_permute     out[r][j] = sign[j] * x[r][perm[j]]: the mirrored rows that the networks see
+ *   ks_mirror_pairs       the rows and their images side by side, in one pass
  *   ks_mirror_loss_grad   with y (rows, n) the network's output on the rows and ym (rows, n) its output on the mirrored
  *                         rows:  loss[r] = scale * mean_j (y[r][j] - sign[j] ym[r][perm[j]])^2  (train.py:1466-1469; for
  *                         a critic n = 1, perm = {0}, sign = {1}: scale * (v - vm)^2, train.py:1477), and the gradient of
@@ -852,6 +853,9 @@ int ks_lowpass_scan_backward(ks_stream_t stream, int64_t T, int64_t M, int32_t n
                              const uint8_t* fresh /*(T,M) nullable*/, float* g /*(T,M,ld) in place*/, float* d_y0 /*nullable*/);
 int ks_signed_permute(ks_stream_t stream, int64_t rows, int32_t n, const float* x, const int32_t* perm, const float* sign,
                       float* out);
+/* groups of `group` rows, x (groups, group, n) -> out (groups, 2 group, n): each group's rows, then their mirror images */
+int ks_mirror_pairs(ks_stream_t stream, int64_t groups, int64_t group, int32_t n, const float* x, const int32_t* perm, const float* sign,
+                    float* out);
 int ks_mirror_loss_grad(ks_stream_t stream, int64_t rows, int32_t n, float scale, const float* y, const float* ym,
                         const int32_t* perm, const float* sign, float* dy, float* dym, float* loss /*(rows), nullable*/);
 /* ksim/task/ppo.py:546-563 (adaptive KL in _single_step), without a trip to the host: with

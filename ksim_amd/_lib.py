@@ -69,6 +69,8 @@ def load() -> ctypes.CDLL:
     lib.ks_ppo_loss_grad.restype = c_int32
     lib.ks_signed_permute.argtypes = [p, c_int64, c_int32, p, p, p, p]
     lib.ks_signed_permute.restype = c_int32
+    lib.ks_mirror_pairs.argtypes = [p, c_int64, c_int64, c_int32, p, p, p, p]
+    lib.ks_mirror_pairs.restype = c_int32
     lib.ks_mirror_loss_grad.argtypes = [p, c_int64, c_int32, c_float, p, p, p, p, p, p, p]
     lib.ks_mirror_loss_grad.restype = c_int32
     lib.ks_lowpass_scan.argtypes = [p, c_int64, c_int64, c_int32, c_int32, c_float, c_float, p, p, p, c_int64, c_int32, c_int32, p, p, p, p]

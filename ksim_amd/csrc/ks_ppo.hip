@@ -1090,14 +1090,37 @@ __global__ __launch_bounds__(256) void lowpass_scan_backward_kernel(int64_t T, i
   if (d_y0) d_y0[idx] = carry;
 }
 
-// mirrored rows: out[r][j] = sign[j] * x[r][perm[j]]
-__global__ __launch_bounds__(256) void signed_permute_kernel(int64_t total, int n, const float* __restrict__ x, const int* __restrict__ perm,
-                                                             const float* __restrict__ sign, float* __restrict__ out) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const int64_t r = idx / n;
-  const int j = (int)(idx - r * n);
-  out[idx] = sign[j] * x[r * n + perm[j]];
+// Mirrored rows: mirror[r][j] = sign[j] * x[r][perm[j]], and a copy of the rows in `same` where the caller wants both.  Row r goes
+// (r / group) * group rows further down in either output, so that whole groups of rows and of images can alternate in one buffer.
+// Bound by memory.  A thread takes four columns of a row at a time; the last four of a row overlap the ones before where the width is odd
+// (the same values twice).  `magic` divides by the row's quads, of which a workgroup has few enough for it to be exact.
+//   100 x 512 rows of 475 and their images: 154 us as a permutation and a concatenation, 77 here
+struct __attribute__((packed, aligned(4))) RowQuad { float v[4]; };  // rows of an odd width start at any float; a 16-byte access needs no more
+__global__ __launch_bounds__(256) void mirror_rows_kernel(int64_t rows, int n, int per, unsigned magic, int64_t group, const float* __restrict__ x,
+                                                          const int* __restrict__ perm, const float* __restrict__ sign, float* __restrict__ same,
+                                                          float* __restrict__ mirror) {
+  const int64_t row0 = (int64_t)blockIdx.x * per, g0 = row0 / group, rest0 = row0 - g0 * group;
+  const int here = (int)(rows - row0 < per ? rows - row0 : per), quads = (n + 3) >> 2, count = here * quads;
+  const float* src = x + row0 * n;
+  for (int e = threadIdx.x; e < count; e += 256) {
+    const int r = per == 1 ? 0 : quads == 1 ? e : (int)__umulhi((unsigned)e, magic);
+    const int q = 4 * (e - r * quads), j = n >= 4 && q > n - 4 ? n - 4 : q;
+    const int64_t g = rest0 + r < group ? g0 : g0 + (rest0 + r) / group;
+    const int64_t at = (row0 + r + g * (same ? group : 0)) * n + j;
+    const float* row = src + (int64_t)r * n;
+    if (n >= 4) {
+      RowQuad m;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) m.v[k] = sign[j + k] * row[perm[j + k]];
+      if (same) *reinterpret_cast<RowQuad*>(same + at) = *reinterpret_cast<const RowQuad*>(row + j);
+      *reinterpret_cast<RowQuad*>(mirror + at) = m;
+    } else {
+      for (int k = 0; k < n; ++k) {
+        if (same) same[at + k] = row[k];
+        mirror[at + k] = sign[k] * row[perm[k]];
+      }
+    }
+  }
 }
 
 // One thread per (row, j): diff = y[r][j] - sign[j] ym[r][perm[j]].  perm is a bijection, so the thread owns dym[r][perm[j]].
@@ -1162,15 +1185,30 @@ extern "C" int ks_lowpass_scan_backward(ks_stream_t stream, int64_t T, int64_t M
   return ks::check_launch("ks_lowpass_scan_backward");
 }
 
+static int mirror_rows(const char* who, ks_stream_t stream, int64_t rows, int64_t group, int32_t n, const float* x, const int32_t* perm,
+                       const float* sign, float* same, float* mirror) {
+  const int quads = n / 4 + (n % 4 != 0), per = quads >= 1024 ? 1 : 1024 / quads;  // a thousand quads or one row per workgroup
+  const int64_t grid = (rows + per - 1) / per;
+  if (grid > 0x7fffffff) return ks::fail(KS_ELIMIT, "%s: too many elements", who);
+  hipLaunchKernelGGL(ks::mirror_rows_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, rows, n, per,
+                     (unsigned)((1ull << 32) / (unsigned)quads + 1), group, x, perm, sign, same, mirror);
+  return ks::check_launch(who);
+}
+
 extern "C" int ks_signed_permute(ks_stream_t stream, int64_t rows, int32_t n, const float* x, const int32_t* perm, const float* sign,
                                  float* out) {
   if (rows < 0 || n < 1) return ks::fail(KS_EINVAL, "ks_signed_permute: bad shape");
   if (rows == 0) return KS_OK;
   if (!x || !perm || !sign || !out || x == out) return ks::fail(KS_EINVAL, "ks_signed_permute: null pointer, or in place");
-  const int64_t total = rows * n, grid = (total + 255) / 256;
-  if (grid > 0x7fffffff) return ks::fail(KS_ELIMIT, "ks_signed_permute: too many elements");
-  hipLaunchKernelGGL(ks::signed_permute_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, total, n, x, perm, sign, out);
-  return ks::check_launch("ks_signed_permute");
+  return mirror_rows("ks_signed_permute", stream, rows, rows, n, x, perm, sign, nullptr, out);
+}
+
+extern "C" int ks_mirror_pairs(ks_stream_t stream, int64_t groups, int64_t group, int32_t n, const float* x, const int32_t* perm, const float* sign,
+                               float* out) {
+  if (groups < 0 || group < 0 || n < 1) return ks::fail(KS_EINVAL, "ks_mirror_pairs: bad shape");
+  if (groups == 0 || group == 0) return KS_OK;
+  if (!x || !perm || !sign || !out || x == out) return ks::fail(KS_EINVAL, "ks_mirror_pairs: null pointer, or in place");
+  return mirror_rows("ks_mirror_pairs", stream, groups * group, group, n, x, perm, sign, out, out + group * n);
 }
 
 extern "C" int ks_mirror_loss_grad(ks_stream_t stream, int64_t rows, int32_t n, float scale, const float* y, const float* ym,

@@ -146,9 +146,9 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
         perm, sign = policy.mirror.device(name, x.device)
         if perm.numel() != x.shape[1]:
             raise _lib.KsError(f"the {name} mirror map has {perm.numel()} entries, the rows have {x.shape[1]}")
+        x = x.to(torch.float32).contiguous()
         both = torch.empty(2 * rows, x.shape[1], dtype=torch.float32, device=x.device)
-        both[:rows].copy_(x)
-        _lib.check(lib.ks_signed_permute(st, rows, x.shape[1], _lib.addr(both[:rows]), _lib.addr(perm), _lib.addr(sign), _lib.addr(both[rows:])))
+        _lib.check(lib.ks_mirror_pairs(st, 1, rows, x.shape[1], _lib.addr(x), _lib.addr(perm), _lib.addr(sign), _lib.addr(both)))
         return both
 
     a_in = with_mirrored(a_obs, "actor_obs") if mirror_a else a_obs
@@ -369,9 +369,9 @@ def single_step_recurrent(policy: RecurrentHeadPolicy, cfg: PPOUpdateConfig, act
         if perm.numel() != x.shape[-1]:
             raise _lib.KsError(f"the {name} mirror map has {perm.numel()} entries, the rows have {x.shape[-1]}")
         x = x.contiguous()
-        xm = torch.empty_like(x)
-        _lib.check(lib.ks_signed_permute(st, rows, x.shape[-1], _lib.addr(x), _lib.addr(perm), _lib.addr(sign), _lib.addr(xm)))
-        return torch.cat([x, xm], dim=1).contiguous()
+        pairs = torch.empty(Tn, 2 * b, x.shape[-1], dtype=torch.float32, device=dev)
+        _lib.check(lib.ks_mirror_pairs(st, Tn, b, x.shape[-1], _lib.addr(x), _lib.addr(perm), _lib.addr(sign), _lib.addr(pairs)))
+        return pairs
 
     fresh2 = torch.cat([fresh, fresh], dim=1).contiguous() if (mirror_a or mirror_c) else None
     a_in = both(actor_obs, "actor_obs") if mirror_a else actor_obs.contiguous()

@@ -883,3 +883,20 @@ def test_weight_gradient_from_a_block_of_columns(dims, dtype, M, wide, first):
             continue
         with pytest.raises(KsError):
             net.layer_weight_grad(bad, dy)
+
+
+@pytest.mark.parametrize("groups,group,n", [(1, 1, 1), (3, 5, 2), (2, 700, 3), (7, 3, 4), (5, 9, 5), (4, 33, 65), (2, 100, 475), (3, 2, 4099), (0, 4, 8)])
+def test_rows_and_their_mirror_images_in_one_pass(groups, group, n):
+    """Rows narrower than four, wider than a workgroup's share, groups that a workgroup straddles; against indexing."""
+    from ksim_amd import _lib
+
+    rng = np.random.default_rng(n)
+    x = t32(rng.normal(size=(groups, group, n)))
+    perm, sign = rng.permutation(n), rng.choice([-1.0, 1.0], size=n)
+    p, s = torch.from_numpy(perm.astype(np.int32)).to(DEV), t32(sign)
+    image = x[..., torch.from_numpy(perm).to(DEV)] * s
+    lib, st = _lib.load(), _lib.current_stream()
+    out, alone = torch.full((groups, 2 * group, n), float("nan"), device=DEV), torch.full_like(x, float("nan"))
+    _lib.check(lib.ks_mirror_pairs(st, groups, group, n, _lib.addr(x), _lib.addr(p), _lib.addr(s), _lib.addr(out)))
+    _lib.check(lib.ks_signed_permute(st, groups * group, n, _lib.addr(x), _lib.addr(p), _lib.addr(s), _lib.addr(alone)))
+    assert torch.equal(out, torch.cat([x, image], dim=1)) and torch.equal(alone, image)
