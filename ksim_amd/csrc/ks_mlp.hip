@@ -74,14 +74,14 @@ __device__ __forceinline__ u32x4 load_first(const float* __restrict__ x, int64_t
 // BM: rows per workgroup (128, or 64 for small batches so that the grid still covers every CU twice).
 // The K loop is software-pipelined: the global loads of slice k+1 are issued into registers before the MFMAs
 // of slice k run out of LDS, so HBM/L2 latency overlaps the matrix-core work.
-template <typename T, bool FIRST, bool LAST, int ACT, int BM, int BN, int WAVES_M, int WAVES_N, int KMUL = 1>
+template <typename T, bool FIRST, bool LAST, int ACT, int BM, int BN, int WAVES_M, int WAVES_N>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void mlp_layer_kernel(int64_t M, int K /*padded to BK*/, int Kreal, int Nreal,
                                                         const void* __restrict__ xin, int64_t ldx,
                                                         const T* __restrict__ W /*(Np, K)*/,
                                                         const float* __restrict__ bias /*(Np)*/,
                                                         void* __restrict__ yout, int64_t ldy) {
   static_assert(sizeof(T) == 2, "fp32 layers have a kernel of their own");
-  constexpr int BK = 64 * KMUL;          // elements of K per slice (KMUL 2: half the barriers per flop, twice the LDS)
+  constexpr int BK = 64;                 // elements of K per slice
   constexpr int PAD = 8;                 // keeps 16-byte row alignment and spreads LDS banks
   constexpr int VEC = 16 / sizeof(T);    // elements per 16-byte load
   constexpr int NT = 64 * WAVES_M * WAVES_N;    // threads per workgroup
@@ -646,12 +646,9 @@ struct FusedArgs {
   // training forward: hidden layer l's activations also go to save[l], (M, save_ld[l]) row-major in working precision, for the backward pass
   void* save[KS_MAX_LAYERS];
   int save_ld[KS_MAX_LAYERS];
-  // training forward for the whole-network backward kernel: hidden layer l's activations transposed, keep_t[l]: (width, ldt).
-  // The weight-gradient product takes them as they are, and the backward kernel's epilogue reads its f'(Y) from them.
-  __bf16* keep_t[KS_MAX_LAYERS];
-  __bf16* keep_t_in;  // the network input, transposed: (in_t_width, ldt), zero beyond the real inputs
-  int in_t_width;
-  int64_t ldt;
+  int64_t save_rows;  // rows of the saved arrays: M, or the whole tiles' (what the padding rows hold is finite and of no use)
+  void* save_in;      // nullable: the network input as well, (save_rows, in_width) in working precision, zero beyond the real inputs
+  int in_width;       // 0 without save_in
 };
 
 #ifdef KS_PROFILE
@@ -743,11 +740,9 @@ __device__ __forceinline__ void fused_bias_init(f32x16& acc, const float* __rest
 }
 
 // Hidden layer: activation, round to bf16, back into the tile (4 consecutive features = one 8-byte LDS store).
-// `keep_t` (nullable) points at the transposed copy's entry (feature 0, this lane's row): across the 32 lanes of a half the
-// same register holds 32 consecutive rows of one feature, so a 2-byte store per lane writes two whole 64-byte runs.
 template <int ACT, typename T>
 __device__ __forceinline__ void fused_store_hidden(const f32x16& acc, T* __restrict__ act, int lda, int j,
-                                                   int row, int lane, __bf16* __restrict__ keep_t = nullptr, int64_t ldt = 0) {
+                                                   int row, int lane) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int f0 = j * 32 + 8 * g + 4 * (lane >> 5);
@@ -759,36 +754,19 @@ __device__ __forceinline__ void fused_store_hidden(const f32x16& acc, T* __restr
     const uint2 packed = {pack_bf16(activate<ACT, true>(acc[4 * g]), activate<ACT, true>(acc[4 * g + 1])),
                           pack_bf16(activate<ACT, true>(acc[4 * g + 2]), activate<ACT, true>(acc[4 * g + 3]))};
     *reinterpret_cast<uint2*>(act + row * lda + f0) = packed;
-    if (keep_t) {
-      unsigned short* o = reinterpret_cast<unsigned short*>(keep_t) + (int64_t)f0 * ldt;
-      o[0] = (unsigned short)packed.x; o[ldt] = (unsigned short)(packed.x >> 16);
-      o[2 * ldt] = (unsigned short)packed.y; o[3 * ldt] = (unsigned short)(packed.y >> 16);
-    }
   }
 }
 
-// The finished 128-row tile, transposed, to dst (width, ld): thread p takes the columns 2 p and 2 p + 1 of the tile (one
-// 4-byte LDS read per row), 8 rows per 16-byte store (a run of 256 bytes per column and tile), and returns the columns' sums.
-__device__ __forceinline__ f32x2 tile_transposed_out(const __bf16* __restrict__ act, int lda, int p, __bf16* __restrict__ dst, int64_t ld,
-                                                     int64_t m0) {
-  f32x2 s = {0.f, 0.f};
-  __bf16* out0 = dst + (int64_t)(2 * p) * ld + m0;
-  __bf16* out1 = out0 + ld;
-#pragma unroll 2
-  for (int r0 = 0; r0 < 128; r0 += 8) {
-    bf16x2 v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const bf16x2*>(act + (r0 + k) * lda + 2 * p);
-    __bf16 a[8], b[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      a[k] = v[k][0]; b[k] = v[k][1];
-      s[0] += (float)a[k]; s[1] += (float)b[k];
-    }
-    *reinterpret_cast<uint4*>(out0 + r0) = *reinterpret_cast<const uint4*>(a);
-    *reinterpret_cast<uint4*>(out1 + r0) = *reinterpret_cast<const uint4*>(b);
-  }
-  return s;
+// The first `ld` columns of the finished tile's rows (zeros from column `held` on), 16 bytes per thread and pass, to rows m0.. of dst (M, ld); rows
+// from M on are left out.  ld: whole 16-byte pieces, at most one pass of the workgroup.
+template <typename T, int ROWS>
+__device__ __forceinline__ void tile_rows_out(const T* __restrict__ act, int lda, T* __restrict__ dst, int ld, int held, int64_t m0, int64_t M) {
+  constexpr int PC = 16 / (int)sizeof(T);  // entries of a piece
+  const int pieces = ld / PC, per = 64 * kFusedWaves / pieces, r0 = (int)threadIdx.x / pieces, c = ((int)threadIdx.x - r0 * pieces) * PC;
+  if (r0 >= per) return;
+  const int rows = M - m0 < ROWS ? (int)(M - m0) : ROWS;
+  for (int r = r0; r < rows; r += per)
+    *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c) = c < held ? *reinterpret_cast<const uint4*>(act + r * lda + c) : uint4{0u, 0u, 0u, 0u};
 }
 
 // Output layer: fp32 rows of the caller's (M, out_dim) matrix.
@@ -834,7 +812,7 @@ __host__ __device__ inline int fused_share(int nt, int lda) {
 }
 
 // One layer of the whole-network kernel for one wavefront: MFMA work, barrier, epilogue, barrier.
-template <int ACT, typename T, int MI, bool LAST, bool KEEP, bool SWAP = false>
+template <int ACT, typename T, int MI, bool LAST, bool SWAP = false>
 __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __restrict__ act, int64_t m0, int lane,
                                             int wave, int64_t tile) {
   const int nk = a.fk[l], nt = a.fn[l], lda = a.lda;
@@ -925,30 +903,18 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
         for (int i = 0; i < MI; ++i) {
           if (SWAP) fused_store_output_swapped(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32, lane);
           else if (LAST) fused_store_output(acc[t][i], a.y, a.M, a.out_dim, j, m0 + i * 32 + row, lane);
-          else fused_store_hidden<ACT, T>(acc[t][i], act, lda, j, i * 32 + row, lane,
-                                       (KEEP && MI == 4) ? a.keep_t[l] + m0 + i * 32 + row : nullptr, a.ldt);
+          else fused_store_hidden<ACT, T>(acc[t][i], act, lda, j, i * 32 + row, lane);
         }
       }
   }
   __syncthreads();
   KS_MLP_STAMP2(4 + 3 * l)
-  if (!LAST && a.save[l]) {
-    // the finished tile, 16 bytes per thread and pass, rows as contiguous runs; the next layer only reads the tile until every
-    // wavefront (this copy included, which sits before its matrix work in program order) has passed the next barrier
-    constexpr int PC = 16 / (int)sizeof(T);  // entries of a 16-byte piece
-    T* dst = reinterpret_cast<T*>(a.save[l]);
-    // rows are as wide as the backward pass's layers, which is more than the tile's (zeros) where the width is no multiple of 128
-    const int ld = a.save_ld[l], w8 = ld / PC, held = nt * (32 / PC);
-    for (int idx = threadIdx.x; idx < MI * 32 * w8; idx += 64 * kFusedWaves) {
-      const int r = idx / w8, c8 = idx - r * w8;
-      if (m0 + r < a.M)
-        *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c8 * PC) =
-            c8 < held ? *reinterpret_cast<const uint4*>(act + r * lda + c8 * PC) : uint4{0u, 0u, 0u, 0u};
-    }
-  }
+  // The next layer only reads the tile until every wavefront (this copy included, which sits before its matrix work in program order) has passed
+  // the next barrier.  Rows are as wide as the backward pass's layers, which is more than the tile's (zeros) where the width is no multiple of 128.
+  if (!LAST && a.save[l]) tile_rows_out<T, MI * 32>(act, lda, reinterpret_cast<T*>(a.save[l]), a.save_ld[l], nt * 32, m0, a.save_rows);
 }
 
-template <int ACT, typename T, int BM, bool KEEP = false, bool SINGLE = false>
+template <int ACT, typename T, int BM, bool SINGLE = false>
 __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile) {
   constexpr int MI = BM / 32;
   constexpr int NTHR = 64 * kFusedWaves;
@@ -961,7 +927,7 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   KS_MLP_STAMP(0)
   {  // network input -> tile; zero beyond the batch and in the K padding of the first layer
     const int in_dim = a.in_dim;
-    const int K0 = (KEEP && a.in_t_width > a.fk[0] * SK) ? a.in_t_width : a.fk[0] * SK;  // the transposed copy is padded further
+    const int K0 = a.in_width > a.fk[0] * SK ? a.in_width : a.fk[0] * SK;  // the copy that is kept is padded further
     const int64_t rows_left = a.M - m0;
     const int rows = rows_left < BM ? (int)rows_left : BM;
     const float* src = a.x + m0 * in_dim;
@@ -1016,19 +982,17 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   }
   __syncthreads();
   KS_MLP_STAMP(1)
-  if constexpr (KEEP && BM == 128) if (a.keep_t_in && tid < a.in_t_width / 2)  // the first layer overwrites the tile only after its barrier
-    (void)tile_transposed_out(act, lda, tid, a.keep_t_in, a.ldt, m0);
+  if (a.save_in) tile_rows_out<T, BM>(act, lda, reinterpret_cast<T*>(a.save_in), a.in_width, a.in_width, m0, a.save_rows);  // the tile stays until the first layer's barrier
   if constexpr (!SINGLE)
-    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false, KEEP>(a, l, act, m0, lane, wave, tile);
-  fused_layer<ACT, T, MI, true, KEEP, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
+    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false>(a, l, act, m0, lane, wave, tile);
+  fused_layer<ACT, T, MI, true, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
 }
 
-// KEEP: the training forward that also stores every hidden layer's activations and the network input transposed
-// (FusedArgs::keep_t, keep_t_in; 128-row tiles only).  SINGLE: one bf16 layer
-template <int ACT, typename T, int BM, bool KEEP = false, bool SINGLE = false>
+// SINGLE: one bf16 layer
+template <int ACT, typename T, int BM, bool SINGLE = false>
 __global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
 void mlp_fused_kernel(const FusedArgs a) {
-  mlp_fused_body<ACT, T, BM, KEEP, SINGLE>(a, blockIdx.x);
+  mlp_fused_body<ACT, T, BM, SINGLE>(a, blockIdx.x);
 }
 
 // Two networks over the same rows in one launch (actor and critic of a control step): blockIdx.y picks the network, so
@@ -1213,23 +1177,24 @@ void mlp_split_layer_kernel(const SplitLayer p, const SplitLayer q) {
 }
 
 // ---------------------------------------------------------------- whole-network backward pass of the hidden layers
-// dZ_{l-1} = (dZ_l W_l) * f'(Y_{l-1}) for l = L-1 .. 1 in one launch, a 128-row tile per workgroup that never leaves LDS: the
-// product is the forward kernel's K loop over the fragment-ordered transposed weights, its epilogue reads f'(Y) from the
-// transposed activations the training forward stored (FusedArgs::keep_t) and writes the new tile both into LDS and, transposed,
-// to memory (the operand of the weight-gradient product: in the accumulator layout the 32 lanes of a half hold 32 consecutive
-// rows of one feature, so 2-byte loads and stores per lane move whole 64-byte runs), and the tile's column sums follow (the
-// bias gradient, one partial row per tile).
+// dZ_{l-1} = (dZ_l W_l) * f'(Y_{l-1}) for l = L-1 .. 1 in one launch, a 128-row tile per workgroup that never leaves LDS: the product is the
+// forward kernel's K loop over the fragment-ordered transposed weights, its epilogue multiplies by f' of the activations that the training
+// forward left, and the finished tile goes out row by row (an operand of the weight gradients below) with its column sums (the bias
+// gradient, one partial row per tile).
+// Bound by the products (58 us at the rate of a large product) and the tile's way in and out of memory (80 at the copy rate), which a single
+// workgroup per CU does one after the other.  65536 rows of 68-512-512-512-20: 174 -> 157 us (203 -> 185 just behind other kernels) since
+// activations and gradients move as whole rows; as transposes every lane loaded and stored 2 bytes at a time.  Column sums over half the rows
+// a thread would keep all wavefronts busy with them, but their partial rows cost the final sum more than that gains.
 struct FusedBwdArgs {
   int64_t M;
   int n_layers, lda;
   int fk[KS_MAX_LAYERS], fn[KS_MAX_LAYERS];   // the forward kernel's K steps and output tiles per layer
   const u32x4* WtP[KS_MAX_LAYERS];            // l >= 1: W_l^T in fragment order, [input tile][step over outputs][lane] x 16 bytes
   const float* dy;                            // (M, out_dim): gradient of the network output, in the caller's layout
-  int out_dim, np_last;                       // np_last: rows of dzT[L-1] (the output width padded for the weight-gradient product)
-  const __bf16* yT[KS_MAX_LAYERS];            // hidden layer l's activations, transposed (width, ldt), as the training forward left them
-  __bf16* dzT[KS_MAX_LAYERS];                 // out, every layer: dZ_l^T (width, ldt)
+  int out_dim, np_last;                       // np_last: columns of dz[L-1] (the output width padded for the weight-gradient product)
+  const __bf16* y[KS_MAX_LAYERS];             // hidden layer l's activations, row-major, as the training forward left them
+  __bf16* dz[KS_MAX_LAYERS];                  // out, every layer: dZ_l (whole tiles of rows, width); zero beyond the batch
   float* bias_part[KS_MAX_LAYERS];            // out, every layer: (tiles, width) column sums of dZ_l per tile
-  int64_t ldt;
 };
 
 template <int ACT>
@@ -1250,12 +1215,21 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     }
   }
   __syncthreads();
-  if (tid < a.np_last / 2) {  // its transpose and column sums; the first K loop below only reads the tile
-    const f32x2 cs = tile_transposed_out(act, lda, tid, a.dzT[L - 1], a.ldt, m0);
-    float* part = a.bias_part[L - 1] + tile * a.np_last + 2 * tid;
+  // The finished tile and its column sums (the bias gradient's share) go out while the next K loop reads the tile, as this does
+  auto tile_out = [&](__bf16* dst, float* bias_part, int width) {
+    tile_rows_out<__bf16, BM>(act, lda, dst, width, width, m0, m0 + BM);
+    if (tid >= width / 2) return;
+    f32x2 cs = {0.f, 0.f};
+#pragma unroll 8
+    for (int r = 0; r < BM; ++r) {
+      const bf16x2 v = *reinterpret_cast<const bf16x2*>(act + r * lda + 2 * tid);
+      cs[0] += (float)v[0]; cs[1] += (float)v[1];
+    }
+    float* part = bias_part + tile * width + 2 * tid;
     part[0] = cs[0];
     part[1] = cs[1];
-  }
+  };
+  tile_out(a.dz[L - 1], a.bias_part[L - 1], a.np_last);
   const __bf16* arow = act + (lane & 31) * lda + (lane >> 5) * 8;
   const int row = lane & 31;
   for (int l = L - 1; l >= 1; --l) {
@@ -1274,67 +1248,171 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     const u32x4* w1 = a.WtP[l] + (int64_t)j1 * nk * 64 + lane;
     if (mine == 2) fused_layer_mma<__bf16, 2, MI, kPF>(acc, w0, w1, nk, arow, lda);
     else if (mine == 1) fused_layer_mma<__bf16, 1, MI, kPF>(acc, w0, w0, nk, arow, lda);
-    __syncthreads();  // every wavefront has read dZ_l; the tile can take dZ_{l-1}
-    // Epilogue in blocks of one (feature tile, row tile) pair = 16 accumulator registers.  A block's 16 activations Y_{l-1} come
-    // from the transposed copy (per feature, 32 lanes read 32 consecutive rows); the next block's loads are issued before this
-    // block is worked on, so their latency hides behind it instead of adding up 32 times per layer.
-    auto y_block = [&](int blk, unsigned short (&yv)[16]) {
-      const int t = blk >> 2, i = blk & 3;
-      const int j = t == 0 ? j0 : j1;
-      const unsigned short* y = reinterpret_cast<const unsigned short*>(a.yT[l - 1]) + m0 + i * 32 + row;
+    // Y_{l-1} takes dZ_l's place in the tile on its way to the lanes that need it, and every lane leaves dZ_{l-1} where it read Y: whole rows in
+    // 16-byte pieces in and out of memory, 8 bytes per lane of the tile.
+    const int width = nt * 32, pieces = width / 8, per = NTHR / pieces, yr = tid / pieces, yc = (tid - yr * pieces) * 8;
+    u32x4 yv[16];  // a width of 512: 8 rows a pass
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const unsigned short* yg = y + (int64_t)(j * 32 + 8 * g + 4 * (lane >> 5)) * a.ldt;
+    for (int u = 0; u < 16; ++u) {
+      const int r = yr + u * per;
+      yv[u] = u32x4{0u, 0u, 0u, 0u};
+      if (yr < per && r < BM && m0 + r < a.M) yv[u] = *reinterpret_cast<const u32x4*>(a.y[l - 1] + (m0 + r) * width + yc);
+    }
+    __syncthreads();  // every wavefront has read dZ_l
 #pragma unroll
-        for (int e = 0; e < 4; ++e) yv[4 * g + e] = yg[e * a.ldt];
-      }
-    };
-    unsigned short ya[16], yb[16];
-    const int nblk = mine * MI;
-    if (nblk > 0) y_block(0, ya);
-#pragma unroll
-    for (int blk = 0; blk < 2 * MI; ++blk) {
-      if (blk < nblk) {
-        unsigned short (&cur)[16] = (blk & 1) ? yb : ya;
-        unsigned short (&nxt)[16] = (blk & 1) ? ya : yb;
-        if (blk + 1 < nblk) y_block(blk + 1, nxt);
-        const int t = blk >> 2, i = blk & 3;
-        const int j = t == 0 ? j0 : j1;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float d[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float yv = __builtin_bit_cast(float, (unsigned)cur[4 * g + e] << 16);
-            d[e] = 1.f;
-            if (ACT == KS_ACT_ELU) d[e] = yv > 0.f ? 1.f : yv + 1.f;
-            if (ACT == KS_ACT_RELU) d[e] = yv > 0.f ? 1.f : 0.f;
-            if (ACT == KS_ACT_TANH) d[e] = 1.f - yv * yv;
-            d[e] *= acc[t][i][4 * g + e];
-          }
-          const int f0 = j * 32 + 8 * g + 4 * (lane >> 5);
-          const uint2 packed = {pack_bf16(d[0], d[1]), pack_bf16(d[2], d[3])};
-          *reinterpret_cast<uint2*>(act + (i * 32 + row) * lda + f0) = packed;
-          // transposed, straight from the registers: 32 lanes hold 32 consecutive rows of one feature
-          unsigned short* o = reinterpret_cast<unsigned short*>(a.dzT[l - 1]) + (int64_t)f0 * a.ldt + m0 + i * 32 + row;
-          o[0] = (unsigned short)packed.x; o[a.ldt] = (unsigned short)(packed.x >> 16);
-          o[2 * a.ldt] = (unsigned short)packed.y; o[3 * a.ldt] = (unsigned short)(packed.y >> 16);
-        }
-      }
+    for (int u = 0; u < 16; ++u) {
+      const int r = yr + u * per;
+      if (yr < per && r < BM) *reinterpret_cast<u32x4*>(act + r * lda + yc) = yv[u];
     }
     __syncthreads();
-    if (tid < nt * 16) {  // column sums of the new tile (the bias gradient's share); the next K loop only reads the tile, as this does
-      f32x2 cs = {0.f, 0.f};
-#pragma unroll 8
-      for (int r = 0; r < BM; ++r) {
-        const bf16x2 v = *reinterpret_cast<const bf16x2*>(act + r * lda + 2 * tid);
-        cs[0] += (float)v[0]; cs[1] += (float)v[1];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (t < mine) {
+        const int j = t == 0 ? j0 : j1;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            uint2* at = reinterpret_cast<uint2*>(act + (i * 32 + row) * lda + j * 32 + 8 * g + 4 * (lane >> 5));
+            const uint2 y4 = *at;
+            float d[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const unsigned w = e < 2 ? y4.x : y4.y;
+              const float yv1 = __builtin_bit_cast(float, (e & 1) ? w & 0xffff0000u : w << 16);
+              d[e] = 1.f;
+              if (ACT == KS_ACT_ELU) d[e] = yv1 > 0.f ? 1.f : yv1 + 1.f;
+              if (ACT == KS_ACT_RELU) d[e] = yv1 > 0.f ? 1.f : 0.f;
+              if (ACT == KS_ACT_TANH) d[e] = 1.f - yv1 * yv1;
+              d[e] *= acc[t][i][4 * g + e];
+            }
+            *at = uint2{pack_bf16(d[0], d[1]), pack_bf16(d[2], d[3])};
+          }
       }
-      float* part = a.bias_part[l - 1] + tile * (nt * 32) + 2 * tid;
-      part[0] = cs[0];
-      part[1] = cs[1];
-    }
+    __syncthreads();
+    tile_out(a.dz[l - 1], a.bias_part[l - 1], width);
   }
+}
+
+// Weight gradients behind it: slice z of C (np, kp) = dZ^T Y over rows [z kslice, (z + 1) kslice) of dZ (lda = np columns) and Y (ldb columns), both
+// row-major as the kernels above left them, in whole tiles of 128 rows of which dZ's are zero beyond the batch; 128 x 128 tiles.  Both operands are wanted with their rows as the reduction, which is what the
+// transposing LDS read gives: sixteen lanes that point at four rows of sixteen columns receive four rows of one column each.  A row of the tile
+// is padded by 64 bytes, so that four rows lie on different banks.
+// Eight wavefronts: two groups of four take one half of the slice's rows each, every wavefront a quarter of the tile; the second group hands its
+// sums over through LDS at the end, so a slice is one copy of the gradient.  A stage is 32 rows, the next one's pieces are in flight over the
+// products and go to the other buffer behind them: one barrier per stage.  The pieces of two stages are on their way at a time.
+// 65536 rows, against the products of transposes that this replaces: 512 x 512 63 -> 50 us (34 GFLOP, 28 us at the rate of a large product; 134
+// MB of operands, 26), 512 x 128 and 128 x 512 33 and 29 -> 24, and the sum of half as many slices 26 -> 24.  128 x 256 tiles take 48 us and
+// leave twice the slices; two workgroups per CU on half the rows each take 52.  Whole gradient of 68-512-512-512-20: 392 -> 336 us.
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+constexpr int kCwRows = 32, kCwStride = 2 * 128 + 64 /* bytes */, kCwLds = 2 * 2 * 2 * kCwRows * kCwStride;  // group, buffer, operand
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void chain_wgrad_kernel(int64_t Mp, int np, int ldb, int kp, int kslice, const __bf16* __restrict__ A, const __bf16* __restrict__ B,
+                        float* __restrict__ C) {
+  constexpr int S = kCwStride, BUF = 2 * kCwRows * S, NP = kCwRows * 16 / 256;  // a stage; 16-byte pieces of an operand's stage per thread
+  extern __shared__ __attribute__((aligned(16))) unsigned char mlp_lds[];
+  // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD
+  int tile = blockIdx.x, z = blockIdx.y;
+  {
+    const int l = blockIdx.y * gridDim.x + blockIdx.x, q = l >> 3;
+    tile = q % gridDim.x;
+    z = (q / gridDim.x) * 8 + (l & 7);
+  }
+  const int tiles_j = ldb / 128, i0 = tile / tiles_j * 128, j0 = tile % tiles_j * 128;
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t = threadIdx.x & 255, wave = t >> 6, lane = t & 63;
+  const int64_t zbeg = min(Mp, (int64_t)z * kslice), zend = min(Mp, zbeg + kslice);
+  const int half = (int)((zend - zbeg) / 2), stages = half / kCwRows;  // an even number of whole stages, the same for both groups
+  const int64_t kbeg = zbeg + grp * half;
+  unsigned char* buf = mlp_lds + grp * 2 * BUF;
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+  const int row = t >> 4, piece = t & 15;  // the thread's pieces of a stage: rows `row` and row + 16
+  const unsigned oa = row * np + 8 * piece, ob = row * ldb + 8 * piece;
+  u32x4 ra[2][NP], rb[2][NP];
+  auto fetch = [&](int n, u32x4 (&ra)[NP], u32x4 (&rb)[NP]) __attribute__((always_inline)) {
+    const int64_t k0 = kbeg + (int64_t)min(n, stages - 1) * kCwRows;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) ra[u] = *reinterpret_cast<const u32x4*>(A + (k0 + 16 * u) * np + i0 + oa);
+#pragma unroll
+    for (int u = 0; u < NP; ++u) rb[u] = *reinterpret_cast<const u32x4*>(B + (k0 + 16 * u) * ldb + j0 + ob);
+  };
+  auto put = [&](unsigned char* to, const u32x4 (&ra)[NP], const u32x4 (&rb)[NP]) __attribute__((always_inline)) {
+    to += row * S + 16 * piece;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) *reinterpret_cast<u32x4*>(to + 16 * u * S) = ra[u];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) *reinterpret_cast<u32x4*>(to + (kCwRows + 16 * u) * S) = rb[u];
+  };
+  // lane's part of a fragment of 32 columns and 16 rows: column lane % 32, rows 8 (lane / 32) + 0..7, four per read
+  const int frow = 8 * (lane >> 5) + ((lane & 15) >> 2), fcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  typedef s16x4_t __attribute__((address_space(3))) * lds_quad;
+  auto frag = [&](const unsigned char* at) __attribute__((always_inline)) {
+    const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_quad)(at)), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_quad)(at + 4 * S));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
+  if (stages > 0) {
+    fetch(0, ra[0], rb[0]);
+    fetch(1, ra[1], rb[1]);
+    put(buf, ra[0], rb[0]);
+  }
+  for (int n = 0; n < stages; n += 2)
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    fetch(n + u + 2, ra[u], rb[u]);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS only: the requested pieces stay in flight
+    const unsigned char* from = buf + u * BUF;
+    bf16x8 fa[kCwRows / 16][2], fb[kCwRows / 16][2];
+#pragma unroll
+    for (int s = 0; s < kCwRows / 16; ++s) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) fa[s][a] = frag(from + (16 * s + frow) * S + 2 * (wi + 32 * a + fcol));
+#pragma unroll
+      for (int b = 0; b < 2; ++b) fb[s][b] = frag(from + (kCwRows + 16 * s + frow) * S + 2 * (wj + 32 * b + fcol));
+    }
+#pragma unroll
+    for (int s = 0; s < kCwRows / 16; ++s)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][a], fb[s][b], acc[a][b], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    put(buf + (1 - u) * BUF, ra[1 - u], rb[1 - u]);  // the last one's is not read
+  }
+  // the second group's sums, a row of matrix tiles at a time
+  float* mine = reinterpret_cast<float*>(mlp_lds) + t;
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    __syncthreads();
+    if (grp == 1)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mine[(16 * b + r) * 256] = acc[a][b][r];
+    __syncthreads();
+    if (grp == 0)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][b][r] += mine[(16 * b + r) * 256];
+  }
+  if (grp == 1) return;
+  float* out = C + (int64_t)z * np * kp;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int gj = j0 + wj + 32 * b + (lane & 31);
+      if (gj >= kp) continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) out[(int64_t)(i0 + wi + 32 * a + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kp + gj] = acc[a][b][r];
+    }
 }
 
 struct DevMlp {
@@ -1359,7 +1437,7 @@ struct DevMlp {
   float *m1W[KS_MAX_LAYERS], *m2W[KS_MAX_LAYERS], *m1b[KS_MAX_LAYERS], *m2b[KS_MAX_LAYERS];
   void* Wt[KS_MAX_LAYERS];      // (kpad, npad) working-precision transpose
   void* WtP[KS_MAX_LAYERS];     // whole-network kernel only, l >= 1 or a single layer: W_l^T in fragment order, for the input gradients
-  int chain_saved;              // the last training forward kept the activations in the whole-network backward pass's formats
+  int chain_saved;              // the last training forward kept what the whole-network backward pass reads
   int bias_frozen[KS_MAX_LAYERS];  // leading bias entries of the layer that the optimiser leaves alone
   float* zero_bias;             // zeros, as wide as the widest GEMM output
   double* sq_part;              // kSqBlocks partial sums of squares per gradient tensor (weights and biases of every layer)
@@ -1833,16 +1911,16 @@ static uint16_t f32_to_bf16_rne(float f) {
   return (uint16_t)(u >> 16);
 }
 
-template <typename T, bool FIRST, bool LAST, int BM, int BN, int WAVES_M, int WAVES_N, int KMUL = 1>
+template <typename T, bool FIRST, bool LAST, int BM, int BN, int WAVES_M, int WAVES_N>
 static int launch_layer_tile(int act, hipStream_t s, int64_t M, int npad, int K, int Kreal, int Nreal, const void* x,
                              int64_t ldx, const void* W, const float* b, void* y, int64_t ldy, int ksplit = 1) {
-  constexpr int BK = 64 * KMUL, PAD = 8;
+  constexpr int BK = 64, PAD = 8;
   constexpr int lds = (int)sizeof(T) * (BM + BN) * (BK + PAD);
   const dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)(npad / BN), (unsigned)ksplit);
   const dim3 block(64 * WAVES_M * WAVES_N);
 #define KS_LAUNCH(A)                                                                                           \
   {                                                                                                            \
-    auto kfn = mlp_layer_kernel<T, FIRST, LAST, A, BM, BN, WAVES_M, WAVES_N, KMUL>;                            \
+    auto kfn = mlp_layer_kernel<T, FIRST, LAST, A, BM, BN, WAVES_M, WAVES_N>;                                  \
     if (lds > 64 * 1024 &&                                                                                     \
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
       return fail(KS_ELAUNCH, "ks_mlp_forward: cannot raise the LDS limit to %d bytes", lds);                  \
@@ -2017,19 +2095,21 @@ static FusedArgs fused_args(const DevMlp& m, int64_t M, const float* x, float* y
 // A single bf16 layer given by its arguments (no hidden layers, nothing kept), on the row tiles of launch_fused
 static int launch_fused_args(const FusedArgs& a, hipStream_t s);
 
-struct TrainWs;
-static void keep_args(FusedArgs& a, const DevMlp& m, const TrainWs* ws);
-
 template <typename T, int BM>
 static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const float* x, float* y, char* const* save,
-                             const TrainWs* keep = nullptr) {
+                             char* save_in = nullptr) {
   FusedArgs a = fused_args(m, M, x, y);
   if (save)
     for (int l = 0; l + 1 < m.n_layers; ++l) {
       a.save[l] = save[l];
       a.save_ld[l] = m.npad[l];
     }
-  if (keep) keep_args(a, m, keep);
+  a.save_rows = M;
+  if (save_in) {
+    a.save_in = save_in;
+    a.save_rows = (M + 127) / 128 * 128;
+    a.in_width = round_up(m.kpad[0], kBN);
+  }
 #ifdef KS_PROFILE
   if (const char* e = getenv("KS_MLP_PROF_PTR")) a.prof = (long long*)strtoull(e, nullptr, 16);
 #endif
@@ -2038,10 +2118,9 @@ static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const fl
   if (blocks > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward: too many rows");
 #define KS_LAUNCH(A)                                                                                           \
   {                                                                                                            \
-    constexpr bool kKeep = BM == 128 && sizeof(T) == 2;                                                        \
-    auto kfn = (keep && kKeep) ? mlp_fused_kernel<A, T, BM, kKeep> : mlp_fused_kernel<A, T, BM, false>;        \
+    auto kfn = mlp_fused_kernel<A, T, BM>;                                                                     \
     if constexpr (sizeof(T) == 2 && BM != 64)                                                                  \
-      if (m.n_layers == 1) kfn = mlp_fused_kernel<KS_ACT_NONE, T, BM, false, true>;                            \
+      if (m.n_layers == 1) kfn = mlp_fused_kernel<KS_ACT_NONE, T, BM, true>;                                   \
     if (lds > 64 * 1024 &&                                                                                     \
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)  \
       return fail(KS_ELAUNCH, "ks_mlp_forward: cannot raise the LDS limit to %d bytes", lds);                  \
@@ -2084,7 +2163,7 @@ static int launch_fused(const DevMlp& m, hipStream_t s, int64_t M, const float* 
 
 static int launch_fused_args(const FusedArgs& a, hipStream_t s) {
   const int bm = a.M >= 128 * 256 ? 128 : 32, lds = bm * a.lda * 2;
-  auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128, false, true> : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32, false, true>;
+  auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128, true> : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32, true>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
   hipLaunchKernelGGL(kfn, dim3((unsigned)((a.M + bm - 1) / bm)), dim3(64 * kFusedWaves), lds, s, a);
@@ -2413,11 +2492,12 @@ static void refresh_layers(DevMlp& m, hipStream_t s) {
 }
 
 constexpr int kDwSplit = 32;  // slices the weight-gradient reduction over the rows is cut into
-// Behind the whole-network backward pass: more slices where 32 of them leave CUs without a tile, down to 512 rows each
-// (65536 x 512 x 128, 4 tiles: 42 us with 32 slices, 31.5 with 64; 128 add 9 us to the slices' sum for nothing).
+// Slices of the whole-network backward pass's weight gradients (chain_wgrad_kernel): a workgroup per CU, at most 64 slices (every slice is a copy
+// of the gradient to write and to add up: 65536 x 512 x 512 with 32 instead of 16, 52 us instead of 50 and 27 instead of 24 for the sums) of 512
+// rows or more.
 static int chain_dw_slices(int np, int kp128, int64_t Mp) {
-  int ks = kDwSplit;
-  while (ks < 64 && ks * (np / 128) * (kp128 / 128) < 512 && Mp >= 1024 * (int64_t)ks) ks *= 2;
+  int ks = 8;
+  while (ks < 64 && ks * (np / 128) * (kp128 / 128) < 256 && Mp >= 1024 * (int64_t)ks) ks *= 2;
   return ks;
 }
 // Slices of the row reduction of a single layer's weight gradient (wgrad_kernel, 128 x 128 tiles): a workgroup per CU (its registers
@@ -2439,9 +2519,9 @@ struct TrainWs {
   char *d0, *d1, *t0, *t1, *t2;
   float* part;  // partial sums of the split reductions
   int64_t Mp;
-  // whole-network backward pass (chain_ok): per hidden layer the activations transposed, per layer dZ^T and one row of bias
-  // partial sums per 128-row tile; all transposes have the row stride Mp128
-  char *yT[KS_MAX_LAYERS], *dzT[KS_MAX_LAYERS];
+  // whole-network backward pass (chain_ok): the network input as the kernels multiply it, (M, its width in whole 128), per layer dZ in whole
+  // 128-row tiles and one row of bias partial sums per tile
+  char *in, *dz[KS_MAX_LAYERS];
   float *bpart[KS_MAX_LAYERS], *wpart[KS_MAX_LAYERS];  // wpart: the row slices of each layer's weight-gradient product
   int64_t Mp128;
 };
@@ -2453,7 +2533,7 @@ static bool chain_ok(const DevMlp& m, int64_t M) {
   if (!m.fused || m.dtype != KS_MLP_BF16 || m.activation == KS_ACT_GELU || m.n_layers < 2 || M < 128 * 256) return false;
   for (int l = 0; l + 1 < m.n_layers; ++l)
     if (m.npad[l] != m.fn[l] * 32 || m.fn[l] * 4 <= kFusedWaves || !m.WtP[l + 1]) return false;
-  // the transposed copies of the input and of the output gradient are cut from the LDS tile at their padded widths
+  // the kept input and the output gradient are cut from the LDS tile at their padded widths
   if (round_up(m.kpad[0], kBN) + 8 > m.lda || m.npad[m.n_layers - 1] + 8 > m.lda) return false;
   return true;
 }
@@ -2469,7 +2549,8 @@ static int64_t carve_train(const DevMlp& m, int64_t M, char* base, TrainWs* ws) 
   };
   TrainWs w;
   std::memset(&w, 0, sizeof(w));
-  for (int l = 0; l + 1 < m.n_layers; ++l) w.act[l] = take(M * m.npad[l] * esz);
+  const int64_t rows = chain_ok(m, M) ? (M + 127) / 128 * 128 : M;  // the whole-network backward pass reads whole tiles
+  for (int l = 0; l + 1 < m.n_layers; ++l) w.act[l] = take(rows * m.npad[l] * esz);
   if (m.activation == KS_ACT_GELU)
     for (int l = 0; l + 1 < m.n_layers; ++l) w.pre[l] = take(M * m.npad[l] * esz);
   w.d0 = take(M * wz * esz);
@@ -2487,26 +2568,15 @@ static int64_t carve_train(const DevMlp& m, int64_t M, char* base, TrainWs* ws) 
   w.Mp128 = (M + 127) / 128 * 128;
   if (chain_ok(m, M)) {
     const int64_t tiles = w.Mp128 / 128;
-    for (int l = 0; l + 1 < m.n_layers; ++l) {
-      w.yT[l] = take((int64_t)m.npad[l] * w.Mp128 * esz);
+    for (int l = 0; l < m.n_layers; ++l) {
+      w.dz[l] = take((int64_t)m.npad[l] * w.Mp128 * esz);
       w.bpart[l] = (float*)take(tiles * m.npad[l] * 4);
+      w.wpart[l] = (float*)take((int64_t)chain_dw_slices(m.npad[l], round_up(m.kpad[l], kBN), w.Mp128) * m.npad[l] * m.kpad[l] * 4);
     }
-    for (int l = 0; l < m.n_layers; ++l) w.dzT[l] = take((int64_t)m.npad[l] * w.Mp128 * esz);
-    w.bpart[m.n_layers - 1] = (float*)take(tiles * m.npad[m.n_layers - 1] * 4);
-    for (int l = 0; l < m.n_layers; ++l) w.wpart[l] = (float*)take((int64_t)chain_dw_slices(m.npad[l], round_up(m.kpad[l], kBN), w.Mp128) * m.npad[l] * m.kpad[l] * 4);
-    w.yT[m.n_layers - 1] = take((int64_t)round_up(m.kpad[0], kBN) * w.Mp128 * esz);  // the network input, transposed
+    w.in = take((int64_t)round_up(m.kpad[0], kBN) * w.Mp128 * esz);
   }
   if (ws) *ws = w;
   return off;
-}
-
-static void keep_args(FusedArgs& a, const DevMlp& m, const TrainWs* ws) {
-  for (int l = 0; l + 1 < m.n_layers; ++l) {
-    a.keep_t[l] = (__bf16*)ws->yT[l];
-  }
-  a.keep_t_in = (__bf16*)ws->yT[m.n_layers - 1];
-  a.in_t_width = round_up(m.kpad[0], kBN);
-  a.ldt = ws->Mp128;
 }
 
 extern "C" int64_t ks_mlp_train_workspace_bytes(const KsMlp* h, int64_t M) {
@@ -2522,9 +2592,9 @@ static int train_forward(DevMlp& m, hipStream_t s, int64_t M, const float* x, fl
   if (sizeof(T) == 2)  // bf16 networks of other widths take the per-layer kernel
     for (int l = 0; whole && l + 1 < m.n_layers; ++l) whole = m.npad[l] == m.fn[l] * 32;
   m.chain_saved = 0;
-  if (whole && chain_ok(m, M)) {  // activations in the formats of the whole-network backward pass, not row-major
+  if (whole && chain_ok(m, M)) {
     m.chain_saved = 1;
-    return launch_fused_tile<__bf16, 128>(m, s, M, x, y, nullptr, &ws);
+    return launch_fused_tile<__bf16, 128>(m, s, M, x, y, ws.act, ws.in);
   }
   if (whole) return launch_fused(m, s, M, x, y, ws.act);
   const void* in = x;
@@ -2563,23 +2633,31 @@ extern "C" int ks_mlp_train_forward(KsMlp* h, ks_stream_t stream, int64_t M, con
   return rc != KS_OK ? rc : check_launch("ks_mlp_train_forward");
 }
 
-// The backward pass of a network whose forward kept the whole-network formats (chain_ok): the last layer's gradient by the small
-// kernels, every hidden layer's in one launch of mlp_fused_bwd_kernel, then one weight-gradient product per layer.
-template <typename T>
-static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float* x, const float* dy, const TrainWs& ws) {
+static int chain_wgrad(hipStream_t s, int slices, int64_t Mp, int np, int ldb, int kp, const __bf16* dz, const __bf16* y, float* part) {
+  const int64_t kslice = ((Mp + slices - 1) / slices + 4 * kCwRows - 1) / (4 * kCwRows) * (4 * kCwRows);  // slices past the last row add zeros
+  if (hipFuncSetAttribute((const void*)chain_wgrad_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kCwLds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", kCwLds);
+  hipLaunchKernelGGL(chain_wgrad_kernel, dim3((unsigned)((np / 128) * (ldb / 128)), (unsigned)slices), dim3(512), kCwLds, s, Mp, np, ldb, kp, (int)kslice,
+                     dz, y, part);
+  return KS_OK;
+}
+
+// The backward pass of a network whose forward kept what it reads (chain_ok): every layer's gradient in one launch of mlp_fused_bwd_kernel,
+// then one weight-gradient product per layer.
+static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float* dy, const TrainWs& ws) {
   const int L = m.n_layers;
   const int64_t Mp = ws.Mp128, tiles = Mp / 128;
   const int npl = m.npad[L - 1];
   {
     FusedBwdArgs a;
     std::memset(&a, 0, sizeof(a));
-    a.M = M; a.n_layers = L; a.lda = m.lda; a.ldt = Mp;
+    a.M = M; a.n_layers = L; a.lda = m.lda;
     a.dy = dy; a.out_dim = m.dims[L]; a.np_last = npl;
     for (int l = 0; l < L; ++l) {
       a.fk[l] = m.fk[l]; a.fn[l] = m.fn[l];
       a.WtP[l] = (const u32x4*)m.WtP[l];
-      if (l + 1 < L) a.yT[l] = (const __bf16*)ws.yT[l];
-      a.dzT[l] = (__bf16*)ws.dzT[l];
+      if (l + 1 < L) a.y[l] = (const __bf16*)ws.act[l];
+      a.dz[l] = (__bf16*)ws.dz[l];
       a.bias_part[l] = ws.bpart[l];
     }
     const int lds = 128 * m.lda * 2;
@@ -2599,21 +2677,16 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
     }
 #undef KS_LAUNCH
   }
-  (void)x;  // the training forward left its transpose behind
-  const T* xT = (const T*)ws.yT[L - 1];
   GradFinishArgs g;
   std::memset(&g, 0, sizeof(g));
   g.n_layers = L; g.tiles = (int)tiles;
   int wblocks = 0, bblocks = 0;
   for (int l = L - 1; l >= 0; --l) {
     const int np = m.npad[l], kp = m.kpad[l], kp128 = round_up(kp, kBN);
-    const T* dzT = (const T*)ws.dzT[l];
-    const T* yT = l > 0 ? (const T*)ws.yT[l - 1] : xT;
-    const int ksplit = chain_dw_slices(np, kp128, Mp);
-    const int rc = launch_layer_tile<T, false, true, 128, 128, 2, 2, 2>(KS_ACT_NONE, s, np, kp128, (int)Mp, (int)Mp, kp, dzT, Mp, yT, m.zero_bias,
-                                                                        (void*)ws.wpart[l], kp, ksplit);
+    const int slices = chain_dw_slices(np, kp128, Mp);
+    const int rc = chain_wgrad(s, slices, Mp, np, kp128, kp, (const __bf16*)ws.dz[l], l > 0 ? (const __bf16*)ws.act[l - 1] : (const __bf16*)ws.in, ws.wpart[l]);
     if (rc != KS_OK) return rc;
-    g.nz[l] = ksplit; g.nW[l] = (int64_t)np * kp; g.nb[l] = np;
+    g.nz[l] = slices; g.nW[l] = (int64_t)np * kp; g.nb[l] = np;
     g.wpart[l] = ws.wpart[l]; g.bpart[l] = ws.bpart[l]; g.gW[l] = m.gW[l]; g.gb[l] = m.gb[l];
   }
   for (int l = 0; l < L; ++l) {
@@ -2675,14 +2748,7 @@ static int train_backward(DevMlp& m, hipStream_t s, int64_t M, const float* x, c
   const int L = m.n_layers;
   const int64_t Mp = ws.Mp;
   if (L == 1) return train_backward_single<T>(m, s, M, x, m.dims[0], dy, ws, dx, want_w, accumulate_dx, zero_rows);
-  if constexpr (sizeof(T) == 2) if (m.chain_saved) {
-    if (want_w && !dx) return train_backward_chain<T>(m, s, M, x, dy, ws);
-    // the layer-by-layer pass below reads row-major activations: rebuild them from the transposed copies
-    for (int l = 0; l + 1 < L; ++l)
-      hipLaunchKernelGGL((transpose_kernel<T, T>), dim3((unsigned)((m.npad[l] + 31) / 32), (unsigned)((M + 31) / 32)), dim3(256), 0, s,
-                         (int64_t)m.npad[l], (int)M, ws.Mp128, (const T*)ws.yT[l], (int)M, (int64_t)m.npad[l], (T*)ws.act[l]);
-    m.chain_saved = 0;
-  }
+  if constexpr (sizeof(T) == 2) if (m.chain_saved && want_w && !dx) return train_backward_chain(m, s, M, dy, ws);
   T* dz = (T*)ws.d0;
   T* dnext = (T*)ws.d1;
   {  // the output gradient in working precision, padded to the last layer's width

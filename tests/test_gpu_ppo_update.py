@@ -900,3 +900,34 @@ def test_rows_and_their_mirror_images_in_one_pass(groups, group, n):
     _lib.check(lib.ks_mirror_pairs(st, groups, group, n, _lib.addr(x), _lib.addr(p), _lib.addr(s), _lib.addr(out)))
     _lib.check(lib.ks_signed_permute(st, groups * group, n, _lib.addr(x), _lib.addr(p), _lib.addr(s), _lib.addr(alone)))
     assert torch.equal(out, torch.cat([x, image], dim=1)) and torch.equal(alone, image)
+
+
+@pytest.mark.parametrize("dims,M", [((68, 512, 512, 20), 32768), ((40, 384, 512, 12), 32769), ((33, 512, 384, 256, 128, 1), 40000),
+                                    ((7, 128, 128, 130), 65536 + 127)])
+def test_weight_gradients_of_whole_networks_are_exact_on_integers(dims, M):
+    """Every tile shape of the weight-gradient product, slices that the rows do not fill, padding rows and columns.  Weights that pass each
+    input to one output, small integers: every product and sum is a whole number below 2^24, and the gradients are exact."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    ws = []
+    for l, (i, o) in enumerate(zip(dims[:-1], dims[1:])):
+        w = np.zeros((o, i), np.float32)
+        if l == 0:
+            w[np.arange(o), np.arange(o) % i] = rng.choice([-1.0, 1.0], size=o)
+        else:
+            w[np.arange(i) % o, rng.permutation(i)] = rng.choice([-1.0, 1.0], size=i)
+        ws.append(w)
+    net = MLP(ws, [np.zeros(o, np.float32) for o in dims[1:]], activation="none", dtype="bf16")
+    net.train_init()
+    x, dy = t32(rng.integers(-1, 2, size=(M, dims[0]))), t32(rng.integers(-1, 2, size=(M, dims[-1])))
+    acts, grads = [x.double()], [dy.double()]
+    for w in ws:
+        acts.append(acts[-1] @ t32(w).double().t().contiguous())
+    for w in ws[:0:-1]:
+        grads.append(grads[-1] @ t32(w).double())
+    assert max(float(a.abs().max()) for a in acts[:-1]) <= 256
+    net.train_forward(x)
+    net.backward(x, dy)
+    for (gw, gb), a, d in zip(net.parameters(gradients=True), acts, grads[::-1]):
+        assert torch.equal(gw.double(), d.t().contiguous() @ a) and torch.equal(gb.double(), d.sum(0))
