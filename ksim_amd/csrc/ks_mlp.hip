@@ -812,7 +812,7 @@ __host__ __device__ inline int fused_share(int nt, int lda) {
 }
 
 // One layer of the whole-network kernel for one wavefront: MFMA work, barrier, epilogue, barrier.
-template <int ACT, typename T, int MI, bool LAST, bool SWAP = false>
+template <int ACT, typename T, int MI, bool LAST, bool SAVE, bool SWAP = false>
 __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __restrict__ act, int64_t m0, int lane,
                                             int wave, int64_t tile) {
   const int nk = a.fk[l], nt = a.fn[l], lda = a.lda;
@@ -911,10 +911,22 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
   KS_MLP_STAMP2(4 + 3 * l)
   // The next layer only reads the tile until every wavefront (this copy included, which sits before its matrix work in program order) has passed
   // the next barrier.  Rows are as wide as the backward pass's layers, which is more than the tile's (zeros) where the width is no multiple of 128.
-  if (!LAST && a.save[l]) tile_rows_out<T, MI * 32>(act, lda, reinterpret_cast<T*>(a.save[l]), a.save_ld[l], nt * 32, m0, a.save_rows);
+  if constexpr (sizeof(T) == 2) {
+    if (SAVE && !LAST) tile_rows_out<T, MI * 32>(act, lda, reinterpret_cast<T*>(a.save[l]), a.save_ld[l], nt * 32, m0, a.save_rows);
+  } else if (!LAST && a.save[l]) {  // one form for both in fp32, whose code without this is 4 % slower (8192 rows of 71-256-256-256-21: 31.5 -> 32.9 us)
+    T* dst = reinterpret_cast<T*>(a.save[l]);
+    const int ld = a.save_ld[l], w4 = ld / 4, held = nt * 8;
+    for (int idx = threadIdx.x; idx < MI * 32 * w4; idx += 64 * kFusedWaves) {
+      const int r = idx / w4, c4 = idx - r * w4;
+      if (m0 + r < a.M)
+        *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c4 * 4) =
+            c4 < held ? *reinterpret_cast<const uint4*>(act + r * lda + c4 * 4) : uint4{0u, 0u, 0u, 0u};
+    }
+  }
 }
 
-template <int ACT, typename T, int BM, bool SINGLE = false>
+// SAVE: the training forward of bf16 networks (FusedArgs::save, save_in)
+template <int ACT, typename T, int BM, bool SINGLE = false, bool SAVE = false>
 __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile) {
   constexpr int MI = BM / 32;
   constexpr int NTHR = 64 * kFusedWaves;
@@ -927,7 +939,7 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   KS_MLP_STAMP(0)
   {  // network input -> tile; zero beyond the batch and in the K padding of the first layer
     const int in_dim = a.in_dim;
-    const int K0 = a.in_width > a.fk[0] * SK ? a.in_width : a.fk[0] * SK;  // the copy that is kept is padded further
+    const int K0 = SAVE && a.in_width > a.fk[0] * SK ? a.in_width : a.fk[0] * SK;  // the copy that is kept is padded further
     const int64_t rows_left = a.M - m0;
     const int rows = rows_left < BM ? (int)rows_left : BM;
     const float* src = a.x + m0 * in_dim;
@@ -982,17 +994,17 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   }
   __syncthreads();
   KS_MLP_STAMP(1)
-  if (a.save_in) tile_rows_out<T, BM>(act, lda, reinterpret_cast<T*>(a.save_in), a.in_width, a.in_width, m0, a.save_rows);  // the tile stays until the first layer's barrier
+  if (SAVE && a.save_in) tile_rows_out<T, BM>(act, lda, reinterpret_cast<T*>(a.save_in), a.in_width, a.in_width, m0, a.save_rows);  // the tile stays until the first layer's barrier
   if constexpr (!SINGLE)
-    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false>(a, l, act, m0, lane, wave, tile);
-  fused_layer<ACT, T, MI, true, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
+    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false, SAVE>(a, l, act, m0, lane, wave, tile);
+  fused_layer<ACT, T, MI, true, SAVE, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
 }
 
 // SINGLE: one bf16 layer
-template <int ACT, typename T, int BM, bool SINGLE = false>
+template <int ACT, typename T, int BM, bool SINGLE = false, bool SAVE = false>
 __global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
 void mlp_fused_kernel(const FusedArgs a) {
-  mlp_fused_body<ACT, T, BM, SINGLE>(a, blockIdx.x);
+  mlp_fused_body<ACT, T, BM, SINGLE, SAVE>(a, blockIdx.x);
 }
 
 // Two networks over the same rows in one launch (actor and critic of a control step): blockIdx.y picks the network, so
@@ -2118,7 +2130,7 @@ static int launch_fused_tile(const DevMlp& m, hipStream_t s, int64_t M, const fl
   if (blocks > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp_forward: too many rows");
 #define KS_LAUNCH(A)                                                                                           \
   {                                                                                                            \
-    auto kfn = mlp_fused_kernel<A, T, BM>;                                                                     \
+    auto kfn = sizeof(T) == 2 && save ? mlp_fused_kernel<A, T, BM, false, sizeof(T) == 2> : mlp_fused_kernel<A, T, BM>; \
     if constexpr (sizeof(T) == 2 && BM != 64)                                                                  \
       if (m.n_layers == 1) kfn = mlp_fused_kernel<KS_ACT_NONE, T, BM, true>;                                   \
     if (lds > 64 * 1024 &&                                                                                     \
