@@ -6,7 +6,6 @@ use plain MLP stacks.  Weights are given as (out, in) fp32 arrays, like the refe
 from __future__ import annotations
 
 import ctypes
-import threading
 from typing import Sequence
 
 import numpy as np
@@ -48,7 +47,6 @@ class MLP:
         self._lib = lib
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_mlp_create(ctypes.byref(d), ctypes.byref(self._handle)))
-        self._ws: dict | None = None
 
     @property
     def in_dim(self) -> int:
@@ -61,18 +59,12 @@ class MLP:
     def flops_per_row(self) -> int:
         return 2 * sum(a * b for a, b in zip(self.dims[:-1], self.dims[1:]))
 
-    def workspace(self, M: int, device) -> torch.Tensor:
-        """Scratch of the paths that take several launches, one buffer per stream and thread: calls on different streams may overlap
-        on the GPU, and the launches of two threads may alternate on one stream."""
+    def workspace(self, M: int, device) -> torch.Tensor | None:
+        """Scratch of one call on `M` rows, None where the call needs none.  It belongs to the call: taken from torch's allocator on the
+        current stream and given back there when the launches are queued.  Calls on other streams, in other threads and in other captured
+        graphs never share it, and a replayed graph finds it in the graph's own memory."""
         need = int(self._lib.ks_mlp_workspace_bytes(self._handle, M))
-        key = (_lib.current_stream(), threading.get_ident()) if need else 0
-        if self._ws is None:
-            self._ws = {}
-        ws = self._ws.get(key)
-        if ws is None or ws.numel() < need or ws.device != torch.device(device):
-            ws = torch.empty(need, dtype=torch.uint8, device=device)
-            self._ws[key] = ws
-        return ws
+        return torch.empty(need, dtype=torch.uint8, device=device) if need else None
 
     def __call__(self, x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         _lib.require_cuda(x, dtype=torch.float32)
@@ -99,10 +91,10 @@ class MLP:
             _lib.require_cuda(o, dtype=torch.float32)
             if tuple(a.shape) != (M, net.in_dim) or tuple(o.shape) != (M, net.out_dim):
                 raise _lib.KsError(f"expected input (M, {net.in_dim}) and output (M, {net.out_dim})")
+        ws, ws_other = self.workspace(M, x.device), other.workspace(M, x.device)  # both held until both are launched
         _lib.check(self._lib.ks_mlp_forward_pair(self._handle, other._handle, _lib.current_stream(), M, _lib.addr(x),
-                                                 _lib.addr(out), _lib.addr(x_other), _lib.addr(out_other),
-                                                 _lib.addr(self.workspace(M, x.device)),
-                                                 _lib.addr(other.workspace(M, x.device))))
+                                                 _lib.addr(out), _lib.addr(x_other), _lib.addr(out_other), _lib.addr(ws),
+                                                 _lib.addr(ws_other)))
 
     # ------------------------------------------------------------------ training (ksim/task/ppo.py:495-565)
     def train_init(self) -> None:
@@ -189,7 +181,6 @@ class MLP:
         """A view of a network that another object owns (the projections inside a GRU cell): never destroyed here."""
         self = cls.__new__(cls)
         self._lib, self._handle, self.dims, self.dtype, self.activation = lib, handle, list(dims), dtype, "none"
-        self._ws = None
         self._borrowed = True
         return self
 

@@ -404,3 +404,37 @@ def test_parameters_of_several_networks_in_one_launch():
     assert mlp.copy_parameters([]) == []
     with pytest.raises(_lib.KsError):  # a network without a training state, behind one that has it
         mlp.copy_parameters([nets[0], MLP([np.ones((2, 3), np.float32)], [np.ones(2, np.float32)], activation="elu", dtype="f32")])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_one_network_called_by_two_threads(dtype):
+    """Two threads on one stream, whose launches may alternate, and two on streams of their own: every call's rows are its own."""
+    import threading
+
+    from ksim_amd.mlp import random_mlp
+
+    net, _, _ = random_mlp((68, 512, 512, 512, 20), seed=5, dtype=dtype)
+    xs = [[torch.from_numpy(np.random.default_rng(10 * k + i).normal(size=(1 + 13 * i, 68)).astype(np.float32)).to(DEV) for i in range(5)] for k in range(2)]
+    want = [[net(x) for x in rows] for rows in xs]
+    shared = torch.cuda.Stream()
+    for streams in ([shared, shared], [torch.cuda.Stream(), torch.cuda.Stream()]):
+        got, errors = [None, None], []
+        torch.cuda.synchronize()
+
+        def work(k):
+            try:
+                with torch.cuda.stream(streams[k]):
+                    got[k] = [[net(x) for x in xs[k]] for _ in range(20)]
+            except Exception as e:  # shown by the assertion below
+                errors.append(e)
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+        torch.cuda.synchronize()
+        assert not errors and not any(t.is_alive() for t in threads)
+        for k in range(2):
+            for rep in got[k]:
+                assert all(torch.equal(a, b) for a, b in zip(rep, want[k]))

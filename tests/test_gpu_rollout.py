@@ -735,6 +735,41 @@ def test_split_rollout_replayed_from_per_group_graphs_equals_its_eager_run():
             assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_graphs_of_groups_that_share_wide_networks_replay_side_by_side(dtype):
+    """3 x 512 networks over few rows go through several launches with scratch between them: each group's graph has its own, whatever else
+    the networks are called with between the replays."""
+    import dataclasses
+
+    from ksim_amd.mlp import random_mlp
+    from ksim_amd.rollout import SplitRollout
+
+    N, T, G = 96, 6, 3
+    outs = []
+    for graph in (False, True):
+        m, c, rnd_, _, _, EnvState = build(N, T, seed=8, min_height=0.9)
+        actor, critic = (random_mlp((c.terms.obs_dim, 512, 512, 512, o), seed=o, dtype=dtype)[0] for o in (m.nu, 1))
+        c = dataclasses.replace(c, actor=actor, critic=critic)
+        n = N // G
+        envs = []
+        for g in range(G):
+            rows = {k: v[g * n:(g + 1) * n].contiguous() for k, v in rnd_.items()}
+            envs.append(EnvState(c.engine.reset(c.physics_model, 1.0, 3 + g, n, rows), rows, torch.zeros(n, 2, device=DEV), None, seed=11 + g))
+        sro = SplitRollout(c, N, T, splits=G)
+        run = []
+        for k in range(5):
+            res = sro.unroll(envs, graph=graph)
+            run.append([x.clone() for ro, (traj, rew) in zip(sro.parts, res) for x in (traj.obs["noisy_obs"], traj.action, ro.values, rew.total)])
+            for rows in (n, 256, 4000):  # the same networks elsewhere, and the memory that those calls gave back written over
+                actor(torch.ones(rows, c.terms.obs_dim, device=DEV))
+            torch.full((1 << 22,), 255, dtype=torch.uint8, device=DEV)
+        torch.cuda.synchronize()
+        outs.append(run)
+    for a, b in zip(*outs):
+        for x, y in zip(a, b):
+            assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
 def test_motion_resets_symmetry_rewards_and_imu_misalignment_in_the_rollout():
     """The pieces an AMP / sim-to-real task adds, together in one rollout on a model read from MJCF: episodes that start from
     a frame of a reference motion with a random pitch / roll and heading, a misaligned IMU site per env read by the gyro,

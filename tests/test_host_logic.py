@@ -556,3 +556,22 @@ def test_every_public_oracle_function_is_named_in_a_cpu_test():
                 if f"{mod}.{node.name}" not in plumbing and not re.search(r"\b" + re.escape(node.name) + r"\b", text):
                     missing.append(f"{mod}.{node.name}")
     assert not missing, f"oracle functions that no CPU test names: {missing}"
+
+
+def test_a_networks_scratch_belongs_to_the_call(monkeypatch):
+    """Two graphs captured on torch's one capture stream, or two threads on one stream, must not be handed the same scratch: activations and
+    arrival counters of one call would be overwritten by the other's launches.  Both allocations are alive here, so they differ unless the
+    network keeps one for its next caller."""
+    from ksim_amd.mlp import MLP
+
+    class Lib:
+        @staticmethod
+        def ks_mlp_workspace_bytes(handle, rows):
+            return 64 * rows
+
+    monkeypatch.setattr(_lib, "current_stream", lambda: 7)
+    net = MLP._borrow(Lib, ctypes.c_void_p(), (4, 4), "bf16")
+    a, b = net.workspace(8, "cpu"), net.workspace(8, "cpu")
+    assert a.numel() >= 512 and b.numel() >= 512 and a.data_ptr() != b.data_ptr()
+    assert not any(t is a or t is b for t in vars(net).values())
+    assert net.workspace(0, "cpu") is None
