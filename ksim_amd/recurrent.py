@@ -91,14 +91,11 @@ class GRUCell:
         self._lib = lib
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_gru_create(ctypes.byref(d), ctypes.byref(self._handle)))
-        self._ws: torch.Tensor | None = None
         self._proj: MLP | None = None
 
     def workspace(self, M: int, device) -> torch.Tensor:
-        need = int(self._lib.ks_gru_workspace_bytes(self._handle, M))
-        if self._ws is None or self._ws.numel() < need or self._ws.device != torch.device(device):
-            self._ws = torch.empty(need, dtype=torch.uint8, device=device)
-        return self._ws
+        """Scratch of one call, as `MLP.workspace`."""
+        return torch.empty(int(self._lib.ks_gru_workspace_bytes(self._handle, M)), dtype=torch.uint8, device=device)
 
     def __call__(self, x: torch.Tensor, h: torch.Tensor, fresh: torch.Tensor | None = None,
                  out: torch.Tensor | None = None) -> torch.Tensor:
@@ -140,8 +137,9 @@ class GRUCell:
         M, H = x.shape[0], self.hidden_size
         if tuple(x.shape) != (M, self.input_size) or tuple(h.shape) != (M, H) or tuple(out.shape) != (M, H) or tuple(saved.shape) != (M, 5 * H):
             raise _lib.KsError("expected x (M, input), h and out (M, H), saved (M, 5H)")
+        ws = self.workspace(M, x.device)
         _lib.check(self._lib.ks_gru_train_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h), _lib.addr(fresh),
-                                                  _lib.addr(out), _lib.addr(saved), _lib.addr(self.workspace(M, x.device))))
+                                                  _lib.addr(out), _lib.addr(saved), _lib.addr(ws)))
         return out
 
     @property
@@ -243,14 +241,11 @@ class LSTMCell:
         self._lib = lib
         self._handle = ctypes.c_void_p()
         _lib.check(lib.ks_lstm_create(ctypes.byref(d), ctypes.byref(self._handle)))
-        self._ws: torch.Tensor | None = None
         self._proj: MLP | None = None
 
     def workspace(self, M: int, device) -> torch.Tensor:
-        need = int(self._lib.ks_lstm_workspace_bytes(self._handle, M))
-        if self._ws is None or self._ws.numel() < need or self._ws.device != torch.device(device):
-            self._ws = torch.empty(need, dtype=torch.uint8, device=device)
-        return self._ws
+        """Scratch of one call, as `MLP.workspace`."""
+        return torch.empty(int(self._lib.ks_lstm_workspace_bytes(self._handle, M)), dtype=torch.uint8, device=device)
 
     def __call__(self, x: torch.Tensor, h: torch.Tensor, c: torch.Tensor, fresh: torch.Tensor | None = None,
                  out: tuple | None = None) -> tuple[torch.Tensor, torch.Tensor]:
@@ -290,9 +285,9 @@ class LSTMCell:
         M, H = x.shape[0], self.hidden_size
         if tuple(x.shape) != (M, self.input_size) or any(tuple(t.shape) != (M, H) for t in (h, c, h_out, c_out)) or tuple(saved.shape) != (M, 7 * H):
             raise _lib.KsError("expected x (M, input), h, c and outputs (M, H), saved (M, 7H)")
+        ws = self.workspace(M, x.device)
         _lib.check(self._lib.ks_lstm_train_forward(self._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(h), _lib.addr(c),
-                                                   _lib.addr(fresh), _lib.addr(h_out), _lib.addr(c_out), _lib.addr(saved),
-                                                   _lib.addr(self.workspace(M, x.device))))
+                                                   _lib.addr(fresh), _lib.addr(h_out), _lib.addr(c_out), _lib.addr(saved), _lib.addr(ws)))
 
     @property
     def sequence_supported(self) -> bool:
@@ -389,7 +384,6 @@ class RecurrentNetwork:
         self.lstm = bool(self.cells) and isinstance(self.cells[0], LSTMCell)
         self.hidden_size, self.depth = H, len(self.cells)
         self.in_dim, self.out_dim = self.input_proj.in_dim, output_proj.out_dim
-        self._x: torch.Tensor | None = None
 
     def initial_carry(self, num_envs: int, device="cuda") -> torch.Tensor:
         shape = (self.depth, 2, num_envs, self.hidden_size) if self.lstm else (self.depth, num_envs, self.hidden_size)
@@ -402,9 +396,7 @@ class RecurrentNetwork:
         want = (self.depth, 2, N, self.hidden_size) if self.lstm else (self.depth, N, self.hidden_size)
         if tuple(carry.shape) != want:
             raise _lib.KsError(f"carry must be {want}")
-        if self._x is None or self._x.shape[0] != N or self._x.device != obs.device:
-            self._x = torch.empty(N, self.hidden_size, dtype=torch.float32, device=obs.device)
-        x = self.input_proj(obs, out=self._x)
+        x = self.input_proj(obs)
         for i, cell in enumerate(self.cells):  # the layer's new hidden state is also the next layer's input
             if self.lstm:
                 x, _ = cell(x, carry[i, 0], carry[i, 1], fresh, out=(carry[i, 0], carry[i, 1]))

@@ -402,7 +402,7 @@ class SplitRollout:
         if splits < 1 or num_envs % splits:
             raise _lib.KsError("the env count must be a multiple of the number of groups")
         if any(isinstance(n, RecurrentNetwork) for n in (constants.actor, constants.critic)):
-            raise _lib.KsError("recurrent networks keep one workspace per cell: roll them out on a single stream")
+            raise _lib.KsError("recurrent networks are rolled out on a single stream")
         self.c, self.N, self.T, self.splits = constants, int(num_envs), int(rollout_length), int(splits)
         self.parts = [Rollout(constants, num_envs // splits, rollout_length) for _ in range(splits)]
         self.streams = _group_streams(splits)

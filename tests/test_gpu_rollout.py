@@ -770,6 +770,29 @@ def test_graphs_of_groups_that_share_wide_networks_replay_side_by_side(dtype):
             assert torch.isfinite(x).all() and torch.equal(x, y)
 
 
+def test_recurrent_rollout_replayed_after_the_networks_saw_other_batches():
+    """A captured rollout of recurrent networks, its scratch first used eagerly, then replayed after the same networks ran larger and smaller
+    batches and the memory those gave back was written over."""
+    N, T = 24, 6
+    runs = []
+    for graph in (False, True):
+        m, c, rnd_, _, ro, EnvState = build(N, T, seed=17, min_height=0.95, recurrent=True, head="gaussian-wide")
+        env = EnvState(c.engine.reset(c.physics_model, 1.0, 3, N, rnd_), rnd_, torch.zeros(N, 2, device=DEV), None, seed=21)
+        run = []
+        for it in range(4):
+            traj, rew = ro.unroll(env, graph=graph and it > 0)
+            run.append([x.clone() for x in (traj.action, ro.values, env.actor_carry, env.critic_carry, rew.total)])
+            for rows in (7, 3000):
+                for net in (c.actor, c.critic):
+                    net(torch.ones(rows, c.terms.obs_dim, device=DEV), net.initial_carry(rows))
+            for size in (1 << 10, 1 << 14, 1 << 18, 1 << 22):
+                torch.full((size,), 255, dtype=torch.uint8, device=DEV)
+        torch.cuda.synchronize()
+        runs.append(run)
+    for a, b in zip(*runs):
+        assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(a, b))
+
+
 def test_motion_resets_symmetry_rewards_and_imu_misalignment_in_the_rollout():
     """The pieces an AMP / sim-to-real task adds, together in one rollout on a model read from MJCF: episodes that start from
     a frame of a reference motion with a random pitch / roll and heading, a misaligned IMU site per env read by the gyro,

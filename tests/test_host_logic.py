@@ -575,3 +575,19 @@ def test_a_networks_scratch_belongs_to_the_call(monkeypatch):
     assert a.numel() >= 512 and b.numel() >= 512 and a.data_ptr() != b.data_ptr()
     assert not any(t is a or t is b for t in vars(net).values())
     assert net.workspace(0, "cpu") is None
+
+
+@pytest.mark.parametrize("cell", ["GRUCell", "LSTMCell"])
+def test_a_recurrent_cells_scratch_belongs_to_the_call(cell):
+    """As the plain networks': a rollout captured as a graph goes on using the addresses it was captured with, whatever larger batch the cell
+    sees afterwards (a policy update's)."""
+    from ksim_amd import recurrent
+
+    class Lib:
+        ks_gru_workspace_bytes = ks_lstm_workspace_bytes = staticmethod(lambda handle, rows: 64 * rows)
+
+    c = object.__new__(getattr(recurrent, cell))
+    c._lib, c._handle = Lib, None
+    c._ws = None
+    a, b = c.workspace(8, "cpu"), c.workspace(8, "cpu")
+    assert a.numel() >= 512 and b.numel() >= 512 and a.data_ptr() != b.data_ptr()
