@@ -210,6 +210,12 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     return metrics
 
 
+def _gather_extent(t: torch.Tensor, d: int) -> tuple[int, int]:
+    """(blocks of columns, bytes of a column) of a contiguous array whose columns lie along axis `d`.  From the sizes alone: the stride of an axis
+    of size one says nothing, and torch leaves it as it was before a transpose or a permutation."""
+    return math.prod(t.shape[:d]), math.prod(t.shape[d + 1:]) * t.element_size()
+
+
 def _columns(idx: torch.Tensor, own: bool, arrays: Sequence[tuple[torch.Tensor | None, int]]) -> list:
     """The env columns `idx` of every (array, env axis), contiguous, in one launch.  Only for indices that were drawn here (`own`): a caller's are
     checked where torch checks them, as are arrays that are not plain contiguous device memory."""
@@ -225,8 +231,7 @@ def _columns(idx: torch.Tensor, own: bool, arrays: Sequence[tuple[torch.Tensor |
         shape = list(t.shape)
         shape[d] = picked
         out[k] = torch.empty(shape, dtype=t.dtype, device=t.device)
-        inner = t.stride(d) * t.element_size()
-        table.append(T.KsGatherArray(t.data_ptr(), out[k].data_ptr(), math.prod(shape[:d]), inner))
+        table.append(T.KsGatherArray(t.data_ptr(), out[k].data_ptr(), *_gather_extent(t, d)))
     if table:
         rc = _lib.load().ks_gather_columns(_lib.current_stream(), len(table), (T.KsGatherArray * len(table))(*table), N, picked, keep.data_ptr())
         _lib.check(rc)

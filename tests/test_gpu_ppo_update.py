@@ -836,6 +836,22 @@ def test_minibatch_columns_equal_index_select(T_, N, picked):
             assert torch.equal(got.view(torch.uint8) if got.dtype != torch.bool else got, want.contiguous().view(torch.uint8) if got.dtype != torch.bool else want)
 
 
+@pytest.mark.parametrize("picked", [0, 1])
+def test_minibatch_columns_of_one_env_with_strides_of_another_layout(picked):
+    """Arrays of one env that came from a transpose, a permutation or a slice: contiguous, with strides that do not describe the env axis."""
+    from ksim_amd import ppo_update as pu
+
+    arrays = [(torch.randn(1, 24, device="cuda").t(), 1), (torch.randn(3, 2, 128, 1, device="cuda").permute(0, 1, 3, 2), 2),
+              (torch.randn(1, 24, 17, device="cuda").permute(1, 0, 2), 1), ((torch.randn(1, 24, device="cuda") > 0).t(), 1),
+              (torch.randn(5, 7, 3, device="cuda")[:, 2:3].transpose(0, 1).contiguous().transpose(0, 1), 1)]
+    idx = torch.zeros(picked, dtype=torch.int64, device="cuda")
+    for (t, d), got in zip(arrays, pu._columns(idx, True, arrays)):
+        assert t.shape[d] == 1 and t.is_contiguous()
+        blocks, inner = pu._gather_extent(t, d)
+        assert blocks * inner == t.numel() * t.element_size()
+        assert torch.equal(got, t.index_select(d, idx))
+
+
 @pytest.mark.parametrize("dims,M", [((475, 128), 2051), ((33, 130), 4097), ((3, 5), 60001), ((65, 36), 8193), ((64, 128), 3000)])
 def test_single_fp32_layers_over_rows_at_any_float(dims, M):
     """Rows that start 0 to 3 floats past a 16-byte boundary, the last one at the end of its allocation: the bits of the aligned rows, and the

@@ -591,3 +591,19 @@ def test_a_recurrent_cells_scratch_belongs_to_the_call(cell):
     c._ws = None
     a, b = c.workspace(8, "cpu"), c.workspace(8, "cpu")
     assert a.numel() >= 512 and b.numel() >= 512 and a.data_ptr() != b.data_ptr()
+
+
+@pytest.mark.parametrize("make,d", [(lambda t: t.zeros(1, 24).t(), 1), (lambda t: t.zeros(2, 2, 128, 1).permute(0, 1, 3, 2), 2),
+                                    (lambda t: t.zeros(1, 3, 5).permute(1, 0, 2), 1), (lambda t: t.zeros(7, 4, 1)[:1], 0),
+                                    (lambda t: t.zeros(1, 7, 3).expand(1, 7, 3).transpose(0, 1), 1), (lambda t: t.zeros(6, 5, 4), 1),
+                                    (lambda t: t.zeros(0, 5, 4), 1), (lambda t: t.zeros(6, 1, 0), 1)])
+def test_the_minibatch_gather_copies_what_the_array_holds(make, d):
+    """Contiguous arrays of one env keep strides from before a transpose or a permutation; blocks x envs x bytes is the array all the same."""
+    import torch
+
+    from ksim_amd.ppo_update import _gather_extent
+
+    t = make(torch)
+    assert t.is_contiguous()
+    blocks, inner = _gather_extent(t, d)
+    assert blocks * t.shape[d] * inner == t.numel() * t.element_size()
