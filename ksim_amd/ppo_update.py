@@ -216,16 +216,22 @@ def _gather_extent(t: torch.Tensor, d: int) -> tuple[int, int]:
     return math.prod(t.shape[:d]), math.prod(t.shape[d + 1:]) * t.element_size()
 
 
+def _gather_fits(t: torch.Tensor, d: int, picked: int) -> bool:
+    """Whether `picked` columns can be counted in the launch's 32 bits even if they have to be moved byte by byte."""
+    return math.prod(_gather_extent(t, d)) * picked <= 0xffffffff
+
+
 def _columns(idx: torch.Tensor, own: bool, arrays: Sequence[tuple[torch.Tensor | None, int]]) -> list:
     """The env columns `idx` of every (array, env axis), contiguous, in one launch.  Only for indices that were drawn here (`own`): a caller's are
-    checked where torch checks them, as are arrays that are not plain contiguous device memory."""
+    checked where torch checks them, as are arrays that are not plain contiguous memory of the indices' device, or too large for one launch."""
     N = next(t.shape[d] for t, d in arrays if t is not None)
     picked, out = idx.numel(), [None] * len(arrays)
     table, keep = [], idx.contiguous()
     for k, (t, d) in enumerate(arrays):
         if t is None:
             continue
-        if not own or t.shape[d] != N or not t.is_contiguous() or not t.is_cuda or t.requires_grad or len(table) == T.KS_GATHER_ARRAYS:
+        if (not own or t.shape[d] != N or not t.is_contiguous() or not t.is_cuda or t.device != idx.device or t.requires_grad
+                or len(table) == T.KS_GATHER_ARRAYS or not _gather_fits(t, d, picked)):
             out[k] = t.index_select(d, idx).contiguous()
             continue
         shape = list(t.shape)

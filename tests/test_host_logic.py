@@ -607,3 +607,27 @@ def test_the_minibatch_gather_copies_what_the_array_holds(make, d):
     assert t.is_contiguous()
     blocks, inner = _gather_extent(t, d)
     assert blocks * t.shape[d] * inner == t.numel() * t.element_size()
+
+
+def test_the_minibatch_gather_leaves_what_it_cannot_count_to_torch():
+    """Minibatches of 2^32 bytes and more are not refused: index_select takes them, as it takes arrays of another device than the indices'."""
+    import torch
+
+    from ksim_amd import ppo_update as pu
+
+    big = torch.empty(100, 90000, 475, device="meta")
+    assert not pu._gather_fits(big, 1, 45000) and pu._gather_fits(big, 1, 20000)
+    b = torch.empty(1, 2, 1 << 31, dtype=torch.uint8, device="meta")
+    assert pu._gather_fits(b, 1, 1) and not pu._gather_fits(b, 1, 2)
+
+    class Cuda:  # a contiguous array of another GPU, as far as the rule looks
+        shape, is_cuda, requires_grad, device = (2, 3), True, False, torch.device("cuda", 1)
+
+        def is_contiguous(self):
+            return True
+
+        def index_select(self, d, idx):
+            raise RuntimeError("expected all tensors on the same device")
+
+    with pytest.raises(RuntimeError, match="same device"):
+        pu._columns(torch.zeros(1, dtype=torch.int64), True, [(Cuda(), 1)])
