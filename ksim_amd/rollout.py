@@ -176,7 +176,8 @@ class Rollout:
                         fresh=self.reset_mask if (c.terms.carry_dim or c.terms.has_bias) else None,
                         site_pose=(env.randomization_dict or {}).get("site_pose"))
 
-        if self._obs_done != (id(env), t, step, _relative_step):  # else the launch that ended the previous step wrote it
+        ahead = self._obs_done
+        if ahead is None or ahead[0] is not env or ahead[1:] != (t, step, _relative_step):  # else the launch that ended the previous step wrote it
             c.terms.observe(src, self.N, bias_redraw=noise.get("obs_bias_redraw"), noise_normal=noise.get("obs_normal"),
                             noise_uniform=noise.get("obs_uniform"), carry_uniform=noise.get("obs_carry_uniform"),
                             **observe_args(t, step))
@@ -267,7 +268,7 @@ class Rollout:
         if self._fuse_obs and t + 1 < self.T and not noise:
             # the next step's observation rides in this launch (its random numbers are those of step + 1)
             c.terms.terminate_reset_observe(st, term_args, src, observe_args(t + 1, step + 1))
-            self._obs_done = (id(env), t + 1, step + 1, _relative_step)
+            self._obs_done = (env, t + 1, step + 1, _relative_step)
         else:
             c.terms.terminate_reset(st, **term_args)
         # refresh the derived fields and the warm start of the reset envs (engine.py:213); in the deferred mode the next
@@ -304,8 +305,7 @@ class Rollout:
     def _capture(self, env: RolloutEnvState, level: float) -> bool:
         """Captures the rollout of `env` at `level` as a HIP graph unless that is the graph already held; True when it
         captured (which synchronises the device)."""
-        key = (id(env), float(level))
-        if self._graph is not None and self._graph[0] == key:
+        if self._graph is not None and self._graph[0][0] is env and self._graph[0][1] == float(level):
             return False
         self.step_base.fill_(env.step)
         self.c.engine.prepare(self.step_base.device)
@@ -318,7 +318,7 @@ class Rollout:
             traj = self.trajectory()
             rewards = self._rewards(traj, env, level)
             self.step_base += self.T
-        self._graph = (key, g, traj, rewards)
+        self._graph = ((env, float(level)), g, traj, rewards)  # with the env state itself: the graph writes to its buffers
         self._graph_step = int(env.step)
         return True
 

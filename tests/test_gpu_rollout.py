@@ -770,6 +770,31 @@ def test_graphs_of_groups_that_share_wide_networks_replay_side_by_side(dtype):
             assert torch.isfinite(x).all() and torch.equal(x, y)
 
 
+def test_a_captured_rollout_keeps_its_env_state():
+    """The graph writes to the buffers of the env state it was captured for, so it holds that object: another state, which may get the address of
+    one that the program has dropped, is captured anew and gives its own rollout."""
+    import gc
+    import weakref
+
+    N, T = 16, 4
+    runs = []
+    for graph in (False, True):
+        m, c, rnd_, _, ro, EnvState = build(N, T, seed=9)
+        run = []
+        for seed in (21, 22, 23):
+            env = EnvState(c.engine.reset(c.physics_model, 1.0, seed, N, rnd_), rnd_, torch.zeros(N, 2, device=DEV), None, seed=seed)
+            traj, rew = ro.unroll(env, graph=graph)
+            run.append([x.clone() for x in (traj.qpos, traj.action, rew.total)])
+            alive = weakref.ref(env)
+            torch.cuda.synchronize()
+            del env
+            gc.collect()
+            assert (alive() is not None) == graph
+        runs.append(run)
+    for a, b in zip(*runs):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
 def test_recurrent_rollout_replayed_after_the_networks_saw_other_batches():
     """A captured rollout of recurrent networks, its scratch first used eagerly, then replayed after the same networks ran larger and smaller
     batches and the memory those gave back was written over."""
