@@ -673,3 +673,77 @@ def test_per_env_model_field_overrides_match_oracle():
         assert (buf["nefc"] >= m.nv - 6).all()  # a friction row per hinge in every env
     with pytest.raises(Exception, match="come together"):
         physics.control_step(dm, dict(buf, sph_radius=None), substeps=1, actuator_type=KS_ACT_TORQUE)
+
+
+def tree_model(n_hinges, spheres, joint_range=None, frictionloss=0.0, feet=2, spacing=0.03, **opts):
+    """Free root, `n_hinges` hinges in four limbs, `spheres` contact spheres at the ends of the first `feet`."""
+    rng = np.random.default_rng(n_hinges)
+    mb = km.ModelBuilder(dt=0.005, **opts)
+    root = mb.add_capsule_body(0, (0.0, 0.0, 1.05), (0.0, 0.0, 1.0), 0.35, 0.1, 12.0, joint="free")
+    ends = []
+    for limb in range(4):
+        side, high = (-1) ** limb, limb // 2
+        parent, pos, d = root, np.array([0.0, 0.1 * side, 0.3 * high]), np.array([0.0, 0.3 * high * side, -1.0])
+        for k in range(n_hinges // 4 + (limb < n_hinges % 4)):
+            ln = rng.uniform(0.08, 0.2)
+            parent = mb.add_capsule_body(parent, pos, d, ln, 0.04, rng.uniform(0.5, 2.0), joint="hinge", axis=np.eye(3)[(k + limb) % 3], damping=0.2,
+                                         armature=rng.uniform(0.01, 0.05), range=joint_range, frictionloss=frictionloss)
+            mb.add_actuator(parent)
+            pos = d / np.linalg.norm(d) * ln
+        ends.append((parent, pos))
+    for s in range(spheres):
+        body, tip = ends[s % feet]
+        mb.add_contact_sphere(body, tip + np.array([spacing * (s // 2) - 0.08, spacing * (s // 4) - 0.05, 0.0]), 0.02)
+    return mb.build()
+
+
+_ROWS = dict(integrator="implicitfast", joint_range=(-0.45, 0.5), frictionloss=0.2)
+_FOOT = dict(feet=1, spacing=0.002)  # every sphere on one foot, close together: all of them touch at once, four rows each
+
+
+@pytest.mark.parametrize("nv,spheres,opts", [(17, 8, {}), (23, 8, _ROWS), (24, 12, {}), (24, 4, dict(_ROWS, condim=1)), (25, 8, _ROWS), (28, 8, {}),
+                                             (29, 8, _ROWS), (31, 12, {}), (32, 12, _ROWS), (32, 4, dict(condim=1)),
+                                             (20, 16, _FOOT), (32, 16, dict(_ROWS, **_FOOT))])
+def test_every_padded_width_of_the_step_kernel(nv, spheres, opts):
+    """Both ends of the 24, 28 and 32 wide instantiations (the last has no spare column for a right-hand side), with and without rows on the dof
+    lanes, up to the 64 constraint rows of 16 contacts.  Tolerance: the file's, or four times single precision's own distance from the float64 oracle on these very
+    states where that is more: the worst of the oracle's float32 build over the inputs and seven copies of them moved by up to one rounding
+    (2^-24 of each number).  That matters only with dry friction, whose rows change their zone at a last bit: 5e-4 of qvel after one step of 25
+    dofs, 9e-4 after ten of 23."""
+    from ksim_amd import physics
+    from ksim_amd._lib_dyn import KS_ACT_TORQUE
+
+    m = tree_model(nv - 6, spheres, **opts)
+    assert m.nv == nv
+    N = 24
+    qpos, qvel = random_states(m, N, seed=11, vel_scale=0.3, joint_range=0.5, contact_fraction=0.8)
+    ctrl = np.random.default_rng(12).normal(size=(N, m.nu)) * 3
+    dm = physics.DeviceModel(m)
+
+    want, singles = {}, {}
+    for steps in (0, 1, 10):
+        want[steps] = oracle_forward(m, qpos, qvel, ctrl, steps=steps)
+        singles[steps] = []
+        for k in range(8):
+            near = np.random.default_rng(k)
+            moved = [x * (1 + 2.0 ** -24 * near.uniform(-1, 1, x.shape)) if k else x for x in (qpos, qvel, ctrl)]
+            singles[steps].append(oracle_forward(m, *moved, steps=steps, dtype=np.float32))
+
+    def compare(got, key, steps, tol):
+        err = rel_err(got.cpu().numpy(), want[steps][key]).max()
+        bound = max(tol, 4 * max(rel_err(f32[key], want[steps][key]).max() for f32 in singles[steps]))
+        assert err <= bound, f"{nv} dofs, {key} after {steps} steps: {err:.2e} > {bound:.2e}"
+
+    buf = dict(qpos=t32(qpos), qvel=t32(qvel), qacc_warmstart=zeros(N, nv), ctrl_in=t32(ctrl), qacc=zeros(N, nv), nefc=zeros(N, dtype=torch.int32),
+               dbg_M=zeros(N, nv * nv), dbg_bias=zeros(N, nv), dbg_qacc_smooth=zeros(N, nv), cfrc_ext=zeros(N, m.nb * 6))
+    physics.forward(dm, buf)
+    assert np.array_equal(buf["nefc"].cpu().numpy(), want[0]["nefc"]) and (want[0]["nefc"] > 0).sum() >= N // 2
+    for name, key, tol in (("dbg_M", "M", 1e-5), ("dbg_bias", "qfrc_bias", 1e-5), ("dbg_qacc_smooth", "qacc_smooth", 1e-4), ("qacc", "qacc", ONE_STEP_TOL),
+                           ("cfrc_ext", "cfrc_ext", 2e-3)):
+        compare(buf[name], key, 0, tol)
+    buf = dict(qpos=t32(qpos), qvel=t32(qvel), qacc_warmstart=zeros(N, nv), time=zeros(N), last_ctrl=t32(ctrl), action=t32(ctrl))
+    for step in range(1, 11):
+        physics.control_step(dm, buf, substeps=1, actuator_type=KS_ACT_TORQUE)
+        if step in (1, 10):
+            for key in ("qpos", "qvel"):
+                compare(buf[key], key, step, ONE_STEP_TOL if step == 1 else TEN_STEP_TOL)
