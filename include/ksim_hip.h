@@ -697,7 +697,8 @@ int ks_sample_action_mixture(ks_stream_t stream, int64_t N, int32_t nu, const fl
  * product, infinities and NaN as in the fp32 product; an operand below 2^-110 counts with an error of up to 2^-133.
  * ks_mlp_create uploads (allocates); ks_mlp_forward allocates nothing: the caller
  * provides ks_mlp_workspace_bytes(mlp, M) bytes of device scratch, which also do for any smaller batch (as do those of
- * the other *_workspace_bytes functions).
+ * the other *_workspace_bytes functions).  Scratch belongs to one call in flight: calls that may overlap on the GPU, and graphs
+ * replayed side by side, each need their own.
  */
 #define KS_MAX_LAYERS 8
 enum { KS_ACT_NONE = 0, KS_ACT_ELU = 1, KS_ACT_RELU = 2, KS_ACT_TANH = 3,
