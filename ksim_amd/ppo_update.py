@@ -210,34 +210,36 @@ def single_step(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, crit
     return metrics
 
 
-def _gather_extent(t: torch.Tensor, d: int) -> tuple[int, int]:
-    """(blocks of columns, bytes of a column) of a contiguous array whose columns lie along axis `d`.  From the sizes alone: the stride of an axis
-    of size one says nothing, and torch leaves it as it was before a transpose or a permutation."""
-    return math.prod(t.shape[:d]), math.prod(t.shape[d + 1:]) * t.element_size()
-
-
-def _gather_fits(t: torch.Tensor, d: int, picked: int) -> bool:
-    """Whether `picked` columns can be counted in the launch's 32 bits even if they have to be moved byte by byte."""
-    return math.prod(_gather_extent(t, d)) * picked <= 0xffffffff
+def _gather_extent(t: torch.Tensor, d: int, picked: int) -> tuple[int, int] | None:
+    """(blocks of columns, bytes of a column) of a contiguous array whose columns lie along axis `d`, or None where `picked` of them cannot be
+    counted in the launch's 32 bits even if they have to be moved byte by byte.  From the sizes alone: the stride of an axis of size one says
+    nothing, and torch leaves it as it was before a transpose or a permutation."""
+    shape, inner = t.shape, t.element_size()
+    blocks = math.prod(shape[:d])
+    for n in shape[d + 1:]:
+        inner *= n
+    return (blocks, inner) if blocks * inner * picked <= 0xffffffff else None
 
 
 def _columns(idx: torch.Tensor, own: bool, arrays: Sequence[tuple[torch.Tensor | None, int]]) -> list:
     """The env columns `idx` of every (array, env axis), contiguous, in one launch.  Only for indices that were drawn here (`own`): a caller's are
     checked where torch checks them, as are arrays that are not plain contiguous memory of the indices' device, or too large for one launch."""
     N = next(t.shape[d] for t, d in arrays if t is not None)
-    picked, out = idx.numel(), [None] * len(arrays)
+    picked, out, device = idx.numel(), [None] * len(arrays), idx.device
     table, keep = [], idx.contiguous()
     for k, (t, d) in enumerate(arrays):
         if t is None:
             continue
-        if (not own or t.shape[d] != N or not t.is_contiguous() or not t.is_cuda or t.device != idx.device or t.requires_grad
-                or len(table) == T.KS_GATHER_ARRAYS or not _gather_fits(t, d, picked)):
+        extent = None
+        if own and t.is_cuda and t.device == device and t.shape[d] == N and t.is_contiguous() and not t.requires_grad and len(table) < T.KS_GATHER_ARRAYS:
+            extent = _gather_extent(t, d, picked)
+        if extent is None:
             out[k] = t.index_select(d, idx).contiguous()
             continue
         shape = list(t.shape)
         shape[d] = picked
-        out[k] = torch.empty(shape, dtype=t.dtype, device=t.device)
-        table.append(T.KsGatherArray(t.data_ptr(), out[k].data_ptr(), *_gather_extent(t, d)))
+        out[k] = torch.empty(shape, dtype=t.dtype, device=device)
+        table.append(T.KsGatherArray(t.data_ptr(), out[k].data_ptr(), *extent))
     if table:
         rc = _lib.load().ks_gather_columns(_lib.current_stream(), len(table), (T.KsGatherArray * len(table))(*table), N, picked, keep.data_ptr())
         _lib.check(rc)

@@ -847,7 +847,7 @@ def test_minibatch_columns_of_one_env_with_strides_of_another_layout(picked):
     idx = torch.zeros(picked, dtype=torch.int64, device="cuda")
     for (t, d), got in zip(arrays, pu._columns(idx, True, arrays)):
         assert t.shape[d] == 1 and t.is_contiguous()
-        blocks, inner = pu._gather_extent(t, d)
+        blocks, inner = pu._gather_extent(t, d, picked)
         assert blocks * inner == t.numel() * t.element_size()
         assert torch.equal(got, t.index_select(d, idx))
 

@@ -605,7 +605,7 @@ def test_the_minibatch_gather_copies_what_the_array_holds(make, d):
 
     t = make(torch)
     assert t.is_contiguous()
-    blocks, inner = _gather_extent(t, d)
+    blocks, inner = _gather_extent(t, d, 1)
     assert blocks * t.shape[d] * inner == t.numel() * t.element_size()
 
 
@@ -616,9 +616,9 @@ def test_the_minibatch_gather_leaves_what_it_cannot_count_to_torch():
     from ksim_amd import ppo_update as pu
 
     big = torch.empty(100, 90000, 475, device="meta")
-    assert not pu._gather_fits(big, 1, 45000) and pu._gather_fits(big, 1, 20000)
+    assert pu._gather_extent(big, 1, 45000) is None and pu._gather_extent(big, 1, 20000) == (100, 1900)
     b = torch.empty(1, 2, 1 << 31, dtype=torch.uint8, device="meta")
-    assert pu._gather_fits(b, 1, 1) and not pu._gather_fits(b, 1, 2)
+    assert pu._gather_extent(b, 1, 1) == (1, 1 << 31) and pu._gather_extent(b, 1, 2) is None
 
     class Cuda:  # a contiguous array of another GPU, as far as the rule looks
         shape, is_cuda, requires_grad, device = (2, 3), True, False, torch.device("cuda", 1)
