@@ -150,12 +150,20 @@ __device__ __forceinline__ float halves(float x, float y, int half) {
   return __builtin_bit_cast(float, half ? r[1] : r[0]);
 }
 
+// Lanes first .. first + count - 1, known at compile time, as the condition of a select: one scalar instruction, which costs the vector issue
+// nothing, instead of a compare (4.5 cycles of it).  `site` is a zero the compiler cannot see through, one per call of a solver: shared between
+// the call sites the masks would be sixty-odd scalar register pairs that live across the solver and are read back from spill lanes.
+// 4096 humanoids 336 -> 329 us per control step, 8192 mixed robots 491 -> 486, 64 robots 235 -> 233 (volatile instead of `site`: 329, 487, 235).
+__device__ __forceinline__ bool in_lanes(int first, int count, int site) {
+  unsigned long long mask;
+  asm("s_bfm_b64 %0, %1, %2" : "=s"(mask) : "i"(count), "i"(first), "s"(site));
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
+}
+
 template <int NP>
-__device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myinv, int lane, int nv) {
-  // The lane id is made opaque so that the per-step lane masks are compared where they are used: shared between the call
-  // sites they would be sixty-odd scalar register pairs that live across the solver and are read back from spill lanes.
-  asm volatile("" : "+v"(lane));
-  const int c = lane & 31, half = lane >> 5;
+__device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myinv, int nv) {
+  int site = 0;
+  asm volatile("" : "+s"(site));
   myinv = 1.f;
   // a pivot below 1e-30 (or not a number) counts as 1e-30: the reciprocal root is capped instead of the pivot floored,
   // which is the same number and one instruction less on the chain
@@ -165,21 +173,21 @@ __device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myin
     if (j >= padded_from(NP) && j >= nv) continue;  // padded columns: unit pivots, nothing below or right of them
     const int hj = (j >> 2) & 1, rho = 4 * (j >> 3) + (j & 3), own = j + 32 * hj;
     const float inv0 = inv_root(lane_bcast(T[rho], own));
-    myinv = lane == j ? inv0 : myinv;
-    const bool right0 = half == hj && c > j;
+    myinv = in_lanes(j, 1, site) ? inv0 : myinv;
+    const bool right0 = in_lanes(own + 1, 31 - j, site);
     float a0 = right0 ? T[rho] : 0.f;  // beside the reciprocal root, not behind it
     a0 *= inv0;
     T[rho] = right0 ? a0 : T[rho];
     const float v = T[rho + 1] - a0 * lane_bcast(a0, own + 1);
     const float inv1 = inv_root(lane_bcast(v, own + 1));
-    myinv = lane == j + 1 ? inv1 : myinv;
-    const bool right1 = half == hj && c > j + 1;
+    myinv = in_lanes(j + 1, 1, site) ? inv1 : myinv;
+    const bool right1 = in_lanes(own + 2, 30 - j, site);
     float a1 = right1 ? v : 0.f;
     a1 *= inv1;
     T[rho + 1] = right1 ? a1 : v;
     // the last real columns have nothing right of or below them
     if (j + 2 < NP && !(j + 2 >= padded_from(NP) && j + 2 >= nv)) {
-      const float b = halves(a0, a1, hj), na = lane == j + 1 ? 0.f : -b;
+      const float b = halves(a0, a1, hj), na = in_lanes(j + 1, 1, site) ? 0.f : -b;
       T = __builtin_amdgcn_mfma_f32_32x32x2f32(na, b, T, 0, 0, 0);
     }
   }
@@ -211,13 +219,15 @@ __device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ 
 // L^T x = y, lane i holding y_i and returning x_i.  With w_i = y_i / L[i][i] a step is w_i -= (R[k] / L[i][i]^2) x_k, x_k = w_k: the scaled
 // and masked coefficient does not wait for the step before, so the chain is one broadcast and one fused multiply-add per column.
 template <int NP>
-__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, int lane, float y, int nv) {
+__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, float y, int nv) {
+  int site = 0;
+  asm volatile("" : "+s"(site));
   const float myinv2 = myinv * myinv;
   float w = y * myinv;
 #pragma unroll
   for (int k = NP - 1; k >= 0; --k) {
     if (k >= padded_from(NP) && k >= nv) continue;  // padded unknowns are zero and couple to nothing
-    const float coef = lane < k ? R[k] * myinv2 : 0.f;
+    const float coef = in_lanes(0, k, site) ? R[k] * myinv2 : 0.f;
     w -= coef * lane_bcast(w, k);
   }
   return w;
@@ -225,16 +235,17 @@ __device__ __forceinline__ float back_substitute(const float (&R)[NP], float myi
 
 // x = (L L^T)^-1 b, lane i holding b_i and returning x_i
 template <int NP>
-__device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, int lane, float b, int nv) {
-  asm volatile("" : "+v"(lane));  // as in chol_tile: the masks lane > j, lane < k are rebuilt here, not kept
+__device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, float b, int nv) {
+  int site = 0;
+  asm volatile("" : "+s"(site));
   float y = b * myinv;
 #pragma unroll
   for (int j = 0; j < NP; ++j) {  // L y = b in the same form
     if (j >= padded_from(NP) && j >= nv) continue;
-    const float coef = lane > j ? R[j] * myinv : 0.f;
+    const float coef = in_lanes(j + 1, 31 - j, site) ? R[j] * myinv : 0.f;
     y -= coef * lane_bcast(y, j);
   }
-  return back_substitute<NP>(R, myinv, lane, y, nv);
+  return back_substitute<NP>(R, myinv, y, nv);
 }
 
 // Factors the tile and returns x = (L L^T)^-1 b, lane i holding b_i (zero beyond nv).  A matrix of fewer than 32 columns carries b
@@ -243,9 +254,9 @@ __device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, i
 // floats).  A substitution step is four instructions of a chain, 26 of them for 26 dofs.
 template <int NP>
 __device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& myinv, int lane, float b, int nv, float* vbuf) {
-  chol_tile<NP>(T, R, myinv, lane, nv);
+  chol_tile<NP>(T, R, myinv, nv);
   if constexpr (NP == 32) {
-    return solve_regs<NP>(R, myinv, lane, b, nv);
+    return solve_regs<NP>(R, myinv, b, nv);
   } else {
     asm volatile("" : "+v"(lane));
     KS_SYNC();
@@ -257,7 +268,7 @@ __device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& my
     KS_SYNC();
     const float y = vbuf[lane & 31];
     KS_SYNC();
-    return back_substitute<NP>(R, myinv, lane, y, nv);
+    return back_substitute<NP>(R, myinv, y, nv);
   }
 }
 
@@ -1201,7 +1212,7 @@ void step_kernel(StepArgs a) {
           amd_factored = amd;
           have_factor = true;
         } else {
-          step_all = solve_regs<NP>(R, myinv, lane, grad, nv);
+          step_all = solve_regs<NP>(R, myinv, grad, nv);
         }
         const float search = is_dof ? -step_all : 0.f;
         KS_PHASE(12)
