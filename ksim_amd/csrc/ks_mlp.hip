@@ -679,10 +679,15 @@ __device__ __forceinline__ f32x16 fused_mma(const u32x4& w, const u32x4& b, f32x
 // One layer's MFMA work of one wavefront: NT output tiles (weights w[t]) times MI row tiles.  `arow` points at
 // this lane's activation fragment of K step 0 (row lane % 32 of the first row tile, k half lane / 32).
 // Weight fragments sit in a register ring kPF steps ahead; activation fragments are read one step ahead.
-template <typename T, int NT, int MI, int kPF, bool SWAP = false>
+// side: memory traffic of the tile that goes on beside the products, side.even(step) and side.odd(step) in turn.
+struct NoSide {
+  __device__ __forceinline__ void even(int) {}
+  __device__ __forceinline__ void odd(int) {}
+};
+template <typename T, int NT, int MI, int kPF, bool SWAP = false, typename Side = NoSide>
 __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x4* __restrict__ w0,
                                                 const u32x4* __restrict__ w1, int nk, const T* __restrict__ arow,
-                                                int lda) {
+                                                int lda, Side&& side = Side{}) {
   static_assert(kPF % 2 == 0, "the activation double buffer relies on an even ring depth");
   constexpr int SK = 32 / (int)sizeof(T);  // k per step
   u32x4 rw[kPF][NT];
@@ -713,6 +718,8 @@ __device__ __forceinline__ void fused_layer_mma(f32x16 (&acc)[2][MI], const u32x
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < MI; ++i) acc[t][i] = fused_mma<T, SWAP>(wf[t], bq[u & 1][i], acc[t][i]);
+      if (u & 1) side.odd(step);
+      else side.even(step);
     }
   }
 #pragma unroll
@@ -759,15 +766,45 @@ __device__ __forceinline__ void fused_store_hidden(const f32x16& acc, T* __restr
 
 // The first `ld` columns of the finished tile's rows (zeros from column `held` on), 16 bytes per thread and pass, to rows m0.. of dst (M, ld); rows
 // from M on are left out.  ld: whole 16-byte pieces, at most one pass of the workgroup.
+// A pass every two steps of the K loop that reads the tile next (a tile of n columns is n / 16 steps and n / 32 passes), the rest behind it.  All at
+// once before the loop, the stores stood ahead of its weights, which are waited for in order: XXX
 template <typename T, int ROWS>
-__device__ __forceinline__ void tile_rows_out(const T* __restrict__ act, int lda, T* __restrict__ dst, int ld, int held, int64_t m0, int64_t M) {
-  constexpr int PC = 16 / (int)sizeof(T);  // entries of a piece
-  const int pieces = ld / PC, per = 64 * kFusedWaves / pieces, r0 = (int)threadIdx.x / pieces, c = ((int)threadIdx.x - r0 * pieces) * PC;
-  if (r0 >= per) return;
-  const int rows = M - m0 < ROWS ? (int)(M - m0) : ROWS;
-  for (int r = r0; r < rows; r += per)
-    *reinterpret_cast<uint4*>(dst + (m0 + r) * ld + c) = c < held ? *reinterpret_cast<const uint4*>(act + r * lda + c) : uint4{0u, 0u, 0u, 0u};
-}
+struct TileRowsOut {
+  static constexpr int PC = 16 / (int)sizeof(T);  // entries of a piece
+  const T* from = nullptr;
+  T* to = nullptr;
+  int64_t to_step = 0;
+  int from_step = 0, per = 1, left = 0;  // left: rows from this thread's next one on
+  bool real = false;
+  uint4 v = {0u, 0u, 0u, 0u};
+
+  __device__ __forceinline__ TileRowsOut() {}
+  __device__ __forceinline__ TileRowsOut(const T* act, int lda, T* dst, int ld, int held, int64_t m0, int64_t M) {
+    const int pieces = ld / PC, r0 = (int)threadIdx.x / pieces, c = ((int)threadIdx.x - r0 * pieces) * PC;
+    per = 64 * kFusedWaves / pieces;
+    left = r0 < per ? (M - m0 < ROWS ? (int)(M - m0) : ROWS) - r0 : 0;
+    real = c < held;
+    from = act + r0 * lda + c;
+    from_step = per * lda;
+    to = dst + (m0 + r0) * ld + c;
+    to_step = (int64_t)per * ld;
+  }
+  __device__ __forceinline__ void even(int) {
+    if (left > 0 && real) v = *reinterpret_cast<const uint4*>(from);
+  }
+  __device__ __forceinline__ void odd(int) {
+    if (left > 0) *reinterpret_cast<uint4*>(to) = v;
+    from += from_step;
+    to += to_step;
+    left -= per;
+  }
+  __device__ __forceinline__ void finish() {
+    while (left > 0) {
+      even(0);
+      odd(0);
+    }
+  }
+};
 
 // Output layer: fp32 rows of the caller's (M, out_dim) matrix.
 __device__ __forceinline__ void fused_store_output(const f32x16& acc, float* __restrict__ y, int64_t M, int out_dim,
@@ -814,10 +851,19 @@ __host__ __device__ inline int fused_share(int nt, int lda) {
 // One layer of the whole-network kernel for one wavefront: MFMA work, barrier, epilogue, barrier.
 template <int ACT, typename T, int MI, bool LAST, bool SAVE, bool SWAP = false>
 __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __restrict__ act, int64_t m0, int lane,
-                                            int wave, int64_t tile) {
+                                            int wave, int64_t tile, TileRowsOut<T, MI * 32>& out) {
   const int nk = a.fk[l], nt = a.fn[l], lda = a.lda;
   const T* arow = act + (lane & 31) * lda + (lane >> 5) * (16 / (int)sizeof(T));
   const int row = lane & 31;
+  // what the layer before left (or the network input) goes out beside this one's products; smaller tiles share the CU with other workgroups,
+  // which do the same, and have no registers for it
+  constexpr bool LATER = SAVE && sizeof(T) == 2 && MI == 4;
+  if constexpr (SAVE && sizeof(T) == 2 && !LATER) out.finish();
+  NoSide none;
+  auto& side = [&]() -> auto& {
+    if constexpr (LATER) return out;
+    else return none;
+  }();
   if (sizeof(T) == 4 && MI <= 2 && nt <= 2) {
     // Few tiles in fp32 (an output layer of 21 or 1 columns): one wavefront's 8 k per 256 cycles would leave the others idle for the
     // layer's whole reduction (256 wide: 3.4 us of 25), so 2 or 4 wavefronts cut a tile's reduction and add up through the tile's
@@ -863,7 +909,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
     }
     acc[1][0] = acc[0][0];
     const u32x4* w0 = a.Wp[l] + (int64_t)j * nk * 64 + lane;
-    if (busy) fused_layer_mma<T, 1, 1, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow + i * 32 * lda, lda);
+    if (busy) fused_layer_mma<T, 1, 1, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow + i * 32 * lda, lda, side);
+    if constexpr (LATER) out.finish();
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();  // every wavefront has read this layer's input; the tile can be overwritten
     KS_MLP_STAMP2(3 + 3 * l)
@@ -890,8 +937,9 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
     }
     const u32x4* w0 = a.Wp[l] + (int64_t)j0 * nk * 64 + lane;
     const u32x4* w1 = a.Wp[l] + (int64_t)j1 * nk * 64 + lane;
-    if (mine == 2) fused_layer_mma<T, 2, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w1, nk, arow, lda);
-    else if (mine == 1) fused_layer_mma<T, 1, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow, lda);
+    if (mine == 2) fused_layer_mma<T, 2, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w1, nk, arow, lda, side);
+    else if (mine == 1) fused_layer_mma<T, 1, MI, (MI == 2 ? 2 : kPF), SWAP>(acc, w0, w0, nk, arow, lda, side);
+    if constexpr (LATER) out.finish();
     KS_MLP_STAMP2(2 + 3 * l)
     __syncthreads();
     KS_MLP_STAMP2(3 + 3 * l)
@@ -909,10 +957,10 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
   }
   __syncthreads();
   KS_MLP_STAMP2(4 + 3 * l)
-  // The next layer only reads the tile until every wavefront (this copy included, which sits before its matrix work in program order) has passed
+  // The next layer only reads the tile until every wavefront (this copy included, which sits before that barrier in program order) has passed
   // the next barrier.  Rows are as wide as the backward pass's layers, which is more than the tile's (zeros) where the width is no multiple of 128.
   if constexpr (sizeof(T) == 2) {
-    if (SAVE && !LAST) tile_rows_out<T, MI * 32>(act, lda, reinterpret_cast<T*>(a.save[l]), a.save_ld[l], nt * 32, m0, a.save_rows);
+    if (SAVE && !LAST) out = TileRowsOut<T, MI * 32>(act, lda, reinterpret_cast<T*>(a.save[l]), a.save_ld[l], nt * 32, m0, a.save_rows);
   } else if (!LAST && a.save[l]) {  // one form for both in fp32, whose code without this is 4 % slower (8192 rows of 71-256-256-256-21: 31.5 -> 32.9 us)
     T* dst = reinterpret_cast<T*>(a.save[l]);
     const int ld = a.save_ld[l], w4 = ld / 4, held = nt * 8;
@@ -994,10 +1042,11 @@ __device__ __forceinline__ void mlp_fused_body(const FusedArgs& a, int64_t tile)
   }
   __syncthreads();
   KS_MLP_STAMP(1)
-  if (SAVE && a.save_in) tile_rows_out<T, BM>(act, lda, reinterpret_cast<T*>(a.save_in), a.in_width, a.in_width, m0, a.save_rows);  // the tile stays until the first layer's barrier
+  TileRowsOut<T, BM> out;
+  if (SAVE && a.save_in) out = TileRowsOut<T, BM>(act, lda, reinterpret_cast<T*>(a.save_in), a.in_width, a.in_width, m0, a.save_rows);  // the tile stays until the first layer's barrier
   if constexpr (!SINGLE)
-    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false, SAVE>(a, l, act, m0, lane, wave, tile);
-  fused_layer<ACT, T, MI, true, SAVE, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile);
+    for (int l = 0; l + 1 < a.n_layers; ++l) fused_layer<ACT, T, MI, false, SAVE>(a, l, act, m0, lane, wave, tile, out);
+  fused_layer<ACT, T, MI, true, SAVE, SINGLE>(a, SINGLE ? 0 : a.n_layers - 1, act, m0, lane, wave, tile, out);
 }
 
 // SINGLE: one bf16 layer
@@ -1227,9 +1276,10 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     }
   }
   __syncthreads();
-  // The finished tile and its column sums (the bias gradient's share) go out while the next K loop reads the tile, as this does
+  // The finished tile's column sums (the bias gradient's share) go out before the next K loop reads the tile, the tile itself beside it
+  TileRowsOut<__bf16, BM> out;
   auto tile_out = [&](__bf16* dst, float* bias_part, int width) {
-    tile_rows_out<__bf16, BM>(act, lda, dst, width, width, m0, m0 + BM);
+    out = TileRowsOut<__bf16, BM>(act, lda, dst, width, width, m0, m0 + BM);
     if (tid >= width / 2) return;
     f32x2 cs = {0.f, 0.f};
 #pragma unroll 8
@@ -1258,8 +1308,9 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
         for (int r = 0; r < 16; ++r) acc[t][i][r] = 0.f;
     const u32x4* w0 = a.WtP[l] + (int64_t)j0 * nk * 64 + lane;
     const u32x4* w1 = a.WtP[l] + (int64_t)j1 * nk * 64 + lane;
-    if (mine == 2) fused_layer_mma<__bf16, 2, MI, kPF>(acc, w0, w1, nk, arow, lda);
-    else if (mine == 1) fused_layer_mma<__bf16, 1, MI, kPF>(acc, w0, w0, nk, arow, lda);
+    if (mine == 2) fused_layer_mma<__bf16, 2, MI, kPF>(acc, w0, w1, nk, arow, lda, out);
+    else if (mine == 1) fused_layer_mma<__bf16, 1, MI, kPF>(acc, w0, w0, nk, arow, lda, out);
+    out.finish();
     // Y_{l-1} takes dZ_l's place in the tile on its way to the lanes that need it, and every lane leaves dZ_{l-1} where it read Y: whole rows in
     // 16-byte pieces in and out of memory, 8 bytes per lane of the tile.
     const int width = nt * 32, pieces = width / 8, per = NTHR / pieces, yr = tid / pieces, yc = (tid - yr * pieces) * 8;
@@ -1304,6 +1355,7 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     __syncthreads();
     tile_out(a.dz[l - 1], a.bias_part[l - 1], width);
   }
+  out.finish();
 }
 
 // Weight gradients behind it: slice z of C (np, kp) = dZ^T Y over rows [z kslice, (z + 1) kslice) of dZ (lda = np columns) and Y (ldb columns), both
