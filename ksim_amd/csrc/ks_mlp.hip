@@ -1710,7 +1710,10 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(int64_t n, int nz, const
 
 // Every gradient of a network from its partial sums, in one launch (the whole-network backward pass): weight gradient l =
 // the sum of its nz[l] row slices, z ascending as in sum_parts_kernel; bias gradient l = the sum over the row tiles of the
-// per-tile column sums, four columns per workgroup with one wavefront each and the fixed tree of sum_parts_tree_kernel.
+// per-tile column sums, in the order of sum_parts_tree_kernel.
+// Bound by memory.  Weights (padded to whole matrix tiles) go four to a thread in 16-byte loads.  A workgroup takes sixteen columns of bias sums, a
+// row of them 64 bytes: a wavefront per column fetched 64 rows for 4 bytes of each.  XXX
+constexpr int kFinishCols = 16;
 struct GradFinishArgs {
   int n_layers, tiles;
   int nz[KS_MAX_LAYERS], nb[KS_MAX_LAYERS];
@@ -1720,35 +1723,62 @@ struct GradFinishArgs {
   float *gW[KS_MAX_LAYERS], *gb[KS_MAX_LAYERS];
 };
 __global__ __launch_bounds__(256) void grad_finish_kernel(GradFinishArgs a) {
-  const int b = blockIdx.x;
-  if (b < a.first_w[a.n_layers]) {
+  __shared__ float lanes[64][kFinishCols + 1];
+  const int nbias = a.first_b[a.n_layers], t = threadIdx.x;
+  if ((int)blockIdx.x >= nbias) {  // the biases first: their chains are the longer ones
+    const int b = blockIdx.x - nbias;
     int l = 0;
     while (l + 1 < a.n_layers && b >= a.first_w[l + 1]) ++l;
-    const int64_t i = (int64_t)(b - a.first_w[l]) * 256 + threadIdx.x, n = a.nW[l];
+    const int64_t i = ((int64_t)(b - a.first_w[l]) * 256 + t) * 4, n = a.nW[l];
     if (i >= n) return;
-    float s = 0.f;
-    const float* part = a.wpart[l];
+    float4 s = {0.f, 0.f, 0.f, 0.f};
+    const float* part = a.wpart[l] + i;
     const int nz = a.nz[l];
     for (int z0 = 0; z0 < nz; z0 += 8) {  // eight slices' loads in flight, added in slice order
-      float v[8];
+      float4 v[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = z0 + k < nz ? part[(int64_t)(z0 + k) * n + i] : 0.f;
+      for (int k = 0; k < 8; ++k) v[k] = z0 + k < nz ? *reinterpret_cast<const float4*>(part + (int64_t)(z0 + k) * n) : float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (z0 + k < nz) s += v[k];
+        if (z0 + k < nz) { s.x += v[k].x; s.y += v[k].y; s.z += v[k].z; s.w += v[k].w; }
     }
-    a.gW[l][i] = s;
+    *reinterpret_cast<float4*>(a.gW[l] + i) = s;
     return;
   }
-  const int bb = b - a.first_w[a.n_layers];
+  const int b = blockIdx.x;
   int l = 0;
-  while (l + 1 < a.n_layers && bb >= a.first_b[l + 1]) ++l;
-  const int c = (bb - a.first_b[l]) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, n = a.nb[l];
-  if (c >= n) return;
-  float s = 0.f;
-  for (int z = lane; z < a.tiles; z += 64) s += a.bpart[l][(int64_t)z * n + c];
-  for (int w = 32; w > 0; w >>= 1) s += __shfl_down(s, w);  // lane k adds lane k + w: the same tree for every column
-  if (lane == 0) a.gb[l][c] = s;
+  while (l + 1 < a.n_layers && b >= a.first_b[l + 1]) ++l;
+  const int n = a.nb[l], c0 = (b - a.first_b[l]) * kFinishCols, c = t % kFinishCols, k0 = t / kFinishCols;
+  {  // thread (column c, k0) is lanes k0, k0 + 16, + 32 and + 48 of the column's sum: lane k adds the tiles k, k + 64, ...
+    constexpr int Q = 64 * kFinishCols / 256;
+    float s[Q] = {};
+    if (c0 + c < n) {
+      const float* part = a.bpart[l] + c0 + c;
+      for (int z0 = 0; z0 < a.tiles; z0 += 128) {  // two rounds of the lanes in flight
+        float v[2][Q];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            const int z = z0 + 64 * h + k0 + 16 * q;
+            v[h][q] = z < a.tiles ? part[(int64_t)z * n] : 0.f;
+          }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) s[q] += v[h][q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) lanes[k0 + 16 * q][c] = s[q];
+  }
+  __syncthreads();
+  const int lane = t & 63;
+  for (int cc = t >> 6; cc < kFinishCols; cc += 4) {
+    float s = lanes[lane][cc];
+    for (int w = 32; w > 0; w >>= 1) s += __shfl_down(s, w);  // lane k adds lane k + w: the same tree for every column
+    if (lane == 0 && c0 + cc < n) a.gb[l][c0 + cc] = s;
+  }
 }
 
 
@@ -2755,8 +2785,8 @@ static int train_backward_chain(DevMlp& m, hipStream_t s, int64_t M, const float
   }
   for (int l = 0; l < L; ++l) {
     g.first_w[l] = wblocks; g.first_b[l] = bblocks;
-    wblocks += (int)((g.nW[l] + 255) / 256);
-    bblocks += (g.nb[l] + 3) / 4;
+    wblocks += (int)((g.nW[l] + 1023) / 1024);
+    bblocks += (g.nb[l] + kFinishCols - 1) / kFinishCols;
   }
   g.first_w[L] = wblocks; g.first_b[L] = bblocks;
   hipLaunchKernelGGL(grad_finish_kernel, dim3((unsigned)(wblocks + bblocks)), dim3(256), 0, s, g);
