@@ -767,7 +767,8 @@ __device__ __forceinline__ void fused_store_hidden(const f32x16& acc, T* __restr
 // The first `ld` columns of the finished tile's rows (zeros from column `held` on), 16 bytes per thread and pass, to rows m0.. of dst (M, ld); rows
 // from M on are left out.  ld: whole 16-byte pieces, at most one pass of the workgroup.
 // A pass every two steps of the K loop that reads the tile next (a tile of n columns is n / 16 steps and n / 32 passes), the rest behind it.  All at
-// once before the loop, the stores stood ahead of its weights, which are waited for in order: XXX
+// once before the loop, the stores stood ahead of its weights, which are waited for in order: 65536 rows of 68-512-512-512-20, training forward
+// 120 -> 114 us, backward 171 -> 167.
 template <typename T, int ROWS>
 struct TileRowsOut {
   static constexpr int PC = 16 / (int)sizeof(T);  // entries of a piece
@@ -1712,7 +1713,8 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(int64_t n, int nz, const
 // the sum of its nz[l] row slices, z ascending as in sum_parts_kernel; bias gradient l = the sum over the row tiles of the
 // per-tile column sums, in the order of sum_parts_tree_kernel.
 // Bound by memory.  Weights (padded to whole matrix tiles) go four to a thread in 16-byte loads.  A workgroup takes sixteen columns of bias sums, a
-// row of them 64 bytes: a wavefront per column fetched 64 rows for 4 bytes of each.  XXX
+// row of them 64 bytes: a wavefront per column fetched 64 rows for 4 bytes of each.  68-512-512-512-20
+// over 65536 rows: 25 -> 16.7 us (65 MB of slices).
 constexpr int kFinishCols = 16;
 struct GradFinishArgs {
   int n_layers, tiles;
