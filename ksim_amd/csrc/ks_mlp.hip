@@ -3,6 +3,7 @@
 // whole-network kernels.  Output fragment layout (both): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "ks_common.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <cstdlib>
@@ -12,6 +13,7 @@ namespace ks {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;  // a 16-byte register vector (plain vector type, so arrays of it stay in registers)
@@ -3405,6 +3407,247 @@ __global__ __launch_bounds__(1024) void disc_wgrad_kernel(SgemmGroup t, DiscLoss
   sgemm_tile<false, false, 16>(g, tile % gx, tile / gx, at / (gx * gy), gx, gy, t.slices[l]);
 }
 
+// Everything of the discriminator's gradient that stays inside a frame, in one launch: the forward pass, the input gradient's chain and the sweep
+// back through it on the real rows, the ordinary backward pass.  A workgroup takes 16 rows through all of it, the operand of the next product in
+// LDS, 16 columns of a product to a wavefront on v_mfma_f32_16x16x4_f32, the weights straight from L2.  Arrays that a later phase reads by entry
+// (y, a, r) are read by the thread that wrote them.
+// Few frames are bound by the chain of products itself (63 us for 2 x 1024 frames of 71-256-256-1, of which the matrix instructions are 17), where
+// a launch per product (sgemm_kernel) added a launch, its gap and a trip of the operands through memory to each.  The whole gradient of
+// 71-256-256-1, launches per product -> this: 2 x 32 frames 77 -> 65 us, 2 x 1024 100 -> 79, 2 x 12288 537 -> 381, 2 x 131072 5560 -> 3980;
+// 71-128-128-1 65 -> 35, 71 -> 44, 241 -> 178, 2290 -> 1870; 60-256-1 43 -> 24, 51 -> 31, 194 -> 111, 1900 -> 1110.
+// Requesting a product's first weights before the stores of the one before it was slower (63 -> 68 us).
+struct DiscRowsArgs {
+  int L, act, penalty, lda, zeros, tiles_real;
+  int64_t R, M;
+  float scale;
+  const float *real, *sim;
+  int dims[KS_MAX_LAYERS + 1], ld[KS_MAX_LAYERS];
+  const float *W[KS_MAX_LAYERS], *b[KS_MAX_LAYERS];
+  float *y[KS_MAX_LAYERS], *a[KS_MAX_LAYERS], *d[KS_MAX_LAYERS], *r[KS_MAX_LAYERS], *v[KS_MAX_LAYERS], *dz[KS_MAX_LAYERS];
+  float *g, *ones;
+  double* sums;  // one sum of squares per tile of real rows
+  unsigned* zero;
+};
+constexpr int kDrRows = 16, kDrWaves = 16;
+
+// Columns j0 .. j0 + 15 of op (16 rows, K) times W^T (KC: W stored (j, k)) or W (stored (k, j)); op: this lane's row at its first k, zeros from K to
+// the next multiple of 16.  A lane of quarter h feeds k = 16 s + 4 h + e to instruction e of step s; four steps' weights are in flight under four
+// steps' products.  Columns from N on repeat the last one.
+template <bool KC>
+__device__ __forceinline__ f32x4 disc_product(const float* __restrict__ op, const float* __restrict__ W, int ld, int K, int N, int j0, int lane) {
+  const int j = min(j0 + (lane & 15), N - 1), h = lane >> 4, nk = (K + 15) / 16;
+  float w[16], next[16];
+  const unsigned own = KC ? (unsigned)(j * ld + 4 * h) : (unsigned)(4 * h * ld + j);  // beside an address that the whole wavefront shares
+  auto fetch = [&](float (&t)[16], int s0) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k0 = 16 * min(s0 + s, nk - 1);
+      if (KC) {
+        const float4 x = *reinterpret_cast<const float4*>(W + k0 + own);
+        t[4 * s] = x.x; t[4 * s + 1] = x.y; t[4 * s + 2] = x.z; t[4 * s + 3] = x.w;
+      } else if (k0 + 16 <= K) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[4 * s + e] = (W + (int64_t)(k0 + e) * ld)[own];
+      } else {  // the reduction ends inside the step: rows past it repeat the last one, the operand is zero there
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[4 * s + e] = W[(int64_t)min(k0 + 4 * h + e, K - 1) * ld + j];
+      }
+    }
+  };
+  f32x4 even = {0.f, 0.f, 0.f, 0.f}, odd = {0.f, 0.f, 0.f, 0.f};
+  fetch(w, 0);
+  for (int s0 = 0; s0 < nk; s0 += 4) {
+    if (s0 + 4 < nk) fetch(next, s0 + 4);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s0 + s < nk) {
+        const float4 x = *reinterpret_cast<const float4*>(op + 16 * (s0 + s));
+        even = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, w[4 * s], even, 0, 0, 0);
+        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, w[4 * s + 1], odd, 0, 0, 0);
+        even = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, w[4 * s + 2], even, 0, 0, 0);
+        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, w[4 * s + 3], odd, 0, 0, 0);
+      }
+#pragma unroll
+    for (int s = 0; s < 16; ++s) w[s] = next[s];
+  }
+  return even + odd;
+}
+
+__global__ __launch_bounds__(64 * kDrWaves) void disc_rows_kernel(const DiscRowsArgs a) {
+  extern __shared__ __align__(16) float disc_rows_lds[];
+  __shared__ float err[kDrRows];
+  __shared__ double sred[kDrWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, h = lane >> 4, L = a.L, lda = a.lda;
+  const bool real = (int)blockIdx.x < a.tiles_real, pen = real && a.penalty;
+  const int64_t row0 = real ? (int64_t)blockIdx.x * kDrRows : a.R + (int64_t)((int)blockIdx.x - a.tiles_real) * kDrRows;
+  const int64_t left = (real ? a.R : a.M) - row0;
+  const int rows = left < kDrRows ? (int)left : kDrRows;
+  float *cur = disc_rows_lds, *nxt = cur + kDrRows * lda, *top = nxt + kDrRows * lda;
+  const int at = c * lda + 4 * h;  // this lane's operand
+  if (blockIdx.x == 0)
+    for (int x = tid; x < a.zeros; x += 64 * kDrWaves) a.zero[x] = 0;
+  {
+    const int K = a.dims[0], w16 = (K + 15) / 16 * 16;
+    const float* x = real ? a.real + row0 * K : a.sim + (row0 - a.R) * K;
+    for (int e = tid; e < kDrRows * w16; e += 64 * kDrWaves) {
+      const int i = e / w16, k = e - i * w16;
+      cur[i * lda + k] = i < rows && k < K ? x[i * K + k] : 0.f;
+    }
+  }
+  __syncthreads();
+  auto turn = [&]() {
+    __syncthreads();  // the next operand is whole; the one before it can be overwritten
+    float* t = cur;
+    cur = nxt;
+    nxt = t;
+  };
+  // own entries (4 h + r, j) of a row-major array of width N, zero where there is none
+  auto own = [&](const float* p, int N, int j, float (&v)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = j < N && 4 * h + r < rows ? p[(row0 + 4 * h + r) * N + j] : 0.f;
+  };
+
+  for (int l = 0; l + 1 < L; ++l) {
+    const int N = a.dims[l + 1];
+    const bool opens = pen && l == L - 2;
+    for (int j0 = 16 * wave; j0 < N; j0 += 16 * kDrWaves) {
+      const f32x4 z = disc_product<true>(cur + at, a.W[l], a.ld[l], a.dims[l], N, j0, lane);
+      const int j = j0 + c;
+      const float bias = j < N ? a.b[l][j] : 0.f, x = opens && j < N ? a.W[L - 1][j] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 4 * h + r;
+        const bool held = j < N && i < rows;
+        float y = z[r] + bias, d1, d2;
+        if (a.act == KS_ACT_ELU) y = y > 0.f ? y : expm1f(y);
+        else if (a.act == KS_ACT_RELU) y = fmaxf(y, 0.f);
+        else if (a.act == KS_ACT_TANH) y = tanhf(y);
+        nxt[i * lda + j] = j < N ? y : 0.f;
+        const int64_t o = (row0 + i) * N + j;
+        if (held) a.y[l][o] = y;
+        if (!opens) continue;
+        act_derivatives(a.act, y, d1, d2);
+        const float dd = d1 * x;
+        top[i * lda + j] = j < N ? dd : 0.f;
+        if (held) { a.a[l][o] = x; a.d[l][o] = dd; }
+      }
+    }
+    turn();
+  }
+  {  // the output layer, a row to a wavefront
+    float s = 0.f;
+    for (int k = lane; k < a.dims[L - 1]; k += 64) s += cur[wave * lda + k] * a.W[L - 1][k];
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) s += __shfl_xor(s, w);
+    if (lane == 0) {
+      const float e = s + a.b[L - 1][0] - (real ? 1.f : -1.f);
+      err[wave] = e;
+      if (wave < rows) {
+        a.dz[L - 1][row0 + wave] = e;
+        if (real) a.ones[row0 + wave] = 1.f;
+      }
+    }
+  }
+  __syncthreads();
+
+  if (pen) {
+    float* t = cur;  // the chain starts from the d that the last hidden layer left
+    cur = top;
+    top = t;
+    for (int l = L - 2; l > 0; --l) {
+      const int N = a.dims[l];
+      for (int j0 = 16 * wave; j0 < N; j0 += 16 * kDrWaves) {
+        const int j = j0 + c;
+        float y[4], d1, d2;
+        own(a.y[l - 1], N, j, y);
+        const f32x4 z = disc_product<false>(cur + at, a.W[l], a.ld[l], a.dims[l + 1], N, j0, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * h + r;
+          act_derivatives(a.act, y[r], d1, d2);
+          const float dd = d1 * z[r];
+          nxt[i * lda + j] = j < N ? dd : 0.f;
+          if (j < N && i < rows) { a.a[l - 1][(row0 + i) * N + j] = z[r]; a.d[l - 1][(row0 + i) * N + j] = dd; }
+        }
+      }
+      turn();
+    }
+    double sq = 0.0;
+    {
+      const int N = a.dims[0];
+      for (int j0 = 16 * wave; j0 < N; j0 += 16 * kDrWaves) {
+        const f32x4 z = disc_product<false>(cur + at, a.W[0], a.ld[0], a.dims[1], N, j0, lane);
+        const int j = j0 + c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * h + r;
+          const float gg = a.scale * z[r];
+          nxt[i * lda + j] = j < N ? gg : 0.f;
+          if (j < N && i < rows) {
+            a.g[(row0 + i) * N + j] = gg;
+            sq += (double)z[r] * z[r];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) sq += __shfl_down(sq, w);
+    if (lane == 0) sred[wave] = sq;
+    turn();
+    if (tid == 0) {
+      double s = 0.0;
+      for (int w = 0; w < kDrWaves; ++w) s += sred[w];
+      a.sums[blockIdx.x] = s;
+    }
+    for (int l = 1; l < L; ++l) {
+      const int N = a.dims[l];
+      for (int j0 = 16 * wave; j0 < N; j0 += 16 * kDrWaves) {
+        const int j = j0 + c;
+        float y[4], x[4], d1, d2;
+        own(a.y[l - 1], N, j, y);
+        own(a.a[l - 1], N, j, x);
+        const f32x4 z = disc_product<true>(cur + at, a.W[l - 1], a.ld[l - 1], a.dims[l - 1], N, j0, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * h + r;
+          act_derivatives(a.act, y[r], d1, d2);
+          const float vv = z[r] * d1;
+          nxt[i * lda + j] = j < N ? vv : 0.f;
+          if (j < N && i < rows) { a.r[l - 1][(row0 + i) * N + j] = z[r] * x[r] * d2; a.v[l - 1][(row0 + i) * N + j] = vv; }
+        }
+      }
+      turn();
+    }
+  }
+
+  for (int l = L; l > 1; --l) {  // gradient of z_{l-1}
+    const int N = a.dims[l - 1];
+    for (int j0 = 16 * wave; j0 < N; j0 += 16 * kDrWaves) {
+      const int j = j0 + c;
+      float y[4], x[4] = {0.f, 0.f, 0.f, 0.f}, d1, d2;
+      own(a.y[l - 2], N, j, y);
+      if (pen) own(a.r[l - 2], N, j, x);
+      f32x4 z;
+      if (l == L) {
+        const float w = j < N ? a.W[L - 1][j] : 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[r] = err[4 * h + r] * w;
+      } else {
+        z = disc_product<false>(cur + at, a.W[l - 1], a.ld[l - 1], a.dims[l], N, j0, lane);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 4 * h + r;
+        act_derivatives(a.act, y[r], d1, d2);
+        const float dd = z[r] * d1 + x[r];
+        nxt[i * lda + j] = j < N ? dd : 0.f;
+        if (j < N && i < rows) a.dz[l - 2][(row0 + i) * N + j] = dd;
+      }
+    }
+    turn();
+  }
+}
+
 // The weight and bias gradient of a single layer over many rows, C(i, j) = sum_k A(k, i) B(k, j) with both operands fp32 and stored
 // (k, .), on the bf16 matrix instruction.  PARTS = 1: operands rounded to bf16, what a bf16 network's products take.  PARTS = 3: fp32, every
 // value cut in three (cut_bf16, mma_cut).
@@ -3636,6 +3879,19 @@ struct DiscWs {
 
 static int64_t disc_penalty_tiles(const DevMlp& m, int64_t R) { return ((R + 31) / 32) * ((m.dims[0] + 31) / 32); }
 
+// Floats of a row in disc_rows_kernel's LDS, 0 where the launches per product are to run: a linear network has no chain, and three operands of 16
+// rows in the 64 KiB that a launch has without asking end at 320 columns.  Layers narrower than 128 leave wavefronts of the chain idle, which
+// counts once the rows fill the chip many times over (40-48-1: 53 -> 36 us at 6144 rows, 93 -> 82 at 24576, but 535 -> 600 at 262144).
+static int disc_rows_lda(const DevMlp& m, int64_t M) {
+  int w = 0;
+  for (int l = 0; l < m.n_layers; ++l) {
+    const int r = round_up(m.dims[l], 16);
+    if (m.kpad[l] < r || m.kpad[l] % 4) return 0;
+    w = r > w ? r : w;
+  }
+  return m.n_layers > 1 && w <= 320 && (w >= 128 || M <= 65536) ? w + 4 : 0;
+}
+
 static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, DiscWs* ws) {
   int64_t off = 0;
   auto take = [&](int64_t floats) {
@@ -3655,7 +3911,7 @@ static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, Dis
   }
   w.g = take(R * m.dims[0]);
   w.ones = take(R);
-  w.sums = (double*)take(2 * disc_penalty_tiles(m, R));
+  w.sums = (double*)take(2 * std::max(disc_penalty_tiles(m, R), (R + ks::kDrRows - 1) / ks::kDrRows));
   w.part = take((int64_t)m.n_layers * 512 * kTilePart);  // a sliced product has at most 512 (slice, tile) pairs
   w.counters = (unsigned*)take((int64_t)m.n_layers * 512);
   if (ws) *ws = w;
@@ -3754,52 +4010,68 @@ extern "C" int ks_mlp_disc_loss_grad(KsMlp* h, ks_stream_t stream, int64_t n_rea
   DiscWs ws;
   carve_disc(m, R, M, (char*)workspace, &ws);
   SgemmArgs z = {};  // fields left out below are zero
-  // forward over the real rows, then the simulated ones; the last hidden layer also opens the input gradient's chain (a, d of its output), the
-  // output layer leaves the gradient of the squared errors
-  for (int l = 0; l < L; ++l) {
-    SgemmArgs g = z;
-    g.M = (int)M; g.N = m.dims[l + 1]; g.K = m.dims[l];
-    if (l > 0) g.A = ws.y[l - 1];
-    else if (R == 0 || n_sim == 0) g.A = R ? real : sim;
-    else { g.A = real; g.A2 = sim; g.a_split = (int)R; }
-    g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l];
-    g.ldc = g.N; g.bias = m.mb[l]; g.act = act; g.x_rows = (int)R;
-    if (l == 0) { g.zero = ws.counters; g.zeros = 512 * L; }
-    if (l == L - 1) { g.epi = kEpiOut; g.C = ws.dz[l]; g.C2 = ws.ones; }
-    else if (l == L - 2 && penalty) { g.epi = kEpiTop; g.C = ws.y[l]; g.X = m.mW[L - 1]; g.C2 = ws.a[l]; g.C3 = ws.d[l]; }
-    else { g.epi = kEpiLayer; g.C = ws.y[l]; }
-    sgemm_go<true>(s, g);
-  }
-
-  DiscLosses losses_of = {R, M, 0, ws.dz[L - 1], ws.sums, 0.0, losses};
-  if (penalty) {
-    // input gradient on the real rows: d_L = 1, d_{L-1} from the forward pass, down to g = d_1 W_1, which leaves its tiles as the penalty's
-    // gradient
-    for (int l = L > 1 ? L - 2 : 0; l >= 0; --l) {  // hidden layer l (its output is y[l - 1]); l = 0: the input
-      SgemmArgs g = z;
-      g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l + 1];
-      g.A = l + 1 == L ? ws.ones : ws.d[l]; g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l]; g.ldc = g.N; g.act = act;
-      if (l > 0) { g.C = ws.a[l - 1]; g.C2 = ws.d[l - 1]; g.Y = ws.y[l - 1]; g.epi = kEpiDelta; }
-      else { g.C = ws.g; g.epi = kEpiPenalty; g.scale = grad_penalty_coef * (1.f / (float)n_motions); g.sums = ws.sums; }
-      sgemm_go<false>(s, g);
+  DiscLosses losses_of = {R, M, 0, ws.dz[L - 1], ws.sums, penalty ? 0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions) : 0.0, losses};
+  const float penalty_scale = penalty ? grad_penalty_coef * (1.f / (float)n_motions) : 0.f;
+  const int lda = disc_rows_lda(m, M);
+  if (lda) {
+    DiscRowsArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.L = L; a.act = act; a.penalty = penalty; a.lda = lda; a.zeros = 512 * L; a.zero = ws.counters;
+    a.R = R; a.M = M; a.scale = penalty_scale; a.real = real; a.sim = sim; a.g = ws.g; a.ones = ws.ones; a.sums = ws.sums;
+    a.tiles_real = (int)((R + kDrRows - 1) / kDrRows);
+    for (int l = 0; l < L; ++l) {
+      a.dims[l] = m.dims[l]; a.ld[l] = m.kpad[l]; a.W[l] = m.mW[l]; a.b[l] = m.mb[l]; a.y[l] = ws.y[l]; a.a[l] = ws.a[l];
+      a.d[l] = ws.d[l]; a.r[l] = ws.r[l]; a.v[l] = ws.v[l]; a.dz[l] = ws.dz[l];
     }
-    losses_of.tiles = disc_penalty_tiles(m, R);
-    losses_of.factor = 0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions);
-    for (int l = 1; l < L; ++l) {  // the sweep back through that computation, first layer to last
+    a.dims[L] = 1;
+    if (penalty) losses_of.tiles = a.tiles_real;
+    const int tiles = a.tiles_real + (int)((n_sim + kDrRows - 1) / kDrRows);
+    hipLaunchKernelGGL(disc_rows_kernel, dim3((unsigned)tiles), dim3(64 * kDrWaves), 3 * kDrRows * lda * sizeof(float), s, a);
+  } else {
+    // forward over the real rows, then the simulated ones; the last hidden layer also opens the input gradient's chain (a, d of its output), the
+    // output layer leaves the gradient of the squared errors
+    for (int l = 0; l < L; ++l) {
       SgemmArgs g = z;
-      g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l - 1];
-      g.A = l == 1 ? ws.g : ws.v[l - 2]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
-      g.C = ws.v[l - 1]; g.C2 = ws.r[l - 1]; g.ldc = g.N; g.Y = ws.y[l - 1]; g.X = ws.a[l - 1]; g.act = act; g.epi = kEpiTangent;
+      g.M = (int)M; g.N = m.dims[l + 1]; g.K = m.dims[l];
+      if (l > 0) g.A = ws.y[l - 1];
+      else if (R == 0 || n_sim == 0) g.A = R ? real : sim;
+      else { g.A = real; g.A2 = sim; g.a_split = (int)R; }
+      g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l];
+      g.ldc = g.N; g.bias = m.mb[l]; g.act = act; g.x_rows = (int)R;
+      if (l == 0) { g.zero = ws.counters; g.zeros = 512 * L; }
+      if (l == L - 1) { g.epi = kEpiOut; g.C = ws.dz[l]; g.C2 = ws.ones; }
+      else if (l == L - 2 && penalty) { g.epi = kEpiTop; g.C = ws.y[l]; g.X = m.mW[L - 1]; g.C2 = ws.a[l]; g.C3 = ws.d[l]; }
+      else { g.epi = kEpiLayer; g.C = ws.y[l]; }
       sgemm_go<true>(s, g);
     }
-  }
+    if (penalty) {
+      // input gradient on the real rows: d_L = 1, d_{L-1} from the forward pass, down to g = d_1 W_1, which leaves its tiles as the penalty's
+      // gradient
+      for (int l = L > 1 ? L - 2 : 0; l >= 0; --l) {  // hidden layer l (its output is y[l - 1]); l = 0: the input
+        SgemmArgs g = z;
+        g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l + 1];
+        g.A = l + 1 == L ? ws.ones : ws.d[l]; g.lda = g.K; g.B = m.mW[l]; g.ldb = m.kpad[l]; g.ldc = g.N; g.act = act;
+        if (l > 0) { g.C = ws.a[l - 1]; g.C2 = ws.d[l - 1]; g.Y = ws.y[l - 1]; g.epi = kEpiDelta; }
+        else { g.C = ws.g; g.epi = kEpiPenalty; g.scale = penalty_scale; g.sums = ws.sums; }
+        sgemm_go<false>(s, g);
+      }
+      losses_of.tiles = disc_penalty_tiles(m, R);
+      for (int l = 1; l < L; ++l) {  // the sweep back through that computation, first layer to last
+        SgemmArgs g = z;
+        g.M = (int)R; g.N = m.dims[l]; g.K = m.dims[l - 1];
+        g.A = l == 1 ? ws.g : ws.v[l - 2]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+        g.C = ws.v[l - 1]; g.C2 = ws.r[l - 1]; g.ldc = g.N; g.Y = ws.y[l - 1]; g.X = ws.a[l - 1]; g.act = act; g.epi = kEpiTangent;
+        sgemm_go<true>(s, g);
+      }
+    }
 
-  // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows
-  for (int l = L; l > 1; --l) {
-    SgemmArgs g = z;
-    g.M = (int)M; g.N = m.dims[l - 1]; g.K = m.dims[l]; g.A = ws.dz[l - 1]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
-    g.C = ws.dz[l - 2]; g.ldc = g.N; g.Y = ws.y[l - 2]; g.X = ws.r[l - 2]; g.x_rows = penalty ? (int)R : 0; g.act = act; g.epi = kEpiDz;
-    sgemm_go<false>(s, g);
+    // ordinary backward pass of the squared-error terms over all rows, with r_l added on the real rows
+    for (int l = L; l > 1; --l) {
+      SgemmArgs g = z;
+      g.M = (int)M; g.N = m.dims[l - 1]; g.K = m.dims[l]; g.A = ws.dz[l - 1]; g.lda = g.K; g.B = m.mW[l - 1]; g.ldb = m.kpad[l - 1];
+      g.C = ws.dz[l - 2]; g.ldc = g.N; g.Y = ws.y[l - 2]; g.X = ws.r[l - 2]; g.x_rows = penalty ? (int)R : 0; g.act = act; g.epi = kEpiDz;
+      sgemm_go<false>(s, g);
+    }
   }
 
   // weight gradients: d_l^T v_{l-1} over the real rows, where there is a penalty, then dz_l^T y_{l-1} over all rows; the bias gradients are the

@@ -65,6 +65,22 @@ def test_discriminator_many_rows_split_reduction(dims):
     _check(disc, ws, bs, real, sim, 10.0, "elu")
 
 
+@pytest.mark.parametrize("act,dims,real_rows,sim_rows", [("elu", [17, 320, 272, 31, 1], 16, 1), ("tanh", [16, 300, 1], 15, 17), ("elu", [48, 16, 1], 33, 0),
+                                                         ("tanh", [9, 130, 64, 50, 1], 1, 47), ("relu", [33, 321, 40, 1], 17, 16), ("elu", [321, 64, 1], 5, 33)])
+def test_discriminator_rows_at_the_edges_of_their_launch(act, dims, real_rows, sim_rows):
+    """Sixteen rows and sixteen columns at a time, up to 320 wide, in the launch that takes a frame through the whole chain: ragged ends of both,
+    reductions that end inside a step, more columns than one pass of the wavefronts, three hidden layers, and the first width of the general route."""
+    from ksim_amd.mlp import MLP
+
+    ws, bs = _params(dims, seed=sum(dims))
+    disc = MLP(ws, bs, activation=act, dtype="f32")
+    disc.train_init()
+    rng = np.random.default_rng(real_rows)
+    real, sim = (rng.normal(size=(n, 1, dims[0])).astype(np.float32) for n in (real_rows, sim_rows))
+    _check(disc, ws, bs, real, sim, 10.0, act)
+    _check(disc, ws, bs, real, sim, 0.0, act)
+
+
 def test_discriminator_update_learns_and_matches_oracle_steps():
     """Three optimiser steps on fixed batches against the oracle's Adam (the optax chain restated for the policy update),
     then the loop with sampled batches: the loss on separable data goes down."""
