@@ -324,21 +324,26 @@ struct LsPoint {
 };
 
 // wave_sum of three or four values side by side: their steps fill each other's waits, and the two last ones leave the rows they do not reach as they
-// are instead of adding a zero to them (a move and an addition each); the same sums.  A substep takes seven such sets: 64 robots 233 -> 228 us per
-// control step, 8192 mixed robots 486 -> 480, 4096 humanoids 329 -> 325.  (A value is read by the DPP step two instructions after it was written.)
+// are instead of adding a zero to them (a move and an addition each).  The first step is the compiler's, as in wave_sum: where a value is a product
+// it goes into that addition unrounded, which a sum that begins in the assembly loses (qacc in the last bits).  A substep takes seven such sets.
+// Against one sum after the other, in turn on one card: control step of 64 robots 231.9 -> 228.4 us, 8192 mixed robots 482 -> 478, 4096 humanoids
+// 328.9 -> 326.8, the same bits (spread of a side 0.1 to 0.4 %).
+// The compiler does not look into the assembly for hazards.  Covered here: a DPP read needs two instructions behind the write of its register (s_nop 1
+// ahead of the first step, the other values' steps between two of its own) and a lane read one behind it (s_nop 0).  Not covered: values that come
+// straight from a matrix instruction, and a vector write of the lane mask (v_cmpx) just ahead.
 #define KS_SUM_STEP(CTRL) "v_add_f32_dpp %0, %0, %0 " CTRL "\n\tv_add_f32_dpp %1, %1, %1 " CTRL "\n\tv_add_f32_dpp %2, %2, %2 " CTRL "\n\t"
 #define KS_SUM_STEP4(CTRL) KS_SUM_STEP(CTRL) "v_add_f32_dpp %3, %3, %3 " CTRL "\n\t"
 #define KS_ROW "row_mask:0xf bank_mask:0xf bound_ctrl:1"
+#define KS_SUM_STEPS(STEP) "s_nop 1\n\t" STEP("row_shr:2 " KS_ROW) STEP("row_shr:4 " KS_ROW) STEP("row_shr:8 " KS_ROW) \
+    STEP("row_bcast:15 row_mask:0xa bank_mask:0xf") STEP("row_bcast:31 row_mask:0xc bank_mask:0xf") "s_nop 0"
 __device__ __forceinline__ void wave_sums(float& x, float& y, float& z) {
-  asm("s_nop 1\n\t" KS_SUM_STEP("row_shr:1 " KS_ROW) KS_SUM_STEP("row_shr:2 " KS_ROW) KS_SUM_STEP("row_shr:4 " KS_ROW)
-      KS_SUM_STEP("row_shr:8 " KS_ROW) KS_SUM_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf") KS_SUM_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
-      "s_nop 0" : "+v"(x), "+v"(y), "+v"(z));
+  x += dpp_shift<0x111, 0xf>(x); y += dpp_shift<0x111, 0xf>(y); z += dpp_shift<0x111, 0xf>(z);
+  asm(KS_SUM_STEPS(KS_SUM_STEP) : "+v"(x), "+v"(y), "+v"(z));
   x = lane_bcast(x, 63); y = lane_bcast(y, 63); z = lane_bcast(z, 63);
 }
 __device__ __forceinline__ void wave_sums(float& x, float& y, float& z, float& w) {
-  asm("s_nop 1\n\t" KS_SUM_STEP4("row_shr:1 " KS_ROW) KS_SUM_STEP4("row_shr:2 " KS_ROW) KS_SUM_STEP4("row_shr:4 " KS_ROW)
-      KS_SUM_STEP4("row_shr:8 " KS_ROW) KS_SUM_STEP4("row_bcast:15 row_mask:0xa bank_mask:0xf") KS_SUM_STEP4("row_bcast:31 row_mask:0xc bank_mask:0xf")
-      "s_nop 0" : "+v"(x), "+v"(y), "+v"(z), "+v"(w));
+  x += dpp_shift<0x111, 0xf>(x); y += dpp_shift<0x111, 0xf>(y); z += dpp_shift<0x111, 0xf>(z); w += dpp_shift<0x111, 0xf>(w);
+  asm(KS_SUM_STEPS(KS_SUM_STEP4) : "+v"(x), "+v"(y), "+v"(z), "+v"(w));
   x = lane_bcast(x, 63); y = lane_bcast(y, 63); z = lane_bcast(z, 63); w = lane_bcast(w, 63);
 }
 

@@ -747,3 +747,27 @@ def test_every_padded_width_of_the_step_kernel(nv, spheres, opts):
         if step in (1, 10):
             for key in ("qpos", "qvel"):
                 compare(buf[key], key, step, ONE_STEP_TOL if step == 1 else TEN_STEP_TOL)
+
+
+def test_centre_of_mass_keeps_the_products_of_its_first_additions():
+    """The sums over the bodies start from products that are not rounded before their first addition: of bodies of 8, 5 and 3 kg the third one's share
+    goes into the second one's by a fused multiply-add.  Every other operation is exact here (frames at the centres of mass, a total of 16 kg, a root
+    within a factor of two of the centre), so the centre follows bit for bit from the body positions."""
+    import dataclasses
+
+    from ksim_amd import physics
+
+    m = tree_model(2, 0)
+    m = dataclasses.replace(m, body_mass=np.array([0.0, 8.0, 5.0, 3.0]), body_ipos=np.zeros((m.nb, 3)))
+    N = 256
+    qpos, qvel = random_states(m, N, seed=3)
+    qpos[:, :3] = np.random.default_rng(4).uniform(3.0, 5.0, (N, 3))
+    buf = dict(qpos=t32(qpos), qvel=t32(qvel), ctrl_in=zeros(N, m.nu), xpos=zeros(N, m.nb * 3), cinert=zeros(N, m.nb * 10))
+    physics.forward(physics.DeviceModel(m), buf)
+    f32, f64 = np.float32, np.float64
+    x = buf["xpos"].cpu().numpy().reshape(N, m.nb, 3)
+    com = x[:, 1] - buf["cinert"].cpu().numpy().reshape(N, m.nb, 10)[:, 1, 6:9] / f32(8)
+    second, third = (f32(5) * x[:, 2]).astype(f64), f64(3) * x[:, 3].astype(f64)  # the latter exact in 64 bits
+    fused, rounded = (((second + t).astype(f32) + f32(8) * x[:, 1]) / f32(16) for t in (third, third.astype(f32).astype(f64)))
+    assert (fused != rounded).mean() > 0.05  # the two differ on these states
+    assert np.array_equal(com, fused)
