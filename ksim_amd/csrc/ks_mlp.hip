@@ -3448,9 +3448,13 @@ __device__ __forceinline__ f32x4 disc_product(const float* __restrict__ op, cons
       } else if (k0 + 16 <= K) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[4 * s + e] = (W + (int64_t)(k0 + e) * ld)[own];
-      } else {  // the reduction ends inside the step: rows past it repeat the last one, the operand is zero there
+      } else {  // the reduction ends inside the step: zeros past it, as the operand's (a repeated row that holds an infinity would make them NaN)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[4 * s + e] = W[(int64_t)min(k0 + 4 * h + e, K - 1) * ld + j];
+        for (int e = 0; e < 4; ++e) {
+          const int k = k0 + 4 * h + e;
+          const float x = W[(int64_t)min(k, K - 1) * ld + j];
+          t[4 * s + e] = k < K ? x : 0.f;
+        }
       }
     }
   };

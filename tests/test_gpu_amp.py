@@ -81,6 +81,27 @@ def test_discriminator_rows_at_the_edges_of_their_launch(act, dims, real_rows, s
     _check(disc, ws, bs, real, sim, 0.0, act)
 
 
+def test_discriminator_reduction_tail_leaves_infinite_weights_alone():
+    """A reduction over 20 units is padded to 32: an infinite weight in its last row reaches the gradients as the infinity it is (every other
+    factor is positive and finite), not as the NaN of an infinity times a padding zero."""
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(4)
+    dims = [4, 20, 20, 1]
+    ws = [rng.uniform(0.1, 1.0, size=(o, i)).astype(np.float32) for i, o in zip(dims[:-1], dims[1:])]
+    bs = [np.zeros(o, dtype=np.float32) for o in dims[1:]]
+    ws[1][19, 7] = np.inf
+    disc = MLP(ws, bs, activation="relu", dtype="f32")
+    disc.train_init()
+    x = rng.uniform(0.1, 1.0, size=(1, 5, 4)).astype(np.float32)
+    disc.disc_loss_grad(torch.tensor(x, device=DEV), torch.tensor(x + 1.0, device=DEV), 0.0)
+    tw, tb = ([torch.tensor(p, dtype=torch.float64, requires_grad=True) for p in params] for params in (ws, bs))
+    sum(0.5 * ((oup.mlp(torch.tensor(f, dtype=torch.float64), tw, tb, "relu") - t) ** 2).sum() for f, t in ((x, 1.0), (x + 1.0, -1.0))).backward()
+    for (got, _), want in zip(disc.parameters(gradients=True), tw):
+        assert torch.isposinf(want.grad).all()
+        assert torch.isposinf(got).all()
+
+
 def test_discriminator_update_learns_and_matches_oracle_steps():
     """Three optimiser steps on fixed batches against the oracle's Adam (the optax chain restated for the policy update),
     then the loop with sampled batches: the loss on separable data goes down."""
