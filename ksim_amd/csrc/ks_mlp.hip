@@ -3883,17 +3883,26 @@ struct DiscWs {
 
 static int64_t disc_penalty_tiles(const DevMlp& m, int64_t R) { return ((R + 31) / 32) * ((m.dims[0] + 31) / 32); }
 
-// Floats of a row in disc_rows_kernel's LDS, 0 where the launches per product are to run: a linear network has no chain, and three operands of 16
-// rows in the 64 KiB that a launch has without asking end at 320 columns.  Layers narrower than 128 leave wavefronts of the chain idle, which
-// counts once the rows fill the chip many times over (40-48-1: 53 -> 36 us at 6144 rows, 93 -> 82 at 24576, but 535 -> 600 at 262144).
-static int disc_rows_lda(const DevMlp& m, int64_t M) {
-  int w = 0;
+// Floats of a row in disc_rows_kernel's LDS, 0 where the launches per product are to run: a linear network has no chain, and of networks wider than
+// 320 only a few fit three operands of 16 rows into the 64 KiB that a launch has without asking (336 would; 320 is what was measured).  A second pass of the
+// wavefronts over 257 columns and more costs less than the products' launches (71-272-272-1, launches -> chain, 2 x 32 / 1024 / 131072 frames: 88 -> 78,
+// 127 -> 95, 8009 -> 5459 us; 71-320-320-1 93 -> 86, 150 -> 109, 9288 -> 5630).
+// A hidden layer occupies a wavefront per 16 of its columns; where that leaves most of the sixteen idle, the launches per product win once the rows
+// fill the chip, the sooner the narrower the widest hidden layer is and the fewer products there are, whatever the input's width.  Time of the chain over
+// that of the launches at M rows in all, 20, 71 and 300 inputs, one and two hidden layers, with the penalty | without:
+//   16 and 32 wide: M = 8192 0.56 to 0.70 | 0.68 to 0.91, 16384 0.80 to 0.90 | 0.92 to 1.16, 24576 0.89 to 1.01 | 1.11 to 1.18, 262144 1.16 to 1.53 | 1.41 to 1.74
+//   48 wide: 16384 0.71 to 0.85 | 0.83 to 0.99, 65536 0.83 to 0.98 | one layer 1.02 to 1.09, two 0.90 to 0.98, 262144 0.89 to 1.08 | 0.97 to 1.16
+//   64 wide, one layer: 16384 0.76 to 0.84 | 0.91 to 0.97, 65536 0.84 to 0.97 | 0.99 to 1.07, 262144 0.87 to 1.10 | 1.04 to 1.13
+//   64 wide, two layers: 0.42 to 0.92 | 0.49 to 1.00 up to 262144 rows; 80 wide and wider 0.48 to 0.95 | 0.53 to 1.01
+static int disc_rows_lda(const DevMlp& m, int64_t M, bool penalty) {
+  int w = 0, hidden = 0;
   for (int l = 0; l < m.n_layers; ++l) {
-    const int r = round_up(m.dims[l], 16);
-    if (m.kpad[l] < r || m.kpad[l] % 4) return 0;
-    w = r > w ? r : w;
+    w = std::max(w, round_up(m.dims[l], 16));
+    if (l > 0) hidden = std::max(hidden, m.dims[l]);
   }
-  return m.n_layers > 1 && w <= 320 && (w >= 128 || M <= 65536) ? w + 4 : 0;
+  const bool deep = m.n_layers > 2;
+  const int64_t most = hidden > 64 || (hidden > 48 && deep) ? M : hidden > 32 ? (penalty || deep ? 65536 : 16384) : (penalty ? 24576 : 8192);
+  return m.n_layers > 1 && w <= 320 && M <= most ? w + 4 : 0;
 }
 
 static int64_t carve_disc(const DevMlp& m, int64_t R, int64_t M, char* base, DiscWs* ws) {
@@ -4016,7 +4025,7 @@ extern "C" int ks_mlp_disc_loss_grad(KsMlp* h, ks_stream_t stream, int64_t n_rea
   SgemmArgs z = {};  // fields left out below are zero
   DiscLosses losses_of = {R, M, 0, ws.dz[L - 1], ws.sums, penalty ? 0.5 * (double)grad_penalty_coef * (double)(1.f / (float)n_motions) : 0.0, losses};
   const float penalty_scale = penalty ? grad_penalty_coef * (1.f / (float)n_motions) : 0.f;
-  const int lda = disc_rows_lda(m, M);
+  const int lda = disc_rows_lda(m, M, penalty);
   if (lda) {
     DiscRowsArgs a;
     std::memset(&a, 0, sizeof(a));

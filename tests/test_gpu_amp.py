@@ -81,6 +81,22 @@ def test_discriminator_rows_at_the_edges_of_their_launch(act, dims, real_rows, s
     _check(disc, ws, bs, real, sim, 0.0, act)
 
 
+@pytest.mark.parametrize("dims,limit,coef", [([12, 32, 16, 1], 24576, 10.0), ([140, 32, 1], 8192, 0.0), ([40, 33, 1], 65536, 10.0),
+                                             ([9, 64, 1], 16384, 0.0), ([9, 40, 48, 1], 65536, 0.0), ([9, 49, 20, 1], 65536, 10.0), ([9, 65, 1], 16384, 0.0)])
+def test_discriminator_on_both_sides_of_the_row_limits(dims, limit, coef):
+    """Narrow hidden layers change from one launch for the whole chain to a launch per product where the rows fill the chip: the last row count of the one
+    and the first of the other, and the narrowest networks that never change.  Sums of up to 65537 rows in fp32 slices of a few hundred: far inside the file's tolerance."""
+    from ksim_amd.mlp import MLP
+
+    ws, bs = _params(dims, seed=sum(dims))
+    disc = MLP(ws, bs, activation="elu", dtype="f32")
+    disc.train_init()
+    rng = np.random.default_rng(limit)
+    for rows in (limit, limit + 1):
+        real, sim = (rng.normal(size=(n, 1, dims[0])).astype(np.float32) for n in (rows // 3, rows - rows // 3))
+        _check(disc, ws, bs, real, sim, coef, "elu")
+
+
 def test_discriminator_reduction_tail_leaves_infinite_weights_alone():
     """A reduction over 20 units is padded to 32: an infinite weight in its last row reaches the gradients as the infinity it is (every other
     factor is positive and finite), not as the NaN of an infinity times a padding zero."""
