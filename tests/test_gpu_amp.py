@@ -81,6 +81,22 @@ def test_discriminator_rows_at_the_edges_of_their_launch(act, dims, real_rows, s
     _check(disc, ws, bs, real, sim, 0.0, act)
 
 
+@pytest.mark.parametrize("act", ["elu", "tanh"])
+@pytest.mark.parametrize("dims,rows", [([33, 321, 40, 1], (17, 16)), ([20, 64, 330, 17, 1], (33, 40)), ([324, 32, 70, 33, 1], (3, 65))])
+def test_discriminator_chain_of_launches(act, dims, rows):
+    """A launch per product (a layer or the input over 320 wide): hidden chains whose second derivative counts, so that what one hidden layer's launch leaves
+    for the penalty's sweep back (W^T d and d itself) reaches the next one's gradient.  Rows and widths around the 32 x 32 tiles."""
+    from ksim_amd.mlp import MLP
+
+    ws, bs = _params(dims, seed=sum(dims))
+    disc = MLP(ws, bs, activation=act, dtype="f32")
+    disc.train_init()
+    rng = np.random.default_rng(rows[0])
+    real, sim = (rng.normal(size=(n, 1, dims[0])).astype(np.float32) for n in rows)
+    assert _check(disc, ws, bs, real, sim, 10.0, act)[2] > 1e-3
+    _check(disc, ws, bs, real, sim, 0.0, act)
+
+
 @pytest.mark.parametrize("dims,limit,coef", [([12, 32, 16, 1], 24576, 10.0), ([140, 32, 1], 8192, 0.0), ([40, 33, 1], 65536, 10.0),
                                              ([9, 64, 1], 16384, 0.0), ([9, 40, 48, 1], 65536, 0.0), ([9, 49, 20, 1], 65536, 10.0), ([9, 65, 1], 16384, 0.0)])
 def test_discriminator_on_both_sides_of_the_row_limits(dims, limit, coef):
@@ -193,7 +209,7 @@ def test_discriminator_argument_errors():
 @pytest.mark.parametrize("dims,shapes", [((5, 33, 1), ((1, 1), (2, 3))), ((71, 128, 96, 1), ((3, 11), (1, 33))), ((64, 32, 1), ((4, 8), (0, 1))),
                                          ((64, 32, 1), ((0, 1), (4, 8))), ((40, 256, 64, 1), ((2, 700), (3, 1000)))])
 def test_discriminator_gradient_at_the_edges_of_its_tiles(dims, shapes):
-    """Rows and widths around the 32 x 32 tiles and the 32-step chunks of the products, frames that are not 16-byte rows, either set
+    """Rows and widths around the 32 x 32 tiles and the 32-step chunks of the weight gradients, frames that are not 16-byte rows, either set
     of motions empty, and row counts that cut the weight gradients into slices.  fp32 against float64 autograd: sums of up to 4400
     rows, each rounded at 2^-24 of its size."""
     from ksim_amd.mlp import random_mlp
