@@ -113,6 +113,33 @@ def test_discriminator_on_both_sides_of_the_row_limits(dims, limit, coef):
         _check(disc, ws, bs, real, sim, coef, "elu")
 
 
+def test_discriminator_products_are_as_precise_as_four_partial_sums():
+    """A product over 256 columns in the launch for a frame's whole chain is no further from 64 bits than the launches per product, whose four wavefronts
+    sum a quarter of the reduction each (here restated in numpy: fused multiply-adds in fp32, then the four sums).  With output weights of zero
+    the one real frame's error is -1 and the simulated frame of zeros leaves nothing, so the output weights' gradient is minus the hidden layer, bit for bit."""
+    from ksim_amd.mlp import MLP
+
+    K, got, four = 256, [], []
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        w, x = (rng.normal(size=s).astype(np.float32) for s in ((K, K), K))
+        disc = MLP([w, np.zeros((1, K), np.float32)], [np.zeros(K, np.float32), np.zeros(1, np.float32)], activation="relu", dtype="f32")
+        disc.train_init()
+        disc.disc_loss_grad(torch.tensor(x, device=DEV).reshape(1, 1, K), torch.zeros(1, 1, K, device=DEV), 0.0)
+        y = -disc.parameters(gradients=True)[1][0].double().cpu().numpy().ravel()
+        exact = w.astype(np.float64) @ x.astype(np.float64)
+        sums = np.zeros((4, K), np.float32)
+        for k in range(K // 4):
+            for q in range(4):
+                sums[q] = (sums[q] + w[:, q * K // 4 + k].astype(np.float64) * x[q * K // 4 + k]).astype(np.float32)
+        total = ((sums[0] + sums[1]) + sums[2]) + sums[3]
+        scale = np.linalg.norm(np.maximum(exact, 0))
+        got.append((y - np.maximum(exact, 0)) / scale)
+        four.append((np.maximum(total, 0) - np.maximum(exact, 0)) / scale)
+    # 1000 entries' root mean square: its own spread is 2 %, two long sums would be 1.35 times the bound and the present ones are 0.65 of it
+    assert np.linalg.norm(got) <= np.linalg.norm(four)
+
+
 def test_discriminator_reduction_tail_leaves_infinite_weights_alone():
     """A reduction over 20 units is padded to 32: an infinite weight in its last row reaches the gradients as the infinity it is (every other
     factor is positive and finite), not as the NaN of an infinity times a padding zero."""
