@@ -134,7 +134,8 @@ __device__ __forceinline__ void load_row(const float* p, float (&v)[NP]) {
 // two go to one MFMA as both operands, -l l^T, one in each lane half (the instruction's two k), which updates every entry right of and below
 // them at once; row j + 1, already up to date, is left out of the left operand.  The instruction holds a SIMD's vector issue for 64 cycles
 // whether its second k is used or not (fp32 MFMAs and vector instructions take turns), and with one column per step that was a fifth of the
-// kernel: 8192 mixed robots 507 -> 474 us per control step, 4096 humanoids 356 -> 338.
+// kernel: 8192 mixed robots 507 -> 474 us per control step, 4096 humanoids 356 -> 338.  (Here and below the two figures of a pair are from one
+// card in turn; cards differ by up to 4 %, so pairs do not continue one another.)
 // Column j below the diagonal is left as it was when the pivot was reached
 // (L[k][j] * L[j][j]) and row j right of the diagonal holds L[k][j]: read down a lane, that is row c of L to the
 // left of the diagonal and the scaled column c below it, exactly what the column-oriented substitutions take,

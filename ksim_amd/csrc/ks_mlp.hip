@@ -3413,8 +3413,8 @@ __global__ __launch_bounds__(1024) void disc_wgrad_kernel(SgemmGroup t, DiscLoss
 // (y, a, r) are read by the thread that wrote them.
 // Few frames are bound by the chain of products itself (63 us for 2 x 1024 frames of 71-256-256-1, of which the matrix instructions are 17), where
 // a launch per product (sgemm_kernel) added a launch, its gap and a trip of the operands through memory to each.  The whole gradient of
-// 71-256-256-1, launches per product -> this: 2 x 32 frames 77 -> 65 us, 2 x 1024 100 -> 79, 2 x 12288 537 -> 381, 2 x 131072 5560 -> 3980;
-// 71-128-128-1 65 -> 35, 71 -> 44, 241 -> 178, 2290 -> 1870; 60-256-1 43 -> 24, 51 -> 31, 194 -> 111, 1900 -> 1110.
+// 71-256-256-1, launches per product -> this: 2 x 32 frames 78 -> 66 us, 2 x 1024 101 -> 81, 2 x 12288 538 -> 382, 2 x 131072 5575 -> 3982;
+// 71-128-128-1 67 -> 36, 73 -> 46, 243 -> 181, 2298 -> 1897; 60-256-1 44 -> 24, 50 -> 31, 194 -> 112, 1907 -> 1130.
 // Requesting a product's first weights before the stores of the one before it was slower (63 -> 68 us).
 struct DiscRowsArgs {
   int L, act, penalty, lda, zeros, tiles_real;
@@ -3891,14 +3891,16 @@ static int64_t disc_penalty_tiles(const DevMlp& m, int64_t R) { return ((R + 31)
 // Floats of a row in disc_rows_kernel's LDS, 0 where the launches per product are to run: a linear network has no chain, and of networks wider than
 // 320 only a few fit three operands of 16 rows into the 64 KiB that a launch has without asking (336 would; 320 is what was measured).  A second pass of the
 // wavefronts over 257 columns and more costs less than the products' launches (71-272-272-1, launches -> chain, 2 x 32 / 1024 / 131072 frames: 88 -> 78,
-// 127 -> 95, 8009 -> 5459 us; 71-320-320-1 93 -> 86, 150 -> 109, 9288 -> 5630).
+// 127 -> 95, 8079 -> 5548 us; 71-320-320-1 93 -> 86, 150 -> 109, 9285 -> 5612).
 // A hidden layer occupies a wavefront per 16 of its columns; where that leaves most of the sixteen idle, the launches per product win once the rows
 // fill the chip, the sooner the narrower the widest hidden layer is and the fewer products there are, whatever the input's width.  Time of the chain over
 // that of the launches at M rows in all, 20, 71 and 300 inputs, one and two hidden layers, with the penalty | without:
 //   16 and 32 wide: M = 8192 0.56 to 0.70 | 0.68 to 0.91, 16384 0.80 to 0.90 | 0.92 to 1.16, 24576 0.89 to 1.01 | 1.11 to 1.18, 262144 1.16 to 1.53 | 1.41 to 1.74
 //   48 wide: 16384 0.71 to 0.85 | 0.83 to 0.99, 65536 0.83 to 0.98 | one layer 1.02 to 1.09, two 0.90 to 0.98, 262144 0.89 to 1.08 | 0.97 to 1.16
 //   64 wide, one layer: 16384 0.76 to 0.84 | 0.91 to 0.97, 65536 0.84 to 0.97 | 0.99 to 1.07, 262144 0.87 to 1.10 | 1.04 to 1.13
-//   64 wide, two layers: 0.42 to 0.92 | 0.49 to 1.00 up to 262144 rows; 80 wide and wider 0.48 to 0.95 | 0.53 to 1.01
+//   64 wide, two layers: 0.42 to 0.96 | 0.49 to 1.00 up to 262144 rows; 80 wide and wider 0.48 to 0.96 | 0.53 to 1.01
+// (before a product's sums were folded every 64 columns, which adds up to 0.03 to the narrow ones: 20-65-1 at 262144 1.03 | 0.92, 20-16-1 at
+// 24576 1.03, the others at the last rows of the rule below 0.79 to 1.00).
 static int disc_rows_lda(const DevMlp& m, int64_t M, bool penalty) {
   int w = 0, hidden = 0;
   for (int l = 0; l < m.n_layers; ++l) {
