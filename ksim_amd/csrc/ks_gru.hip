@@ -197,6 +197,22 @@ __device__ __forceinline__ float seq_tanh(float x) { return 1.f - 2.f * __builti
 // ahead for the next step) before every barrier, a memory round trip per step of the sequence.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// The LSTM forward kernel's way in and out of memory: a step's inputs are requested a step ahead of their use and its results leave behind it, one
+// load or store (KS_SEQ_SIDE, a single instruction from a uniform address) after every eight matrix instructions.  All together at a step's
+// end they held the CU's wavefronts up at once, and a store or load under a condition makes the compiler wait for the step's stores before the
+// next step: loads and stores are counted together and waited for in order.  Hence no conditions (the outputs that a launch has are template
+// arguments, rows past the batch repeat the last row and store its values once more, the last step requests its own inputs again) and nothing
+// pending where the loop is entered.  2 x 1024 rows x 100 steps with kept activations: 394 -> 366 us; without them 380 -> 363; a rollout's control
+// step of 4096 envs (T = 1, several sets of rows per workgroup) 437 -> 424.  What is left is issue and power: 2048 of 3500 cycles of a step are
+// matrix instructions, at 2.0 to 2.2 GHz.  The backward kernel (342 -> 361 us) and the GRU's (31 us either way) did not gain from the same order.
+__device__ __forceinline__ void seq_loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+#define KS_SEQ_SIDE(OP)                \
+  {                                    \
+    __builtin_amdgcn_sched_barrier(0); \
+    OP;                                \
+    __builtin_amdgcn_sched_barrier(0); \
+  }
+
 // where hidden unit u of a row sits in the LDS copy of the state: unit u = 16 q + b is register q of block b (see the forward
 // kernel), and a lane reads its block's 8 registers as 8 consecutive floats
 __device__ __forceinline__ int seq_slot(int u) { return 8 * (u & 15) + (u >> 4); }
@@ -234,6 +250,7 @@ __device__ __forceinline__ float rows_reduce_scatter(float v0, float v1, float v
   return lo + hi;
 }
 
+template <bool CELL, bool SAVE>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
   constexpr int H = kSeqH;
@@ -268,32 +285,33 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
   for (int grp = 0; grp < groups; ++grp) {
   const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * kSeqRows;
   if (r0 >= M) break;  // the same for every thread of the workgroup
-  const int64_t m = r0 + j;
-  const bool row_ok = m < M;
-  const int64_t mc = row_ok ? m : M - 1;  // loads of the rows past the batch are clamped, their stores dropped
+  const unsigned jr = r0 + j < M ? j : (unsigned)(M - 1 - r0);
+  const int64_t m = r0 + jr;
   if (grp > 0) __syncthreads();  // the previous set's last read of the state buffers is over
-  float c = c0[mc * H + unit];
-  float hprev = h0[mc * H + unit];  // the state this lane's (unit, row) enters the step with
+  float c = c0[m * H + unit];
+  float hprev = h0[m * H + unit];  // the state this lane's (unit, row) enters the step with
   sh[0][j][seq_slot(unit)] = hprev;
-  __syncthreads();
-  int cur = 0;
-  // the step's inputs from memory are fetched one step ahead: their latency would otherwise stand between the matrix work and the gates
-  float gnext[4];
-  uint8_t fnext = 0;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) gnext[g] = gi[mc * 4 * H + g * H + unit];
-  if (fresh) fnext = fresh[mc];
-  for (int t = 0; t < T; ++t) {
-    float gin[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) gin[g] = gnext[g];
-    const bool f = fnext != 0;
-    if (t + 1 < T) {
-      const int64_t tn = (int64_t)(t + 1) * M + mc;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) gnext[g] = gi[tn * 4 * H + g * H + unit];
-      if (fresh) fnext = fresh[tn];
+  struct In { float g[4]; unsigned f; } in0 = {}, in1 = {};
+  float si = 0.f, sf = 0.f, tg = 0.f, so = 0.f, tc = 0.f, cp = 0.f, hu = 0.f;
+  auto load = [&](int t, In& in, int k) __attribute__((always_inline)) {
+    const int64_t o = (int64_t)(t < T ? t : T - 1) * M + r0;
+    if (k < 4) in.g[k] = (gi + (o * 4 + k) * H)[jr * 4 * H + unit];
+    else if (fresh) in.f = (fresh + o)[jr];
+  };
+  auto store = [&](int t, int k) __attribute__((always_inline)) {
+    const int64_t o = (int64_t)t * M + r0;
+    if (k == 0) (hs + o * H)[jr * H + unit] = hprev;
+    if (CELL && k == 1) (cs + o * H)[jr * H + unit] = c;
+    if (SAVE && k >= 2) {
+      const float v[7] = {si, sf, tg, so, tc, cp, hu};
+      (saved + (o * 7 + k - 2) * H)[jr * 7 * H + unit] = v[k - 2];
     }
+  };
+#pragma unroll
+  for (int k = 0; k < 5; ++k) load(0, in0, k);
+  seq_loads_done();
+  __syncthreads();
+  auto step = [&](int t, auto cur, bool first, const In& in, In& next) __attribute__((always_inline)) {
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
     float ha[8];
     {
@@ -305,40 +323,45 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
 #define KS_SEQ_MFMA(K0)                                                                                            \
     acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[(K0) >> 4], wa[(K0)], acc0, 4, (K0) & 15, 0);                       \
     acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[((K0) + 1) >> 4], wa[(K0) + 1], acc1, 4, ((K0) + 1) & 15, 0);
-#define KS_SEQ_MFMA8(K0) KS_SEQ_MFMA(K0) KS_SEQ_MFMA((K0) + 2) KS_SEQ_MFMA((K0) + 4) KS_SEQ_MFMA((K0) + 6)
-#define KS_SEQ_MFMA32(K0) KS_SEQ_MFMA8(K0) KS_SEQ_MFMA8((K0) + 8) KS_SEQ_MFMA8((K0) + 16) KS_SEQ_MFMA8((K0) + 24)
-    KS_SEQ_MFMA32(0) KS_SEQ_MFMA32(32) KS_SEQ_MFMA32(64) KS_SEQ_MFMA32(96)
-#undef KS_SEQ_MFMA32
+#define KS_SEQ_MFMA8(N, OP) KS_SEQ_MFMA(8 * N) KS_SEQ_MFMA(8 * N + 2) KS_SEQ_MFMA(8 * N + 4) KS_SEQ_MFMA(8 * N + 6) KS_SEQ_SIDE(OP)
+#define KS_SEQ_OUT(N) KS_SEQ_MFMA8(N, if (!first) store(t - 1, N))
+#define KS_SEQ_IN(N) KS_SEQ_MFMA8(N, load(t + 1, next, 13 - N))
+    KS_SEQ_OUT(0) KS_SEQ_OUT(1) KS_SEQ_OUT(2) KS_SEQ_OUT(3) KS_SEQ_OUT(4) KS_SEQ_OUT(5) KS_SEQ_OUT(6) KS_SEQ_OUT(7) KS_SEQ_OUT(8)
+    KS_SEQ_IN(9) KS_SEQ_IN(10) KS_SEQ_IN(11) KS_SEQ_IN(12) KS_SEQ_IN(13) KS_SEQ_MFMA8(14, ) KS_SEQ_MFMA8(15, )
+#undef KS_SEQ_IN
+#undef KS_SEQ_OUT
 #undef KS_SEQ_MFMA8
 #undef KS_SEQ_MFMA
     // lane (unit, gate lane % 4) now holds that gate for the four rows in its four registers; the gates want the transpose
     // within each group of four lanes: lane (unit, row j) with the four gates
     float pre[4];
     quad_transpose(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3], j, pre);
-    const float cp = f ? 0.f : c, hu = f ? 0.f : hprev;
+    const bool f = in.f != 0;
+    cp = f ? 0.f : c;
+    hu = f ? 0.f : hprev;
     // the hardware exponential and reciprocal (about 1 ulp each) instead of the library's expf, tanhf and IEEE division: a
     // fifth of the instructions, and the gates are as many instructions per step as the matrix work is cycles
-    const float si = seq_sigmoid(gin[0] + (f ? 0.f : pre[0]));
-    const float sf = seq_sigmoid(gin[1] + (f ? 0.f : pre[1]));
-    const float tg = seq_tanh(gin[2] + (f ? 0.f : pre[2]));
-    const float so = seq_sigmoid(gin[3] + (f ? 0.f : pre[3]));
+    si = seq_sigmoid(in.g[0] + (f ? 0.f : pre[0]));
+    sf = seq_sigmoid(in.g[1] + (f ? 0.f : pre[1]));
+    tg = seq_tanh(in.g[2] + (f ? 0.f : pre[2]));
+    so = seq_sigmoid(in.g[3] + (f ? 0.f : pre[3]));
     c = sf * cp + si * tg;
-    const float tc = seq_tanh(c);
-    const float hn = so * tc;
-    hprev = hn;
-    sh[cur ^ 1][j][seq_slot(unit)] = hn;
-    if (row_ok) {
-      const int64_t o = (int64_t)t * M + m;
-      hs[o * H + unit] = hn;
-      if (cs) cs[o * H + unit] = c;
-      if (saved) {
-        float* sv = saved + o * 7 * H + unit;
-        sv[0] = si; sv[H] = sf; sv[2 * H] = tg; sv[3 * H] = so; sv[4 * H] = tc; sv[5 * H] = cp; sv[6 * H] = hu;
-      }
-    }
+    tc = seq_tanh(c);
+    hprev = so * tc;
+    sh[cur ^ 1][j][seq_slot(unit)] = hprev;
     lds_barrier();  // the new hidden state is complete; the buffer just read is free for the step after next
-    cur ^= 1;
+  };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  step(0, even, true, in0, in1);
+  int t = 1;
+  for (; t + 1 < T; t += 2) {
+    step(t, odd, false, in1, in0);
+    step(t + 1, even, false, in0, in1);
   }
+  if (t < T) step(t, odd, false, in1, in0);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) store(T - 1, k);
   }
 }
 
@@ -1056,8 +1079,19 @@ extern "C" int ks_lstm_sequences_forward(ks_stream_t stream, int32_t n, int64_t 
   };
   return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) {
     const int groups = seq_groups(T, sets);
-    hipLaunchKernelGGL(lstm_seq_forward_kernel, dim3((unsigned)((sets + groups - 1) / groups), (unsigned)count), dim3(64 * kSeqWaves), 0,
-                       (hipStream_t)stream, (int)T, groups, s[0], s[1]);
+    const dim3 grid((unsigned)((sets + groups - 1) / groups), (unsigned)count);
+    auto run = [&](dim3 grid, const Seq& first, const Seq& second) {
+      const bool cell = first.out1 != nullptr, save = first.saved != nullptr;
+      hipLaunchKernelGGL(cell ? (save ? lstm_seq_forward_kernel<true, true> : lstm_seq_forward_kernel<true, false>)
+                              : (save ? lstm_seq_forward_kernel<false, true> : lstm_seq_forward_kernel<false, false>),
+                         grid, dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, groups, first, second);
+    };
+    if (count == 2 && (!s[0].out1 != !s[1].out1 || !s[0].saved != !s[1].saved)) {  // a kernel writes the same outputs for both of its layers
+      run(dim3(grid.x), s[0], s[0]);
+      run(dim3(grid.x), s[1], s[1]);
+    } else {
+      run(grid, s[0], s[1]);
+    }
   });
 }
 

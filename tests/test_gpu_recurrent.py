@@ -471,3 +471,32 @@ def test_two_layers_in_one_launch_match_one_by_one(kind, dtype, rows, steps):
     run_sequences(backward)
     for k, (a, b) in enumerate(want):
         assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("rows,steps", [((5, 6), 1), ((1, 37), 2), ((45, 4), 3), ((7, 2), 4)])
+def test_lstm_sequences_write_the_outputs_they_are_given_and_no_others(rows, steps):
+    """Cell states and saved activations are optional, and each combination is a kernel of its own: states bit for bit those of the call
+    that writes everything, for two layers of one call whose outputs differ, with ragged sets of 4 rows and odd and even step counts."""
+    from ksim_amd.recurrent import LSTMCell, run_sequences
+
+    H = 128
+    rng = np.random.default_rng(71 + steps)
+    t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    layers = []
+    for M in rows:
+        cell = LSTMCell(*(rng.normal(scale=H ** -0.5, size=s) for s in ((4 * H, H), (4 * H, H), (4 * H,))), dtype="f32")
+        x, h0, c0 = t(steps, M, H), t(M, H), t(M, H)
+        fresh = torch.from_numpy((rng.random((steps, M)) < 0.2).astype(np.uint8)).cuda()
+        want = [torch.full((steps, M, n * H), 3.0, device="cuda") for n in (1, 1, 7)]
+        cell.sequence_forward(x, h0, c0, fresh, *want)
+        layers.append((cell, (x, h0, c0, fresh), want))
+    kinds = [(cs, sv) for cs in (False, True) for sv in (False, True)]
+    for k, first in enumerate(kinds):
+        calls, pairs = [], []
+        for (cell, given, want), (cs, sv) in zip(layers, (first, kinds[(k + 1) % 4])):
+            got = [torch.full_like(w, 5.0) if on else None for w, on in zip(want, (True, cs, sv))]
+            calls.append(cell.sequence_call(*given, *got))
+            pairs += [(g, w) for g, w in zip(got, want) if g is not None]
+        run_sequences(calls)
+        for g, w in pairs:
+            assert torch.equal(g, w), (k, tuple(w.shape))
