@@ -721,7 +721,7 @@ int ks_mlp_forward(const KsMlp* mlp, ks_stream_t stream, int64_t M, const float*
 /* Two networks over the same M rows, e.g. the actor on the noisy observations and the critic on the clean ones
  * (ksim/task/rl.py:892-926 and the value call of examples/walking.py:626-638, which XLA schedules side by side).  Same
  * results as two ks_mlp_forward calls; when both networks run as whole-network kernels with one activation and M is
- * below 16384 they share a single launch, so the second network's workgroups overlap the first one's. */
+ * below 16384, or are single bf16 layers that take the same row tile, they share a single launch, so the second network's workgroups overlap the first one's. */
 int ks_mlp_forward_pair(const KsMlp* mlp0, const KsMlp* mlp1, ks_stream_t stream, int64_t M, const float* x0,
                         float* y0, const float* x1, float* y1, void* workspace0, void* workspace1);
 
@@ -797,6 +797,18 @@ int ks_mlp_train_backward_dx(KsMlp* mlp, ks_stream_t stream, int64_t M, const fl
                              void* workspace);
 /* The weight and bias gradient of a network of one layer from input rows that lie ldx floats apart (ldx >= in). */
 int ks_mlp_layer_weight_grad(KsMlp* mlp, ks_stream_t stream, int64_t M, const float* x, int64_t ldx, const float* dy, void* workspace);
+/* The backward pass of several networks of one layer, e.g. the projections of a recurrent actor and critic: same results as
+ * ks_mlp_train_backward_dx and ks_mlp_layer_weight_grad one by one, in fewer launches.  No two of them may write the same gradient. */
+typedef struct KsLayerBackward {
+  KsMlp* mlp;
+  int64_t M;
+  const float* x;  /* (M, in) rows ldx floats apart; NULL: no weight and bias gradient */
+  int64_t ldx;
+  const float* dy; /* (M, out) */
+  float* dx;       /* (M, in) out; NULL: no input gradient */
+} KsLayerBackward;
+int64_t ks_mlps_layer_backward_workspace_bytes(int32_t n, const KsLayerBackward* layers /*host*/);
+int ks_mlps_layer_backward(int32_t n, const KsLayerBackward* layers /*host*/, ks_stream_t stream, void* workspace);
 /* The first `count` bias entries of a layer are constants: the optimiser and the gradient norm skip them. */
 int ks_mlp_freeze_bias_prefix(KsMlp* mlp, int32_t layer, int32_t count);
 

@@ -184,6 +184,10 @@ class KsLstmDesc(ctypes.Structure):
                 ("weight_hh", c_void_p), ("bias", c_void_p)]
 
 
+class KsLayerBackward(ctypes.Structure):
+    _fields_ = [("mlp", c_void_p), ("M", c_int64), ("x", c_void_p), ("ldx", c_int64), ("dy", c_void_p), ("dx", c_void_p)]
+
+
 class KsSequence(ctypes.Structure):
     _fields_ = [("cell", c_void_p), ("M", c_int64)] + [(n, c_void_p) for n in ("in_", "h0", "c0", "fresh", "saved", "out0", "out1", "dh0", "dc0")]
 
@@ -249,6 +253,10 @@ def bind(lib) -> None:
     lib.ks_mlp_train_backward.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_layer_weight_grad.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p]
     lib.ks_mlp_layer_weight_grad.restype = c_int32
+    lib.ks_mlps_layer_backward_workspace_bytes.argtypes = [c_int32, POINTER(KsLayerBackward)]
+    lib.ks_mlps_layer_backward_workspace_bytes.restype = c_int64
+    lib.ks_mlps_layer_backward.argtypes = [c_int32, POINTER(KsLayerBackward), c_void_p, c_void_p]
+    lib.ks_mlps_layer_backward.restype = c_int32
     lib.ks_grad_sqnorm.argtypes = [c_void_p, c_int64, c_void_p, c_void_p]
     lib.ks_mlp_train_backward_dx.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
                                              c_void_p, c_void_p]

@@ -1078,6 +1078,15 @@ void mlp_fused_pair_kernel(const FusedArgs a, const FusedArgs b) {
   else mlp_fused_body<ACT, T, BM>(b, tile);
 }
 
+// Two single bf16 layers, e.g. the actor's and the critic's projection of one depth, or the input gradients of both: a few thousand rows of one
+// fill the chip for less time than a launch costs (12288 x 128 -> 384: 9.7 us each one after the other, 14.2 both).
+template <int BM>
+__global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(BM <= 64 ? 4 : 2, BM <= 64 ? 4 : 2)))
+void mlp_single_pair_kernel(const FusedArgs a, const FusedArgs b, unsigned tiles_a) {
+  if (blockIdx.x < tiles_a) mlp_fused_body<KS_ACT_NONE, __bf16, BM, true>(a, blockIdx.x);
+  else mlp_fused_body<KS_ACT_NONE, __bf16, BM, true>(b, blockIdx.x - tiles_a);
+}
+
 // ---------------------------------------------------------------- few rows through a wide bf16 network
 // Over a few row tiles the whole-network kernel is bound by how fast a CU takes in weights (66 GB/s whatever is in flight: 1.1 MB of a
 // 3 x 512 network are 16 us), so here the 32-wide output tiles of a layer go to as many CUs.  A layer needs the whole of the one before
@@ -2259,12 +2268,31 @@ static int launch_fused(const DevMlp& m, hipStream_t s, int64_t M, const float* 
   return launch_fused_tile<__bf16, 32>(m, s, M, x, y, save);
 }
 
+// The row tile that a single bf16 layer takes in the form with a lane per feature, 0 where it takes another form (launch_fused)
+static int single_bm(const DevMlp& m, int64_t M) {
+  if (!m.fused || m.dtype != KS_MLP_BF16 || m.n_layers != 1) return 0;
+  if (M >= 128 * 256) return 128;
+  return M >= 64 * 256 && m.fn[0] <= 2 ? 0 : 32;
+}
+
 static int launch_fused_args(const FusedArgs& a, hipStream_t s) {
   const int bm = a.M >= 128 * 256 ? 128 : 32, lds = bm * a.lda * 2;
   auto kfn = bm == 128 ? mlp_fused_kernel<KS_ACT_NONE, __bf16, 128, true> : mlp_fused_kernel<KS_ACT_NONE, __bf16, 32, true>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
   hipLaunchKernelGGL(kfn, dim3((unsigned)((a.M + bm - 1) / bm)), dim3(64 * kFusedWaves), lds, s, a);
+  return KS_OK;
+}
+
+// Two of them, of one row tile, in one launch
+static int launch_single_pair(const FusedArgs& a, const FusedArgs& b, int bm, hipStream_t s) {
+  const int lds = bm * (a.lda > b.lda ? a.lda : b.lda) * 2;
+  const int64_t ta = (a.M + bm - 1) / bm, tb = (b.M + bm - 1) / bm;
+  if (ta + tb > 0x7fffffff) return fail(KS_ELIMIT, "ks_mlp: too many rows");
+  auto kfn = bm == 128 ? mlp_single_pair_kernel<128> : mlp_single_pair_kernel<32>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp: cannot raise the LDS limit to %d bytes", lds);
+  hipLaunchKernelGGL(kfn, dim3((unsigned)(ta + tb)), dim3(64 * kFusedWaves), lds, s, a, b, (unsigned)ta);
   return KS_OK;
 }
 
@@ -2430,6 +2458,11 @@ extern "C" int ks_mlp_forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t
   if (split_ok(h0->m, M) && split_ok(h1->m, M) && h0->m.n_layers == h1->m.n_layers && h0->m.activation == h1->m.activation && workspace0 &&
       workspace1 && workspace0 != workspace1)
     return launch_split(h0->m, &h1->m, s, M, x0, y0, workspace0, x1, y1, workspace1);
+  // single layers
+  if (const int bm = single_bm(h0->m, M); bm && bm == single_bm(h1->m, M)) {
+    const int rc = launch_single_pair(fused_args(h0->m, M, x0, y0), fused_args(h1->m, M, x1, y1), bm, s);
+    return rc != KS_OK ? rc : check_launch("ks_mlp_forward_pair");
+  }
   // one launch when both networks run as whole-network kernels with the same activation and row tile; else one each
   if (h0->m.fused && h1->m.fused && h0->m.activation == h1->m.activation && h0->m.dtype == h1->m.dtype && M < 64 * 256) {
     if (h0->m.dtype == KS_MLP_F32) return launch_fused_pair_tile<float, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1);
@@ -2801,6 +2834,17 @@ template <int PARTS>
 static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                  int64_t ldc, float* part, float* colsum);
 
+// dX = dZ W of a single bf16 layer as a layer over the transposed fragments
+static FusedArgs single_dx_args(const DevMlp& m, int64_t M, const float* dy, float* dx) {
+  FusedArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.M = M; a.n_layers = 1; a.in_dim = m.dims[1]; a.out_dim = m.dims[0]; a.lda = 32 * m.fn[0] + 8;
+  a.fk[0] = 2 * m.fn[0]; a.fn[0] = (m.fk[0] + 1) / 2;
+  a.Wp[0] = (const u32x4*)m.WtP[0]; a.bp[0] = m.zero_bias;
+  a.x = dy; a.y = dx;
+  return a;
+}
+
 // Backward pass of a single layer (the projections of the recurrent cells and their networks, over all the (step, env) rows of a
 // trajectory slice): no activation to pass through, so the caller's gradient and input are the operands of both products as they are.
 template <typename T>
@@ -2810,13 +2854,7 @@ static int train_backward_single(DevMlp& m, hipStream_t s, int64_t M, const floa
   const bool plain = !accumulate_dx && !zero_rows;
   if (dx && sizeof(T) == 2 && plain && m.WtP[0]) {
     // dX = dZ W: the whole-network kernel over the transposed fragments
-    FusedArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.M = M; a.n_layers = 1; a.in_dim = out; a.out_dim = in; a.lda = 32 * m.fn[0] + 8;
-    a.fk[0] = 2 * m.fn[0]; a.fn[0] = (m.fk[0] + 1) / 2;
-    a.Wp[0] = (const u32x4*)m.WtP[0]; a.bp[0] = m.zero_bias;
-    a.x = dy; a.y = dx;
-    const int rc = launch_fused_args(a, s);
+    const int rc = launch_fused_args(single_dx_args(m, M, dy, dx), s);
     if (rc != KS_OK) return rc;
   } else if (dx) {
     int rc;
@@ -3667,8 +3705,11 @@ __global__ __launch_bounds__(64 * kDrWaves) void disc_rows_kernel(const DiscRows
 // 4 l + e of the tile goes to slot 32 e + l, so that neighbouring lanes write neighbouring fragments; a matrix tile is then every fourth
 // column.
 // `colsum` also receives sum_k A(k, i), the bias gradient, from the fp32 values in the loaders' registers.
-// gridDim.y cuts the k range into slices of kslice; with more than one slice, slice z writes its partial product (M, N) densely to
+// The k range is cut into slices of kslice; with more than one slice, slice z writes its partial product (M, N) densely to
 // C + z * M * N and its column sums to colsum + z * M, and sum_slices_kernel adds them up in a fixed order.
+// A launch takes the products of several layers, whose workgroups follow one another: each by itself cuts a few thousand rows into as many
+// slices as there are CUs and is over in two launches of a few microseconds (twelve layers of a GRU actor and critic, 12288 rows: 24 launches,
+// 194 us -> two, 135 us; a seventh of the slices for each of the twelve: the same, at that many rows the operands' way in sets the pace).
 // Bound by the matrix instructions (eight per product of 16 rows, 64 us at the first size below) and the cuts beside them; the operands
 // take 44 us at the card's copy rate.  The predecessor multiplied on the fp32 instruction, whose time alone is 87 us there.
 //   102400 x 512 x 128, fp32: 122 -> 93 us (110 -> 145 TFLOP/s); relative error against 64 bits 7.3e-7 -> 1.9e-7
@@ -3677,17 +3718,39 @@ __global__ __launch_bounds__(64 * kDrWaves) void disc_rows_kernel(const DiscRows
 constexpr int kTnKB = 32;  // rows of a stage
 __host__ __device__ constexpr int tn_buf(int parts) { return parts * (kTnKB / 8) * 256; }  // one group's LDS buffer, in 16-byte fragments
 
+struct WgradJob {
+  int M, N, K, kslice, tiles, slices;
+  const float *A, *B;
+  int64_t lda, ldb, ldc;
+  float *C, *colsum;        // the gradients
+  float *part, *colpart;    // partial products and column sums, where there is more than one slice
+  unsigned first, first_sum;  // the job's first workgroup in wgrad_kernel and in sum_slices_kernel
+};
+constexpr int kWgradJobs = 12;
+struct WgradTable {
+  int n;
+  WgradJob job[kWgradJobs];
+};
+
 template <int PARTS, bool EDGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
-                  float* __restrict__ C, int64_t ldc, int kslice, float* __restrict__ colsum) {
+void wgrad_kernel(const WgradTable table) {
   extern __shared__ __attribute__((aligned(16))) u32x4 tn_lds[];  // [group][part][8 rows][slot: 128 of A, 128 of B]
+  int which = 0;
+  while (which + 1 < table.n && blockIdx.x >= table.job[which + 1].first) ++which;
+  const WgradJob& job = table.job[which];
+  const int M = job.M, N = job.N, K = job.K, kslice = job.kslice, tiles = job.tiles, slices = job.slices, lb = (int)(blockIdx.x - job.first);
+  if (lb >= tiles * slices) return;  // the workgroups that fill up the job's last eight
+  const float *__restrict__ A = job.A, *__restrict__ B = job.B;
+  const int64_t lda = job.lda, ldb = job.ldb, ldc = job.ldc;
+  const bool sliced = slices > 1;
+  float *__restrict__ C = sliced ? job.part : job.C, *__restrict__ colsum = sliced ? job.colpart : job.colsum;
   // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD one after the other
-  int tile = blockIdx.x, z = blockIdx.y;
-  if (gridDim.y % 8 == 0) {
-    const int l = blockIdx.y * gridDim.x + blockIdx.x, q = l >> 3;
-    tile = q % gridDim.x;
-    z = (q / gridDim.x) * 8 + (l & 7);
+  int tile = lb % tiles, z = lb / tiles;
+  if (slices % 8 == 0) {
+    const int q = lb >> 3;
+    tile = q % tiles;
+    z = (q / tiles) * 8 + (lb & 7);
   }
   const int tiles_n = (N + 127) / 128;
   const int grp = threadIdx.x >> 8, t = threadIdx.x & 255, i0 = tile / tiles_n * 128, j0 = tile % tiles_n * 128;
@@ -3812,7 +3875,6 @@ void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
     }
     __syncthreads();
   }
-  const bool sliced = gridDim.y > 1;
   if (colsum && j0 == 0) {
     float* sums = reinterpret_cast<float*>(tn_lds);  // [group][8 rows][128]
     if (!isb) *reinterpret_cast<float4*>(sums + (grp * 4 + kg) * 128 + 4 * l) = cs;
@@ -3846,12 +3908,18 @@ void wgrad_kernel(int M, int N, int K, const float* __restrict__ A, int64_t lda,
 
 // C = the sum of nz slices of (M, N), and colsum = the sum of nz rows of M behind it in the same launch.  A workgroup takes 64 entries,
 // a quarter of the slices to each wavefront with 16 loads in flight, then adds the four in order.
-__global__ __launch_bounds__(256) void sum_slices_kernel(int M, int N, int nz, const float* __restrict__ part, float* __restrict__ C,
-                                                         int64_t ldc, const float* __restrict__ colpart, float* __restrict__ colsum) {
+__global__ __launch_bounds__(256) void sum_slices_kernel(const WgradTable table) {
   __shared__ float sh[256];
-  const int64_t mn = (int64_t)M * N, wblocks = (mn + 63) / 64;
-  const bool col = blockIdx.x >= wblocks;
-  const int64_t n = col ? M : mn, idx = ((int64_t)blockIdx.x - (col ? wblocks : 0)) * 64 + (threadIdx.x & 63);
+  int which = 0;
+  while (which + 1 < table.n && blockIdx.x >= table.job[which + 1].first_sum) ++which;
+  const WgradJob& job = table.job[which];
+  const int M = job.M, N = job.N, nz = job.slices;
+  const float *__restrict__ part = job.part, *__restrict__ colpart = job.colpart;
+  float *__restrict__ C = job.C, *__restrict__ colsum = job.colsum;
+  const int64_t ldc = job.ldc;
+  const int64_t mn = (int64_t)M * N, wblocks = (mn + 63) / 64, block = blockIdx.x - job.first_sum;
+  const bool col = block >= wblocks;
+  const int64_t n = col ? M : mn, idx = (block - (col ? wblocks : 0)) * 64 + (threadIdx.x & 63);
   const float* src = col ? colpart : part;
   const int w = threadIdx.x >> 6, per = (nz + 3) / 4, zb = w * per, ze = min(nz, zb + per);
   float s = 0.f;
@@ -3988,23 +4056,128 @@ static int group_blocks(SgemmGroup& t) {
 }
 
 // C (M, N) = A^T B over K rows with the column sums of A beside it, on 128 x 128 tiles: the weight and bias gradient of a single layer.
+static WgradJob wgrad_job(int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C, int64_t ldc, float* part,
+                          float* colsum) {
+  WgradJob j;
+  j.M = (int)M; j.N = N; j.K = (int)K; j.A = A; j.lda = lda; j.B = B; j.ldb = ldb; j.C = C; j.ldc = ldc; j.colsum = colsum; j.part = part;
+  j.tiles = (int)(((M + 127) / 128) * ((N + 127) / 128));
+  j.slices = wgrad_slices(M, N, K);  // the layer's own number, so that a gradient does not depend on what it shares the launch with
+  j.kslice = (int)(((K + j.slices - 1) / j.slices + 2 * kTnKB - 1) / (2 * kTnKB)) * 2 * kTnKB;  // slices past the last row add zeros
+  j.colpart = part + (int64_t)j.slices * M * N;
+  j.first = j.first_sum = 0;
+  return j;
+}
+
+// Several of them, of one kind: a launch for the products and one for the sums of their slices
+template <int PARTS>
+static int wgrads(hipStream_t s, WgradTable& t) {
+  unsigned blocks = 0, sums = 0;
+  bool edge = false;
+  for (int k = 0; k < t.n; ++k) {
+    WgradJob& j = t.job[k];
+    edge |= j.M % 4 || j.N % 4;
+    j.first = blocks;
+    blocks += (unsigned)round_up(j.tiles * j.slices, 8);  // the next job's slices stay on the XCDs they are meant for
+    j.first_sum = sums;
+    if (j.slices > 1) sums += (unsigned)(((int64_t)j.M * j.N + 63) / 64 + (j.M + 63) / 64);
+  }
+  constexpr int lds = 2 * tn_buf(PARTS) * 16;
+  auto kfn = edge ? wgrad_kernel<PARTS, true> : wgrad_kernel<PARTS, false>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
+  hipLaunchKernelGGL(kfn, dim3(blocks), dim3(512), lds, s, t);
+  if (sums) hipLaunchKernelGGL(sum_slices_kernel, dim3(sums), dim3(256), 0, s, t);
+  return KS_OK;
+}
+
 template <int PARTS>
 static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                  int64_t ldc, float* part, float* colsum) {
-  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  const int slices = wgrad_slices(M, N, K);
-  const int kslice = (int)(((K + slices - 1) / slices + 2 * kTnKB - 1) / (2 * kTnKB)) * 2 * kTnKB;  // slices past the last row add zeros
-  constexpr int lds = 2 * tn_buf(PARTS) * 16;
-  float* colpart = part + (int64_t)slices * M * N;
-  auto kfn = M % 4 || N % 4 ? wgrad_kernel<PARTS, true> : wgrad_kernel<PARTS, false>;
-  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
-  hipLaunchKernelGGL(kfn, dim3((unsigned)tiles, (unsigned)slices), dim3(512), lds, s, (int)M, N, (int)K, A, lda, B, ldb,
-                     slices > 1 ? part : C, ldc, kslice, slices > 1 ? colpart : colsum);
-  if (slices > 1)
-    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((M * N + 63) / 64 + (M + 63) / 64)), dim3(256), 0, s, (int)M, N, slices, part, C, ldc,
-                       colpart, colsum);
+  WgradTable t;
+  t.n = 1;
+  t.job[0] = wgrad_job(M, N, K, A, lda, B, ldb, C, ldc, part, colsum);
+  return wgrads<PARTS>(s, t);
+}
+
+// ---------------------------------------------------------------------------------------------
+// backward pass of several single layers, e.g. all projections of a recurrent actor and critic
+// ---------------------------------------------------------------------------------------------
+// The gradient of the network input by a single layer of bf16: the whole-network kernel over the transposed fragments
+static bool single_dx_ok(const DevMlp& m) { return m.dtype == KS_MLP_BF16 && m.WtP[0]; }
+
+static int64_t wgrad_part_floats(const DevMlp& m, int64_t M) { return (int64_t)wgrad_slices(m.dims[1], m.dims[0], M) * m.dims[1] * (m.dims[0] + 1); }
+
+static int check_layer_backward(const KsLayerBackward& q) {
+  if (!q.mlp || !q.mlp->m.train) return fail(KS_EINVAL, "ks_mlps_layer_backward: call ks_mlp_train_init first");
+  if (q.mlp->m.n_layers != 1) return fail(KS_EINVAL, "ks_mlps_layer_backward: the network has %d layers, not one", q.mlp->m.n_layers);
+  if (q.M <= 0 || !q.dy || (!q.x && !q.dx) || (q.x && q.ldx < q.mlp->m.dims[0])) return fail(KS_EINVAL, "ks_mlps_layer_backward: bad argument");
+  if (q.M > (1 << 30)) return fail(KS_ELIMIT, "ks_mlps_layer_backward: too many rows");
   return KS_OK;
+}
+
+extern "C" int64_t ks_mlps_layer_backward_workspace_bytes(int32_t n, const KsLayerBackward* q) {
+  int64_t parts = 0, most = 0;
+  for (int k = 0; q && k < n; ++k) {
+    if (!q[k].mlp || q[k].M < 0) return 0;
+    const DevMlp& m = q[k].mlp->m;
+    if (q[k].x) parts += (wgrad_part_floats(m, q[k].M) * 4 + 255) / 256 * 256;
+    if (q[k].dx && m.dtype == KS_MLP_BF16 && !single_dx_ok(m)) most = std::max(most, carve_train(m, q[k].M, nullptr, nullptr));
+  }
+  return std::max(parts, most) + 256;
+}
+
+extern "C" int ks_mlps_layer_backward(int32_t n, const KsLayerBackward* q, ks_stream_t stream, void* workspace) {
+  if (n < 0 || (n > 0 && (!q || !workspace))) return fail(KS_EINVAL, "ks_mlps_layer_backward: bad argument");
+  for (int k = 0; k < n; ++k)
+    if (const int rc = check_layer_backward(q[k])) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  // input gradients: those of bf16 layers two to a launch, each with the next one that has its row tile
+  FusedArgs held;
+  int held_bm = 0;
+  for (int k = 0; k < n; ++k) {
+    if (!q[k].dx) continue;
+    DevMlp& m = q[k].mlp->m;
+    int rc = KS_OK;
+    if (single_dx_ok(m)) {
+      const FusedArgs a = single_dx_args(m, q[k].M, q[k].dy, q[k].dx);
+      const int bm = a.M >= 128 * 256 ? 128 : 32;
+      if (held_bm == bm) {
+        rc = launch_single_pair(held, a, bm, s);
+        held_bm = 0;
+      } else {
+        if (held_bm) rc = launch_fused_args(held, s);
+        held = a;
+        held_bm = bm;
+      }
+    } else if (m.dtype == KS_MLP_BF16) {
+      TrainWs ws;
+      carve_train(m, q[k].M, (char*)workspace, &ws);
+      rc = train_backward_single<__bf16>(m, s, q[k].M, nullptr, 0, q[k].dy, ws, q[k].dx, false, false, nullptr);
+    } else {
+      rc = train_backward_single<float>(m, s, q[k].M, nullptr, 0, q[k].dy, TrainWs{}, q[k].dx, false, false, nullptr);  // writes dx itself: no workspace
+    }
+    if (rc != KS_OK) return rc;
+  }
+  if (held_bm)
+    if (const int rc = launch_fused_args(held, s)) return rc;
+  // weight gradients, those of a precision together
+  char* part = (char*)workspace;
+  for (int bf16 = 0; bf16 < 2; ++bf16) {
+    WgradTable t;
+    t.n = 0;
+    for (int k = 0; k <= n; ++k) {
+      if (t.n == kWgradJobs || (k == n && t.n > 0)) {
+        const int rc = bf16 ? wgrads<1>(s, t) : wgrads<3>(s, t);
+        if (rc != KS_OK) return rc;
+        t.n = 0;
+      }
+      if (k == n || !q[k].x || (q[k].mlp->m.dtype == KS_MLP_BF16) != (bf16 != 0)) continue;
+      DevMlp& m = q[k].mlp->m;
+      t.job[t.n++] = wgrad_job(m.dims[1], m.dims[0], q[k].M, q[k].dy, m.dims[1], q[k].x, q[k].ldx, m.gW[0], m.kpad[0], (float*)part, m.gb[0]);
+      part += (wgrad_part_floats(m, q[k].M) * 4 + 255) / 256 * 256;
+    }
+  }
+  return check_launch("ks_mlps_layer_backward");
 }
 
 extern "C" int64_t ks_mlp_disc_workspace_bytes(const KsMlp* h, int64_t n_real, int64_t n_sim) {

@@ -24,6 +24,10 @@ from .mlp import MLP
 SEQUENCE_ROWS = 131072
 
 
+# (step, env) rows up to which `RecurrentNetwork.backward` puts all weight gradients into one launch at its end
+LATER_ROWS = 32768
+
+
 def _f32(a) -> np.ndarray:
     return np.ascontiguousarray(a.detach().cpu().numpy() if isinstance(a, torch.Tensor) else a, dtype=np.float32)
 
@@ -50,19 +54,87 @@ def run_sequences(calls: Sequence[SequenceCall]) -> None:
         del calls[:n]
 
 
+class LayerForward:
+    """A single layer over rows x (M, in), ready to launch; `out` (M, out) holds the result then."""
+
+    def __init__(self, net: MLP, x: torch.Tensor, out: torch.Tensor | None = None):
+        self.net, self.x = net, x
+        self.out = torch.empty((x.shape[0], net.out_dim), dtype=torch.float32, device=x.device) if out is None else out
+
+
+class LayerBackward:
+    """The backward pass of a single layer from the gradient dy (M, out) of its output, ready to launch: weight and bias gradient into its
+    handle where the input x (M, in; a block of columns of wider rows, if need be) is given, gradient of the input into `dx` where that is."""
+
+    def __init__(self, net: MLP, dy: torch.Tensor, x: torch.Tensor | None = None, dx: torch.Tensor | None = None):
+        M = dy.shape[0]
+        _lib.require_cuda(dy, dx, dtype=torch.float32)
+        if (tuple(dy.shape) != (M, net.out_dim) or (dx is not None and tuple(dx.shape) != (M, net.in_dim))
+                or (x is not None and (tuple(x.shape) != (M, net.in_dim) or x.dtype != torch.float32 or not x.is_cuda
+                                       or x.stride(1) != 1 or x.stride(0) < net.in_dim))):
+            raise _lib.KsError("dy must be (M, out), dx and x (M, in) fp32 rows on the GPU, the columns of x side by side")
+        self.net, self.dy, self.x, self.dx = net, dy, x, dx
+
+    def record(self) -> "T.KsLayerBackward":
+        return T.KsLayerBackward(self.net._handle.value, self.dy.shape[0], _lib.addr(self.x), 0 if self.x is None else self.x.stride(0),
+                                 _lib.addr(self.dy), _lib.addr(self.dx))
+
+
+def run_layers(calls: Sequence[LayerForward]) -> None:
+    """Launches single layers, two over as many rows each in one launch where the library can (`ks_mlp_forward_pair`)."""
+    calls = list(calls)
+    while calls:
+        a = calls.pop(0)
+        if calls and calls[0].x.shape[0] == a.x.shape[0]:
+            b = calls.pop(0)
+            a.net.forward_pair(a.x, a.out, b.net, b.x, b.out)
+        else:
+            a.net(a.x, out=a.out)
+
+
+def run_layers_backward(calls: Sequence[LayerBackward]) -> None:
+    """Launches the backward passes of single layers, together where the library can."""
+    lib, table = _lib.load(), (T.KsLayerBackward * len(calls))(*(c.record() for c in calls))
+    ws = torch.empty(int(lib.ks_mlps_layer_backward_workspace_bytes(len(calls), table)), dtype=torch.uint8, device=calls[0].dy.device)
+    _lib.check(lib.ks_mlps_layer_backward(len(calls), table, _lib.current_stream(), _lib.addr(ws)))
+
+
+def _listed(calls) -> list:
+    return calls if isinstance(calls, list) else [calls]
+
+
+def run_calls(calls) -> None:
+    """Launches what the passes of several networks have ready, calls of a kind together."""
+    for kind, run in ((LayerForward, run_layers), (SequenceCall, run_sequences), (LayerBackward, run_layers_backward)):
+        some = [c for c in calls if isinstance(c, kind)]
+        if some:
+            run(some)
+
+
 def lockstep(*passes):
-    """Runs generators that yield the `SequenceCall`s of their layers side by side, launching what they yield together; returns their results."""
+    """Runs generators that yield calls (`SequenceCall`, `LayerForward`, lists of `LayerBackward`) side by side, launching what they yield
+    together; returns their results."""
     results, live = [None] * len(passes), list(range(len(passes)))
     while live:
         calls = []
         for k in tuple(live):
             try:
-                calls.append(next(passes[k]))
+                calls += _listed(next(passes[k]))
             except StopIteration as stop:
                 results[k] = stop.value
                 live.remove(k)
-        run_sequences(calls)
+        run_calls(calls)
     return results
+
+
+def _layer(net: MLP, x: torch.Tensor, out: torch.Tensor | None = None):
+    """A network's forward pass inside a pass over a trajectory: single bf16 layers, which rows of a trajectory hardly fill the chip with, are left
+    to `lockstep`, which puts those of two networks into one launch."""
+    if len(net.dims) == 2 and net.dtype == "bf16":
+        call = LayerForward(net, x, out)
+        yield call
+        return call.out
+    return net(x, out=out)
 
 
 class GRUCell:
@@ -155,7 +227,7 @@ class GRUCell:
             self._proj = MLP._borrow(self._lib, pi, (self.input_size, 3 * self.hidden_size), self.dtype)
         return self._proj
 
-    def sequence_call(self, x, h0, fresh, hs, saved) -> "SequenceCall":
+    def sequence_call(self, x, h0, fresh, hs, saved, gi=None) -> "SequenceCall":
         """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`)."""
         _lib.require_cuda(x, h0, hs, saved, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
@@ -163,7 +235,8 @@ class GRUCell:
         if (tuple(x.shape) != (Tn, M, self.input_size) or tuple(h0.shape) != (M, H) or tuple(hs.shape) != (Tn, M, H)
                 or (saved is not None and tuple(saved.shape) != (Tn, M, 5 * H)) or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected x (T, M, input), h0 (M, H), hs (T, M, H), saved (T, M, 5H), fresh (T, M)")
-        gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
+        if gi is None:
+            gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
         return SequenceCall("ks_gru_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, None, fresh, saved, hs, None)
 
     def sequence_forward(self, x, h0, fresh, hs, saved) -> None:
@@ -208,7 +281,7 @@ class GRUCell:
     def parameters(self, gradients: bool = False) -> dict:
         """Copies of weight_ih, weight_hh, bias (3H) and bias_n (H), or of their gradients."""
         ((wi, bi),), ((wh, bh),) = mlp_mod.copy_parameters((self.proj_i, self.proj_h), gradients)
-        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:].clone())
+        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:])
 
     def __del__(self):
         h = getattr(self, "_handle", None)
@@ -302,8 +375,9 @@ class LSTMCell:
             self._proj = MLP._borrow(self._lib, pi, (self.input_size, 4 * self.hidden_size), self.dtype)
         return self._proj
 
-    def sequence_call(self, x, h0, c0, fresh, hs, cs, saved) -> "SequenceCall":
-        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`)."""
+    def sequence_call(self, x, h0, c0, fresh, hs, cs, saved, gi=None) -> "SequenceCall":
+        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`); `gi`: the projected input, where
+        the caller has it."""
         _lib.require_cuda(x, h0, c0, hs, cs, saved, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
@@ -311,7 +385,8 @@ class LSTMCell:
                 or any(t is not None and tuple(t.shape) != (Tn, M, H) for t in (hs, cs))
                 or (saved is not None and tuple(saved.shape) != (Tn, M, 7 * H)) or tuple(fresh.shape) != (Tn, M)):
             raise _lib.KsError("expected x (T, M, input), h0, c0 (M, H), hs, cs (T, M, H), saved (T, M, 7H), fresh (T, M)")
-        gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
+        if gi is None:
+            gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
         return SequenceCall("ks_lstm_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, c0, fresh, saved, hs, cs)
 
     def sequence_forward(self, x, h0, c0, fresh, hs, cs, saved) -> None:
@@ -428,16 +503,17 @@ class RecurrentNetwork:
         carry = [carry0[i].unbind(0) if self.lstm else (carry0[i],) for i in range(self.depth)]  # per layer (h, c) or (h,)
         for t0 in range(0, T_, steps):
             n = min(steps, T_ - t0)
-            x = self.input_proj(obs[t0:t0 + n].contiguous().view(n * M, self.in_dim)).view(n, M, H)
+            x = (yield from _layer(self.input_proj, obs[t0:t0 + n].contiguous().view(n * M, self.in_dim))).view(n, M, H)
             for i, cell in enumerate(self.cells):
                 states = [torch.empty(n, M, H, dtype=torch.float32, device=obs.device)]
                 if self.lstm:  # the cell state only where another stretch starts from it
                     states.append(torch.empty_like(states[0]) if t0 + n < T_ else None)
-                yield cell.sequence_call(x, *carry[i], fresh[t0:t0 + n], *states, None)
+                # the projected rows, as large as four states, are gone before the next layer's come
+                yield cell.sequence_call(x, *carry[i], fresh[t0:t0 + n], *states, None, (yield from _layer(cell._input_projection(), x.view(n * M, H))))
                 x = states[0]
                 if t0 + n < T_:
                     carry[i] = tuple(s[-1].clone() for s in states)
-            self.output_proj(x.view(n * M, H), out=out[t0:t0 + n].view(n * M, self.out_dim))
+            yield from _layer(self.output_proj, x.view(n * M, H), out[t0:t0 + n].view(n * M, self.out_dim))
         return out
 
     # ------------------------------------------------------------------ training: backward pass through time
@@ -464,27 +540,31 @@ class RecurrentNetwork:
         if tuple(obs.shape) != (T_, M, self.in_dim) or tuple(carry0.shape) != want or tuple(fresh.shape) != (T_, M):
             raise _lib.KsError(f"expected obs (T, M, in), carry0 {want}, fresh (T, M)")
         obs = obs.contiguous()
-        x = self.input_proj(obs.view(T_ * M, self.in_dim)).view(T_, M, H)
+        x = (yield from _layer(self.input_proj, obs.view(T_ * M, self.in_dim))).view(T_, M, H)
         xs, saved = [], []
         for i, cell in enumerate(self.cells):
             hs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
             sv = torch.empty(T_, M, (7 if self.lstm else 5) * H, dtype=torch.float32, device=dev)
             if self.lstm and getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
-                yield cell.sequence_call(x, carry0[i, 0], carry0[i, 1], fresh, hs, None, sv)
+                yield cell.sequence_call(x, carry0[i, 0], carry0[i, 1], fresh, hs, None, sv, (yield from _layer(cell.proj_i, x.view(T_ * M, H))))
             elif self.lstm:
                 cs = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
                 for t in range(T_):
                     h0, c0 = (carry0[i, 0], carry0[i, 1]) if t == 0 else (hs[t - 1], cs[t - 1])
                     cell.train_forward(x[t], h0, c0, fresh[t], hs[t], cs[t], sv[t])
             elif getattr(cell, "proj_i", None) is not None and cell.sequence_supported:
-                yield cell.sequence_call(x, carry0[i], fresh, hs, sv)
+                yield cell.sequence_call(x, carry0[i], fresh, hs, sv, (yield from _layer(cell.proj_i, x.view(T_ * M, H))))
             else:
                 for t in range(T_):
                     cell.train_forward(x[t], carry0[i] if t == 0 else hs[t - 1], fresh[t], hs[t], sv[t])
             xs.append(x)
             saved.append(sv)
             x = hs
-        out = self.output_proj.train_forward(x.view(T_ * M, H)).view(T_, M, self.out_dim)
+        if len(self.output_proj.dims) == 2 and self.output_proj.dtype == "bf16":  # a single layer keeps nothing for its backward pass
+            out = yield from _layer(self.output_proj, x.view(T_ * M, H))
+        else:
+            out = self.output_proj.train_forward(x.view(T_ * M, H))
+        out = out.view(T_, M, self.out_dim)
         self._tape = dict(obs=obs, xs=xs, saved=saved, top=x, fresh=fresh.contiguous(), T=T_, M=M)
         return out
 
@@ -505,7 +585,21 @@ class RecurrentNetwork:
         if tuple(d_out.shape) != (T_, M, self.out_dim):
             raise _lib.KsError("d_out must have the shape of the output")
         dH = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
-        self.output_proj.backward_dx(tp["top"].view(T_ * M, H), d_out.contiguous().view(T_ * M, self.out_dim), dH.view(T_ * M, H))
+        # Few rows: the weight gradients of all layers wait for the last of them and share a launch.  Many rows fill the chip layer by layer, and
+        # the gate gradients, which the weight gradients read, are as large as all that the forward pass keeps.
+        later: list[LayerBackward] | None = [] if T_ * M <= LATER_ROWS else None
+
+        def layer(net, x, dy, dx=None):  # calls of a layer's backward pass that are due now
+            if later is None:
+                return [LayerBackward(net, dy, x, dx)]
+            later.append(LayerBackward(net, dy, x))
+            return [] if dx is None else [LayerBackward(net, dy, None, dx)]
+
+        top, d_top = tp["top"].view(T_ * M, H), d_out.contiguous().view(T_ * M, self.out_dim)
+        if len(self.output_proj.dims) == 2:
+            yield layer(self.output_proj, top, d_top, dH.view(T_ * M, H))
+        else:
+            self.output_proj.backward_dx(top, d_top, dH.view(T_ * M, H))
         for i in range(self.depth - 1, -1, -1):
             cell, sv = self.cells[i], tp["saved"][i]
             d_gi = torch.empty(T_, M, G * H, dtype=torch.float32, device=dev)
@@ -525,11 +619,11 @@ class RecurrentNetwork:
                 else:
                     cell.backward_step(dH[t], sv[t], tp["fresh"][t], d_gi[t], d_gh[t], carry[(t + 1) & 1])
             h_used = sv.view(T_ * M, sv.shape[2])[:, (6 if self.lstm else 4) * H:]
-            cell.proj_h.layer_weight_grad(h_used, d_gh.view(T_ * M, G * H))
             dX = torch.empty(T_, M, H, dtype=torch.float32, device=dev)
-            cell.proj_i.backward_dx(tp["xs"][i].reshape(T_ * M, H), d_gi.view(T_ * M, G * H), dX.view(T_ * M, H))
+            yield (layer(cell.proj_h, h_used, d_gh.view(T_ * M, G * H))
+                   + layer(cell.proj_i, tp["xs"][i].reshape(T_ * M, H), d_gi.view(T_ * M, G * H), dX.view(T_ * M, H)))
             dH = dX
-        self.input_proj.backward(tp["obs"].view(T_ * M, self.in_dim), dH.view(T_ * M, H))
+        yield (later or []) + [LayerBackward(self.input_proj, dH.view(T_ * M, H), tp["obs"].view(T_ * M, self.in_dim))]
 
     def networks(self) -> list[MLP]:
         """Every network whose parameters an optimiser step updates: the projections and both products of every cell."""

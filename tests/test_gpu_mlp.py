@@ -438,3 +438,45 @@ def test_one_network_called_by_two_threads(dtype):
         for k in range(2):
             for rep in got[k]:
                 assert all(torch.equal(a, b) for a, b in zip(rep, want[k]))
+
+
+@pytest.mark.parametrize("M", [1, 37, 193, 1544, 16411, 32771])
+def test_single_layers_in_shared_launches_match_one_by_one(M):
+    """Backward passes of single layers of both precisions in one call (more of them than a launch takes, odd widths, inputs that are columns
+    of wider rows, without input or without weight gradient) and pairs of forward passes, bit for bit the calls by themselves."""
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import LayerBackward, LayerForward, run_layers, run_layers_backward
+
+    rng = np.random.default_rng(M)
+    t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    shapes = [(43, 128), (128, 384), (128, 384), (128, 510), (340, 128), (128, 1), (128, 40)]
+    nets = []
+    for dtype in ("bf16", "f32"):
+        for k, (i, o) in enumerate(shapes * (2 if dtype == "bf16" and M < 2000 else 1)):  # two layers of a shape: two launches of weight gradients
+            net = MLP([rng.normal(scale=i ** -0.5, size=(o, i))], [0.1 * rng.normal(size=o)], activation="none", dtype=dtype)
+            net.train_init()
+            nets.append((net, k))
+    calls, want = [], []
+    for net, k in nets:
+        i, o = net.in_dim, net.out_dim
+        wide = t(M, i + 32)
+        x, dy = (wide[:, 32:] if k % 3 == 0 else t(M, i)), t(M, o)
+        dx = torch.empty(M, i, device="cuda") if k % 4 != 3 else None
+        w = k % 5 != 4 or dx is None
+        if w:
+            net.layer_weight_grad(x, dy)
+        grads = [g.clone() for pair in net.parameters(gradients=True) for g in pair]
+        one = None if dx is None else net.backward_dx(None, dy, torch.empty_like(dx), weight_gradients=False)
+        net.layer_weight_grad(t(M, i), t(M, o))  # something else in the handle
+        other = [g.clone() for pair in net.parameters(gradients=True) for g in pair]
+        calls.append(LayerBackward(net, dy, x if w else None, dx))
+        want.append((grads if w else other, one))
+    run_layers_backward(calls)
+    for (net, k), call, (grads, one) in zip(nets, calls, want):
+        got = [g for pair in net.parameters(gradients=True) for g in pair]
+        assert all(torch.equal(a, b) for a, b in zip(got, grads)), (net.dims, net.dtype)
+        assert one is None or torch.equal(call.dx, one), (net.dims, net.dtype)
+    forward = [LayerForward(net, t(M, net.in_dim)) for net, _ in nets]
+    run_layers(forward)
+    for call in forward:
+        assert torch.equal(call.out, call.net(call.x)), (call.net.dims, call.net.dtype)
