@@ -834,6 +834,13 @@ typedef struct KsGatherArray {
   int64_t outer, inner;
 } KsGatherArray;
 int ks_gather_columns(ks_stream_t stream, int32_t n, const KsGatherArray* arrays /*host*/, int64_t columns, int64_t picked, const int64_t* index);
+/* The batches of a discriminator step (ksim/task/amp.py:570-652): real_out (batch, window_t, frame) the windows that begin at frame start[k] of
+ * clip clip[k] of motions (clips, clip_t, frame), wrapping round at the clip's end; sim_out the sequences env[k] of sim (envs, window_t, frame).
+ * The drawn indices are host memory and are read before the call returns. */
+#define KS_WINDOWS 128
+int ks_gather_windows(ks_stream_t stream, int32_t batch, int64_t window_t, int64_t frame, int64_t clips, int64_t clip_t, int64_t envs,
+                      const float* motions, const float* sim, const int64_t* clip /*host*/, const int64_t* start /*host*/,
+                      const int64_t* env /*host*/, float* real_out, float* sim_out);
 /* Mirror (left / right symmetry) losses of a task, examples/kbot/train.py:1458-1477, for networks applied to flat rows.
  * A mirror map is a signed permutation: mirrored[j] = sign[j] * x[perm[j]] (mirror_joints / mirror_obs / mirror_cmd,
  * train.py:1565-1760, each negate and reorder entries of their vector).

@@ -193,6 +193,7 @@ class KsSequence(ctypes.Structure):
 
 
 KS_GATHER_ARRAYS = 24
+KS_WINDOWS = 128
 
 
 class KsGatherArray(ctypes.Structure):
@@ -314,6 +315,8 @@ def bind(lib) -> None:
         getattr(lib, name).restype = c_int32
     lib.ks_gather_columns.argtypes = [c_void_p, c_int32, POINTER(KsGatherArray), c_int64, c_int64, c_void_p]
     lib.ks_gather_columns.restype = c_int32
+    lib.ks_gather_windows.argtypes = [c_void_p, c_int32] + [c_int64] * 5 + [c_void_p] * 7
+    lib.ks_gather_windows.restype = c_int32
     lib.ks_mlps_grad_sqnorm.argtypes = [c_void_p, c_int32, c_void_p, c_void_p]
     lib.ks_mlps_adam_step.argtypes = [c_void_p, c_int32, c_void_p, POINTER(KsAdamParams), c_void_p]
     lib.ks_adam_step.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(KsAdamParams), c_void_p]

@@ -66,6 +66,26 @@ def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Gen
     return sim_motions.index_select(0, _on_device(torch.randperm(num_envs, generator=generator)[:batch_b], sim_motions.device))
 
 
+def _batches(motions: torch.Tensor, sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> tuple[torch.Tensor, torch.Tensor]:
+    """`make_real_batch` and `make_sim_batch` of one step, in one launch where both are plain fp32 arrays of frames on one GPU."""
+    window_t = sim_motions.shape[1]
+    plain = (1 <= batch_b <= T.KS_WINDOWS and motions.dim() == sim_motions.dim() == 3 and motions.shape[2] == sim_motions.shape[2]
+             and motions.dtype == sim_motions.dtype == torch.float32 and motions.is_cuda and motions.device == sim_motions.device
+             and motions.is_contiguous() and sim_motions.is_contiguous() and motions.numel() > 0 and sim_motions.numel() > 0
+             and sim_motions.shape[0] % batch_b == 0 and (motions.shape[1] + window_t) * motions.shape[2] < 1 << 27
+             and motions.device.index == torch._C._cuda_getDevice())
+    if not plain:
+        return make_real_batch(motions, window_t, batch_b, generator), make_sim_batch(sim_motions, batch_b, generator)
+    (n, t_clip, frame), num_envs = motions.shape, sim_motions.shape[0]
+    clip_idx = torch.randint(0, n, (batch_b,), generator=generator)  # the draws of the two functions above, in their order
+    starts = torch.randint(0, t_clip, (batch_b,), generator=generator)
+    envs = torch.randperm(num_envs, generator=generator)
+    real, sim = (torch.empty((batch_b, window_t, frame), dtype=torch.float32, device=motions.device) for _ in range(2))
+    _lib.check(_lib.load().ks_gather_windows(_lib.current_stream(), batch_b, window_t, frame, n, t_clip, num_envs, motions.data_ptr(), sim_motions.data_ptr(),
+                                             clip_idx.data_ptr(), starts.data_ptr(), envs.data_ptr(), real.data_ptr(), sim.data_ptr()))
+    return real, sim
+
+
 class DiscriminatorUpdate:
     """Owns the discriminator's optimiser state; `step` is one pass of amp.py:486-527, `update` all of them."""
 
@@ -95,11 +115,8 @@ class DiscriminatorUpdate:
 
     def update(self, motions: torch.Tensor, sim_motions: torch.Tensor, generator: torch.Generator) -> dict[str, torch.Tensor]:
         """`disc_num_passes` steps, each on fresh batches; the metrics are averaged over the passes (amp.py:529-536)."""
-        window_t = sim_motions.shape[1]
         sums: dict[str, torch.Tensor] = {}
         for _ in range(self.cfg.disc_num_passes):
-            real = make_real_batch(motions, window_t, self.cfg.amp_reference_batch_size, generator)
-            sim = make_sim_batch(sim_motions, self.cfg.amp_reference_batch_size, generator)
-            for k, v in self.step(real, sim).items():
+            for k, v in self.step(*_batches(motions, sim_motions, self.cfg.amp_reference_batch_size, generator)).items():
                 sums[k] = v if k not in sums else sums[k] + v
         return sums if self.cfg.disc_num_passes == 1 else {k: v / self.cfg.disc_num_passes for k, v in sums.items()}

@@ -328,3 +328,22 @@ def test_discriminator_of_five_layers(rows, coef):
     real, sim = (rng.normal(size=(*s, dims[0])).astype(np.float32) for s in rows)
     for _ in range(2):  # counters and partial sums of the first call do not reach the second
         _check(disc, ws, bs, real, sim, coef, "tanh")
+
+
+@pytest.mark.parametrize("batch,envs,window_t,clips,clip_t,frame", [(1, 1, 1, 1, 1, 1), (6, 12, 10, 4, 7, 2), (2, 4, 40, 3, 3, 65), (32, 64, 32, 9, 50, 71),
+                                                                    (128, 128, 24, 5, 24, 86), (129, 129, 8, 3, 9, 3)])
+def test_both_batches_of_a_step_in_one_launch(batch, envs, window_t, clips, clip_t, frame):
+    """The batches that `update` draws are those of `make_real_batch` and `make_sim_batch` from the same generator: windows that wrap once and
+    several times, the largest batch of the launch and one more than it takes, and arrays that it leaves to them."""
+    from ksim_amd import amp
+
+    g = torch.Generator(device=DEV).manual_seed(batch)
+    motions, sims = torch.randn(clips, clip_t, frame, device=DEV, generator=g), torch.randn(envs, window_t, frame, device=DEV, generator=g)
+    strided = torch.randn(clips, 2 * clip_t, frame, device=DEV, generator=g)[:, ::2]
+    for m, s in ((motions, sims), (strided, sims), (motions.double(), sims.double()), (motions, sims.expand(envs, window_t, frame))):
+        one, two = torch.Generator().manual_seed(7), torch.Generator().manual_seed(7)
+        real, sim = amp._batches(m, s, batch, one)
+        assert torch.equal(real, amp.make_real_batch(m, window_t, batch, two)) and torch.equal(sim, amp.make_sim_batch(s, batch, two))
+        assert torch.equal(one.get_state(), two.get_state())
+    with pytest.raises(ValueError, match="must divide"):
+        amp._batches(motions, torch.cat([sims, sims[:1]]) if batch > 1 else sims, 2 if batch == 1 else batch, torch.Generator())
