@@ -408,6 +408,40 @@ def test_lowpass_scan_kernels_match_the_oracle():
     assert lib.ks_lowpass_scan(_lib.current_stream(), Tn, M, nu, 2 * nu, dt, fc, _lib.ptr(d_raw), None, add, I, nu - 1, 2, None, None, _lib.ptr(out), None) != 0
 
 
+@pytest.mark.parametrize("Tn", [1, 9, 10, 11, 20, 21, 33])
+@pytest.mark.parametrize("given", [True, False])
+def test_lowpass_scan_over_whole_and_broken_groups_of_steps(Tn, given):
+    """The filter and its sweep back at both sides of the groups of steps that are requested together, into another buffer and in place,
+    with and without the optional operands, against the numpy restatement at the tolerance of the test above."""
+    from ksim_amd import _lib
+    from oracle import terms as ot
+
+    lib = _lib.load()
+    rng = np.random.default_rng(Tn)
+    M, nu, ld, dt, fc = 19, 5, 7, 0.02, 6.0
+    raw, obs, g = rng.normal(size=(Tn, M, ld)), rng.normal(size=(Tn, M, 3)), rng.normal(size=(Tn, M, ld))
+    bias, y0, fresh = rng.normal(size=nu) * 0.2, rng.normal(size=(M, nu)), rng.random((Tn, M)) < 0.2
+    x = raw[..., :nu] + (bias if given else 0.0)
+    if given:
+        x[..., 1:4] += obs
+    none = np.zeros_like(fresh)
+    want, want_last = ot.lowpass_scan(x, dt, fc, y0 if given else np.zeros_like(y0), fresh if given else none)
+    d_obs, d_bias, d_y0, d_f = t32(obs), t32(bias), t32(y0), torch.tensor(fresh, dtype=torch.uint8, device=DEV)
+    opt = (_lib.ptr(d_bias), _lib.ptr(d_obs), 3, 1, 3, _lib.ptr(d_y0), _lib.ptr(d_f)) if given else (None, None, 0, 0, 0, None, None)
+    for in_place in (False, True):
+        src, last = t32(raw), torch.empty(M, nu, device=DEV)
+        out = src if in_place else torch.empty_like(src)
+        _lib.check(lib.ks_lowpass_scan(_lib.current_stream(), Tn, M, nu, ld, dt, fc, _lib.ptr(src), *opt, _lib.ptr(out), _lib.ptr(last)))
+        np.testing.assert_allclose(out.cpu().numpy()[..., :nu], want, rtol=2e-5, atol=2e-6)
+        assert np.array_equal(out.cpu().numpy()[..., nu:], raw[..., nu:].astype(np.float32))
+        np.testing.assert_allclose(last.cpu().numpy(), want_last, rtol=2e-5, atol=2e-6)
+    want_dx, want_dy0 = ot.lowpass_scan_backward(g[..., :nu], dt, fc, fresh if given else none)
+    d_g, d_d = t32(g), torch.empty(M, nu, device=DEV)
+    _lib.check(lib.ks_lowpass_scan_backward(_lib.current_stream(), Tn, M, nu, ld, dt, fc, _lib.ptr(d_f) if given else None, _lib.ptr(d_g), _lib.ptr(d_d)))
+    np.testing.assert_allclose(d_g.cpu().numpy()[..., :nu], want_dx, rtol=2e-5, atol=2e-6)
+    np.testing.assert_allclose(d_d.cpu().numpy(), want_dy0, rtol=2e-5, atol=2e-6)
+
+
 @pytest.mark.parametrize("symmetric", [False, True])
 def test_kbot_training_step_with_filter_and_mirror_carries_matches_oracle(symmetric):
     """The K-Bot task's minibatch step as shipped (examples/kbot/train.py:903-934, 1439-1533): LSTM actor whose biased means
