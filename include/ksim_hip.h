@@ -724,6 +724,17 @@ int ks_mlp_forward(const KsMlp* mlp, ks_stream_t stream, int64_t M, const float*
  * below 16384, or are single bf16 layers that take the same row tile, they share a single launch, so the second network's workgroups overlap the first one's. */
 int ks_mlp_forward_pair(const KsMlp* mlp0, const KsMlp* mlp1, ks_stream_t stream, int64_t M, const float* x0,
                         float* y0, const float* x1, float* y1, void* workspace0, void* workspace1);
+/* ks_mlp_forward_pair on an actor and a critic, and ks_sample_action on the actor's output, in the same launch where the two networks share one:
+ * same results as the two calls. */
+typedef struct KsActionSample {
+  const float* log_std;      /* (nu), NULL: the mean */
+  const float* noise_normal; /* (M, nu), NULL: drawn from rng */
+  KsRng rng;
+  float clip_max;
+  float* action; /* (M, nu) out */
+} KsActionSample;
+int ks_mlp_forward_pair_sample(const KsMlp* actor, const KsMlp* critic, ks_stream_t stream, int64_t M, const float* x0, float* y0, const float* x1,
+                               float* y1, void* workspace0, void* workspace1, const KsActionSample* sample /*host*/);
 
 /* ------------------------------------------------------------------ GRU cell (recurrent policies, forward)
  * The recurrent actors / critics of the shipped examples (examples/walking.py:40-208: input projection, a stack of

@@ -184,6 +184,10 @@ class KsLstmDesc(ctypes.Structure):
                 ("weight_hh", c_void_p), ("bias", c_void_p)]
 
 
+class KsActionSample(ctypes.Structure):
+    _fields_ = [("log_std", c_void_p), ("noise_normal", c_void_p), ("rng", KsRng), ("clip_max", c_float), ("action", c_void_p)]
+
+
 class KsLayerBackward(ctypes.Structure):
     _fields_ = [("mlp", c_void_p), ("M", c_int64), ("x", c_void_p), ("ldx", c_int64), ("dy", c_void_p), ("dx", c_void_p)]
 
@@ -247,6 +251,8 @@ def bind(lib) -> None:
     lib.ks_mlp_forward.argtypes = [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]
     lib.ks_mlp_forward_pair.argtypes = [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                                         c_void_p, c_void_p]
+    lib.ks_mlp_forward_pair_sample.argtypes = [c_void_p, c_void_p, c_void_p, c_int64] + [c_void_p] * 6 + [POINTER(KsActionSample)]
+    lib.ks_mlp_forward_pair_sample.restype = c_int32
     lib.ks_mlp_train_init.argtypes = [c_void_p]
     lib.ks_mlp_train_workspace_bytes.argtypes = [c_void_p, c_int64]
     lib.ks_mlp_train_workspace_bytes.restype = c_int64

@@ -42,4 +42,21 @@ __device__ inline Philox4 draw(uint64_t seed, uint64_t step, int purpose, uint64
                        (uint32_t)seed, (uint32_t)(seed >> 32) ^ (uint32_t)(step >> 32));
 }
 
+// action = mean + exp(log_std) N(0, 1) of element u of env e, scrubbed and clipped (ksim/task/rl.py:998-1001)
+__device__ __forceinline__ float sampled_action(float mean, const float* __restrict__ log_std, const float* __restrict__ noise, const KsRng& rng, float clip_max,
+                                                int64_t e, int u, int64_t idx) {
+  float a = mean;
+  if (log_std) {
+    float z;
+    if (noise) z = noise[idx];
+    else {
+      const Philox4 r = draw(rng.seed, rng.step + (rng.step_base ? *rng.step_base : 0ull), kRngAction, (uint64_t)e, (uint32_t)u);
+      z = normal_from(r.x, r.y);
+    }
+    a += expf(log_std[u]) * z;
+  }
+  if (a != a) a = 0.f;                       // NaN -> 0, rl.py:999-1000
+  return fminf(fmaxf(a, -clip_max), clip_max);  // rl.py:1001
+}
+
 }  // namespace ks

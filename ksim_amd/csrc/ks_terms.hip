@@ -499,19 +499,7 @@ __global__ __launch_bounds__(256) void sample_action_kernel(int64_t n, int nu, c
   if (idx >= n) return;
   const int64_t e = idx / nu;
   const int u = (int)(idx - e * nu);
-  float a = mean[idx];
-  if (log_std) {
-    float z;
-    if (noise) z = noise[idx];
-    else {
-      const Philox4 r = draw(rng.seed, rng.step + (rng.step_base ? *rng.step_base : 0ull), kRngAction, (uint64_t)e, (uint32_t)u);
-      z = normal_from(r.x, r.y);
-    }
-    a += expf(log_std[u]) * z;
-  }
-  if (a != a) a = 0.f;                         // NaN -> 0, rl.py:999-1000
-  a = fminf(fmaxf(a, -clip_max), clip_max);    // rl.py:1001
-  action[idx] = a;
+  action[idx] = sampled_action(mean[idx], log_std, noise, rng, clip_max, e, u, idx);
 }
 
 // Gaussian head with a state-dependent standard deviation: the network emits (mean, raw std) per actuator.

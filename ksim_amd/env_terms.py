@@ -290,21 +290,27 @@ class EnvTerms:
             pass
 
 
+def action_sample(mean: torch.Tensor, log_std: torch.Tensor | None, *, noise: torch.Tensor | None = None, seed: int = 0, step: int = 0, step_base=None,
+                  clip_max: float = 1e3, out: torch.Tensor) -> T.KsActionSample:
+    """The operands of `sample_action`, checked, for the launch that makes the mean (`MLP.forward_pair`)."""
+    _lib.require_cuda(mean, log_std, noise, out, dtype=torch.float32)
+    if log_std is not None and tuple(log_std.shape) != (mean.shape[1],):
+        raise _lib.KsError("log_std must have shape (nu,)")
+    if noise is not None and noise.shape != mean.shape:
+        raise _lib.KsError("noise must match the mean's shape")
+    return T.KsActionSample(_lib.addr(log_std), _lib.addr(noise), _rng(seed, step, step_base), float(clip_max), _lib.addr(out))
+
+
 def sample_action(mean: torch.Tensor, log_std: torch.Tensor | None, *, noise: torch.Tensor | None = None,
                   seed: int = 0, step: int = 0, step_base=None, clip_max: float = 1e3,
                   out: torch.Tensor | None = None):
     """action = mean + exp(log_std) * N(0,1); NaN -> 0; clip to +-clip_max (ksim/task/rl.py:998-1001)."""
     lib = _lib.load()
-    _lib.require_cuda(mean, log_std, noise, out, dtype=torch.float32)
-    N, nu = mean.shape
-    if log_std is not None and tuple(log_std.shape) != (nu,):
-        raise _lib.KsError("log_std must have shape (nu,)")
-    if noise is not None and noise.shape != mean.shape:
-        raise _lib.KsError("noise must match the mean's shape")
     if out is None:
         out = torch.empty_like(mean)
-    _lib.check(lib.ks_sample_action(_lib.current_stream(), N, nu, _lib.addr(mean), _lib.addr(log_std), _lib.addr(noise),
-                                    _rng(seed, step, step_base), float(clip_max), _lib.addr(out)))
+    args = action_sample(mean, log_std, noise=noise, seed=seed, step=step, step_base=step_base, clip_max=clip_max, out=out)
+    N, nu = mean.shape
+    _lib.check(lib.ks_sample_action(_lib.current_stream(), N, nu, _lib.addr(mean), args.log_std, args.noise_normal, args.rng, args.clip_max, args.action))
     return out
 
 

@@ -83,8 +83,9 @@ class MLP:
         return out
 
     def forward_pair(self, x: torch.Tensor, out: torch.Tensor, other: "MLP", x_other: torch.Tensor,
-                     out_other: torch.Tensor) -> None:
-        """This network on ``x`` and ``other`` on ``x_other`` (same row count), in one launch when the library can."""
+                     out_other: torch.Tensor, sample: "T.KsActionSample | None" = None) -> None:
+        """This network on ``x`` and ``other`` on ``x_other`` (same row count), in one launch when the library can; with ``sample``
+        (`env_terms.action_sample`) also the actions of this network's output."""
         M = x.shape[0]
         for net, a, o in ((self, x, out), (other, x_other, out_other)):
             _lib.require_cuda(a, dtype=torch.float32)
@@ -92,9 +93,9 @@ class MLP:
             if tuple(a.shape) != (M, net.in_dim) or tuple(o.shape) != (M, net.out_dim):
                 raise _lib.KsError(f"expected input (M, {net.in_dim}) and output (M, {net.out_dim})")
         ws, ws_other = self.workspace(M, x.device), other.workspace(M, x.device)  # both held until both are launched
-        _lib.check(self._lib.ks_mlp_forward_pair(self._handle, other._handle, _lib.current_stream(), M, _lib.addr(x),
-                                                 _lib.addr(out), _lib.addr(x_other), _lib.addr(out_other), _lib.addr(ws),
-                                                 _lib.addr(ws_other)))
+        args = (self._handle, other._handle, _lib.current_stream(), M, _lib.addr(x), _lib.addr(out), _lib.addr(x_other), _lib.addr(out_other),
+                _lib.addr(ws), _lib.addr(ws_other))
+        _lib.check(self._lib.ks_mlp_forward_pair(*args) if sample is None else self._lib.ks_mlp_forward_pair_sample(*args, ctypes.byref(sample)))
 
     # ------------------------------------------------------------------ training (ksim/task/ppo.py:495-565)
     def train_init(self) -> None:

@@ -19,7 +19,7 @@ from . import ppo as ppo_mod
 from .actions import LowPass
 from .commands import CommandSet
 from .engine import HipEngine
-from .env_terms import EnvTerms, sample_action, sample_action_head, sample_action_mixture
+from .env_terms import EnvTerms, action_sample, sample_action, sample_action_head, sample_action_mixture
 from .mlp import MLP
 from .physics import DeviceModel
 from .recurrent import RecurrentNetwork
@@ -192,9 +192,13 @@ class Rollout:
                 if self.critic_carry0 is not None:
                     self.critic_carry0.copy_(env.critic_carry)
         critic_joined = True
-        if isinstance(c.actor, MLP) and isinstance(c.critic, MLP):
-            # two plain MLPs over the same rows share one launch
-            c.actor.forward_pair(self.noisy_obs[t], self.mean, c.critic, self.obs[t], self.values[t])
+        plain_head = not isinstance(c.head, (GaussianHead, MixtureHead))
+        sampling = dict(noise=noise.get("action_normal"), seed=env.seed, step=step, step_base=step_base, clip_max=c.action_clip_max, out=self.action[t])
+        paired = isinstance(c.actor, MLP) and isinstance(c.critic, MLP)
+        if paired:
+            # two plain MLPs over the same rows share one launch, and the actions of a plain head are made in it
+            c.actor.forward_pair(self.noisy_obs[t], self.mean, c.critic, self.obs[t], self.values[t],
+                                 action_sample(self.mean, c.log_std, **sampling) if plain_head else None)
         else:
             def run_critic() -> None:
                 if isinstance(c.critic, RecurrentNetwork):
@@ -243,9 +247,8 @@ class Rollout:
                                   var_scale=c.head.var_scale, mean_bias=c.head.mean_bias, clip_lo=c.head.clip_lo,
                                   clip_hi=c.head.clip_hi, uniform=noise.get("action_uniform"), noise=noise.get("action_normal"),
                                   seed=env.seed, step=step, step_base=step_base, clip_max=c.action_clip_max, out=self.action[t])
-        else:
-            sample_action(self.mean, c.log_std, noise=noise.get("action_normal"), seed=env.seed, step=step,
-                          step_base=step_base, clip_max=c.action_clip_max, out=self.action[t])
+        elif not paired:
+            sample_action(self.mean, c.log_std, **sampling)
         # the step kernel also writes ctrl / xpos / xquat of the post-step data into the transition slot
         c.engine.step(self.action[t], c.physics_model, ps, level, env.seed + env.step, env.randomization_dict,
                       noise=noise.get("engine"), record=dict(ctrl=self.ctrl[t], xpos=self.xpos[t], xquat=self.xquat[t]),

@@ -480,3 +480,32 @@ def test_single_layers_in_shared_launches_match_one_by_one(M):
     run_layers(forward)
     for call in forward:
         assert torch.equal(call.out, call.net(call.x)), (call.net.dims, call.net.dtype)
+
+
+@pytest.mark.parametrize("hidden,dtype,act,M", [(256, "bf16", "elu", 1), (256, "bf16", "elu", 64), (256, "f32", "tanh", 37), (128, "bf16", "relu", 4099), (512, "bf16", "elu", 64),
+                                                (512, "f32", "elu", 45), (256, "f32", "elu", 2500), (64, "bf16", "elu", 16383), (64, "bf16", "elu", 16390)])
+def test_actions_sampled_in_the_networks_launch_match_the_launch_of_their_own(hidden, dtype, act, M):
+    """Actor, critic and actions in one call against `forward_pair` and `sample_action`, bit for bit: every form of the pair's launch (the last
+    rows of a tile, few rows of a wide network, rows beyond the pair's limit), drawn, given and no noise, a step counted on the device,
+    means that are clipped or not a number."""
+    from ksim_amd.env_terms import action_sample, sample_action
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    nets = []
+    for out in (20, 1):
+        dims = (68, hidden, hidden, hidden, out)
+        nets.append(MLP([rng.normal(scale=i ** -0.5, size=(o, i)) for i, o in zip(dims[:-1], dims[1:])], [0.1 * rng.normal(size=o) for o in dims[1:]],
+                        activation=act, dtype=dtype))
+    actor, critic = nets
+    t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    xa, xc, log_std, noise, base = t(M, 68), t(M, 68), t(20), t(M, 20), torch.tensor([5], dtype=torch.int64, device="cuda")
+    xa[M // 2, 3] = float("nan")
+    for given in (dict(log_std=log_std, seed=11, step=3), dict(log_std=log_std, seed=11, step=3, step_base=base), dict(log_std=log_std, noise=noise), dict(log_std=None)):
+        got, want = [[torch.full(s, 7.0, device="cuda") for s in ((M, 20), (M, 1), (M, 20))] for _ in range(2)]
+        actor.forward_pair(xa, want[0], critic, xc, want[1])
+        sample_action(want[0], clip_max=0.75, out=want[2], **given)
+        actor.forward_pair(xa, got[0], critic, xc, got[1], action_sample(got[0], clip_max=0.75, out=got[2], **given))
+        for g, w in zip(got, want):
+            assert torch.equal(torch.nan_to_num(g, nan=123.0), torch.nan_to_num(w, nan=123.0)), (g.shape, given.keys())
+        assert bool(torch.isfinite(got[2]).all()) and got[2].abs().max().item() <= 0.75
