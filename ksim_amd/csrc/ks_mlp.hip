@@ -1269,7 +1269,8 @@ void mlp_split_layer_kernel(const SplitLayer p, const SplitLayer q) {
 // gradient, one partial row per tile).
 // Bound by the products (58 us at the rate of a large product) and the tile's way in and out of memory (80 at the copy rate), which a single
 // workgroup per CU does one after the other.  65536 rows of 68-512-512-512-20: 174 -> 157 us (203 -> 185 just behind other kernels) since
-// activations and gradients move as whole rows; as transposes every lane loaded and stored 2 bytes at a time.  Column sums over half the rows
+// activations and gradients move as whole rows; as transposes every lane loaded and stored 2 bytes at a time.  167 -> 146 between other kernels
+// since no load stands behind a condition: the entry's tile was 32 loads one after the other and a layer's activations three groups.  Column sums over half the rows
 // a thread would keep all wavefronts busy with them, but their partial rows cost the final sum more than that gains.
 struct FusedBwdArgs {
   int64_t M;
@@ -1292,12 +1293,25 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tile = blockIdx.x, m0 = tile * BM;
   const int lda = a.lda, L = a.n_layers;
-  {  // the last layer's gradient tile from the caller's fp32 rows; zero in the padding columns and beyond the batch (such rows
-     // stay zero through every layer)
+  {  // the last layer's gradient tile from the caller's fp32 rows, which are one piece of memory; zero in the padding columns and beyond the
+     // batch (such rows stay zero through every layer).  Eight entries of a thread are requested at a time.
     const int np = a.np_last, od = a.out_dim;
-    for (int idx = tid; idx < BM * np; idx += NTHR) {
-      const int r = idx / np, c = idx - r * np;
-      act[r * lda + c] = (__bf16)((c < od && m0 + r < a.M) ? a.dy[(m0 + r) * od + c] : 0.f);
+    for (int idx = tid; idx < BM * (np / 8); idx += NTHR)
+      *reinterpret_cast<u32x4*>(act + (idx / (np / 8)) * lda + idx % (np / 8) * 8) = u32x4{0u, 0u, 0u, 0u};
+    const int held = (int)(a.M - m0 < BM ? a.M - m0 : BM) * od;  // at least one row
+    const float* dy = a.dy + m0 * od;
+    __syncthreads();
+    for (int first = tid; first < held; first += 8 * NTHR) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = dy[min(first + u * NTHR, held - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(v[u]));  // keeps the loads out of the conditions below
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int at = first + u * NTHR, r = at / od;
+        if (at < held) act[r * lda + at - r * od] = (__bf16)v[u];
+      }
     }
   }
   __syncthreads();
@@ -1307,7 +1321,7 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     out = TileRowsOut<__bf16, BM>(act, lda, dst, width, width, m0, m0 + BM);
     if (tid >= width / 2) return;
     f32x2 cs = {0.f, 0.f};
-#pragma unroll 8
+#pragma unroll 32
     for (int r = 0; r < BM; ++r) {
       const bf16x2 v = *reinterpret_cast<const bf16x2*>(act + r * lda + 2 * tid);
       cs[0] += (float)v[0]; cs[1] += (float)v[1];
@@ -1339,18 +1353,18 @@ void mlp_fused_bwd_kernel(const FusedBwdArgs a) {
     // Y_{l-1} takes dZ_l's place in the tile on its way to the lanes that need it, and every lane leaves dZ_{l-1} where it read Y: whole rows in
     // 16-byte pieces in and out of memory, 8 bytes per lane of the tile.
     const int width = nt * 32, pieces = width / 8, per = NTHR / pieces, yr = tid / pieces, yc = (tid - yr * pieces) * 8;
+    // Requested without a condition, the row held back to the last one: behind conditions the loads were waited for in three groups, and each of
+    // them for the stores ahead of it.
+    const int rows = (int)(a.M - m0 < BM ? a.M - m0 : BM);
+    const __bf16* yt = a.y[l - 1] + m0 * width + yc;
     u32x4 yv[16];  // a width of 512: 8 rows a pass
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int r = yr + u * per;
-      yv[u] = u32x4{0u, 0u, 0u, 0u};
-      if (yr < per && r < BM && m0 + r < a.M) yv[u] = *reinterpret_cast<const u32x4*>(a.y[l - 1] + (m0 + r) * width + yc);
-    }
+    for (int u = 0; u < 16; ++u) yv[u] = *reinterpret_cast<const u32x4*>(yt + min(yr + u * per, rows - 1) * width);
     __syncthreads();  // every wavefront has read dZ_l
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const int r = yr + u * per;
-      if (yr < per && r < BM) *reinterpret_cast<u32x4*>(act + r * lda + yc) = yv[u];
+      if (yr < per && r < BM) *reinterpret_cast<u32x4*>(act + r * lda + yc) = r < rows ? yv[u] : u32x4{0u, 0u, 0u, 0u};
     }
     __syncthreads();
 #pragma unroll
