@@ -261,7 +261,7 @@ def update_model(policy: GaussianMlpPolicy, cfg: PPOUpdateConfig, actor_obs, cri
     # on-policy variables of the whole rollout with the pre-update parameters (ppo.py:603-607)
     on_lp, on_v, _, _ = get_ppo_variables(policy, actor_obs.reshape(Tn * N, -1), critic_obs.reshape(Tn * N, -1),
                                           action.reshape(Tn * N, nu))
-    on_lp, on_v = on_lp.view(Tn, N, nu).clone(), on_v.view(Tn, N).clone()
+    on_lp, on_v = on_lp.view(Tn, N, nu), on_v.view(Tn, N)
     bs = min(cfg.batch_size, N)
     if N % bs:
         raise _lib.KsError("the env count must be a multiple of the batch size (ppo.py:647 reshapes the permutation)")
