@@ -281,7 +281,7 @@ class GRUCell:
     def parameters(self, gradients: bool = False) -> dict:
         """Copies of weight_ih, weight_hh, bias (3H) and bias_n (H), or of their gradients."""
         ((wi, bi),), ((wh, bh),) = mlp_mod.copy_parameters((self.proj_i, self.proj_h), gradients)
-        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:])
+        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:].clone())
 
     def __del__(self):
         h = getattr(self, "_handle", None)
