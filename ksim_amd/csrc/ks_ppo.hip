@@ -813,19 +813,26 @@ struct PpoGradIO {
   float* d_value;
 };
 
+// What a thread needs of its row (thread r takes row row0 + r; a thread without one reads the last), requested ahead of the pairs' work.
+struct PpoRow {
+  float adv, v, on_v, tgt;
+};
+__device__ __forceinline__ PpoRow row_fetch(const PpoGradIO& io, int64_t M, int64_t row0, int rows) {
+  const int64_t m = min(row0 + min((int)threadIdx.x, rows - 1), M - 1);
+  return {io.adv[m], io.v[m], io.on_v[m], io.tgt[m]};
+}
+
 // sel[r] <- gradient factor of row row0 + r from the per-pair differences el[r * nu + a]; also writes the rows' value gradients.
-// Barriers on both sides; every thread of the workgroup calls it.
-__device__ __forceinline__ void row_factors(const PpoGradIO& io, const KsPpoLossParams& p, float kl_scale, float inv_m, int64_t M, int64_t row0,
-                                            int rows, int nu, const float* el, float* sel) {
+// Barriers on both sides; every thread of the workgroup calls it, which has at least as many threads as rows.
+__device__ __forceinline__ void row_factors(const PpoRow& in, float* __restrict__ d_value, const KsPpoLossParams& p, float kl_scale, float inv_m, int64_t M,
+                                            int64_t row0, int rows, int nu, const float* el, float* sel) {
   __syncthreads();
-  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
-    const int64_t m = row0 + r;
-    if (m < M) {
-      float logr = 0.f;
-      for (int a = 0; a < nu; ++a) logr += el[r * nu + a];
-      sel[r] = surrogate_grad(p, kl_scale, logr, io.adv[m], inv_m);
-      io.d_value[m] = value_grad(p, io.v[m], io.on_v[m], io.tgt[m], inv_m);
-    }
+  const int r = threadIdx.x;
+  if (r < rows && row0 + r < M) {
+    float logr = 0.f;
+    for (int a = 0; a < nu; ++a) logr += el[r * nu + a];
+    sel[r] = surrogate_grad(p, kl_scale, logr, in.adv, inv_m);
+    d_value[row0 + r] = value_grad(p, in.v, in.on_v, in.tgt, inv_m);
   }
   __syncthreads();
 }
@@ -833,7 +840,9 @@ __device__ __forceinline__ void row_factors(const PpoGradIO& io, const KsPpoLoss
 // Gaussian with one log deviation per action.  The log-std gradient of a thread's action is accumulated in its register over the
 // workgroup's rows (blockDim.x / nu whole rows at a time, so a thread keeps its action), then over the threads in a fixed order:
 // block partials, then ppo_grad_finish_kernel, so the result does not depend on scheduling.  1024 threads: at most 256 workgroups
-// (the partials' buffer) still keep 16 wavefronts per CU in flight (65536 rows x 20 actions: 36 -> 19 us).
+// (the partials' buffer) still keep 16 wavefronts per CU in flight (65536 rows x 20 actions: 36 -> 19 us).  The next rows' pairs are
+// requested as soon as these are used up and the row's own values ahead of the pairs': a workgroup walks its rows a launch's width apart, five
+// times there, and waited for memory twice each time (19.6 -> 12.0 us).
 __global__ __launch_bounds__(1024) void ppo_loss_grad_kernel(int64_t M, int nu, KsPpoLossParams p, const float* __restrict__ mean,
                                                             const float* __restrict__ log_std, PpoGradIO io, float* __restrict__ d_mean,
                                                             float* __restrict__ partial) {
@@ -842,16 +851,24 @@ __global__ __launch_bounds__(1024) void ppo_loss_grad_kernel(int64_t M, int nu, 
   const bool mine = r < rows;
   const float inv_m = 1.0f / (float)M, kl_scale = kl_scale_of(p), g_ent = -p.entropy_coef * inv_m;
   const float ls = mine ? log_std[a] : 0.f, is = __expf(-ls);
-  float dls = 0.f;
-  for (int64_t row0 = (int64_t)blockIdx.x * rows; row0 < M; row0 += (int64_t)gridDim.x * rows) {
+  float dls = 0.f, f_action, f_mean, f_on_lp;
+  auto fetch = [&](int64_t row0) __attribute__((always_inline)) {
+    const int64_t i = min(row0 * nu + threadIdx.x, M * nu - 1);
+    f_action = io.action[i];
+    f_mean = mean[i];
+    f_on_lp = io.on_lp[i];
+  };
+  const int64_t first = (int64_t)blockIdx.x * rows, stride = (int64_t)gridDim.x * rows;
+  fetch(first);
+  PpoRow in = row_fetch(io, M, first, rows);
+  for (int64_t row0 = first; row0 < M; row0 += stride) {
     const bool ok = mine && row0 + r < M;
     const int64_t i = row0 * nu + threadIdx.x;  // the pairs of whole rows are contiguous
-    float z = 0.f;
-    if (ok) {
-      z = (io.action[i] - mean[i]) * is;
-      el[threadIdx.x] = (-0.5f * z * z - ls - kHalfLog2Pi) - io.on_lp[i];
-    }
-    row_factors(io, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
+    const float z = (f_action - f_mean) * is;
+    if (ok) el[threadIdx.x] = (-0.5f * z * z - ls - kHalfLog2Pi) - f_on_lp;
+    fetch(row0 + stride);
+    row_factors(in, io.d_value, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
+    in = row_fetch(io, M, row0 + stride, rows);
     if (ok) {
       const float g_lp = sel[r];
       d_mean[i] = g_lp * z * is;
@@ -992,15 +1009,17 @@ __global__ __launch_bounds__(256) void ppo_loss_grad_pairs_kernel(int64_t M, int
     const int rows = 256 / nu, r = threadIdx.x / nu, a = threadIdx.x - r * nu;
     const int64_t row0 = (int64_t)blockIdx.x * rows, m = row0 + r;
     const bool ok = r < rows && m < M;
+    const PpoRow in = row_fetch(io, M, row0, rows);
     if (ok) el[threadIdx.x] = pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]) - io.on_lp[m * nu + a];
-    row_factors(io, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
+    row_factors(in, io.d_value, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
     if (ok) pair.grad(hd, sel[r], g_ent, m, a, nu, d_raw);
   } else {
     const int64_t m = blockIdx.x;
+    const PpoRow in = row_fetch(io, M, m, 1);
     float part = 0.f;
     for (int a = threadIdx.x; a < nu; a += 256) part += pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]) - io.on_lp[m * nu + a];
     el[threadIdx.x] = part;
-    row_factors(io, p, kl_scale, inv_m, M, m, 1, 256, el, sel);
+    row_factors(in, io.d_value, p, kl_scale, inv_m, M, m, 1, 256, el, sel);
     for (int a = threadIdx.x; a < nu; a += 256) {
       pair.eval(hd, raw, m, a, nu, io.action[m * nu + a]);
       pair.grad(hd, sel[0], g_ent, m, a, nu, d_raw);
