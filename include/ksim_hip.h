@@ -914,6 +914,9 @@ int ks_mlp_get_all_params(const KsMlp* mlp, ks_stream_t stream, float* out /*dev
 int ks_mlp_copy_params(const KsMlp* mlp, ks_stream_t stream, float* const* weights, float* const* biases, int32_t gradients);
 /* The same for `count` networks, whose layers follow one another in the tables. */
 int ks_mlps_copy_params(const KsMlp* const* mlps, int32_t count, ks_stream_t stream, float* const* weights, float* const* biases, int32_t gradients);
+/* The same, of every bias only the entries from bias_first[layer] (host table, nullable: all) to the end. */
+int ks_mlps_copy_params_from(const KsMlp* const* mlps, int32_t count, ks_stream_t stream, float* const* weights, float* const* biases,
+                             const int32_t* bias_first, int32_t gradients);
 
 /* Backward pass through time of a GRU stack (the jax.grad through the lax.scan over the trajectory in
  * PPOTask._single_step, ksim/task/ppo.py:572-694, for the recurrent actors and critics of examples/walking.py:40-208).

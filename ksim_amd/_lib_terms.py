@@ -334,6 +334,8 @@ def bind(lib) -> None:
     lib.ks_mlp_copy_params.restype = c_int32
     lib.ks_mlps_copy_params.argtypes = [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int32]
     lib.ks_mlps_copy_params.restype = c_int32
+    lib.ks_mlps_copy_params_from.argtypes = [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32]
+    lib.ks_mlps_copy_params_from.restype = c_int32
     lib.ks_mlp_get_params.argtypes = [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32]
     lib.ks_gaussian_log_prob.argtypes = [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     for name in ("ks_mlp_train_init", "ks_mlp_train_forward", "ks_mlp_train_backward", "ks_grad_sqnorm",

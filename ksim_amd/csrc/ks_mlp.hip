@@ -4383,14 +4383,17 @@ extern "C" int64_t ks_mlp_param_floats(const KsMlp* h, int32_t layer) {
   return off;
 }
 
-extern "C" int ks_mlps_copy_params(const KsMlp* const* nets, int32_t count, ks_stream_t stream, float* const* weights, float* const* biases,
-                                   int32_t gradients) {
+extern "C" int ks_mlps_copy_params_from(const KsMlp* const* nets, int32_t count, ks_stream_t stream, float* const* weights, float* const* biases,
+                                        const int32_t* bias_first, int32_t gradients) {
   if (count < 0 || (count > 0 && (!nets || !weights || !biases))) return fail(KS_EINVAL, "ks_mlp_copy_params: null pointer");
   int at = 0;  // layer in the tables
   for (int k = 0; k < count; ++k) {
     if (!nets[k] || !nets[k]->m.train) return fail(KS_EINVAL, "ks_mlp_copy_params: call ks_mlp_train_init first");
-    for (int l = 0; l < nets[k]->m.n_layers; ++l, ++at)
+    for (int l = 0; l < nets[k]->m.n_layers; ++l, ++at) {
       if (!weights[at] || !biases[at]) return fail(KS_EINVAL, "ks_mlp_copy_params: layer %d has no destination", l);
+      if (bias_first && (bias_first[at] < 0 || bias_first[at] >= nets[k]->m.dims[l + 1]))
+        return fail(KS_EINVAL, "ks_mlp_copy_params: layer %d has no bias %d", l, (int)bias_first[at]);
+    }
   }
   at = 0;
   for (int k = 0; k < count;) {  // as many networks at a time as the table holds
@@ -4402,9 +4405,10 @@ extern "C" int ks_mlps_copy_params(const KsMlp* const* nets, int32_t count, ks_s
       for (int l = 0; l < m.n_layers; ++l, ++at) {
         const int o = m.dims[l + 1], i = m.dims[l], w = a.n, b = a.n + 1;
         a.rows[w] = o; a.cols[w] = i; a.ld[w] = m.kpad[l]; a.src[w] = gradients ? m.gW[l] : m.mW[l]; a.dst[w] = weights[at];
-        a.rows[b] = 1; a.cols[b] = o; a.ld[b] = o; a.src[b] = gradients ? m.gb[l] : m.mb[l]; a.dst[b] = biases[at];
+        const int f = bias_first ? bias_first[at] : 0, nb = o - f;
+        a.rows[b] = 1; a.cols[b] = nb; a.ld[b] = nb; a.src[b] = (gradients ? m.gb[l] : m.mb[l]) + f; a.dst[b] = biases[at];
         a.first_block[w] = blocks; blocks += (int)(((int64_t)o * i + 255) / 256);
-        a.first_block[b] = blocks; blocks += (o + 255) / 256;
+        a.first_block[b] = blocks; blocks += (nb + 255) / 256;
         a.n += 2;
       }
     }
@@ -4412,6 +4416,11 @@ extern "C" int ks_mlps_copy_params(const KsMlp* const* nets, int32_t count, ks_s
     hipLaunchKernelGGL(unpad_net_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
   }
   return check_launch("ks_mlp_copy_params");
+}
+
+extern "C" int ks_mlps_copy_params(const KsMlp* const* nets, int32_t count, ks_stream_t stream, float* const* weights, float* const* biases,
+                                   int32_t gradients) {
+  return ks_mlps_copy_params_from(nets, count, stream, weights, biases, nullptr, gradients);
 }
 
 extern "C" int ks_mlp_copy_params(const KsMlp* h, ks_stream_t stream, float* const* weights, float* const* biases, int32_t gradients) {

@@ -280,8 +280,14 @@ class GRUCell:
 
     def parameters(self, gradients: bool = False) -> dict:
         """Copies of weight_ih, weight_hh, bias (3H) and bias_n (H), or of their gradients."""
-        ((wi, bi),), ((wh, bh),) = mlp_mod.copy_parameters((self.proj_i, self.proj_h), gradients)
-        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bh[2 * self.hidden_size:].clone())
+        H, empty, f32, dev = self.hidden_size, torch.empty, torch.float32, torch.device("cuda", torch._C._cuda_getDevice())
+        wi, wh = empty((3 * H, self.input_size), dtype=f32, device=dev), empty((3 * H, H), dtype=f32, device=dev)
+        bi, bn = empty((3 * H,), dtype=f32, device=dev), empty((H,), dtype=f32, device=dev)
+        pair = ctypes.c_void_p * 2  # of the hidden projection's bias only the new gate's entries hold anything
+        _lib.check(self._lib.ks_mlps_copy_params_from(pair(self.proj_i._handle, self.proj_h._handle), 2, _lib.current_stream(),
+                                                      pair(wi.data_ptr(), wh.data_ptr()), pair(bi.data_ptr(), bn.data_ptr()),
+                                                      (ctypes.c_int32 * 2)(0, 2 * H), int(gradients)))
+        return dict(weight_ih=wi, weight_hh=wh, bias=bi, bias_n=bn)
 
     def __del__(self):
         h = getattr(self, "_handle", None)

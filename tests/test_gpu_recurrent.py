@@ -500,3 +500,28 @@ def test_lstm_sequences_write_the_outputs_they_are_given_and_no_others(rows, ste
         run_sequences(calls)
         for g, w in pairs:
             assert torch.equal(g, w), (k, tuple(w.shape))
+
+
+@pytest.mark.parametrize("inputs,hidden", [(4, 1), (5, 85), (130, 128), (7, 171), (3, 256), (9, 300)])
+def test_parameters_of_a_gru_cell_as_they_were_given(inputs, hidden):
+    """The hidden projection's bias leaves from its last third on: inside, at and past the edge of a block."""
+    import ctypes
+
+    from ksim_amd import _lib
+    from ksim_amd.recurrent import GRUCell
+
+    rng = np.random.default_rng(hidden)
+    given = {k: rng.normal(size=n).astype(np.float32) for k, n in
+             dict(weight_ih=(3 * hidden, inputs), weight_hh=(3 * hidden, hidden), bias=3 * hidden, bias_n=hidden).items()}
+    cell = GRUCell(**given, dtype="f32")
+    cell.train_init()
+    got = cell.parameters()
+    assert got.keys() == given.keys()
+    for k, v in given.items():
+        assert np.array_equal(got[k].cpu().numpy(), v) and got[k]._base is None
+    out = torch.empty(3 * hidden * max(inputs, hidden), device="cuda")
+    one = lambda x: (ctypes.c_void_p * 1)(x)
+    for first in (-1, 3 * hidden):
+        with pytest.raises(_lib.KsError):
+            _lib.check(cell._lib.ks_mlps_copy_params_from(one(cell.proj_h._handle), 1, _lib.current_stream(), one(out.data_ptr()), one(out.data_ptr()),
+                                                          (ctypes.c_int32 * 1)(first), 0))
