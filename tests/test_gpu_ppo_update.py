@@ -952,6 +952,13 @@ def test_rows_and_their_mirror_images_in_one_pass(groups, group, n):
     assert torch.equal(out, torch.cat([x, image], dim=1)) and torch.equal(alone, image)
 
 
+@pytest.mark.parametrize("n", [2, 4, 512, 516, 1021, 1024, 1025, 2049])
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 8, 9, 1025])
+def test_mirror_images_where_a_workgroup_ends(rows, n):
+    """Rows on both sides of a workgroup's four and eight, a row that fills the workgroup's threads and one that takes them twice."""
+    test_rows_and_their_mirror_images_in_one_pass(1, rows, n)
+
+
 @pytest.mark.parametrize("dims,M", [((68, 512, 512, 20), 32768), ((40, 384, 512, 12), 32769), ((33, 512, 384, 256, 128, 1), 40000),
                                     ((7, 128, 128, 130), 65536 + 127)])
 def test_weight_gradients_of_whole_networks_are_exact_on_integers(dims, M):
