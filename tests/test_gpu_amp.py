@@ -347,3 +347,20 @@ def test_both_batches_of_a_step_in_one_launch(batch, envs, window_t, clips, clip
         assert torch.equal(one.get_state(), two.get_state())
     with pytest.raises(ValueError, match="must divide"):
         amp._batches(motions, torch.cat([sims, sims[:1]]) if batch > 1 else sims, 2 if batch == 1 else batch, torch.Generator())
+
+
+@pytest.mark.parametrize("device", ["meta", "cuda"])
+def test_indices_drawn_off_the_host_are_not_read_there(device, monkeypatch):
+    """Under a default device the draws are not host memory, which is where the launcher of both batches reads them: such a call goes to the
+    functions of the single batches, which refuse it."""
+    from ksim_amd import _lib, amp
+
+    class Library:
+        def __getattr__(self, name):
+            raise AssertionError(name)
+
+    motions, sims = torch.randn(3, 7, 5, device=DEV), torch.randn(4, 6, 5, device=DEV)
+    monkeypatch.setattr(_lib, "load", lambda: Library())
+    generator = torch.Generator(device="cpu" if device == "meta" else DEV)
+    with torch.device(device), pytest.raises(RuntimeError):
+        amp._batches(motions, sims, 2, generator)
