@@ -81,7 +81,8 @@ def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Gen
 
 def _batches(motions: torch.Tensor, sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> tuple[torch.Tensor, torch.Tensor]:
     """`make_real_batch` and `make_sim_batch` of one step, in one launch where both are plain fp32 arrays of frames on one GPU and what was drawn
-    is in host memory, where the launcher reads it (a default device and a generator of its kind draw elsewhere)."""
+    is in host memory, where the launcher reads it (a default device and a generator of its kind draw elsewhere).  Not while the stream is captured:
+    a graph would replay one step's draws for ever, and the functions of the single batches refuse that."""
     window_t = sim_motions.shape[1]
     clip_idx, starts = _draw_clips(motions, batch_b, generator)
     envs = _draw_envs(sim_motions.shape[0], batch_b, generator)
@@ -89,7 +90,8 @@ def _batches(motions: torch.Tensor, sim_motions: torch.Tensor, batch_b: int, gen
              and motions.dtype == sim_motions.dtype == torch.float32 and motions.is_cuda and motions.device == sim_motions.device
              and motions.is_contiguous() and sim_motions.is_contiguous() and motions.numel() > 0 and sim_motions.numel() > 0
              and (motions.shape[1] + window_t) * motions.shape[2] < 1 << 27
-             and motions.device.index == torch._C._cuda_getDevice() and all(i.device.type == "cpu" for i in (clip_idx, starts, envs)))
+             and motions.device.index == torch._C._cuda_getDevice() and all(i.device.type == "cpu" for i in (clip_idx, starts, envs))
+             and not torch.cuda.is_current_stream_capturing())
     if not plain:
         return _windows(motions, window_t, clip_idx, starts), _sequences(sim_motions, envs)
     n, t_clip, frame = motions.shape

@@ -364,3 +364,20 @@ def test_indices_drawn_off_the_host_are_not_read_there(device, monkeypatch):
     generator = torch.Generator(device="cpu" if device == "meta" else DEV)
     with torch.device(device), pytest.raises(RuntimeError):
         amp._batches(motions, sims, 2, generator)
+
+
+def test_batches_drawn_under_capture_are_left_to_the_functions_that_refuse_them(monkeypatch):
+    """A graph that held a step's draws would replay them for ever; the upload of the drawn indices is what no capture takes."""
+    from ksim_amd import amp
+
+    def windows(*args):
+        raise NotImplementedError("left to the single batches")
+
+    motions, sims = torch.randn(3, 7, 5, device=DEV), torch.randn(4, 6, 5, device=DEV)
+    monkeypatch.setattr(amp, "_windows", windows)
+    with pytest.raises(NotImplementedError), torch.cuda.graph(torch.cuda.CUDAGraph()):
+        sims + 1.0
+        amp._batches(motions, sims, 2, torch.Generator())
+    monkeypatch.undo()
+    real, sim = amp._batches(motions, sims, 2, torch.Generator())
+    assert real.shape == sim.shape == (2, 6, 5)
