@@ -849,6 +849,7 @@ int ks_gather_columns(ks_stream_t stream, int32_t n, const KsGatherArray* arrays
  * clip clip[k] of motions (clips, clip_t, frame), wrapping round at the clip's end; sim_out the sequences env[k] of sim (envs, window_t, frame).
  * The drawn indices are host memory and are read before the call returns. */
 #define KS_WINDOWS 128
+#define KS_WINDOW_FLOATS (65535 * 2048) /* window_t * frame at most */
 int ks_gather_windows(ks_stream_t stream, int32_t batch, int64_t window_t, int64_t frame, int64_t clips, int64_t clip_t, int64_t envs,
                       const float* motions, const float* sim, const int64_t* clip /*host*/, const int64_t* start /*host*/,
                       const int64_t* env /*host*/, float* real_out, float* sim_out);

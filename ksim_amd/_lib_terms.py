@@ -197,7 +197,7 @@ class KsSequence(ctypes.Structure):
 
 
 KS_GATHER_ARRAYS = 24
-KS_WINDOWS = 128
+KS_WINDOWS, KS_WINDOW_FLOATS = 128, 65535 * 2048
 
 
 class KsGatherArray(ctypes.Structure):

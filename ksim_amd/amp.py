@@ -89,7 +89,7 @@ def _batches(motions: torch.Tensor, sim_motions: torch.Tensor, batch_b: int, gen
     plain = (1 <= batch_b <= T.KS_WINDOWS and motions.dim() == sim_motions.dim() == 3 and motions.shape[2] == sim_motions.shape[2]
              and motions.dtype == sim_motions.dtype == torch.float32 and motions.is_cuda and motions.device == sim_motions.device
              and motions.is_contiguous() and sim_motions.is_contiguous() and motions.numel() > 0 and sim_motions.numel() > 0
-             and (motions.shape[1] + window_t) * motions.shape[2] < 1 << 27
+             and (motions.shape[1] + window_t) * motions.shape[2] <= T.KS_WINDOW_FLOATS
              and motions.device.index == torch._C._cuda_getDevice() and all(i.device.type == "cpu" for i in (clip_idx, starts, envs))
              and not torch.cuda.is_current_stream_capturing())
     if not plain:

@@ -539,7 +539,7 @@ extern "C" int ks_gather_windows(ks_stream_t stream, int32_t batch, int64_t wind
   if (clip_t > 0x7fffffff || window_t > 0x7fffffff || frame > 0x7fffffff || (clip_t + window_t) * frame > 0x7fffffff - 2048)
     return fail(KS_ELIMIT, "ks_gather_windows: clips or windows too long");
   const int64_t floats = window_t * frame;
-  if ((floats + 2047) / 2048 > 65535) return fail(KS_ELIMIT, "ks_gather_windows: windows too long");
+  if (floats > KS_WINDOW_FLOATS) return fail(KS_ELIMIT, "ks_gather_windows: windows too long");  // a block per 2048 floats on the grid's y axis
   WindowTable t;
   for (int k = 0; k < batch; ++k) {
     if (clip[k] < 0 || clip[k] >= clips || start[k] < 0 || start[k] >= clip_t || env[k] < 0 || env[k] >= envs || clips > 0x7fffffff || envs > 0x7fffffff)

@@ -381,3 +381,15 @@ def test_batches_drawn_under_capture_are_left_to_the_functions_that_refuse_them(
     monkeypatch.undo()
     real, sim = amp._batches(motions, sims, 2, torch.Generator())
     assert real.shape == sim.shape == (2, 6, 5)
+
+
+@pytest.mark.parametrize("window_t", [134214, 134215, 134216])
+def test_windows_at_the_launch_limit(window_t):
+    """The longest windows that the launch takes, and those that it leaves to the functions of the single batches: 1000 floats a frame, a clip of one
+    frame, at most 65535 blocks of 2048 floats of clip and window."""
+    from ksim_amd import amp
+
+    motions, sims = torch.randn(1, 1, 1000, device=DEV), torch.randn(1, window_t, 1000, device=DEV)
+    one, two = torch.Generator().manual_seed(7), torch.Generator().manual_seed(7)
+    real, sim = amp._batches(motions, sims, 1, one)
+    assert torch.equal(real, amp.make_real_batch(motions, window_t, 1, two)) and torch.equal(sim, amp.make_sim_batch(sims, 1, two))
