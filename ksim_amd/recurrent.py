@@ -228,13 +228,15 @@ class GRUCell:
         return self._proj
 
     def sequence_call(self, x, h0, fresh, hs, saved, gi=None) -> "SequenceCall":
-        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`)."""
-        _lib.require_cuda(x, h0, hs, saved, dtype=torch.float32)
+        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`); `gi`: the projected input (T M, 3H),
+        where the caller has it."""
+        _lib.require_cuda(x, h0, hs, saved, gi, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
         if (tuple(x.shape) != (Tn, M, self.input_size) or tuple(h0.shape) != (M, H) or tuple(hs.shape) != (Tn, M, H)
-                or (saved is not None and tuple(saved.shape) != (Tn, M, 5 * H)) or tuple(fresh.shape) != (Tn, M)):
-            raise _lib.KsError("expected x (T, M, input), h0 (M, H), hs (T, M, H), saved (T, M, 5H), fresh (T, M)")
+                or (saved is not None and tuple(saved.shape) != (Tn, M, 5 * H)) or tuple(fresh.shape) != (Tn, M)
+                or (gi is not None and tuple(gi.shape) != (Tn * M, 3 * H))):
+            raise _lib.KsError("expected x (T, M, input), h0 (M, H), hs (T, M, H), saved (T, M, 5H), fresh (T, M), gi (T M, 3H)")
         if gi is None:
             gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
         return SequenceCall("ks_gru_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, None, fresh, saved, hs, None)
@@ -382,15 +384,16 @@ class LSTMCell:
         return self._proj
 
     def sequence_call(self, x, h0, c0, fresh, hs, cs, saved, gi=None) -> "SequenceCall":
-        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`); `gi`: the projected input, where
-        the caller has it."""
-        _lib.require_cuda(x, h0, c0, hs, cs, saved, dtype=torch.float32)
+        """`sequence_forward` up to the recurrence itself, whose launch the caller makes (`run_sequences`); `gi`: the projected input (T M, 4H),
+        where the caller has it."""
+        _lib.require_cuda(x, h0, c0, hs, cs, saved, gi, dtype=torch.float32)
         _lib.require_cuda(fresh, dtype=torch.uint8)
         Tn, M, H = x.shape[0], x.shape[1], self.hidden_size
         if (tuple(x.shape) != (Tn, M, self.input_size) or any(tuple(t.shape) != (M, H) for t in (h0, c0))
                 or any(t is not None and tuple(t.shape) != (Tn, M, H) for t in (hs, cs))
-                or (saved is not None and tuple(saved.shape) != (Tn, M, 7 * H)) or tuple(fresh.shape) != (Tn, M)):
-            raise _lib.KsError("expected x (T, M, input), h0, c0 (M, H), hs, cs (T, M, H), saved (T, M, 7H), fresh (T, M)")
+                or (saved is not None and tuple(saved.shape) != (Tn, M, 7 * H)) or tuple(fresh.shape) != (Tn, M)
+                or (gi is not None and tuple(gi.shape) != (Tn * M, 4 * H))):
+            raise _lib.KsError("expected x (T, M, input), h0, c0 (M, H), hs, cs (T, M, H), saved (T, M, 7H), fresh (T, M), gi (T M, 4H)")
         if gi is None:
             gi = self._input_projection()(x.reshape(Tn * M, self.input_size))
         return SequenceCall("ks_lstm_sequences_forward", self.dtype, Tn, M, self._handle, gi, h0, c0, fresh, saved, hs, cs)

@@ -525,3 +525,30 @@ def test_parameters_of_a_gru_cell_as_they_were_given(inputs, hidden):
         with pytest.raises(_lib.KsError):
             _lib.check(cell._lib.ks_mlps_copy_params_from(one(cell.proj_h._handle), 1, _lib.current_stream(), one(out.data_ptr()), one(out.data_ptr()),
                                                           (ctypes.c_int32 * 1)(first), 0))
+
+
+@pytest.mark.parametrize("kind", ["gru", "lstm"])
+def test_a_given_projected_input_is_checked(kind):
+    """Rows too few, rows of another width, another type, gaps between rows, host memory: nothing of this is handed to a launch."""
+    from ksim_amd import _lib
+    from ksim_amd.recurrent import GRUCell, LSTMCell, run_sequences
+
+    steps, rows, H, G = 3, 5, 128, 3 if kind == "gru" else 4
+    rng = np.random.default_rng(0)
+    w = [rng.normal(scale=H ** -0.5, size=s) for s in ((G * H, H), (G * H, H), (G * H,))]
+    cell = GRUCell(*w, rng.normal(size=H), dtype="f32") if kind == "gru" else LSTMCell(*w, dtype="f32")
+    x, fresh = torch.randn(steps, rows, H, device="cuda"), torch.zeros(steps, rows, dtype=torch.uint8, device="cuda")
+    carry = [torch.randn(rows, H, device="cuda") for _ in range(1 if kind == "gru" else 2)]
+
+    def call(gi):
+        outs = [torch.empty(steps, rows, H, device="cuda") for _ in carry]
+        return cell.sequence_call(x, *carry, fresh, *outs, None, gi), outs
+
+    good = cell._input_projection()(x.view(steps * rows, H))
+    for bad in (good[:-1], good[:, :-1].contiguous(), good.view(steps, rows, G * H), good.double(), good.half(), torch.cat([good, good], 1)[:, : G * H], good.cpu()):
+        with pytest.raises(_lib.KsError):
+            call(bad)
+    (given, got), (own, want) = call(good), call(None)
+    run_sequences([given])
+    run_sequences([own])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
