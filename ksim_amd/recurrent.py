@@ -569,7 +569,8 @@ class RecurrentNetwork:
             xs.append(x)
             saved.append(sv)
             x = hs
-        if len(self.output_proj.dims) == 2 and self.output_proj.dtype == "bf16":  # a single layer keeps nothing for its backward pass
+        # a single layer keeps nothing for its backward pass; what the training forward refuses (no rows, no train_init) is left to it
+        if len(self.output_proj.dims) == 2 and self.output_proj.dtype == "bf16" and T_ * M > 0 and getattr(self.output_proj, "_training", False):
             out = yield from _layer(self.output_proj, x.view(T_ * M, H))
         else:
             out = self.output_proj.train_forward(x.view(T_ * M, H))

@@ -552,3 +552,32 @@ def test_a_given_projected_input_is_checked(kind):
     run_sequences([given])
     run_sequences([own])
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_training_forward_of_what_cannot_be_trained_is_refused(dtype):
+    """An output layer without its training buffers, and a trajectory of no steps: the same answer in both precisions."""
+    from ksim_amd import _lib
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import GRUCell, RecurrentNetwork
+
+    rng = np.random.default_rng(3)
+    w = lambda *s: rng.normal(scale=0.1, size=s)  # noqa: E731
+
+    def net(H):
+        return RecurrentNetwork((w(H, 6), w(H)), [GRUCell(w(3 * H, H), w(3 * H, H), w(3 * H), w(H), dtype=dtype)],
+                                MLP([w(4, H)], [w(4)], activation="none", dtype=dtype), dtype=dtype)
+
+    def args(T, M, H):
+        return torch.randn(T, M, 6, device="cuda"), torch.zeros(1, M, H, device="cuda"), torch.zeros(T, M, dtype=torch.uint8, device="cuda")
+
+    part = net(128)
+    part.input_proj.train_init()
+    part.cells[0].train_init()
+    with pytest.raises(_lib.KsError, match="ks_mlp_train_init"):
+        part.train_forward(*args(2, 3, 128))
+    whole = net(64)  # a width whose cells step one by one
+    whole.train_init()
+    with pytest.raises(_lib.KsError):
+        whole.train_forward(*args(0, 3, 64))
+    assert whole.train_forward(*args(2, 3, 64)).shape == (2, 3, 4)
