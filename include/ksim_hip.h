@@ -721,7 +721,8 @@ int ks_mlp_forward(const KsMlp* mlp, ks_stream_t stream, int64_t M, const float*
 /* Two networks over the same M rows, e.g. the actor on the noisy observations and the critic on the clean ones
  * (ksim/task/rl.py:892-926 and the value call of examples/walking.py:626-638, which XLA schedules side by side).  Same
  * results as two ks_mlp_forward calls; when both networks run as whole-network kernels with one activation and M is
- * below 16384, or are single bf16 layers that take the same row tile, they share a single launch, so the second network's workgroups overlap the first one's. */
+ * below 16384, or are single bf16 layers that take the same row tile, they share a single launch, so the second network's
+ * workgroups overlap the first one's.  Two that touch one another's memory, as where x1 is y0, run one after the other. */
 int ks_mlp_forward_pair(const KsMlp* mlp0, const KsMlp* mlp1, ks_stream_t stream, int64_t M, const float* x0,
                         float* y0, const float* x1, float* y1, void* workspace0, void* workspace1);
 /* ks_mlp_forward_pair on an actor and a critic, and ks_sample_action on the actor's output, in the same launch where the two networks share one:

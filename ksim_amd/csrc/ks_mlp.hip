@@ -2469,6 +2469,13 @@ static int launch_split(const DevMlp& a, const DevMlp* b, hipStream_t s, int64_t
   return check_launch("ks_mlp_forward");
 }
 
+// Whether two pieces of memory share a float
+struct Span {
+  const float* p;
+  int64_t n;
+};
+static bool meet(Span a, Span b) { return a.p && b.p && (uintptr_t)a.p < (uintptr_t)(b.p + b.n) && (uintptr_t)b.p < (uintptr_t)(a.p + a.n); }
+
 // `sample`: what the launch also makes of the first network's output where the two share one; its `action` is NULL on return then
 static int forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t stream, int64_t M, const float* x0, float* y0, const float* x1, float* y1,
                         void* workspace0, void* workspace1, KsActionSample& sample) {
@@ -2478,6 +2485,12 @@ static int forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t stream, in
   if (!x0 || !y0 || !x1 || !y1) return fail(KS_EINVAL, "ks_mlp_forward_pair: null pointer");
   if (y0 == y1) return fail(KS_EINVAL, "ks_mlp_forward_pair: the two outputs must differ");
   hipStream_t s = (hipStream_t)stream;
+  const Span in0 = {x0, M * h0->m.dims[0]}, in1 = {x1, M * h1->m.dims[0]}, out0 = {y0, M * h0->m.dims[h0->m.n_layers]},
+             out1 = {y1, M * h1->m.dims[h1->m.n_layers]};
+  if (meet(out0, in1) || meet(out1, in0) || meet(out0, out1)) {  // e.g. the second reads what the first writes: one after the other
+    const int rc = ks_mlp_forward(h0, stream, M, x0, y0, workspace0);
+    return rc != KS_OK ? rc : ks_mlp_forward(h1, stream, M, x1, y1, workspace1);
+  }
   if (small_ok(h0->m, M) && small_ok(h1->m, M) && h0->m.n_layers == h1->m.n_layers && h0->m.n_layers > 1 && workspace0 && workspace1 &&
       workspace0 != workspace1)
     return launch_small(h0->m, &h1->m, s, M, x0, y0, workspace0, x1, y1, workspace1);
@@ -2491,8 +2504,13 @@ static int forward_pair(const KsMlp* h0, const KsMlp* h1, ks_stream_t stream, in
   }
   // one launch when both networks run as whole-network kernels with the same activation and row tile; else one each
   if (h0->m.fused && h1->m.fused && h0->m.activation == h1->m.activation && h0->m.dtype == h1->m.dtype && M < 64 * 256) {
-    const KsActionSample with = sample;
-    sample.action = nullptr;
+    KsActionSample with = sample;
+    // actions over rows that another workgroup has yet to read or write, and deviations or noise that the networks write, wait for both networks
+    const Span act = {sample.action, out0.n}, noise = {sample.noise_normal, out0.n}, dev = {sample.log_std, h0->m.dims[h0->m.n_layers]};
+    bool apart = act.p != out0.p && meet(act, out0);
+    for (const Span& x : {in0, in1, out1}) apart |= meet(act, x);
+    for (const Span& y : {out0, out1}) apart |= meet(noise, y) || meet(dev, y);
+    (apart ? with : sample).action = nullptr;
     if (h0->m.dtype == KS_MLP_F32) return launch_fused_pair_tile<float, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1, with);
     return launch_fused_pair_tile<__bf16, 32>(h0->m, h1->m, s, M, x0, y0, x1, y1, with);
   }

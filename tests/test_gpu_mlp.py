@@ -509,3 +509,38 @@ def test_actions_sampled_in_the_networks_launch_match_the_launch_of_their_own(hi
         for g, w in zip(got, want):
             assert torch.equal(torch.nan_to_num(g, nan=123.0), torch.nan_to_num(w, nan=123.0)), (g.shape, given.keys())
         assert bool(torch.isfinite(got[2]).all()) and got[2].abs().max().item() <= 0.75
+
+
+@pytest.mark.parametrize("dims,dtype", [((128, 128), "bf16"), ((128, 128, 128, 128), "bf16"), ((128, 512, 512, 128), "bf16"), ((128, 128, 128), "f32"),
+                                        ((128, 512, 128), "f32")])
+@pytest.mark.parametrize("M", [40, 300, 5000, 40000])
+def test_pairs_that_touch_one_anothers_memory_run_one_after_the_other(dims, dtype, M):
+    """The second network on the first one's output, the first on rows that the second overwrites, outputs that overlap, and actions that take the place
+    of an input: what the calls give one by one, in every form of the pair's launch."""
+    from ksim_amd.env_terms import action_sample, sample_action
+    from ksim_amd.mlp import MLP
+
+    rng = np.random.default_rng(M)
+    a, b = (MLP([rng.normal(scale=i ** -0.5, size=(o, i)) for i, o in zip(dims[:-1], dims[1:])], [0.1 * rng.normal(size=o) for o in dims[1:]],
+                activation="elu", dtype=dtype) for _ in range(2))
+    n = M * 128
+    given = torch.from_numpy(rng.normal(size=4 * n + 64).astype(np.float32)).cuda()
+    rows = lambda buf, first: buf[first : first + n].view(M, 128)  # noqa: E731
+    for xa, ya, xb, yb in ((0, n, n, 2 * n), (0, n, n + 64, 3 * n), (0, n, 2 * n, 0), (0, n, 3 * n, n + 64), (0, n, 3 * n, n - 64)):
+        want, got = given.clone(), given.clone()
+        a(rows(want, xa), out=rows(want, ya))
+        b(rows(want, xb), out=rows(want, yb))
+        a.forward_pair(rows(got, xa), rows(got, ya), b, rows(got, xb), rows(got, yb))
+        assert torch.equal(got, want), (xa, ya, xb, yb)
+    log_std = torch.full((128,), -1.0, device="cuda")
+    for out, noise in ((0, None), (n, None), (2 * n, None), (3 * n, None), (None, n), (None, 3 * n)):
+        results = []
+        for in_launch in (False, True):
+            buf, apart = given.clone(), torch.empty(M, 128, device="cuda")
+            sampling = dict(seed=3, clip_max=1.5, out=apart if out is None else rows(buf, out), noise=None if noise is None else rows(buf, noise))
+            args = (rows(buf, 0), rows(buf, n), b, rows(buf, 2 * n), rows(buf, 3 * n))
+            a.forward_pair(*args, action_sample(args[1], log_std, **sampling) if in_launch else None)
+            if not in_launch:
+                sample_action(args[1], log_std, **sampling)
+            results.append(buf if out is not None else torch.cat([buf, apart.view(-1)]))
+        assert torch.equal(*results), (out, noise)
