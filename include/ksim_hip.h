@@ -810,7 +810,8 @@ int ks_mlp_train_backward_dx(KsMlp* mlp, ks_stream_t stream, int64_t M, const fl
 /* The weight and bias gradient of a network of one layer from input rows that lie ldx floats apart (ldx >= in). */
 int ks_mlp_layer_weight_grad(KsMlp* mlp, ks_stream_t stream, int64_t M, const float* x, int64_t ldx, const float* dy, void* workspace);
 /* The backward pass of several networks of one layer, e.g. the projections of a recurrent actor and critic: same results as
- * ks_mlp_train_backward_dx and ks_mlp_layer_weight_grad one by one, in fewer launches.  No two of them may write the same gradient. */
+ * ks_mlp_train_backward_dx and ks_mlp_layer_weight_grad one by one, in fewer launches where no dx lies in another entry's arrays and no
+ * network occurs twice with weight gradients; else one by one. */
 typedef struct KsLayerBackward {
   KsMlp* mlp;
   int64_t M;

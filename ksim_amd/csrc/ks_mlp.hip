@@ -4191,6 +4191,22 @@ extern "C" int ks_mlps_layer_backward(int32_t n, const KsLayerBackward* q, ks_st
   if (n < 0 || (n > 0 && (!q || !workspace))) return fail(KS_EINVAL, "ks_mlps_layer_backward: bad argument");
   for (int k = 0; k < n; ++k)
     if (const int rc = check_layer_backward(q[k])) return rc;
+  // entries that need one another's results, or write one gradient, by themselves in their order
+  bool apart = true;
+  for (int k = 0; k < n; ++k) {
+    const Span dx = {q[k].dx, q[k].M * q[k].mlp->m.dims[0]};
+    for (int j = 0; j < n; ++j) {
+      if (j == k) continue;
+      const int in = q[j].mlp->m.dims[0];
+      apart &= !(meet(dx, {q[j].x, (q[j].M - 1) * q[j].ldx + in}) || meet(dx, {q[j].dy, q[j].M * q[j].mlp->m.dims[1]}) || meet(dx, {q[j].dx, q[j].M * in}) ||
+                 (q[j].mlp == q[k].mlp && q[j].x && q[k].x));
+    }
+  }
+  if (!apart) {
+    for (int k = 0; k < n; ++k)
+      if (const int rc = ks_mlps_layer_backward(1, q + k, stream, workspace)) return rc;
+    return KS_OK;
+  }
   hipStream_t s = (hipStream_t)stream;
   // input gradients: those of bf16 layers two to a launch, each with the next one that has its row tile
   FusedArgs held;

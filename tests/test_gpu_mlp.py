@@ -544,3 +544,39 @@ def test_pairs_that_touch_one_anothers_memory_run_one_after_the_other(dims, dtyp
                 sample_action(args[1], log_std, **sampling)
             results.append(buf if out is not None else torch.cat([buf, apart.view(-1)]))
         assert torch.equal(*results), (out, noise)
+
+
+@pytest.mark.parametrize("M", [37, 1544])
+def test_layers_that_need_one_another_go_backward_in_their_order(M):
+    """A chain of layers whose gradients are one another's operands, a gradient over another's input rows, and one network twice, in one call: what
+    the calls give one by one."""
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import LayerBackward, run_layers_backward
+
+    rng = np.random.default_rng(M)
+    t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    nets = []
+    for dtype in ("bf16", "bf16", "f32"):
+        nets.append(MLP([rng.normal(scale=0.1, size=(128, 128))], [0.1 * rng.normal(size=128)], activation="none", dtype=dtype))
+        nets[-1].train_init()
+    a, b, c = nets
+    x, dy, wide = t(M, 128), t(M, 128), t(M, 160)
+
+    def entries(d1, d2, rows):
+        return [[LayerBackward(a, dy, x, d1), LayerBackward(b, d1, x, d2), LayerBackward(c, d2, x)],  # down a chain
+                [LayerBackward(a, dy, rows[:, 32:]), LayerBackward(b, dy, None, rows.view(-1)[64:][: M * 128].view(M, 128))],  # over rows read before
+                [LayerBackward(b, dy, None, d1), LayerBackward(a, dy, None, d1)],  # one place twice
+                [LayerBackward(a, dy, x), LayerBackward(a, x, dy), LayerBackward(c, dy, x)]]  # one gradient twice
+
+    for k in range(4):
+        results = []
+        for together in (False, True):
+            d1, d2, rows = torch.zeros(M, 128, device="cuda"), torch.zeros(M, 128, device="cuda"), wide.clone()
+            calls = entries(d1, d2, rows)[k]
+            if together:
+                run_layers_backward(calls)
+            else:
+                for call in calls:
+                    run_layers_backward([call])
+            results.append([d1, d2, rows] + [g for net in nets for pair in net.parameters(gradients=True) for g in pair])
+        assert all(torch.equal(u, v) for u, v in zip(*results)), k
