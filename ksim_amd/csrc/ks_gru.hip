@@ -197,14 +197,18 @@ __device__ __forceinline__ float seq_tanh(float x) { return 1.f - 2.f * __builti
 // ahead for the next step) before every barrier, a memory round trip per step of the sequence.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The LSTM forward kernel's way in and out of memory: a step's inputs are requested a step ahead of their use and its results leave behind it, one
-// load or store (KS_SEQ_SIDE, a single instruction from a uniform address) after every eight matrix instructions.  All together at a step's
-// end they held the CU's wavefronts up at once, and a store or load under a condition makes the compiler wait for the step's stores before the
-// next step: loads and stores are counted together and waited for in order.  Hence no conditions (the outputs that a launch has are template
-// arguments, rows past the batch repeat the last row and store its values once more, the last step requests its own inputs again) and nothing
-// pending where the loop is entered.  2 x 1024 rows x 100 steps with kept activations: 394 -> 366 us; without them 380 -> 363; a rollout's control
-// step of 4096 envs (T = 1, several sets of rows per workgroup) 437 -> 424.  What is left is issue and power: 2048 of 3500 cycles of a step are
-// matrix instructions, at 2.0 to 2.2 GHz.  The backward kernel (342 -> 361 us) and the GRU's (31 us either way) did not gain from the same order.
+// The LSTM forward kernel's way in and out of memory: a step's inputs are requested a step ahead of their use.  Where the activations are kept, nine
+// results a step leave behind it, one load or store (KS_SEQ_SIDE, a single instruction from a uniform address) after every eight matrix instructions
+// of the next.  All together at a step's end they held the CU's wavefronts up at once, and a store or load under a condition makes the compiler wait
+// for the step's stores before the next step: loads and stores are counted together and waited for in order.  Hence no conditions (the outputs that
+// a launch has are template arguments, rows past the batch repeat the last row and store its values once more, the last step requests its own inputs
+// again) and nothing pending where the loop is entered.  Without kept activations a step stores one or two values, and the order imposed on its
+// matrix instructions costs more than it gives: loads at its start, stores at its end, the rest as the compiler likes.
+// Two layers, everything at the step's end and under conditions -> one after every eight -> as here:
+//   1024 rows x 100 steps, kept 372 -> 358 -> 358 us, not kept 302 -> 314 -> 298; 64 x 100, not kept 145 -> 155 -> 136; 512 x 24 with cell states
+//   43.9 -> 45.7 -> 41.7; one step (a rollout's call) of 4096 rows 34.6 -> 34.4 -> 33.6, of 64 10.3 -> 10.5 -> 10.3
+// What is left is issue and power: 2048 of 3500 cycles of a step are matrix instructions, at 2.0 to 2.2 GHz.  The backward kernel (342 -> 361 us) and
+// the GRU's (31 us either way) did not gain from the same order.
 __device__ __forceinline__ void seq_loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
 #define KS_SEQ_SIDE(OP)                \
   {                                    \
@@ -312,6 +316,10 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
   seq_loads_done();
   __syncthreads();
   auto step = [&](int t, auto cur, bool first, const In& in, In& next) __attribute__((always_inline)) {
+    if constexpr (!SAVE) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) load(t + 1, next, k);
+    }
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
     float ha[8];
     {
@@ -323,7 +331,7 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
 #define KS_SEQ_MFMA(K0)                                                                                            \
     acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[(K0) >> 4], wa[(K0)], acc0, 4, (K0) & 15, 0);                       \
     acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[((K0) + 1) >> 4], wa[(K0) + 1], acc1, 4, ((K0) + 1) & 15, 0);
-#define KS_SEQ_MFMA8(N, OP) KS_SEQ_MFMA(8 * N) KS_SEQ_MFMA(8 * N + 2) KS_SEQ_MFMA(8 * N + 4) KS_SEQ_MFMA(8 * N + 6) KS_SEQ_SIDE(OP)
+#define KS_SEQ_MFMA8(N, OP) KS_SEQ_MFMA(8 * N) KS_SEQ_MFMA(8 * N + 2) KS_SEQ_MFMA(8 * N + 4) KS_SEQ_MFMA(8 * N + 6) if constexpr (SAVE) KS_SEQ_SIDE(OP)
 #define KS_SEQ_OUT(N) KS_SEQ_MFMA8(N, if (!first) store(t - 1, N))
 #define KS_SEQ_IN(N) KS_SEQ_MFMA8(N, load(t + 1, next, 13 - N))
     KS_SEQ_OUT(0) KS_SEQ_OUT(1) KS_SEQ_OUT(2) KS_SEQ_OUT(3) KS_SEQ_OUT(4) KS_SEQ_OUT(5) KS_SEQ_OUT(6) KS_SEQ_OUT(7) KS_SEQ_OUT(8)
@@ -349,6 +357,7 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
     tc = seq_tanh(c);
     hprev = so * tc;
     sh[cur ^ 1][j][seq_slot(unit)] = hprev;
+    if constexpr (!SAVE) { store(t, 0); store(t, 1); }
     lds_barrier();  // the new hidden state is complete; the buffer just read is free for the step after next
   };
   constexpr std::integral_constant<int, 0> even{};
@@ -360,8 +369,10 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
     step(t + 1, even, false, in0, in1);
   }
   if (t < T) step(t, odd, false, in1, in0);
+  if constexpr (SAVE) {
 #pragma unroll
-  for (int k = 0; k < 9; ++k) store(T - 1, k);
+    for (int k = 0; k < 9; ++k) store(T - 1, k);
+  }
   }
 }
 
