@@ -978,36 +978,56 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, T* __rest
 }
 
 // The network's input rows, one piece of memory, into the tile; zero beyond the batch and from column in_dim to K0.  V: what a thread requests at a
-// time, and Q of them before it waits: the loads stand behind no condition (the index is held back to the last one), as behind one they are waited
-// for one by one.  The zeros go in as 16-byte pieces, one of which may hold a row's last columns too: hence the barrier.
-// An entry of the padding at a time, each with a division, and up to eight waits for memory, against two pieces a thread and one wait: 524288 rows of
-// 68-512-512-512-20 615 -> 611 us, the update of 65536 rows 1198 -> 1195.
+// time, and Q of them before it waits.  bf16 tiles of 64 rows and more (kHeld): the loads stand behind no condition (the index is held back to the
+// last one), as behind one they are waited for one by one, and the zeros go in as 16-byte pieces, one of which may hold a row's last columns too:
+// hence the barrier.  Tiles of 32 rows are two to five loads a thread, of which most would be repeats, and the barrier costs as much as the entries
+// of padding; fp32 networks read beside six matrix instructions a product.  In us, behind conditions -> held back:
+//   68-3 x 128-20, 4096 rows 6.87 -> 7.02, 12000 rows 8.78 -> 8.00; 120-3 x 128-20 7.02 -> 7.21 and 8.09 -> 8.37; 71-3 x 256-20, 12000 rows 12.98 -> 14.15;
+//   43-3 x 128-20, 12000 rows 7.63 -> 8.19; a pair 68-3 x 256, 64 rows 9.45 -> 9.57; fp32 71-3 x 128-20, 20000 rows 36.4 -> 36.9
+//   68-3 x 128-20, 20000 rows 10.28 -> 9.49; 71-3 x 512-20, 20000 rows, four at a time 37.9 -> 39.6, six 37.7; 67-3 x 256-20, 65536 rows 39.6 -> 37.5; 67-2 x 256-20, 524288 rows 242 -> 206; training forward of 65536
+//   rows of 67-3 x 128-20 40.5 -> 34.7; worst of a sweep: 55-2 x 256-20, 30000 rows 13.8 -> 14.4
 template <typename T, int BM, typename V>
 __device__ __forceinline__ void mlp_input_tile(T* __restrict__ act, int lda, const float* __restrict__ src, int rows, int in_dim, int K0) {
-  constexpr int NTHR = 64 * kFusedWaves, E = sizeof(V) / 4, Q = BM >= 128 ? 8 : 4, PC = 16 / (int)sizeof(T);
+  constexpr bool kHeld = sizeof(T) == 2 && BM >= 64;
+  constexpr int NTHR = 64 * kFusedWaves, E = sizeof(V) / 4, Q = BM >= 128 ? 8 : kHeld && E == 1 ? 6 : 4, PC = 16 / (int)sizeof(T);
   const int tid = threadIdx.x, total = rows * in_dim / E;
   const V* from = reinterpret_cast<const V*>(src);
-  V v[Q];
-  auto fetch = [&](int base) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) v[q] = from[min(base + q * NTHR, total - 1)];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(v[q]));
-  };
-  if (K0 > in_dim || rows < BM) {
-    const int first = in_dim / PC, pieces = K0 / PC - first;
-    for (int idx = tid; idx < BM * pieces; idx += NTHR) {
-      const int r = idx / pieces;
-      *reinterpret_cast<u32x4*>(act + r * lda + (first + idx - r * pieces) * PC) = u32x4{0u, 0u, 0u, 0u};
+  if constexpr (kHeld) {
+    if (K0 > in_dim || rows < BM) {
+      const int first = in_dim / PC, pieces = K0 / PC - first;
+      for (int idx = tid; idx < BM * pieces; idx += NTHR) {
+        const int r = idx / pieces;
+        *reinterpret_cast<u32x4*>(act + r * lda + (first + idx - r * pieces) * PC) = u32x4{0u, 0u, 0u, 0u};
+      }
+      for (int idx = rows * first + tid; idx < BM * first; idx += NTHR) {
+        const int r = idx / first;
+        *reinterpret_cast<u32x4*>(act + r * lda + (idx - r * first) * PC) = u32x4{0u, 0u, 0u, 0u};
+      }
+      __syncthreads();
     }
-    for (int idx = rows * first + tid; idx < BM * first; idx += NTHR) {
-      const int r = idx / first;
-      *reinterpret_cast<u32x4*>(act + r * lda + (idx - r * first) * PC) = u32x4{0u, 0u, 0u, 0u};
+  } else {
+    const int padw = K0 - in_dim;
+    for (int idx = tid; idx < BM * padw; idx += NTHR) {
+      const int r = idx / padw, c = idx - r * padw;
+      act[r * lda + in_dim + c] = (T)0.0f;
     }
-    __syncthreads();
+    for (int idx = rows * in_dim + tid; idx < BM * in_dim; idx += NTHR) {
+      const int r = idx / in_dim, c = idx - r * in_dim;
+      act[r * lda + c] = (T)0.0f;
+    }
   }
   for (int base = tid; base < total; base += NTHR * Q) {
-    fetch(base);
+    V v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int idx = base + q * NTHR;
+      if constexpr (kHeld) v[q] = from[min(idx, total - 1)];
+      else v[q] = idx < total ? from[idx] : V{};
+    }
+    if constexpr (kHeld) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) asm volatile("" : "+v"(v[q]));  // keeps the loads out of the conditions below
+    }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int idx = base + q * NTHR;
