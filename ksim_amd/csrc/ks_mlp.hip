@@ -3808,26 +3808,39 @@ struct WgradJob {
   unsigned first, first_sum;  // the job's first workgroup in wgrad_kernel and in sum_slices_kernel
 };
 constexpr int kWgradJobs = 12;
+// A layer by itself has kernels of its own (JOBS = 1): the search for a workgroup's job and its place in it are two or three loads and a division one
+// after the other (bf16, 12288 rows of 128 -> 384: 15.2 us, 16.0 through the search; of 128 -> 1: 10.9 and 11.3).
+template <int JOBS>
 struct WgradTable {
   int n;
-  WgradJob job[kWgradJobs];
+  WgradJob job[JOBS];
 };
-
-template <int PARTS, bool EDGE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void wgrad_kernel(const WgradTable table) {
-  extern __shared__ __attribute__((aligned(16))) u32x4 tn_lds[];  // [group][part][8 rows][slot: 128 of A, 128 of B]
+template <int JOBS>
+__device__ __forceinline__ const WgradJob& wgrad_find(const WgradTable<JOBS>& table, unsigned WgradJob::*first) {
   int which = 0;
-  while (which + 1 < table.n && blockIdx.x >= table.job[which + 1].first) ++which;
-  const WgradJob& job = table.job[which];
-  const int M = job.M, N = job.N, K = job.K, kslice = job.kslice, tiles = job.tiles, slices = job.slices, lb = (int)(blockIdx.x - job.first);
-  if (lb >= tiles * slices) return;  // the workgroups that fill up the job's last eight
+  if constexpr (JOBS > 1)
+    while (which + 1 < table.n && blockIdx.x >= table.job[which + 1].*first) ++which;
+  return table.job[which];
+}
+
+template <int PARTS, bool EDGE, int JOBS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void wgrad_kernel(const WgradTable<JOBS> table) {
+  extern __shared__ __attribute__((aligned(16))) u32x4 tn_lds[];  // [group][part][8 rows][slot: 128 of A, 128 of B]
+  const WgradJob& job = wgrad_find(table, &WgradJob::first);
+  const int M = job.M, N = job.N, K = job.K, kslice = job.kslice, tiles = JOBS > 1 ? job.tiles : gridDim.x, slices = JOBS > 1 ? job.slices : gridDim.y;
+  const int lb = JOBS > 1 ? (int)(blockIdx.x - job.first) : (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  if (JOBS > 1 && lb >= tiles * slices) return;  // the workgroups that fill up the job's last eight
   const float *__restrict__ A = job.A, *__restrict__ B = job.B;
   const int64_t lda = job.lda, ldb = job.ldb, ldc = job.ldc;
   const bool sliced = slices > 1;
   float *__restrict__ C = sliced ? job.part : job.C, *__restrict__ colsum = sliced ? job.colpart : job.colsum;
   // Workgroup l runs on XCD l % 8: the tiles of one slice, which read the same rows, go to one XCD one after the other
-  int tile = lb % tiles, z = lb / tiles;
+  int tile = blockIdx.x, z = blockIdx.y;
+  if constexpr (JOBS > 1) {
+    tile = lb % tiles;
+    z = lb / tiles;
+  }
   if (slices % 8 == 0) {
     const int q = lb >> 3;
     tile = q % tiles;
@@ -3989,11 +4002,10 @@ void wgrad_kernel(const WgradTable table) {
 
 // C = the sum of nz slices of (M, N), and colsum = the sum of nz rows of M behind it in the same launch.  A workgroup takes 64 entries,
 // a quarter of the slices to each wavefront with 16 loads in flight, then adds the four in order.
-__global__ __launch_bounds__(256) void sum_slices_kernel(const WgradTable table) {
+template <int JOBS>
+__global__ __launch_bounds__(256) void sum_slices_kernel(const WgradTable<JOBS> table) {
   __shared__ float sh[256];
-  int which = 0;
-  while (which + 1 < table.n && blockIdx.x >= table.job[which + 1].first_sum) ++which;
-  const WgradJob& job = table.job[which];
+  const WgradJob& job = wgrad_find(table, &WgradJob::first_sum);
   const int M = job.M, N = job.N, nz = job.slices;
   const float *__restrict__ part = job.part, *__restrict__ colpart = job.colpart;
   float *__restrict__ C = job.C, *__restrict__ colsum = job.colsum;
@@ -4150,8 +4162,19 @@ static WgradJob wgrad_job(int64_t M, int N, int64_t K, const float* A, int64_t l
 }
 
 // Several of them, of one kind: a launch for the products and one for the sums of their slices
-template <int PARTS>
-static int wgrads(hipStream_t s, WgradTable& t) {
+template <int PARTS, int JOBS>
+static int launch_wgrads(hipStream_t s, const WgradTable<JOBS>& t, dim3 grid, unsigned sums, bool edge) {
+  constexpr int lds = 2 * tn_buf(PARTS) * 16;
+  auto kfn = edge ? wgrad_kernel<PARTS, true, JOBS> : wgrad_kernel<PARTS, false, JOBS>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
+  hipLaunchKernelGGL(kfn, grid, dim3(512), lds, s, t);
+  if (sums) hipLaunchKernelGGL(sum_slices_kernel<JOBS>, dim3(sums), dim3(256), 0, s, t);
+  return KS_OK;
+}
+
+template <int PARTS, int JOBS>
+static int wgrads(hipStream_t s, WgradTable<JOBS>& t) {
   unsigned blocks = 0, sums = 0;
   bool edge = false;
   for (int k = 0; k < t.n; ++k) {
@@ -4162,19 +4185,15 @@ static int wgrads(hipStream_t s, WgradTable& t) {
     j.first_sum = sums;
     if (j.slices > 1) sums += (unsigned)(((int64_t)j.M * j.N + 63) / 64 + (j.M + 63) / 64);
   }
-  constexpr int lds = 2 * tn_buf(PARTS) * 16;
-  auto kfn = edge ? wgrad_kernel<PARTS, true> : wgrad_kernel<PARTS, false>;
-  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-    return fail(KS_ELAUNCH, "ks_mlp_train_backward: cannot raise the LDS limit to %d bytes", lds);
-  hipLaunchKernelGGL(kfn, dim3(blocks), dim3(512), lds, s, t);
-  if (sums) hipLaunchKernelGGL(sum_slices_kernel, dim3(sums), dim3(256), 0, s, t);
-  return KS_OK;
+  if (t.n > 1) return launch_wgrads<PARTS>(s, t, dim3(blocks), sums, edge);
+  const WgradTable<1> one = {1, {t.job[0]}};
+  return launch_wgrads<PARTS>(s, one, dim3((unsigned)one.job[0].tiles, (unsigned)one.job[0].slices), sums, edge);
 }
 
 template <int PARTS>
 static int wgrad(hipStream_t s, int64_t M, int N, int64_t K, const float* A, int64_t lda, const float* B, int64_t ldb, float* C,
                  int64_t ldc, float* part, float* colsum) {
-  WgradTable t;
+  WgradTable<1> t;
   t.n = 1;
   t.job[0] = wgrad_job(M, N, K, A, lda, B, ldb, C, ldc, part, colsum);
   return wgrads<PARTS>(s, t);
@@ -4260,7 +4279,7 @@ extern "C" int ks_mlps_layer_backward(int32_t n, const KsLayerBackward* q, ks_st
   // weight gradients, those of a precision together
   char* part = (char*)workspace;
   for (int bf16 = 0; bf16 < 2; ++bf16) {
-    WgradTable t;
+    WgradTable<kWgradJobs> t;
     t.n = 0;
     for (int k = 0; k <= n; ++k) {
       if (t.n == kWgradJobs || (k == n && t.n > 0)) {
