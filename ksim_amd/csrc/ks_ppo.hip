@@ -842,7 +842,8 @@ __device__ __forceinline__ void row_factors(const PpoRow& in, float* __restrict_
 // block partials, then ppo_grad_finish_kernel, so the result does not depend on scheduling.  1024 threads: at most 256 workgroups
 // (the partials' buffer) still keep 16 wavefronts per CU in flight (65536 rows x 20 actions: 36 -> 19 us).  The next rows' pairs are
 // requested as soon as these are used up and the row's own values ahead of the pairs': a workgroup walks its rows a launch's width apart, five
-// times there, and waited for memory twice each time (19.6 -> 12.0 us).
+// times there, and waited for memory twice each time (14.4 -> 11.2 us).  At the last stop nothing more is requested, as the barrier waits for it
+// (12288 rows 7.0, 6.7 requesting the last rows again, 6.5; 1000 rows of one action 15.2, 15.8, 15.3).
 __global__ __launch_bounds__(1024) void ppo_loss_grad_kernel(int64_t M, int nu, KsPpoLossParams p, const float* __restrict__ mean,
                                                             const float* __restrict__ log_std, PpoGradIO io, float* __restrict__ d_mean,
                                                             float* __restrict__ partial) {
@@ -866,9 +867,10 @@ __global__ __launch_bounds__(1024) void ppo_loss_grad_kernel(int64_t M, int nu, 
     const int64_t i = row0 * nu + threadIdx.x;  // the pairs of whole rows are contiguous
     const float z = (f_action - f_mean) * is;
     if (ok) el[threadIdx.x] = (-0.5f * z * z - ls - kHalfLog2Pi) - f_on_lp;
-    fetch(row0 + stride);
+    const bool more = row0 + stride < M;
+    if (more) fetch(row0 + stride);
     row_factors(in, io.d_value, p, kl_scale, inv_m, M, row0, rows, nu, el, sel);
-    in = row_fetch(io, M, row0 + stride, rows);
+    if (more) in = row_fetch(io, M, row0 + stride, rows);
     if (ok) {
       const float g_lp = sel[r];
       d_mean[i] = g_lp * z * is;
