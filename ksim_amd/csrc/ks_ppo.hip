@@ -580,6 +580,10 @@ extern "C" int64_t ks_abi_sizeof(int32_t which) {
     case 20: return sizeof(KsMixtureHead);
     case 21: return sizeof(KsNoiseStage);
     case 22: return sizeof(KsRandomVar);
+    case 23: return sizeof(KsActionSample);
+    case 24: return sizeof(KsLayerBackward);
+    case 25: return sizeof(KsGatherArray);
+    case 26: return sizeof(KsSequence);
     default: return -1;
   }
 }

@@ -580,3 +580,30 @@ def test_layers_that_need_one_another_go_backward_in_their_order(M):
                     run_layers_backward([call])
             results.append([d1, d2, rows] + [g for net in nets for pair in net.parameters(gradients=True) for g in pair])
         assert all(torch.equal(u, v) for u, v in zip(*results)), k
+
+
+@pytest.mark.parametrize("M", [37, 1544])
+def test_layers_too_wide_for_the_whole_network_kernel_in_shared_launches(M):
+    """A bf16 layer of more outputs than the whole-network kernel holds takes its input gradient through the call's workspace, which the weight
+    gradients of all layers use behind it; more weight gradients of one precision than a launch's table takes beside them."""
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import LayerBackward, run_layers_backward
+
+    rng = np.random.default_rng(M)
+    t = lambda *s: torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda()  # noqa: E731
+    results, shapes = [], [(128, 768), (128, 384), (256, 768), (128, 2048)] + [(43, 128)] * 10
+    nets = [MLP([rng.normal(scale=i ** -0.5, size=(o, i))], [0.1 * rng.normal(size=o)], activation="none", dtype="bf16") for i, o in shapes]
+    rows = [(t(M, n.in_dim), t(M, n.out_dim)) for n in nets]
+    for n in nets:
+        n.train_init()
+    for together in (False, True):
+        dxs = [torch.empty(M, n.in_dim, device="cuda") for n in nets]
+        for n, (x, dy), dx in zip(nets, rows, dxs):
+            if together:
+                n.layer_weight_grad(dy.new_ones(M, n.in_dim), torch.ones_like(dy))  # something else in the handle
+            else:
+                n.backward_dx(x, dy, dx)
+        if together:
+            run_layers_backward([LayerBackward(n, dy, x, dx) for n, (x, dy), dx in zip(nets, rows, dxs)])
+        results.append(dxs + [g.clone() for n in nets for pair in n.parameters(gradients=True) for g in pair])
+    assert all(torch.equal(a, b) for a, b in zip(*results))

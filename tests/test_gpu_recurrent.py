@@ -581,3 +581,37 @@ def test_training_forward_of_what_cannot_be_trained_is_refused(dtype):
     with pytest.raises(_lib.KsError):
         whole.train_forward(*args(0, 3, 64))
     assert whole.train_forward(*args(2, 3, 64)).shape == (2, 3, 4)
+
+
+@pytest.mark.parametrize("kind,dtype,H", [("gru", "bf16", 128), ("gru", "f32", 128), ("gru", "bf16", 64), ("lstm", "f32", 128), ("lstm", "f32", 96)])
+def test_weight_gradients_layer_by_layer_are_those_of_one_launch(kind, dtype, H, monkeypatch):
+    """Above `LATER_ROWS` rows every layer's gradients are launched when they are due, below it all weight gradients at the end: the same bits, for two
+    networks side by side, with cells of the sequence kernels and without."""
+    from ksim_amd import recurrent
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import GRUCell, LSTMCell, RecurrentNetwork, lockstep
+
+    steps, rows, G = 5, 37, 3 if kind == "gru" else 4
+    rng = np.random.default_rng(H)
+    w = lambda *s: rng.normal(scale=s[-1] ** -0.5, size=s)  # noqa: E731
+
+    def net(inputs, outputs):
+        cells = [GRUCell(w(G * H, H), w(G * H, H), w(G * H), w(H), dtype=dtype) if kind == "gru" else LSTMCell(w(G * H, H), w(G * H, H), w(G * H), dtype=dtype)
+                 for _ in range(2)]
+        return RecurrentNetwork((w(H, inputs), w(H)), cells, MLP([w(outputs, H)], [w(outputs)], activation="none", dtype=dtype), dtype=dtype)
+
+    nets, passes = [net(43, 40), net(65, 1)], []
+    for n in nets:
+        n.train_init()
+        carry = torch.from_numpy(0.3 * rng.normal(size=(2, 2, rows, H) if kind == "lstm" else (2, rows, H)).astype(np.float32)).cuda()
+        obs, d_out = (torch.from_numpy(rng.normal(size=(steps, rows, k)).astype(np.float32)).cuda() for k in (n.in_dim, n.out_dim))
+        passes.append((obs, carry, torch.from_numpy((rng.random((steps, rows)) < 0.1).astype(np.uint8)).cuda(), d_out))
+    results = []
+    for limit in (steps * rows, steps * rows - 1):
+        monkeypatch.setattr(recurrent, "LATER_ROWS", limit)
+        for n, (obs, carry, fresh, _) in zip(nets, passes):
+            n.train_forward(obs, carry, fresh)
+        lockstep(*(n.backward_pass(d_out) for n, (_, _, _, d_out) in zip(nets, passes)))
+        results.append([g.clone() for n in nets for m in n.networks() for pair in m.parameters(gradients=True) for g in pair])
+    assert len(results[0]) == 24 and all(bool(g.any()) for g in results[0])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
