@@ -1096,8 +1096,8 @@ void mlp_fused_pair_kernel(const FusedArgs a, const FusedArgs b, const KsActionS
   if (net == 0) mlp_fused_body<ACT, T, BM>(a, tile);
   else mlp_fused_body<ACT, T, BM>(b, tile);
   // The actions of the actor's rows, by all wavefronts from the means that the last layer's have just written (the layer ends with a barrier),
-  // instead of one more small launch per control step (8192 K-Bots in two groups 472 -> 467 us, 64 of them 219.8 -> 219.0,
-  // 4096 humanoids 330.8 -> 329.7).
+  // instead of one more small launch per control step: 8192 K-Bots in two groups 448.9 -> 444.0 us, 64 of them 226.7 -> 225.7, 4096 humanoids
+  // 320.1 -> 319.3 (four processes a side in turn on one card, which differed by 0.2 % at most).
   if (net != 0 || !s.action) return;
   const int nu = a.out_dim;
   const int64_t m0 = tile * BM;
@@ -3807,6 +3807,8 @@ struct WgradJob {
   float *part, *colpart;    // partial products and column sums, where there is more than one slice
   unsigned first, first_sum;  // the job's first workgroup in wgrad_kernel and in sum_slices_kernel
 };
+// Twelve: two networks of two recurrent layers.  A table of 36 changes nothing up to three layers and gives 1 to 2 % of an update at five (LSTM, 12800
+// rows: 2643 -> 2588 us).
 constexpr int kWgradJobs = 12;
 // A layer by itself has kernels of its own (JOBS = 1): the search for a workgroup's job and its place in it are two or three loads and a division one
 // after the other (bf16, 12288 rows of 128 -> 384: 15.2 us, 16.0 through the search; of 128 -> 1: 10.9 and 11.3).
