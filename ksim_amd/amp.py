@@ -42,14 +42,15 @@ def _on_device(rows: torch.Tensor, device: torch.device) -> torch.Tensor:
     return rows
 
 
-def _draw_clips(motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> tuple[torch.Tensor, torch.Tensor]:
-    return (torch.randint(0, motions.shape[0], (batch_b,), generator=generator), torch.randint(0, motions.shape[1], (batch_b,), generator=generator))
+def _draw_clips(n: int, t_clip: int, batch_b: int, generator: torch.Generator) -> tuple[torch.Tensor, torch.Tensor]:
+    return torch.randint(0, n, (batch_b,), generator=generator), torch.randint(0, t_clip, (batch_b,), generator=generator)
 
 
 def _draw_envs(num_envs: int, batch_b: int, generator: torch.Generator) -> torch.Tensor:
+    """All envs in the order drawn; the first `batch_b` are the batch's."""
     if num_envs % batch_b != 0:
         raise ValueError(f"amp_reference_batch_size ({batch_b}) must divide batch_size ({num_envs}).")
-    return torch.randperm(num_envs, generator=generator)[:batch_b]
+    return torch.randperm(num_envs, generator=generator)
 
 
 def _windows(motions: torch.Tensor, window_t: int, clip_idx: torch.Tensor, starts: torch.Tensor) -> torch.Tensor:
@@ -71,33 +72,33 @@ def _sequences(sim_motions: torch.Tensor, envs: torch.Tensor) -> torch.Tensor:
 def make_real_batch(motions: torch.Tensor, window_t: int, batch_b: int, generator: torch.Generator) -> torch.Tensor:
     """`batch_b` windows from reference clips (N, T_clip, F): a clip drawn uniformly, then a uniform start in it
     (amp.py:570-625; the draws come from `generator`, not from jax's key splitting)."""
-    return _windows(motions, window_t, *_draw_clips(motions, batch_b, generator))
+    return _windows(motions, window_t, *_draw_clips(motions.shape[0], motions.shape[1], batch_b, generator))
 
 
 def make_sim_batch(sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> torch.Tensor:
     """`batch_b` distinct envs of the rollout's motions (num_envs, T, F) (amp.py:627-652)."""
-    return _sequences(sim_motions, _draw_envs(sim_motions.shape[0], batch_b, generator))
+    return _sequences(sim_motions, _draw_envs(sim_motions.shape[0], batch_b, generator)[:batch_b])
 
 
 def _batches(motions: torch.Tensor, sim_motions: torch.Tensor, batch_b: int, generator: torch.Generator) -> tuple[torch.Tensor, torch.Tensor]:
     """`make_real_batch` and `make_sim_batch` of one step, in one launch where both are plain fp32 arrays of frames on one GPU and what was drawn
     is in host memory, where the launcher reads it (a default device and a generator of its kind draw elsewhere).  Not while the stream is captured:
     a graph would replay one step's draws for ever, and the functions of the single batches refuse that."""
-    window_t = sim_motions.shape[1]
-    clip_idx, starts = _draw_clips(motions, batch_b, generator)
-    envs = _draw_envs(sim_motions.shape[0], batch_b, generator)
-    plain = (1 <= batch_b <= T.KS_WINDOWS and motions.dim() == sim_motions.dim() == 3 and motions.shape[2] == sim_motions.shape[2]
+    shape, (num_envs, window_t) = motions.shape, sim_motions.shape[:2]
+    clip_idx, starts = _draw_clips(shape[0], shape[1], batch_b, generator)
+    envs = _draw_envs(num_envs, batch_b, generator)
+    plain = (1 <= batch_b <= T.KS_WINDOWS and len(shape) == sim_motions.dim() == 3 and shape[2] == sim_motions.shape[2]
              and motions.dtype == sim_motions.dtype == torch.float32 and motions.is_cuda and motions.device == sim_motions.device
              and motions.is_contiguous() and sim_motions.is_contiguous() and motions.numel() > 0 and sim_motions.numel() > 0
-             and (motions.shape[1] + window_t) * motions.shape[2] <= T.KS_WINDOW_FLOATS
-             and motions.device.index == torch._C._cuda_getDevice() and all(i.device.type == "cpu" for i in (clip_idx, starts, envs))
-             and not torch.cuda.is_current_stream_capturing())
+             and (shape[1] + window_t) * shape[2] <= T.KS_WINDOW_FLOATS
+             and motions.device.index == torch._C._cuda_getDevice() and clip_idx.is_cpu and starts.is_cpu and envs.is_cpu
+             and not torch._C._cuda_isCurrentStreamCapturing())
     if not plain:
-        return _windows(motions, window_t, clip_idx, starts), _sequences(sim_motions, envs)
-    n, t_clip, frame = motions.shape
+        return _windows(motions, window_t, clip_idx, starts), _sequences(sim_motions, envs[:batch_b])
+    n, t_clip, frame = shape
     real, sim = (torch.empty((batch_b, window_t, frame), dtype=torch.float32, device=motions.device) for _ in range(2))
-    _lib.check(_lib.load().ks_gather_windows(_lib.current_stream(), batch_b, window_t, frame, n, t_clip, sim_motions.shape[0], motions.data_ptr(),
-                                             sim_motions.data_ptr(), clip_idx.data_ptr(), starts.data_ptr(), envs.data_ptr(), real.data_ptr(), sim.data_ptr()))
+    _lib.check(_lib.load().ks_gather_windows(_lib.current_stream(), batch_b, window_t, frame, n, t_clip, num_envs, motions.data_ptr(), sim_motions.data_ptr(),
+                                             clip_idx.data_ptr(), starts.data_ptr(), envs.data_ptr(), real.data_ptr(), sim.data_ptr()))
     return real, sim
 
 
