@@ -71,15 +71,16 @@ class LayerBackward:
     def __init__(self, net: MLP, dy: torch.Tensor, x: torch.Tensor | None = None, dx: torch.Tensor | None = None):
         M = dy.shape[0]
         _lib.require_cuda(dy, dx, dtype=torch.float32)
+        # of a contiguous input the strides say nothing where it has one row or one column
+        ldx = 0 if x is None else net.in_dim if x.is_contiguous() else x.stride(0)
         if (tuple(dy.shape) != (M, net.out_dim) or (dx is not None and tuple(dx.shape) != (M, net.in_dim))
                 or (x is not None and (tuple(x.shape) != (M, net.in_dim) or x.dtype != torch.float32 or not x.is_cuda
-                                       or x.stride(1) != 1 or x.stride(0) < net.in_dim))):
+                                       or not (x.is_contiguous() or x.stride(1) == 1) or ldx < net.in_dim))):
             raise _lib.KsError("dy must be (M, out), dx and x (M, in) fp32 rows on the GPU, the columns of x side by side")
-        self.net, self.dy, self.x, self.dx = net, dy, x, dx
+        self.net, self.dy, self.x, self.dx, self.ldx = net, dy, x, dx, ldx
 
     def record(self) -> "T.KsLayerBackward":
-        return T.KsLayerBackward(self.net._handle.value, self.dy.shape[0], _lib.addr(self.x), 0 if self.x is None else self.x.stride(0),
-                                 _lib.addr(self.dy), _lib.addr(self.dx))
+        return T.KsLayerBackward(self.net._handle.value, self.dy.shape[0], _lib.addr(self.x), self.ldx, _lib.addr(self.dy), _lib.addr(self.dx))
 
 
 def run_layers(calls: Sequence[LayerForward]) -> None:

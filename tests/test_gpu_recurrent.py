@@ -615,3 +615,26 @@ def test_weight_gradients_layer_by_layer_are_those_of_one_launch(kind, dtype, H,
         results.append([g.clone() for n in nets for m in n.networks() for pair in m.parameters(gradients=True) for g in pair])
     assert len(results[0]) == 24 and all(bool(g.any()) for g in results[0])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_observations_of_one_column_train_whatever_its_stride(dtype):
+    """A contiguous array says nothing by the stride of a dimension of one entry: features first, then permuted, is the same rows."""
+    from ksim_amd.mlp import MLP
+    from ksim_amd.recurrent import GRUCell, RecurrentNetwork
+
+    H, steps, rows = 128, 4, 9
+    rng = np.random.default_rng(5)
+    w = lambda *s: rng.normal(scale=0.1, size=s)  # noqa: E731
+    net = RecurrentNetwork((w(H, 1), w(H)), [GRUCell(w(3 * H, H), w(3 * H, H), w(3 * H), w(H), dtype=dtype)], MLP([w(4, H)], [w(4)], activation="none", dtype=dtype),
+                           dtype=dtype)
+    net.train_init()
+    permuted = torch.randn(1, steps, rows, device="cuda").permute(1, 2, 0)
+    assert permuted.is_contiguous() and permuted.stride(2) != 1
+    carry, fresh, d_out = torch.zeros(1, rows, H, device="cuda"), torch.zeros(steps, rows, dtype=torch.uint8, device="cuda"), torch.randn(steps, rows, 4, device="cuda")
+    results = []
+    for obs in (permuted.clone(memory_format=torch.contiguous_format).view(-1).view(steps, rows, 1), permuted):
+        out = net.train_forward(obs, carry, fresh)
+        net.backward(d_out)
+        results.append([out] + [g.clone() for pair in net.input_proj.parameters(gradients=True) for g in pair])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
