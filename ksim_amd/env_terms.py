@@ -307,6 +307,7 @@ def sample_action(mean: torch.Tensor, log_std: torch.Tensor | None, *, noise: to
     """action = mean + exp(log_std) * N(0,1); NaN -> 0; clip to +-clip_max (ksim/task/rl.py:998-1001)."""
     lib = _lib.load()
     if out is None:
+        _lib.require_cuda(mean, dtype=torch.float32)
         out = torch.empty_like(mean)
     args = action_sample(mean, log_std, noise=noise, seed=seed, step=step, step_base=step_base, clip_max=clip_max, out=out)
     N, nu = mean.shape

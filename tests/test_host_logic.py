@@ -631,3 +631,13 @@ def test_the_minibatch_gather_leaves_what_it_cannot_count_to_torch():
 
     with pytest.raises(RuntimeError, match="same device"):
         pu._columns(torch.zeros(1, dtype=torch.int64), True, [(Cuda(), 1)])
+
+
+def test_sampling_refuses_what_is_no_tensor_on_the_gpu_as_every_entry_does():
+    import torch
+
+    from ksim_amd.env_terms import sample_action
+
+    for mean in (np.zeros((2, 3), np.float32), torch.zeros(2, 3)):
+        with pytest.raises(_lib.KsError, match="resident on the GPU"):
+            sample_action(mean, None)
