@@ -1,6 +1,7 @@
 // GRU and LSTM cells for recurrent policies in the rollout, and the GRU's backward pass through time.  The two gate projections are plain linear
 // layers and run through the MLP entry points (matrix cores for bf16); one streaming kernel then combines the gates.
 #include "ks_common.h"
+#include "ks_cut.h"
 
 #include <type_traits>
 #include <vector>
@@ -131,6 +132,26 @@ __global__ __launch_bounds__(256) void lstm_gate_train_kernel(int64_t M, int H, 
   sv[j] = si; sv[H + j] = sf; sv[2 * H + j] = tg; sv[3 * H + j] = so; sv[4 * H + j] = tc; sv[5 * H + j] = c; sv[6 * H + j] = h;
 }
 
+// What the gate gradients of an LSTM step take from its activations alone: factors of the gradient that reaches the cell state (the hidden state for the
+// output gate), and what of the latter reaches the former.
+struct LstmSlopes {
+  float i, f, g, o, cell, keep;
+  __device__ __forceinline__ void make(float si, float sf, float tg, float so, float tc, float c) {
+    i = tg * si * (1.f - si);
+    f = c * sf * (1.f - sf);
+    g = si * (1.f - tg * tg);
+    o = tc * so * (1.f - so);
+    cell = so * (1.f - tc * tc);
+    keep = sf;
+  }
+  // gate gradients i | f | g | o from those reaching h' and c'; returns that of the cell state
+  __device__ __forceinline__ float gates(float dh, float dc, float (&out)[4]) const {
+    const float dct = fmaf(dh, cell, dc);
+    out[0] = dct * i; out[1] = dct * f; out[2] = dct * g; out[3] = dh * o;
+    return dct;
+  }
+};
+
 // Backward through the gates of one LSTM step: dh_out, dc_out are the gradients reaching h' and c'.  d_g (M, 4H) is the
 // gradient of the summed gate pre-activations, hence of both projections' outputs; dc_in = dc f is the gradient of the
 // incoming cell state and dh_in starts at zero (the hidden projection adds its share afterwards); both are zero for a fresh env.
@@ -144,34 +165,35 @@ __global__ __launch_bounds__(256) void lstm_gate_backward_kernel(int64_t M, int 
   const int j = (int)(idx - m * H);
   const bool f = fresh && fresh[m];
   const float* sv = saved + m * 7 * H;
-  const float si = sv[j], sf = sv[H + j], tg = sv[2 * H + j], so = sv[3 * H + j], tc = sv[4 * H + j], c = sv[5 * H + j];
-  const float dh = dh_out[idx];
-  const float dc = dc_out[idx] + dh * so * (1.f - tc * tc);
+  LstmSlopes slope;
+  slope.make(sv[j], sv[H + j], sv[2 * H + j], sv[3 * H + j], sv[4 * H + j], sv[5 * H + j]);
+  float gate[4];
+  const float dct = slope.gates(dh_out[idx], dc_out[idx], gate);
   float* a = d_g + m * 4 * H;
-  a[j] = dc * tg * si * (1.f - si);
-  a[H + j] = dc * c * sf * (1.f - sf);
-  a[2 * H + j] = dc * si * (1.f - tg * tg);
-  a[3 * H + j] = dh * tc * so * (1.f - so);
-  dc_in[idx] = f ? 0.f : dc * sf;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k * H + j] = gate[k];
+  dc_in[idx] = f ? 0.f : dct * slope.keep;
   dh_in[idx] = 0.f;
 }
 
 // ---------------------------------------------------------------- a whole trajectory of one LSTM layer in one launch
 // The step-by-step path costs two GEMM launches and a gate kernel per step, layer and network: a minibatch of 100 control steps
-// is thousands of launches of a few microseconds each.  Here a workgroup of eight wavefronts owns 4 rows (envs) for all T
-// steps, so that a minibatch of a thousand rows is one workgroup per CU.  The product runs on v_mfma_f32_4x4x1 (sixteen
-// independent 4x4 outer products per instruction): block b = lane / 4 of wavefront w is hidden unit 16 w + b, its four B entries
-// are that unit's input / forget / cell / output rows of W_hh and the four A entries, the same for every block and therefore
-// broadcast from one block, the four rows' hidden state; after K = 128 instructions and a 4 x 4 transpose inside each group of
-// four lanes, lane (b, j) holds the four gate pre-activations of its unit for row j.  The wavefront's slice of W_hh stays in
-// 128 vector registers per lane for the whole sequence, the hidden state of the 4 rows lives in LDS (double buffered), the
-// cell state in a register; a step is 128 MFMAs (the fp32 matrix rate: 4 rows x 512 x 128 multiply-adds per CU), the gate
-// arithmetic of one (unit, row) per lane, and one barrier.  fp32 cells of hidden size 128.
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-// One recurrent layer over a trajectory, as the sequence kernels take it; a launch runs one or two of them (blockIdx.y): the actor's and the
-// critic's layer of one depth, which are as many workgroups as a batch has sets of 4 rows and leave half the chip idle below 1024 rows, each by
-// itself as long as the other.  Whole updates of an LSTM policy: 64 envs x 100 steps 2670 -> 1760 us, 512 x 60 2570 -> 2030, 2 x 128 x 80 with
-// mirror images 4740 -> 3530; with 1024 rows per network nothing changes.
+// is thousands of launches of a few microseconds each.  Here a workgroup of eight wavefronts owns 4 or 8 rows (envs) for all T
+// steps, so that a minibatch of a thousand rows is one workgroup per CU.  A wavefront's 16 units keep their slice of W_hh for the whole sequence, cut
+// in three bf16 parts (ks_cut.h): two parts in registers, the third in LDS.  A step is the products of the cut state with it (CutTile), the gate
+// arithmetic of one or two (unit, row) per lane, and one barrier.  fp32 cells of hidden size 128.
+// On v_mfma_f32_4x4x1, four rows a workgroup, a step's products took 2048 cycles for four rows; cut they take 1536 for four and 2048 for eight, and
+// they round less (the state after 100 steps is 1.8e-7 from 64 bits, the gate gradients 1.73e-7, of 1.78e-7).  Two layers (blockIdx.y), 100 steps, us:
+//   rows a layer:                     64         360 (60 steps)   1024
+//   forward, activations kept     154 -> 128   112 -> 102       435 -> 342
+//   forward, not kept             136 -> 124                    335 -> 236
+//   backward                      139 -> 119   102 -> 97        365 -> 287
+// With activations kept, 1024 rows move 1.2 GB, 240 us at the rate of a large copy.  What is left: issue, since only two vector instructions hide under
+// a 16-cycle matrix instruction (eight rows 4400 cycles a step, of which products 2048), the state's way through LDS at the head of a step (400), and the
+// clock, which falls to 1.9 GHz with every CU at work.  Also built: two sets of four rows half a step apart, one's gates between the other's products
+// (300 us of 240, not kept: nothing more hides, and four rows need 1.5 times the products); the backward product split over the gate rows instead
+// of over the units of dh (175 us of 119 for 64 rows: eight times the tiles' ends, and partial sums to add).
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 struct Seq {
   int64_t M;
   const float* in;  // forward: the input projections (T, M, gates); backward: dH
@@ -197,27 +219,13 @@ __device__ __forceinline__ float seq_tanh(float x) { return 1.f - 2.f * __builti
 // ahead for the next step) before every barrier, a memory round trip per step of the sequence.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The LSTM forward kernel's way in and out of memory: a step's inputs are requested a step ahead of their use.  Where the activations are kept, nine
-// results a step leave behind it, one load or store (KS_SEQ_SIDE, a single instruction from a uniform address) after every eight matrix instructions
-// of the next.  All together at a step's end they held the CU's wavefronts up at once, and a store or load under a condition makes the compiler wait
-// for the step's stores before the next step: loads and stores are counted together and waited for in order.  Hence no conditions (the outputs that
-// a launch has are template arguments, rows past the batch repeat the last row and store its values once more, the last step requests its own inputs
-// again) and nothing pending where the loop is entered.  Without kept activations a step stores one or two values, and the order imposed on its
-// matrix instructions costs more than it gives: loads at its start, stores at its end, the rest as the compiler likes.
-// Two layers, everything at the step's end and under conditions -> one after every eight -> as here:
-//   1024 rows x 100 steps, kept 372 -> 358 -> 358 us, not kept 302 -> 314 -> 298; 64 x 100, not kept 145 -> 155 -> 136; 512 x 24 with cell states
-//   43.9 -> 45.7 -> 41.7; one step (a rollout's call) of 4096 rows 34.6 -> 34.4 -> 33.6, of 64 10.3 -> 10.5 -> 10.3
-// What is left is issue and power: 2048 of 3500 cycles of a step are matrix instructions, at 2.0 to 2.2 GHz.  The backward kernel (342 -> 361 us) and
-// the GRU's (31 us either way) did not gain from the same order.
+// The LSTM kernels' way in and out of memory: a step's inputs are requested a step ahead of their use, and where the activations are kept, the nine
+// results a step leave between the matrix instructions of the next: together at a step's end they hold the CU's wavefronts up at once.  A store or load
+// under a condition makes the compiler wait for the step's stores before the next step (loads and stores are counted together and waited for in order).
+// Hence no conditions: the outputs that a launch has are template arguments, rows past the batch repeat the last row and store its values once more, the
+// last step requests its own inputs again, and nothing is pending where the loop is entered.
 __device__ __forceinline__ void seq_loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
-#define KS_SEQ_SIDE(OP)                \
-  {                                    \
-    __builtin_amdgcn_sched_barrier(0); \
-    OP;                                \
-    __builtin_amdgcn_sched_barrier(0); \
-  }
-
-// where hidden unit u of a row sits in the LDS copy of the state: unit u = 16 q + b is register q of block b (see the forward
+// GRU: where hidden unit u of a row sits in the LDS copy of the state: unit u = 16 q + b is register q of block b (see the forward
 // kernel), and a lane reads its block's 8 registers as 8 consecutive floats
 __device__ __forceinline__ int seq_slot(int u) { return 8 * (u & 15) + (u >> 4); }
 
@@ -254,240 +262,582 @@ __device__ __forceinline__ float rows_reduce_scatter(float v0, float v1, float v
   return lo + hi;
 }
 
-template <bool CELL, bool SAVE>
+constexpr int kLstmStateLd = kSeqH + 8;  // 16-bit entries of a row of the state; the padding puts neighbouring rows on different banks
+constexpr int lstm_forward_lds(int rows) { return kSeqWaves * 16 * 64 * 16 + 2 * 3 * rows * kLstmStateLd * 2; }
+
+constexpr float kLog2e = 1.44269504f;
+constexpr int kStepRows = 16;
+
+// holds a value, and with it the arithmetic that follows, to its place between two matrix instructions
+__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
+
+// A 16-column tile of the product of R rows with fp32 weights, both cut in three (cut_bf16).  The parts are rows of the A operand, which has sixteen:
+//   R = 8: rows 0..7 and 8..15 of `a` are first and second parts, `b` has the third parts twice: four instructions per 32 k.
+//   R = 4: rows 0..3, 4..7, 8..11 of `a` are first, second and third parts, `b` is `a` without the third: three instructions per 32 k.
+// The first and second parts times all parts of the weights and the third parts times the first are seven of the nine products; the two that are left out are
+// below 2^-23 and 2^-32 of the result.  Each part's products go into a sum of their own in order of k, and an entry is s0 + (s1 + s2): its bits do not
+// depend on R.
+//   SPLIT: the weights' second and third parts go into a sum of their own, so that with R = 4 the third parts' rows of it are left out at the end and `b` is
+//   not needed: for a single tile over a long reduction, where masking `a` costs more than four additions.
+template <int R, bool SPLIT>
+struct CutTile {
+  static constexpr int kSteps = R == 8 ? 4 : 3;  // matrix instructions per 32 k
+  f32x4 ab, third, rest;
+  __device__ __forceinline__ void clear() { ab = third = rest = f32x4{0.f, 0.f, 0.f, 0.f}; }
+  __device__ __forceinline__ void add(int step, bf16x8 a, bf16x8 b, bf16x8 w0, bf16x8 w1, bf16x8 w2) {
+    f32x4& low = SPLIT ? rest : ab;
+    if (step == 0) ab = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w0, ab, 0, 0, 0);
+    if (R == 8 && step == 1) third = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, w0, third, 0, 0, 0);
+    if (step == kSteps - 2) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(R == 8 || SPLIT ? a : b, w1, low, 0, 0, 0);
+    if (step == kSteps - 1) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(R == 8 || SPLIT ? a : b, w2, low, 0, 0, 0);
+  }
+  // In kRows pieces, which stand between matrix instructions: lane l gets column l % 16 of rows seq_row<R>(l) + q in out[q].  TAME: no operand is
+  // infinite and no sum overflows; otherwise, with SPLIT, the first parts decide (join_cut).  `upper`, 0 or 1: with R = 8 the lanes 32..63, which hold the
+  // second parts' rows; with R = 4 and SPLIT those that don't hold third parts' rows; 0 with R = 4 otherwise.  The swaps' operands come out of vector
+  // instructions, never straight out of a matrix instruction: nothing inserts that one's wait states into the asm.  (The builtins give the same
+  // result twice where both are used.)
+  static constexpr int kRows = 4;
+  template <bool TAME>
+  __device__ __forceinline__ void rows(int piece, float& upper, float (&t)[4], float (&out)[R / 4]) const {
+    if (piece < 2) {
+      pin(upper);
+#pragma unroll
+      for (int i = 2 * piece; i < 2 * piece + 2; ++i) {
+        if constexpr (SPLIT && R == 4) t[i] = TAME ? fmaf(rest[i], upper, ab[i]) : join_cut(ab[i], upper != 0.f ? rest[i] : 0.f);
+        else if constexpr (SPLIT) t[i] = TAME ? fmaf(third[i], upper, ab[i] + rest[i]) : join_cut(ab[i], rest[i] + (upper != 0.f ? third[i] : 0.f));
+        else t[i] = R == 4 ? ab[i] + upper : fmaf(third[i], upper, ab[i]);
+      }
+    }
+    if constexpr (R == 8) {
+      if (piece == 2)
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
+      if (piece == 3) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) out[q] = TAME ? t[q] + t[q + 2] : join_cut(t[q], t[q + 2]);
+      }
+    } else {
+      if (piece == 2)  // register i of lane row q changes places with register q of lane row i
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
+                     "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1"
+                     : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
+      if (piece == 3) out[0] = TAME ? t[0] + (t[1] + t[2]) : join_cut(t[0], t[1] + t[2]);
+    }
+  }
+};
+template <int R>
+__device__ __forceinline__ int seq_row(int lane) { return R == 8 ? 4 * ((lane >> 4) & 1) + 2 * (lane >> 5) : lane >> 4; }
+template <int R>  // the row of `a` that lane l holds, among R first, R second and R third parts
+__device__ __forceinline__ int cut_row(int lane) { return R == 8 || (lane & 15) < 12 ? lane & 15 : 11; }
+template <int R>
+__device__ __forceinline__ void get_cut(const unsigned short* rows, int ld, int lane, int k, bf16x8& a, bf16x8& b) {
+  a = *reinterpret_cast<const bf16x8*>(rows + cut_row<R>(lane) * ld + k);
+  if constexpr (R == 8) b = *reinterpret_cast<const bf16x8*>(rows + (16 + (lane & 7)) * ld + k);
+  else b = (lane & 8) ? bf16x8{} : a;
+}
+// Sums of 512 products of tame operands do not overflow.  The upper halves of two values at a time; infinities and NaN are larger than all others.
+__device__ __forceinline__ void largest(unsigned halves, u16x2& most) {
+  most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, halves & 0x7fff7fffu));
+}
+__device__ __forceinline__ bool wild(u16x2 most) { return (most.x > most.y ? most.x : most.y) >= 0x5d80; }  // 2^60
+
+// the entry `bytes` after base[entries], whose address is the same for every lane
+template <typename T>
+__device__ __forceinline__ T& at(T* base, int64_t entries, unsigned bytes) {
+  typedef typename std::conditional<std::is_const<T>::value, const char, char>::type Byte;
+  return *reinterpret_cast<T*>(reinterpret_cast<Byte*>(base + entries) + bytes);
+}
+
+template <int R, bool CELL, bool SAVE>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
-  constexpr int H = kSeqH;
+  constexpr int H = kSeqH, KB = H / 32, V = R / 4;
   const Seq s = blockIdx.y == 0 ? first : second;
   const int64_t M = s.M;
   const float* __restrict__ gi = s.in;
   const float* __restrict__ W = (const float*)s.W;
   const int ldw = s.ldw;
   const float *h0 = s.h0, *c0 = s.c0;
-  const uint8_t* __restrict__ fresh = s.fresh;
+  // without episode starts a byte of the inputs is read in the flag's place and masked away
+  const uint8_t* __restrict__ fresh = s.fresh ? s.fresh : (const uint8_t*)s.in;
+  const unsigned fresh_mask = s.fresh ? 0xffu : 0u;
   float *hs = s.out0, *cs = s.out1;  // with T = 1, hs / cs may be h0 / c0
   float* __restrict__ saved = s.saved;
-  __shared__ __attribute__((aligned(16))) float sh[2][kSeqRows][kSeqPadH];
+  if ((int64_t)blockIdx.x * groups * R >= M) return;  // the other layer of the launch has more rows
+  extern __shared__ __attribute__((aligned(16))) unsigned char seq_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int j = lane & 3, unit = 16 * wave + (lane >> 2);
-  // The weights are the B operand: block b, entry lane % 4: W_hh[gate lane % 4, unit][k].  The hidden state is the A operand and
-  // is the same for all sixteen blocks, so it is broadcast from one block per instruction (CBSZ = 4, ABID = k % 16): the four
-  // lanes of block k % 16 hold h[row 0..3][k] in register k / 16, i.e. the 512 values of the state sit once in 8 registers of the
-  // wavefront instead of once per block.  In LDS the state is stored in that order (row, block, register), two 16-byte reads per
-  // lane and step.
-  float wa[H];
-  {
-    const float4* src = reinterpret_cast<const float4*>(W + (int64_t)(j * H + unit) * ldw);
+  const int unit = 16 * wave + (lane & 15), row = seq_row<R>(lane), kq = 8 * (lane >> 4);
+  u32x4* w2 = reinterpret_cast<u32x4*>(seq_lds) + wave * 16 * 64 + lane;  // fragment (tile, k block) 64 entries on
+  typedef unsigned short State[3 * R][kLstmStateLd];
+  State* sh = reinterpret_cast<State*>(seq_lds + kSeqWaves * 16 * 64 * 16);  // of even and odd steps
+  // The tiles of a wavefront are its 16 units' forget, cell, input and output gates, in this order: all but the last one's arithmetic finds
+  // matrix instructions to stand between.  B operand: column lane % 16 is the unit, rows k = 32 kb + 8 (lane / 16) + 0..7.
+  constexpr int kGate[4] = {1, 2, 0, 3};
+  bf16x8 w0[4][KB], w1[4][KB];
+  u16x2 most = {};
 #pragma unroll
-    for (int k4 = 0; k4 < H / 4; ++k4) {
-      const float4 v = src[k4];
-      wa[4 * k4] = v.x; wa[4 * k4 + 1] = v.y; wa[4 * k4 + 2] = v.z; wa[4 * k4 + 3] = v.w;
+  for (int n = 0; n < 4; ++n) {
+    const float* src = W + (int64_t)(kGate[n] * H + unit) * ldw + kq;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const float4 lo = *reinterpret_cast<const float4*>(src + 32 * kb), hi = *reinterpret_cast<const float4*>(src + 32 * kb + 4);
+      const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      u32x4 part[3];
+      cut_bf16<3>(v, part);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) largest(part[0][e], most);
+      w0[n][kb] = __builtin_bit_cast(bf16x8, part[0]);
+      w1[n][kb] = __builtin_bit_cast(bf16x8, part[1]);
+      w2[(n * KB + kb) * 64] = part[2];
     }
   }
-  // A workgroup takes `groups` sets of 4 rows one after the other with the same registers of weights: a single step over
-  // thousands of rows (the rollout's call) would otherwise fetch the 256 KB of W_hh once per 4 rows.
+  // A workgroup takes `groups` sets of R rows one after the other with the same registers of weights: a single step over
+  // thousands of rows (the rollout's call) would otherwise fetch the 256 KB of W_hh once per set.
   for (int grp = 0; grp < groups; ++grp) {
-  const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * kSeqRows;
+  const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * R;
   if (r0 >= M) break;  // the same for every thread of the workgroup
-  const unsigned jr = r0 + j < M ? j : (unsigned)(M - 1 - r0);
-  const int64_t m = r0 + jr;
+  // the lane's rows and their bytes into a step's states, inputs and kept activations; rows past the batch repeat the last one and store its values once more
+  unsigned jr[V], oh[V], og[V], ov[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    jr[q] = r0 + row + q < M ? row + q : (unsigned)(M - 1 - r0);
+    oh[q] = (jr[q] * H + unit) * 4;
+    og[q] = (jr[q] * 4 * H + unit) * 4;
+    ov[q] = (jr[q] * 7 * H + unit) * 4;
+  }
   if (grp > 0) __syncthreads();  // the previous set's last read of the state buffers is over
-  float c = c0[m * H + unit];
-  float hprev = h0[m * H + unit];  // the state this lane's (unit, row) enters the step with
-  sh[0][j][seq_slot(unit)] = hprev;
-  struct In { float g[4]; unsigned f; } in0 = {}, in1 = {};
-  float si = 0.f, sf = 0.f, tg = 0.f, so = 0.f, tc = 0.f, cp = 0.f, hu = 0.f;
-  auto load = [&](int t, In& in, int k) __attribute__((always_inline)) {
+  // c, h: the states this lane's (unit, rows) leave a step with, g: its inputs by gate, requested a step ahead, v: its activations i | f | g | o | tanh(c')
+  // and the states it started from, which are zero in an episode's first step
+  float c[V], h[V], g[V][4], v[V][7];
+  unsigned flag[V];
+  auto load = [&](int t, int gate, int q) __attribute__((always_inline)) {
     const int64_t o = (int64_t)(t < T ? t : T - 1) * M + r0;
-    if (k < 4) in.g[k] = (gi + (o * 4 + k) * H)[jr * 4 * H + unit];
-    else if (fresh) in.f = (fresh + o)[jr];
+    if (gate < 4) g[q][gate] = at(gi, (o * 4 + gate) * H, og[q]);
+    else flag[q] = at(fresh, o, jr[q]);
   };
-  auto store = [&](int t, int k) __attribute__((always_inline)) {
+  auto store = [&](int t, int k, int q) __attribute__((always_inline)) {
     const int64_t o = (int64_t)t * M + r0;
-    if (k == 0) (hs + o * H)[jr * H + unit] = hprev;
-    if (CELL && k == 1) (cs + o * H)[jr * H + unit] = c;
-    if (SAVE && k >= 2) {
-      const float v[7] = {si, sf, tg, so, tc, cp, hu};
-      (saved + (o * 7 + k - 2) * H)[jr * 7 * H + unit] = v[k - 2];
+    if (k == 0) at(hs, o * H, oh[q]) = h[q];
+    if (CELL && k == 1) at(cs, o * H, oh[q]) = c[q];
+    if (SAVE && k >= 2) at(saved, (o * 7 + k - 2) * H, ov[q]) = v[q][k - 2];
+  };
+  float hn[V], cn[V];  // the states the next step starts from
+  auto begin = [&](int to) __attribute__((always_inline)) {
+    unsigned part[3];
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const bool f = (flag[q] & fresh_mask) != 0;
+      hn[q] = f ? 0.f : h[q];
+      cn[q] = f ? 0.f : c[q];
     }
+    cut_pair(hn[0], hn[V - 1], part);
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int q = 0; q < V; ++q) sh[to][p * R + row + q][unit] = (unsigned short)(part[p] >> (16 * q));
+    return part[0];
   };
 #pragma unroll
-  for (int k = 0; k < 5; ++k) load(0, in0, k);
+  for (int q = 0; q < V; ++q) {
+    c[q] = at(c0, r0 * H, oh[q]);
+    h[q] = at(h0, r0 * H, oh[q]);
+#pragma unroll
+    for (int gate = 0; gate < 5; ++gate) load(0, gate, q);
+  }
+  largest(begin(0), most);
   seq_loads_done();
-  __syncthreads();
-  auto step = [&](int t, auto cur, bool first, const In& in, In& next) __attribute__((always_inline)) {
-    if constexpr (!SAVE) {
+  const bool tame = !__syncthreads_or(wild(most));  // later states are below 1
+  auto steps = [&](auto tame) __attribute__((always_inline)) {
+    constexpr bool TAME = decltype(tame)::value;
+    typedef CutTile<R, !TAME> Tile;  // the first parts' products by themselves where they may have to decide
+    float upper = (R == 8 || !TAME) && (lane >= 32) == (R == 8) ? 1.f : 0.f;
+    float x[V] = {}, t4[4] = {};
+    // A tile's gate, in pieces of a few instructions (`x` carries the value from one to the next): activation(x) of the hardware exponential and
+    // reciprocal (about 1 ulp each) instead of the library's expf, tanhf and IEEE division, a fifth of the instructions.
+    constexpr int kAct = R == 8 ? 8 : 5;
+    auto act = [&](int gate, int piece) __attribute__((always_inline)) {
+      auto add_input = [&](int q) { x[q] = g[q][gate] + x[q]; };
+      auto scale = [&](int q) { x[q] *= gate == 2 ? 2.f * kLog2e : -kLog2e; };
+      auto power = [&](int q) { x[q] = __builtin_amdgcn_exp2f(x[q]); };
+      auto invert = [&](int q) { x[q] = __builtin_amdgcn_rcpf(x[q]); };
+      auto finish = [&](int q) { v[q][gate] = gate == 2 ? fmaf(-2.f, x[q], 1.f) : x[q]; };
+      if constexpr (R == 8) {
+        if (piece == 0) add_input(0), add_input(1);
+        if (piece == 1) scale(0), scale(1);
+        if (piece == 2 || piece == 3) power(piece - 2);
+        if (piece == 4) x[0] += 1.f, x[1] += 1.f;
+        if (piece == 5 || piece == 6) invert(piece - 5);
+        if (piece == 7) finish(0), finish(1);
+      } else {
+        if (piece == 0) add_input(0);
+        if (piece == 1) scale(0);
+        if (piece == 2) power(0);
+        if (piece == 3) x[0] += 1.f, invert(0);
+        if (piece == 4) finish(0);
+      }
+    };
+    auto step = [&](int t, auto from, bool first) __attribute__((always_inline)) {
+      bf16x8 a[KB], b[KB];
 #pragma unroll
-      for (int k = 0; k < 5; ++k) load(t + 1, next, k);
+      for (int kb = 0; kb < KB; ++kb) get_cut<R>(&sh[from][0][0], kLstmStateLd, lane, 32 * kb + kq, a[kb], b[kb]);
+      u32x4 ring[2] = {w2[0], w2[64]};
+      Tile tile, done;
+      constexpr int S = Tile::kSteps, N = KB * S;  // matrix instructions per 32 k and per tile
+      constexpr int R0 = 2, A0 = R0 + Tile::kRows, L0 = A0 + kAct;
+      static_assert(L0 + V <= N && 9 * V <= 2 * N, "");
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        if (n > 0) done = tile;
+        tile.clear();
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const int kb = i / S, slot = n * KB + kb;
+          tile.add(i % S, a[kb], b[kb], w0[n][kb], w1[n][kb], __builtin_bit_cast(bf16x8, ring[slot % 2]));
+          if (i % S == S - 1 && slot + 2 < 4 * KB) ring[slot % 2] = w2[(slot + 2) * 64];
+          // between the matrix instructions: under the first tile the last step's results leave; under the next ones the gate of the tile before
+          __builtin_amdgcn_sched_barrier(0);
+          if (n == 0) {
+            if (SAVE && !first) {
+#pragma unroll
+              for (int k = 9 * V * i / N; k < 9 * V * (i + 1) / N; ++k) store(t - 1, k / V, k % V);
+            }
+            if (i == N - 1) {
+#pragma unroll
+              for (int q = 0; q < V; ++q) {
+                load(t + 1, 4, q);
+                v[q][5] = cn[q];
+                v[q][6] = hn[q];
+              }
+            }
+          } else {
+            const int gate = kGate[n - 1];
+            if (i >= R0 && i < L0) {
+#pragma unroll
+              for (int k = 0; k < 4; ++k) pin(t4[k]);
+#pragma unroll
+              for (int q = 0; q < V; ++q) pin(x[q]);
+              if (i < A0) done.template rows<TAME>(i - R0, upper, t4, x);
+              else act(gate, i - A0);
+            }
+            if (i >= L0 && i < L0 + V) load(t + 1, gate, i - L0);
+            if (n == 3 && i == N - 1) {
+#pragma unroll
+              for (int q = 0; q < V; ++q) c[q] = fmaf(v[q][1], v[q][5], v[q][0] * v[q][2]);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      // what has no more matrix instructions to stand between: tanh of the cell state and the output gate
+#pragma unroll
+      for (int k = 0; k < Tile::kRows; ++k) tile.template rows<TAME>(k, upper, t4, x);
+#pragma unroll
+      for (int k = 0; k < kAct; ++k) act(3, k);
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        v[q][4] = seq_tanh(c[q]);
+        h[q] = v[q][3] * v[q][4];
+      }
+      begin(1 - decltype(from)::value);
+#pragma unroll
+      for (int q = 0; q < V; ++q) load(t + 1, 3, q);
+      if constexpr (!SAVE) {
+#pragma unroll
+        for (int k = 0; k < 2 * V; ++k) store(t, k / V, k % V);
+      }
+      lds_barrier();  // the new state is complete; the buffer just read is free for the step after next
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    step(0, even, true);
+    int t = 1;
+    for (; t + 1 < T; t += 2) {
+      step(t, odd, false);
+      step(t + 1, even, false);
     }
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    float ha[8];
-    {
-      const float4 a0 = *reinterpret_cast<const float4*>(&sh[cur][j][8 * (lane >> 2)]);
-      const float4 a1 = *reinterpret_cast<const float4*>(&sh[cur][j][8 * (lane >> 2) + 4]);
-      ha[0] = a0.x; ha[1] = a0.y; ha[2] = a0.z; ha[3] = a0.w; ha[4] = a1.x; ha[5] = a1.y; ha[6] = a1.z; ha[7] = a1.w;
+    if (t < T) step(t, odd, false);
+    if constexpr (SAVE) {
+#pragma unroll
+      for (int k = 0; k < 9 * V; ++k) store(T - 1, k / V, k % V);
     }
-    // k runs 0..127 in order, even k into one accumulator and odd k into the other
-#define KS_SEQ_MFMA(K0)                                                                                            \
-    acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[(K0) >> 4], wa[(K0)], acc0, 4, (K0) & 15, 0);                       \
-    acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ha[((K0) + 1) >> 4], wa[(K0) + 1], acc1, 4, ((K0) + 1) & 15, 0);
-#define KS_SEQ_MFMA8(N, OP) KS_SEQ_MFMA(8 * N) KS_SEQ_MFMA(8 * N + 2) KS_SEQ_MFMA(8 * N + 4) KS_SEQ_MFMA(8 * N + 6) if constexpr (SAVE) KS_SEQ_SIDE(OP)
-#define KS_SEQ_OUT(N) KS_SEQ_MFMA8(N, if (!first) store(t - 1, N))
-#define KS_SEQ_IN(N) KS_SEQ_MFMA8(N, load(t + 1, next, 13 - N))
-    KS_SEQ_OUT(0) KS_SEQ_OUT(1) KS_SEQ_OUT(2) KS_SEQ_OUT(3) KS_SEQ_OUT(4) KS_SEQ_OUT(5) KS_SEQ_OUT(6) KS_SEQ_OUT(7) KS_SEQ_OUT(8)
-    KS_SEQ_IN(9) KS_SEQ_IN(10) KS_SEQ_IN(11) KS_SEQ_IN(12) KS_SEQ_IN(13) KS_SEQ_MFMA8(14, ) KS_SEQ_MFMA8(15, )
-#undef KS_SEQ_IN
-#undef KS_SEQ_OUT
-#undef KS_SEQ_MFMA8
-#undef KS_SEQ_MFMA
-    // lane (unit, gate lane % 4) now holds that gate for the four rows in its four registers; the gates want the transpose
-    // within each group of four lanes: lane (unit, row j) with the four gates
-    float pre[4];
-    quad_transpose(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3], j, pre);
-    const bool f = in.f != 0;
-    cp = f ? 0.f : c;
-    hu = f ? 0.f : hprev;
-    // the hardware exponential and reciprocal (about 1 ulp each) instead of the library's expf, tanhf and IEEE division: a
-    // fifth of the instructions, and the gates are as many instructions per step as the matrix work is cycles
-    si = seq_sigmoid(in.g[0] + (f ? 0.f : pre[0]));
-    sf = seq_sigmoid(in.g[1] + (f ? 0.f : pre[1]));
-    tg = seq_tanh(in.g[2] + (f ? 0.f : pre[2]));
-    so = seq_sigmoid(in.g[3] + (f ? 0.f : pre[3]));
-    c = sf * cp + si * tg;
-    tc = seq_tanh(c);
-    hprev = so * tc;
-    sh[cur ^ 1][j][seq_slot(unit)] = hprev;
-    if constexpr (!SAVE) { store(t, 0); store(t, 1); }
-    lds_barrier();  // the new hidden state is complete; the buffer just read is free for the step after next
   };
-  constexpr std::integral_constant<int, 0> even{};
-  constexpr std::integral_constant<int, 1> odd{};
-  step(0, even, true, in0, in1);
-  int t = 1;
-  for (; t + 1 < T; t += 2) {
-    step(t, odd, false, in1, in0);
-    step(t + 1, even, false, in0, in1);
+  if (tame) steps(std::true_type{});
+  else steps(std::false_type{});
   }
-  if (t < T) step(t, odd, false, in1, in0);
-  if constexpr (SAVE) {
+}
+
+// A single step (a rollout's call: T = 1, hs / cs may be h0 / c0), to the same bits: with no next step to keep the weights for, a workgroup takes sixteen
+// rows, whose three parts are an A operand each, and streams W_hh through its wavefronts, cut on the way.  It asks for neither the registers nor the
+// LDS that would keep a CU to itself.  Two layers, through the sequence kernels -> here: 4096 rows 34.6 -> 22.1 us, 1000 20.2 -> 11.6, 64 10.3 -> 10.7;
+// a rollout's control step of 4096 robots, whose physics runs beside the critic's layers, 421 -> 400.
+template <bool CELL, bool SAVE>
+__global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void lstm_step_kernel(Seq first, Seq second) {
+  constexpr int H = kSeqH, KB = H / 32, R = kStepRows;
+  const Seq s = blockIdx.y == 0 ? first : second;
+  const int64_t M = s.M, r0 = (int64_t)blockIdx.x * R;
+  if (r0 >= M) return;  // the other layer of the launch has more rows
+  const float *W = (const float*)s.W, *gi = s.in;
+  const int ldw = s.ldw;
+  __shared__ __attribute__((aligned(16))) unsigned short sh[3][R][kLstmStateLd];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int unit = 16 * wave + (lane & 15), kq = 8 * (lane >> 4);
+  // the tiles are the unit's gates in the order below, their weights fetched a tile (four blocks of 32 k) ahead
+  constexpr int kGate[4] = {1, 2, 0, 3};
+  float4 w[KB][2];
+  auto fetch = [&](int slot) __attribute__((always_inline)) {
+    const float* src = W + (int64_t)(kGate[slot / KB] * H + unit) * ldw + 32 * (slot % KB) + kq;
+    w[slot % KB][0] = *reinterpret_cast<const float4*>(src);
+    w[slot % KB][1] = *reinterpret_cast<const float4*>(src + 4);
+  };
 #pragma unroll
-    for (int k = 0; k < 9; ++k) store(T - 1, k);
+  for (int slot = 0; slot < KB; ++slot) fetch(slot);
+  {
+    const int row = threadIdx.x >> 5, k = 4 * (threadIdx.x & 31);
+    const int64_t m = r0 + row < M ? r0 + row : M - 1;
+    float4 h = *reinterpret_cast<const float4*>(s.h0 + m * H + k);
+    if (s.fresh && s.fresh[m]) h = float4{0.f, 0.f, 0.f, 0.f};
+    unsigned lo[3], hi[3];
+    cut_pair(h.x, h.y, lo);
+    cut_pair(h.z, h.w, hi);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(&sh[p][row][k]) = uint2{lo[p], hi[p]};
   }
+  // this lane's unit in rows 4 (lane / 16) + 0..3; rows past the batch repeat the last one and store its values once more
+  const int64_t rows_left = M - r0;
+  unsigned row[4];
+  float c[4], h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    row[i] = 4 * (lane >> 4) + i;
+    if (row[i] >= rows_left) row[i] = (unsigned)(rows_left - 1);
+    const bool f = s.fresh && s.fresh[r0 + row[i]];
+    c[i] = f ? 0.f : at(s.c0, r0 * H, (row[i] * H + unit) * 4);
+    if (SAVE) h[i] = f ? 0.f : at(s.h0, r0 * H, (row[i] * H + unit) * 4);
+  }
+  float g[2][4];
+  auto inputs = [&](int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[n % 2][i] = at(gi, (r0 * 4 + kGate[n]) * H, (row[i] * 4 * H + unit) * 4);
+  };
+  inputs(0);
+  __syncthreads();  // all states are read: from here on the outputs may be written over them
+  auto mma = [](bf16x8 x, u32x4 y, f32x4& acc) __attribute__((always_inline)) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, y), acc, 0, 0, 0);
+  };
+  float v[4][4];  // by gate
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int gate = kGate[n];
+    float pre[4];
+    if (n + 1 < 4) inputs(n + 1);
+    f32x4 sum[3] = {};  // of the state's parts: CutTile's products in its order
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int slot = n * KB + kb;
+      const float4 lo = w[kb][0], hi = w[kb][1];
+      if (slot + KB < 4 * KB) fetch(slot + KB);
+      bf16x8 a[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[p] = *reinterpret_cast<const bf16x8*>(&sh[p][lane & 15][32 * kb + kq]);
+      const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      u32x4 part[3];
+      cut_bf16<3>(x, part);
+      mma(a[0], part[0], sum[0]);
+      mma(a[1], part[0], sum[1]);
+      mma(a[2], part[0], sum[2]);
+      mma(a[0], part[1], sum[0]);
+      mma(a[1], part[1], sum[1]);
+      mma(a[0], part[2], sum[0]);
+      mma(a[1], part[2], sum[1]);
+    }
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pre[i] = sum[0][i] + (sum[1][i] + sum[2][i]);
+      finite = finite && fabsf(pre[i]) < __builtin_inff();
+    }
+    if (__any(!finite)) {  // the first parts decide, so their products go by themselves
+      f32x4 one[3] = {}, rest[2] = {};
+#pragma unroll 1
+      for (int kb = 0; kb < KB; ++kb) {
+        const float* src = W + (int64_t)(gate * H + unit) * ldw + 32 * kb + kq;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = src[e];
+        u32x4 part[3];
+        cut_bf16<3>(x, part);
+        bf16x8 b[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) b[p] = *reinterpret_cast<const bf16x8*>(&sh[p][lane & 15][32 * kb + kq]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) mma(b[p], part[0], one[p]);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          mma(b[p], part[1], rest[p]);
+          mma(b[p], part[2], rest[p]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pre[i] = join_cut(join_cut(one[0][i], rest[0][i]), join_cut(one[1][i], rest[1][i] + one[2][i]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // the arithmetic of the sequence kernel's pieces
+      float x = g[n % 2][i] + pre[i];
+      x *= gate == 2 ? 2.f * kLog2e : -kLog2e;
+      x = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      v[gate][i] = gate == 2 ? fmaf(-2.f, x, 1.f) : x;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float cn = fmaf(v[1][i], c[i], v[0][i] * v[2][i]), tc = seq_tanh(cn);
+    at(s.out0, r0 * H, (row[i] * H + unit) * 4) = v[3][i] * tc;
+    if (CELL) at(s.out1, r0 * H, (row[i] * H + unit) * 4) = cn;
+    if (SAVE) {
+      const float out[7] = {v[0][i], v[1][i], v[2][i], v[3][i], tc, c[i], h[i]};
+#pragma unroll
+      for (int k = 0; k < 7; ++k) at(s.saved, (r0 * 7 + k) * H, (row[i] * 7 * H + unit) * 4) = out[k];
+    }
   }
 }
 
 // The reverse sweep of the same layer: dH (T, M, H) is the gradient reaching h_t from the layer above; the gradient through
 // W_hh and that of the cell state are carried in registers.  Per step: the gate derivatives from the saved activations
-// (lstm_gate_backward_kernel's formulas) into d_g (T, M, 4H) and LDS, then dh_{t-1} = d_g W_hh over the transposed weights.
-// Here the sixteen blocks of an MFMA are four quarters of the 4H gate rows (K split four ways: quarter kg = lane / 16 is gate kg) times
-// four groups of four units.  The gate gradients are the A operand (entries = the four rows), the same for the four blocks of a quarter and
-// broadcast to them from one block per instruction (CBSZ = 2, ABID = k mod 4): a lane fetches 32 of its quarter's 128 gate rows, eight 16-byte
-// reads per step.  (Fetched by every block, they were 32 reads per lane, as many cycles of the LDS pipe as the products are of the matrix
-// cores.)  A lane accumulates, for its unit, the four rows' partial sums over its quarter; the quarters are added up and scattered over
-// the lane rows, which leaves lane l with unit 16 w + l % 16 of row l / 16.
-// 1024 rows, 100 steps: 248 -> 169 us, of which the 128 products of two wavefronts per SIMD are 85.
-// where the gradient of gate row g H + u of a row sits in LDS: lane (quarter g, block a = u mod 4, row) reads its 32 as consecutive floats;
-// the paddings put the sixteen lanes of a quarter on different banks
-constexpr int kSeqGateA = 36, kSeqGateRow = 4 * 4 * kSeqGateA + 16;
+// (lstm_gate_backward_kernel's formulas) into d_g (T, M, 4H) and, cut in three, into LDS, then dh_{t-1} = d_g W_hh over the transposed weights: a
+// wavefront's tile is its 16 units, over all 4H gate rows.  The weights' third parts lie in registers for kThirdRegs of the sixteen k blocks and in LDS
+// for the others.
+constexpr int kThirdRegs = 4, kLstmGateLd = 4 * kSeqH + 8;
+constexpr int lstm_backward_lds(int rows) { return kSeqWaves * (16 - kThirdRegs) * 64 * 16 + 2 * 3 * rows * kLstmGateLd * 2; }
 
+template <int R>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lstm_seq_backward_kernel(int T, Seq first, Seq second) {
-  constexpr int H = kSeqH;
+  constexpr int H = kSeqH, V = R / 4, KB = 4 * H / 32;
   const Seq s = blockIdx.y == 0 ? first : second;
   const int64_t M = s.M;
   const float* __restrict__ dH = s.in;
   const float* __restrict__ saved = s.saved;
-  const uint8_t* __restrict__ fresh = s.fresh;
+  const uint8_t* __restrict__ fresh = s.fresh ? s.fresh : (const uint8_t*)s.in;  // as in the forward kernel
+  const unsigned fresh_mask = s.fresh ? 0xffu : 0u;
   const float* __restrict__ Wt = (const float*)s.W;
   const int ldwt = s.ldw;
   float* __restrict__ d_g = s.out0;
   float *dh0 = s.dh0, *dc0 = s.dc0;
-  if ((int64_t)blockIdx.x * kSeqRows >= M) return;  // the other layer of the launch has more rows
-  __shared__ __attribute__((aligned(16))) float sg[2][kSeqRows * kSeqGateRow];
+  const int64_t r0 = (int64_t)blockIdx.x * R;
+  if (r0 >= M) return;  // the other layer of the launch has more rows
+  extern __shared__ __attribute__((aligned(16))) unsigned char seq_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kg = lane >> 4, blk = (lane >> 2) & 3, i = lane & 3;
-  const int unit = 16 * wave + (lane & 15);  // the (unit, row kg) whose gate arithmetic and carried gradients this lane owns
-  const int64_t r0 = (int64_t)blockIdx.x * kSeqRows;
-  const int64_t m = r0 + kg;
-  const bool row_ok = m < M;
-  const int64_t mc = row_ok ? m : M - 1;
-  // B operand, entry lane % 4 of block (kg, lane / 4 % 4): Wt[unit][gate row 128 kg + s]
-  float wa[128];
-  {
-    const float4* src = reinterpret_cast<const float4*>(Wt + (int64_t)unit * ldwt + 128 * kg);
+  const int unit = 16 * wave + (lane & 15), row = seq_row<R>(lane), kq = 8 * (lane >> 4);  // the (unit, rows) whose gates this lane owns
+  float upper = (lane >= 32) == (R == 8) ? 1.f : 0.f;
+  u32x4* w2 = reinterpret_cast<u32x4*>(seq_lds) + wave * (16 - kThirdRegs) * 64 + lane;  // k block kThirdRegs and on
+  typedef unsigned short Gates[3 * R][kLstmGateLd];
+  Gates* sg = reinterpret_cast<Gates*>(seq_lds + kSeqWaves * (16 - kThirdRegs) * 64 * 16);  // of even and odd steps
+  // the lane's rows and their bytes into a step's states, gates and kept activations; rows past the batch repeat the last one and store its values once more
+  unsigned jr[V], oh[V], og[V], ov[V];
 #pragma unroll
-    for (int s4 = 0; s4 < 32; ++s4) {
-      const float4 v = src[s4];
-      wa[4 * s4] = v.x; wa[4 * s4 + 1] = v.y; wa[4 * s4 + 2] = v.z; wa[4 * s4 + 3] = v.w;
-    }
+  for (int q = 0; q < V; ++q) {
+    jr[q] = r0 + row + q < M ? row + q : (unsigned)(M - 1 - r0);
+    oh[q] = (jr[q] * H + unit) * 4;
+    og[q] = (jr[q] * 4 * H + unit) * 4;
+    ov[q] = (jr[q] * 7 * H + unit) * 4;
   }
-  float dhc = 0.f, dc = 0.f;
-  const int put = kg * kSeqGateRow + (unit & 3) * kSeqGateA + (unit >> 2);  // of gate 0; the next gate 4 kSeqGateA on
-  const int get = i * kSeqGateRow + (4 * kg + blk) * kSeqGateA;
-  // the step's inputs from memory are fetched one step ahead, under the matrix work of the step before
-  float nx[7];
-  uint8_t fnext = 0;
-  {
-    const int64_t o = (int64_t)(T - 1) * M + mc;
-    const float* sv = saved + o * 7 * H + unit;
+  // B operand: column lane % 16 is the unit, rows the gate rows 32 kb + 8 (lane / 16) + 0..7
+  bf16x8 w0[KB], w1[KB], w2r[kThirdRegs];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) nx[k] = sv[k * H];
-    nx[6] = dH[o * H + unit];
-    if (fresh) fnext = fresh[o];
+  for (int kb = 0; kb < KB; ++kb) {
+    const float* src = Wt + (int64_t)unit * ldwt + 32 * kb + kq;
+    const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
+    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    u32x4 part[3];
+    cut_bf16<3>(v, part);
+    w0[kb] = __builtin_bit_cast(bf16x8, part[0]);
+    w1[kb] = __builtin_bit_cast(bf16x8, part[1]);
+    if (kb < kThirdRegs) w2r[kb < kThirdRegs ? kb : 0] = __builtin_bit_cast(bf16x8, part[2]);
+    else w2[(kb - kThirdRegs) * 64] = part[2];
   }
-  int cur = 0;
-  for (int t = T - 1; t >= 0; --t) {
-    const bool f = fnext != 0;
-    const float si = nx[0], sf = nx[1], tg = nx[2], so = nx[3], tc = nx[4], cp = nx[5];
-    const float dh = nx[6] + dhc;
-    if (t > 0) {
-      const int64_t o = (int64_t)(t - 1) * M + mc;
-      const float* sv = saved + o * 7 * H + unit;
+  float dhc[V], dc[V];
+  // a step's inputs i | f | g | o | tanh(c') | c | dH, requested under the products of the step before
+  float in[V][7];
+  unsigned flag[V];
+  auto load = [&](int t, int k, int q) __attribute__((always_inline)) {
+    const int64_t o = (int64_t)(t > 0 ? t : 0) * M + r0;
+    if (k < 6) in[q][k] = at(saved, (o * 7 + k) * H, ov[q]);
+    else if (k == 6) in[q][k] = at(dH, o * H, oh[q]);
+    else flag[q] = at(fresh, o, jr[q]);
+  };
 #pragma unroll
-      for (int k = 0; k < 6; ++k) nx[k] = sv[k * H];
-      nx[6] = dH[o * H + unit];
-      if (fresh) fnext = fresh[o];
+  for (int q = 0; q < V; ++q) {
+    dhc[q] = dc[q] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) load(T - 1, k, q);
+  }
+  float t4[4] = {};
+  auto step = [&](int t, auto cur) __attribute__((always_inline)) {
+    bool f[V];
+    float gate[V][4];
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      f[q] = (flag[q] & fresh_mask) != 0;
+      LstmSlopes slope;
+      slope.make(in[q][0], in[q][1], in[q][2], in[q][3], in[q][4], in[q][5]);
+      const float dct = slope.gates(in[q][6] + dhc[q], dc[q], gate[q]);
+      dc[q] = f[q] ? 0.f : dct * slope.keep;
     }
-    const float dct = dc + dh * so * (1.f - tc * tc);
-    const float gI = dct * tg * si * (1.f - si), gF = dct * cp * sf * (1.f - sf), gG = dct * si * (1.f - tg * tg),
-                gO = dh * tc * so * (1.f - so);
-    dc = f ? 0.f : dct * sf;
-    float* to = &sg[cur][put];
-    to[0] = gI; to[4 * kSeqGateA] = gF; to[8 * kSeqGateA] = gG; to[12 * kSeqGateA] = gO;
-    if (row_ok) {
-      float* dg = d_g + ((int64_t)t * M + m) * 4 * H + unit;
-      dg[0] = gI; dg[H] = gF; dg[2 * H] = gG; dg[3 * H] = gO;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      unsigned part[3];
+      cut_pair(gate[0][g], gate[V - 1][g], part);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int q = 0; q < V; ++q) sg[cur][p * R + row + q][g * H + unit] = (unsigned short)(part[p] >> (16 * q));
     }
     lds_barrier();  // the gate gradients are complete; the buffer of the step before is free for the step after
-    float ga[32];
-    {
-      const float4* src = reinterpret_cast<const float4*>(&sg[cur][get]);
+    bf16x8 a[4], b[4];
 #pragma unroll
-      for (int q4 = 0; q4 < 8; ++q4) {
-        const float4 v = src[q4];
-        ga[4 * q4] = v.x; ga[4 * q4 + 1] = v.y; ga[4 * q4 + 2] = v.z; ga[4 * q4 + 3] = v.w;
+    for (int kb = 0; kb < 3; ++kb) get_cut<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * kb + kq, a[kb], b[kb]);
+    CutTile<R, true> tile;
+    tile.clear();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (kb + 3 < KB) get_cut<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * (kb + 3) + kq, a[(kb + 3) % 4], b[(kb + 3) % 4]);
+#pragma unroll
+      for (int i = 0; i < CutTile<R, true>::kSteps; ++i)
+        tile.add(i, a[kb % 4], b[kb % 4], w0[kb], w1[kb],
+                 kb < kThirdRegs ? w2r[kb < kThirdRegs ? kb : 0] : __builtin_bit_cast(bf16x8, w2[(kb - (kb < kThirdRegs ? kb : kThirdRegs)) * 64]));
+      // between the products the step's gate gradients leave and the inputs of the next come
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        if (kb < 8) load(t - 1, kb, q);
+        else if (kb < 12) at(d_g, (((int64_t)t * M + r0) * 4 + kb - 8) * H, og[q]) = gate[q][kb - 8];
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    float x[V];
 #pragma unroll
-    for (int q = 0; q < 32; ++q) {  // k = 4 q .. 4 q + 3 of the quarter, even k into one accumulator and odd k into the other
-      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q], acc0, 2, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 1], acc1, 2, 1, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 2], acc0, 2, 2, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_4x4x1f32(ga[q], wa[4 * q + 3], acc1, 2, 3, 0);
+    for (int k = 0; k < CutTile<R, true>::kRows; ++k) tile.template rows<true>(k, upper, t4, x);
+    if (__any(!(fabsf(x[0]) < __builtin_inff()) || !(fabsf(x[V - 1]) < __builtin_inff()))) {  // where all is finite the other way would be no different
+#pragma unroll
+      for (int k = 0; k < CutTile<R, true>::kRows; ++k) tile.template rows<false>(k, upper, t4, x);
     }
-    const float mine = rows_reduce_scatter(acc0[0] + acc1[0], acc0[1] + acc1[1], acc0[2] + acc1[2], acc0[3] + acc1[3]);
-    dhc = f ? 0.f : mine;
-    cur ^= 1;
+#pragma unroll
+    for (int q = 0; q < V; ++q) dhc[q] = f[q] ? 0.f : x[q];
+  };
+  int t = T - 1;
+  for (; t >= 1; t -= 2) {
+    step(t, std::integral_constant<int, 0>{});
+    step(t - 1, std::integral_constant<int, 1>{});
   }
-  if (row_ok) {
-    if (dh0) dh0[m * H + unit] = dhc;
-    if (dc0) dc0[m * H + unit] = dc;
+  if (t == 0) step(0, std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    if (dh0) at(dh0, r0 * H, oh[q]) = dhc[q];
+    if (dc0) at(dc0, r0 * H, oh[q]) = dc[q];
   }
 }
 
 // ---------------------------------------------------------------- a whole trajectory of one GRU layer in one launch
-// The layout of the LSTM kernels above: eight wavefronts own 4 rows for all T steps, block b = lane / 4 of wavefront w is hidden
+// As for the LSTM, eight wavefronts own 4 rows for all T steps: block b = lane / 4 of wavefront w is hidden
 // unit 16 w + b, its B entries are that unit's reset / update / candidate rows of W_hh (the fourth entry is zero), and the four
 // rows' state is the A operand broadcast from one block per instruction.  fp32 cells multiply with v_mfma_f32_4x4x1 (128 per step);
 // bf16 cells with v_mfma_f32_4x4x4 bf16 (32 per step), for which the state, kept in fp32 in a register of the lane that owns it,
@@ -536,7 +886,7 @@ void gru_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
     }
   }
   const float bn = bias_n[unit];
-  for (int grp = 0; grp < groups; ++grp) {  // as in the LSTM kernel: several sets of 4 rows with the same registers of weights
+  for (int grp = 0; grp < groups; ++grp) {  // several sets of 4 rows with the same registers of weights
     const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * kSeqRows;
     if (r0 >= M) break;  // the same for every thread of the workgroup
     const int64_t m = r0 + j;
@@ -618,7 +968,9 @@ void gru_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
 }
 
 // The reverse sweep (gru_gate_backward_kernel's formulas): dh_{t-1} = dh_t z + d_gh W_hh.  Sixteen blocks = four quarters of the 3H gate
-// rows (96 each) times four groups of four units, operands and sums as in the LSTM's sweep; in bf16 a step of four k is one block's entry.
+// rows (96 each) times four groups of four units, in bf16 a step of four k is one
+// block's entry.  The gate gradients are the A operand (entries = the four rows), the same for the four blocks of a quarter and broadcast to them from one
+// block per instruction (CBSZ = 2, ABID = k mod 4); a lane's partial sums over its quarter are added up and scattered over the lane rows.
 template <bool BF>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gru_seq_backward_kernel(int T, Seq first, Seq second) {
@@ -833,8 +1185,8 @@ static int run_sequences(const char* who, int32_t n, int64_t T, const KsSequence
   if (m == 0) return KS_OK;
   if ((rows + kSeqRows - 1) / kSeqRows > 0x7fffffff || T > 0x7fffffff) return fail(KS_ELIMIT, "%s: too many rows or steps", who);
   if (m == 1) s[1] = s[0];
-  launch(s, m, (rows + kSeqRows - 1) / kSeqRows);
-  return check_launch(who);
+  const int rc = launch(s, m, (rows + kSeqRows - 1) / kSeqRows);
+  return rc != KS_OK ? rc : check_launch(who);
 }
 
 extern "C" int ks_gru_sequences_forward(ks_stream_t stream, int32_t n, int64_t T, const KsSequence* q) {
@@ -852,10 +1204,11 @@ extern "C" int ks_gru_sequences_forward(ks_stream_t stream, int32_t n, int64_t T
     s.bias_n = g->bn();
     return KS_OK;
   };
-  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) {
+  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) -> int {
     const int groups = seq_groups(T, sets);
     hipLaunchKernelGGL(bf[0] ? gru_seq_forward_kernel<true> : gru_seq_forward_kernel<false>, dim3((unsigned)((sets + groups - 1) / groups), (unsigned)count),
                        dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, groups, s[0], s[1]);
+    return KS_OK;
   });
 }
 
@@ -872,9 +1225,10 @@ extern "C" int ks_gru_sequences_backward(ks_stream_t stream, int32_t n, int64_t 
     if (m == 2 && bf[0] != bf[1]) return fail(KS_EINVAL, "%s: two layers of one precision", who);
     return KS_OK;
   };
-  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) {
+  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) -> int {
     hipLaunchKernelGGL(bf[0] ? gru_seq_backward_kernel<true> : gru_seq_backward_kernel<false>, dim3((unsigned)sets, (unsigned)count), dim3(64 * kSeqWaves), 0,
                        (hipStream_t)stream, (int)T, s[0], s[1]);
+    return KS_OK;
   });
 }
 
@@ -1071,6 +1425,19 @@ static bool lstm_seq_weights(const KsLstm* g, const float** W, int* ldw, const f
   return w != nullptr;
 }
 
+// Rows per workgroup: 8 once sets of 4 are more than the CUs, which hold one workgroup each.
+static bool lstm_wide(int count, const Seq& a, const Seq& b) {
+  return (a.M + 3) / 4 + (count > 1 ? (b.M + 3) / 4 : 0) > 256;
+}
+
+template <typename... P, typename... A>
+static int launch_lstm(const char* who, void (*fn)(P...), dim3 grid, int lds, ks_stream_t stream, A... args) {
+  if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return fail(KS_ELAUNCH, "%s: cannot reserve %d bytes of LDS", who, lds);
+  hipLaunchKernelGGL(fn, grid, dim3(64 * kSeqWaves), lds, (hipStream_t)stream, args...);
+  return KS_OK;
+}
+
 extern "C" int ks_lstm_sequence_supported(const KsLstm* g) {
   const float *W, *Wt;
   int a, b;
@@ -1088,21 +1455,31 @@ extern "C" int ks_lstm_sequences_forward(ks_stream_t stream, int32_t n, int64_t 
     s.W = W;
     return KS_OK;
   };
-  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) {
-    const int groups = seq_groups(T, sets);
-    const dim3 grid((unsigned)((sets + groups - 1) / groups), (unsigned)count);
-    auto run = [&](dim3 grid, const Seq& first, const Seq& second) {
+  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) -> int {
+    auto run = [&](int count, const Seq& first, const Seq& second) -> int {
       const bool cell = first.out1 != nullptr, save = first.saved != nullptr;
-      hipLaunchKernelGGL(cell ? (save ? lstm_seq_forward_kernel<true, true> : lstm_seq_forward_kernel<true, false>)
-                              : (save ? lstm_seq_forward_kernel<false, true> : lstm_seq_forward_kernel<false, false>),
-                         grid, dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, groups, first, second);
+      if (T == 1) {
+        const int64_t most = first.M > second.M ? first.M : second.M;
+        hipLaunchKernelGGL(cell ? (save ? lstm_step_kernel<true, true> : lstm_step_kernel<true, false>)
+                                : (save ? lstm_step_kernel<false, true> : lstm_step_kernel<false, false>),
+                           dim3((unsigned)((most + kStepRows - 1) / kStepRows), (unsigned)count), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, first, second);
+        return KS_OK;
+      }
+      const bool wide = lstm_wide(count, first, second);
+      const int rows = wide ? 8 : 4, groups = wide ? (seq_groups(T, sets) + 1) / 2 : seq_groups(T, sets);
+      auto fn = wide ? (cell ? (save ? lstm_seq_forward_kernel<8, true, true> : lstm_seq_forward_kernel<8, true, false>)
+                            : (save ? lstm_seq_forward_kernel<8, false, true> : lstm_seq_forward_kernel<8, false, false>))
+                    : (cell ? (save ? lstm_seq_forward_kernel<4, true, true> : lstm_seq_forward_kernel<4, true, false>)
+                            : (save ? lstm_seq_forward_kernel<4, false, true> : lstm_seq_forward_kernel<4, false, false>));
+      const int64_t M = first.M > second.M ? first.M : second.M;
+      return launch_lstm(who, fn, dim3((unsigned)((M + rows * groups - 1) / (rows * groups)), (unsigned)count), lstm_forward_lds(rows), stream, (int)T, groups,
+                         first, second);
     };
     if (count == 2 && (!s[0].out1 != !s[1].out1 || !s[0].saved != !s[1].saved)) {  // a kernel writes the same outputs for both of its layers
-      run(dim3(grid.x), s[0], s[0]);
-      run(dim3(grid.x), s[1], s[1]);
-    } else {
-      run(grid, s[0], s[1]);
+      const int rc = run(1, s[0], s[0]);
+      return rc != KS_OK ? rc : run(1, s[1], s[1]);
     }
+    return run(count, s[0], s[1]);
   });
 }
 
@@ -1117,8 +1494,10 @@ extern "C" int ks_lstm_sequences_backward(ks_stream_t stream, int32_t n, int64_t
     s.W = Wt;
     return KS_OK;
   };
-  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) {
-    hipLaunchKernelGGL(lstm_seq_backward_kernel, dim3((unsigned)sets, (unsigned)count), dim3(64 * kSeqWaves), 0, (hipStream_t)stream, (int)T, s[0], s[1]);
+  return run_sequences(who, n, T, q, fill, [&](const Seq* s, int count, int64_t sets) -> int {
+    const bool wide = lstm_wide(count, s[0], s[1]);
+    return launch_lstm(who, wide ? lstm_seq_backward_kernel<8> : lstm_seq_backward_kernel<4>, dim3((unsigned)(wide ? (sets + 1) / 2 : sets), (unsigned)count),
+                       lstm_backward_lds(wide ? 8 : 4), stream, (int)T, s[0], s[1]);
   });
 }
 

@@ -638,3 +638,56 @@ def test_observations_of_one_column_train_whatever_its_stride(dtype):
         net.backward(d_out)
         results.append([out] + [g.clone() for pair in net.input_proj.parameters(gradients=True) for g in pair])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("rows", [3, 1027])
+def test_lstm_sequences_take_infinite_and_very_large_operands_as_a_plain_product_does(rows):
+    """The products are made of three parts per operand, of which those of an infinity are NaN and those of large values overflow by themselves:
+    against the same steps in 64 bits, forward with such weights and initial states, backward with such gradients and weights, four and
+    eight rows per workgroup.  Finite entries to 2e-6 (a gate's preactivation to 1e-6 of a sum of 128 terms below 1, the hardware
+    exponential and reciprocal beside it), the others in kind."""
+    from ksim_amd.recurrent import LSTMCell
+
+    H, Tn = 128, 3
+    rng = np.random.default_rng(83)
+    for kind in ("ordinary", "infinite state", "large state", "infinite weight", "infinite gradient", "large gradient", "NaN gradient"):
+        w = [rng.normal(scale=H ** -0.5, size=s).astype(np.float32) for s in ((4 * H, H), (4 * H, H), (4 * H,))]
+        h0, c0 = (0.5 * rng.normal(size=(rows, H)).astype(np.float32) for _ in range(2))
+        x, dH = (rng.normal(size=(Tn, rows, H)).astype(np.float32) for _ in range(2))
+        if kind == "infinite state":
+            h0[rows - 1, 5] = np.inf
+        elif kind == "large state":
+            h0[0, 7] = -3e37
+        elif kind == "infinite weight":
+            w[1][3 * H + 9, 11] = -np.inf
+        elif kind.endswith("gradient"):
+            dH[1, rows - 1, 64] = {"infinite": -np.inf, "large": 1e36, "NaN": np.nan}[kind.split()[0]]
+        cell = LSTMCell(*w, dtype="f32")
+        cell.train_init()
+        z = lambda n: torch.zeros(Tn, rows, n * H, device=DEV)  # noqa: E731
+        hs, cs, sv, dg = z(1), z(1), z(7), z(4)
+        fresh = torch.zeros(Tn, rows, dtype=torch.uint8, device=DEV)
+        cell.sequence_forward(t32(x), t32(h0), t32(c0), fresh, hs, cs, sv)
+        wi, wh, b = (torch.from_numpy(a).double() for a in w)
+        h, c, want = torch.from_numpy(h0).double(), torch.from_numpy(c0).double(), []
+        for t in range(Tn):
+            i, f, g, o = (torch.from_numpy(x[t]).double() @ wi.T + b + h @ wh.T).chunk(4, 1)
+            i, f, g, o = i.sigmoid(), f.sigmoid(), g.tanh(), o.sigmoid()
+            cn = f * c + i * g
+            want.append((i, f, g, o, cn.tanh(), c))
+            h, c = o * cn.tanh(), cn
+            torch.testing.assert_close(hs[t].cpu().double(), h, rtol=2e-6, atol=2e-6, equal_nan=True, msg=lambda m: f"{kind}, step {t}: {m}")
+        if "state" in kind or "weight" in kind:
+            continue
+        cell.sequence_backward(t32(dH), sv, fresh, dg)
+        dh = dc = torch.zeros(rows, H, dtype=torch.float64)
+        for t in reversed(range(Tn)):
+            i, f, g, o, tc, cp = want[t]
+            d = torch.from_numpy(dH[t]).double() + dh
+            dct = dc + d * o * (1 - tc * tc)
+            gates = torch.cat([dct * g * i * (1 - i), dct * cp * f * (1 - f), dct * i * (1 - g * g), d * tc * o * (1 - o)], 1)
+            got = dg[t].cpu().double()
+            assert torch.equal(got.isnan(), gates.isnan()) and torch.equal(got.isinf(), gates.isinf()), (kind, t)
+            scale = gates.abs().nan_to_num(0, 0, 0).amax(1, keepdim=True).clamp_min(1)
+            torch.testing.assert_close((got / scale).nan_to_num(0, 0, 0), (gates / scale).nan_to_num(0, 0, 0), rtol=0, atol=4e-6, msg=lambda m: f"{kind}, step {t}: {m}")
+            dc, dh = dct * f, gates @ wh
