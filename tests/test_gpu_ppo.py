@@ -193,3 +193,36 @@ def test_outputs_are_tensors_of_their_own():
         assert t._base is None and t.is_contiguous() and t.data_ptr() % 16 == 0
         assert t.untyped_storage().nbytes() == t.numel() * 4
         t.mul_(scale)  # raises on one of several views
+
+
+@pytest.mark.parametrize("n,A", [(1, 3), (256, 1), (257, 20), (1024 * 256 + 77, 2)])
+def test_ppo_loss_total_of_any_number_of_blocks_and_in_a_graph(n, A):
+    """The mean is finished by the launch's last block: one block, two, and the most there are; whatever the scratch held before, and in a
+    graph, whose replays share their mark in it, with eager calls between them.  A double sum of the terms, rounded once."""
+    from ksim_amd import ppo
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    on = ppo.PPOVariables(rn(n, 1, A), rn(n, 1))
+    off = ppo.PPOVariables(on.log_probs + 0.05 * rn(n, 1, A), on.values + 0.05 * rn(n, 1), rn(n, 1, A).abs())
+    inputs = ppo.PPOInputs(rn(n, 1), rn(n, 1), None, None)
+
+    def check(out):
+        terms = out["policy"] + out["value"] + out["kl"] + out["entropy"]
+        want = (terms.double().sum() / n).item()
+        assert abs(out["total"].item() - want) <= 2 ** -23 * terms.abs().double().mean().item()
+
+    for fill in (0, 0x5A, 0xFF):
+        scratch = ppo._workspace("cuda").fill_(fill)
+        del scratch
+        check(ppo.compute_ppo_loss(inputs, on, off))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ppo.compute_ppo_loss(inputs, on, off)
+    for _ in range(4):
+        inputs.advantages_bt.mul_(-0.7).add_(0.1)
+        out["total"].fill_(7.0)
+        graph.replay()
+        check(out)
+        assert torch.equal(out["total"], ppo.compute_ppo_loss(inputs, on, off)["total"])
