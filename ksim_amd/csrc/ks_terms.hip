@@ -272,19 +272,27 @@ __device__ inline float rv_value(const KsRandomVar& rv, float u, float z, float 
 // Termination comparisons are strict and done in fp32 on the stored state, so the integer outputs are
 // reproducible bit for bit.
 constexpr int kTermEnvs = 32;
-// In the launch that also observes, a workgroup takes fewer envs: the observation is one thread per element, and with 32
-// envs per workgroup a launch over a few thousand envs would be too few workgroups to fill the chip.
-constexpr int kTermObsEnvs = 8;
+// In the launch that also observes, one thread per element, a workgroup takes at most 8: with 32 a launch over a few thousand envs would be too
+// few workgroups to fill the chip.  Fewer still, as many as observe in one round of its 256 threads, while that is no more workgroups than the chip
+// holds at once (kTermObsBlocks): a second and third round are 2 us each, and one is all there is to wait for.  68 elements, 8 -> 3 envs: 64 and 1024
+// envs 15.6 -> 10.2 us, 4096 16.4 -> 12.9; at 16384, where the rule stays with 8, 34.5 -> 40.6.
+constexpr int kTermObsEnvs = 8, kTermObsBlocks = 2048;
 
 // s_bad: non-finite state seen; s_reset: env starts a fresh episode; s_frame: its frame of the reference motion
-template <int ENVS>
-__device__ __forceinline__ void terminate_block(const TerminateArgs& a, int* s_bad, int* s_reset, int* s_frame) {
+__device__ __forceinline__ void terminate_block(const TerminateArgs& a, int envs, int* s_bad, int* s_reset, int* s_frame) {
   const KsTermsDesc& d = a.t->d;
   const int tid = threadIdx.x;
-  const int64_t e0 = (int64_t)blockIdx.x * ENVS;
-  const int ne = a.N - e0 < ENVS ? (int)(a.N - e0) : ENVS;
+  const int64_t e0 = (int64_t)blockIdx.x * envs;
+  const int ne = a.N - e0 < envs ? (int)(a.N - e0) : envs;
   const int nq = a.nq, nv = a.nv, nu = a.nu;
-  if (tid < ENVS) s_bad[tid] = 0;
+  if (tid < envs) s_bad[tid] = 0;
+  // what an env's own lane decides by is under way with the rows
+  float tm = 0.f;
+  int length = 0;
+  if (tid < ne) {
+    if (a.time) tm = a.time[e0 + tid];
+    if (a.episode_length) length = a.episode_length[e0 + tid];
+  }
   __syncthreads();
   // ---- flat pass 1: transition record (post-step state) and finiteness
   float* qb = a.qpos + e0 * nq;
@@ -305,7 +313,6 @@ __device__ __forceinline__ void terminate_block(const TerminateArgs& a, int* s_b
     const int64_t e = e0 + tid;
     const float* q = qb + tid * nq;
     const float* v = vb + tid * nv;
-    const float tm = a.time ? a.time[e] : 0.f;
     bool done = false, succ = true;
     for (int j = 0; j < a.n_terms; ++j) {
       const KsTermDesc td = d.terms[j];
@@ -344,7 +351,7 @@ __device__ __forceinline__ void terminate_block(const TerminateArgs& a, int* s_b
     const bool do_reset = a.apply_reset == 2 || (done && a.apply_reset == 1);
     s_reset[tid] = do_reset ? 1 : 0;
     if (a.reset_mask) a.reset_mask[e] = do_reset ? 1 : 0;
-    if (a.episode_length) a.episode_length[e] = do_reset ? 0 : a.episode_length[e] + 1;
+    if (a.episode_length) a.episode_length[e] = do_reset ? 0 : length + 1;
     int frame = 0;
     if (do_reset && a.reset_motion_qpos) {  // resets.py:291: randint(0, num_frames)
       if (a.reset_frame) frame = a.reset_frame[e];
@@ -473,21 +480,21 @@ __device__ __forceinline__ void terminate_block(const TerminateArgs& a, int* s_b
 
 __global__ __launch_bounds__(256) void terminate_kernel(TerminateArgs a) {
   __shared__ int s_bad[kTermEnvs], s_reset[kTermEnvs], s_frame[kTermEnvs];
-  terminate_block<kTermEnvs>(a, s_bad, s_reset, s_frame);
+  terminate_block(a, kTermEnvs, s_bad, s_reset, s_frame);
 }
 
 // The termination pass of control step t and the observation of step t + 1 in one launch: a workgroup takes the decisions
 // for its envs, resets the finished ones, and then observes those same envs in the state the next step will start from
 // (one thread per element, striding over the workgroup's envs).  What the first half wrote (state rows, the reset mask that
 // the observation takes as its `fresh` flags) is read back by other threads of the same workgroup only.
-__global__ __launch_bounds__(256) void terminate_observe_kernel(TerminateArgs a, ObserveArgs o) {
+__global__ __launch_bounds__(256) void terminate_observe_kernel(TerminateArgs a, ObserveArgs o, int envs) {
   __shared__ int s_bad[kTermObsEnvs], s_reset[kTermObsEnvs], s_frame[kTermObsEnvs];
-  terminate_block<kTermObsEnvs>(a, s_bad, s_reset, s_frame);
+  terminate_block(a, envs, s_bad, s_reset, s_frame);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  const int64_t e0 = (int64_t)blockIdx.x * kTermObsEnvs;
-  const int ne = a.N - e0 < kTermObsEnvs ? (int)(a.N - e0) : kTermObsEnvs;
+  const int64_t e0 = (int64_t)blockIdx.x * envs;
+  const int ne = a.N - e0 < envs ? (int)(a.N - e0) : envs;
   for (int i = threadIdx.x; i < ne * o.obs_dim; i += 256) observe_one(o, e0 * o.obs_dim + i);
 }
 
@@ -1412,9 +1419,11 @@ extern "C" int ks_terminate_reset_observe(const KsTerms* t, ks_stream_t stream, 
   // the observation half takes the episode starts from the mask the termination half writes in the same launch
   if (oio->fresh && oio->fresh != tio->reset_mask) return fail(KS_EINVAL, "ks_terminate_reset_observe: the observation's fresh flags must be the reset mask of this call");
   if (empty_o) { o.obs_dim = 0; }
-  const int64_t grid = (a.N + kTermObsEnvs - 1) / kTermObsEnvs;
+  int envs = o.obs_dim > 0 && o.obs_dim < 256 ? 256 / o.obs_dim : 1;
+  if (envs > kTermObsEnvs || (a.N + envs - 1) / envs > kTermObsBlocks) envs = kTermObsEnvs;
+  const int64_t grid = (a.N + envs - 1) / envs;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_terminate_reset_observe: too many envs");
-  hipLaunchKernelGGL(terminate_observe_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a, o);
+  hipLaunchKernelGGL(terminate_observe_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a, o, envs);
   return check_launch("ks_terminate_reset_observe");
 }
 

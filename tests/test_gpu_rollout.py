@@ -980,3 +980,23 @@ def test_reset_forward_inside_the_next_step_gives_the_same_trajectories():
         for a, b in zip(runs[0], other):
             for x, y in zip(a, b):
                 assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("N", [1, 7, 6144, 6145])
+def test_observation_in_the_terminating_launch_at_any_number_of_envs(N):
+    """The launch takes as many envs per workgroup as observe in one round of its threads, more beyond 2048 workgroups: the last workgroup
+    part full, on both sides of that line, against the two launches, bit for bit."""
+    import dataclasses
+
+    from ksim_amd.rollout import Rollout
+
+    T, runs = 3, []
+    for fuse in (False, True):
+        m, c, rnd_, _, _, EnvState = build(N, T, seed=9, min_height=0.86)
+        assert 2048 * (256 // c.terms.obs_dim) == 6144
+        ro = Rollout(dataclasses.replace(c, fuse_next_observation=fuse), N, T)
+        ps = c.engine.reset(c.physics_model, 1.0, 5, N, rnd_)
+        traj, _ = ro.unroll(EnvState(ps, rnd_, torch.zeros(N, 2, device=DEV), None, seed=31))
+        runs.append([x.clone() for x in (traj.obs["obs"], traj.obs["noisy_obs"], traj.done, traj.qpos, traj.timestep, ro.reset_mask, ps.data.qpos)])
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
