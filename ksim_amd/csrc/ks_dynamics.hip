@@ -722,8 +722,8 @@ void step_kernel(StepArgs a) {
           sincosf(0.5f * (l.qpos[b_qadr] - b_q0), &hs, &hc);
           const Quat jr = {hc, b_jaxis.x * hs, b_jaxis.y * hs, b_jaxis.z * hs};
           // rotation about the joint anchor: p + R_b (a - R_j a) with a the anchor in the body frame
-          const V3 ra = mul(q2mat(jr), b_jpos);
-          tl = b_pos + mul(q2mat(b_quat), b_jpos - ra);
+          const V3 arm = qrot(jr, V3{-b_jpos.x, -b_jpos.y, -b_jpos.z}, b_jpos);
+          tl = qrot(b_quat, arm, b_pos);
           ql = qmul(b_quat, jr);
         }
       }
@@ -744,11 +744,11 @@ void step_kernel(StepArgs a) {
         const V3 t0 = ld3(p0), t1 = ld3(p1);
         const Quat q0 = {p0[3], p0[4], p0[5], p0[6]}, q1 = {p1[3], p1[4], p1[5], p1[6]};
         if (k < b_depth) {
-          pos = pos + mul(q2mat(quat), t0);
+          pos = qrot(quat, t0, pos);
           quat = qmul(quat, q0);
         }
         if (k + 1 < b_depth) {
-          pos = pos + mul(q2mat(quat), t1);
+          pos = qrot(quat, t1, pos);
           quat = qmul(quat, q1);
         }
 #pragma unroll
@@ -814,9 +814,8 @@ void step_kernel(StepArgs a) {
         if (d_k < 3) {
           my_cdof.l = {d_k == 0 ? 1.f : 0.f, d_k == 1 ? 1.f : 0.f, d_k == 2 ? 1.f : 0.f};
         } else {
-          const Mat3 Rb = q2mat({l.xquat[4 * d_body], l.xquat[4 * d_body + 1], l.xquat[4 * d_body + 2], l.xquat[4 * d_body + 3]});
-          const float* R = Rb.m;
-          const V3 ax = d_k == 3 ? V3{R[0], R[3], R[6]} : d_k == 4 ? V3{R[1], R[4], R[7]} : V3{R[2], R[5], R[8]};
+          const V3 ax = qrot({l.xquat[4 * d_body], l.xquat[4 * d_body + 1], l.xquat[4 * d_body + 2], l.xquat[4 * d_body + 3]},
+                             V3{d_k == 3 ? 1.f : 0.f, d_k == 4 ? 1.f : 0.f, d_k == 5 ? 1.f : 0.f}, V3{0.f, 0.f, 0.f});
           my_cdof = {ax, cross(ax, off)};
         }
       } else {
@@ -830,7 +829,7 @@ void step_kernel(StepArgs a) {
     KS_PHASE(2)
     // ---- composite inertias (subtree = contiguous body range) and the mass matrix
     for (int idx = lane; idx < nb * 10; idx += 64) {
-      const int b = idx / 10, k = idx - 10 * b;
+      const int b = idx * 205 >> 11, k = idx - 10 * b;  // idx / 10 below 1024
       l.crb[idx] = b > 0 ? range_sum(l.cinert + k, 10, b, l.sub_end[b]) : 0.f;
     }
     KS_SYNC();
@@ -873,15 +872,11 @@ void step_kernel(StepArgs a) {
           hinge(cd0, qd0);
         } else if (e & (1u << 11)) {
           const int da = (int)((e >> 5) & 31u);
-          v = v + cd0 * qd0;
-          for (int c = 1; c < 3; ++c) v = v + ld6(l.cdof + 6 * (da + c)) * l.qvel[da + c];
-          Sp dv = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-          for (int c = 3; c < 6; ++c) {
-            const Sp cd = ld6(l.cdof + 6 * (da + c));
-            const float qd = l.qvel[da + c];
-            acc = acc + cross_motion(v, cd) * qd;
-            dv = dv + cd * qd;
-          }
+          // the translations' axes are the world's, and the three rotations act on one velocity, so their sum does
+          v.l = v.l + V3{qd0, l.qvel[da + 1], l.qvel[da + 2]};
+          const Sp dv = ld6(l.cdof + 6 * (da + 3)) * l.qvel[da + 3] + ld6(l.cdof + 6 * (da + 4)) * l.qvel[da + 4] +
+                        ld6(l.cdof + 6 * (da + 5)) * l.qvel[da + 5];
+          acc = acc + cross_motion(v, dv);
           v = v + dv;
         }
       };
@@ -959,7 +954,7 @@ void step_kernel(StepArgs a) {
     }
     KS_SYNC();
     for (int idx = lane; idx < nb * 6; idx += 64) {
-      const int b = idx / 6, k = idx - 6 * b;
+      const int b = idx * 171 >> 10, k = idx - 6 * b;  // idx / 6 below 500
       l.fsub[idx] = b > 0 ? range_sum(l.cfrc + k, 6, b, l.sub_end[b]) : 0.f;
     }
     KS_SYNC();
@@ -986,11 +981,7 @@ void step_kernel(StepArgs a) {
     float dist = 1.f;
     V3 cpos = {0.f, 0.f, 0.f};
     if (is_sph) {
-      const Mat3 Rb = q2mat({l.xquat[4 * s_body], l.xquat[4 * s_body + 1], l.xquat[4 * s_body + 2], l.xquat[4 * s_body + 3]});
-      const float* R = Rb.m;
-      const V3 c = ld3(l.xpos + 3 * s_body) + V3{R[0] * s_pos.x + R[1] * s_pos.y + R[2] * s_pos.z,
-                                                R[3] * s_pos.x + R[4] * s_pos.y + R[5] * s_pos.z,
-                                                R[6] * s_pos.x + R[7] * s_pos.y + R[8] * s_pos.z};
+      const V3 c = qrot({l.xquat[4 * s_body], l.xquat[4 * s_body + 1], l.xquat[4 * s_body + 2], l.xquat[4 * s_body + 3]}, s_pos, ld3(l.xpos + 3 * s_body));
       dist = c.z - s_rad;
       cpos = {c.x, c.y, c.z - s_rad - 0.5f * dist};
       if (a.contact_dist) a.contact_dist[env * ns + lane] = dist;
