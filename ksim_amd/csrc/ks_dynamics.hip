@@ -569,7 +569,26 @@ void step_kernel(StepArgs a) {
   // step does it itself, as a pass `sub = -1` that neither actuates nor integrates, instead of a masked launch of the
   // forward-only kernel between the termination pass and this step.
   const bool fresh_env = !FWD && a.fresh && a.fresh[env];  // wave-uniform
+  // The arguments, and the sizes and LDS offsets that follow from them, are taken afresh in each substep and in the
+  // write-back: `s_load`s through the scalar cache and a little scalar arithmetic.  Taken once, the ~60 pointers, sizes and
+  // offsets stay live across the solver, which leaves SGPRs for a third of them: the rest lay in VGPR lanes (194
+  // `v_writelane`s and ~280 `v_readlane`s, all of them VALU work, and two VGPRs of a file that is full; now 33 and 54, and
+  // none of the scratch that went with it).  4096 humanoid envs: 82.4 M -> 79.1 M VALU instructions a launch, 253.3 -> 246.6
+  // us; the pointers alone, without sizes and offsets, 248.1 us.
+  const auto arguments = []() -> const StepArgs& {
+    typedef const __attribute__((address_space(4))) StepArgs* ArgsPtr;
+    ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();  // the kernel's one parameter lies at its start
+    asm volatile("" : "+s"(p));
+    return *(const StepArgs*)p;
+  };
   for (int sub = fresh_env ? -1 : 0; sub < nsub; ++sub) {
+    const StepArgs& a = arguments();
+    const DevModel& m = *a.model;
+    const ModelHead& mh = a.head;
+    const int nb = mh.nb, nq = mh.nq, nv = mh.nv, nu = mh.nu, ns = mh.ns;
+    Lds l = carve<NP>(lds_raw, lds_raw, nb, nq, nv, nu, ns);
+    const int rq = mh.root_free ? 7 : 0;
+    const int rv = rq ? 6 : 0;
     const bool fwd = FWD || sub < 0;
     // The lane id is re-materialised per substep so that per-lane LDS addresses are recomputed inside the loop
     // instead of being hoisted out of it into ~130 long-lived registers (which would halve the occupancy).
@@ -1456,28 +1475,32 @@ void step_kernel(StepArgs a) {
   if (a.dbg_M && lane == 0) for (int k = 0; k < 16; ++k) a.dbg_M[env * nv * nv + k] = prof[k];
 #endif
   // ---- write back
-  if (!FWD) {
-    for (int i = lane; i < nq; i += 64) a.qpos[env * nq + i] = l.qpos[i];
-    if (lane < nv) a.qvel[env * nv + lane] = l.qvel[lane];
-    if (a.work && lane == 0) a.work[env] = work;
-    if (a.time && lane == 0) {  // dt added once per substep in fp32, like the reference's accumulation
-      float time = a.time[env];
-      for (int k = 0; k < nsub; ++k) time += mh.dt;
-      a.time[env] = time;
+  {
+    const StepArgs& a = arguments();
+    const ModelHead& mh = a.head;
+    if (!FWD) {
+      for (int i = lane; i < nq; i += 64) a.qpos[env * nq + i] = l.qpos[i];
+      if (lane < nv) a.qvel[env * nv + lane] = l.qvel[lane];
+      if (a.work && lane == 0) a.work[env] = work;
+      if (a.time && lane == 0) {  // dt added once per substep in fp32, like the reference's accumulation
+        float time = a.time[env];
+        for (int k = 0; k < nsub; ++k) time += mh.dt;
+        a.time[env] = time;
+      }
+      if (a.last_ctrl) {
+        const int na = a.actuator_type == KS_ACT_POSITION_VELOCITY ? 2 * nu : nu;
+        for (int i = lane; i < na; i += 64) a.last_ctrl[env * na + i] = a.action[env * na + i];
+      }
     }
-    if (a.last_ctrl) {
-      const int na = a.actuator_type == KS_ACT_POSITION_VELOCITY ? 2 * nu : nu;
-      for (int i = lane; i < na; i += 64) a.last_ctrl[env * na + i] = a.action[env * na + i];
-    }
+    if (a.qacc_warmstart && lane < nv) a.qacc_warmstart[env * nv + lane] = l.warm[lane];
+    if (a.ctrl_out) for (int i = lane; i < nu; i += 64) a.ctrl_out[env * nu + i] = l.tau[i];
+    if (a.xpos) for (int i = lane; i < nb * 3; i += 64) a.xpos[env * nb * 3 + i] = l.xpos[i];
+    if (a.xquat) for (int i = lane; i < nb * 4; i += 64) a.xquat[env * nb * 4 + i] = l.xquat[i];
+    if (a.cvel) for (int i = lane; i < nb * 6; i += 64) a.cvel[env * nb * 6 + i] = l.cvel[i];
+    if (a.traj_ctrl) for (int i = lane; i < nu; i += 64) a.traj_ctrl[env * nu + i] = l.tau[i];
+    if (a.traj_xpos) for (int i = lane; i < nb * 3; i += 64) a.traj_xpos[env * nb * 3 + i] = l.xpos[i];
+    if (a.traj_xquat) for (int i = lane; i < nb * 4; i += 64) a.traj_xquat[env * nb * 4 + i] = l.xquat[i];
   }
-  if (a.qacc_warmstart && lane < nv) a.qacc_warmstart[env * nv + lane] = l.warm[lane];
-  if (a.ctrl_out) for (int i = lane; i < nu; i += 64) a.ctrl_out[env * nu + i] = l.tau[i];
-  if (a.xpos) for (int i = lane; i < nb * 3; i += 64) a.xpos[env * nb * 3 + i] = l.xpos[i];
-  if (a.xquat) for (int i = lane; i < nb * 4; i += 64) a.xquat[env * nb * 4 + i] = l.xquat[i];
-  if (a.cvel) for (int i = lane; i < nb * 6; i += 64) a.cvel[env * nb * 6 + i] = l.cvel[i];
-  if (a.traj_ctrl) for (int i = lane; i < nu; i += 64) a.traj_ctrl[env * nu + i] = l.tau[i];
-  if (a.traj_xpos) for (int i = lane; i < nb * 3; i += 64) a.traj_xpos[env * nb * 3 + i] = l.xpos[i];
-  if (a.traj_xquat) for (int i = lane; i < nb * 4; i += 64) a.traj_xquat[env * nb * 4 + i] = l.xquat[i];
 }
 
 }  // namespace ks
