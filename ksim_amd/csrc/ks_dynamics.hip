@@ -317,6 +317,12 @@ struct LaneRec {
 static_assert(sizeof(LaneRec) == sizeof(DevModel::lane_rec) / 64, "LaneRec must fill the record");
 static_assert(kMaxB <= 32 && kMaxV <= 32 && kMaxDepth % 2 == 0, "a link of b_chain holds 5 + 5 bits");
 constexpr int kRecPieces = sizeof(LaneRec) / 16;
+// ... and what the env itself may bring beside them
+struct LaneIn {
+  LaneRec rec;
+  V3 ipos, inertia, sph_pos;  // of the lane's body and contact sphere
+  float mass_scale, damping_scale, armature_scale, sph_radius;
+};
 // one field of a lane's record
 #define KS_REC(m, lane, field) (__builtin_bit_cast(decltype(LaneRec::field), (m).lane_rec[offsetof(LaneRec, field) / 16][lane][offsetof(LaneRec, field) / 4 % 4]))
 
@@ -581,6 +587,27 @@ void step_kernel(StepArgs a) {
     asm volatile("" : "+s"(p));
     return *(const StepArgs*)p;
   };
+  const auto load_lane = [env](const StepArgs& a, LaneIn& in) __attribute__((always_inline)) {
+    const DevModel& m = *a.model;
+    const int nb = a.head.nb, nv = a.head.nv, ns = a.head.ns;
+    int lane = threadIdx.x;
+    asm volatile("" : "+v"(lane));
+    uint4* dst = reinterpret_cast<uint4*>(&in.rec);
+#pragma unroll
+    for (int k = 0; k < kRecPieces; ++k) dst[k] = *reinterpret_cast<const uint4*>(m.lane_rec[k][lane]);
+    // the row of an optional operand: this env's, or row 0 of what stands in for it
+    auto row_of = [&](unsigned bit) -> int64_t { return (a.given & bit) ? env : 0; };
+    const int bl = lane < nb ? lane : 0, dl = lane < nv ? lane : 0, sl = lane < ns ? lane : 0;
+    in.ipos = ld3(a.body_ipos + (row_of(kOptIpos) * nb + bl) * 3);
+    in.inertia = ld3(a.body_inertia + (row_of(kOptInertia) * nb + bl) * 3);
+    in.mass_scale = a.mass_scale[row_of(kOptMass) * nb + bl];
+    in.damping_scale = a.damping_scale[row_of(kOptDamping) * nv + dl];
+    in.armature_scale = a.armature_scale[row_of(kOptArmature) * nv + dl];
+    in.sph_pos = ld3(a.sph_pos + (row_of(kOptSphere) * ns + sl) * 3);
+    in.sph_radius = a.sph_radius[row_of(kOptSphere) * ns + sl];
+  };
+  LaneIn in;
+  load_lane(arguments(), in);
   for (int sub = fresh_env ? -1 : 0; sub < nsub; ++sub) {
     const StepArgs& a = arguments();
     const DevModel& m = *a.model;
@@ -595,38 +622,28 @@ void step_kernel(StepArgs a) {
     int lane_v = threadIdx.x;
     asm volatile("" : "+v"(lane_v));
     const int lane = lane_v;
-      // ---- per-lane model constants: re-read every substep (they hit the vector L1) so that they do not stay live
-      // across the solver, whose register rows set the occupancy
+    // ---- the lane's constants, as the end of the last substep has requested them
     const bool is_body = lane > 0 && lane < nb;
-    const int bl = is_body ? lane : 0;
     const bool is_dof = lane < nv;
     const bool is_sph = lane < ns;
-    LaneRec rec;
-    {
-      uint4* dst = reinterpret_cast<uint4*>(&rec);
-#pragma unroll
-      for (int k = 0; k < kRecPieces; ++k) dst[k] = *reinterpret_cast<const uint4*>(m.lane_rec[k][lane]);
-    }
+    const LaneRec& rec = in.rec;
     // the row of an optional operand: this env's, or row 0 of what stands in for it
     auto row_of = [&](unsigned bit) -> int64_t { return (a.given & bit) ? env : 0; };
     const int b_jtype = rec.b_jtype, b_qadr = rec.b_qadr, b_dofadr = rec.b_dofadr, b_depth = rec.b_depth;
     const V3 b_pos = {rec.b_pos[0], rec.b_pos[1], rec.b_pos[2]};
-    const V3 b_ipos = ld3(a.body_ipos + (row_of(kOptIpos) * nb + bl) * 3);          // per-env centres of mass
-    const V3 b_inertia = ld3(a.body_inertia + (row_of(kOptInertia) * nb + bl) * 3);  // and principal inertias
+    const V3 b_ipos = in.ipos, b_inertia = in.inertia;
     const V3 b_jaxis = {rec.b_jaxis[0], rec.b_jaxis[1], rec.b_jaxis[2]}, b_jpos = {rec.b_jpos[0], rec.b_jpos[1], rec.b_jpos[2]};
     const Quat b_quat = {rec.b_quat[0], rec.b_quat[1], rec.b_quat[2], rec.b_quat[3]};
     const Quat b_iquat = {rec.b_iquat[0], rec.b_iquat[1], rec.b_iquat[2], rec.b_iquat[3]};
     const float b_q0 = rec.b_q0;
-    const float b_scale = a.mass_scale[row_of(kOptMass) * nb + bl];
-    const float b_mass = is_body ? rec.b_mass * b_scale : 0.f;
+    const float b_mass = is_body ? rec.b_mass * in.mass_scale : 0.f;
     const int d_body = rec.d_body, d_act = rec.d_act, d_jtype = rec.d_jtype, d_k = rec.d_k;
-    const int dl = is_dof ? lane : 0;
-    const float d_damping = rec.d_damping * a.damping_scale[row_of(kOptDamping) * nv + dl];
-    const float d_armature = rec.d_armature * a.armature_scale[row_of(kOptArmature) * nv + dl];
+    const float d_damping = rec.d_damping * in.damping_scale;
+    const float d_armature = rec.d_armature * in.armature_scale;
     const float d_gear = rec.d_gear, d_lo = rec.d_lo, d_hi = rec.d_hi;
-    const int s_body = rec.s_body, sl = is_sph ? lane : 0;
-    const V3 s_pos = ld3(a.sph_pos + (row_of(kOptSphere) * ns + sl) * 3);  // per-env contact spheres
-    const float s_rad = a.sph_radius[row_of(kOptSphere) * ns + sl];
+    const int s_body = rec.s_body;
+    const V3 s_pos = in.sph_pos;
+    const float s_rad = in.sph_radius;
     const float s_invw = rec.s_invw;
     const unsigned s_mask = rec.s_mask;
     unsigned chain[kMaxDepth / 2];
@@ -1418,14 +1435,17 @@ void step_kernel(StepArgs a) {
     if (is_dof) l.warm[lane] = qacc;
 
     KS_PHASE(14)
+    // Behind the solver, whose register rows set the occupancy: for the next substep, and what the integration needs of it.
+    // Requested at the top of a substep, and three fields of it once more here, a wavefront waited twice: 64 robots' control
+    // step 0.8 %, 1024 K-Bots' and 4096 humanoids' 0.3 % slower.  The actuator's inputs requested here as well cost more
+    // (16 spilled registers) than they save, and so did reading the joint's addresses from LDS instead (446 us of 442).
+    load_lane(a, in);
     // ---- semi-implicit Euler
     if (!fwd) {
-      // What this stage needs of the lane's constants is read again here (through an opaque lane id, so that the loads
-      // are not merged with those at the top of the substep): nothing of it stays live across the solver.
       int lane_e = threadIdx.x;
       asm volatile("" : "+v"(lane_e));
-      const int b_jtype = KS_REC(m, lane_e, b_jtype), b_qadr = KS_REC(m, lane_e, b_qadr), b_dofadr = KS_REC(m, lane_e, b_dofadr);
-      const float d_damping = KS_REC(m, lane_e, d_damping) * a.damping_scale[((a.given & kOptDamping) ? env : 0) * nv + (lane_e < nv ? lane_e : 0)];
+      const int b_jtype = in.rec.b_jtype, b_qadr = in.rec.b_qadr, b_dofadr = in.rec.b_dofadr;
+      const float d_damping = in.rec.d_damping * in.damping_scale;
       const float my_qvel = lane_e < nv ? l.qvel[lane_e] : 0.f;
       float qacc_int = qacc;
       if (mh.eulerdamp) {
