@@ -136,11 +136,10 @@ __device__ __forceinline__ void load_row(const float* p, float (&v)[NP]) {
 // whether its second k is used or not (fp32 MFMAs and vector instructions take turns), and with one column per step that was a fifth of the
 // kernel: 8192 mixed robots 507 -> 474 us per control step, 4096 humanoids 356 -> 338.  (Here and below the two figures of a pair are from one
 // card in turn; cards differ by up to 4 %, so pairs do not continue one another.)
-// Column j below the diagonal is left as it was when the pivot was reached
-// (L[k][j] * L[j][j]) and row j right of the diagonal holds L[k][j]: read down a lane, that is row c of L to the
-// left of the diagonal and the scaled column c below it, exactly what the column-oriented substitutions take,
+// Column j below the diagonal and row j right of it are left as they were when the pivot was reached, L[k][j] * L[j][j] (the scaled row
+// goes into the MFMA only): read down a lane, that is what both substitutions take in their square-root-free form (back_steps),
 // once the upper lane half has handed its 16 registers to the lower one.  On return, in lane i < NP:
-//   R[j], j < i : L[i][j]              R[k], k > i : L[k][i] * L[i][i]              myinv = 1 / L[i][i]
+//   R[j], j < i : L[i][j] * L[j][j]              R[k], k > i : L[k][i] * L[i][i]              myinv = 1 / L[i][i]
 // `nv` (wave-uniform) is the real size: the steps of the padded columns, which would multiply zeros, are branched over
 // (only steps past the next smaller instantiation's size carry the test).
 constexpr int padded_from(int np) { return np > 28 ? 28 : (np > 24 ? 24 : (np > 16 ? 16 : (np > 8 ? 8 : 0))); }
@@ -178,20 +177,20 @@ __device__ __forceinline__ void chol_tile(f32x16& T, float (&R)[NP], float& myin
     const bool right0 = in_lanes(own + 1, 31 - j, site);
     float a0 = right0 ? T[rho] : 0.f;  // beside the reciprocal root, not behind it
     a0 *= inv0;
-    T[rho] = right0 ? a0 : T[rho];
     const float v = T[rho + 1] - a0 * lane_bcast(a0, own + 1);
+    T[rho + 1] = v;
     const float inv1 = inv_root(lane_bcast(v, own + 1));
     myinv = in_lanes(j + 1, 1, site) ? inv1 : myinv;
     const bool right1 = in_lanes(own + 2, 30 - j, site);
     float a1 = right1 ? v : 0.f;
     a1 *= inv1;
-    T[rho + 1] = right1 ? a1 : v;
     // the last real columns have nothing right of or below them
     if (j + 2 < NP && !(j + 2 >= padded_from(NP) && j + 2 >= nv)) {
       const float b = halves(a0, a1, hj), na = in_lanes(j + 1, 1, site) ? 0.f : -b;
       T = __builtin_amdgcn_mfma_f32_32x32x2f32(na, b, T, 0, 0, 0);
     }
   }
+  asm volatile("s_nop 15\n\ts_nop 3" : "+v"(T));  // the substitutions' assembly takes these registers as vector instructions leave them
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -217,42 +216,101 @@ __device__ __forceinline__ void load_mtile(f32x16& T, const float* __restrict__ 
   }
 }
 
-// L^T x = y, lane i holding y_i and returning x_i.  With w_i = y_i / L[i][i] a step is w_i -= (R[k] / L[i][i]^2) x_k, x_k = w_k: the scaled
-// and masked coefficient does not wait for the step before, so the chain is one broadcast and one fused multiply-add per column.
 template <int NP>
-__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, float y, int nv) {
-  int site = 0;
-  asm volatile("" : "+s"(site));
-  const float myinv2 = myinv * myinv;
-  float w = y * myinv;
-#pragma unroll
-  for (int k = NP - 1; k >= 0; --k) {
-    if (k >= padded_from(NP) && k >= nv) continue;  // padded unknowns are zero and couple to nothing
-    const float coef = in_lanes(0, k, site) ? R[k] * myinv2 : 0.f;
-    w -= coef * lane_bcast(w, k);
+__device__ __forceinline__ bool padded_out(int k, int nv) { return k >= padded_from(NP) && k >= nv; }  // such unknowns are zero and couple to nothing
+
+// A substitution step: w_i += w_K c_i in the COUNT lanes from FIRST on, lane K being in their row of 16.  `v_fmac` takes lane K of its row through
+// DPP, which wants two wait states behind the write of any of its registers (s_nop 1); the mask is one scalar instruction.  Broadcast to
+// all 32 rows through a scalar register, the step was a lane read, two wait states and the multiply-add, for every column one after the
+// other; now the chains are 16 columns at most, and what one row of lanes takes off the other are products side by side (row_products).  With the
+// rows kept unscaled (two selects per pair of columns less) a wavefront alone factors and solves M in 4570 cycles instead of 4970, and 4096
+// humanoids' control step has 76.5 M vector instructions instead of 79 M: rollout steps of 64 and of 1024 K-Bots, of 4096 humanoids and of an
+// LSTM policy 1.1, 1.3, 1.3 and 1.0 % faster.  Error of qacc_smooth against 64 bits, rms: 0.70e-6 -> 0.72e-6 (kbot_scale_model), 1.76e-6 -> 1.67e-6
+// (humanoid_model with joint limits), of qacc 1.17e-6 -> 0.96e-6 and 1.75e-6 -> 1.64e-6.
+template <int K, int FIRST, int COUNT>
+__device__ __forceinline__ void row_step(float& w, float c) {
+  unsigned long long mask;
+  asm("s_bfm_b64 %1, %4, %3\n\tv_cndmask_b32_e64 %2, 0, %2, %1\n\ts_nop 1\n\tv_fmac_f32_dpp %0, %0, %2 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+      : "+v"(w), "=&s"(mask), "+v"(c) : "i"(FIRST), "i"(COUNT), "i"(K % 16));
+}
+// columns K down to LO + 1 of the backward substitution, K up to HI - 1 of the forward one, within a row of 16 lanes: with w_i = y_i / L[i][i]
+// a step is w_i -= (R[k] / L[i][i]^2) w_k (m = -1 / L[i][i]^2)
+template <int NP, int K, int LO>
+__device__ __forceinline__ void back_steps(const float (&R)[NP], float m, float& w, int nv) {
+  if constexpr (K > LO) {
+    if (!padded_out<NP>(K, nv)) row_step<K, LO, K - LO>(w, R[K] * m);
+    back_steps<NP, K - 1, LO>(R, m, w, nv);
   }
+}
+template <int NP, int K, int HI>
+__device__ __forceinline__ void forward_steps(const float (&R)[NP], float m, float& w, int nv) {
+  if constexpr (K < HI) {
+    if (!padded_out<NP>(K, nv)) row_step<K, K + 1, HI - K>(w, R[K] * m);
+    forward_steps<NP, K + 1, HI>(R, m, w, nv);
+  }
+}
+// sum over K < END, a multiple of four of them, of R[K] x_K, x_K in lane K % 16 of each row of 16
+#define KS_ROW_PRODUCT(OP, T, R, LANE) OP " %" #T ", %4, %" #R " row_newbcast:%" #LANE " row_mask:0xf bank_mask:0xf\n\t"
+#define KS_ROW_PRODUCTS(OP) "s_nop 1\n\t" KS_ROW_PRODUCT(OP, 0, 5, 9) KS_ROW_PRODUCT(OP, 1, 6, 10) KS_ROW_PRODUCT(OP, 2, 7, 11) KS_ROW_PRODUCT(OP, 3, 8, 12)
+template <int NP, int K, int END>
+__device__ __forceinline__ void row_products_from(const float (&R)[NP], float x, float (&t)[4]) {
+  if constexpr (K < END) {
+    asm(KS_ROW_PRODUCTS("v_fmac_f32_dpp") : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3])
+        : "v"(x), "v"(R[K]), "v"(R[K + 1]), "v"(R[K + 2]), "v"(R[K + 3]), "i"(K % 16), "i"(K % 16 + 1), "i"(K % 16 + 2), "i"(K % 16 + 3));
+    row_products_from<NP, K + 4, END>(R, x, t);
+  }
+}
+template <int NP, int K, int END>
+__device__ __forceinline__ float row_products(const float (&R)[NP], float x) {
+  float t[4];
+  asm(KS_ROW_PRODUCTS("v_mul_f32_dpp") : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
+      : "v"(x), "v"(R[K]), "v"(R[K + 1]), "v"(R[K + 2]), "v"(R[K + 3]), "i"(K % 16), "i"(K % 16 + 1), "i"(K % 16 + 2), "i"(K % 16 + 3));
+  row_products_from<NP, K + 4, END>(R, x, t);
+  return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
+// lanes 0..15 of x in lanes 0..15 and 16..31 of `lower`, lanes 16..31 in both of `upper` (assembly: the builtin's two results come out the same)
+__device__ __forceinline__ void lane_rows(float x, float& lower, float& upper) {
+  lower = upper = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lower), "+v"(upper));
+}
+
+// L^T x = y, lane i holding w_i = y_i / L[i][i] and returning x_i.  Of more than 16 rows the upper lane row comes first; what it takes off the
+// lower one are products without a chain.
+template <int NP>
+__device__ __forceinline__ float back_substitute(const float (&R)[NP], float myinv, float w, int nv) {
+  const float m = -myinv * myinv;
+  if constexpr (NP > 16) {
+    back_steps<NP, NP - 1, 16>(R, m, w, nv);
+    float upper, lower;
+    lane_rows(w, lower, upper);
+    const float below = fmaf(row_products<NP, 16, NP>(R, upper), m, w);
+    w = in_lanes(0, 16, 0) ? below : w;
+  }
+  back_steps<NP, (NP > 16 ? 15 : NP - 1), 0>(R, m, w, nv);
   return w;
 }
 
 // x = (L L^T)^-1 b, lane i holding b_i and returning x_i
 template <int NP>
 __device__ __forceinline__ float solve_regs(const float (&R)[NP], float myinv, float b, int nv) {
-  int site = 0;
-  asm volatile("" : "+s"(site));
-  float y = b * myinv;
-#pragma unroll
-  for (int j = 0; j < NP; ++j) {  // L y = b in the same form
-    if (j >= padded_from(NP) && j >= nv) continue;
-    const float coef = in_lanes(j + 1, 31 - j, site) ? R[j] * myinv : 0.f;
-    y -= coef * lane_bcast(y, j);
+  const float m = -myinv * myinv;
+  float w = b * myinv * myinv;
+  forward_steps<NP, 0, (NP > 16 ? 15 : NP - 1)>(R, m, w, nv);
+  if constexpr (NP > 16) {
+    float upper, lower;
+    lane_rows(w, lower, upper);
+    const float above = fmaf(row_products<NP, 0, 16>(R, lower), m, w);
+    w = in_lanes(16, 16, 0) ? above : w;
+    forward_steps<NP, 16, NP - 1>(R, m, w, nv);
   }
-  return back_substitute<NP>(R, myinv, y, nv);
+  return back_substitute<NP>(R, myinv, w, nv);
 }
 
 // Factors the tile and returns x = (L L^T)^-1 b, lane i holding b_i (zero beyond nv).  A matrix of fewer than 32 columns carries b
 // along as column 31 of its tile (load_mtile): the rank-1 updates of the factorisation then are the forward substitution too, and what
-// is left of it is to hand y = L^-1 b, which the two lanes of that column hold, to the lanes of its rows, through LDS (`vbuf`, 32
-// floats).  A substitution step is four instructions of a chain, 26 of them for 26 dofs.
+// is left of it is to hand y = L^-1 b, times L[i][i], which the two lanes of that column hold, to the lanes of its rows, through LDS (`vbuf`,
+// 32 floats).
 template <int NP>
 __device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& myinv, int lane, float b, int nv, float* vbuf) {
   chol_tile<NP>(T, R, myinv, nv);
@@ -267,9 +325,9 @@ __device__ __forceinline__ float chol_solve(f32x16& T, float (&R)[NP], float& my
       for (int g = 0; g < 4; ++g) dst[2 * g] = {T[4 * g], T[4 * g + 1], T[4 * g + 2], T[4 * g + 3]};
     }
     KS_SYNC();
-    const float y = vbuf[lane & 31];
+    const float y = vbuf[lane & 31];  // times L[i][i]
     KS_SYNC();
-    return back_substitute<NP>(R, myinv, y, nv);
+    return back_substitute<NP>(R, myinv, y * myinv * myinv, nv);
   }
 }
 

@@ -749,6 +749,13 @@ def test_every_padded_width_of_the_step_kernel(nv, spheres, opts):
                 compare(buf[key], key, step, ONE_STEP_TOL if step == 1 else TEN_STEP_TOL)
 
 
+@pytest.mark.parametrize("nv,opts", [(7, _ROWS), (8, {}), (8, _ROWS), (9, {}), (15, _ROWS), (16, _ROWS), (18, _ROWS), (26, _ROWS), (27, {})])
+def test_substitutions_at_the_edges_of_a_lane_row(nv, opts):
+    """A substitution runs within rows of 16 lanes, with the products between two rows apart: one row not full, full, and a second one of two to
+    eleven dofs.  With rows on the dof lanes the factor is kept between Newton iterations, which takes the forward substitution by itself too."""
+    test_every_padded_width_of_the_step_kernel(nv, 8, opts)
+
+
 def test_centre_of_mass_keeps_the_products_of_its_first_additions():
     """The sums over the bodies start from products that are not rounded before their first addition: of bodies of 8, 5 and 3 kg the third one's share
     goes into the second one's by a fused multiply-add.  Every other operation is exact here (frames at the centres of mass, a total of 16 kg, a root
