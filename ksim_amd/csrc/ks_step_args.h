@@ -14,6 +14,9 @@ enum StepOptional : unsigned {
   kOptMass = 1u << 0, kOptDamping = 1u << 1, kOptArmature = 1u << 2, kOptIpos = 1u << 3, kOptInertia = 1u << 4, kOptSphere = 1u << 5,
   kOptKp = 1u << 6, kOptKd = 1u << 7, kOptLimit = 1u << 8, kOptZero = 1u << 9, kOptDrop = 1u << 10, kOptActionBias = 1u << 11,
   kOptTorqueBias = 1u << 12, kOptActionNoise = 1u << 13, kOptTorqueNoise = 1u << 14,
+  // what else a substep asks about: outputs that are wanted, and events
+  kOutCinert = 1u << 15, kOutBias = 1u << 16, kOutM = 1u << 17, kOutDist = 1u << 18, kOutSmooth = 1u << 19, kOutCfrc = 1u << 20,
+  kOutQacc = 1u << 21, kOutNiter = 1u << 22, kOutNefc = 1u << 23, kHasEvents = 1u << 24, kHasForceEvents = 1u << 25,
 };
 
 struct StepArgs {
