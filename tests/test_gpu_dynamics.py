@@ -756,6 +756,33 @@ def test_substitutions_at_the_edges_of_a_lane_row(nv, opts):
     test_every_padded_width_of_the_step_kernel(nv, 8, opts)
 
 
+@pytest.mark.parametrize("rate", [0.0, 1e-8, 1e-3, 3.0, 150.0, 200.0, 700.0])
+def test_free_joint_turns_by_its_angular_velocity(rate):
+    """The turn of one step of 5 ms, q exp(w dt), on both sides of the half angle of 1/2 (|w| = 200 / s) up to which it comes from series.  Tolerance:
+    h = |w| dt / 2 <= 1.8 carries three roundings, sine, cosine, the product of quaternions and its normalisation ten of numbers up to 1, 2^-24 each."""
+    from ksim_amd import physics
+    from ksim_amd._lib_dyn import KS_ACT_TORQUE
+
+    m = tree_model(1, 0)
+    N = 96
+    rng = np.random.default_rng(5)
+    qpos, qvel = np.tile(m.qpos0, (N, 1)), np.zeros((N, m.nv))
+    quat, axis = rng.normal(size=(N, 4)), rng.normal(size=(N, 3))
+    qpos[:, 3:7] = quat / np.linalg.norm(quat, axis=1, keepdims=True)
+    qvel[:, 3:6] = axis / np.linalg.norm(axis, axis=1, keepdims=True) * rate
+    buf = dict(qpos=t32(qpos), qvel=t32(qvel), qacc_warmstart=zeros(N, m.nv), time=zeros(N), last_ctrl=zeros(N, m.nu), action=zeros(N, m.nu))
+    q0 = buf["qpos"].cpu().numpy()[:, 3:7].astype(np.float64)
+    physics.control_step(physics.DeviceModel(m), buf, substeps=1, actuator_type=KS_ACT_TORQUE)
+    w = buf["qvel"].cpu().numpy()[:, 3:6].astype(np.float64)  # the velocity that the step moves with
+    n = np.linalg.norm(w, axis=1, keepdims=True)
+    turn = np.concatenate([np.cos(0.5 * n * m.dt), w * 0.5 * m.dt * np.sinc(0.5 * n * m.dt / np.pi)], axis=1)
+    want = np.stack([q0[:, 0] * turn[:, 0] - (q0[:, 1:] * turn[:, 1:]).sum(1),
+                     *(q0[:, :1] * turn[:, 1:] + q0[:, 1:] * turn[:, :1] + np.cross(q0[:, 1:], turn[:, 1:])).T], axis=1)
+    want /= np.linalg.norm(want, axis=1, keepdims=True)
+    err = np.abs(buf["qpos"].cpu().numpy()[:, 3:7] - want).max()
+    assert err <= (3 * 1.8 + 10) * 2.0 ** -24, f"{rate} / s: {err:.2e}"
+
+
 def test_centre_of_mass_keeps_the_products_of_its_first_additions():
     """The sums over the bodies start from products that are not rounded before their first addition: of bodies of 8, 5 and 3 kg the third one's share
     goes into the second one's by a fused multiply-add.  Every other operation is exact here (frames at the centres of mass, a total of 16 kg, a root
