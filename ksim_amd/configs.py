@@ -94,8 +94,7 @@ def kbot_lstm_rollout(num_envs: int = 4096, rollout_length: int = 100, seed: int
     """The K-Bot-scale rollout with the K-Bot example's policy instead of the benchmark's MLPs (examples/kbot/train.py:80-95,
     837-995, 1754-1757): LSTM actor and critic, projection -> 2 x 128 -> linear head in fp32, the actor's head means |
     deviations with a mean bias and the one-pole low-pass (10 Hz) whose state rides in the model carry; 4096 envs, 2 s of
-    control steps per rollout.  The critic runs on a side stream (RolloutConstants.critic_on_side_stream), and the next step's observation
-    rides in the launch that ends a step (4096 envs 400 -> 398 us a control step)."""
+    control steps per rollout.  The critic runs on a side stream (RolloutConstants.critic_on_side_stream)."""
     import dataclasses
 
     from .actions import LowPass
@@ -116,15 +115,14 @@ def kbot_lstm_rollout(num_envs: int = 4096, rollout_length: int = 100, seed: int
     head = GaussianHead(min_std=0.01, max_std=1.0, var_scale=0.5, mean_bias=torch.zeros(nu, device="cuda"),
                         lowpass=LowPass(ctrl_dt=0.02, cutoff_frequency=10.0))
     consts = dataclasses.replace(consts, actor=net(2 * nu, 0.1), critic=net(1, 1.0), log_std=None, head=head,
-                                 critic_on_side_stream=True, fuse_next_observation=True)
+                                 critic_on_side_stream=True)
     env = _kbot_env_state(m, consts, num_envs, seed)
     return consts, env, Rollout(consts, num_envs, rollout_length), gains
 
 
 def humanoid_rollout(num_envs: int = 4096, rollout_length: int = 16, seed: int = 1003, min_height: float = 0.6):
     """Benchmark config 3: free root + 21 hinges in a 5-limb tree, 4 foot spheres, friction 1.0, 21 PD actuators, root height
-    1.3 m, joints ~U(-0.1, 0.1), dt 0.005 with 4 substeps, fp32 actor 71 -> 3 x 256 (ELU) -> 21 means.  A reset's forward pass and the next
-    observation ride in other launches, as in `kbot_rollout`: four launches a control step instead of six, 328 -> 308 us for 4096 envs."""
+    1.3 m, joints ~U(-0.1, 0.1), dt 0.005 with 4 substeps, fp32 actor 71 -> 3 x 256 (ELU) -> 21 means."""
     m = km.humanoid_model(seed=seed)
     rng = np.random.default_rng(seed)
     act = actuators.PositionActuators(kps=tuple(rng.uniform(20.0, 150.0, m.nu)), kds=tuple(rng.uniform(0.5, 1.5, m.nu)))
@@ -144,7 +142,7 @@ def humanoid_rollout(num_envs: int = 4096, rollout_length: int = 16, seed: int =
     critic = _net((71, 256, 256, 256, 1), rng, dtype="f32")
     rewards = {"stay_alive": rw.StayAliveReward(scale=1.0), "upright": rw.UprightReward(scale=0.2)}
     consts = RolloutConstants(physics_model=dm, engine=eng, terms=terms, rewards=rewards, actor=actor, critic=critic,
-                              log_std=torch.full((m.nu,), -2.0, device=dev), defer_reset_forward=True, fuse_next_observation=True)
+                              log_std=torch.full((m.nu,), -2.0, device=dev))
     gen = torch.Generator(device=dev)
     gen.manual_seed(seed)
     ps = eng.reset(dm, 1.0, gen, num_envs, {})

@@ -1000,3 +1000,34 @@ def test_observation_in_the_terminating_launch_at_any_number_of_envs(N):
         runs.append([x.clone() for x in (traj.obs["obs"], traj.obs["noisy_obs"], traj.done, traj.qpos, traj.timestep, ro.reset_mask, ps.data.qpos)])
     for a, b in zip(*runs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("robot", ["humanoid", "kbot-lstm"])
+def test_a_state_written_between_two_control_steps_is_the_one_observed(robot):
+    """A program that pushes its robots between two `step_engine` calls: the next observation is of the pushed state, however it was
+    written.  And after a step that reset envs, the humanoid's warm starts are those of the new episodes."""
+    import dataclasses
+
+    from ksim_amd import configs
+    from ksim_amd.rollout import Rollout
+
+    N, T, runs = 48, 4, []
+    for apart in (False, True):
+        if robot == "humanoid":
+            c, env, ro = configs.humanoid_rollout(N, T, min_height=1.29)
+            off = dict(fuse_next_observation=False, defer_reset_forward=False)
+        else:
+            c, env, ro, _ = configs.kbot_lstm_rollout(N, T)
+            off = dict(fuse_next_observation=False)
+        if apart:
+            ro = Rollout(dataclasses.replace(c, **off), N, T)
+        d = env.physics_state.data
+        out = []
+        for t in range(T):
+            ro.step_engine(env, t)
+            out += [x.clone() for x in (ro.done[t], d.qpos, d.qacc_warmstart if robot == "humanoid" else d.qvel, d.contact_dist)]
+            d.qvel.data[:, 3:6] += 0.5
+        runs.append(out + [ro.obs.clone(), ro.action.clone()])
+        assert robot != "humanoid" or int(ro.done.sum()) > N // 4
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
