@@ -242,6 +242,7 @@ class HipEngine(PhysicsEngine):
         if mask is None:
             terms.terminate_reset(st, level=float(curriculum_level), seed=seed, step=step, apply_reset=2,
                                   reset_uniform=reset_uniform, episode=self.episode_args(state, episode_draws))
+            state._written = getattr(state, "_written", 0) + 1
         self.forward(physics_model, state, mask, randomization)
 
     def forward(self, physics_model, state: PhysicsState, mask=None, randomization=None, live=None) -> None:
@@ -351,6 +352,7 @@ class HipEngine(PhysicsEngine):
             raise ValueError(f"Unsupported actuators: {type(act).__name__}")
         if sched is not None:
             physics.work_order(physics_model, sched[1], sched[0])
+        physics_state._written = getattr(physics_state, "_written", 0) + 1
         return physics_state
 
 

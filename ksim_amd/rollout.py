@@ -75,7 +75,11 @@ class RolloutConstants:  # the static pieces, ksim/task/rl.py:138-150
     defer_reset_forward: bool = False
     # The observation of control step t + 1 is computed by the launch that ends step t (terminations, transition record,
     # resets): `ks_terminate_reset_observe`, one launch instead of two, the same numbers.  Taken when the task has no
-    # command set to advance in between and its observations read no derived field of the live state.
+    # command set to advance in between and its observations read no derived field of the live state.  A step that is called
+    # with other arguments than it was made for (level, noise), on other tensors, or on tensors that torch or the engine has
+    # written to since, observes afresh.  What writes behind torch's back (a program's own kernels, `.data`, replays of graphs)
+    # goes unnoticed: a program that does so between two steps leaves the switch off.  Stateful observations, which cannot
+    # be made twice, ride along inside `unroll` only.
     fuse_next_observation: bool = False
     head: GaussianHead | MixtureHead | None = None  # None: one mean per action entry and the log_std vector
     # A critic that does not share a launch with the actor (a recurrent one: a dozen short launches per control step) runs on a
@@ -149,15 +153,26 @@ class Rollout:
         reads_derived = any(src in used for src in need)
         self._defer = bool(c.defer_reset_forward) and not reads_derived
         self._fuse_obs = bool(c.fuse_next_observation) and not reads_derived and c.commands is None
-        self._obs_done = None  # (env state, slot, step) whose observation the previous step's last launch has written
+        self._obs_done = None  # `_observation_key` of the observation that the previous step's last launch has written
         self._side = None      # the critic's stream and its fork / join events (critic_on_side_stream), made on first use
         if c.actor.in_dim != c.terms.obs_dim or c.actor.out_dim != self.mean.shape[1]:
             raise _lib.KsError("actor must map the observation vector to one mean per action entry (or to what its head takes)")
         if c.critic is not None and (c.critic.in_dim != c.terms.obs_dim or c.critic.out_dim != 1):
             raise _lib.KsError("critic must map the observation vector to one value")
 
+    def _observation_key(self, env: RolloutEnvState, sources: Mapping, t: int, step: int, relative: bool, level: float):
+        """What the observation of slot t is made of: objects, and numbers with how often the engine and torch have written to them.
+        None where torch does not count that (inference mode)."""
+        site = (env.randomization_dict or {}).get("site_pose")
+        tensors = [x for x in (*sources.values(), env.physics_state.zero_offset, env.obs_bias, env.obs_carry, site, self.reset_mask,
+                               self.obs, self.noisy_obs) if x is not None]
+        if any(x.is_inference() for x in tensors):
+            return None
+        written = getattr(env.physics_state, "_written", 0)
+        return [env, self.c.terms, *tensors], [t, step, relative, float(level), env.seed, written, *(x._version for x in tensors)]
+
     def step_engine(self, env: RolloutEnvState, t: int, level: float = 1.0, noise: Mapping | None = None,
-                    _relative_step: bool = False) -> None:
+                    _relative_step: bool = False, _in_loop: bool = False) -> None:
         """One control step of every env; the transition lands in slot t of the buffers."""
         c, ps = self.c, env.physics_state
         d, noise = ps.data, noise or {}
@@ -176,8 +191,9 @@ class Rollout:
                         fresh=self.reset_mask if (c.terms.carry_dim or c.terms.has_bias) else None,
                         site_pose=(env.randomization_dict or {}).get("site_pose"))
 
-        ahead = self._obs_done
-        if ahead is None or ahead[0] is not env or ahead[1:] != (t, step, _relative_step):  # else the launch that ended the previous step wrote it
+        ahead = self._obs_done if not noise else None
+        now = ahead and self._observation_key(env, src, t, step, _relative_step, level)
+        if not now or ahead[1] != now[1] or any(a is not b for a, b in zip(ahead[0], now[0])):  # else the launch that ended the previous step wrote it
             c.terms.observe(src, self.N, bias_redraw=noise.get("obs_bias_redraw"), noise_normal=noise.get("obs_normal"),
                             noise_uniform=noise.get("obs_uniform"), carry_uniform=noise.get("obs_carry_uniform"),
                             **observe_args(t, step))
@@ -268,10 +284,11 @@ class Rollout:
                          event_reset_uniform=noise.get("event_reset_uniform"),
                          event_force=ps.event_states.get("_force_buffer") if ps.event_states else None,
                          contact_dist=d.contact_dist if "contact_dist" in self._live else None, episode=c.engine.episode_args(ps, noise.get("episode")))
-        if self._fuse_obs and t + 1 < self.T and not noise:
+        if self._fuse_obs and t + 1 < self.T and not noise and (_in_loop or _relative_step or not c.terms.carry_dim):
+            self._obs_done = self._observation_key(env, src, t + 1, step + 1, _relative_step, level)
+        if self._obs_done is not None:
             # the next step's observation rides in this launch (its random numbers are those of step + 1)
             c.terms.terminate_reset_observe(st, term_args, src, observe_args(t + 1, step + 1))
-            self._obs_done = (env, t + 1, step + 1, _relative_step)
         else:
             c.terms.terminate_reset(st, **term_args)
         # refresh the derived fields and the warm start of the reset envs (engine.py:213); in the deferred mode the next
@@ -290,7 +307,7 @@ class Rollout:
         if graph:
             return self._unroll_graph(env, level)
         for t in range(self.T):
-            self.step_engine(env, t, level)
+            self.step_engine(env, t, level, _in_loop=True)
         traj = self.trajectory()
         return traj, self._rewards(traj, env, level)
 

@@ -1031,3 +1031,47 @@ def test_a_state_written_between_two_control_steps_is_the_one_observed(robot):
         assert robot != "humanoid" or int(ro.done.sum()) > N // 4
     for a, b in zip(*runs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("change", ["level", "noise", "qvel", "command", "state", "step", "reset", "carry", "inference"])
+def test_an_observation_made_ahead_is_used_only_where_nothing_changed(change):
+    """`fuse_next_observation`: a step with other arguments, or on a state that was written to or replaced since, observes what it
+    is given, bit for bit as the launch of its own does."""
+    import dataclasses
+
+    from ksim_amd import observation as ob
+    from ksim_amd.env_terms import EnvTerms
+    from ksim_amd.rollout import Rollout
+
+    N, T, runs = 24, 4, []
+    with torch.inference_mode(change == "inference"):
+        for fuse in (False, True):
+            m, c, rnd_, _, _, EnvState = build(N, T, seed=9, min_height=0.86)
+            if change == "carry":  # an average: observed twice, it would move on twice
+                smooth = dict(c.terms.observations, g=ob.ProjectedGravityObservation(noise=0.01, min_lag=0.2, max_lag=0.6))
+                c = dataclasses.replace(c, terms=EnvTerms(m, smooth, c.terms.terminations, c.terms.resets, command_dim=2))
+                assert c.terms.carry_dim
+            ro = Rollout(dataclasses.replace(c, fuse_next_observation=fuse), N, T)
+            ps = c.engine.reset(c.physics_model, 1.0, 5, N, rnd_)
+            env = EnvState(ps, rnd_, torch.zeros(N, 2, device=DEV), None, seed=31)
+            ro.step_engine(env, 0)
+            level, noise = 1.0, None
+            if change == "level":
+                level = 0.25
+            elif change == "noise":
+                noise = {k: torch.rand(N, c.terms.obs_dim, device=DEV, generator=torch.Generator(DEV).manual_seed(3)) for k in ("obs_normal", "obs_uniform")}
+            elif change == "command":
+                env.commands[:, 1] = 0.5
+            elif change == "state":
+                ps = env.physics_state = c.engine.reset(c.physics_model, 1.0, 6, N, rnd_)
+            elif change == "step":
+                c.engine.step(ro.action[0], c.physics_model, ps, 1.0, 0, rnd_)
+            elif change == "reset":
+                c.engine.reset_where(c.physics_model, ps, None, 1.0, 7, 0, rnd_)
+            else:
+                ps.data.qvel[:, 3:6] += 0.5
+            for t in range(1, T):
+                ro.step_engine(env, t, level, noise if t == 1 else None)
+            runs.append([ro.obs.clone(), ro.noisy_obs.clone(), ro.action.clone(), ps.data.qpos.clone()])
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
