@@ -182,18 +182,19 @@ __global__ __launch_bounds__(256) void lstm_gate_backward_kernel(int64_t M, int 
 // steps, so that a minibatch of a thousand rows is one workgroup per CU.  A wavefront's 16 units keep their slice of W_hh for the whole sequence, cut
 // in three bf16 parts (ks_cut.h): two parts in registers, the third in LDS.  A step is the products of the cut state with it (CutTile), the gate
 // arithmetic of one or two (unit, row) per lane, and one barrier.  fp32 cells of hidden size 128.
-// On v_mfma_f32_4x4x1, four rows a workgroup, a step's products took 2048 cycles for four rows; cut they take 1536 for four and 2048 for eight, and
-// they round less (the state after 100 steps is 1.8e-7 from 64 bits, the gate gradients 1.73e-7, of 1.78e-7).  Two layers (blockIdx.y), 100 steps, us:
+// On v_mfma_f32_4x4x1, four rows a workgroup, a step's products took 2048 cycles for four rows; cut they take 1536 for four and 2560 for eight, and
+// a sum rounds no more (the state after 100 steps is 1.8e-7 from 64 bits as it was, the gate gradients 1.6e-7, of 1.8e-7).  Two layers (blockIdx.y), 100 steps, us:
 //   rows a layer:                     64         360 (60 steps)   1024
-//   forward, activations kept     154 -> 128   112 -> 102       435 -> 342
-//   forward, not kept             136 -> 124                    335 -> 236
-//   backward                      139 -> 119   102 -> 97        365 -> 287
+//   forward, activations kept     154 -> 134   112 -> 103       400 -> 340
+//   forward, not kept             135 -> 132                    327 -> 268
+//   backward                      139 -> 118    99 -> 94        348 -> 296
+// 24 steps of 512 rows, every CU at work once: 53 -> 50, not kept 44.7 -> 46.7 (the weights' cut), backward 54 -> 52.
 // With activations kept, 1024 rows move 1.2 GB, 240 us at the rate of a large copy.  What is left: issue, since only two vector instructions hide under
-// a 16-cycle matrix instruction (eight rows 4400 cycles a step, of which products 2048), the state's way through LDS at the head of a step (400), and the
+// a 16-cycle matrix instruction (eight rows 5100 cycles a step, of which products 2560), the state's way through LDS at the head of a step (400), and the
 // clock, which falls to 1.9 GHz with every CU at work.  Also built: two sets of four rows half a step apart, one's gates between the other's products
-// (300 us of 240, not kept: nothing more hides, and four rows need 1.5 times the products); the backward product split over the gate rows instead
-// of over the units of dh (175 us of 119 for 64 rows: eight times the tiles' ends, and partial sums to add).
-typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+// (not kept 300 us: nothing more hides, and four rows need 1.2 times the products); the backward product split over the gate rows instead
+// of over the units of dh (175 us of 119 for 64 rows: eight times the tiles' ends, and partial sums to add); all weights requested before the first is cut (the
+// same); a copy of the steps for operands that cannot overflow, without the check for it (64 rows 129, not kept 126, 1024 rows kept 378: the copies' registers).
 struct Seq {
   int64_t M;
   const float* in;  // forward: the input projections (T, M, gates); backward: dH
@@ -272,74 +273,88 @@ constexpr int kStepRows = 16;
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 
 // A 16-column tile of the product of R rows with fp32 weights, both cut in three (cut_bf16).  The parts are rows of the A operand, which has sixteen:
-//   R = 8: rows 0..7 and 8..15 of `a` are first and second parts, `b` has the third parts twice: four instructions per 32 k.
-//   R = 4: rows 0..3, 4..7, 8..11 of `a` are first, second and third parts, `b` is `a` without the third: three instructions per 32 k.
-// The first and second parts times all parts of the weights and the third parts times the first are seven of the nine products; the two that are left out are
-// below 2^-23 and 2^-32 of the result.  Each part's products go into a sum of their own in order of k, and an entry is s0 + (s1 + s2): its bits do not
-// depend on R.
-//   SPLIT: the weights' second and third parts go into a sum of their own, so that with R = 4 the third parts' rows of it are left out at the end and `b` is
-//   not needed: for a single tile over a long reduction, where masking `a` costs more than four additions.
+//   R = 8: rows 0..7 and 8..15 of `a` are first and second parts, of `b` third and again first parts: five instructions per 32 k.
+//   R = 4: rows 0..3, 4..7, 8..11, 12..15 of `a` are first, second, third and again first parts, `b` is `a` without the latter two: three instructions per 32 k.
+// Eight of the nine products, all but the one of the third parts, below 2^-32 of the result.  With s(i, j) the sum of the products of the state's part i with
+// the weights' part j in order of k, and s(i, 12) of both smaller parts' together, an entry is s(0, 0) + ((s(0, 12) + (s(2, 0) + s(2, 1))) + (s(1, 0) + s(1, 12))):
+// the largest products by themselves, so that a sum of one term, or of one among zeros, is rounded once.  Its bits do not depend on R, nor on other rows.
+//   SPLIT: s(i, 12) is s(i, 1) + s(i, 2), so that with R = 4 the product of the third parts is left out at the end and `b` is not needed: for a single tile over
+//   a long reduction, where masking `a` costs more than the additions.
+// Without the state's third times the weights' second parts, and with the smaller products in the sum of the largest, eight rows took four instructions per 32 k (1024
+// rows 240 us instead of 268, kept 325 instead of 340, backward 280 instead of 296), but a single product was up to 3.5 times 2^-24 off, instead of once.
 template <int R, bool SPLIT>
 struct CutTile {
-  static constexpr int kSteps = R == 8 ? 4 : 3;  // matrix instructions per 32 k
-  f32x4 ab, third, rest;
-  __device__ __forceinline__ void clear() { ab = third = rest = f32x4{0.f, 0.f, 0.f, 0.f}; }
+  static constexpr int kSteps = R == 8 ? 5 : 3;  // matrix instructions per 32 k
+  f32x4 a0, a1, a2, b0, b1;                      // the sums over `a` and `b` by the weights' parts; without SPLIT a1 has those of a2 as well
+  __device__ __forceinline__ void clear() { a0 = a1 = a2 = b0 = b1 = f32x4{0.f, 0.f, 0.f, 0.f}; }
   __device__ __forceinline__ void add(int step, bf16x8 a, bf16x8 b, bf16x8 w0, bf16x8 w1, bf16x8 w2) {
-    f32x4& low = SPLIT ? rest : ab;
-    if (step == 0) ab = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w0, ab, 0, 0, 0);
-    if (R == 8 && step == 1) third = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, w0, third, 0, 0, 0);
-    if (step == kSteps - 2) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(R == 8 || SPLIT ? a : b, w1, low, 0, 0, 0);
-    if (step == kSteps - 1) low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(R == 8 || SPLIT ? a : b, w2, low, 0, 0, 0);
+    f32x4& to = SPLIT ? a2 : a1;
+    if (step == 0) a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w0, a0, 0, 0, 0);
+    if (step == kSteps / 2) a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w1, a1, 0, 0, 0);
+    if (step == kSteps - 1) to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(R == 8 || SPLIT ? a : b, w2, to, 0, 0, 0);
+    if (R == 8 && step == 1) b0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, w0, b0, 0, 0, 0);
+    if (R == 8 && step == 3) b1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, w1, b1, 0, 0, 0);
   }
-  // In kRows pieces, which stand between matrix instructions: lane l gets column l % 16 of rows seq_row<R>(l) + q in out[q].  TAME: no operand is
-  // infinite and no sum overflows; otherwise, with SPLIT, the first parts decide (join_cut).  `upper`, 0 or 1: with R = 8 the lanes 32..63, which hold the
-  // second parts' rows; with R = 4 and SPLIT those that don't hold third parts' rows; 0 with R = 4 otherwise.  The swaps' operands come out of vector
-  // instructions, never straight out of a matrix instruction: nothing inserts that one's wait states into the asm.  (The builtins give the same
-  // result twice where both are used.)
-  static constexpr int kRows = 4;
-  template <bool TAME>
-  __device__ __forceinline__ void rows(int piece, float& upper, float (&t)[4], float (&out)[R / 4]) const {
-    if (piece < 2) {
-      pin(upper);
+  // which of a lane's sums count, as factors (0 or 1): R = 8 lanes 32..63 and 0..31, R = 4 lane rows 1 to 3 and 0 to 2; `kept` R = 4's lane rows 0 and 1
+  struct Lanes {
+    float upper, lower, kept;
+    __device__ __forceinline__ explicit Lanes(int lane) : upper(lane >= 4 * R ? 1.f : 0.f), lower(lane < (R == 8 ? 32 : 48) ? 1.f : 0.f), kept(lane < 32 ? 1.f : 0.f) {}
+  };
+  // In kRows pieces, which stand between matrix instructions: lane l gets column l % 16 of rows seq_row<R>(l) + q in out[q].  `t` carries values from one
+  // piece to the next.  The swaps' operands come out of vector instructions, never straight out of a matrix instruction: nothing inserts that one's wait
+  // states into the asm.  (The builtins give the same result twice where both are used.)
+  static constexpr int kRows = R == 8 ? 8 : 4;
+  __device__ __forceinline__ void rows(int piece, Lanes& lanes, float (&t)[4], float (&out)[R / 4]) const {
+    constexpr int kEach = R == 8 ? 1 : 2, kSwap = 4 / kEach;
+    if (piece < kSwap) {
+      pin(lanes.upper);
+      pin(lanes.lower);
 #pragma unroll
-      for (int i = 2 * piece; i < 2 * piece + 2; ++i) {
-        if constexpr (SPLIT && R == 4) t[i] = TAME ? fmaf(rest[i], upper, ab[i]) : join_cut(ab[i], upper != 0.f ? rest[i] : 0.f);
-        else if constexpr (SPLIT) t[i] = TAME ? fmaf(third[i], upper, ab[i] + rest[i]) : join_cut(ab[i], rest[i] + (upper != 0.f ? third[i] : 0.f));
-        else t[i] = R == 4 ? ab[i] + upper : fmaf(third[i], upper, ab[i]);
+      for (int i = kEach * piece; i < kEach * piece + kEach; ++i) {
+        if constexpr (R == 8) t[i] = fmaf(b0[i] + b1[i], lanes.lower, fmaf(a0[i], lanes.upper, SPLIT ? a1[i] + a2[i] : a1[i]));
+        else if constexpr (!SPLIT) t[i] = fmaf(a1[i], lanes.lower, a0[i] * lanes.upper);
+        else t[i] = lanes.lower != 0.f ? fmaf(a0[i], lanes.upper, fmaf(a2[i], lanes.kept, a1[i])) : a0[i];  // whose infinities have to arrive as such
       }
     }
     if constexpr (R == 8) {
-      if (piece == 2)
+      if (piece == kSwap)
         asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
-      if (piece == 3) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) out[q] = TAME ? t[q] + t[q + 2] : join_cut(t[q], t[q + 2]);
+      if (piece == kSwap + 1) t[0] += t[2], t[1] += t[3];
+      if (piece == kSwap + 2) {  // the first parts' sums of the lane's rows
+        const bool upper = (threadIdx.x & 32) != 0;
+        t[2] = upper ? b0[2] : a0[0], t[3] = upper ? b0[3] : a0[1];
       }
+      if (piece == kSwap + 3) out[0] = t[2] + t[0], out[1] = t[3] + t[1];
     } else {
-      if (piece == 2)  // register i of lane row q changes places with register q of lane row i
+      if (piece == kSwap)  // register i of lane row q changes places with register q of lane row i
         asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
                      "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1"
                      : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
-      if (piece == 3) out[0] = TAME ? t[0] + (t[1] + t[2]) : join_cut(t[0], t[1] + t[2]);
+      if (piece == kSwap + 1) out[0] = t[3] + ((t[0] + t[2]) + t[1]);
     }
+  }
+  // for the lane's rows, from the sums of `a`'s rows over a matrix instruction (its wait states included), those of the first parts
+  static __device__ __forceinline__ void first_rows(const f32x4& sum, float (&p)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = sum[i];
+    asm volatile("s_nop 15\n\ts_nop 15\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+    if (R == 4) asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(p[0]), "+v"(p[1]));
   }
 };
 template <int R>
 __device__ __forceinline__ int seq_row(int lane) { return R == 8 ? 4 * ((lane >> 4) & 1) + 2 * (lane >> 5) : lane >> 4; }
-template <int R>  // the row of `a` that lane l holds, among R first, R second and R third parts
-__device__ __forceinline__ int cut_row(int lane) { return R == 8 || (lane & 15) < 12 ? lane & 15 : 11; }
+// the operands' rows (CutTile) out of R first, R second and R third parts
 template <int R>
-__device__ __forceinline__ void get_cut(const unsigned short* rows, int ld, int lane, int k, bf16x8& a, bf16x8& b) {
-  a = *reinterpret_cast<const bf16x8*>(rows + cut_row<R>(lane) * ld + k);
-  if constexpr (R == 8) b = *reinterpret_cast<const bf16x8*>(rows + (16 + (lane & 7)) * ld + k);
-  else b = (lane & 8) ? bf16x8{} : a;
+__device__ __forceinline__ bf16x8 get_a(const unsigned short* rows, int ld, int lane, int k) {
+  const int row = lane & 15;
+  return *reinterpret_cast<const bf16x8*>(rows + (R == 8 || row < 12 ? row : row - 12) * ld + k);
 }
-// Sums of 512 products of tame operands do not overflow.  The upper halves of two values at a time; infinities and NaN are larger than all others.
-__device__ __forceinline__ void largest(unsigned halves, u16x2& most) {
-  most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, halves & 0x7fff7fffu));
+template <int R>
+__device__ __forceinline__ bf16x8 get_b(const unsigned short* rows, int ld, int lane, int k, bf16x8 a) {
+  const int row = lane & 15;
+  if constexpr (R == 8) return *reinterpret_cast<const bf16x8*>(rows + (row < 8 ? 16 + row : row - 8) * ld + k);
+  else return (row & 8) ? bf16x8{} : a;
 }
-__device__ __forceinline__ bool wild(u16x2 most) { return (most.x > most.y ? most.x : most.y) >= 0x5d80; }  // 2^60
-
 // the entry `bytes` after base[entries], whose address is the same for every lane
 template <typename T>
 __device__ __forceinline__ T& at(T* base, int64_t entries, unsigned bytes) {
@@ -373,7 +388,6 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
   // matrix instructions to stand between.  B operand: column lane % 16 is the unit, rows k = 32 kb + 8 (lane / 16) + 0..7.
   constexpr int kGate[4] = {1, 2, 0, 3};
   bf16x8 w0[4][KB], w1[4][KB];
-  u16x2 most = {};
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const float* src = W + (int64_t)(kGate[n] * H + unit) * ldw + kq;
@@ -383,8 +397,6 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
       const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       u32x4 part[3];
       cut_bf16<3>(v, part);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) largest(part[0][e], most);
       w0[n][kb] = __builtin_bit_cast(bf16x8, part[0]);
       w1[n][kb] = __builtin_bit_cast(bf16x8, part[1]);
       w2[(n * KB + kb) * 64] = part[2];
@@ -434,7 +446,6 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
     for (int p = 0; p < 3; ++p)
 #pragma unroll
       for (int q = 0; q < V; ++q) sh[to][p * R + row + q][unit] = (unsigned short)(part[p] >> (16 * q));
-    return part[0];
   };
 #pragma unroll
   for (int q = 0; q < V; ++q) {
@@ -443,125 +454,159 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
 #pragma unroll
     for (int gate = 0; gate < 5; ++gate) load(0, gate, q);
   }
-  largest(begin(0), most);
+  begin(0);
   seq_loads_done();
-  const bool tame = !__syncthreads_or(wild(most));  // later states are below 1
-  auto steps = [&](auto tame) __attribute__((always_inline)) {
-    constexpr bool TAME = decltype(tame)::value;
-    typedef CutTile<R, !TAME> Tile;  // the first parts' products by themselves where they may have to decide
-    float upper = (R == 8 || !TAME) && (lane >= 32) == (R == 8) ? 1.f : 0.f;
-    float x[V] = {}, t4[4] = {};
-    // A tile's gate, in pieces of a few instructions (`x` carries the value from one to the next): activation(x) of the hardware exponential and
-    // reciprocal (about 1 ulp each) instead of the library's expf, tanhf and IEEE division, a fifth of the instructions.
-    constexpr int kAct = R == 8 ? 8 : 5;
-    auto act = [&](int gate, int piece) __attribute__((always_inline)) {
-      auto add_input = [&](int q) { x[q] = g[q][gate] + x[q]; };
-      auto scale = [&](int q) { x[q] *= gate == 2 ? 2.f * kLog2e : -kLog2e; };
-      auto power = [&](int q) { x[q] = __builtin_amdgcn_exp2f(x[q]); };
-      auto invert = [&](int q) { x[q] = __builtin_amdgcn_rcpf(x[q]); };
-      auto finish = [&](int q) { v[q][gate] = gate == 2 ? fmaf(-2.f, x[q], 1.f) : x[q]; };
-      if constexpr (R == 8) {
-        if (piece == 0) add_input(0), add_input(1);
-        if (piece == 1) scale(0), scale(1);
-        if (piece == 2 || piece == 3) power(piece - 2);
-        if (piece == 4) x[0] += 1.f, x[1] += 1.f;
-        if (piece == 5 || piece == 6) invert(piece - 5);
-        if (piece == 7) finish(0), finish(1);
-      } else {
-        if (piece == 0) add_input(0);
-        if (piece == 1) scale(0);
-        if (piece == 2) power(0);
-        if (piece == 3) x[0] += 1.f, invert(0);
-        if (piece == 4) finish(0);
-      }
-    };
-    auto step = [&](int t, auto from, bool first) __attribute__((always_inline)) {
-      bf16x8 a[KB], b[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) get_cut<R>(&sh[from][0][0], kLstmStateLd, lane, 32 * kb + kq, a[kb], b[kb]);
-      u32x4 ring[2] = {w2[0], w2[64]};
-      Tile tile, done;
-      constexpr int S = Tile::kSteps, N = KB * S;  // matrix instructions per 32 k and per tile
-      constexpr int R0 = 2, A0 = R0 + Tile::kRows, L0 = A0 + kAct;
-      static_assert(L0 + V <= N && 9 * V <= 2 * N, "");
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        if (n > 0) done = tile;
-        tile.clear();
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const int kb = i / S, slot = n * KB + kb;
-          tile.add(i % S, a[kb], b[kb], w0[n][kb], w1[n][kb], __builtin_bit_cast(bf16x8, ring[slot % 2]));
-          if (i % S == S - 1 && slot + 2 < 4 * KB) ring[slot % 2] = w2[(slot + 2) * 64];
-          // between the matrix instructions: under the first tile the last step's results leave; under the next ones the gate of the tile before
-          __builtin_amdgcn_sched_barrier(0);
-          if (n == 0) {
-            if (SAVE && !first) {
-#pragma unroll
-              for (int k = 9 * V * i / N; k < 9 * V * (i + 1) / N; ++k) store(t - 1, k / V, k % V);
-            }
-            if (i == N - 1) {
-#pragma unroll
-              for (int q = 0; q < V; ++q) {
-                load(t + 1, 4, q);
-                v[q][5] = cn[q];
-                v[q][6] = hn[q];
-              }
-            }
-          } else {
-            const int gate = kGate[n - 1];
-            if (i >= R0 && i < L0) {
-#pragma unroll
-              for (int k = 0; k < 4; ++k) pin(t4[k]);
-#pragma unroll
-              for (int q = 0; q < V; ++q) pin(x[q]);
-              if (i < A0) done.template rows<TAME>(i - R0, upper, t4, x);
-              else act(gate, i - A0);
-            }
-            if (i >= L0 && i < L0 + V) load(t + 1, gate, i - L0);
-            if (n == 3 && i == N - 1) {
-#pragma unroll
-              for (int q = 0; q < V; ++q) c[q] = fmaf(v[q][1], v[q][5], v[q][0] * v[q][2]);
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      // what has no more matrix instructions to stand between: tanh of the cell state and the output gate
-#pragma unroll
-      for (int k = 0; k < Tile::kRows; ++k) tile.template rows<TAME>(k, upper, t4, x);
-#pragma unroll
-      for (int k = 0; k < kAct; ++k) act(3, k);
-#pragma unroll
-      for (int q = 0; q < V; ++q) {
-        v[q][4] = seq_tanh(c[q]);
-        h[q] = v[q][3] * v[q][4];
-      }
-      begin(1 - decltype(from)::value);
-#pragma unroll
-      for (int q = 0; q < V; ++q) load(t + 1, 3, q);
-      if constexpr (!SAVE) {
-#pragma unroll
-        for (int k = 0; k < 2 * V; ++k) store(t, k / V, k % V);
-      }
-      lds_barrier();  // the new state is complete; the buffer just read is free for the step after next
-    };
-    constexpr std::integral_constant<int, 0> even{};
-    constexpr std::integral_constant<int, 1> odd{};
-    step(0, even, true);
-    int t = 1;
-    for (; t + 1 < T; t += 2) {
-      step(t, odd, false);
-      step(t + 1, even, false);
-    }
-    if (t < T) step(t, odd, false);
-    if constexpr (SAVE) {
-#pragma unroll
-      for (int k = 0; k < 9 * V; ++k) store(T - 1, k / V, k % V);
+  __syncthreads();
+  typedef CutTile<R, false> Tile;
+  typename Tile::Lanes lanes(lane);
+  float x[V] = {}, t4[4] = {}, bad = 0.f;
+  auto activate = [](int gate, float x) {
+    x = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * (gate == 2 ? 2.f * kLog2e : -kLog2e)) + 1.f);
+    return gate == 2 ? fmaf(-2.f, x, 1.f) : x;
+  };
+  // A tile's gate, in pieces of a few instructions (`x` carries the value from one to the next): activation(x) of the hardware exponential and
+  // reciprocal (about 1 ulp each) instead of the library's expf, tanhf and IEEE division, a fifth of the instructions.
+  constexpr int kAct = R == 8 ? 8 : 5;
+  auto act = [&](int gate, int piece) __attribute__((always_inline)) {
+    auto add_input = [&](int q) { x[q] = g[q][gate] + x[q]; };
+    auto scale = [&](int q) { x[q] *= gate == 2 ? 2.f * kLog2e : -kLog2e; };
+    auto check = [&](int q) { bad = fmaf(x[q], 0.f, bad); };  // NaN once a preactivation is not finite
+    auto power = [&](int q) { x[q] = __builtin_amdgcn_exp2f(x[q]); };
+    auto invert = [&](int q) { x[q] = __builtin_amdgcn_rcpf(x[q]); };
+    auto finish = [&](int q) { v[q][gate] = gate == 2 ? fmaf(-2.f, x[q], 1.f) : x[q]; };
+    if constexpr (R == 8) {
+      if (piece == 0) add_input(0), add_input(1);
+      if (piece == 1) scale(0), scale(1);
+      if (piece == 2 || piece == 3) check(piece - 2), power(piece - 2);
+      if (piece == 4) x[0] += 1.f, x[1] += 1.f;
+      if (piece == 5 || piece == 6) invert(piece - 5);
+      if (piece == 7) finish(0), finish(1);
+    } else {
+      if (piece == 0) add_input(0);
+      if (piece == 1) check(0), scale(0);
+      if (piece == 2) power(0);
+      if (piece == 3) x[0] += 1.f, invert(0);
+      if (piece == 4) finish(0);
     }
   };
-  if (tame) steps(std::true_type{});
-  else steps(std::false_type{});
+  auto cells = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < V; ++q) c[q] = fmaf(v[q][1], v[q][5], v[q][0] * v[q][2]);
+  };
+  auto leave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      v[q][4] = seq_tanh(c[q]);
+      h[q] = v[q][3] * v[q][4];
+    }
+  };
+  // Step t's gates whose sums of the first parts' products are not finite: those decide, the other parts of an infinity are NaN.
+  auto first_parts = [&](int t, int from) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      f32x4 sum = {};
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(get_a<R>(&sh[from][0][0], kLstmStateLd, lane, 32 * kb + kq), w0[n][kb], sum, 0, 0, 0);
+      float p[4];
+      Tile::first_rows(sum, p);
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const float gate = activate(kGate[n], at(gi, (((int64_t)t * M + r0) * 4 + kGate[n]) * H, og[q]) + p[q]);
+        v[q][kGate[n]] = fabsf(p[q]) < __builtin_inff() ? v[q][kGate[n]] : gate;
+      }
+    }
+    cells();
+  };
+  auto step = [&](int t, auto from, bool first) __attribute__((always_inline)) {
+    constexpr int B = R == 8 ? 2 : KB;  // eight rows read `b` again for each tile
+    bf16x8 a[KB], b[B];
+    auto load_b = [&](int kb) __attribute__((always_inline)) { b[kb % B] = get_b<R>(&sh[from][0][0], kLstmStateLd, lane, 32 * kb + kq, a[kb]); };
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) a[kb] = get_a<R>(&sh[from][0][0], kLstmStateLd, lane, 32 * kb + kq);
+#pragma unroll
+    for (int kb = 0; kb < B; ++kb) load_b(kb);
+    u32x4 ring[2] = {w2[0], w2[64]};
+    Tile tile, done;
+    constexpr int S = Tile::kSteps, N = KB * S;  // matrix instructions per 32 k and per tile
+    constexpr int R0 = 2, A0 = R0 + Tile::kRows, L0 = A0 + kAct;
+    static_assert(L0 + V <= N && 9 * V <= 2 * N, "");
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      if (n > 0) done = tile;
+      tile.clear();
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int kb = i / S, slot = n * KB + kb;
+        tile.add(i % S, a[kb], b[kb % B], w0[n][kb], w1[n][kb], __builtin_bit_cast(bf16x8, ring[slot % 2]));
+        if (i % S == S - 1 && slot + 2 < 4 * KB) {
+          ring[slot % 2] = w2[(slot + 2) * 64];
+          if (B < KB) load_b((kb + B) % KB);
+        }
+        // between the matrix instructions: under the first tile the last step's results leave; under the next ones the gate of the tile before
+        __builtin_amdgcn_sched_barrier(0);
+        if (n == 0) {
+          if (SAVE && !first) {
+#pragma unroll
+            for (int k = 9 * V * i / N; k < 9 * V * (i + 1) / N; ++k) store(t - 1, k / V, k % V);
+          }
+          if (i == N - 1) {
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+              load(t + 1, 4, q);
+              v[q][5] = cn[q];
+              v[q][6] = hn[q];
+            }
+          }
+        } else {
+          const int gate = kGate[n - 1];
+          if (i >= R0 && i < L0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) pin(t4[k]);
+#pragma unroll
+            for (int q = 0; q < V; ++q) pin(x[q]);
+              if (i < A0) done.rows(i - R0, lanes, t4, x);
+            else act(gate, i - A0);
+          }
+          if (i >= L0 && i < L0 + V) load(t + 1, gate, i - L0);
+          if (n == 3 && i == N - 1) cells();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // what has no more matrix instructions to stand between: tanh of the cell state and the output gate
+#pragma unroll
+    for (int k = 0; k < Tile::kRows; ++k) tile.rows(k, lanes, t4, x);
+#pragma unroll
+    for (int k = 0; k < kAct; ++k) act(3, k);
+    leave();
+    if (__builtin_expect(__any(!(bad == 0.f)), 0)) {
+      bad = 0.f;
+      first_parts(t, from);
+      leave();
+    }
+    begin(1 - decltype(from)::value);
+#pragma unroll
+    for (int q = 0; q < V; ++q) load(t + 1, 3, q);
+    if constexpr (!SAVE) {
+#pragma unroll
+      for (int k = 0; k < 2 * V; ++k) store(t, k / V, k % V);
+    }
+    lds_barrier();  // the new state is complete; the buffer just read is free for the step after next
+  };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  step(0, even, true);
+  int t = 1;
+  for (; t + 1 < T; t += 2) {
+    step(t, odd, false);
+    step(t + 1, even, false);
+  }
+  if (t < T) step(t, odd, false);
+  if constexpr (SAVE) {
+#pragma unroll
+    for (int k = 0; k < 9 * V; ++k) store(T - 1, k / V, k % V);
+  }
   }
 }
 
@@ -629,7 +674,7 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
     const int gate = kGate[n];
     float pre[4];
     if (n + 1 < 4) inputs(n + 1);
-    f32x4 sum[3] = {};  // of the state's parts: CutTile's products in its order
+    f32x4 first[3] = {}, low[3] = {};  // by the state's parts: CutTile's products in its order
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const int slot = n * KB + kb;
@@ -641,18 +686,17 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
       const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       u32x4 part[3];
       cut_bf16<3>(x, part);
-      mma(a[0], part[0], sum[0]);
-      mma(a[1], part[0], sum[1]);
-      mma(a[2], part[0], sum[2]);
-      mma(a[0], part[1], sum[0]);
-      mma(a[1], part[1], sum[1]);
-      mma(a[0], part[2], sum[0]);
-      mma(a[1], part[2], sum[1]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) mma(a[p], part[0], first[p]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) mma(a[p], part[1], low[p]);
+      mma(a[0], part[2], low[0]);
+      mma(a[1], part[2], low[1]);
     }
     bool finite = true;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      pre[i] = sum[0][i] + (sum[1][i] + sum[2][i]);
+      pre[i] = first[0][i] + ((low[0][i] + (first[2][i] + low[2][i])) + (first[1][i] + low[1][i]));
       finite = finite && fabsf(pre[i]) < __builtin_inff();
     }
     if (__any(!finite)) {  // the first parts decide, so their products go by themselves
@@ -703,15 +747,16 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
 // The reverse sweep of the same layer: dH (T, M, H) is the gradient reaching h_t from the layer above; the gradient through
 // W_hh and that of the cell state are carried in registers.  Per step: the gate derivatives from the saved activations
 // (lstm_gate_backward_kernel's formulas) into d_g (T, M, 4H) and, cut in three, into LDS, then dh_{t-1} = d_g W_hh over the transposed weights: a
-// wavefront's tile is its 16 units, over all 4H gate rows.  The weights' third parts lie in registers for kThirdRegs of the sixteen k blocks and in LDS
-// for the others.
-constexpr int kThirdRegs = 4, kLstmGateLd = 4 * kSeqH + 8;
-constexpr int lstm_backward_lds(int rows) { return kSeqWaves * (16 - kThirdRegs) * 64 * 16 + 2 * 3 * rows * kLstmGateLd * 2; }
+// wavefront's tile is its 16 units, over all 4H gate rows.  The weights' third parts lie in registers for third_regs of the sixteen k blocks and in LDS
+// for the others; eight rows, which have more sums, leave as few there as LDS allows and read the gate gradients a block less ahead.
+constexpr int kLstmGateLd = 4 * kSeqH + 8;
+constexpr int third_regs(int rows) { return rows == 8 ? 3 : 4; }
+constexpr int lstm_backward_lds(int rows) { return kSeqWaves * (16 - third_regs(rows)) * 64 * 16 + 2 * 3 * rows * kLstmGateLd * 2; }
 
 template <int R>
 __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lstm_seq_backward_kernel(int T, Seq first, Seq second) {
-  constexpr int H = kSeqH, V = R / 4, KB = 4 * H / 32;
+  constexpr int H = kSeqH, V = R / 4, KB = 4 * H / 32, kThirdRegs = third_regs(R), kAhead = R == 8 ? 2 : 3;
   const Seq s = blockIdx.y == 0 ? first : second;
   const int64_t M = s.M;
   const float* __restrict__ dH = s.in;
@@ -727,7 +772,7 @@ void lstm_seq_backward_kernel(int T, Seq first, Seq second) {
   extern __shared__ __attribute__((aligned(16))) unsigned char seq_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int unit = 16 * wave + (lane & 15), row = seq_row<R>(lane), kq = 8 * (lane >> 4);  // the (unit, rows) whose gates this lane owns
-  float upper = (lane >= 32) == (R == 8) ? 1.f : 0.f;
+  typename CutTile<R, true>::Lanes lanes(lane);
   u32x4* w2 = reinterpret_cast<u32x4*>(seq_lds) + wave * (16 - kThirdRegs) * 64 + lane;  // k block kThirdRegs and on
   typedef unsigned short Gates[3 * R][kLstmGateLd];
   Gates* sg = reinterpret_cast<Gates*>(seq_lds + kSeqWaves * (16 - kThirdRegs) * 64 * 16);  // of even and odd steps
@@ -792,17 +837,22 @@ void lstm_seq_backward_kernel(int T, Seq first, Seq second) {
         for (int q = 0; q < V; ++q) sg[cur][p * R + row + q][g * H + unit] = (unsigned short)(part[p] >> (16 * q));
     }
     lds_barrier();  // the gate gradients are complete; the buffer of the step before is free for the step after
-    bf16x8 a[4], b[4];
+    constexpr int D = kAhead + 1;
+    bf16x8 a[D], b[D];
+    auto load_ab = [&](int kb) __attribute__((always_inline)) {
+      a[kb % D] = get_a<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * kb + kq);
+      if constexpr (R == 8) b[kb % D] = get_b<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * kb + kq, a[kb % D]);
+    };
 #pragma unroll
-    for (int kb = 0; kb < 3; ++kb) get_cut<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * kb + kq, a[kb], b[kb]);
+    for (int kb = 0; kb < kAhead; ++kb) load_ab(kb);
     CutTile<R, true> tile;
     tile.clear();
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      if (kb + 3 < KB) get_cut<R>(&sg[cur][0][0], kLstmGateLd, lane, 32 * (kb + 3) + kq, a[(kb + 3) % 4], b[(kb + 3) % 4]);
+      if (kb + kAhead < KB) load_ab(kb + kAhead);
 #pragma unroll
       for (int i = 0; i < CutTile<R, true>::kSteps; ++i)
-        tile.add(i, a[kb % 4], b[kb % 4], w0[kb], w1[kb],
+        tile.add(i, a[kb % D], b[kb % D], w0[kb], w1[kb],
                  kb < kThirdRegs ? w2r[kb < kThirdRegs ? kb : 0] : __builtin_bit_cast(bf16x8, w2[(kb - (kb < kThirdRegs ? kb : kThirdRegs)) * 64]));
       // between the products the step's gate gradients leave and the inputs of the next come
       __builtin_amdgcn_sched_barrier(0);
@@ -815,10 +865,11 @@ void lstm_seq_backward_kernel(int T, Seq first, Seq second) {
     }
     float x[V];
 #pragma unroll
-    for (int k = 0; k < CutTile<R, true>::kRows; ++k) tile.template rows<true>(k, upper, t4, x);
-    if (__any(!(fabsf(x[0]) < __builtin_inff()) || !(fabsf(x[V - 1]) < __builtin_inff()))) {  // where all is finite the other way would be no different
+    for (int k = 0; k < CutTile<R, true>::kRows; ++k) tile.rows(k, lanes, t4, x);
 #pragma unroll
-      for (int k = 0; k < CutTile<R, true>::kRows; ++k) tile.template rows<false>(k, upper, t4, x);
+    for (int q = 0; q < V; ++q) {  // the first parts decide, entry by entry
+      const float first = t4[R == 8 ? 2 + q : 3];
+      x[q] = fabsf(first) < __builtin_inff() ? x[q] : first;
     }
 #pragma unroll
     for (int q = 0; q < V; ++q) dhc[q] = f[q] ? 0.f : x[q];

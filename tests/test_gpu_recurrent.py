@@ -691,3 +691,68 @@ def test_lstm_sequences_take_infinite_and_very_large_operands_as_a_plain_product
             scale = gates.abs().nan_to_num(0, 0, 0).amax(1, keepdim=True).clamp_min(1)
             torch.testing.assert_close((got / scale).nan_to_num(0, 0, 0), (gates / scale).nan_to_num(0, 0, 0), rtol=0, atol=4e-6, msg=lambda m: f"{kind}, step {t}: {m}")
             dc, dh = dct * f, gates @ wh
+
+
+def _largest_error(got, exact, size):
+    """in units of 2^-24 of the terms' size, which is what one rounding may cost at most"""
+    return float(((got.double() - exact).abs() / size).max() * 2 ** 24)
+
+
+@pytest.mark.parametrize("terms", [1, 2])
+@pytest.mark.parametrize("rows,Tn", [(5, 1), (5, 2), (1030, 1), (1030, 2)])
+def test_lstm_recurrent_products_of_few_terms_round_as_often_as_they_have_terms(rows, Tn, terms):
+    """States with one or two entries that are not zero, and gate inputs that take the rounded product away again, so that a preactivation is
+    what the product was rounded by.  One step and sequences, four and eight rows per workgroup, against 64 bits: an fp32 sum of n terms
+    may be off by n times 2^-24 of their size.  Beside it the sums of the smaller parts' products, below 2^-6 of a term, round four times at
+    most, 2^-4 of that unit, and the activations' own 2e-6 of a unit slope are 0.06 of it for terms of 512 and more."""
+    from ksim_amd import _lib
+    from ksim_amd.recurrent import LSTMCell
+
+    H = 128
+    rng = np.random.default_rng(7)
+    wh = (rng.choice([-1, 1], (4 * H, H)) * rng.uniform(32, 64, (4 * H, H))).astype(np.float32)
+    cell = LSTMCell(np.zeros((4 * H, H), np.float32), wh, np.zeros(4 * H, np.float32), dtype="f32")
+    cell.train_init()
+    h0 = np.zeros((rows, H), np.float32)
+    for m in range(rows):
+        h0[m, rng.choice(H, terms, replace=False)] = rng.uniform(16, 32, terms)
+    exact, size = h0.astype(np.float64) @ wh.T.astype(np.float64), np.abs(h0).astype(np.float64) @ np.abs(wh.T).astype(np.float64)
+    gi = np.zeros((Tn, rows, 4 * H), np.float32)
+    gi[0] = -exact
+    d, z = t32(gi), lambda *s: torch.zeros(*s, device=DEV)  # noqa: E731
+    hs, sv, h, c = z(Tn, rows, H), z(Tn, rows, 7 * H), t32(h0), z(rows, H)
+    lib = _lib.load()
+    _lib.check(lib.ks_lstm_sequence_forward(cell._handle, _lib.current_stream(), Tn, rows, _lib.ptr(d), _lib.ptr(h), _lib.ptr(c), None, _lib.ptr(hs), None,
+                                            _lib.ptr(sv)))
+    act = sv[0, :, : 4 * H].cpu().double()  # i | f | g | o; i, f and o are sigmoids, g is a tanh
+    pre = torch.logit(act)
+    pre[:, 2 * H : 3 * H] = torch.atanh(act[:, 2 * H : 3 * H])
+    assert _largest_error(pre, torch.from_numpy(exact + gi[0]), torch.from_numpy(size)) <= terms * (1 + 2**-4) + 0.1
+
+
+@pytest.mark.parametrize("terms", [1, 2])
+@pytest.mark.parametrize("rows", [5, 1030])
+def test_lstm_gate_gradients_of_few_terms_round_as_often_as_they_have_terms(rows, terms):
+    """The same of the backward product: activations that leave the output gate's gradient alone, a quarter of the hidden state's, one or
+    two units with a gradient at the last step, and one before it that takes the rounded product away; no activation rounds here."""
+    from ksim_amd import _lib
+    from ksim_amd.recurrent import LSTMCell
+
+    H, Tn = 128, 2
+    rng = np.random.default_rng(8)
+    wh = rng.standard_normal((4 * H, H)).astype(np.float32)
+    cell = LSTMCell(np.zeros((4 * H, H), np.float32), wh, np.zeros(4 * H, np.float32), dtype="f32")
+    cell.train_init()
+    sv = torch.zeros(Tn, rows, 7, H, device=DEV)
+    sv[:, :, 3] = 0.5  # the output gate
+    sv[:, :, 4] = 1.0  # tanh of the cell state: nothing reaches that
+    dH = np.zeros((Tn, rows, H), np.float32)
+    for m in range(rows):
+        dH[1, m, rng.choice(H, terms, replace=False)] = rng.standard_normal(terms)
+    gate, w = 0.25 * dH[1].astype(np.float64), wh[3 * H :].astype(np.float64)
+    exact, size = gate @ w, np.abs(gate) @ np.abs(w)
+    dH[0] = -exact
+    d_g = torch.zeros(Tn, rows, 4 * H, device=DEV)
+    lib, d = _lib.load(), t32(dH)
+    _lib.check(lib.ks_lstm_sequence_backward(cell._handle, _lib.current_stream(), Tn, rows, _lib.ptr(d), _lib.ptr(sv), None, _lib.ptr(d_g), None, None))
+    assert _largest_error(4 * d_g[0, :, 3 * H :].cpu(), torch.from_numpy(exact + dH[0]), torch.from_numpy(size)) <= terms * (1 + 2**-4)
