@@ -756,3 +756,38 @@ def test_lstm_gate_gradients_of_few_terms_round_as_often_as_they_have_terms(rows
     lib, d = _lib.load(), t32(dH)
     _lib.check(lib.ks_lstm_sequence_backward(cell._handle, _lib.current_stream(), Tn, rows, _lib.ptr(d), _lib.ptr(sv), None, _lib.ptr(d_g), None, None))
     assert _largest_error(4 * d_g[0, :, 3 * H :].cpu(), torch.from_numpy(exact + dH[0]), torch.from_numpy(size)) <= terms * (1 + 2**-4)
+
+
+@pytest.mark.parametrize("rows", [5, 1030])
+def test_a_row_that_is_not_finite_leaves_the_other_rows_bits_alone(rows):
+    """An infinite, a NaN and a very large entry in one row's state or gradient: every other row gets the bits that it has without them, in one
+    step, in a sequence and in its backward pass, whose workgroups hold sixteen, four and eight rows."""
+    from ksim_amd.recurrent import LSTMCell
+
+    H, Tn, bad = 128, 3, rows - 3
+    rng = np.random.default_rng(11)
+    w = [rng.normal(scale=H ** -0.5, size=s).astype(np.float32) for s in ((4 * H, H), (4 * H, H), (4 * H,))]
+    cell = LSTMCell(*w, dtype="f32")
+    cell.train_init()
+    h0, c0 = (t32(0.5 * rng.normal(size=(rows, H))) for _ in range(2))
+    x, dH = (t32(rng.normal(size=(Tn, rows, H))) for _ in range(2))
+    fresh = torch.zeros(Tn, rows, dtype=torch.uint8, device=DEV)
+    others = torch.arange(rows, device=DEV) != bad
+
+    def run(value):
+        z = lambda t, n: torch.zeros(t, rows, n * H, device=DEV)  # noqa: E731
+        h, d = h0.clone(), dH.clone()
+        if value is not None:
+            h[bad, 5] = d[1, bad, 64] = value
+        hs, cs, sv, dg, hs1, cs1, sv1 = z(Tn, 1), z(Tn, 1), z(Tn, 7), z(Tn, 4), z(1, 1), z(1, 1), z(1, 7)
+        cell.sequence_forward(x, h, c0, fresh, hs, cs, sv)
+        cell.sequence_forward(x[:1].contiguous(), h, c0, fresh[:1].contiguous(), hs1, cs1, sv1)
+        assert all(torch.equal(a[0].nan_to_num(7.0), b[0].nan_to_num(7.0)) for a, b in ((hs, hs1), (cs, cs1), (sv, sv1))), value  # a step is a sequence of one
+        finite = z(Tn, 7)
+        cell.sequence_forward(x, h0, c0, fresh, z(Tn, 1), None, finite)
+        cell.sequence_backward(d, finite, fresh, dg)
+        return [a[:, others] for a in (hs, cs, sv, dg, hs1, cs1, sv1)]
+
+    want = run(None)
+    for value in (float("inf"), float("nan"), 3e37):
+        assert all(torch.equal(a, b) for a, b in zip(run(value), want)), value
