@@ -512,7 +512,9 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
       Tile::first_rows(sum, p);
 #pragma unroll
       for (int q = 0; q < V; ++q) {
-        const float gate = activate(kGate[n], at(gi, (((int64_t)t * M + r0) * 4 + kGate[n]) * H, og[q]) + p[q]);
+        const int64_t o = (int64_t)t * M + r0;
+        const bool starts = (at(fresh, o, jr[q]) & fresh_mask) != 0;  // an episode's first step has no product, whatever the weights are
+        const float gate = activate(kGate[n], at(gi, (o * 4 + kGate[n]) * H, og[q]) + (starts ? 0.f : p[q]));
         v[q][kGate[n]] = fabsf(p[q]) < __builtin_inff() ? v[q][kGate[n]] : gate;
       }
     }
@@ -650,14 +652,17 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
   const int64_t rows_left = M - r0;
   unsigned row[4];
   float c[4], h[4];
+  int live = 0;  // bit i: row i goes on with an episode, whose first step has no product, whatever the weights are
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     row[i] = 4 * (lane >> 4) + i;
     if (row[i] >= rows_left) row[i] = (unsigned)(rows_left - 1);
     const bool f = s.fresh && s.fresh[r0 + row[i]];
+    live |= f ? 0 : 1 << i;
     c[i] = f ? 0.f : at(s.c0, r0 * H, (row[i] * H + unit) * 4);
     if (SAVE) h[i] = f ? 0.f : at(s.h0, r0 * H, (row[i] * H + unit) * 4);
   }
+  asm volatile("" : "+v"(live));  // as selects on four flags it became branches: 34.7 us of 21.6 for 4096 rows
   float g[2][4];
   auto inputs = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
@@ -698,7 +703,7 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
       pre[i] = join_cut(first[0][i], (low[0][i] + (first[2][i] + low[2][i])) + (first[1][i] + low[1][i]));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // the arithmetic of the sequence kernel's pieces
-      float x = g[n % 2][i] + pre[i];
+      float x = g[n % 2][i] + __builtin_bit_cast(float, __builtin_bit_cast(int, pre[i]) & ((int)((unsigned)live << (31 - i)) >> 31));
       x *= gate == 2 ? 2.f * kLog2e : -kLog2e;
       x = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
       v[gate][i] = gate == 2 ? fmaf(-2.f, x, 1.f) : x;

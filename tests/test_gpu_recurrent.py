@@ -791,3 +791,35 @@ def test_a_row_that_is_not_finite_leaves_the_other_rows_bits_alone(rows):
     want = run(None)
     for value in (float("inf"), float("nan"), 3e37):
         assert all(torch.equal(a, b) for a, b in zip(run(value), want)), value
+
+
+@pytest.mark.parametrize("rows", [5, 1030])
+@pytest.mark.parametrize("steps", [1, 3])
+def test_an_episode_start_drops_the_recurrent_product_whatever_the_weights(rows, steps):
+    """A fresh row's gates are its input projection alone: an infinite recurrent weight, an infinite or NaN state carried over from the old
+    episode change nothing in it, as in the gate kernel of the other hidden sizes."""
+    from ksim_amd.recurrent import LSTMCell
+
+    H = 128
+    rng = np.random.default_rng(17)
+    w = [rng.normal(scale=H ** -0.5, size=s).astype(np.float32) for s in ((4 * H, H), (4 * H, H), (4 * H,))]
+    h0, c0 = (0.5 * rng.normal(size=(rows, H)).astype(np.float32) for _ in range(2))
+    x = rng.normal(size=(steps, rows, H)).astype(np.float32)
+    fresh = rng.random((steps, rows)) < 0.5
+    results = []
+    for value in (None, np.inf, -np.inf, np.nan):
+        wh, h = w[1].copy(), h0.copy()
+        if value is not None:
+            wh[::7, 11] = value
+            h[::2, 3] = value
+        cell = LSTMCell(w[0], wh, w[2], dtype="f32")
+        cell.train_init()
+        hs, cs, sv = (torch.zeros(steps, rows, n * H, device=DEV) for n in (1, 1, 7))
+        cell.sequence_forward(t32(x), t32(h), t32(c0), torch.from_numpy(fresh).to(DEV, torch.uint8), hs, cs, sv)
+        results.append([a[torch.from_numpy(fresh).to(DEV)] for a in (hs, cs, sv)])
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))
+    g = torch.from_numpy(x[fresh]).double() @ torch.from_numpy(w[0]).double().T + torch.from_numpy(w[2]).double()
+    i, _, c, o = g.chunk(4, 1)  # zero states: no share of the forget gate
+    want = o.sigmoid() * (i.sigmoid() * c.tanh()).tanh()
+    torch.testing.assert_close(results[0][0].cpu().double(), want, rtol=0, atol=2e-6)  # a sum of 128 terms and the hardware's exponentials
