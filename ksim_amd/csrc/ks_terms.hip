@@ -274,9 +274,14 @@ __device__ inline float rv_value(const KsRandomVar& rv, float u, float z, float 
 constexpr int kTermEnvs = 32;
 // In the launch that also observes, one thread per element, a workgroup takes at most 8: with 32 a launch over a few thousand envs would be too
 // few workgroups to fill the chip.  Fewer still, as many as observe in one round of its 256 threads, while that is no more workgroups than the chip
-// holds at once (kTermObsBlocks): a second and third round are 2 us each, and one is all there is to wait for.  68 elements, 8 -> 3 envs: 64 and 1024
-// envs 15.6 -> 10.2 us, 4096 16.4 -> 12.9; at 16384, where the rule stays with 8, 34.5 -> 40.6.
-constexpr int kTermObsEnvs = 8, kTermObsBlocks = 2048;
+// holds at once, six per CU (kTermObsBlocks): a second and third round are 2 us each, and one is all there is to wait for.  One env to a workgroup, where
+// eight are five rounds and more, still pays with two more per CU (kTermObsBlocks1).  us of the launch in a graph, 8 envs -> this rule (-> without the limit):
+//   elements   envs: 64         1024           last of the rule      beyond it
+//   43        10.3 -> 8.0      10.4 -> 8.3     7500: 12.7 -> 11.5    8500: 13.8 (-> 15.6), 10000: 14.0 (-> 16.2)
+//   68        13.1 -> 8.2      12.9 -> 8.5     4600: 14.6 -> 11.0    4800: 14.7 (-> 14.7), 6000: 14.9 (-> 16.2)
+//   148       16.3 -> 8.0      16.5 -> 8.9     2000: 16.7 -> 14.8    3000: 18.1
+//   468       36.6 -> 10.1     37.3 -> 12.5    2048: 38.0 -> 23.1    3000: 40.3
+constexpr int kTermObsEnvs = 8, kTermObsBlocks = 1536, kTermObsBlocks1 = 2048;
 
 // s_bad: non-finite state seen; s_reset: env starts a fresh episode; s_frame: its frame of the reference motion
 __device__ __forceinline__ void terminate_block(const TerminateArgs& a, int envs, int* s_bad, int* s_reset, int* s_frame) {
@@ -1419,8 +1424,8 @@ extern "C" int ks_terminate_reset_observe(const KsTerms* t, ks_stream_t stream, 
   // the observation half takes the episode starts from the mask the termination half writes in the same launch
   if (oio->fresh && oio->fresh != tio->reset_mask) return fail(KS_EINVAL, "ks_terminate_reset_observe: the observation's fresh flags must be the reset mask of this call");
   if (empty_o) { o.obs_dim = 0; }
-  int envs = o.obs_dim > 0 && o.obs_dim < 256 ? 256 / o.obs_dim : 1;
-  if (envs > kTermObsEnvs || (a.N + envs - 1) / envs > kTermObsBlocks) envs = kTermObsEnvs;
+  int envs = o.obs_dim == 0 ? kTermObsEnvs : o.obs_dim < 256 ? 256 / o.obs_dim : 1;
+  if (envs > kTermObsEnvs || (a.N + envs - 1) / envs > (envs == 1 ? kTermObsBlocks1 : kTermObsBlocks)) envs = kTermObsEnvs;
   const int64_t grid = (a.N + envs - 1) / envs;
   if (grid > 0x7fffffff) return fail(KS_ELIMIT, "ks_terminate_reset_observe: too many envs");
   hipLaunchKernelGGL(terminate_observe_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a, o, envs);

@@ -982,9 +982,9 @@ def test_reset_forward_inside_the_next_step_gives_the_same_trajectories():
                 assert torch.equal(x, y)
 
 
-@pytest.mark.parametrize("N", [1, 7, 6144, 6145])
+@pytest.mark.parametrize("N", [1, 7, 4608, 4609])
 def test_observation_in_the_terminating_launch_at_any_number_of_envs(N):
-    """The launch takes as many envs per workgroup as observe in one round of its threads, more beyond 2048 workgroups: the last workgroup
+    """The launch takes as many envs per workgroup as observe in one round of its threads, more beyond 1536 workgroups: the last workgroup
     part full, on both sides of that line, against the two launches, bit for bit."""
     import dataclasses
 
@@ -993,7 +993,7 @@ def test_observation_in_the_terminating_launch_at_any_number_of_envs(N):
     T, runs = 3, []
     for fuse in (False, True):
         m, c, rnd_, _, _, EnvState = build(N, T, seed=9, min_height=0.86)
-        assert 2048 * (256 // c.terms.obs_dim) == 6144
+        assert 1536 * (256 // c.terms.obs_dim) == 4608
         ro = Rollout(dataclasses.replace(c, fuse_next_observation=fuse), N, T)
         ps = c.engine.reset(c.physics_model, 1.0, 5, N, rnd_)
         traj, _ = ro.unroll(EnvState(ps, rnd_, torch.zeros(N, 2, device=DEV), None, seed=31))
