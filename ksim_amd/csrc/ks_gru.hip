@@ -268,6 +268,7 @@ constexpr int lstm_forward_lds(int rows) { return kSeqWaves * 16 * 64 * 16 + 2 *
 
 constexpr float kLog2e = 1.44269504f;
 constexpr int kStepRows = 16;
+typedef f32x4 f32x4_any __attribute__((aligned(4)));  // a state lies where the caller has it: one load all the same
 
 // holds a value, and with it the arithmetic that follows, to its place between two matrix instructions
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
@@ -640,11 +641,11 @@ __global__ __launch_bounds__(64 * kSeqWaves) __attribute__((amdgpu_waves_per_eu(
   {
     const int row = threadIdx.x >> 5, k = 4 * (threadIdx.x & 31);
     const int64_t m = r0 + row < M ? r0 + row : M - 1;
-    float4 h = *reinterpret_cast<const float4*>(s.h0 + m * H + k);
-    if (s.fresh && s.fresh[m]) h = float4{0.f, 0.f, 0.f, 0.f};
+    f32x4 h = *reinterpret_cast<const f32x4_any*>(s.h0 + m * H + k);
+    if (s.fresh && s.fresh[m]) h = f32x4{0.f, 0.f, 0.f, 0.f};
     unsigned lo[3], hi[3];
-    cut_pair(h.x, h.y, lo);
-    cut_pair(h.z, h.w, hi);
+    cut_pair(h[0], h[1], lo);
+    cut_pair(h[2], h[3], hi);
 #pragma unroll
     for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(&sh[p][row][k]) = uint2{lo[p], hi[p]};
   }

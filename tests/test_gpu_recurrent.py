@@ -823,3 +823,23 @@ def test_an_episode_start_drops_the_recurrent_product_whatever_the_weights(rows,
     i, _, c, o = g.chunk(4, 1)  # zero states: no share of the forget gate
     want = o.sigmoid() * (i.sigmoid() * c.tanh()).tanh()
     torch.testing.assert_close(results[0][0].cpu().double(), want, rtol=0, atol=2e-6)  # a sum of 128 terms and the hardware's exponentials
+
+
+@pytest.mark.parametrize("rows,steps", [(19, 1), (19, 2), (1030, 2)])
+def test_lstm_states_may_lie_at_any_float(rows, steps):
+    """Initial states that are views one float into a buffer, as float addresses allow: the same bits as at aligned ones."""
+    from ksim_amd.recurrent import LSTMCell
+
+    H = 128
+    rng = np.random.default_rng(23)
+    cell = LSTMCell(*(rng.normal(scale=H ** -0.5, size=s) for s in ((4 * H, H), (4 * H, H), (4 * H,))), dtype="f32")
+    h0, c0, x = (t32(rng.normal(size=s)) for s in ((rows, H), (rows, H), (steps, rows, H)))
+    fresh = torch.zeros(steps, rows, dtype=torch.uint8, device=DEV)
+    results = []
+    for shift in (0, 1):
+        h, c, hs, cs = (torch.zeros(n * rows * H + 1, device=DEV)[shift : shift + n * rows * H].view(n, rows, H) for n in (1, 1, steps, steps))
+        h.copy_(h0[None])
+        c.copy_(c0[None])
+        cell.sequence_forward(x, h[0], c[0], fresh, hs, cs, None)
+        results.append((hs.clone(), cs.clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
