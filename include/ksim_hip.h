@@ -89,7 +89,9 @@ int ks_normalize_advantages_static(ks_stream_t stream, int64_t n, const float* g
  *   n = B*T elements, A = action dims; log-probs / entropy are (n, A) row-major.
  *   entropy may be NULL (term omitted, ppo.py:237-239).
  *   policy/value/kl/entropy_loss: per-element outputs (n), each may be NULL.
- *   loss_out: one f32 (device), may be NULL.  workspace as above.
+ *   loss_out: one f32 (device), may be NULL.  workspace as above, all of it written; it holds the blocks' sums until the
+ *   launch's last block has added them up, so it belongs to one call, or one graph's replay, in flight.  Two that overlap on one workspace get
+ *   a NaN for loss_out, and a block of theirs stays on the GPU for up to twenty seconds.
  */
 typedef struct KsPpoLossParams {
   float clip_param;      /* ppo.py:259 default 0.2 */

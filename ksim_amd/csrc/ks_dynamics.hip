@@ -225,8 +225,9 @@ __device__ __forceinline__ bool padded_out(int k, int nv) { return k >= padded_f
 // other; now the chains are 16 columns at most, and what one row of lanes takes off the other are products side by side (row_products).  With the
 // rows kept unscaled (two selects per pair of columns less) a wavefront alone factors and solves M in 4570 cycles instead of 4970, and 4096
 // humanoids' control step has 76.5 M vector instructions instead of 79 M: rollout steps of 64 and of 1024 K-Bots, of 4096 humanoids and of an
-// LSTM policy 1.1, 1.3, 1.3 and 1.0 % faster.  Error of qacc_smooth against 64 bits, rms: 0.70e-6 -> 0.72e-6 (kbot_scale_model), 1.76e-6 -> 1.67e-6
-// (humanoid_model with joint limits), of qacc 1.17e-6 -> 0.96e-6 and 1.75e-6 -> 1.64e-6.
+// LSTM policy 1.1, 1.3, 1.3 and 1.0 % faster.  Error against 64 bits over 6000 random states, as shares of the largest
+// entry, the rotations by quaternions (qrot) included: of qacc_smooth, rms, 0.71e-6 -> 0.70e-6 (kbot_scale_model) and 1.69e-6 -> 1.70e-6 (humanoid_model with joint limits), of qacc, the
+// median env's largest, 2.6e-6 -> 2.2e-6 and 4.1e-6 -> 3.7e-6.
 template <int K, int FIRST, int COUNT>
 __device__ __forceinline__ void row_step(float& w, float c) {
   unsigned long long mask;
@@ -634,9 +635,9 @@ void step_kernel(StepArgs a) {
   // The arguments, and the sizes and LDS offsets that follow from them, are taken afresh in each substep and in the
   // write-back: `s_load`s through the scalar cache and a little scalar arithmetic.  Taken once, the ~60 pointers, sizes and
   // offsets stay live across the solver, which leaves SGPRs for a third of them: the rest lay in VGPR lanes (194
-  // `v_writelane`s and ~280 `v_readlane`s, all of them VALU work, and two VGPRs of a file that is full; now 33 and 54, and
-  // none of the scratch that went with it).  4096 humanoid envs: 82.4 M -> 79.1 M VALU instructions a launch, 253.3 -> 246.6
-  // us; the pointers alone, without sizes and offsets, 248.1 us.
+  // `v_writelane`s and ~280 `v_readlane`s, all of them VALU work, and two VGPRs of a file that is full; now 38 of the former; three
+  // VGPRs of the 28-dof instance spill, 768 B of scratch an env and step).  4096 humanoid envs: 82.4 M -> 79.1 M VALU
+  // instructions a launch, 253.3 -> 246.6 us; the pointers alone, without sizes and offsets, 248.1 us.
   const auto arguments = []() -> const StepArgs& {
     typedef const __attribute__((address_space(4))) StepArgs* ArgsPtr;
     ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();  // the kernel's one parameter lies at its start

@@ -211,8 +211,7 @@ constexpr int kSeqRows = 4, kSeqH = 128, kSeqWaves = 8, kSeqPadH = kSeqH + 4;
 
 __device__ __forceinline__ float sigmoid_ks(float x) { return 1.f / (1.f + expf(-x)); }
 
-// 1 / (1 + e^-x) and tanh x = 1 - 2 / (e^2x + 1) on v_exp_f32 and v_rcp_f32; both saturate correctly (e^y = inf gives 0 and -1 + 2 = 1)
-__device__ __forceinline__ float seq_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+// tanh x = 1 - 2 / (e^2x + 1) on v_exp_f32 and v_rcp_f32; it saturates correctly (e^y = inf gives 1, e^y = 0 gives -1)
 __device__ __forceinline__ float seq_tanh(float x) { return 1.f - 2.f * __builtin_amdgcn_rcpf(__expf(2.f * x) + 1.f); }
 
 // Barrier for data that the wavefronts of a workgroup hand each other through LDS only: it waits for this wavefront's LDS
@@ -376,7 +375,7 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
   // without episode starts a byte of the inputs is read in the flag's place and masked away
   const uint8_t* __restrict__ fresh = s.fresh ? s.fresh : (const uint8_t*)s.in;
   const unsigned fresh_mask = s.fresh ? 0xffu : 0u;
-  float *hs = s.out0, *cs = s.out1;  // with T = 1, hs / cs may be h0 / c0
+  float *hs = s.out0, *cs = s.out1;
   float* __restrict__ saved = s.saved;
   if ((int64_t)blockIdx.x * groups * R >= M) return;  // the other layer of the launch has more rows
   extern __shared__ __attribute__((aligned(16))) unsigned char seq_lds[];
@@ -403,8 +402,8 @@ void lstm_seq_forward_kernel(int T, int groups, Seq first, Seq second) {
       w2[(n * KB + kb) * 64] = part[2];
     }
   }
-  // A workgroup takes `groups` sets of R rows one after the other with the same registers of weights: a single step over
-  // thousands of rows (the rollout's call) would otherwise fetch the 256 KB of W_hh once per set.
+  // A workgroup takes `groups` sets of R rows one after the other with the same registers of weights: a few steps over
+  // thousands of rows would otherwise fetch and cut the 256 KB of W_hh once per set (two layers, 4096 rows x 2 steps 51.5 us of 38, 8192 x 8 215 of 179).
   for (int grp = 0; grp < groups; ++grp) {
   const int64_t r0 = ((int64_t)blockIdx.x * groups + grp) * R;
   if (r0 >= M) break;  // the same for every thread of the workgroup
