@@ -8,6 +8,7 @@ per-launch host cost out of the loop (`Rollout.unroll(..., graph=True)`).
 """
 from __future__ import annotations
 
+import operator
 from dataclasses import dataclass
 from typing import Mapping, Sequence
 
@@ -161,15 +162,15 @@ class Rollout:
             raise _lib.KsError("critic must map the observation vector to one value")
 
     def _observation_key(self, env: RolloutEnvState, sources: Mapping, t: int, step: int, relative: bool, level: float):
-        """What the observation of slot t is made of: objects, and numbers with how often the engine and torch have written to them.
-        None where torch does not count that (inference mode)."""
-        site = (env.randomization_dict or {}).get("site_pose")
-        tensors = [x for x in (*sources.values(), env.physics_state.zero_offset, env.obs_bias, env.obs_carry, site, self.reset_mask,
-                               self.obs, self.noisy_obs) if x is not None]
-        if any(x.is_inference() for x in tensors):
+        """What an observation ahead of slot t is made of (it reads no derived field): objects, and numbers with how often the engine and
+        torch have written to them.  None where torch does not count that (inference mode)."""
+        ps = env.physics_state
+        read = (env, self.c.terms, sources[T.SRC_QPOS], sources[T.SRC_QVEL], sources[T.SRC_LAST_ACTION], sources[T.SRC_COMMAND], sources[T.SRC_TIME],
+                ps.zero_offset, env.obs_bias, env.obs_carry, (env.randomization_dict or {}).get("site_pose"), self.reset_mask, self.obs, self.noisy_obs)
+        try:
+            return read, (t, step, relative, float(level), env.seed, getattr(ps, "_written", 0), *[x._version for x in read[2:] if x is not None])
+        except RuntimeError:
             return None
-        written = getattr(env.physics_state, "_written", 0)
-        return [env, self.c.terms, *tensors], [t, step, relative, float(level), env.seed, written, *(x._version for x in tensors)]
 
     def step_engine(self, env: RolloutEnvState, t: int, level: float = 1.0, noise: Mapping | None = None,
                     _relative_step: bool = False, _in_loop: bool = False) -> None:
@@ -193,7 +194,7 @@ class Rollout:
 
         ahead = self._obs_done if not noise else None
         now = ahead and self._observation_key(env, src, t, step, _relative_step, level)
-        if not now or ahead[1] != now[1] or any(a is not b for a, b in zip(ahead[0], now[0])):  # else the launch that ended the previous step wrote it
+        if not now or ahead[1] != now[1] or not all(map(operator.is_, ahead[0], now[0])):  # else the launch that ended the previous step wrote it
             c.terms.observe(src, self.N, bias_redraw=noise.get("obs_bias_redraw"), noise_normal=noise.get("obs_normal"),
                             noise_uniform=noise.get("obs_uniform"), carry_uniform=noise.get("obs_carry_uniform"),
                             **observe_args(t, step))
