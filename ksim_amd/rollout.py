@@ -285,11 +285,13 @@ class Rollout:
                          event_reset_uniform=noise.get("event_reset_uniform"),
                          event_force=ps.event_states.get("_force_buffer") if ps.event_states else None,
                          contact_dist=d.contact_dist if "contact_dist" in self._live else None, episode=c.engine.episode_args(ps, noise.get("episode")))
+        ahead = None
         if self._fuse_obs and t + 1 < self.T and not noise and (_in_loop or _relative_step or not c.terms.carry_dim):
-            self._obs_done = self._observation_key(env, src, t + 1, step + 1, _relative_step, level)
-        if self._obs_done is not None:
+            ahead = self._observation_key(env, src, t + 1, step + 1, _relative_step, level)
+        if ahead is not None:
             # the next step's observation rides in this launch (its random numbers are those of step + 1)
             c.terms.terminate_reset_observe(st, term_args, src, observe_args(t + 1, step + 1))
+            self._obs_done = ahead
         else:
             c.terms.terminate_reset(st, **term_args)
         # refresh the derived fields and the warm start of the reset envs (engine.py:213); in the deferred mode the next
